@@ -10,6 +10,7 @@
 // rotation are applied by k_qk_rope_store before the keys enter the cache, the values have a size of their own, the sink has a fixed
 // score and the window may be unlimited; a layer may read the cache rows that an earlier layer has written.
 #include <algorithm>
+#include <vector>
 #include "ifa_host.h"
 #include "ifa_f32_common.h"
 #include "inferflow_amd.h"
@@ -180,13 +181,15 @@ __global__ void __launch_bounds__(64) k_attn_window_combine(WinAttnArgs P)
     }
 }
 
-// ---- prompts: 128 queries of one sequence per workgroup, the visible keys walked in blocks of 32 that are staged ONCE per workgroup
+typedef float f32x16w __attribute__((ext_vector_type(16)));
+constexpr int WT_K = 32;          // keys of a block
+
+// ---- prompts without a workspace: 128 queries of one sequence per workgroup, the visible keys walked in blocks of 32 that are staged ONCE per workgroup
 // in LDS; each wave owns 32 queries, one per lane of each half: S^T = K Q^T and O^T += V^T P^T on the fp32 matrix cores
 // (v_mfma_f32_32x32x2_f32: scores and weights stay 32-bit).  In the transposed products a lane's accumulators hold 16 keys of ITS
 // query, so the online softmax (running maximum, weights, rescaling of O^T) is lane-local but for one exchange between the halves,
 // and the weights are the second product's B operand as they lie in the accumulators: no trip through LDS.
-typedef float f32x16w __attribute__((ext_vector_type(16)));
-constexpr int WT_Q = 128, WT_K = 32;
+constexpr int WT_Q = 128;
 
 // Key rows of dim <= 32 NTK and value rows of vdim <= 32 NTV floats; the columns beyond are zero in LDS.
 template <int NTK, int NTV>
@@ -353,6 +356,470 @@ __global__ void __launch_bounds__(256) k_attn_window_tile(WinAttnArgs P, int n_s
     }
 }
 
+// ---- prompts with a workspace, on the bfloat16 matrix cores.  A workgroup of eight waves holds 32 queries of up to four query heads that share a key / value head
+// (hpw heads; the waves take further queries beyond them) and walks a share of their visible keys in blocks of 32.  The products are transposed as above.
+// Arithmetic: every 32-bit operand is the sum of three bfloat16 values (24 bits: nothing is lost but the last rounding), and a product takes
+// the six of the nine partial products that reach 2^-24 of the largest: 6 x 32 matrix-core cycles per 16 columns where the fp32 instructions
+// take 512.  Error against 64 bits: no larger than the fp32 instructions' (test_tiled_attention_with_a_workspace_against_64_bits_and_the_fp32_tiles).
+// An infinite value in a V row gives NaN (0 x inf of a lower part) where fp32 gives inf.
+// The fp32 tiles above took 487 us for 2048 causal tokens of 8 heads of 128 (16 tiles x 8 heads on half of the compute units, the last tile alone walking 64 blocks)
+// and 420 us for 16 heads with a window of 1024, soft cap and bias; this form 83 and 146 us, of it 6 us for the operands and 14 us for joining the
+// shares.  Bound by matrix cores and vector instructions in turn (3072 and ~2500 cycles per wave and block; the waves of a SIMD do not drift apart enough to
+// overlap them).  Hence the operands are split and laid out once per layer by k_attn_parts, not by every tile that reads them (staged and split per
+// workgroup: 126 us), and the key blocks of long tiles go to several workgroups (chunks of cb blocks, joined by k_attn_tile_combine).
+typedef __bf16 bf16x8w __attribute__((ext_vector_type(8)));
+constexpr int WT_WAVES = 8, WT_MAX_CHUNKS = 32, WT_SLOTS = 256;
+
+typedef float f32x4w __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(1))) float gfloat;
+typedef const __attribute__((address_space(1))) f32x4w gf32x4;
+typedef const __attribute__((address_space(1))) void wa_glb_t;
+typedef __attribute__((address_space(3))) void wa_lds_t;
+
+struct Parts { bf16x8w p[3]; };
+
+__device__ __forceinline__ Parts parts_of(const float *v)
+{
+    Parts r;
+    float big = 0.0f, d[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) big = fmaxf(big, __builtin_fabsf(v[e]));
+#pragma unroll
+    for (int e = 0; e < 8; e++) { r.p[0][e] = (__bf16)v[e]; d[e] = v[e] - (float)r.p[0][e]; }
+    if (__builtin_amdgcn_ballot_w64(big > 3.38e38f)) {          // (infinities stay in the first part)
+#pragma unroll
+        for (int e = 0; e < 8; e++) d[e] = __builtin_fabsf(v[e]) > 3.38e38f ? 0.0f : d[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) { r.p[1][e] = (__bf16)d[e]; r.p[2][e] = (__bf16)(d[e] - (float)r.p[1][e]); }
+    return r;
+}
+
+// the five partial products below the leading one, smallest first
+__device__ __forceinline__ f32x16w mfma_rest(const Parts &a, const Parts &b, f32x16w c)
+{
+    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[2], b.p[0], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0], b.p[2], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[1], b.p[1], c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[1], b.p[0], c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0], b.p[1], c, 0, 0, 0);
+}
+
+// exp(x) for x <= 0 to within a rounding or two: the rounding of x log2(e) is carried along (the exponential of a plain fp32 product would be off
+// by |x| 2^-24); NaN stays NaN
+__device__ __forceinline__ float exp_neg(float x)
+{
+    x = x < -1.0e4f ? -1.0e4f : x;
+    const float hi = x * 1.44269502f, lo = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269502f, -hi));
+    const float e = __builtin_amdgcn_exp2f(hi);
+    return fmaf(e, lo * 0.693147182f, e);
+}
+
+// tanh(y) to within two roundings, without a branch: the continued fraction y / (1 + y^2 / (3 + y^2 / (5 + y^2 / (7 + y^2 / 9)))) as a quotient where |y| < 0.6
+// (its remainder is below 1e-9 there), (1 - e) / (1 + e) with e = exp(-2 |y|) elsewhere
+__device__ __forceinline__ float tanh_sel(float y)
+{
+    const float a = __builtin_fabsf(y), z = y * y, e = exp_neg(-2.0f * a);
+    const bool small = a < 0.6f;
+    const float n = small ? a * fmaf(z, z + 105.0f, 945.0f) : 1.0f - e, d = small ? fmaf(z, fmaf(z, 15.0f, 420.0f), 945.0f) : 1.0f + e;
+    const float r = __builtin_amdgcn_rcpf(d), t = n * r;
+    return __builtin_copysignf(fmaf(fmaf(-t, d, n), r, t), y);
+}
+
+// The key blocks of a sequence are counted in absolute positions (block = position / 32).  What k_attn_parts lays out for a step: the blocks of the
+// kept first tokens, then those from the first one that the step's first query sees to the last.
+struct SeqBlocks { int kept, first, count; };
+__host__ __device__ __forceinline__ SeqBlocks seq_blocks(int pos0, int n, int window, int keep_first)
+{
+    const int lo = pos0 - window + 1 > 0 ? pos0 - window + 1 : 0, end = pos0 + n, keep = keep_first < end ? keep_first : end;
+    SeqBlocks s;
+    s.kept = (keep + WT_K - 1) / WT_K;
+    s.first = s.kept > lo / WT_K ? s.kept : lo / WT_K;
+    const int more = (end - 1) / WT_K - s.first + 1;
+    s.count = s.kept + (more > 0 ? more : 0);
+    return s;
+}
+// the blocks that nq queries from position p0 on see: 0 .. kept - 1, then `first` and on, nb in all
+struct TileBlocks { int kept, first, nb; };
+__host__ __device__ __forceinline__ TileBlocks tile_blocks(int p0, int nq, int window, int keep_first)
+{
+    const int lo = p0 - window + 1 > 0 ? p0 - window + 1 : 0, keep = keep_first < lo ? keep_first : lo;
+    TileBlocks t;
+    t.kept = (keep + WT_K - 1) / WT_K;
+    t.first = t.kept > lo / WT_K ? t.kept : lo / WT_K;
+    const int more = (p0 + nq - 1) / WT_K - t.first + 1;
+    t.nb = t.kept + (more > 0 ? more : 0);
+    return t;
+}
+
+struct TileArgs { int n_seqs, hpw, cb, tiles; size_t shares; };      // shares: where the chunks' partial results begin in the workspace (floats), behind the operands
+
+// the sequence and the tile of it (tiles of qw queries, numbered over the sequences) and the operand blocks of the sequences before it, or false
+__device__ __forceinline__ bool tile_of(const WinAttnArgs &P, int n_seqs, int qw, int &tile, SeqDesc &sd, int &block0)
+{
+    block0 = 0;
+    for (int sq = 0; sq < n_seqs; sq++) {
+        sd = P.seqs[sq];
+        const int nt = (sd.n + qw - 1) / qw;
+        if (tile < nt) return true;
+        tile -= nt;
+        block0 += seq_blocks(sd.pos0, sd.n, P.window, P.keep_first).count;
+    }
+    return false;
+}
+
+// The id-th chunk of the step, the chunks numbered tile by tile from the last tile on: its tile and its number there.  A grid of tiles x chunks would do without
+// this, but its empty places leave some XCD with more chunks than compute units, and the launch takes twice as long (100 against 50 us at 2048 tokens).
+__device__ __forceinline__ bool chunk_of(const WinAttnArgs &P, const TileArgs &A, int qw, int id, int &tile_g, int &chunk)
+{
+    const int lane = threadIdx.x & 63;
+    for (int t0 = 0; t0 < A.tiles; t0 += 64) {
+        int n = 0, tile = A.tiles - 1 - t0 - lane, block0;
+        SeqDesc sd;
+        if (tile >= 0 && tile_of(P, A.n_seqs, qw, tile, sd, block0))
+            n = (tile_blocks(sd.pos0 + tile * qw, min(qw, sd.n - tile * qw), P.window, P.keep_first).nb + A.cb - 1) / A.cb;
+        int upto = n;
+#pragma unroll
+        for (int k = 1; k < 64; k <<= 1) { const int x = __shfl_up(upto, k, 64); if (lane >= k) upto += x; }
+        const uint64_t past = __builtin_amdgcn_ballot_w64(upto > id);
+        if (past) {
+            const int at = __builtin_ctzll(past);
+            tile_g = A.tiles - 1 - t0 - at;
+            chunk = id - (__builtin_amdgcn_readlane(upto, at) - __builtin_amdgcn_readlane(n, at));
+            return true;
+        }
+        id -= __builtin_amdgcn_readlane(upto, 63);
+    }
+    return false;
+}
+
+// Operands of one block of 32 keys as the matrix instructions take them, [part][16 columns][lane][8]: keys (lane = 32 g + key, columns 16 ks + 8 g ..), then
+// values transposed (lane = 32 g + column, keys in the order in which the scores' accumulators hold them).  Columns beyond the rows' ends are zero.
+template <int NTK, int NTV> constexpr int kBlockPieces = 3 * 64 * (2 * NTK + 2 * NTV);
+
+// grid (kv heads, blocks of the step): the cache rows of a block into its operands -- once per layer and step, not once per tile that reads the block.
+// Bound by its launch and one trip to memory (reads 4, writes 6 bytes per value).  Rows past the sequence's last: that row again (their scores are masked).
+template <int NTK, int NTV>
+__global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, int n_seqs)
+{
+    constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK;
+    const int tid = threadIdx.x, kvh = blockIdx.x, dk = P.dim, dv = P.vdim;
+    int at = blockIdx.y, sq = 0;
+    SeqDesc sd;
+    SeqBlocks sb;
+    for (; sq < n_seqs; sq++) {
+        sd = P.seqs[sq];
+        sb = seq_blocks(sd.pos0, sd.n, P.window, P.keep_first);
+        if (at < sb.count) break;
+        at -= sb.count;
+    }
+    if (sq >= n_seqs) return;
+    const int kb0 = (at < sb.kept ? at : sb.first + at - sb.kept) * WT_K, last = sd.pos0 + sd.n - 1;
+    const size_t kvd = (size_t)P.kv_heads * dk, vvd = (size_t)P.kv_heads * dv;
+    gfloat *kc = (gfloat *)(P.slot_base[sd.slot] + P.k_off + (size_t)kvh * dk), *vc = (gfloat *)(P.slot_base[sd.slot] + P.v_off + (size_t)kvh * dv);
+    bf16x8w *dst = (bf16x8w *)P.ws + ((size_t)blockIdx.y * P.kv_heads + kvh) * kBlockPieces<NTK, NTV>;
+    const bool vec = dk % 4 == 0 && P.k_off % 4 == 0;      // (arena bases are 256-byte aligned)
+    for (int e = tid; e < WT_K * (DK / 8); e += 256) {
+        const int key = e / (DK / 8), c8 = e % (DK / 8), c = 8 * c8;
+        gfloat *row = kc + (size_t)min(kb0 + key, last) * kvd;
+        float v[8];
+        if (vec) {
+            const f32x4w lo = *(gf32x4 *)(row + min(c, dk - 4)), hi = *(gf32x4 *)(row + min(c + 4, dk - 4));
+#pragma unroll
+            for (int x = 0; x < 4; x++) { v[x] = c < dk ? lo[x] : 0.0f; v[4 + x] = c + 4 < dk ? hi[x] : 0.0f; }
+        } else {
+#pragma unroll
+            for (int x = 0; x < 8; x++) { const float f = row[min(c + x, dk - 1)]; v[x] = c + x < dk ? f : 0.0f; }
+        }
+        const Parts t = parts_of(v);
+#pragma unroll
+        for (int pl = 0; pl < 3; pl++) dst[(pl * KS + (c8 >> 1)) * 64 + 32 * (c8 & 1) + key] = t.p[pl];
+    }
+    dst += 3 * KS * 64;
+    for (int e = tid; e < 4 * DV; e += 256) {
+        const int d = e % DV, sg = e / DV, k0 = 16 * (sg >> 1) + 4 * (sg & 1);
+        float v[8];
+#pragma unroll
+        for (int x = 0; x < 8; x++) { const float f = vc[(size_t)min(kb0 + k0 + 8 * (x >> 2) + (x & 3), last) * vvd + min(d, dv - 1)]; v[x] = d < dv ? f : 0.0f; }
+        const Parts t = parts_of(v);
+#pragma unroll
+        for (int pl = 0; pl < 3; pl++) dst[((pl * NTV + (d >> 5)) * 2 + (sg >> 1)) * 64 + 32 * (sg & 1) + (d & 31)] = t.p[pl];
+    }
+}
+
+// Key rows of dim <= 32 NTK and value rows of vdim <= 32 NTV floats.  VEC: rows of whole, aligned 16-byte pieces in q and the output.
+template <int NTK, int NTV, bool VEC>
+__global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, TileArgs A)
+{
+    constexpr int KS = 2 * NTK, PIECES = kBlockPieces<NTK, NTV>;
+    extern __shared__ bf16x8w ops[];                          // two blocks' operands, then a bias table per wave
+    float *bias = (float *)(ops + 2 * PIECES) + 64 * (threadIdx.x >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5;
+    const int h = blockIdx.x * A.hpw + wave % A.hpw, qsub = wave / A.hpw, kvh = blockIdx.x * A.hpw / (P.heads / P.kv_heads), dk = P.dim, dv = P.vdim;
+    const int qw = 32 * (WT_WAVES / A.hpw);
+    int tile_g, chunk, block0;
+    if (!chunk_of(P, A, qw, blockIdx.y, tile_g, chunk)) return;
+    int tile = tile_g;
+    SeqDesc sd;
+    if (!tile_of(P, A.n_seqs, qw, tile, sd, block0)) return;
+    const int r0 = sd.row0 + tile * qw, nq = min(qw, sd.n - tile * qw), p0 = sd.pos0 + tile * qw;
+    const SeqBlocks sb = seq_blocks(sd.pos0, sd.n, P.window, P.keep_first);
+    const TileBlocks tb = tile_blocks(p0, nq, P.window, P.keep_first);
+    const int nch = (tb.nb + A.cb - 1) / A.cb, b0 = chunk * A.cb, b1 = min(tb.nb, b0 + A.cb);
+    const int nq_w = min(32, max(0, nq - 32 * qsub)), qlo = p0 + 32 * qsub, qhi = qlo + nq_w - 1;          // queries of this wave, their positions
+    const bool qin = i < nq_w;
+    const float inv_cap = P.softcap > 0.0f ? 1.0f / P.softcap : 0.0f;
+    // a block's operands go from memory to LDS directly, asked for behind the scores of the block before (whose operand reads would wait for them):
+    // they land under its softmax
+    auto fetch = [&](int b) {
+        const int block = b < tb.kept ? b : tb.first + b - tb.kept, at = block < sb.kept ? block : sb.kept + block - sb.first;
+        const bf16x8w *src = (const bf16x8w *)P.ws + ((size_t)(block0 + at) * P.kv_heads + kvh) * PIECES;
+        bf16x8w *dst = ops + (b & 1) * PIECES;
+#pragma unroll
+        for (int u = 0; u < PIECES / 64; u += WT_WAVES)
+            if (u + wave < PIECES / 64)
+                __builtin_amdgcn_global_load_lds((wa_glb_t *)(src + (u + wave) * 64 + lane), (wa_lds_t *)(dst + (u + wave) * 64), 16, 0, 0);
+    };
+    fetch(b0);
+    // the lane's query, normed, in three parts (queries past the tile's last: that one again, not stored)
+    Parts q[KS];
+    {
+        gfloat *qr = (gfloat *)P.q + (size_t)(r0 + min(32 * qsub + i, nq - 1)) * P.ldq + (size_t)h * dk;
+        auto piece = [&](int c, float (&v)[8]) {
+            if constexpr (VEC) {
+                const f32x4w lo = *(gf32x4 *)(qr + min(c, dk - 4)), hi = *(gf32x4 *)(qr + min(c + 4, dk - 4));
+#pragma unroll
+                for (int x = 0; x < 4; x++) { v[x] = c < dk ? lo[x] : 0.0f; v[4 + x] = c + 4 < dk ? hi[x] : 0.0f; }
+            } else {
+#pragma unroll
+                for (int x = 0; x < 8; x++) { const float f = qr[min(c + x, dk - 1)]; v[x] = c + x < dk ? f : 0.0f; }
+            }
+        };
+        float v[8], r = 1.0f;
+        if (P.norm_q) {
+            float s = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {
+                piece(16 * ks + 8 * g, v);
+#pragma unroll
+                for (int x = 0; x < 8; x++) s = fmaf(v[x], v[x], s);
+            }
+            r = 1.0f / sqrtf((s + __shfl_xor(s, 32, 64)) / (float)dk + P.eps);
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            piece(16 * ks + 8 * g, v);
+#pragma unroll
+            for (int x = 0; x < 8; x++) v[x] *= r;
+            q[ks] = parts_of(v);
+            if (ks & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    f32x16w o[NTV];
+    float m = -INFINITY, l = 0.0f;          // of the lane's query
+#pragma unroll
+    for (int nt = 0; nt < NTV; nt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[nt][r] = 0.0f;
+    for (int b = b0; b < b1; b++) {
+        const int kb0 = (b < tb.kept ? b : tb.first + b - tb.kept) * WT_K;
+        const bool active = nq_w > 0 && kb0 <= qhi && (kb0 + WT_K - 1 >= qlo - P.window + 1 || kb0 < P.keep_first);
+        // this wave's share of the block has landed, and behind the barrier every wave's, and no wave reads the other buffer any more
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (!active) { if (b + 1 < b1) fetch(b + 1); continue; }
+        const bf16x8w *Kp = ops + (b & 1) * PIECES, *Vp = Kp + 3 * KS * 64;
+        f32x16w acc;
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+        {
+            Parts k[2];
+            auto read_k = [&](int ks) {
+#pragma unroll
+                for (int pl = 0; pl < 3; pl++) k[ks & 1].p[pl] = Kp[(pl * KS + ks) * 64 + lane];
+            };
+            read_k(0);
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {          // (the next operands are on their way behind the products of these; no further ahead: registers)
+                if (ks + 1 < KS) read_k(ks + 1);
+                acc = mfma_rest(k[ks & 1], q[ks], acc);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k[ks & 1].p[0], q[ks].p[0], acc, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[r] *= P.scale;
+        if (P.softcap > 0.0f) {
+            __builtin_amdgcn_sched_barrier(0);          // (or the branch is turned into computing it always)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[r] = P.softcap * tanh_sel(acc[r] * inv_cap);
+        }
+        if (P.rel) {           // the bias by distance, one distance a lane: entry 31 + i - kk of the block
+            const int dist = qlo - kb0 - 31 + lane;
+            bias[lane] = dist >= 0 && dist <= qhi - kb0 && (dist < P.window || kb0 < P.keep_first) ? bf2f(P.rel[(size_t)P.bucket_of[dist] * P.heads + h]) : 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[r] += bias[31 + i - ((r & 3) + 8 * (r >> 2) + 4 * g)];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (b + 1 < b1) fetch(b + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        // (blocks that every query of the wave sees whole need no masks)
+        if (!(nq_w == 32 && kb0 + WT_K - 1 <= qlo && (qhi - kb0 < P.window || kb0 + WT_K <= P.keep_first))) {
+            const int iq = qlo + i;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int j = kb0 + (r & 3) + 8 * (r >> 2) + 4 * g;
+                if (!(qin && j <= iq && (iq - j < P.window || j < P.keep_first))) acc[r] = -INFINITY;
+            }
+        }
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; r++) mloc = fmaxf(mloc, acc[r]);
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+        const float m_new = fmaxf(m, mloc), m_use = m_new == -INFINITY ? 0.0f : m_new;      // (-inf only while nothing was visible: sums are 0)
+        const float corr = m == -INFINITY ? 1.0f : exp_neg(m - m_new);
+        float psum = 0.0f, w[2][8];
+#pragma unroll
+        for (int r = 0; r < 16; r++) { const float p = exp_neg(acc[r] - m_use); w[r >> 3][r & 7] = p; psum += p; }
+        l = l * corr + psum;             // (the keys of this half of the wave; the halves are added at the end)
+        m = m_new;
+        const Parts w0 = parts_of(w[0]), w1 = parts_of(w[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        Parts v[2];
+        auto read_v = [&](int u) {
+#pragma unroll
+            for (int pl = 0; pl < 3; pl++) v[u & 1].p[pl] = Vp[(pl * NTV * 2 + u) * 64 + lane];
+        };
+        read_v(0);
+#pragma unroll
+        for (int u = 0; u < 2 * NTV; u++) {
+            if (u + 1 < 2 * NTV) read_v(u + 1);
+            f32x16w &on = o[u >> 1];
+            if (!(u & 1)) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) on[r] *= corr;
+            }
+            on = mfma_rest(v[u & 1], u & 1 ? w1 : w0, on);
+            on = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v[u & 1].p[0], (u & 1 ? w1 : w0).p[0], on, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // the lane holds value columns 32 nt + (r & 3) + 8 (r >> 2) + 4 g of its query
+    const float ls = l + __shfl_xor(l, 32, 64);
+    if (nch > 1) {                       // this chunk's share: [maximum][sum][columns] x 32 queries
+        float *dst = P.ws + A.shares + ((((size_t)tile_g * gridDim.x + blockIdx.x) * P.nsplit + chunk) * WT_WAVES + wave) * 32 * (dv + 2) + i;
+        if (g == 0) { dst[0] = m; dst[32] = ls; }
+#pragma unroll
+        for (int nt = 0; nt < NTV; nt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int c = 32 * nt + (r & 3) + 8 * (r >> 2) + 4 * g;
+                if (c < dv) dst[(size_t)(2 + c) * 32] = o[nt][r];
+            }
+        return;
+    }
+    if (!qin) return;
+    const float snk = sink_of(P, h);
+    const float M = fmaxf(m, snk);
+    const float f = expf(m - M);
+    const float sc = f / (ls * f + (has_sink(P) ? expf(snk - M) : 0.0f));
+    float *dst = P.out + (size_t)(r0 + 32 * qsub + i) * P.ldo + (size_t)h * dv;
+#pragma unroll
+    for (int nt = 0; nt < NTV; nt++)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+            const int c = 32 * nt + 8 * (r >> 2) + 4 * g;
+            if constexpr (VEC) { if (c < dv) *reinterpret_cast<float4 *>(dst + c) = make_float4(o[nt][r] * sc, o[nt][r + 1] * sc, o[nt][r + 2] * sc, o[nt][r + 3] * sc); }
+            else {
+#pragma unroll
+                for (int x = 0; x < 4; x++) if (c + x < dv) dst[c + x] = o[nt][r + x] * sc;
+            }
+        }
+}
+
+// the chunks' shares of 32 queries of a head and its sink into the output rows: grid (heads / hpw, tiles, waves of k_attn_tile)
+__global__ void __launch_bounds__(256) k_attn_tile_combine(WinAttnArgs P, TileArgs A)
+{
+    __shared__ float fs[WT_MAX_CHUNKS][32], rows[32][129];
+    const int tid = threadIdx.x, wave = blockIdx.z, h = blockIdx.x * A.hpw + wave % A.hpw, qsub = wave / A.hpw, dv = P.vdim, qw = 32 * (WT_WAVES / A.hpw), tile_g = blockIdx.y;
+    int tile = tile_g, block0;
+    SeqDesc sd;
+    if (!tile_of(P, A.n_seqs, qw, tile, sd, block0)) return;
+    const int nq = min(qw, sd.n - tile * qw), nq_w = min(32, nq - 32 * qsub);
+    const int nch = (tile_blocks(sd.pos0 + tile * qw, nq, P.window, P.keep_first).nb + A.cb - 1) / A.cb;
+    if (nch <= 1 || nq_w <= 0) return;
+    const size_t share = (size_t)WT_WAVES * 32 * (dv + 2);
+    const float *src = P.ws + A.shares + (((size_t)tile_g * gridDim.x + blockIdx.x) * P.nsplit * WT_WAVES + wave) * 32 * (dv + 2);
+    if (tid < 32) {
+        const float snk = sink_of(P, h);
+        float M = snk, L = 0.0f, m[WT_MAX_CHUNKS], ls[WT_MAX_CHUNKS];
+#pragma unroll
+        for (int c = 0; c < WT_MAX_CHUNKS; c++) {
+            const size_t at = (size_t)min(c, nch - 1) * share + tid;
+            m[c] = src[at]; ls[c] = src[at + 32];
+        }
+#pragma unroll
+        for (int c = 0; c < WT_MAX_CHUNKS; c++) M = fmaxf(M, m[c]);
+#pragma unroll
+        for (int c = 0; c < WT_MAX_CHUNKS; c++) {
+            m[c] = c >= nch || m[c] == -INFINITY ? 0.0f : expf(m[c] - M);
+            L += ls[c] * m[c];
+        }
+        if (has_sink(P)) L += expf(snk - M);
+#pragma unroll
+        for (int c = 0; c < WT_MAX_CHUNKS; c++) fs[c][tid] = m[c] / L;
+    }
+    __syncthreads();
+    // (a thread's columns side by side, two chunks ahead: the loads are what this launch waits for)
+    const int q = tid & 31;
+    float o[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) o[k] = 0.0f;
+#pragma unroll 2
+    for (int c = 0; c < nch; c++)
+#pragma unroll
+        for (int k = 0; k < 16; k++) o[k] = fmaf(src[c * share + (size_t)(2 + min((tid >> 5) + 8 * k, dv - 1)) * 32 + q], fs[c][q], o[k]);
+#pragma unroll
+    for (int k = 0; k < 16; k++) rows[q][(tid >> 5) + 8 * k] = o[k];
+    __syncthreads();
+    float *dst = P.out + (size_t)(sd.row0 + tile * qw + 32 * qsub) * P.ldo + (size_t)h * dv;
+    for (int e = tid; e < nq_w * dv; e += 256) dst[(size_t)(e / dv) * P.ldo + e % dv] = rows[e / dv][e % dv];
+}
+
+// How a step's tiles are shared out: hpw query heads and qw queries per workgroup, cb key blocks per chunk, up to `chunks` chunks per tile, so that the
+// chunks just fill the compute units once (one workgroup each: registers and LDS); below two blocks a chunk the partial results cost more than
+// the wait they save.  op_bytes: workspace of the blocks' operands, bytes: with the chunks' shares (none with one chunk).
+struct TilePlan { int hpw, qw, cb, chunks; size_t tiles, groups, blocks, op_bytes, bytes; };
+TilePlan tile_plan(const ifa_seq_desc *sh, int n_seqs, int heads, int kv_heads, int dim, int vdim, int window, int keep_first, size_t ws_bytes)
+{
+    TilePlan t;
+    const int group = heads / kv_heads, NTK = (dim + 31) / 32, NTV = (vdim + 31) / 32;
+    t.hpw = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+    t.qw = 32 * (WT_WAVES / t.hpw);
+    t.blocks = 0;
+    std::vector<int> nbs;
+    size_t total = 0, most = 1;
+    for (int q = 0; q < n_seqs; q++) {
+        t.blocks += (size_t)seq_blocks(sh[q].pos0, sh[q].n, window, keep_first).count;
+        for (int at = 0; at < sh[q].n; at += t.qw) {
+            nbs.push_back(tile_blocks(sh[q].pos0 + at, std::min(t.qw, sh[q].n - at), window, keep_first).nb);
+            total += (size_t)nbs.back(); most = std::max(most, (size_t)nbs.back());
+        }
+    }
+    t.tiles = nbs.size();
+    t.op_bytes = t.blocks * (size_t)kv_heads * 3 * 64 * 16 * (size_t)(2 * NTK + 2 * NTV);
+    const size_t hx = (size_t)(heads / t.hpw), share = (size_t)WT_WAVES * 32 * ((size_t)vdim + 2) * 4;
+    size_t cb = std::max<size_t>({2, total * hx / WT_SLOTS, (most + WT_MAX_CHUNKS - 1) / WT_MAX_CHUNKS});
+    auto chunks = [&]() { return (most + cb - 1) / cb; };
+    auto groups = [&]() { size_t n = 0; for (int nb : nbs) n += ((size_t)nb + cb - 1) / cb; return n; };
+    while (chunks() > 1 && groups() * hx > WT_SLOTS) cb++;
+    while (chunks() > 1 && t.op_bytes + t.tiles * hx * chunks() * share > ws_bytes) cb = std::max(cb + 1, (most + chunks() - 2) / (chunks() - 1));
+    t.cb = (int)cb; t.chunks = (int)chunks(); t.groups = groups();
+    t.bytes = t.op_bytes + (t.chunks > 1 ? t.tiles * hx * (size_t)t.chunks * share : 0);
+    return t;
+}
+
 // ---- rotated queries and keys.  One workgroup per row, a wave per head at a time: RMS norm over the head's dim values with a weight
 // (norm_w bf16 [dim], null: none), then the first rot_dims dimensions turn in pairs (i, i + rot_dims / 2) -- pairing 1: (2i, 2i + 1) -- by the angle pos * freq[i]
 // (formed in double: at position 1000 one fp32 ulp of the angle is already 1e-4); the rest pass unchanged.  Query heads are rewritten in
@@ -516,7 +983,34 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
     P.sink = (const bf16_t *)sink_bf16; P.sink_fixed = sink_fixed; P.sink_score = sink_score;
     P.seqs = (const SeqDesc *)seqs_dev; P.row_seq = row_seq_dev; P.slot_base = (float *const *)slot_base_dev;
     P.k_off = k_off; P.v_off = v_off; P.out = (float *)out_f32; P.ldo = ldo; P.ws = nullptr; P.nsplit = 1;
-    // prompts: the tiled matrix-core kernel (heads of up to 128 dimensions, zero-padded to whole 32s); single tokens and other sizes: a workgroup per row
+    // prompts: the tiled matrix-core kernels (heads of up to 128 dimensions, zero-padded to whole 32s); single tokens and other sizes: a workgroup per row.
+    // With a workspace the bfloat16 form, from the smallest tiled step on (8 heads of 128: 16 rows 15.5 against 17.8 us, 256 rows 33 against 71, 64 rows behind 3000 keys 49 against 719)
+    if (rows >= (size_t)tile_min_rows && n_seqs > 0 && dim <= 128 && vdim <= 128 && ws_f32 && (uintptr_t)ws_f32 % 16 == 0) {
+        const TilePlan t = tile_plan((const ifa_seq_desc *)seqs_host, n_seqs, heads, kv_heads, dim, vdim, window, keep_first, ws_bytes);
+        IFA_REQUIRE(t.tiles < 65536 && t.groups < 65536 && t.blocks < 65536, "%s: %zu query tiles, %zu key blocks in one step", who, t.tiles, t.blocks);
+        if (t.bytes <= ws_bytes) {
+            const int NTK = (dim + 31) / 32, NTV = (vdim + 31) / 32;
+            TileArgs A;
+            A.n_seqs = n_seqs; A.hpw = t.hpw; A.cb = t.cb; A.tiles = (int)t.tiles; A.shares = t.op_bytes / 4;
+            P.ws = (float *)ws_f32; P.nsplit = t.chunks;
+            const bool vec = dim % 4 == 0 && vdim % 4 == 0 && ldq % 4 == 0 && ldo % 4 == 0 && (uintptr_t)q_f32 % 16 == 0 && (uintptr_t)out_f32 % 16 == 0;
+            const dim3 grid((unsigned)(heads / t.hpw), (unsigned)t.groups);
+#define IFA_WT(K, V) { const size_t smem_t = (size_t)2 * kBlockPieces<K, V> * 16 + WT_WAVES * 64 * 4; \
+                       const void *fn = vec ? (const void *)k_attn_tile<K, V, true> : (const void *)k_attn_tile<K, V, false>; \
+                       IFA_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_t)); \
+                       hipLaunchKernelGGL((k_attn_parts<K, V>), dim3((unsigned)kv_heads, (unsigned)t.blocks), dim3(256), 0, ifa_s(stream), P, n_seqs); \
+                       if (vec) hipLaunchKernelGGL((k_attn_tile<K, V, true>), grid, dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A); \
+                       else hipLaunchKernelGGL((k_attn_tile<K, V, false>), grid, dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A); }
+#define IFA_WTV(K) { if (NTV == 1) IFA_WT(K, 1) else if (NTV == 2) IFA_WT(K, 2) else if (NTV == 3) IFA_WT(K, 3) else IFA_WT(K, 4) }
+            if (NTK == 1) IFA_WTV(1) else if (NTK == 2) IFA_WTV(2) else if (NTK == 3) IFA_WTV(3) else IFA_WTV(4)
+#undef IFA_WTV
+#undef IFA_WT
+            if (t.chunks > 1) hipLaunchKernelGGL(k_attn_tile_combine, dim3(grid.x, (unsigned)t.tiles, WT_WAVES), dim3(256), 0, ifa_s(stream), P, A);
+            IFA_LAUNCH_CHECK();
+            return IFA_OK;
+        }
+    }
+    // prompts without a workspace (or with one that the operands do not fit)
     if (rows >= (size_t)tile_min_rows && n_seqs > 0 && dim <= 128 && vdim <= 128) {
         const ifa_seq_desc *sh = (const ifa_seq_desc *)seqs_host;
         size_t tiles = 0;
@@ -554,6 +1048,12 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
     if (nsplit > 1) hipLaunchKernelGGL(k_attn_window_combine, dim3((unsigned)rows, (unsigned)heads), dim3(64), 0, ifa_s(stream), P);
     IFA_LAUNCH_CHECK();
     return IFA_OK;
+}
+
+size_t ifa_attention_tile_workspace_bytes(const void *seqs_host, int n_seqs, int heads, int kv_heads, int dim, int vdim, int window, int keep_first)
+{
+    if (!seqs_host || n_seqs <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || dim <= 0 || vdim <= 0 || dim > 128 || vdim > 128) return 0;
+    return tile_plan((const ifa_seq_desc *)seqs_host, n_seqs, heads, kv_heads, dim, vdim, window > 0 ? window : (1 << 30), keep_first, (size_t)-1).bytes;
 }
 
 int ifa_attention_window_f32(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int norm_q, float eps, float scale, float softcap,

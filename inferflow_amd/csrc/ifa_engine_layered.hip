@@ -112,6 +112,7 @@ struct LayeredNet {
     int opt_fuse_post = 1;                 // POSTNORM layers, steps of at most 8 rows: norm-add, depth average, next input convolution and its tail in one launch
                                            // SANDWICH layers, every step size: the norm behind a sub-layer and the norm in front of the next one in one launch
                                            // PRENORM layers: the start of a looped pass inside the norm's launch; steps of at most 8 rows: the norm inside the router's launch
+    float *tile_ws = nullptr; size_t tile_ws_bytes = 0;      // the same for prompts through the tiled attention (grown by the steps that need more)
     float *attn_ws = nullptr; size_t attn_ws_bytes = 0;      // partial results of the windowed attention when a (row, head)'s keys are shared out
     bf16_t *a16 = nullptr, *h16 = nullptr; size_t a16_cap = 0, h16_cap = 0; int opt_a16_min = 17;          // activations of a prompt's product rounded to bfloat16; steps of at least this many rows (0: never)
     int opt_attn_tile_min = 16;            // steps of at least this many rows run the windowed attention through the tiled kernel
@@ -576,7 +577,7 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
     else {
         const int H = sp.a_heads, G = sp.a_kv_heads, D = sp.a_dim, DV = sp.a_vdim;
         const size_t OV = (size_t)H * DV;
-        const bool own = sp.a_kv_layer == 0;
+        const bool own = sp.a_kv_layer == 0, tile = T >= (size_t)n->opt_attn_tile_min;
         const LLayer &KV = own ? L : n->layers[(size_t)sp.a_kv_layer - 1];
         if ((rc = linear_in(m, L.w_in, NI, W, n->h, h16, T, L.b_in, n->proj, NI))) return rc;
         if ((rc = ifa_qk_rope_store_f32(n->proj + L.c_aq, NI, H, own ? n->proj + L.c_ak : nullptr, NI, own ? n->proj + L.c_av : nullptr, NI, G, D, DV,
@@ -584,7 +585,7 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
                                         slots, KV.o_k, KV.o_v, s))) return rc;
         if ((rc = ifa_attention_kv_f32(n->proj + L.c_aq, NI, H, G, D, DV, sp.a_scale, sp.a_window, sp.a_keep_first, sp.a_sink, sp.a_sink_score, n->seqs_dev,
                                        n->row_seq_dev, T, slots, KV.o_k, KV.o_v, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min,
-                                       c.max_ctx, n->attn_ws, n->attn_ws_bytes, s))) return rc;
+                                       c.max_ctx, tile ? n->tile_ws : n->attn_ws, tile ? n->tile_ws_bytes : n->attn_ws_bytes, s))) return rc;
         if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, OV, n->m1, OV, T, nullptr, nullptr, 1.0f, 0, n->m2, W))) return rc;
     }
     if ((rc = close_sub(n->m2, L.T(IFA_LT_NORM1B).data, any_ffn ? L.T(IFA_LT_NORM2).data : next_norm, in16 && !(any_ffn && moe)))) return rc;
@@ -650,17 +651,18 @@ int run_prenorm_layer(ifa_model *m, LLayer &L, size_t T, int nseq, int pass, boo
     if (sp.mixer == IFA_MIX_ROTARY) {
         const int H = sp.a_heads, G = sp.a_kv_heads, D = sp.a_dim, DV = sp.a_vdim;
         const size_t OV = (size_t)H * DV;
+        const bool tile = T >= (size_t)n->opt_attn_tile_min;
         if ((rc = ifa_qkv_rope_store_f32(n->proj + L.c_aq, NI, H, n->proj + L.c_ak, NI, n->proj + L.c_av, NI, G, D, DV, L.T(IFA_LT_A_Q_NORM).data, L.T(IFA_LT_A_K_NORM).data,
                                          c.eps, sp.a_rot_dims, L.freq, sp.a_vnorm, sp.a_vrot ? L.freq_v : nullptr, n->seqs_dev, n->row_seq_dev, T, slots, L.o_k + po,
                                          L.o_v + po, s))) return rc;
         if (sp.a_sink == 2)
             rc = ifa_attention_kv_sinks_f32(n->proj + L.c_aq, NI, H, G, D, DV, sp.a_scale, sp.a_window, sp.a_keep_first, L.T(IFA_LT_A_SINK).data, n->seqs_dev, n->row_seq_dev, T,
-                                            slots, L.o_k + po, L.o_v + po, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, c.max_ctx, n->attn_ws,
-                                            n->attn_ws_bytes, s);
+                                            slots, L.o_k + po, L.o_v + po, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, c.max_ctx, tile ? n->tile_ws : n->attn_ws,
+                                            tile ? n->tile_ws_bytes : n->attn_ws_bytes, s);
         else
             rc = ifa_attention_kv_f32(n->proj + L.c_aq, NI, H, G, D, DV, sp.a_scale, sp.a_window, sp.a_keep_first, sp.a_sink, sp.a_sink_score, n->seqs_dev, n->row_seq_dev, T,
-                                      slots, L.o_k + po, L.o_v + po, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, c.max_ctx, n->attn_ws,
-                                      n->attn_ws_bytes, s);
+                                      slots, L.o_k + po, L.o_v + po, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, c.max_ctx, tile ? n->tile_ws : n->attn_ws,
+                                      tile ? n->tile_ws_bytes : n->attn_ws_bytes, s);
         if (rc) return rc;
         // the sum over values that entered the cache turned by their positions is turned back by the row's own position
         if (sp.a_vrot && (rc = ifa_rotate_heads_f32(n->m1, OV, H, DV, DV & ~1, L.freq_v, -1.0f, n->seqs_dev, n->row_seq_dev, T, s))) return rc;
@@ -876,12 +878,13 @@ int run_layers(ifa_model *m, size_t T, int nseq)
         }
         if (sp.mixer == IFA_MIX_WINDOW_LINEAR) {
             const size_t AQ = (size_t)sp.a_heads * sp.a_dim, LV = (size_t)sp.l_heads * sp.l_vdim;
+            const bool tile = T >= (size_t)n->opt_attn_tile_min;
             // windowed attention: the values are the keys as projected; the cache's K rows hold the normed keys
             if ((rc = ifa_kv_store_f32(n->proj + L.c_ak, NI, n->proj + L.c_ak, NI, sp.a_kv_heads, sp.a_dim, 1, c.eps, n->seqs_dev, n->row_seq_dev, T, slots,
                                        L.o_k, L.o_v, s))) return rc;
             if ((rc = ifa_attention_window_f32(n->proj + L.c_aq, NI, sp.a_heads, sp.a_kv_heads, sp.a_dim, 1, c.eps, sp.a_scale, sp.a_softcap, sp.a_window,
                                                sp.a_keep_first, L.T(IFA_LT_A_REL).data, L.bucket_of, sp.a_buckets, L.T(IFA_LT_A_SINK).data, n->seqs_dev,
-                                               n->row_seq_dev, T, slots, L.o_k, L.o_v, n->m1, AQ, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, n->attn_ws, n->attn_ws_bytes, s))) return rc;
+                                               n->row_seq_dev, T, slots, L.o_k, L.o_v, n->m1, AQ, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, tile ? n->tile_ws : n->attn_ws, tile ? n->tile_ws_bytes : n->attn_ws_bytes, s))) return rc;
             if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, AQ, n->m1, AQ, T, nullptr, ls1, sp.a_out_scale, 1, n->x, W))) return rc;
             // decayed linear attention
             if ((rc = ifa_state_scan_f32(0, 0, n->proj + L.c_lq, NI, n->proj + L.c_lk, NI, n->proj + L.c_lv, NI, sp.l_heads, sp.l_heads, sp.l_dim, sp.l_vdim,
@@ -976,7 +979,7 @@ int lay_destroy(ifa_model *m)
     for (float *p : n->slot_ptr) lay_free(p);
     lay_free(n->slot_base_dev);
     if (n->tab_pin) (void)hipHostFree(n->tab_pin);
-    lay_free(n->attn_ws); lay_free(n->a16); lay_free(n->h16);
+    lay_free(n->attn_ws); lay_free(n->tile_ws); lay_free(n->a16); lay_free(n->h16);
     lay_free(n->tab_dev); lay_free(n->excl_dev); lay_free(n->next_dev); lay_free(n->ring_dev);
     float *bufs[] = {n->x, n->h, n->proj, n->m1, n->m2, n->m3, n->beta, n->decay, n->logits, n->taps};
     for (float *b : bufs) lay_free(b);
@@ -1448,6 +1451,21 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
                 IFA_HIP_CHECK(hipMalloc(&n->ssm_ws, need));
                 n->ssm_ws_bytes = need;
             }
+        }
+    }
+    if (T >= (size_t)std::max(n->opt_attn_tile_min, 1)) {
+        size_t need = 0;
+        for (const LLayer &L : n->layers) {
+            const ifa_layer_spec &sp = L.spec;
+            if (sp.mixer == IFA_MIX_WINDOW_LINEAR || sp.mixer == IFA_MIX_ROTARY)
+                need = std::max(need, ifa_attention_tile_workspace_bytes(n->seqs_host.data(), nseq, sp.a_heads, sp.a_kv_heads, sp.a_dim,
+                                                                         sp.mixer == IFA_MIX_ROTARY ? sp.a_vdim : sp.a_dim, sp.a_window, sp.a_keep_first));
+        }
+        if (need > n->tile_ws_bytes) {
+            IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
+            lay_free(n->tile_ws); n->tile_ws = nullptr; n->tile_ws_bytes = 0;
+            IFA_HIP_CHECK(hipMalloc((void **)&n->tile_ws, need));
+            n->tile_ws_bytes = need;
         }
     }
     if ((rc = run_layers(m, T, nseq))) return rc;

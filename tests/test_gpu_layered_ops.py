@@ -279,6 +279,110 @@ def test_windowed_attention_tiles_over_several_sequences():
             r += n; at[s_] += n
 
 
+def dense_attention_64(q, k, v, pos0, heads, kv_heads, scale, window, keep, cap=0.0, rel=None, bucket_of=None, sink=None, norm_eps=None):
+    """rows at positions pos0 .. over all keys, float64; q [n, heads, d], k [T, kv_heads, d], v [T, kv_heads, dv]"""
+    n, T = q.shape[0], k.shape[0]
+    i, j = torch.arange(pos0, pos0 + n)[:, None], torch.arange(T)[None, :]
+    see = (j <= i) & ((i - j < window) | (j < keep))
+    if norm_eps is not None:
+        q = orc.rms_unit(q, norm_eps)
+    out = []
+    for h in range(heads):
+        g = h // (heads // kv_heads)
+        sc = q[:, h] @ k[:, g].T * scale
+        if cap:
+            sc = cap * torch.tanh(sc / cap)
+        if rel is not None:
+            sc = sc + rel[:, h][bucket_of[(i - j).clamp(min=0)]]
+        sc = sc.masked_fill(~see, -np.inf)
+        m = sc.max(-1, keepdim=True).values
+        e = torch.exp(sc - m)
+        den = e.sum(-1, keepdim=True) + (torch.exp(sink[h] - m) if sink is not None else 0.0)
+        out.append(e / den @ v[:, g])
+    return torch.stack(out, 1).reshape(n, -1)
+
+
+# edges of the tiled kernel with a workspace: query tiles of 64 / 128 / 256 (groups of 4, 2, 1 heads), key blocks of 32, windows and kept tokens that begin and end
+# inside blocks and meet in one, one chunk and many (short and long key ranges beside each other), continued sequences, head sizes that are not whole 32s or 4s
+TILE_WS = [(4, 1, 128, 128, 1 << 30, 0, [(0, 16)], 1.0), (8, 2, 128, 128, 1 << 30, 0, [(0, 65)], 1.0), (8, 2, 64, 128, 1 << 30, 0, [(0, 700), (0, 3), (610, 90)], 1.0),
+           (4, 2, 96, 32, 40, 0, [(0, 257)], 1.0), (3, 3, 32, 96, 33, 31, [(0, 300), (500, 33)], 1.0), (6, 2, 128, 64, 64, 33, [(95, 70), (0, 64)], 1.0),
+           (4, 1, 36, 20, 100, 70, [(0, 310)], 1.0), (2, 1, 127, 101, 32, 0, [(0, 129), (31, 32)], 1.0), (8, 2, 128, 128, 1024, 4, [(0, 1300)], 1.0),
+           (5, 1, 5, 3, 17, 300, [(200, 150)], 1.0), (8, 2, 128, 128, 1 << 30, 0, [(0, 200)], 1e4), (8, 2, 128, 128, 1 << 30, 0, [(0, 200)], 1e-7)]
+
+
+@pytest.mark.parametrize("form", ["plain", "capped"])
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,window,keep,seqs,size", TILE_WS)
+def test_tiled_attention_with_a_workspace_against_64_bits_and_the_fp32_tiles(heads, kv_heads, dim, vdim, window, keep, seqs, size, form):
+    """Three bfloat16 parts per operand leave the results no further from 64 bits than fp32 operands do.  Bound: dim + 2 fp32 roundings of a score, |scores| below
+    ~6, weights that sum to one -> 1e-6 of the largest value; measured 2e-7 .. 5e-7 on either side."""
+    if form == "capped":
+        vdim = dim
+    rng = np.random.default_rng(heads * 100 + dim + window % 1000)
+    ctx = max(a + n for a, n in seqs) + 3
+    k_off, v_off = 4, 4 + (ctx * kv_heads * dim + 3) // 4 * 4
+    sl = Slots(len(seqs), v_off + ctx * kv_heads * vdim)
+    ks, vs = [], []
+    for s_, (pos0, n) in enumerate(seqs):
+        k, v = rng.standard_normal((pos0 + n, kv_heads, dim)).astype(np.float32), (size * rng.standard_normal((pos0 + n, kv_heads, vdim))).astype(np.float32)
+        if form == "plain":
+            k *= np.float32(size)
+        sl.mem[s_][k_off:k_off + k.size] = dev32(k.reshape(-1)); sl.mem[s_][v_off:v_off + v.size] = dev32(v.reshape(-1))
+        ks.append(k); vs.append(v)
+    host, r = [], 0
+    for s_, (pos0, n) in enumerate(seqs):
+        host += [r, n, pos0, s_]; r += n
+    host = (C.c_int * len(host))(*host)
+    d, rs, T = seq_tables([(n, pos0, s_) for s_, (pos0, n) in enumerate(seqs)])
+    q = rng.standard_normal((T, heads * dim)).astype(np.float32)
+    rel, sink, cap = orc.bf16_round(rng.standard_normal((6, heads))), orc.bf16_round(rng.standard_normal(heads)), 5.0
+    bucket = rng.integers(0, 6, ctx)
+    scale = (1.0 if form == "capped" else 1.0 / size) * dim ** -0.5
+    nb = capi().ifa_attention_tile_workspace_bytes(host, len(seqs), heads, kv_heads, dim, vdim, window, keep)
+    assert nb > 0
+    got = []
+    for ws_bytes in (nb, 0):
+        ws = torch.full((nb // 4,), float("nan"), dtype=torch.float32, device="cuda")
+        out = torch.full((T, heads * vdim + 4), float("nan"), dtype=torch.float32, device="cuda")
+        a = (p(d), p(rs), T, p(sl.table), k_off, v_off, p(out), heads * vdim + 4, host, len(seqs), 16)
+        w = (p(ws) if ws_bytes else None, ws_bytes, None)
+        if form == "capped":
+            ia.check(capi().ifa_attention_window_f32(p(dev32(q)), heads * dim, heads, kv_heads, dim, 1, 1e-6, scale, cap, window, keep, p(devbf(rel)), p(devi(bucket)), 6,
+                                                     p(devbf(sink)), *a, *w))
+        else:
+            ia.check(capi().ifa_attention_kv_f32(p(dev32(q)), heads * dim, heads, kv_heads, dim, vdim, scale, 0 if window == 1 << 30 else window, keep, 0, 0.0, *a, 0, *w))
+        sync()
+        got.append(out.cpu().numpy()[:, :heads * vdim])
+    r = 0
+    for s_, (pos0, n) in enumerate(seqs):
+        extra = dict(cap=cap, rel=orc.t64(rel), bucket_of=torch.from_numpy(bucket), sink=orc.t64(sink), norm_eps=1e-6) if form == "capped" else {}
+        want = dense_attention_64(orc.t64(q[r:r + n]).reshape(n, heads, dim), orc.t64(ks[s_]), orc.t64(vs[s_]), pos0, heads, kv_heads, scale, window, keep, **extra).numpy()
+        off = [np.abs(g[r:r + n] - want).max() / np.abs(want).max() for g in got]
+        print(form, heads, dim, (pos0, n), "parts %.2g fp32 %.2g" % tuple(off), "rms %.3g %.3g" % tuple(np.linalg.norm(g[r:r + n] - want) / np.linalg.norm(want) for g in got))
+        assert off[0] < 1e-6 and np.linalg.norm(got[0][r:r + n] - want) < 1.1 * np.linalg.norm(got[1][r:r + n] - want) + 2e-8 * np.linalg.norm(want), (pos0, n)
+        r += n
+
+
+def test_tiled_attention_takes_fewer_chunks_where_the_workspace_is_small():
+    """2000 keys: with all the workspace many chunks per tile, with just the operands' bytes and one share more none; both the same sums in another grouping"""
+    rng = np.random.default_rng(3)
+    heads, kv_heads, dim, T = 4, 1, 32, 2000
+    sl = Slots(1, 2 * T * dim)
+    sl.mem[0].copy_(dev32(rng.standard_normal(2 * T * dim)))
+    host = (C.c_int * 4)(0, T, 0, 0)
+    d, rs, _ = seq_tables([(T, 0, 0)])
+    q = dev32(rng.standard_normal((T, heads * dim)))
+    nb = capi().ifa_attention_tile_workspace_bytes(host, 1, heads, kv_heads, dim, dim, 0, 0)
+    ops = (T + 31) // 32 * 3 * 64 * 16 * 4
+    res = []
+    for ws_bytes in (nb, nb - 4, ops + 64, ops - 4):          # (the last: the operands do not fit, the fp32 tiles)
+        ws, out = torch.empty(nb, dtype=torch.uint8, device="cuda"), torch.empty((T, heads * dim), dtype=torch.float32, device="cuda")
+        ia.check(capi().ifa_attention_kv_f32(p(q), heads * dim, heads, kv_heads, dim, dim, dim ** -0.5, 0, 0, 0, 0.0, p(d), p(rs), T, p(sl.table), 0, T * dim, p(out), heads * dim,
+                                             host, 1, 16, 0, p(ws), ws_bytes, None))
+        sync(); res.append(out.cpu().numpy())
+    for r in res[1:]:
+        assert np.abs(r - res[0]).max() < 2e-6 * np.abs(res[0]).max()
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 8])
 def test_row_products_with_the_norm_or_the_gated_gelu_folded_in(T):
     rng = np.random.default_rng(40 + T)
