@@ -514,6 +514,14 @@ int ifa_delta_gates_f32(const void *b_f32, size_t ldb, const void *a_f32, size_t
 int ifa_state_scan_f32(int kind, int in_act, const void *q_f32, size_t ldq, const void *k_f32, size_t ldk, const void *v_f32, size_t ldv, int heads,
                        int qk_heads, int dk, int dv, const void *decay_head_f32, const void *decay_row_f32, const void *beta_row_f32,
                        const void *seqs_dev, int n_seqs, void *const *slot_base_dev, size_t state_off, void *out_f32, size_t ldo, ifa_stream stream);
+/* the same recurrences over prompts, 64 tokens at a time as products on the fp32 matrix cores (csrc/ifa_chunkscan.hip); needs the sequences on the host too and a
+ * workspace: ifa_state_chunked_workspace_bytes(kind, chunks of the step, ...), chunks = sum over the sequences of ceil(n / 64).  Sizes and rows that it takes:
+ * ifa_state_chunked_fits (keys of 64 or 128, values in whole 32s, q / k / output rows of whole aligned 16 bytes); decay_row in [0, 1]. */
+int ifa_state_chunked_fits(int kind, const void *q_f32, size_t ldq, const void *k_f32, size_t ldk, const void *v_f32, size_t ldv, int dk, int dv, const void *out_f32, size_t ldo);
+size_t ifa_state_chunked_workspace_bytes(int kind, size_t chunks, int heads, int dk, int dv);
+int ifa_state_chunked_f32(int kind, const void *q_f32, size_t ldq, const void *k_f32, size_t ldk, const void *v_f32, size_t ldv, int heads, int qk_heads, int dk, int dv,
+                          const void *decay_head_f32, const void *decay_row_f32, const void *beta_row_f32, const void *seqs_dev, const void *seqs_host, int n_seqs,
+                          void *const *slot_base_dev, size_t state_off, void *ws, size_t ws_bytes, void *out_f32, size_t ldo, ifa_stream stream);
 /* y = o / sqrt(mean_group(o^2) + eps) * w[c % wlen] * act(gate); gate_act 0 sigmoid, 1 silu; groups of `group` channels; y may be o */
 int ifa_gated_groupnorm_f32(const void *o_f32, size_t ldo, size_t rows, int channels, int group, const void *w_bf16, int wlen, const void *gate_f32,
                             size_t ldg, int gate_act, float eps, void *y_f32, size_t ldy, ifa_stream stream);

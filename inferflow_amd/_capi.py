@@ -207,6 +207,9 @@ SIGNATURES = {
     "ifa_ssm_gates_ring_f32": (_i, [_vp, _sz, _i, _sz, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _vp, _i, _vp, _sz, _vp]),
     "ifa_ssm_step_f32": (_i, [_vp, _sz, _vp, _sz, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _sz, _sz, _vp, _sz, _vp]),
     "ifa_attention_tile_workspace_bytes": (_sz, [_vp, _i, _i, _i, _i, _i, _i, _i]),
+    "ifa_state_chunked_fits": (_i, [_i, _vp, _sz, _vp, _sz, _vp, _sz, _i, _i, _vp, _sz]),
+    "ifa_state_chunked_workspace_bytes": (_sz, [_i, _sz, _i, _i, _i]),
+    "ifa_state_chunked_f32": (_i, [_i, _vp, _sz, _vp, _sz, _vp, _sz, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp, _sz, _vp, _sz, _vp, _sz, _vp]),
     "ifa_ssm_chunked_workspace_bytes": (_sz, [_sz, _i, _i, _i, _i]),
     "ifa_ssm_chunked_f32": (_i, [_vp, _sz, _vp, _sz, _vp, _sz, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp, _sz, _vp, _sz, _vp, _sz, _vp]),
     "ifa_moe_experts_routed_rows_f32": (_i, [_i, _i, _f, _f, _vp, _sz, _vp, _i, _f, _vp, _sz, _sz, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _sz, _i, _vp]),

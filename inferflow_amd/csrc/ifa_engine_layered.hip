@@ -124,6 +124,10 @@ struct LayeredNet {
     bool any_depth_avg = false, any_latent = false, any_moe = false, latent_tile_ok = true, step_expand = false;
     std::vector<int> ctx0_host; size_t step_ctx_rows = 0;
     // state-space layers: steps whose longest sequence brings at least opt_ssm_chunk_min tokens run in chunks (ssm_chunks > 0), their workspace
+    // the recurrences of WINDOW_LINEAR and GATED_DELTA layers: steps whose longest sequence brings at least this many tokens run in chunks of 64 (scan_chunks > 0).
+    // Measured where the two meet (whole Gelarax prompts, chunks / token by token): 96 tokens 1494 / 1467 and 2198 / 2163 us (widths 1024 / 2048), 128 tokens
+    // 1520 / 1560 and 2219 / 2269
+    int opt_scan_chunk_min = 112; size_t scan_chunks = 0, scan_ws_bytes = 0; void *scan_ws = nullptr;
     bool any_ssm = false; int opt_ssm_chunk_min = 48; size_t ssm_chunks = 0, ssm_ws_bytes = 0; void *ssm_ws = nullptr;
     hipGraphExec_t step_exec = nullptr; hipGraph_t step_graph = nullptr; int step_slot = -1;
 };
@@ -797,6 +801,19 @@ int run_streams_layer(ifa_model *m, LLayer &L, size_t T, int nseq, int pass, LLa
     return streams_step(m, T, false, n->m1, &L, 2, next_in, next_norm);
 }
 
+// a recurrence of the step's rows: prompts in chunks of 64 tokens where the sizes allow it, else token by token
+int run_state(ifa_model *m, int kind, const float *q, size_t ldq, const float *k, size_t ldk, const float *v, size_t ldv, int heads, int qk_heads, int dk, int dv,
+              const void *decay_head, const void *decay_row, const void *beta_row, int nseq, size_t state_off, float *out, size_t ldo)
+{
+    LayeredNet *n = m->lay;
+    ifa_stream s = (ifa_stream)m->stream;
+    void *const *slots = (void *const *)n->slot_base_dev;
+    if (n->scan_chunks && ifa_state_chunked_fits(kind, q, ldq, k, ldk, v, ldv, dk, dv, out, ldo))
+        return ifa_state_chunked_f32(kind, q, ldq, k, ldk, v, ldv, heads, qk_heads, dk, dv, decay_head, decay_row, beta_row, n->seqs_dev, n->seqs_host.data(), nseq, slots,
+                                     state_off, n->scan_ws, n->scan_ws_bytes, out, ldo, s);
+    return ifa_state_scan_f32(kind, 0, q, ldq, k, ldk, v, ldv, heads, qk_heads, dk, dv, decay_head, decay_row, beta_row, n->seqs_dev, nseq, slots, state_off, out, ldo, s);
+}
+
 // the layers of one step over T rows / nseq sequences whose tables are already on the device; leaves the residual in n->x
 int run_layers(ifa_model *m, size_t T, int nseq)
 {
@@ -887,8 +904,8 @@ int run_layers(ifa_model *m, size_t T, int nseq)
                                                n->row_seq_dev, T, slots, L.o_k, L.o_v, n->m1, AQ, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, tile ? n->tile_ws : n->attn_ws, tile ? n->tile_ws_bytes : n->attn_ws_bytes, s))) return rc;
             if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, AQ, n->m1, AQ, T, nullptr, ls1, sp.a_out_scale, 1, n->x, W))) return rc;
             // decayed linear attention
-            if ((rc = ifa_state_scan_f32(0, 0, n->proj + L.c_lq, NI, n->proj + L.c_lk, NI, n->proj + L.c_lv, NI, sp.l_heads, sp.l_heads, sp.l_dim, sp.l_vdim,
-                                         L.T(IFA_LT_L_DECAY).data, nullptr, nullptr, n->seqs_dev, nseq, slots, L.o_lin, n->m2, LV, s))) return rc;
+            if ((rc = run_state(m, 0, n->proj + L.c_lq, NI, n->proj + L.c_lk, NI, n->proj + L.c_lv, NI, sp.l_heads, sp.l_heads, sp.l_dim, sp.l_vdim,
+                                L.T(IFA_LT_L_DECAY).data, nullptr, nullptr, nseq, L.o_lin, n->m2, LV))) return rc;
             if ((rc = ifa_gated_groupnorm_f32(n->m2, LV, T, (int)LV, (int)LV, L.T(IFA_LT_L_NORM).data, (int)LV, n->proj + L.c_lg, NI, 0, c.eps, n->m2, LV, s))) return rc;
             if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_L_O).data, W, LV, n->m2, LV, T, nullptr, ls1, sp.l_out_scale, 1, n->x, W))) return rc;
         } else {
@@ -898,8 +915,8 @@ int run_layers(ifa_model *m, size_t T, int nseq)
             if ((rc = ifa_shortconv_tail_f32(n->proj + L.c_dq, NI, (int)C, sp.d_conv, n->seqs_dev, nseq, slots, L.o_conv, s))) return rc;
             if ((rc = ifa_delta_gates_f32(n->proj + L.c_db, NI, n->proj + L.c_da, NI, sp.d_heads, T, L.T(IFA_LT_D_ALOG).data, L.T(IFA_LT_D_DTBIAS).data,
                                           n->beta, n->decay, s))) return rc;
-            if ((rc = ifa_state_scan_f32(1, 0, n->m1, C, n->m1 + QK, C, n->m1 + 2 * QK, C, sp.d_heads, sp.d_kv_heads, sp.d_dim, sp.d_vdim, nullptr, n->decay,
-                                         n->beta, n->seqs_dev, nseq, slots, L.o_rec, n->m2, DV, s))) return rc;
+            if ((rc = run_state(m, 1, n->m1, C, n->m1 + QK, C, n->m1 + 2 * QK, C, sp.d_heads, sp.d_kv_heads, sp.d_dim, sp.d_vdim, nullptr, n->decay,
+                                n->beta, nseq, L.o_rec, n->m2, DV))) return rc;
             if ((rc = ifa_gated_groupnorm_f32(n->m2, DV, T, (int)DV, sp.d_vdim, L.T(IFA_LT_D_NORM).data, sp.d_vdim, n->proj + L.c_dg, NI, 1, c.eps, n->m2, DV, s))) return rc;
             if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_D_O).data, W, DV, n->m2, DV, T, nullptr, ls1, 1.0f, 1, n->x, W))) return rc;
         }
@@ -979,7 +996,7 @@ int lay_destroy(ifa_model *m)
     for (float *p : n->slot_ptr) lay_free(p);
     lay_free(n->slot_base_dev);
     if (n->tab_pin) (void)hipHostFree(n->tab_pin);
-    lay_free(n->attn_ws); lay_free(n->tile_ws); lay_free(n->a16); lay_free(n->h16);
+    lay_free(n->attn_ws); lay_free(n->tile_ws); lay_free(n->scan_ws); lay_free(n->a16); lay_free(n->h16);
     lay_free(n->tab_dev); lay_free(n->excl_dev); lay_free(n->next_dev); lay_free(n->ring_dev);
     float *bufs[] = {n->x, n->h, n->proj, n->m1, n->m2, n->m3, n->beta, n->decay, n->logits, n->taps};
     for (float *b : bufs) lay_free(b);
@@ -1318,12 +1335,13 @@ int lay_set_option(ifa_model *m, const char *name, int value)
     if (!strcmp(name, "tap_layers")) { n->opt_tap_layers = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "fuse_rows")) { n->opt_fuse_rows = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "fuse_post")) { n->opt_fuse_post = value; drop_step_graph(n); return IFA_OK; }
+    if (!strcmp(name, "scan_chunk_min")) { n->opt_scan_chunk_min = value; return IFA_OK; }
     if (!strcmp(name, "ssm_chunk_min")) { n->opt_ssm_chunk_min = value; return IFA_OK; }
     if (!strcmp(name, "a16_min")) { n->opt_a16_min = value; return IFA_OK; }
     if (!strcmp(name, "attn_tile_min")) { n->opt_attn_tile_min = value; return IFA_OK; }
     if (!strcmp(name, "graph")) { n->opt_graph = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "ops32")) { IFA_HIP_CHECK(hipStreamSynchronize(m->stream)); n->cfg.ops32 = value ? 1 : 0; drop_step_graph(n); return IFA_OK; }
-    return ifa_fail(IFA_ERR_ARG, "ifa_model_set_option: unknown option '%s' (layer-list model: tap_layers, graph, ops32, attn_tile_min, a16_min, fuse_rows, fuse_post, ssm_chunk_min)", name);
+    return ifa_fail(IFA_ERR_ARG, "ifa_model_set_option: unknown option '%s' (layer-list model: tap_layers, graph, ops32, attn_tile_min, a16_min, fuse_rows, fuse_post, ssm_chunk_min, scan_chunk_min)", name);
 }
 
 int lay_set_excluded(ifa_model *m, const int *ids_host, int cnt)
@@ -1437,6 +1455,24 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
         IFA_HIP_CHECK(hipMalloc((void **)&n->vx, n->step_ctx_rows * n->vx_max * 4));
         n->expand_rows = n->step_ctx_rows;
     }
+    n->scan_chunks = 0;
+    {
+        int longest = 0; size_t chunks = 0, need = 0;
+        for (int q = 0; q < nseq; q++) { longest = std::max(longest, lens[q]); chunks += ((size_t)lens[q] + 63) / 64; }
+        if (longest >= std::max(n->opt_scan_chunk_min, 2))
+            for (const LLayer &L : n->layers) {
+                const ifa_layer_spec &sp = L.spec;
+                if (sp.mixer == IFA_MIX_WINDOW_LINEAR) need = std::max(need, ifa_state_chunked_workspace_bytes(0, chunks, sp.l_heads, sp.l_dim, sp.l_vdim));
+                else if (sp.mixer == IFA_MIX_GATED_DELTA) need = std::max(need, ifa_state_chunked_workspace_bytes(1, chunks, sp.d_heads, sp.d_dim, sp.d_vdim));
+            }
+        if (need) n->scan_chunks = chunks;
+        if (need > n->scan_ws_bytes) {
+            IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
+            lay_free(n->scan_ws); n->scan_ws = nullptr; n->scan_ws_bytes = 0;
+            IFA_HIP_CHECK(hipMalloc(&n->scan_ws, need));
+            n->scan_ws_bytes = need;
+        }
+    }
     n->ssm_chunks = 0;
     if (n->any_ssm) {
         int longest = 0; size_t chunks = 0, need = 0;
@@ -1534,7 +1570,7 @@ int lay_decode(ifa_model *m, int first_token, int start_pos, int n_steps, int *o
     if ((rc = check_span(m, n_steps, start_pos, nullptr)) || (rc = ensure_slot(m, n->cur_slot)) || (rc = ensure_rows(m, 1, 1)) || (rc = ensure_logits(m, 1))) return rc;
     if (n->opt_graph && !n->opt_tap_layers && !n->step_exec) {      // (the slot is read from the device tables: one capture serves every slot)
         drop_step_graph(n);
-        n->step_expand = false;
+        n->step_expand = false; n->scan_chunks = 0;
         n->seqs_host.assign(1, ifa_seq_desc{0, 1, start_pos, n->cur_slot});      // (the launches are shaped by it: one sequence, one row)
         IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
         IFA_HIP_CHECK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
@@ -1553,7 +1589,7 @@ int lay_decode(ifa_model *m, int first_token, int start_pos, int n_steps, int *o
     std::vector<int> tok(1, first_token), pos(1, start_pos), rs(1, 0);
     std::vector<ifa_seq_desc> sq(1); sq[0] = ifa_seq_desc{0, 1, start_pos, n->cur_slot};
     if ((rc = upload_tables(m, tok, pos, rs, sq))) return rc;
-    n->step_expand = false;
+    n->step_expand = false; n->scan_chunks = 0;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (elapsed_ms) { IFA_HIP_CHECK(hipEventCreate(&e0)); IFA_HIP_CHECK(hipEventCreate(&e1)); IFA_HIP_CHECK(hipEventRecord(e0, m->stream)); }
     for (int st = 0; st < n_steps; st++) {

@@ -302,6 +302,68 @@ def dense_attention_64(q, k, v, pos0, heads, kv_heads, scale, window, keep, cap=
     return torch.stack(out, 1).reshape(n, -1)
 
 
+# chunks of 64: one token more or less than a chunk, several chunks, sequences that end inside one, continued states, shared q / k heads, one value tile and odd counts of them
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("heads,qk_heads,dk,dv,steps", [(2, 2, 64, 128, [[(0, 1)], [(0, 63)], [(0, 64)]]), (4, 2, 128, 32, [[(0, 65), (1, 200)], [(1, 64), (0, 1)]]),
+                                                        (3, 1, 64, 96, [[(0, 130), (1, 3), (2, 64)], [(2, 66)]]), (2, 1, 128, 160, [[(0, 257)], [(0, 31)]])])
+def test_state_recurrences_in_chunks(kind, heads, qk_heads, dk, dv, steps):
+    """Against the float64 recurrence, beside the token-by-token kernel on the same states: fp32 sums of up to 64 + dk terms in another grouping (bound 1e-5 of the
+    largest value; measured 1e-7 .. 1e-6 on either side).  One head's decays reach 0.02 per token, another's are 1."""
+    rng = np.random.default_rng(heads * 10 + dk + kind)
+    total = {s_: sum(n for st in steps for q_, n in st if q_ == s_) for s_ in range(3)}
+    unit = lambda a: (a / np.linalg.norm(a.reshape(a.shape[0], -1, dk), axis=-1).repeat(dk, -1).reshape(a.shape)).astype(np.float32)
+    data = {}
+    for s_, L in total.items():
+        q, k = rng.standard_normal((L, qk_heads * dk)).astype(np.float32), rng.standard_normal((L, qk_heads * dk)).astype(np.float32)
+        v = rng.standard_normal((L, heads * dv)).astype(np.float32)
+        g, b = np.exp(-rng.uniform(0, 0.3, (L, heads))).astype(np.float32), rng.uniform(0.05, 1, (L, heads)).astype(np.float32)
+        if L:
+            g[:, 0] = np.exp(-rng.uniform(0, 4, L)); g[:, -1] = 1.0
+        data[s_] = (unit(q) if kind else q, unit(k) if kind else 0.3 * k, v, g, b) if L else None
+    dec = np.array([0.02, 1.0, 0.97, 0.999][:heads], np.float32)
+    want = {}
+    for s_, d in data.items():
+        if d is None:
+            continue
+        q, k, v, g, b = (orc.t64(a) for a in d)
+        if kind:
+            want[s_] = orc.gated_delta_rule(q, k, v, b, g, heads, qk_heads, dk, dv).numpy()
+        else:
+            rep = lambda a: a.reshape(-1, qk_heads, dk).repeat_interleave(heads // qk_heads, 1).reshape(a.shape[0], -1)
+            want[s_] = orc.decayed_linear_attention(rep(q), rep(k), v, heads, dk, dv, orc.t64(dec)).numpy()
+    off = 8
+    slots = [Slots(3, off + heads * dk * dv + 4) for _ in range(2)]
+    at = {0: 0, 1: 0, 2: 0}
+    for st in steps:
+        seqs = [(n, at[s_], s_) for s_, n in st]
+        d, rs, T = seq_tables(seqs)
+        host, r = [], 0
+        for n, pos0, slot in seqs:
+            host += [r, n, pos0, slot]; r += n
+        host = (C.c_int * len(host))(*host)
+        q, k, v, g, b = (dev32(np.concatenate([data[s_][i][at[s_]:at[s_] + n] for s_, n in st], 0)) for i in range(5))
+        chunks = sum((n + 63) // 64 for _, n in st)
+        nb = capi().ifa_state_chunked_workspace_bytes(kind, chunks, heads, dk, dv)
+        ws = torch.full((nb // 4,), float("nan"), dtype=torch.float32, device="cuda")
+        outs = [torch.full((T, heads * dv + 4), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2)]
+        gates = (p(dev32(dec)), None, None) if kind == 0 else (None, p(g), p(b))
+        assert capi().ifa_state_chunked_fits(kind, p(q), qk_heads * dk, p(k), qk_heads * dk, p(v), heads * dv, dk, dv, p(outs[0]), heads * dv + 4)
+        ia.check(capi().ifa_state_chunked_f32(kind, p(q), qk_heads * dk, p(k), qk_heads * dk, p(v), heads * dv, heads, qk_heads, dk, dv, *gates, p(d), host, len(st),
+                                              p(slots[0].table), off, p(ws), nb, p(outs[0]), heads * dv + 4, None))
+        ia.check(capi().ifa_state_scan_f32(kind, 0, p(q), qk_heads * dk, p(k), qk_heads * dk, p(v), heads * dv, heads, qk_heads, dk, dv, *gates, p(d), len(st),
+                                           p(slots[1].table), off, p(outs[1]), heads * dv + 4, None))
+        sync()
+        got, r = [o.cpu().numpy()[:, :heads * dv] for o in outs], 0
+        for s_, n in st:
+            w = want[s_][at[s_]:at[s_] + n]
+            err = [np.abs(x[r:r + n] - w).max() / np.abs(w).max() for x in got]
+            rel = [np.linalg.norm(x[r:r + n] - w) / np.linalg.norm(w) for x in got]
+            print("state", kind, heads, dk, dv, n, "chunks %.2g tokens %.2g" % tuple(err), "rms %.2g %.2g" % tuple(rel))
+            assert err[0] < 1e-5 and rel[0] < 1.5 * rel[1] + 1e-7, (s_, at[s_], n)
+            r += n; at[s_] += n
+        assert (slots[0].mem[st[0][0]][off + heads * dk * dv:] == 1e9).all() and (slots[0].mem[st[0][0]][:off] == 1e9).all()
+
+
 # edges of the tiled kernel with a workspace: query tiles of 64 / 128 / 256 (groups of 4, 2, 1 heads), key blocks of 32, windows and kept tokens that begin and end
 # inside blocks and meet in one, one chunk and many (short and long key ranges beside each other), continued sequences, head sizes that are not whole 32s or 4s
 TILE_WS = [(4, 1, 128, 128, 1 << 30, 0, [(0, 16)], 1.0), (8, 2, 128, 128, 1 << 30, 0, [(0, 65)], 1.0), (8, 2, 64, 128, 1 << 30, 0, [(0, 700), (0, 3), (610, 90)], 1.0),
