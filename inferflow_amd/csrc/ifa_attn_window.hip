@@ -10,10 +10,12 @@
 // rotation are applied by k_qk_rope_store before the keys enter the cache, the values have a size of their own, the sink has a fixed
 // score and the window may be unlimited; a layer may read the cache rows that an earlier layer has written.
 #include <algorithm>
+#include <cstring>
 #include <vector>
 #include "ifa_host.h"
 #include "ifa_f32_common.h"
 #include "inferflow_amd.h"
+#include "ifa_rows_fused.h"
 
 using namespace ifa32;
 
@@ -40,6 +42,11 @@ __global__ void __launch_bounds__(256) k_kv_store_f32(const float *__restrict__ 
     }
 }
 
+typedef float f32x4w __attribute__((ext_vector_type(4)));
+// device memory, said so: loads through a pointer that came out of memory would be FLAT, and those hold up the waits for LDS
+typedef const __attribute__((address_space(1))) float gfloat;
+typedef const __attribute__((address_space(1))) f32x4w gf32x4;
+
 struct WinAttnArgs {
     const float *q; size_t ldq;
     int heads, kv_heads, dim, vdim;
@@ -61,15 +68,18 @@ constexpr int WA_DPL_MAX = 16;    // dim <= 64 * DPL: a lane holds DPL value col
 // grid (rows, heads, splits), four waves: the visible keys (kept first tokens, then the window) are walked in chunks of 16, four
 // lanes per key for the score, one value column per lane for the weighted sum; chunks go round-robin to the waves, each
 // with its own running maximum / sum / accumulator, merged through LDS at the end together with the sink.
-template <int WA_DPL>
-__global__ void __launch_bounds__(256) k_attn_window(WinAttnArgs P)
+// FRESH (steps of one row): the row's own key and value are not in the cache yet.  They are read as projected (F.k, F.v; norm_k: the key by its root mean
+// square) and the first workgroup of their head leaves them there.
+struct FreshRow { const float *k, *v; int norm_k; };
+
+template <int WA_DPL, bool FRESH>
+__device__ __forceinline__ void attn_row(const WinAttnArgs &P, const FreshRow &F, const int t, const int h, const int split, float *sm)
 {
-    extern __shared__ float sm[];
     float *qn = sm;                                   // [dim]
     float *wm = sm + P.dim, *wl = wm + 4;             // per wave: maximum, sum
     float *wacc = wl + 4;                             // [4][vdim]
     __shared__ float red[17];
-    const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int dim = P.dim, vdim = P.vdim, g = h / (P.heads / P.kv_heads);
     const SeqDesc sd = P.seqs[P.row_seq[t]];
     const int i = sd.pos0 + t - sd.row0;
@@ -81,30 +91,47 @@ __global__ void __launch_bounds__(256) k_attn_window(WinAttnArgs P)
         for (int c = tid; c < dim; c += blockDim.x) qn[c] = qr[c] * r;
     }
     __syncthreads();
+    gfloat *own_k = nullptr, *own_v = nullptr;
+    float own_r = 1.0f;
+    if constexpr (FRESH) {
+        own_k = (gfloat *)F.k + (size_t)g * dim; own_v = (gfloat *)F.v + (size_t)g * vdim;
+        if (F.norm_k) {
+            float s = 0.0f;
+            for (int c = tid; c < dim; c += blockDim.x) s = fmaf(own_k[c], own_k[c], s);
+            own_r = 1.0f / sqrtf(block_sum(s, red) / (float)dim + P.eps);
+        }
+        if (split == 0 && h % (P.heads / P.kv_heads) == 0) {
+            float *kd = P.slot_base[sd.slot] + P.k_off + ((size_t)i * P.kv_heads + g) * dim, *vd = P.slot_base[sd.slot] + P.v_off + ((size_t)i * P.kv_heads + g) * vdim;
+            for (int c = tid; c < dim; c += blockDim.x) kd[c] = own_k[c] * own_r;
+            for (int c = tid; c < vdim; c += blockDim.x) vd[c] = own_v[c];
+        }
+    }
     const int lo = max(0, i - P.window + 1), nkeep = min(P.keep_first, lo), nk = nkeep + (i - lo + 1);
     const size_t kvd = (size_t)P.kv_heads * dim, vvd = (size_t)P.kv_heads * vdim;
-    const float *kc = P.slot_base[sd.slot] + P.k_off + (size_t)g * dim, *vc = P.slot_base[sd.slot] + P.v_off + (size_t)g * vdim;
+    gfloat *kc = (gfloat *)(P.slot_base[sd.slot] + P.k_off + (size_t)g * dim), *vc = (gfloat *)(P.slot_base[sd.slot] + P.v_off + (size_t)g * vdim);
     float m = -INFINITY, l = 0.0f, acc[WA_DPL];
 #pragma unroll
     for (int e = 0; e < WA_DPL; e++) acc[e] = 0.0f;
     // 16 keys per wave and step, four lanes per key (each a quarter of the dot product in interleaved 16-byte pieces, finished by a quad sum)
     const int nchunks = (nk + 15) / 16, sub = lane & 3;
-    const int nsplit = max(1, P.nsplit), split = blockIdx.z;
+    const int nsplit = max(1, P.nsplit);
     for (int ch = split * 4 + wave; ch < nchunks; ch += 4 * nsplit) {
         const int vi = ch * 16 + (lane >> 2);
         const bool valid = vi < nk;
         const int j = valid ? (vi < nkeep ? vi : lo + (vi - nkeep)) : i;
-        const float *kr = kc + (size_t)j * kvd;
+        gfloat *kr = FRESH && j == i ? own_k : kc + (size_t)j * kvd;
         float s = 0.0f;
         if ((dim & 3) == 0) {
+#pragma unroll 8
             for (int c = 4 * sub; c < dim; c += 16) {
-                const float4 kv = *reinterpret_cast<const float4 *>(kr + c);
+                const f32x4w kv = *(gf32x4 *)(kr + c);
                 s = fmaf(qn[c], kv.x, s); s = fmaf(qn[c + 1], kv.y, s); s = fmaf(qn[c + 2], kv.z, s); s = fmaf(qn[c + 3], kv.w, s);
             }
         } else {
             for (int c = sub; c < dim; c += 4) s = fmaf(qn[c], kr[c], s);
         }
         s = quad_sum(s) * P.scale;
+        if (FRESH && j == i) s *= own_r;
         if (P.softcap > 0.0f) s = P.softcap * tanhf(s / P.softcap);
         if (P.rel) s += bf2f(P.rel[(size_t)P.bucket_of[i - j] * P.heads + h]);
         if (!valid) s = -INFINITY;
@@ -115,13 +142,23 @@ __global__ void __launch_bounds__(256) k_attn_window(WinAttnArgs P)
 #pragma unroll
         for (int e = 0; e < WA_DPL; e++) acc[e] *= corr;
         m = m_new;
-        const int cnt = min(16, nk - ch * 16);
-        for (int jj = 0; jj < cnt; jj++) {
-            const float pj = __shfl(p, 4 * jj, 64);
-            const int kj = __shfl(j, 4 * jj, 64);
-            const float *vr = vc + (size_t)kj * vvd;
+        // value rows VB at a time, asked for side by side (keys past the last: the row's own, not counted): one after the other they were 16 trips to memory
+        constexpr int VB = WA_DPL <= 2 ? 16 : WA_DPL <= 4 ? 8 : 2;
+        for (int j0 = 0; j0 < 16; j0 += VB) {
+            float v[VB][WA_DPL];
 #pragma unroll
-            for (int e = 0; e < WA_DPL; e++) { const int d = lane + 64 * e; if (d < vdim) acc[e] = fmaf(pj, vr[d], acc[e]); }
+            for (int jj = 0; jj < VB; jj++) {
+                const int kj = __shfl(j, 4 * (j0 + jj), 64);
+                gfloat *vr = FRESH && kj == i ? own_v : vc + (size_t)kj * vvd;
+#pragma unroll
+                for (int e = 0; e < WA_DPL; e++) v[jj][e] = vr[min(lane + 64 * e, vdim - 1)];
+            }
+#pragma unroll
+            for (int jj = 0; jj < VB; jj++) {
+                const float pj = __shfl(p, 4 * (j0 + jj), 64);
+#pragma unroll
+                for (int e = 0; e < WA_DPL; e++) acc[e] = ch * 16 + j0 + jj < nk ? fmaf(pj, v[jj][e], acc[e]) : acc[e];
+            }
         }
     }
     if (lane == 0) { wm[wave] = m; wl[wave] = l; }
@@ -155,13 +192,59 @@ __global__ void __launch_bounds__(256) k_attn_window(WinAttnArgs P)
     }
 }
 
-// grid (rows, heads), one wave: the shares of a (row, head) and its sink into the output row.  Lane sp holds share sp's maximum and
+template <int WA_DPL>
+__global__ void __launch_bounds__(256) k_attn_window(WinAttnArgs P)
+{
+    extern __shared__ float sm[];
+    attn_row<WA_DPL, false>(P, FreshRow(), blockIdx.x, blockIdx.y, blockIdx.z, sm);
+}
+
+// One token of decayed linear attention, S <- d S + k v^T, o = S^T q, for 64 columns of a head: four waves of dk / 4 rows each
+struct StateRow { const float *q, *k, *v, *decay; int heads, dk, dv; size_t state_off; float *out; };
+template <int DK4>
+__device__ __forceinline__ void state_row(const StateRow &R, const SeqDesc &sd, float *state_base, const int h, const int c0, float *sm)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = min(c0 + lane, R.dv - 1), k0 = wave * DK4;
+    float *S = state_base + R.state_off + ((size_t)h * R.dk + k0) * R.dv + c;
+    const float *q = R.q + (size_t)h * R.dk + k0, *k = R.k + (size_t)h * R.dk + k0;
+    const float d = R.decay[h], v = R.v[(size_t)h * R.dv + c];
+    float x[DK4], o = 0.0f;
+#pragma unroll
+    for (int e = 0; e < DK4; e++) x[e] = ((gfloat *)S)[(size_t)e * R.dv];          // (whatever is there before a sequence's first token does not count)
+#pragma unroll
+    for (int e = 0; e < DK4; e++) {
+        x[e] = fmaf(sd.pos0 > 0 ? x[e] : 0.0f, d, k[e] * v);
+        o = fmaf(q[e], x[e], o);
+    }
+    if (c0 + lane < R.dv) {
+#pragma unroll
+        for (int e = 0; e < DK4; e++) S[(size_t)e * R.dv] = x[e];
+    }
+    sm[wave * 64 + lane] = o;
+    __syncthreads();
+    if (wave == 0 && c0 + lane < R.dv) R.out[(size_t)h * R.dv + c] = (sm[lane] + sm[64 + lane]) + (sm[128 + lane] + sm[192 + lane]);
+}
+
+// The mixers of a WINDOW_LINEAR layer for a step of one row in one launch: workgroups [0, heads * nsplit) the attention with the row's own key and value, the rest
+// the decayed linear attention (9 us; three launches of 4, 7.5 and 4 otherwise)
+template <int WA_DPL, int DK4>
+__global__ void __launch_bounds__(256) k_mix_row(WinAttnArgs P, FreshRow F, StateRow R)
+{
+    extern __shared__ float sm[];
+    const int nsplit = max(1, P.nsplit), na = P.heads * nsplit, id = blockIdx.x;
+    if (id < na) { attn_row<WA_DPL, true>(P, F, 0, id % P.heads, id / P.heads, sm); return; }
+    const int per = (R.dv + 63) / 64;
+    const SeqDesc sd = P.seqs[0];
+    state_row<DK4>(R, sd, P.slot_base[sd.slot], (id - na) / per, (id - na) % per * 64, sm);
+}
+
+// grid (rows, heads), one or two waves (a group of 64 columns each): the shares of a (row, head) and its sink into the output row.  Lane sp holds share sp's maximum and
 // sum, so the scale factors come from two wave reductions; the weighted values are then read for all shares at once.
 constexpr int WA_MAX_SPLITS = 32;
 
-__global__ void __launch_bounds__(64) k_attn_window_combine(WinAttnArgs P)
+__global__ void __launch_bounds__(128) k_attn_window_combine(WinAttnArgs P)
 {
-    const int t = blockIdx.x, h = blockIdx.y, dim = P.vdim, nsplit = P.nsplit, lane = threadIdx.x;      // (dim: columns of a value row)
+    const int t = blockIdx.x, h = blockIdx.y, dim = P.vdim, nsplit = P.nsplit, lane = threadIdx.x & 63;      // (dim: columns of a value row)
     const float *src = P.ws + ((size_t)t * P.heads + h) * nsplit * (dim + 2);
     const float snk = sink_of(P, h);
     const float m_sp = lane < nsplit ? src[(size_t)lane * (dim + 2)] : -INFINITY, l_sp = lane < nsplit ? src[(size_t)lane * (dim + 2) + 1] : 0.0f;
@@ -169,14 +252,14 @@ __global__ void __launch_bounds__(64) k_attn_window_combine(WinAttnArgs P)
     const float f_sp = m_sp == -INFINITY ? 0.0f : expf(m_sp - M);
     const float L = wave_sum(l_sp * f_sp) + (has_sink(P) ? expf(snk - M) : 0.0f);
     // (every lane walks every group of 64 columns, also where it has no column of its own: the scale factors come from other lanes)
-    for (int d0 = 0; d0 < dim; d0 += 64) {
+    for (int d0 = threadIdx.x & 64; d0 < dim; d0 += blockDim.x) {
         const int d = d0 + lane;
         float v[WA_MAX_SPLITS];
 #pragma unroll
-        for (int sp = 0; sp < WA_MAX_SPLITS; sp++) v[sp] = (sp < nsplit && d < dim) ? src[(size_t)sp * (dim + 2) + 2 + d] : 0.0f;
+        for (int sp = 0; sp < WA_MAX_SPLITS; sp++) v[sp] = src[(size_t)min(sp, nsplit - 1) * (dim + 2) + 2 + min(d, dim - 1)];      // (no branch: all at once)
         float o = 0.0f;
 #pragma unroll
-        for (int sp = 0; sp < WA_MAX_SPLITS; sp++) o = fmaf(v[sp], __shfl(f_sp, sp, 64), o);
+        for (int sp = 0; sp < WA_MAX_SPLITS; sp++) o = sp < nsplit ? fmaf(v[sp], __shfl(f_sp, sp, 64), o) : o;
         if (d < dim) P.out[(size_t)t * P.ldo + (size_t)h * dim + d] = o / L;
     }
 }
@@ -370,9 +453,6 @@ __global__ void __launch_bounds__(256) k_attn_window_tile(WinAttnArgs P, int n_s
 typedef __bf16 bf16x8w __attribute__((ext_vector_type(8)));
 constexpr int WT_WAVES = 8, WT_MAX_CHUNKS = 32, WT_SLOTS = 256;
 
-typedef float f32x4w __attribute__((ext_vector_type(4)));
-typedef const __attribute__((address_space(1))) float gfloat;
-typedef const __attribute__((address_space(1))) f32x4w gf32x4;
 typedef const __attribute__((address_space(1))) void wa_glb_t;
 typedef __attribute__((address_space(3))) void wa_lds_t;
 
@@ -1045,7 +1125,7 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
     else if (vdim <= 256) hipLaunchKernelGGL(k_attn_window<4>, grid_rows, dim3(256), smem, ifa_s(stream), P);
     else if (vdim <= 640) hipLaunchKernelGGL(k_attn_window<10>, grid_rows, dim3(256), smem, ifa_s(stream), P);
     else hipLaunchKernelGGL(k_attn_window<WA_DPL_MAX>, grid_rows, dim3(256), smem, ifa_s(stream), P);
-    if (nsplit > 1) hipLaunchKernelGGL(k_attn_window_combine, dim3((unsigned)rows, (unsigned)heads), dim3(64), 0, ifa_s(stream), P);
+    if (nsplit > 1) hipLaunchKernelGGL(k_attn_window_combine, dim3((unsigned)rows, (unsigned)heads), dim3(vdim <= 64 ? 64 : 128), 0, ifa_s(stream), P);
     IFA_LAUNCH_CHECK();
     return IFA_OK;
 }
@@ -1152,3 +1232,36 @@ int ifa_attention_kv_sinks_f32(const void *q_f32, size_t ldq, int heads, int kv_
 }
 
 } // extern "C"
+
+int ifa_mix_row(const IfaMixRow &M, int *nsplit, ifa_stream stream)
+{
+    IFA_REQUIRE(M.q && M.k && M.lq && M.lk && M.lv && M.decay && M.seqs && M.row_seq && M.slot_base && M.out && M.lin_out && nsplit, "mix_row: null pointer");
+    IFA_REQUIRE(ifa_mix_row_fits(M), "mix_row: %d / %d heads of %d, %d heads of %d x %d", M.heads, M.kv_heads, M.dim, M.l_heads, M.l_dim, M.l_vdim);
+    WinAttnArgs P;
+    memset(&P, 0, sizeof(P));
+    P.q = M.q; P.heads = M.heads; P.kv_heads = M.kv_heads; P.dim = P.vdim = M.dim; P.norm_q = 1; P.eps = M.eps; P.scale = M.scale; P.softcap = M.softcap;
+    P.window = M.window; P.keep_first = M.keep_first; P.rel = M.rel; P.bucket_of = M.bucket_of; P.n_buckets = M.n_buckets; P.sink = M.sink;
+    P.seqs = (const SeqDesc *)M.seqs; P.row_seq = M.row_seq; P.slot_base = (float *const *)M.slot_base; P.k_off = M.k_off; P.v_off = M.v_off;
+    P.out = M.out; P.ldo = P.ldq = (size_t)M.heads * M.dim;
+    const size_t keys = std::min((size_t)M.window + (size_t)M.keep_first, (size_t)M.max_keys);
+    int ns = (int)std::min<size_t>(IFA_ROW_OUT_SPLITS, (keys + 63) / 64);
+    while (ns > 1 && (size_t)M.heads * ns * ((size_t)M.dim + 2) * 4 > M.ws_bytes) ns--;
+    P.ws = M.ws; P.nsplit = *nsplit = std::max(ns, 1);
+    const FreshRow F{M.k, M.k, 1};
+    const StateRow R{M.lq, M.lk, M.lv, M.decay, M.l_heads, M.l_dim, M.l_vdim, M.l_off, M.lin_out};
+    const size_t smem = std::max((size_t)M.dim + 8 + 4 * (size_t)M.dim, (size_t)256) * 4;
+    const dim3 grid((unsigned)(M.heads * P.nsplit + M.l_heads * ((M.l_vdim + 63) / 64)));
+#define IFA_MR(D) { if (M.l_dim == 64) hipLaunchKernelGGL((k_mix_row<D, 16>), grid, dim3(256), smem, ifa_s(stream), P, F, R); \
+                    else hipLaunchKernelGGL((k_mix_row<D, 32>), grid, dim3(256), smem, ifa_s(stream), P, F, R); }
+    if (M.dim <= 64) IFA_MR(1) else IFA_MR(2)
+#undef IFA_MR
+    IFA_LAUNCH_CHECK();
+    return IFA_OK;
+}
+
+bool ifa_mix_row_fits(const IfaMixRow &M)
+{
+    // (more keys than the shares' workgroups take in eight rounds of 64: more workgroups and a launch that joins them do better)
+    return M.dim <= 128 && M.dim % 4 == 0 && M.k_off % 4 == 0 && M.v_off % 4 == 0 && (uintptr_t)M.k % 16 == 0 && (M.l_dim == 64 || M.l_dim == 128) && M.l_vdim > 0
+           && std::min((size_t)M.window + (size_t)M.keep_first, (size_t)M.max_keys) <= 64 * 8 * IFA_ROW_OUT_SPLITS;
+}

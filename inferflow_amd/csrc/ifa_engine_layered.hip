@@ -44,6 +44,7 @@
 #include <string>
 #include <vector>
 #include "ifa_engine_state.h"
+#include "ifa_rows_fused.h"
 #include "ifa_f32_common.h"
 
 using ifa32::bf16_t;
@@ -115,6 +116,7 @@ struct LayeredNet {
     float *tile_ws = nullptr; size_t tile_ws_bytes = 0;      // the same for prompts through the tiled attention (grown by the steps that need more)
     float *attn_ws = nullptr; size_t attn_ws_bytes = 0;      // partial results of the windowed attention when a (row, head)'s keys are shared out
     bf16_t *a16 = nullptr, *h16 = nullptr; size_t a16_cap = 0, h16_cap = 0; int opt_a16_min = 17;          // activations of a prompt's product rounded to bfloat16; steps of at least this many rows (0: never)
+    int opt_fuse_step = 1;                  // single-token steps of PARALLEL layers: norm inside the input product, everything behind the mixers in one launch
     int opt_attn_tile_min = 16;            // steps of at least this many rows run the windowed attention through the tiled kernel
     std::vector<ifa_seq_desc> seqs_host;   // the current step's sequences (the tiled attention's grid is sized from them)
     // POSTNORM layers: two more mixer buffers, the planes of the depth average ([layers + 1][scratch_rows * width]), the router's choices,
@@ -814,6 +816,61 @@ int run_state(ifa_model *m, int kind, const float *q, size_t ldq, const float *k
     return ifa_state_scan_f32(kind, 0, q, ldq, k, ldk, v, ldv, heads, qk_heads, dk, dv, decay_head, decay_row, beta_row, n->seqs_dev, nseq, slots, state_off, out, ldo, s);
 }
 
+// A PARALLEL layer of a single-token step as few launches: [norm + input product], the mixers, [everything behind them].  *done 0: the layer's sizes do not
+// allow it and nothing has been launched.
+int run_parallel_row(ifa_model *m, LLayer &L, bool *done)
+{
+    LayeredNet *n = m->lay;
+    const ifa_layered_config &c = n->cfg;
+    const ifa_layer_spec &sp = L.spec;
+    const size_t W = (size_t)c.width, NI = L.n_in;
+    ifa_stream s = (ifa_stream)m->stream;
+    void *const *slots = (void *const *)n->slot_base_dev;
+    const bool lin = sp.mixer == IFA_MIX_WINDOW_LINEAR;
+    IfaRowOut O;
+    memset(&O, 0, sizeof(O));
+    O.N = (int)W; O.x = n->x; O.ls1 = (const bf16_t *)L.T(IFA_LT_LS1).data; O.eps = c.eps; O.nsplit = 1; O.s0 = O.s1 = 1.0f;
+    if (lin) {
+        O.k0 = sp.a_heads * sp.a_dim; O.w0 = (const bf16_t *)L.T(IFA_LT_A_O).data; O.s0 = sp.a_out_scale; O.vdim = sp.a_dim; O.sink = (const bf16_t *)L.T(IFA_LT_A_SINK).data;
+        O.a0 = n->m1;
+        O.k1 = sp.l_heads * sp.l_vdim; O.w1 = (const bf16_t *)L.T(IFA_LT_L_O).data; O.s1 = sp.l_out_scale; O.o = n->m2; O.gate = n->proj + L.c_lg;
+        O.norm_w = (const bf16_t *)L.T(IFA_LT_L_NORM).data; O.group = O.wlen = O.k1;
+    } else {
+        O.k1 = sp.d_heads * sp.d_vdim; O.w1 = (const bf16_t *)L.T(IFA_LT_D_O).data; O.o = n->m2; O.gate = n->proj + L.c_dg; O.norm_w = (const bf16_t *)L.T(IFA_LT_D_NORM).data;
+        O.group = O.wlen = sp.d_vdim; O.gate_act = 1;
+    }
+    if (sp.ffn > 0) {
+        O.k2 = sp.ffn; O.w2 = (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data; O.ls2 = (const bf16_t *)L.T(IFA_LT_LS2).data; O.bias2 = (const bf16_t *)L.T(IFA_LT_FFN_DOWN_B).data;
+        O.gate_up = n->proj + L.c_fg;
+    }
+    IfaMixRow M;
+    memset(&M, 0, sizeof(M));
+    if (lin) {
+        M.q = n->proj + L.c_aq; M.k = n->proj + L.c_ak; M.heads = sp.a_heads; M.kv_heads = sp.a_kv_heads; M.dim = sp.a_dim; M.eps = c.eps; M.scale = sp.a_scale;
+        M.softcap = sp.a_softcap; M.window = sp.a_window; M.keep_first = sp.a_keep_first; M.max_keys = c.max_ctx; M.rel = (const bf16_t *)L.T(IFA_LT_A_REL).data;
+        M.bucket_of = L.bucket_of; M.n_buckets = sp.a_buckets; M.sink = O.sink; M.seqs = n->seqs_dev; M.row_seq = n->row_seq_dev; M.slot_base = slots; M.k_off = L.o_k; M.v_off = L.o_v;
+        M.out = n->m1; M.ws = n->attn_ws; M.ws_bytes = n->attn_ws_bytes; M.lq = n->proj + L.c_lq; M.lk = n->proj + L.c_lk; M.lv = n->proj + L.c_lv;
+        M.decay = (const float *)L.T(IFA_LT_L_DECAY).data; M.l_heads = sp.l_heads; M.l_dim = sp.l_dim; M.l_vdim = sp.l_vdim; M.l_off = L.o_lin; M.lin_out = n->m2;
+    }
+    *done = n->opt_fuse_step && W % 8 == 0 && ifa_row_out_fits(O) && (!lin || ifa_mix_row_fits(M));
+    if (!*done) return IFA_OK;
+    int rc;
+    if ((rc = ifa_linear_bf16w_rows(1, L.T(IFA_LT_NORM1).data, c.eps, L.w_in, NI, W, n->x, W, 1, L.b_in, nullptr, 1.0f, 0, n->proj, NI, lin ? (int)L.c_lq : 0,
+                                    lin ? (int)L.c_lg : 0, s))) return rc;
+    if (lin) {
+        if ((rc = ifa_mix_row(M, &O.nsplit, s))) return rc;
+        if (O.nsplit > 1) O.a0 = n->attn_ws;
+    } else {
+        const size_t QK = (size_t)sp.d_kv_heads * sp.d_dim, DV = (size_t)O.k1, C = (size_t)L.conv_ch;
+        if ((rc = ifa_delta_row_prep(n->proj + L.c_dq, NI, (int)C, sp.d_conv, (const bf16_t *)L.w_conv, n->seqs_dev, n->row_seq_dev, 1, slots, L.o_conv, (int)(2 * QK), sp.d_dim,
+                                     1e-6f, (int)QK, 1.0f / sqrtf((float)sp.d_dim), n->m1, C, n->proj + L.c_db, n->proj + L.c_da, sp.d_heads,
+                                     (const bf16_t *)L.T(IFA_LT_D_ALOG).data, (const bf16_t *)L.T(IFA_LT_D_DTBIAS).data, n->beta, n->decay, s))) return rc;
+        if ((rc = ifa_state_scan_f32(1, 0, n->m1, C, n->m1 + QK, C, n->m1 + 2 * QK, C, sp.d_heads, sp.d_kv_heads, sp.d_dim, sp.d_vdim, nullptr, n->decay, n->beta, n->seqs_dev, 1,
+                                     slots, L.o_rec, n->m2, DV, s))) return rc;
+    }
+    return ifa_row_out(O, s);
+}
+
 // the layers of one step over T rows / nseq sequences whose tables are already on the device; leaves the residual in n->x
 int run_layers(ifa_model *m, size_t T, int nseq)
 {
@@ -879,6 +936,15 @@ int run_layers(ifa_model *m, size_t T, int nseq)
             if (n->opt_tap_layers && n->taps && T <= n->taps_rows)
                 IFA_HIP_CHECK(hipMemcpyAsync(n->taps + ri * n->taps_rows * W, n->x, T * W * 4, hipMemcpyDeviceToDevice, m->stream));
             continue;
+        }
+        if (T == 1) {
+            bool done = false;
+            if ((rc = run_parallel_row(m, L, &done))) return rc;
+            if (done) {
+                if (n->opt_tap_layers && n->taps && T <= n->taps_rows)
+                    IFA_HIP_CHECK(hipMemcpyAsync(n->taps + ri * n->taps_rows * W, n->x, T * W * 4, hipMemcpyDeviceToDevice, m->stream));
+                continue;
+            }
         }
         const bf16_t *ls1 = (const bf16_t *)L.T(IFA_LT_LS1).data;
         const size_t NI = L.n_in;
@@ -959,7 +1025,7 @@ int run_head(ifa_model *m, size_t r0, size_t nr)
     LayeredNet *n = m->lay;
     const size_t W = (size_t)n->cfg.width, V = (size_t)n->cfg.vocab;
     int rc;
-    if ((n->opt_fuse_rows & 1) && nr <= 8 && W % 8 == 0 && n->cfg.stem == 0) {
+    if (((n->opt_fuse_rows & 1) || (n->opt_fuse_step && nr == 1)) && nr <= 8 && W % 8 == 0 && n->cfg.stem == 0) {
         if ((rc = ifa_linear_bf16w_rows(1, n->out_norm.data, n->cfg.eps, n->lm_head.data, V, W, n->x + r0 * W, W, nr, nullptr, nullptr, 1.0f, 0, n->logits, V, 0, 0,
                                         (ifa_stream)m->stream))) return rc;
         n->logits_rows = nr;
@@ -1335,13 +1401,14 @@ int lay_set_option(ifa_model *m, const char *name, int value)
     if (!strcmp(name, "tap_layers")) { n->opt_tap_layers = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "fuse_rows")) { n->opt_fuse_rows = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "fuse_post")) { n->opt_fuse_post = value; drop_step_graph(n); return IFA_OK; }
+    if (!strcmp(name, "fuse_step")) { n->opt_fuse_step = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "scan_chunk_min")) { n->opt_scan_chunk_min = value; return IFA_OK; }
     if (!strcmp(name, "ssm_chunk_min")) { n->opt_ssm_chunk_min = value; return IFA_OK; }
     if (!strcmp(name, "a16_min")) { n->opt_a16_min = value; return IFA_OK; }
     if (!strcmp(name, "attn_tile_min")) { n->opt_attn_tile_min = value; return IFA_OK; }
     if (!strcmp(name, "graph")) { n->opt_graph = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "ops32")) { IFA_HIP_CHECK(hipStreamSynchronize(m->stream)); n->cfg.ops32 = value ? 1 : 0; drop_step_graph(n); return IFA_OK; }
-    return ifa_fail(IFA_ERR_ARG, "ifa_model_set_option: unknown option '%s' (layer-list model: tap_layers, graph, ops32, attn_tile_min, a16_min, fuse_rows, fuse_post, ssm_chunk_min, scan_chunk_min)", name);
+    return ifa_fail(IFA_ERR_ARG, "ifa_model_set_option: unknown option '%s' (layer-list model: tap_layers, graph, ops32, attn_tile_min, a16_min, fuse_rows, fuse_post, ssm_chunk_min, scan_chunk_min, fuse_step)", name);
 }
 
 int lay_set_excluded(ifa_model *m, const int *ids_host, int cnt)

@@ -381,6 +381,81 @@ __global__ void __launch_bounds__(256) k_lin_rows(LinArgs P)
     }
 }
 
+// ONE row, layer-normed on the way in (k_lin_rows with prologue 1 formed the norm again for every output row of a wave): each wave forms mean and variance
+// once and keeps its lanes' normed values in registers, then walks output rows, the next row's weights asked for before this one's are summed.  The first
+// row's weights are on their way under the norm, so the norm's own launch (6 us) is saved for about 1 us more here (both 12.4 us, now 7.6, over a token's products of width 1024).
+template <int NP>
+__global__ void __launch_bounds__(256) k_lin_row_norm(LinArgs P)
+{
+    const int lane = threadIdx.x & 63, wave = blockIdx.x * 4 + (threadIdx.x >> 6), nwaves = gridDim.x * 4;
+    u32x4v w[NP], g[NP];
+    float a[NP][8], b = 0.0f;
+    auto request = [&](int n, u32x4v (&to)[NP]) {
+#pragma unroll
+        for (int p = 0; p < NP; p++) to[p] = *reinterpret_cast<const u32x4v *>(P.W + (size_t)n * P.K + min(512 * p + 8 * lane, P.K - 8));
+    };
+    int n = wave;
+    if (n >= P.N) return;
+    float s = 0.0f;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {          // (asked for before the weights: requests come back in order)
+        const int k = min(512 * p + 8 * lane, P.K - 8);
+        const float4 v0 = *reinterpret_cast<const float4 *>(P.A + k), v1 = *reinterpret_cast<const float4 *>(P.A + k + 4);
+        a[p][0] = v0.x; a[p][1] = v0.y; a[p][2] = v0.z; a[p][3] = v0.w; a[p][4] = v1.x; a[p][5] = v1.y; a[p][6] = v1.z; a[p][7] = v1.w;
+        g[p] = *reinterpret_cast<const u32x4v *>(P.norm_w + k);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    request(n, w);
+    if (P.bias) b = bf2f(P.bias[n]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+        if (512 * p + 8 * lane < P.K) s += ((a[p][0] + a[p][1]) + (a[p][2] + a[p][3])) + ((a[p][4] + a[p][5]) + (a[p][6] + a[p][7]));
+    const float mean = wave_sum(s) / (float)P.K;
+    float q = 0.0f;
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+        if (512 * p + 8 * lane < P.K) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) { a[p][e] -= mean; q = fmaf(a[p][e], a[p][e], q); }
+        }
+    const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)P.K + P.norm_eps);
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        const bool in = 512 * p + 8 * lane < P.K;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            a[p][2 * e] = in ? a[p][2 * e] * rstd * __uint_as_float(g[p][e] << 16) : 0.0f;
+            a[p][2 * e + 1] = in ? a[p][2 * e + 1] * rstd * __uint_as_float(g[p][e] & 0xFFFF0000u) : 0.0f;
+        }
+    }
+    while (true) {
+        const int next = n + nwaves;
+        float acc = 0.0f;
+        u32x4v w2[NP];
+        float b2 = 0.0f;
+        if (next < P.N) { request(next, w2); if (P.bias) b2 = bf2f(P.bias[next]); }
+#pragma unroll
+        for (int p = 0; p < NP; p++)
+            if (512 * p + 8 * lane < P.K) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    acc = fmaf(a[p][2 * e], __uint_as_float(w[p][e] << 16), acc);
+                    acc = fmaf(a[p][2 * e + 1], __uint_as_float(w[p][e] & 0xFFFF0000u), acc);
+                }
+            }
+        acc = wave_sum(acc) + b;
+        if (lane == 0) {
+            if (n >= P.act_c0 && n < P.act_c1) acc = silu_exact(acc);
+            P.C[n] = acc;
+        }
+        if (next >= P.N) break;
+        n = next; b = b2;
+#pragma unroll
+        for (int p = 0; p < NP; p++) w[p] = w2[p];
+    }
+}
+
 } // namespace
 
 static int linear_launch(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *bias_bf16,
@@ -405,7 +480,13 @@ static int linear_launch(const void *w_bf16, size_t rows, size_t cols, const voi
         IFA_REQUIRE(tokens <= 8 && P.vec, "%s: a fused prologue needs at most 8 rows and 16-byte aligned rows of whole 8-element pieces", who);
         IFA_REQUIRE(prologue != 1 || (norm_w_bf16 && ((uintptr_t)norm_w_bf16 & 15) == 0), "%s: the norm's weight is missing or unaligned", who);
     }
-    if (tokens <= 8) {
+    if (tokens == 1 && prologue == 1 && cols <= 8 * 512 && !mul_bf16 && alpha == 1.0f && !accumulate && act == 0) {
+        // (up to 16 waves a compute unit: 4096 of them share the output rows)
+        const unsigned grid = (unsigned)std::min<size_t>((rows + 3) / 4, 1024);
+        if (cols <= 2 * 512) hipLaunchKernelGGL(k_lin_row_norm<2>, dim3(grid), dim3(256), 0, s, P);
+        else if (cols <= 4 * 512) hipLaunchKernelGGL(k_lin_row_norm<4>, dim3(grid), dim3(256), 0, s, P);
+        else hipLaunchKernelGGL(k_lin_row_norm<8>, dim3(grid), dim3(256), 0, s, P);
+    } else if (tokens <= 8) {
         const unsigned grid = (unsigned)std::min<size_t>((rows + 3) / 4, 8192);
 #define IFA_LR(TT) { if (prologue == 1) hipLaunchKernelGGL((k_lin_rows<TT, 1>), dim3(grid), dim3(256), 0, s, P); \
                      else if (prologue == 2) hipLaunchKernelGGL((k_lin_rows<TT, 2>), dim3(grid), dim3(256), 0, s, P); \

@@ -305,16 +305,19 @@ __global__ void __launch_bounds__(1024) k_argmax_f32(const float *__restrict__ l
     auto take = [&](float v, int c) { if (c != ex[0] && c != ex[1] && c != ex[2] && (v > best || (v == best && c < idx))) { best = v; idx = c; } };
     int c0 = 0;
     if (((uintptr_t)r & 15) == 0) {          // 16-byte pieces, four requested side by side
-        for (; c0 + 16 * (int)blockDim.x <= n; c0 += 16 * blockDim.x) {
+        // (the last round's pieces past the row: its last one again, which takes nothing a second time.  One by one that round was 15 trips to memory of a row of 32000)
+        const int n4 = n & ~3;
+        for (; c0 < n4; c0 += 16 * blockDim.x) {
             float4 v[4];
 #pragma unroll
-            for (int u = 0; u < 4; u++) v[u] = *reinterpret_cast<const float4 *>(r + c0 + 4 * (threadIdx.x + u * blockDim.x));
+            for (int u = 0; u < 4; u++) v[u] = *reinterpret_cast<const float4 *>(r + min(c0 + 4 * (int)(threadIdx.x + u * blockDim.x), n4 - 4));
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const int c = c0 + 4 * (threadIdx.x + u * blockDim.x);
+                const int c = min(c0 + 4 * (int)(threadIdx.x + u * blockDim.x), n4 - 4);
                 take(v[u].x, c); take(v[u].y, c + 1); take(v[u].z, c + 2); take(v[u].w, c + 3);
             }
         }
+        c0 = n4;
     }
     for (int c = c0 + threadIdx.x; c < n; c += blockDim.x) take(r[c], c);
     for (int o = 32; o > 0; o >>= 1) {

@@ -1,0 +1,39 @@
+// ifa_rows_fused.h -- the second half of a single-token layer as one launch (ifa_rows_fused.hip) and the attention that feeds it
+#pragma once
+#include "ifa_host.h"
+#include "ifa_f32_common.h"
+#include "inferflow_amd.h"
+
+// x[n] += ls1[n] (s0 W0[n] . a0 + s1 W1[n] . a1) + ls2[n] (W2[n] . a2 + bias2[n]) for ONE row; k0 / k1 / k2 columns, multiples of 8 (0: that part is missing):
+//   a0  attention: a finished row (nsplit 1) or the shares of nsplit workgroups per head ([heads][nsplit][maximum, sum, vdim values], joined here with the sink)
+//   a1  o / rms_group(o) * norm_w[c % wlen] * act(gate), act 0 sigmoid, 1 silu
+//   a2  gelu_tanh(gate_up[c]) * gate_up[k2 + c]
+struct IfaRowOut {
+    int N; float *x;
+    const ifa32::bf16_t *w0, *w1, *w2; int k0, k1, k2;
+    float s0, s1; const ifa32::bf16_t *ls1, *ls2, *bias2;
+    const float *a0; int nsplit, vdim; const ifa32::bf16_t *sink;
+    const float *o, *gate; const ifa32::bf16_t *norm_w; int group, wlen, gate_act; float eps;
+    const float *gate_up;
+};
+constexpr int IFA_ROW_OUT_SPLITS = 8;
+// what ifa_row_out takes: sizes, alignment
+bool ifa_row_out_fits(const IfaRowOut &P);
+int ifa_row_out(const IfaRowOut &P, ifa_stream stream);
+
+// the mixers of a WINDOW_LINEAR layer for ONE row: ifa_kv_store_f32 (keys normed, values the keys as projected) + ifa_attention_window_f32 + the decayed linear
+// attention of ifa_state_scan_f32.  *nsplit workgroups per head share the keys and nobody joins their shares (in ws; at most IFA_ROW_OUT_SPLITS; 1: out holds the row)
+struct IfaMixRow {
+    const float *q, *k; int heads, kv_heads, dim; float eps, scale, softcap; int window, keep_first, max_keys;
+    const ifa32::bf16_t *rel; const int *bucket_of; int n_buckets; const ifa32::bf16_t *sink;
+    const ifa_seq_desc *seqs; const int *row_seq; void *const *slot_base; size_t k_off, v_off;
+    float *out, *ws; size_t ws_bytes;
+    const float *lq, *lk, *lv, *decay; int l_heads, l_dim, l_vdim; size_t l_off; float *lin_out;
+};
+bool ifa_mix_row_fits(const IfaMixRow &M);
+int ifa_mix_row(const IfaMixRow &M, int *nsplit, ifa_stream stream);
+
+// GATED_DELTA layers, ONE row per sequence: ifa_shortconv_silu_f32 + ifa_shortconv_tail_f32 + ifa_delta_gates_f32 in one launch (csrc/ifa_seqmix.hip)
+int ifa_delta_row_prep(const float *x, size_t ldx, int channels, int taps, const ifa32::bf16_t *w, const ifa_seq_desc *seqs, const int *row_seq, size_t rows, void *const *slot_base,
+                       size_t state_off, int norm_cols, int group_dim, float l2_eps, int scale_cols, float scale, float *y, size_t ldy, const float *b, const float *a, int heads,
+                       const ifa32::bf16_t *a_log, const ifa32::bf16_t *dt_bias, float *beta, float *decay, ifa_stream stream);

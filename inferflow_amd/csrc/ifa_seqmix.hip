@@ -24,12 +24,22 @@ namespace {
 // sequence's carried tail (rows [taps - 1][C], oldest first) or is zero at the start of a sequence.  Then channels
 // [0, norm_cols) are turned into unit vectors in groups of gdim (x / sqrt(sum x^2 + l2_eps)) and channels [0, scale_cols)
 // are multiplied by qscale.
+// ROW (one row per sequence): the carried tail is advanced too, by the threads that have read it, and the row's gates are formed (G; x's row holds b and a).
+struct RowGates { int b0, a0, heads; const bf16_t *A_log, *dt_bias; float *beta, *g; };
+template <bool ROW>
 __global__ void __launch_bounds__(256) k_shortconv_silu(const float *__restrict__ x, size_t ldx, int C, int taps, const bf16_t *__restrict__ w,
                                                         const SeqDesc *__restrict__ seqs, const int *__restrict__ row_seq,
                                                         float *const *__restrict__ slot_base, size_t state_off, int norm_cols, int gdim,
-                                                        float l2_eps, int scale_cols, float qscale, float *__restrict__ y, size_t ldy, int slice)
+                                                        float l2_eps, int scale_cols, float qscale, float *__restrict__ y, size_t ldy, int slice, RowGates G)
 {
     extern __shared__ float ys[];
+    if (ROW && blockIdx.y == 0)
+        for (int h = threadIdx.x; h < G.heads; h += blockDim.x) {
+            const float *xr = x + (size_t)blockIdx.x * ldx;
+            const size_t at = (size_t)blockIdx.x * G.heads + h;
+            G.beta[at] = sigmoid_f(xr[G.b0 + h]);
+            G.g[at] = expf(-expf(bf2f(G.A_log[h])) * softplus_f(xr[G.a0 + h] + bf2f(G.dt_bias[h])));
+        }
     const int t = blockIdx.x;
     const int c_lo = blockIdx.y * slice, c_hi = min(C, c_lo + slice);      // this workgroup's channels (whole norm groups: slice % gdim == 0)
     const SeqDesc sd = seqs[row_seq[t]];
@@ -43,6 +53,7 @@ __global__ void __launch_bounds__(256) k_shortconv_silu(const float *__restrict_
             if (idx >= 0) v = x[(size_t)(sd.row0 + idx) * ldx + c];
             else v = tail ? tail[(size_t)(taps - 1 + idx) * C + c] : 0.0f;
             acc = fmaf(bf2f(w[(size_t)c * taps + j]), v, acc);
+            if (ROW && j > 0) slot_base[sd.slot][state_off + (size_t)(j - 1) * C + c] = v;          // (its place in the next token's tail: one below where it was read)
         }
         ys[c - c_lo] = silu_exact(acc);
     }
@@ -154,14 +165,15 @@ __global__ void __launch_bounds__(256) k_norm_add_conv_rows(float *__restrict__ 
     }
 }
 
-// grid: one workgroup per sequence.  The carried tail becomes the last taps - 1 inputs of (old tail, this step's rows).
+// grid: (sequences, channels / 256).  The carried tail becomes the last taps - 1 inputs of (old tail, this step's rows).
 __global__ void __launch_bounds__(256) k_shortconv_tail(const float *__restrict__ x, size_t ldx, int C, int taps, const SeqDesc *__restrict__ seqs,
                                                         float *const *__restrict__ slot_base, size_t state_off)
 {
     const SeqDesc sd = seqs[blockIdx.x];
     float *tail = slot_base[sd.slot] + state_off;
     const int keep = taps - 1;
-    for (int c = threadIdx.x; c < C; c += blockDim.x)
+    const int c = blockIdx.y * 256 + threadIdx.x;
+    if (c < C)
         for (int r = 0; r < keep; r++) {          // ascending r: a value read from the old tail lies above what was written so far
             const int idx = sd.n - keep + r;      // index into this step's rows
             float v;
@@ -650,9 +662,9 @@ int ifa_shortconv_silu_f32(const void *x_f32, size_t ldx, int channels, int taps
     const int gd = norm_cols > 0 ? group_dim : 1;
     const int slice = std::min(channels, gd * std::max(1, (512 + gd - 1) / gd));
     IFA_REQUIRE((size_t)slice * 4 <= 64 * 1024, "ifa_shortconv_silu_f32: norm groups of %d channels do not fit the LDS", group_dim);
-    hipLaunchKernelGGL(k_shortconv_silu, dim3((unsigned)rows, ifa_cdiv((size_t)channels, (size_t)slice)), dim3(256), (size_t)slice * 4, ifa_s(stream),
+    hipLaunchKernelGGL(k_shortconv_silu<false>, dim3((unsigned)rows, ifa_cdiv((size_t)channels, (size_t)slice)), dim3(256), (size_t)slice * 4, ifa_s(stream),
                        (const float *)x_f32, ldx, channels, taps, (const bf16_t *)w_bf16, (const SeqDesc *)seqs_dev, row_seq_dev, (float *const *)slot_base_dev,
-                       state_off, norm_cols, group_dim, l2_eps, scale_cols, scale, (float *)y_f32, ldy, slice);
+                       state_off, norm_cols, group_dim, l2_eps, scale_cols, scale, (float *)y_f32, ldy, slice, RowGates());
     IFA_LAUNCH_CHECK();
     return IFA_OK;
 }
@@ -694,7 +706,7 @@ int ifa_shortconv_tail_f32(const void *x_f32, size_t ldx, int channels, int taps
     IFA_REQUIRE(x_f32 && seqs_dev && slot_base_dev, "ifa_shortconv_tail_f32: null pointer");
     IFA_REQUIRE(channels > 0 && taps >= 1 && n_seqs > 0 && ldx >= (size_t)channels, "ifa_shortconv_tail_f32: bad shape");
     if (taps == 1) return IFA_OK;
-    hipLaunchKernelGGL(k_shortconv_tail, dim3((unsigned)n_seqs), dim3(256), 0, ifa_s(stream), (const float *)x_f32, ldx, channels, taps,
+    hipLaunchKernelGGL(k_shortconv_tail, dim3((unsigned)n_seqs, ifa_cdiv((size_t)channels, 256)), dim3(256), 0, ifa_s(stream), (const float *)x_f32, ldx, channels, taps,
                        (const SeqDesc *)seqs_dev, (float *const *)slot_base_dev, state_off);
     IFA_LAUNCH_CHECK();
     return IFA_OK;
@@ -842,3 +854,18 @@ int ifa_gated_groupnorm_f32(const void *o_f32, size_t ldo, size_t rows, int chan
 }
 
 } // extern "C"
+
+int ifa_delta_row_prep(const float *x, size_t ldx, int channels, int taps, const bf16_t *w, const ifa_seq_desc *seqs, const int *row_seq, size_t rows, void *const *slot_base,
+                       size_t state_off, int norm_cols, int group_dim, float l2_eps, int scale_cols, float scale, float *y, size_t ldy, const float *b, const float *a, int heads,
+                       const bf16_t *a_log, const bf16_t *dt_bias, float *beta, float *decay, ifa_stream stream)
+{
+    IFA_REQUIRE(x && w && seqs && row_seq && slot_base && y && b && a && a_log && dt_bias && beta && decay, "delta_row_prep: null pointer");
+    const int gd = norm_cols > 0 ? group_dim : 1, slice = std::min(channels, gd * std::max(1, (512 + gd - 1) / gd));
+    IFA_REQUIRE(channels > 0 && taps >= 1 && taps <= 64 && rows > 0 && heads > 0 && ldx >= (size_t)channels && ldy >= (size_t)channels && (size_t)slice * 4 <= 64 * 1024
+                && (norm_cols == 0 || (group_dim > 0 && norm_cols % group_dim == 0)), "delta_row_prep: bad shape");
+    const RowGates G{(int)(b - x), (int)(a - x), heads, a_log, dt_bias, beta, decay};
+    hipLaunchKernelGGL(k_shortconv_silu<true>, dim3((unsigned)rows, ifa_cdiv((size_t)channels, (size_t)slice)), dim3(256), (size_t)slice * 4, ifa_s(stream), x, ldx, channels, taps,
+                       w, (const SeqDesc *)seqs, row_seq, (float *const *)slot_base, state_off, norm_cols, group_dim, l2_eps, scale_cols, scale, y, ldy, slice, G);
+    IFA_LAUNCH_CHECK();
+    return IFA_OK;
+}

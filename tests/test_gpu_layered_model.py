@@ -297,3 +297,49 @@ def test_ini_route_and_trace_replay_tool(tmp_path):
         g = np.fromfile(out / ("%d.f32" % s), np.float32).reshape(-1, V)
         exp = [wa[19 + s]] + ([wb[5 + s]] if s <= 3 and s != 2 else [])
         assert fx.rel_err(g, np.stack(exp)).max() < TOL32, s
+
+
+@pytest.mark.parametrize("ctx", [340, 60])      # keys of a head by six workgroups whose shares the last launch joins / by one
+def test_single_token_steps_in_few_launches(tmp_path, ctx):
+    """Steps of one token whose layers' sizes allow the norm inside the input product, both mixers in one launch and everything behind them in another: against the
+    oracle and against the same engine with one launch per operation; a layer without feed-forward, windows above and below the context, two norm groups' sizes."""
+    import inferflow_amd as ia
+    cfg = fx.config([fx.parallel_layer(heads=4, kv_heads=2, dim=64, window=2000, keep_first=0, lin_heads=3, lin_dim=64, lin_vdim=96, ff=200),
+                     fx.delta_layer(heads=4, kv_heads=2, dim=16, vdim=32, conv=3, ff=96),
+                     fx.parallel_layer(heads=3, kv_heads=1, dim=100, window=50, keep_first=5, lin_heads=2, lin_dim=128, lin_vdim=40, ff=0),
+                     fx.delta_layer(heads=2, kv_heads=2, dim=32, vdim=128, conv=1, ff=0)], width=136, vocab=97)
+    w = fx.random_weights(cfg, 21)
+    n = ctx - 20
+    toks = tokens_for(cfg, n + 12, 22)
+    want = oracle_logits(cfg, w, toks)
+    rows = []
+    for fused in (1, 0):
+        eng = engine_for(tmp_path, cfg, w, ctx=ctx, queries=2)
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"fuse_step", fused))
+        eng.add_query(toks[:5]); eng.infer()                  # (another query's slot and cache beside it)
+        q = eng.add_query(toks[:n])
+        got = []
+        for t in toks[n:]:
+            eng.infer(); got.append(eng.last_logits_f32(q)[-1])
+            assert eng.commit({q: t})
+        eng.infer(); got.append(eng.last_logits_f32(q)[-1])
+        rows.append(np.stack(got)); eng.close()
+    assert fx.rel_err(rows[0], want[n - 1:]).max() < TOL32 and fx.rel_err(rows[1], want[n - 1:]).max() < TOL32
+    assert fx.rel_err(rows[0][1:], rows[1][1:]).max() < TOL32
+
+
+@pytest.mark.parametrize("K", [8, 120, 512, 520, 1024, 1032, 2048, 2056, 4096])
+@pytest.mark.parametrize("N", [1, 5, 4099])
+def test_one_row_product_with_the_norm_inside(K, N):
+    import inferflow_amd as ia
+    from tests.gpu_util import capi, p
+    from tests.test_gpu_layered_ops import dev32, devbf
+    rng = np.random.default_rng(K + N)
+    W, bias, g = orc.bf16_round(rng.standard_normal((N, K)) / K ** 0.5), orc.bf16_round(rng.standard_normal(N)), orc.bf16_round(1 + 0.2 * rng.standard_normal(K))
+    x = (2 * rng.standard_normal((1, K)) + 1).astype(np.float32)
+    c = torch.full((N + 3,), float("nan"), dtype=torch.float32, device="cuda")
+    ia.check(capi().ifa_linear_bf16w_rows(1, p(devbf(g)), 1e-5, p(devbf(W)), N, K, p(dev32(x)), K, 1, p(devbf(bias)), None, 1.0, 0, p(c), N + 3, 2, 4, None))
+    want = (orc.layer_norm_nobias(orc.t64(x), orc.t64(g), 1e-5) @ orc.t64(W).T + orc.t64(bias))[0]
+    want[2:4] = orc.silu(want[2:4])
+    got = c.cpu().numpy()
+    assert np.abs(got[:N] - want.numpy()).max() < 1e-5 * max(1.0, float(want.abs().max())) and np.isnan(got[N:]).all()
