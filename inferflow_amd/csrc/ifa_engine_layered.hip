@@ -383,6 +383,21 @@ int linear(ifa_model *m, const bf16_t *W, size_t N, size_t K, const float *A, si
     return ifa_linear_bf16w(W, N, K, A, lda, T, bias, mul, alpha, accumulate, m->lay->cfg.ops32, C, ldc, silu0, silu1, (ifa_stream)m->stream);
 }
 
+// the product behind a gated feed-forward's activations: they leave gate | up in the form that the product reads
+int glu_linear(ifa_model *m, int kind, float limit, const float *gate_up, size_t ld, size_t F, const float *row_gate, size_t ldg, const bf16_t *W, size_t N, size_t T,
+               const bf16_t *bias, const bf16_t *mul, int accumulate, float *C)
+{
+    LayeredNet *n = m->lay;
+    ifa_stream s = (ifa_stream)m->stream;
+    int rc;
+    if (takes_a16(n, F, T)) {
+        if ((rc = ensure_a16(m, T, F)) || (rc = ifa_glu_to_bf16(kind, limit, gate_up, ld, T, F, row_gate, ldg, n->a16, a16_stride(F), s))) return rc;
+        return ifa_linear_bf16_both(W, N, F, n->a16, a16_stride(F), T, bias, mul, 1.0f, accumulate, 0, C, nullptr, N, 0, 0, s);
+    }
+    if ((rc = ifa_glu_ex_f32(kind, limit, gate_up, ld, T, F, row_gate, ldg, n->m3, F, s))) return rc;
+    return linear(m, W, N, F, n->m3, F, T, bias, mul, 1.0f, accumulate, C, N);
+}
+
 // product of what a norm has left: bfloat16 rows (h16) or 32-bit rows
 int linear_in(ifa_model *m, const bf16_t *W, size_t N, size_t K, const float *h, const bf16_t *h16, size_t T, const bf16_t *bias, float *C, size_t ldc)
 {
@@ -618,8 +633,7 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
     if ((rc = linear_in(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2))) return rc;
     if (!moe) {
         const size_t F = (size_t)sp.ffn;
-        if ((rc = ifa_glu_ex_f32(3, sp.f_limit, n->proj + L.c2_fg, N2, T, F, nullptr, 0, n->m3, F, s))) return rc;
-        if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, F, n->m3, F, T, nullptr, nullptr, 1.0f, 0, n->m2, W))) return rc;
+        if ((rc = glu_linear(m, 3, sp.f_limit, n->proj + L.c2_fg, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m2))) return rc;
     } else {
         // the router's logits (bias added by the product) are columns of the second product; the chosen experts read norm2's output
         if ((rc = ifa_moe_route_top_f32(n->proj + L.c2_router, N2, T, sp.x_experts, sp.x_top, nullptr, n->moe_idx, n->moe_wgt, s))) return rc;
@@ -627,8 +641,7 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
                                             c.ops32, n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, s))) return rc;
         if (sp.x_shared_ff > 0) {      // the shared expert: its gate sigmoid(w_sg . h) multiplies the activations in front of the down-projection
             const size_t SF = (size_t)sp.x_shared_ff;
-            if ((rc = ifa_glu_ex_f32(0, 0.0f, n->proj + L.c2_shg, N2, T, SF, n->proj + L.c2_sg, N2, n->m3, SF, s))) return rc;
-            if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, W, SF, n->m3, SF, T, nullptr, nullptr, 1.0f, 1, n->m2, W))) return rc;
+            if ((rc = glu_linear(m, 0, 0.0f, n->proj + L.c2_shg, N2, SF, n->proj + L.c2_sg, N2, (const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, W, T, nullptr, nullptr, 1, n->m2))) return rc;
         }
     }
     return close_sub(n->m2, L.T(IFA_LT_NORM2B).data, next_norm, in16);
@@ -779,8 +792,7 @@ int run_streams_layer(ifa_model *m, LLayer &L, size_t T, int nseq, int pass, LLa
     if (!moe) {
         const size_t F = (size_t)sp.ffn, N2 = L.n_in2;
         if ((rc = linear(m, L.w_in2, N2, W, n->h, W, T, nullptr, nullptr, 1.0f, 0, n->proj, N2))) return rc;
-        if ((rc = ifa_glu_f32(0, n->proj, N2, T, F, n->m3, F, s))) return rc;
-        if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, F, n->m3, F, T, nullptr, nullptr, 1.0f, 0, n->m1, W))) return rc;
+        if ((rc = glu_linear(m, 0, 0.0f, n->proj, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m1))) return rc;
     } else {
         const int XA = sp.x_experts;
         if (T <= 8 && XA <= 256 && n->opt_fuse_post) {      // a few rows: the choice inside the experts' first launch
@@ -992,9 +1004,8 @@ int run_layers(ifa_model *m, size_t T, int nseq)
                 if ((rc = ifa_linear_bf16w_rows(2, nullptr, 0.0f, L.T(IFA_LT_FFN_DOWN).data, W, F, n->proj + L.c_fg, NI, T, L.T(IFA_LT_FFN_DOWN_B).data,
                                                 L.T(IFA_LT_LS2).data, 1.0f, 1, n->x, W, 0, 0, s))) return rc;
             } else {
-                if ((rc = ifa_glu_f32(1, n->proj + L.c_fg, NI, T, F, n->m3, F, s))) return rc;
-                if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, F, n->m3, F, T, (const bf16_t *)L.T(IFA_LT_FFN_DOWN_B).data,
-                                 (const bf16_t *)L.T(IFA_LT_LS2).data, 1.0f, 1, n->x, W))) return rc;
+                if ((rc = glu_linear(m, 1, 0.0f, n->proj + L.c_fg, NI, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T,
+                                     (const bf16_t *)L.T(IFA_LT_FFN_DOWN_B).data, (const bf16_t *)L.T(IFA_LT_LS2).data, 1, n->x))) return rc;
             }
         }
         if (n->opt_tap_layers && n->taps && T <= n->taps_rows)

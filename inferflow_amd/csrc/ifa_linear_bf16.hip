@@ -10,12 +10,14 @@
 //             OPS32 = false: operands rounded to bfloat16, v_mfma_f32_32x32x16_bf16;
 //             OPS32 = true : operands stay 32-bit, v_mfma_f32_32x32x2_f32 (the exact mode of the worker)
 //   prompts   k_lin_tile<BM, BN> (ifa_linear_bf16_both: activations rounded to bfloat16 beforehand, by their producer or by k_rows_to_bf16): tiles of up to
-//             128 x 128, both operands straight to LDS; the same sums in the same order as k_lin_mfma<false>
+//             128 x 128 (32 x 32 where there are few), both operands straight to LDS; the same sums in the same order as k_lin_mfma<false>
 // Accumulation is fp32 in every path.  No atomics, no split K: a result does not depend on what else runs.
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include "ifa_host.h"
 #include "ifa_f32_common.h"
+#include "ifa_rows_fused.h"
 
 using namespace ifa32;
 
@@ -158,22 +160,36 @@ __global__ void __launch_bounds__(256) k_lin_mfma(LinArgs P)
 // Workgroups are dealt to the eight XCDs round-robin: the id is remapped so that an XCD works on a compact block of tiles whose operands its L2 shares.
 // A's rows are K rounded up to whole steps long, zero beyond K (what W's requests bring in there -- held inside the row -- does not count).
 constexpr int LT_BK = 64;
+// Up to so many 64 x 64 tiles: 32 x 32 tiles of one wave each, seven steps under way / 64 x 64 tiles, three steps under way.  us with two buffers of 64 x 64, four of 64 x 64,
+// eight of 32 x 32 -- 16 tiles of 4096 columns 30.7, 18.3, 15.4; 64 tiles of 4096 46.0, 19.1, 15.8; 128 of 1024 9.9, 7.1, 6.8; 192 of 1024 10.0, 7.1, 11.3; 400 of 2560
+// 21.7, 18.4, 31.1; 640 of 1024 12.2, 14.2, 26.8; 640 of 4096 50.7, 47.7, 80.9.  (Steps split over two or four groups of waves: 24.0 for 64 tiles of 4096, and other sums.)
+constexpr size_t LT_SMALL = 128, LT_DEEP = 512;
 typedef __attribute__((address_space(3))) void lt_lds_t;
 typedef const __attribute__((address_space(1))) void lt_glb_t;
 
-template <int BM, int BN>
-__global__ void __launch_bounds__(256, 2) k_lin_tile(LinArgs P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
+// NB > 2: NB buffers, a step asked for NB - 1 steps ahead.  For products whose tiles do not fill the chip, which wait for one step after the other (0.4 to 0.7 us a step
+// with two buffers, 0.25 with more: the requests' issue, the fragments' way from LDS and the chain of products).
+// GROUPED: row tiles and matrices from P.tile_map, the rows of A by P.a_rows (null: as they are), each output row times P.row_scale.
+template <int BM, int BN, int NB, bool GROUPED>
+__global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_tile(LinArgs P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
 {
-    constexpr int TA = BM / 64, TB = BN / 64, AI = BM / 32, WI = BN / 32, ROWB = 2 * LT_BK, STEPB = (BM + BN) * ROWB;
-    __shared__ __attribute__((aligned(16))) char smem[2 * STEPB];          // [2 steps][BM rows of A, BN rows of W]
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5, wm = wave & 1, wn = wave >> 1;
-    int t0, n0;
+    constexpr int WAVES = BM == 32 ? 1 : 4, TA = BM == 32 ? 1 : BM / 64, TB = BM == 32 ? 1 : BN / 64, AI = BM / (8 * WAVES), WI = BN / (8 * WAVES), ROWB = 2 * LT_BK, STEPB = (BM + BN) * ROWB;
+    __shared__ __attribute__((aligned(16))) char smem[NB * STEPB];          // [NB steps][BM rows of A, BN rows of W]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5, wm = wave & 1, wn = wave >> 1;          // (BM = 32: one wave, one tile)
+    int t0, n0, t_end = P.T;
+    const bf16_t *Wg = P.W;
     {
         const int nwg = tiles_m * tiles_n, orig = blockIdx.x, xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
         const int wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
         constexpr int GM = 1024 / BM;          // bands of 1024 rows of C, the row tiles of a band fastest
         const int band = wg / (GM * tiles_n), within = wg % (GM * tiles_n), band_m = min(GM, tiles_m - band * GM);
         t0 = (band * GM + within % band_m) * BM; n0 = (within / band_m) * BN;
+        if constexpr (GROUPED) {
+            const int tile = t0 / BM;
+            if (tile >= *P.n_tiles) return;
+            const int *tm = P.tile_map + 3 * tile;
+            Wg += (size_t)tm[0] * P.N * P.K; t0 = tm[1]; t_end = tm[1] + tm[2];
+        }
     }
     auto swz = [](int r) { return (r >> 1) & 7; };
     const bf16_t *asrc[AI], *wsrc[WI];
@@ -181,22 +197,28 @@ __global__ void __launch_bounds__(256, 2) k_lin_tile(LinArgs P, const bf16_t *__
 #pragma unroll
     for (int j = 0; j < AI; j++) {
         const int row = (wave * AI + j) * 8 + (lane >> 3), c = (lane & 7) ^ swz(row);
-        asrc[j] = A16 + (size_t)min(t0 + row, P.T - 1) * lda16 + c * 8;          // (rows beyond the last: repeated, not stored)
+        int at = min(t0 + row, t_end - 1);          // (rows beyond the last: repeated, not stored)
+        if (GROUPED && P.a_rows) at = P.a_rows[at];
+        asrc[j] = A16 + (size_t)at * lda16 + c * 8;
     }
 #pragma unroll
     for (int j = 0; j < WI; j++) {
         const int row = (wave * WI + j) * 8 + (lane >> 3), c = (lane & 7) ^ swz(row);
-        wsrc[j] = P.W + (size_t)min(n0 + row, P.N - 1) * P.K + c * 8;
+        wsrc[j] = Wg + (size_t)min(n0 + row, P.N - 1) * P.K + c * 8;
         wlim[j] = P.K - 8 - c * 8;
     }
-    auto stage = [&](int step, int buf) {
-        char *As = smem + buf * STEPB, *Ws = As + BM * ROWB;
+    const int nsteps = lda16 / LT_BK;
+    auto stage_a = [&](int step, char *to, int j) {
+        __builtin_amdgcn_global_load_lds((lt_glb_t *)(asrc[j] + step * LT_BK), (lt_lds_t *)(to + (wave * AI + j) * 1024), 16, 0, 0);
+    };
+    auto stage_w = [&](int step, char *to, int j) {
+        __builtin_amdgcn_global_load_lds((lt_glb_t *)(wsrc[j] + min(step * LT_BK, wlim[j])), (lt_lds_t *)(to + BM * ROWB + (wave * WI + j) * 1024), 16, 0, 0);
+    };
+    auto stage = [&](int step, char *to) {
 #pragma unroll
-        for (int j = 0; j < AI; j++)
-            __builtin_amdgcn_global_load_lds((lt_glb_t *)(asrc[j] + step * LT_BK), (lt_lds_t *)(As + (wave * AI + j) * 1024), 16, 0, 0);
+        for (int j = 0; j < AI; j++) stage_a(step, to, j);
 #pragma unroll
-        for (int j = 0; j < WI; j++)
-            __builtin_amdgcn_global_load_lds((lt_glb_t *)(wsrc[j] + min(step * LT_BK, wlim[j])), (lt_lds_t *)(Ws + (wave * WI + j) * 1024), 16, 0, 0);
+        for (int j = 0; j < WI; j++) stage_w(step, to, j);
     };
     const int lc = g ^ swz(i), a_off = (wm * (BM / 2) + i) * ROWB, w_off = (BM + wn * (BN / 2) + i) * ROWB;          // (tile rows start at multiples of 32)
     f32x16v acc[TA][TB];
@@ -207,8 +229,7 @@ __global__ void __launch_bounds__(256, 2) k_lin_tile(LinArgs P, const bf16_t *__
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
     bf16x8v af[2][TA], wf[2][TB];
-    auto frags = [&](int buf, int ks, bf16x8v (&fa)[TA], bf16x8v (&fw)[TB]) {
-        const char *base = smem + buf * STEPB;
+    auto frags = [&](const char *base, int ks, bf16x8v (&fa)[TA], bf16x8v (&fw)[TB]) {
         const int so = ((2 * ks) ^ lc) << 4;
 #pragma unroll
         for (int a = 0; a < TA; a++) fa[a] = *reinterpret_cast<const bf16x8v *>(base + a_off + a * 32 * ROWB + so);
@@ -221,30 +242,69 @@ __global__ void __launch_bounds__(256, 2) k_lin_tile(LinArgs P, const bf16_t *__
 #pragma unroll
             for (int b = 0; b < TB; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[a], fw[b], acc[a][b], 0, 0, 0);
     };
-    const int nsteps = lda16 / LT_BK;
-    stage(0, 0);
-    __syncthreads();
-    frags(0, 0, af[0], wf[0]);
-    for (int step = 0; step + 1 < nsteps; step++) {
-        const int cur = step & 1;
-        stage(step + 1, cur ^ 1);
-#pragma unroll
-        for (int ks = 0; ks < 3; ks++) {
-            frags(cur, ks + 1, af[(ks + 1) & 1], wf[(ks + 1) & 1]);
-            mma(af[ks & 1], wf[ks & 1]);
-        }
+    if constexpr (NB == 2) {
+        stage(0, smem);
         __syncthreads();
-        frags(cur ^ 1, 0, af[0], wf[0]);
-        mma(af[1], wf[1]);
-    }
-    {
-        const int cur = (nsteps - 1) & 1;
+        frags(smem, 0, af[0], wf[0]);
+        for (int step = 0; step + 1 < nsteps; step++) {
+            char *cur = smem + (step & 1) * STEPB, *nxt = smem + (~step & 1) * STEPB;
+            stage(step + 1, nxt);
+#pragma unroll
+            for (int ks = 0; ks < 3; ks++) {
+                frags(cur, ks + 1, af[(ks + 1) & 1], wf[(ks + 1) & 1]);
+                mma(af[ks & 1], wf[ks & 1]);
+            }
+            __syncthreads();
+            frags(nxt, 0, af[0], wf[0]);
+            mma(af[1], wf[1]);
+        }
+        const char *cur = smem + ((nsteps - 1) & 1) * STEPB;
 #pragma unroll
         for (int ks = 0; ks < 3; ks++) {
             frags(cur, ks + 1, af[(ks + 1) & 1], wf[(ks + 1) & 1]);
             mma(af[ks & 1], wf[ks & 1]);
         }
         mma(af[1], wf[1]);
+    } else {
+        static_assert(TA == 1 && TB == 1, "a wave reads one tile of each operand");
+        const unsigned lds0 = (unsigned)(uintptr_t)(lt_lds_t *)smem;
+        unsigned at[4];
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) at[ks] = lds0 + (((2 * ks) ^ lc) << 4);
+        // One step: its own requests have arrived (those of the NB - 2 steps behind it may be under way), everybody's with the barrier, before which every wave has
+        // also read the step before: its buffer takes the step NB - 1 further on.  (The reads and their wait are one block: reads that the compiler sees wait for every
+        // request into LDS, once a round of the buffers at the least.)
+        auto one = [&](int step, int j, auto more) {
+            if constexpr (decltype(more)::value) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NB - 2) * (AI + WI)) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            char *to = smem + (j == 0 ? NB - 1 : j - 1) * STEPB;
+            if constexpr (decltype(more)::value && BM > 32) stage(step + NB - 1, to);
+            const unsigned oa = j * STEPB + a_off, ow = j * STEPB + w_off;
+            bf16x8v fa[4], fw[4];
+            asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %4, %12\n\tds_read_b128 %1, %9\n\tds_read_b128 %5, %13\n\tds_read_b128 %2, %10\n\tds_read_b128 %6, %14\n\t"
+                         "ds_read_b128 %3, %11\n\tds_read_b128 %7, %15\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(fa[0]), "=&v"(fa[1]), "=&v"(fa[2]), "=&v"(fa[3]), "=&v"(fw[0]), "=&v"(fw[1]), "=&v"(fw[2]), "=&v"(fw[3])
+                         : "v"(at[0] + oa), "v"(at[1] + oa), "v"(at[2] + oa), "v"(at[3] + oa), "v"(at[0] + ow), "v"(at[1] + ow), "v"(at[2] + ow), "v"(at[3] + ow) : "memory");
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks], fw[ks], acc[0][0], 0, 0, 0);
+                if constexpr (decltype(more)::value && BM == 32) {          // (the only wave: its requests go out under its products, 4096 columns 16.5 -> 15.4 us)
+                    static_assert(BM > 32 || (AI == 4 && WI == 4), "the requests of a step over its four products");
+                    __builtin_amdgcn_sched_barrier(0);
+                    stage_a(step + NB - 1, to, ks);
+                    stage_w(step + NB - 1, to, ks);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+        // (at least NB steps)
+#pragma unroll
+        for (int j = 0; j < NB - 1; j++) stage(j, smem + j * STEPB);
+        int step = 0, j = 0;
+        for (; step + NB - 1 < nsteps; step++) { one(step, j, std::true_type()); j = j + 1 == NB ? 0 : j + 1; }
+        for (; step < nsteps; step++) { one(step, j, std::false_type()); j = j + 1 == NB ? 0 : j + 1; }
     }
     // every (row, column) of the wave's tile: f(C element's place, value behind the bias)
     auto each = [&](auto f) {
@@ -258,10 +318,26 @@ __global__ void __launch_bounds__(256, 2) k_lin_tile(LinArgs P, const bf16_t *__
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int t = t0 + wm * (BM / 2) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
-                    if (t < P.T) f((size_t)t * P.ldc + n, n, acc[a][b][r] + bv, mv);
+                    if (t < t_end) f((size_t)t * P.ldc + n, n, acc[a][b][r] + bv, mv);
                 }
         }
     };
+    if constexpr (GROUPED) {          // (the rows' scales take the place of the columns')
+#pragma unroll
+        for (int a = 0; a < TA; a++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int t = t0 + wm * (BM / 2) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
+                if (t >= t_end) continue;
+                const float sc = P.row_scale ? P.row_scale[t] : 1.0f;
+#pragma unroll
+                for (int b = 0; b < TB; b++) {
+                    const int n = n0 + wn * (BN / 2) + 32 * b + i;
+                    if (n < P.N) P.C[(size_t)t * P.ldc + n] = acc[a][b][r] * sc;
+                }
+            }
+        return;
+    }
     if (P.act_kind == 2) {
         if (P.C16) each([&](size_t at, int, float v, float mv) { v = fmaxf(v, 0.0f); P.C16[at] = __builtin_bit_cast(bf16_t, (__bf16)(v * v * mv)); });
         else each([&](size_t at, int, float v, float mv) { v = fmaxf(v, 0.0f); P.C[at] = v * v * mv; });
@@ -277,11 +353,13 @@ __global__ void __launch_bounds__(256, 2) k_lin_tile(LinArgs P, const bf16_t *__
     }
 }
 
-template <int BM, int BN>
-void launch_lin_tile(const LinArgs &P, const bf16_t *a16, size_t lda16, hipStream_t s)
+template <int BM, int BN, int NB, bool GROUPED>
+int launch_lin_tile(const LinArgs &P, const bf16_t *a16, size_t lda16, size_t row_tiles, hipStream_t s)
 {
-    const int tm = (P.T + BM - 1) / BM, tn = (P.N + BN - 1) / BN;
-    hipLaunchKernelGGL((k_lin_tile<BM, BN>), dim3((unsigned)tm * (unsigned)tn), dim3(256), 0, s, P, a16, (int)lda16, tm, tn);
+    const int tm = (int)row_tiles, tn = (P.N + BN - 1) / BN;
+    hipLaunchKernelGGL((k_lin_tile<BM, BN, NB, GROUPED>), dim3((unsigned)tm * (unsigned)tn), dim3(BM == 32 ? 64 : 256), 0, s, P, a16, (int)lda16, tm, tn);
+    IFA_LAUNCH_CHECK();
+    return IFA_OK;
 }
 
 // rows of 32-bit values to bfloat16, zero up to ldy (a multiple of 8)
@@ -542,11 +620,33 @@ extern "C" int ifa_linear_bf16_both(const void *w_bf16, size_t rows, size_t cols
     // the largest tile that still gives every compute unit its share of workgroups
     const size_t t128 = (tokens + 127) / 128, n128 = (rows + 127) / 128, n64 = (rows + 63) / 64;
     IFA_REQUIRE(((tokens + 63) / 64) * n64 < (1u << 31), "ifa_linear_bf16_both: too many tiles");
-    if (t128 * n128 >= 384) launch_lin_tile<128, 128>(P, a, lda, s);
-    else if (t128 * n64 >= 256) launch_lin_tile<128, 64>(P, a, lda, s);
-    else launch_lin_tile<64, 64>(P, a, lda, s);
-    IFA_LAUNCH_CHECK();
-    return IFA_OK;
+    const size_t t64 = (tokens + 63) / 64;
+    if (t128 * n128 >= 384) return launch_lin_tile<128, 128, 2, false>(P, a, lda, t128, s);
+    if (t128 * n64 >= 256) return launch_lin_tile<128, 64, 2, false>(P, a, lda, t128, s);
+    if (t64 * n64 > LT_DEEP || lda < 4 * LT_BK) return launch_lin_tile<64, 64, 2, false>(P, a, lda, t64, s);
+    if (t64 * n64 > LT_SMALL || lda < 8 * LT_BK) return launch_lin_tile<64, 64, 4, false>(P, a, lda, t64, s);
+    return launch_lin_tile<32, 32, 8, false>(P, a, lda, (tokens + 31) / 32, s);
+}
+
+// ifa_linear_bf16w_grouped over bfloat16 rows (as ifa_linear_bf16_both reads them), tiles of at most tile_rows = 64 or 128 rows of one group
+int ifa_linear_bf16_grouped(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, const int *a_rows_dev, const int *tile_map_dev, const int *n_tiles_dev,
+                            size_t max_tiles, int tile_rows, const void *row_scale_f32, void *c_f32, size_t ldc, ifa_stream stream)
+{
+    IFA_REQUIRE(w_bf16 && a_bf16 && c_f32 && tile_map_dev && n_tiles_dev, "linear_bf16_grouped: null pointer");
+    IFA_REQUIRE(rows > 0 && cols >= (size_t)LT_BK && cols % 8 == 0 && max_tiles > 0 && lda % 64 == 0 && lda >= cols && lda - cols < 64 && ldc >= rows
+                && (tile_rows == 64 || tile_rows == 128) && rows < (1u << 30) && cols < (1u << 30) && (((uintptr_t)a_bf16 | (uintptr_t)w_bf16) & 15) == 0,
+                "linear_bf16_grouped: bad shape (%zu x %zu, lda %zu)", rows, cols, lda);
+    LinArgs P;
+    memset(&P, 0, sizeof(P));
+    P.W = (const bf16_t *)w_bf16; P.C = (float *)c_f32; P.N = (int)rows; P.K = (int)cols; P.ldc = (int)ldc; P.alpha = 1.0f;
+    P.tile_map = tile_map_dev; P.n_tiles = n_tiles_dev; P.a_rows = a_rows_dev; P.row_scale = (const float *)row_scale_f32;
+    const bf16_t *a = (const bf16_t *)a_bf16;
+    const size_t n64 = (rows + 63) / 64;
+    IFA_REQUIRE(max_tiles * n64 < (1u << 31), "linear_bf16_grouped: too many tiles");
+    hipStream_t s = ifa_s(stream);
+    if (tile_rows == 128) return launch_lin_tile<128, 128, 2, true>(P, a, lda, max_tiles, s);
+    if (max_tiles * n64 > LT_DEEP || lda < 4 * LT_BK) return launch_lin_tile<64, 64, 2, true>(P, a, lda, max_tiles, s);
+    return launch_lin_tile<64, 64, 4, true>(P, a, lda, max_tiles, s);
 }
 
 extern "C" int ifa_linear_bf16w_act(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *bias_bf16, int act,

@@ -14,6 +14,7 @@
 #include "ifa_host.h"
 #include "ifa_f32_common.h"
 #include "inferflow_amd.h"
+#include "ifa_rows_fused.h"
 
 using namespace ifa32;
 
@@ -307,11 +308,11 @@ __global__ void __launch_bounds__(256) k_moe_down_rows(const float *__restrict__
 }
 
 // ONE workgroup: pairs (row, choice) sorted by expert.  a_rows[pos] = row of the pair at sorted place pos, pair_pos[p] = place of pair p
-// (-1: identity), w_sorted[pos] = its weight, tile_map = tiles of at most 64 places of one expert, *n_tiles.  The place of a pair inside
+// (-1: identity), w_sorted[pos] = its weight, tile_map = tiles of at most tile_rows places of one expert, *n_tiles.  The place of a pair inside
 // its expert's range comes from an LDS counter: the order there may differ from run to run, the values computed per pair do not.
 __global__ void __launch_bounds__(1024) k_moe_sort(const int *__restrict__ idx, const float *__restrict__ wgt, int n_pairs, int experts, int top,
                                                    int *__restrict__ a_rows, int *__restrict__ pair_pos, float *__restrict__ w_sorted,
-                                                   int *__restrict__ tile_map, int *__restrict__ n_tiles)
+                                                   int *__restrict__ tile_map, int *__restrict__ n_tiles, int tile_rows)
 {
     extern __shared__ int cnt[];           // [experts] counts, then cursors; [experts + 1] offsets
     int *off = cnt + experts;
@@ -323,7 +324,7 @@ __global__ void __launch_bounds__(1024) k_moe_sort(const int *__restrict__ idx, 
         int o = 0, nt = 0;
         for (int e = 0; e < experts; e++) {
             off[e] = o;
-            for (int r = 0; r < cnt[e]; r += 64) { tile_map[3 * nt] = e; tile_map[3 * nt + 1] = o + r; tile_map[3 * nt + 2] = min(64, cnt[e] - r); nt++; }
+            for (int r = 0; r < cnt[e]; r += tile_rows) { tile_map[3 * nt] = e; tile_map[3 * nt + 1] = o + r; tile_map[3 * nt + 2] = min(tile_rows, cnt[e] - r); nt++; }
             o += cnt[e];
             cnt[e] = 0;
         }
@@ -483,18 +484,29 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
         IFA_LAUNCH_CHECK();
         return IFA_OK;
     }
-    const size_t max_tiles = moe_tiles_max(rows, top, experts);
+    // gated experts, products over bfloat16 rows where the activations are rounded anyway: h once (in the place of the down products' output, which is not there yet), the experts'
+    // activations by the launch that forms them; row tiles of 128 where an expert has several on average
+    const size_t lda_h = ((size_t)width + 63) & ~(size_t)63, lda_f = ((size_t)ff + 63) & ~(size_t)63;
+    const bool in16 = gated && !ops32 && width % 8 == 0 && width >= 64 && ff % 8 == 0 && ff >= 64 && lda_f <= 2 * (size_t)ff && lda_h <= 2 * (size_t)width * top
+                      && (((uintptr_t)up_bf16 | (uintptr_t)down_bf16) & 15) == 0;
+    const int tile_rows = in16 && pairs >= (size_t)256 * experts ? 128 : 64;
+    const size_t max_tiles = (pairs + tile_rows - 1) / tile_rows + (size_t)experts;
     IFA_REQUIRE(max_tiles < 65536, "%s: %zu rows x %d choices exceed one step", who, rows, top);
     hipLaunchKernelGGL(k_moe_sort, dim3(1), dim3(1024), (size_t)(2 * experts + 1) * 4, s, idx_dev, (const float *)wgt_f32, (int)pairs, experts, top, a_rows, pair_pos, w_sorted,
-                       tile_map, n_tiles);
+                       tile_map, n_tiles, tile_rows);
     IFA_LAUNCH_CHECK();
     int rc;
-    if (gated) {
+    if (in16) {
+        bf16_t *h16 = (bf16_t *)yp, *a16 = (bf16_t *)actb;
+        if ((rc = ifa_rows_to_bf16(h_f32, ldh, rows, (size_t)width, h16, lda_h, stream))) return rc;
+        if ((rc = ifa_linear_bf16_grouped(up_bf16, (size_t)2 * ff, (size_t)width, h16, lda_h, a_rows, tile_map, n_tiles, max_tiles, tile_rows, nullptr, gub, (size_t)2 * ff, stream))) return rc;
+        if ((rc = ifa_glu_to_bf16(glu_kind, limit, gub, (size_t)2 * ff, pairs, (size_t)ff, nullptr, 0, a16, lda_f, stream))) return rc;
+        if ((rc = ifa_linear_bf16_grouped(down_bf16, (size_t)width, (size_t)ff, a16, lda_f, nullptr, tile_map, n_tiles, max_tiles, tile_rows, w_sorted, yp, (size_t)width, stream))) return rc;
+    } else if (gated) {
         if ((rc = ifa_linear_bf16w_grouped(up_bf16, (size_t)2 * ff, (size_t)width, experts, h_f32, ldh, a_rows, tile_map, n_tiles, max_tiles, nullptr, 0, ops32, gub, (size_t)2 * ff, stream))) return rc;
         if ((rc = ifa_glu_ex_f32(glu_kind, limit, gub, (size_t)2 * ff, pairs, (size_t)ff, nullptr, 0, actb, (size_t)ff, stream))) return rc;
-    } else
-    if ((rc = ifa_linear_bf16w_grouped(up_bf16, (size_t)ff, (size_t)width, experts, h_f32, ldh, a_rows, tile_map, n_tiles, max_tiles, nullptr, 1, ops32, actb, (size_t)ff, stream))) return rc;
-    if ((rc = ifa_linear_bf16w_grouped(down_bf16, (size_t)width, (size_t)ff, experts, actb, (size_t)ff, nullptr, tile_map, n_tiles, max_tiles, w_sorted, 0, ops32, yp, (size_t)width, stream))) return rc;
+    } else if ((rc = ifa_linear_bf16w_grouped(up_bf16, (size_t)ff, (size_t)width, experts, h_f32, ldh, a_rows, tile_map, n_tiles, max_tiles, nullptr, 1, ops32, actb, (size_t)ff, stream))) return rc;
+    if (!in16 && (rc = ifa_linear_bf16w_grouped(down_bf16, (size_t)width, (size_t)ff, experts, actb, (size_t)ff, nullptr, tile_map, n_tiles, max_tiles, w_sorted, 0, ops32, yp, (size_t)width, stream))) return rc;
     hipLaunchKernelGGL(k_moe_combine, dim3(ifa_cdiv((size_t)width, 256), (unsigned)rows), dim3(256), 0, s, h, ldh, width, top, pair_pos, (const float *)wgt_f32, yp,
                        accumulate ? 1 : 0, (float *)y_f32, ldy);
     IFA_LAUNCH_CHECK();

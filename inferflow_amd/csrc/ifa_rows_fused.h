@@ -37,3 +37,10 @@ int ifa_mix_row(const IfaMixRow &M, int *nsplit, ifa_stream stream);
 int ifa_delta_row_prep(const float *x, size_t ldx, int channels, int taps, const ifa32::bf16_t *w, const ifa_seq_desc *seqs, const int *row_seq, size_t rows, void *const *slot_base,
                        size_t state_off, int norm_cols, int group_dim, float l2_eps, int scale_cols, float scale, float *y, size_t ldy, const float *b, const float *a, int heads,
                        const ifa32::bf16_t *a_log, const ifa32::bf16_t *dt_bias, float *beta, float *decay, ifa_stream stream);
+
+// grouped products over bfloat16 rows (csrc/ifa_linear_bf16.hip): see ifa_linear_bf16w_grouped
+int ifa_linear_bf16_grouped(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, const int *a_rows_dev, const int *tile_map_dev, const int *n_tiles_dev,
+                            size_t max_tiles, int tile_rows, const void *row_scale_f32, void *c_f32, size_t ldc, ifa_stream stream);
+// ifa_glu_ex_f32 whose output only products read: bfloat16 rows, zero up to ldo (a multiple of 8; csrc/ifa_ops_f32.hip)
+int ifa_glu_to_bf16(int kind, float limit, const void *gate_up_f32, size_t ld, size_t rows, size_t cols, const void *row_gate_f32, size_t ldg, void *out_bf16, size_t ldo,
+                    ifa_stream stream);

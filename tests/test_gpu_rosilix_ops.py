@@ -314,6 +314,24 @@ def test_products_of_prompts_in_every_tile(T, N, K):
     assert near(out.cpu().numpy(), torch.nn.functional.gelu(z).numpy(), 1e-5)
 
 
+@pytest.mark.parametrize("T,N,K", [(9, 31, 456), (33, 65, 512), (70, 97, 1000), (129, 2900, 200), (130, 2900, 328), (600, 1100, 72), (257, 2080, 520)])
+def test_products_of_prompts_with_steps_under_way(T, N, K):
+    """the tiles of few workgroups: 32 x 32 with at least eight steps, 64 x 64 with at least four, inner sizes on both sides of these counts and of a step's border; the
+    same sums as the product that rounds its activations itself"""
+    rng = np.random.default_rng(T + N + K)
+    Wm, A, b = bf16_round(rng.standard_normal((N, K))), bf16_round(rng.standard_normal((T, K))), bf16_round(rng.standard_normal(N))
+    wd, ad, bd, L, ld = devbf(Wm), dev32(A), devbf(b), capi(), (K + 63) // 64 * 64
+    a16 = torch.full((T, ld), -1, dtype=torch.int16, device="cuda")
+    out, other = (torch.full((T, N + 2), 7.0, dtype=torch.float32, device="cuda") for _ in range(2))
+    ia.check(L.ifa_rows_to_bf16(p(ad), K, T, K, p(a16), ld, None))
+    ia.check(L.ifa_linear_bf16_both(p(wd), N, K, p(a16), ld, T, p(bd), None, 1.0, 0, 0, p(out), None, N + 2, 0, 0, None))
+    ia.check(L.ifa_linear_bf16w(p(wd), N, K, p(ad), K, T, p(bd), None, 1.0, 0, 0, p(other), N + 2, 0, 0, None)); sync()
+    got = out.cpu().numpy()
+    # fp32 sums of exact products: at most K roundings of half a unit of the sum of the magnitudes
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(orc.f64(A)) @ np.abs(orc.f64(Wm)).T + np.abs(orc.f64(b)))
+    assert np.all(np.abs(got[:, :N] - (orc.f64(A) @ orc.f64(Wm).T + orc.f64(b))) <= bound) and np.all(got[:, N:] == 7.0) and torch.equal(out, other)
+
+
 def test_products_of_prompts_decline_bad_arguments():
     L = capi()
     z = torch.zeros(1 << 16, dtype=torch.float32, device="cuda")

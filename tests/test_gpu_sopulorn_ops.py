@@ -262,3 +262,29 @@ def test_gated_experts_in_rows_and_grouped(T, W, F, E, top):
             ref = want + (y0[:, :W] if acc else 0)
             t_ = tol if T > 8 else 2e-5          # (steps of at most 8 rows keep fp32 activations in both modes)
             assert np.abs(y.cpu().numpy()[:, :W] - ref).max() < t_ * max(1.0, np.abs(want).max()), (ops32, acc)
+
+
+@pytest.mark.parametrize("T,W,F,E,top", [(9, 64, 72, 6, 2), (40, 264, 320, 5, 2), (300, 136, 264, 2, 2), (700, 72, 64, 3, 1), (130, 328, 72, 1, 1)])
+def test_gated_experts_over_bfloat16_rows(T, W, F, E, top):
+    """row tiles of 64 and 128, few and many steps, inner sizes that are no multiple of a step: h and the activations rounded to bfloat16 once"""
+    rng = np.random.default_rng(T + W + F)
+    h = bf16_round(rng.standard_normal((T, W)))
+    gu = bf16_round(rng.standard_normal((E, 2 * F, W)) / np.sqrt(W)); dn = bf16_round(rng.standard_normal((E, W, F)) / np.sqrt(F))
+    idx = np.stack([rng.permutation(E)[:top] for _ in range(T)]).astype(np.int32)
+    wgt = rng.uniform(0.1, 1.0, (T, top)).astype(np.float32)
+    want, bound = np.zeros((T, W)), np.zeros((T, W))
+    for e in range(E):
+        g, u = h.astype(np.float64) @ gu[e, :F].astype(np.float64).T, h.astype(np.float64) @ gu[e, F:].astype(np.float64).T
+        a, d = g / (1 + np.exp(-g)) * u, dn[e].astype(np.float64).T
+        w = np.where(idx == e, wgt, 0).sum(1, keepdims=True)
+        want += w * (a @ d)
+        bound += w * (np.abs(a) @ np.abs(d) * 2.0 ** -8 + (np.abs(g) + np.abs(u) + 1) @ np.abs(d) * 2.0 ** -18)          # an activation to 8 bits: half a unit is up to 2^-8 of it; the 32-bit sums in front
+    L = capi()
+    nb = L.ifa_moe_workspace_bytes(T, top, W, 3 * F, E)
+    ws = torch.zeros((nb + 15) // 4, dtype=torch.float32, device="cuda")
+    y = torch.full((T, W + 1), 7.0, dtype=torch.float32, device="cuda")
+    ia.check(L.ifa_moe_experts_gated_f32(p(dev32(h)), W, T, W, F, E, top, p(devbf(gu.reshape(E * 2 * F, W))), p(devbf(dn.reshape(E * W, F))), p(devi(idx)),
+                                         p(dev32(wgt)), 0, p(ws), nb, p(y), W + 1, 0, None)); sync()
+    got = y.cpu().numpy()
+    assert np.all(np.abs(got[:, :W] - want) <= bound) and np.all(got[:, W:] == 7.0)
+
