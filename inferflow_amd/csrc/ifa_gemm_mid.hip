@@ -53,9 +53,6 @@ constexpr int MD_THREADS = IFA_MID_LOADERS ? 2 * MD_NT : MD_NT;     // launched 
 #ifndef IFA_MID_ABL
 #define IFA_MID_ABL 0
 #endif
-#ifndef IFA_MID_PF
-#define IFA_MID_PF 2        // 16-column groups of lead of the activation fragment reads (1: the first form, one group)
-#endif
 #ifndef IFA_MID_WAUX
 #define IFA_MID_WAUX 0       // cache policy of the weight requests (2 = non-temporal)
 #endif
@@ -65,10 +62,11 @@ __device__ __forceinline__ md_u4 md_lds_b128(uint32_t addr) { md_u4 v; asm volat
 __device__ __forceinline__ uint32_t md_lds_b32(uint32_t addr) { uint32_t v; asm volatile("ds_read_b32 %0, %1" : "=v"(v) : "v"(addr)); return v; }
 
 // EPI: GM_PLAIN | GM_RESIDUAL | GM_GLU (a weight tile = 64 rows of w1 and the same 64 rows of w3).  KS: parts of K (workgroups per
-// tile).  NS: stages of the ring.  TA: 32-token accumulator tiles of a wave -- the tile is 32 TA tokens x 128 weight rows (TA = 8 from 512
-// tokens on: every dequantised weight and every request of the weight stream serves twice the products).
-template <int EPI, int KS, int NS, int TA>
-__global__ void __launch_bounds__(MD_THREADS) k_gemm_mid(const GmArgs P, const BigGeo G)
+// tile).  NS: stages of the ring.  TA: 32-token accumulator tiles of a wave -- the tile is 32 TA tokens x 128 weight rows (TA = 2 up to 64 tokens:
+// half of the products, fragment reads, activation requests and exchanged sums of a 128-row tile whose lower half repeats a row -- 37 tokens 4.67 -> 3.83 ms,
+// the same bits; TA = 8: a measurement setting).  LEAD: 16-column groups that the fragments are requested ahead.
+template <int EPI, int KS, int NS, int TA, int LEAD>
+__global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_gemm_mid(const GmArgs P, const BigGeo G)
 {
     constexpr int BM = 32 * TA, BN = MD_BN, BK = MD_BK, NW = MD_NW, NT = MD_NT, ROWB = BK * 2;
     constexpr int MD_A_BYTES = md_a_bytes(TA), MD_STAGE = md_stage(TA), MD_VM = md_vm(TA), XP = TA;      // XP: activation pieces (8 token rows) a wave requests per stage
@@ -219,7 +217,6 @@ __global__ void __launch_bounds__(MD_THREADS) k_gemm_mid(const GmArgs P, const B
         // lgkmcnt(0) at the end of every group -- four waves read 64 KB of LDS per step, 512 cycles of the LDS pipe, as long as the step's
         // MFMAs -- so the waits are counted (LDS returns in order; nothing else of this loop counts on lgkmcnt; the counter holds 15) and
         // the pipe never drains.  TA = 8: a group's eight MFMAs cover the next group's reads, one group of lead.
-        constexpr int LEAD = (IFA_MID_PF >= 2 && TA <= 4) ? 2 : 1;
         if constexpr (LEAD == 2) {
 #pragma unroll
             for (int a = 0; a < TA; a++) fa[1][a] = md_lds_b128(a_off + sb + (uint32_t)(a * 32 * ROWB) + (uint32_t)(((2) ^ lc) << 4));
@@ -294,9 +291,9 @@ __global__ void __launch_bounds__(MD_THREADS) k_gemm_mid(const GmArgs P, const B
                 if (ks + LEAD < 4 && 2 * a + 1 < TA) { frag(ks + LEAD, 2 * a); frag(ks + LEAD, 2 * a + 1); }
                 if (ks < 3) {
                     if (a == 0) dq_a(ks + 1);
-                    else if (a == TA / 4) dq_b();
-                    else if (a == TA / 2) dq_c();
-                    else if (a == 3 * TA / 4) fbn = dq_d();
+                    if (a == TA / 4) dq_b();
+                    if (a == TA / 2) dq_c();
+                    if (a == 3 * TA / 4) fbn = dq_d();
                     if constexpr (!LD) { if (ks * TA + a < XP + 2) issue_piece(nstep, nslot, ks * TA + a); }
                 }
             }
@@ -343,7 +340,7 @@ __global__ void __launch_bounds__(MD_THREADS) k_gemm_mid(const GmArgs P, const B
     if constexpr (KS > 1) {
         char *pt = reinterpret_cast<char *>(G.part) + (size_t)wg * ((size_t)KS * NU * NT * 16);
         const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(pt, 0, KS * NU * NT * 16, 0x00020000);
-        unsigned *arrive = G.flags + 2 * wg, *done = arrive + 1;
+        unsigned *arrive = G.flags + 2 * wg;
 #pragma unroll
         for (int u = 0; u < NU; u++) {
             if (u / UB == kz) continue;                  // (wave-uniform)
@@ -388,16 +385,7 @@ __global__ void __launch_bounds__(MD_THREADS) k_gemm_mid(const GmArgs P, const B
                 acc[u >> 2][4 * (u & 3) + e] = sf;
             }
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        // the part that is last to finish reading puts both counters back to zero (the next launch on this stream finds them clean)
-        if (tid == 0) {
-            const unsigned d = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (d == (unsigned)(KS - 1)) {
-                __hip_atomic_store(arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (the parts' values are in: the count behind the epilogue says so)
     }
 
     // ---- epilogue (k_gemm_big's arithmetic, this part's rows): products -> F16 (+ bias) -> an LDS tile (rows padded by 64 bytes) ->
@@ -454,6 +442,18 @@ __global__ void __launch_bounds__(MD_THREADS) k_gemm_mid(const GmArgs P, const B
             if (tok < T && n < N) *reinterpret_cast<md_h8 *>(Yo + (size_t)tok * ldo + vrow0 + n) = y;
         }
     }
+    if constexpr (KS > 1) {
+        // the part that is last to have read the others' sums puts both counters back to zero (the next launch on this stream finds them clean): behind the output,
+        // whose stores do not wait for the counter's way to memory and back
+        if (tid == 0) {          // (every thread's reads: the epilogue's barriers)
+            unsigned *arrive = G.flags + 2 * wg, *done = arrive + 1;
+            const unsigned d = __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (d == (unsigned)(KS - 1)) {
+                __hip_atomic_store(arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
     if (trc) trc[4] = wall_clock64();
 }
 
@@ -475,8 +475,8 @@ bool gemm_mid_ok(int w_dtype, const GmArgs &P, int epi)
     return true;
 }
 
-template <int EPI, int KS, int NS, int TA>
-static int md_run(const GmArgs &P, BigGeo G, int tn_count, hipStream_t s)
+template <int EPI, int KS, int NS, int TA, int LEAD>
+static int md_run_lead(const GmArgs &P, BigGeo G, int tn_count, hipStream_t s)
 {
     if constexpr (KS > 1) {
         G.err = wait_err_word();
@@ -487,7 +487,7 @@ static int md_run(const GmArgs &P, BigGeo G, int tn_count, hipStream_t s)
         G.flags = (unsigned *)scratch; G.part = (unsigned long long *)((char *)scratch + SPLITK_FLAG_BYTES_H);
     }
     const size_t smem = std::max((size_t)NS * md_stage(TA), (size_t)(32 * TA) * (MD_BN * 2 + 64));
-    auto kern = k_gemm_mid<EPI, KS, NS, TA>;
+    auto kern = k_gemm_mid<EPI, KS, NS, TA, LEAD>;
     static std::atomic<uint64_t> attr_set{0};
     int dev = 0;
     (void)hipGetDevice(&dev);
@@ -528,6 +528,16 @@ static int md_run(const GmArgs &P, BigGeo G, int tn_count, hipStream_t s)
 #define IFA_MID_NS 3
 #endif
 
+// 128-token tiles, two workgroups on a compute unit where there are that many: 120 registers with one group of lead; 136 with two, which keep the second workgroup out.  A step of
+// a lone workgroup takes 0.54 us, of two together 0.84: 384 / 512 / 768 tokens 9.83 -> 9.45, 10.70 -> 10.24, 15.81 -> 15.42 ms.  A lone one needs the lead (96 tokens 4.40 -> 4.49
+// without).
+template <int EPI, int KS, int NS, int TA>
+static int md_run(const GmArgs &P, const BigGeo &G, int tn_count, hipStream_t s)
+{
+    if constexpr (TA == 4) { if ((long long)G.tiles_m * tn_count * KS <= md_num_cus()) return md_run_lead<EPI, KS, NS, TA, 2>(P, G, tn_count, s); }
+    return md_run_lead<EPI, KS, NS, TA, TA == 2 ? 2 : 1>(P, G, tn_count, s);
+}
+
 template <int EPI, int TA>
 static int md_launch(const GmArgs &P, hipStream_t s)
 {
@@ -540,13 +550,11 @@ static int md_launch(const GmArgs &P, hipStream_t s)
     for (int i = P.nsets; i < 3; i++) G.tile0[i] = 1 << 30;
     G.tiles_m = (P.T + MD_BM - 1) / MD_BM; G.K = P.nblk * 32; G.tn0 = 0;
     const int ksteps = G.K / MD_BK;
-    // parts of K: the most that still put ONE workgroup on a CU (two fit -- LDS, registers -- but a grid between one and two per CU
-    // ends when the doubly loaded CUs do: wq | wk | wv of 128 tokens, 96 tiles: 384 workgroups 32.3 us, 192 workgroups 27; of 256
-    // tokens, 192 tiles: one part beats two; wo / w2 of one token tile, 32 tiles: eight parts, 256 workgroups, beat four -- 128 tokens
-    // 5.34 -> 4.86 ms in all, profiles/r06_prefill_mid_parts.log), every part >= MINS steps
+    // parts of K: the most that still put ONE workgroup on a CU.  (Two fit, but parts cost: the exchange of their sums is 4.5 to 8 us of a launch, and with two workgroups on
+    // a CU it is longer than what the shorter loops give -- wo / w2 of 192 and 512 tokens as 512 workgroups: 6.21 -> 7.27 and 9.97 -> 10.5 ms in all; the gated pair of 96
+    // tokens as 344 instead of 172: 4.40 -> 4.64; 37 tokens: the same.)  Every part >= MINS steps
     static const bool two_per_cu = getenv("IFA_MID_TWO_PER_CU") != nullptr;      // (measurement: the first form's limit)
-    // (the gated pair keeps two per CU: 172 tiles of one token tile as 344 workgroups 45.7 us, as 172 workgroups 50.5)
-    const long long tiles = (long long)G.tiles_m * tn_count, cap = ((two_per_cu || EPI == GM_GLU) ? 2ll : 1ll) * md_num_cus();
+    const long long tiles = (long long)G.tiles_m * tn_count, cap = (two_per_cu ? 2ll : 1ll) * md_num_cus();
     static const bool no_glu_split = getenv("IFA_MID_NO_GLU_SPLIT") != nullptr;      // (measurement: the gated pair as ONE part of K, like k_gemm_big's -- bit-identical products)
     const bool may = !P.no_waits && waits_enabled() && !(EPI == GM_GLU && no_glu_split);
     int rc = 1;
@@ -579,6 +587,11 @@ int gemm_mid(const GmArgs &P, int epi, hipStream_t s)
         if (epi == GM_PLAIN) return md_launch<GM_PLAIN, 8>(P, s);
         if (epi == GM_RESIDUAL) return md_launch<GM_RESIDUAL, 8>(P, s);
         return md_launch<GM_GLU, 8>(P, s);
+    }
+    if (force_ta == 2 || (!force_ta && P.T <= 64)) {      // (65 .. 192 tokens: the same time either way)
+        if (epi == GM_PLAIN) return md_launch<GM_PLAIN, 2>(P, s);
+        if (epi == GM_RESIDUAL) return md_launch<GM_RESIDUAL, 2>(P, s);
+        return md_launch<GM_GLU, 2>(P, s);
     }
     if (epi == GM_PLAIN) return md_launch<GM_PLAIN, 4>(P, s);
     if (epi == GM_RESIDUAL) return md_launch<GM_RESIDUAL, 4>(P, s);

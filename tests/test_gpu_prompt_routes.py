@@ -52,6 +52,21 @@ def test_short_prompt_large_tile_route_agrees_with_the_op_by_op_layer(T):
     wk.close()
 
 
+@pytest.mark.parametrize("T", [33, 47, 63, 64])
+def test_prompts_in_64_token_tiles_agree_with_the_128_token_tiles(T):
+    """up to 64 tokens a tile of the mid-length products holds 64 rows: the products and their sums are those of the 128-row tile, which 65 tokens take, so a row is
+    off by no more than one that the other routes (attention and head by prompt length) leave"""
+    wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=160, layers=2, vocab=2000)
+    wk.set_option("prefill_chunk", 0)
+    toks = np.random.default_rng(T).integers(3, s["vocab"], 65).astype(np.int32)
+    short, long_ = _rows(wk, toks[:T], s["vocab"])[1], _rows(wk, toks, s["vocab"])[1][:T]
+    for a, b in zip(short, long_):
+        ok, why = _agree(a, b)
+        assert ok, why
+    print("T=%d rows that differ in a bit: %d" % (T, sum(not np.array_equal(a, b) for a, b in zip(short, long_))))
+    wk.close()
+
+
 @pytest.mark.parametrize("T", [40, 64, 128])
 def test_short_prompt_routes_match_the_oracle(T):
     """... and against the ORACLE (the reference's T > 1 rule: F16 activations x dequantised weights, fp32 sums), not only against each
