@@ -644,18 +644,21 @@ __global__ void __launch_bounds__(256) k_dec_attn(const half_t *pq, const uint8_
 // ------------------------------------------------------------ long contexts: keys split over workgroups
 // k_dec_attn keeps one workgroup per head, which is latency-optimal for a few hundred keys but reads the whole
 // K/V history of a head through ONE compute unit (4K keys: ~190 us per layer).  Past a threshold the decode step
-// uses three kernels instead, with the SAME rounding points (S and P are half, global max and sum):
+// uses two kernels instead, with the SAME rounding points (S and P are half, global max and sum):
 //   k_dec_attn_scores  (head, split): RoPE, KV store of the new row, S_j = half(alpha q.k_j) for its keys -> workspace,
-//                                      local maximum
-//   k_dec_attn_pv      (head, split): global max, the full-row sum of exp (recomputed per split: a few thousand
-//                                      expf), P_j = half(half(e_j) * 1/sum) for its keys, partial P.V in fp32
-//   k_dec_attn_combine (head)       : sum of the partial outputs in split order -> half
-constexpr int DEC_ATTN_MAX_SPLITS = 32;      // splits per head are chosen per decode call from the context it will reach (8 / 16 / 32)
+//                                      their maximum and the sum of exp(S_j - maximum)
+//   k_dec_attn_pv      (head, split): global max and sum from the splits', P_j = half(half(e_j) * 1/sum) for its keys, partial P.V in fp32;
+//                                      the workgroup of a head that is done last (a counter per head: nobody waits) adds the partial outputs up in split order -> half
+// Bound by the chains of a pass behind each launch, not by the bytes (8-bit cache of 2900 keys: 25 MB a layer, 5 us).  As three kernels -- every split summed the whole
+// row's exponentials again, the outputs were added up by a launch of their own -- 8.3 + 9.9 + 5.0 us a layer; a token at 600 / 2900 / 6000 keys 1591 -> 1573, 1896 -> 1831,
+// 2191 -> 2074 us (8-bit cache).  Twice the splits for the scores alone: 1858 at 2900.
+constexpr int DEC_ATTN_MAX_SPLITS = 32;      // splits per head are chosen per decode call from the context it will reach
 
 struct DecAttnSplitWs {
     half_t *S;        // [heads][max_ctx]
-    float *lmax;      // [heads][nsplits]
+    float *ml;        // [heads][nsplits][2]: maximum, sum of exponentials
     float *opart;     // [heads][nsplits][head_dim]
+    unsigned *count;  // [heads]: splits whose values are done; 0 between launches
     int nsplits;      // <= DEC_ATTN_MAX_SPLITS
 };
 
@@ -671,7 +674,7 @@ __global__ void __launch_bounds__(256) k_dec_attn_scores(const DecAttnParams P, 
     __shared__ __attribute__((aligned(16))) half_t qs[HD];
     __shared__ __attribute__((aligned(16))) half_t kn[HD];
     __shared__ __attribute__((aligned(16))) half_t vn[HD];
-    __shared__ float red[4];
+    __shared__ float red[4], red2[4];
     const int h = blockIdx.x, sidx = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int pos = *(const __attribute__((address_space(4))) int *)(P.state + 1), n_ctx = pos + 1;      // (scalar load: see k_dec_attn)
     int j0, j1; dec_split_range(n_ctx, ws.nsplits, sidx, j0, j1);
@@ -769,7 +772,7 @@ __global__ void __launch_bounds__(256) k_dec_attn_scores(const DecAttnParams P, 
     for (int i = 0; i < HD / 8; i++) qreg[i] = *reinterpret_cast<const half8_t *>(qs + 8 * i);
     const float alpha = 1.0f / sqrtf((float)HD) / P.kq_scale;
     const float mk = P.alibi ? alibi_slope(h + P.alibi_base, P.alibi_total) : 0.0f;
-    float lmax = -INFINITY;
+    float lmax = -INFINITY, lsum = 0.0f;
     // F16 cache: a lane's key row (HD halfs) is requested COALESCED -- a wave request covers 64 / (HD/8) whole rows -- and
     // turned through LDS so that every lane then holds its own key's row: one key per lane with its own 16-byte requests
     // touched 64 rows per request (14 us per layer at 4096 keys).  The dot product below is unchanged (fp32 fma in d order).
@@ -844,30 +847,29 @@ __global__ void __launch_bounds__(256) k_dec_attn_scores(const DecAttnParams P, 
         half_t sv = f2h(alpha * c);
         if (P.alibi) { float a = (float)j * mk; sv = f2h(a + h2f(sv)); }
         ws.S[(size_t)h * P.max_ctx + j] = sv;
-        lmax = fmaxf(lmax, P.kq_scale * h2f(sv));
+        // the thread's own maximum and sum so far (a new maximum scales the sum: at most a key in 256 of a thread's)
+        const float sf = P.kq_scale * h2f(sv), mn = fmaxf(lmax, sf);
+        lsum = (lmax == mn ? lsum : lsum * expf(lmax - mn)) + expf(sf - mn);
+        lmax = mn;
     }
-    lmax = wave_max(lmax);
-    if (lane == 0) red[wave] = lmax;
+    const float wm = wave_max(lmax);
+    if (lane == 0) red[wave] = wm;
     __syncthreads();
-    if (tid == 0) ws.lmax[h * ws.nsplits + sidx] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const float bm = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    lsum = wave_sum(lsum > 0.0f ? lsum * expf(lmax - bm) : lsum);          // (0: a thread without keys; NaN stays)
+    if (lane == 0) red2[wave] = lsum;
+    __syncthreads();
+    if (tid == 0) { float *ml = ws.ml + 2 * (h * ws.nsplits + sidx); ml[0] = bm; ml[1] = ((red2[0] + red2[1]) + red2[2]) + red2[3]; }
 }
-
-// Round 6 (second session): the same sums in the same order, fewer memory round trips.  The kernel was a chain of dependent requests --
-// the full-row sum walked S with one 2-byte load per thread and iteration (17 trips at 4096 keys), the P.V loop kept four V rows per
-// thread in flight (five trips per 320-key split), the Q8 loop one key -- 21 us per layer at 4096 keys for 33 MB of V (1.6 TB/s).  Now the
-// score row is staged through LDS in 16-byte pieces, 4096 keys at a time (thread t still adds keys t, t + 256, ... in ascending order),
-// and the V rows of the next eight keys of a thread are requested before the current eight are multiplied.
-constexpr int DEC_PV_STAGE = 4096;      // keys of the score row staged per pass (multiple of 256)
 
 template <int HD, bool Q8>
 __global__ void __launch_bounds__(256) k_dec_attn_pv(const DecAttnParams P, const DecAttnSplitWs ws)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int DG = HD / 8, NSPLIT = 256 / DG;
-    float *red = reinterpret_cast<float *>(smem);                    // [8]
-    float *opart = red + 8;                                          // [NSPLIT][HD]
-    half_t *Sst = reinterpret_cast<half_t *>(opart + NSPLIT * HD);   // [DEC_PV_STAGE + 8] staged piece of the score row
-    half_t *Pl = Sst + DEC_PV_STAGE + 8;                             // this split's probabilities
+    float *opart = reinterpret_cast<float *>(smem);                  // [NSPLIT][HD]
+    half_t *Pl = reinterpret_cast<half_t *>(opart + NSPLIT * HD);    // this split's probabilities
+    __shared__ int last;
     const int h = blockIdx.x, sidx = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int pos = *(const __attribute__((address_space(4))) int *)(P.state + 1), n_ctx = pos + 1;      // (scalar load: see k_dec_attn)
     int j0, j1; dec_split_range(n_ctx, ws.nsplits, sidx, j0, j1);
@@ -901,34 +903,11 @@ __global__ void __launch_bounds__(256) k_dec_attn_pv(const DecAttnParams P, cons
     };
     const int jv0 = vact ? j0 + sp : j1;
     if (jv0 < j1) load_v(vcur, qs_c, qc_c, jv0);
-    float mx = -INFINITY;
-    for (int s2 = 0; s2 < ws.nsplits; s2++) mx = fmaxf(mx, ws.lmax[h * ws.nsplits + s2]);
-    // the full-row sum, in the same order as the one-workgroup kernel (strided by 256, wave tree, 4 waves); the row comes through LDS
-    float lsum = 0.0f;
-    for (int c0 = 0; c0 < n_ctx; c0 += DEC_PV_STAGE) {
-        const int cn = min(DEC_PV_STAGE, n_ctx - c0);
-        const size_t g0 = (size_t)h * P.max_ctx + c0;                // first half of this piece in the workspace
-        const int off = (int)(g0 & 7);                                // ... and its distance from a 16-byte boundary
-        const u32x4 *src = reinterpret_cast<const u32x4 *>(ws.S + (g0 - off));
-        u32x4 piece[DEC_PV_STAGE / 8 / 256 + 1];
-#pragma unroll
-        for (int i2 = 0; i2 < DEC_PV_STAGE / 8 / 256 + 1; i2++) {
-            const int pc = tid + 256 * i2;
-            if (pc * 8 < cn + off) piece[i2] = src[pc];
-        }
-        __syncthreads();                                              // (the previous piece has been read)
-#pragma unroll
-        for (int i2 = 0; i2 < DEC_PV_STAGE / 8 / 256 + 1; i2++) {
-            const int pc = tid + 256 * i2;
-            if (pc * 8 < cn + off) *reinterpret_cast<u32x4 *>(Sst + (size_t)pc * 8) = piece[i2];
-        }
-        __syncthreads();
-        for (int j = c0 + tid; j < c0 + cn; j += 256) lsum += expf(P.kq_scale * h2f(Sst[j - c0 + off]) - mx);
-    }
-    lsum = wave_sum(lsum);
-    if (lane == 0) red[wave] = lsum;
-    __syncthreads();
-    const float inv = 1.0f / (((red[0] + red[1]) + red[2]) + red[3]);
+    // the row's maximum and sum from its splits': lane s holds split s
+    const int ns = ws.nsplits;
+    const float *ml = ws.ml + 2 * (size_t)(h * ns + min(lane, ns - 1));
+    const float ms = ml[0], lsv = ml[1], mx = wave_max(ms);
+    const float inv = 1.0f / wave_sum(lane < ns && ms != -INFINITY ? expf(ms - mx) * lsv : 0.0f);
     for (int j = j0 + tid; j < j1; j += 256) {
         const half_t eh = f2h(expf(P.kq_scale * h2f(Sg[j]) - mx));
         Pl[j - j0] = f2h(h2f(eh) * inv);
@@ -973,23 +952,30 @@ __global__ void __launch_bounds__(256) k_dec_attn_pv(const DecAttnParams P, cons
         for (int e = 0; e < 8; e++) opart[sp * HD + dg * 8 + e] = o[e];
     }
     __syncthreads();
+    float *const og = ws.opart + (size_t)h * ws.nsplits * HD;
     if (tid < HD) {
         float acc = opart[tid];
         for (int s2 = 1; s2 < NSPLIT; s2++) acc = acc + opart[s2 * HD + tid];
-        ws.opart[((size_t)h * ws.nsplits + sidx) * HD + tid] = acc;
+        __hip_atomic_store(og + (size_t)sidx * HD + tid, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);          // (past the caches of this XCD)
     }
-}
-
-template <int HD>
-__global__ void __launch_bounds__(HD) k_dec_attn_combine(const DecAttnSplitWs ws, half_t *__restrict__ out, int8_t *xq, int heads)
-{
-    const int h = blockIdx.x, d = threadIdx.x;
-    const float *p = ws.opart + (size_t)h * ws.nsplits * HD + d;
-    float acc = p[0];
-    for (int s2 = 1; s2 < ws.nsplits; s2++) acc = acc + p[(size_t)s2 * HD];
-    const half_t yh = f2h(acc);
-    out[(size_t)h * HD + d] = yh;
-    if constexpr (HD % 32 == 0) { if (xq) dec_attn_emit_q8<HD>(xq, heads * HD, h, d, yh); }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                    // (written: the count says so)
+    __syncthreads();
+    if (tid == 0) last = __hip_atomic_fetch_add(ws.count + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(ws.nsplits - 1) ? 1 : 0;
+    __syncthreads();
+    if (!last) return;
+    if (tid == 0) __hip_atomic_store(ws.count + h, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid < HD) {
+        float acc = 0.0f, ov[8];
+        for (int b0 = 0; b0 < ws.nsplits; b0 += 8) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) ov[u] = __hip_atomic_load(og + (size_t)min(b0 + u, ws.nsplits - 1) * HD + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int u = 0; u < 8; u++) if (b0 + u < ws.nsplits) acc = b0 + u == 0 ? ov[u] : acc + ov[u];
+        }
+        const half_t yh = f2h(acc);
+        P.out[(size_t)h * HD + tid] = yh;
+        if constexpr (HD % 32 == 0) { if (P.xq) dec_attn_emit_q8<HD>(P.xq, P.heads * HD, h, tid, yh); }
+    }
 }
 
 __host__ __device__ inline size_t dec_attn_scores_smem(int head_dim, bool q8) { return q8 ? 16 : (size_t)256 * (head_dim * 2 + 16); }
@@ -998,7 +984,7 @@ __host__ __device__ inline size_t dec_attn_pv_smem(int head_dim, int max_ctx, in
 {
     const size_t nsplit = 256 / (head_dim / 8);
     const size_t chunk = (((size_t)max_ctx + nsplits - 1) / nsplits + 63) / 64 * 64;
-    return 8 * 4 + nsplit * head_dim * 4 + (size_t)(DEC_PV_STAGE + 8) * 2 + chunk * 2 + 16;      // + the staged piece of the score row
+    return nsplit * head_dim * 4 + chunk * 2 + 16;
 }
 
 __host__ __device__ inline size_t dec_attn_smem(int head_dim, int max_ctx, int ktile_rows = 0)

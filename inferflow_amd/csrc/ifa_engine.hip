@@ -296,7 +296,8 @@ int ifa_model_destroy(ifa_model *m)
     if (m->batch_tab_dev) (void)hipFree(m->batch_tab_dev);
     if (m->batch_tab_pin) (void)hipHostFree(m->batch_tab_pin);
     if (m->attn_ws.S) (void)hipFree(m->attn_ws.S);
-    if (m->attn_ws.lmax) (void)hipFree(m->attn_ws.lmax);
+    if (m->attn_ws.ml) (void)hipFree(m->attn_ws.ml);
+    if (m->attn_ws.count) (void)hipFree(m->attn_ws.count);
     if (m->attn_ws.opart) (void)hipFree(m->attn_ws.opart);
     for (Tensor &t : m->g) free_tensor(t);
     half_t **bufs[] = {&m->x, &m->x2, &m->xn, &m->hn, &m->pn, &m->q, &m->k, &m->v, &m->dqkv, &m->bqkv, &m->att, &m->a, &m->f, &m->t1, &m->t2, &m->logits,
@@ -464,7 +465,9 @@ int ifa_model_finalize(ifa_model *m)
     }
     if (!m->attn_ws.S) {
         IFA_HIP_CHECK(hipMalloc((void **)&m->attn_ws.S, (size_t)c.heads * c.max_ctx * 2 + 64));      // (+ 64: the last row is read in whole 16-byte pieces)
-        IFA_HIP_CHECK(hipMalloc((void **)&m->attn_ws.lmax, (size_t)c.heads * DEC_ATTN_MAX_SPLITS * 4));
+        IFA_HIP_CHECK(hipMalloc((void **)&m->attn_ws.ml, (size_t)c.heads * DEC_ATTN_MAX_SPLITS * 8));
+        IFA_HIP_CHECK(hipMalloc((void **)&m->attn_ws.count, (size_t)c.heads * 4));
+        IFA_HIP_CHECK(hipMemsetAsync(m->attn_ws.count, 0, (size_t)c.heads * 4, m->stream));
         IFA_HIP_CHECK(hipMalloc((void **)&m->attn_ws.opart, (size_t)c.heads * DEC_ATTN_MAX_SPLITS * c.head_dim * 4));
     }
     if (!m->state) {

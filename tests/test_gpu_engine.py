@@ -385,6 +385,26 @@ def test_long_context_split_attention_matches_single_workgroup_kernel(kvd):
 
 
 @pytest.mark.parametrize("kvd", [dt.F16, dt.Q8_B32T2], ids=["kvf16", "kvq8"])
+@pytest.mark.parametrize("keys,splits", [(70, 1), (70, 32), (301, 5), (600, 2), (600, 12), (640, 32)])
+def test_splits_of_a_heads_keys_are_added_up_by_the_last_workgroup(keys, splits, kvd):
+    """splits with several passes of keys, with none, more splits than are added up at a time: the logits of the one-workgroup kernel (the bound of the test above), and the
+    counts are back at zero behind every launch (each step and each layer is another one)"""
+    wk, _, s = synth.build("test_gqa", dt.Q4_B32T1A, kvd, max_ctx=700, quant_threshold=0, std=0.06)
+    prompt = np.random.default_rng(keys).integers(3, s["vocab"], keys).astype(np.int32)
+    tok = wk.forward(prompt, 0)
+    out = {}
+    for ctx in (0, 16):
+        wk.set_option("attn_split_ctx", ctx)
+        wk.set_option("attn_nsplits", splits)
+        toks, _ = wk.decode(tok, keys, 5)
+        out[ctx] = [int(t) for t in toks], wk.read_buffer("logits").view(np.float16).astype(np.float32)
+    a, b = out[0][1], out[16][1]
+    cos = float((a * b).sum() / (np.linalg.norm(a) * np.linalg.norm(b)))
+    assert cos >= 0.9999 and np.abs(a - b).max() <= 0.02 and out[0][0] == out[16][0], (cos, np.abs(a - b).max(), out[0][0], out[16][0])
+    wk.close()
+
+
+@pytest.mark.parametrize("kvd", [dt.F16, dt.Q8_B32T2], ids=["kvf16", "kvq8"])
 def test_dynamic_batching_rows_are_independent_queries(kvd):
     """ifa_model_decode_batch: one new token for each of n queries, every query on its own KV cache slot.  Rows must
     not interact (permutation / duplication give identical bits) and each row must agree with the same query decoded
