@@ -9,6 +9,59 @@
 
 namespace ifa {
 
+// RMS norm of rows of whole 16-byte pieces, at most 1024 of them: a piece a thread (NC: or two) and everything of a row in registers between its one read and its one
+// write.  The canonical order of ifa_math.h: a wave's 64 pieces are a group.  ADD: TensorOpr::Add in front, its half-rounded sum to sum_out.  (k_layernorm's two waves walk a
+// row of 4096 twice, four pieces at a time: 37 / 512 / 2048 rows 5.4 / 6.2 / 8.8 us, here 4.6 / 5.2 / 8.1.)
+template <int NC, bool ADD>
+__global__ void __launch_bounds__(512) k_rmsnorm_rows(const half_t *__restrict__ x, int cols, const half_t *__restrict__ w, const half_t *__restrict__ b, float multi_base,
+                                                      float eps, half_t *__restrict__ y, const half_t *__restrict__ add, half_t *__restrict__ sum_out)
+{
+    __shared__ float part[8 * NC];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6, nchunks = cols >> 3, ngroups = (nchunks + 63) >> 6;
+    const size_t row = (size_t)blockIdx.x * cols;
+    rms_h8 v[NC], wv[NC], bv[NC];
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+        const int c = 64 * (wave + nw * k) + lane, at = min(c, nchunks - 1);
+        v[k] = reinterpret_cast<const rms_h8 *>(x + row)[at];
+        if constexpr (ADD) {
+            const rms_h8 a = reinterpret_cast<const rms_h8 *>(add + row)[at];
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[k][e] = f2h((float)v[k][e] + (float)a[e]);
+            if (c < nchunks) reinterpret_cast<rms_h8 *>(sum_out + row)[c] = v[k];
+        }
+        if (w) wv[k] = reinterpret_cast<const rms_h8 *>(w)[at];
+        if (w && b) bv[k] = reinterpret_cast<const rms_h8 *>(b)[at];
+        if (c >= nchunks) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[k][e] = (half_t)0;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+        const float pg = wave_sum(rms_chunk_sq(v[k]));
+        if (lane == 0) part[wave + nw * k] = pg;
+    }
+    __syncthreads();
+    const float scale = rms_scale_of(rms_total(part, ngroups), cols, eps);
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+        const int c = 64 * (wave + nw * k) + lane;
+        rms_h8 o;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float f = (float)v[k][e] * scale;          // rms_apply
+            if (w) {
+                const float mlt = multi_base + (float)wv[k][e];
+                f = f * mlt;
+                if (b) f = f + (float)bv[k][e];
+            }
+            o[e] = f2h(f);
+        }
+        if (c < nchunks) reinterpret_cast<rms_h8 *>(y + row)[c] = o;
+    }
+}
+
 // Tensor_RmsNorm_Kernel / Tensor_StdNorm_Kernel (src/kernels/unary_tensor_opr.h:216-289, :68-149),
 // launcher block (128,1), grid (1,rows) (src/tensor/tensor_opr.cu:511-520, :568-577).
 // Std norm keeps the reference's partial-sum structure (128 partials, serial final sum); RMS uses the canonical order
@@ -203,7 +256,9 @@ __global__ void __launch_bounds__(256) k_rope(half_t *__restrict__ x, int head_d
     }
 }
 
-// PositionEmbedding(q), PositionEmbedding(k), SetKRows, SetVRows of a prefill step in ONE launch, a workgroup per token:
+constexpr int ROPE_SPLIT_TOKENS = 768;
+
+// PositionEmbedding(q), PositionEmbedding(k), SetKRows, SetVRows of a prefill step in ONE launch, one or four workgroups per token:
 // the token's head_dim/2 angles are evaluated once (LDS), q is rotated in place, k is rotated through LDS and leaves as
 // 16-byte stores to the k buffer and -- F16 caches -- to its cache row, v is copied to its cache row.
 __global__ void __launch_bounds__(256) k_rope_qk_store(half_t *__restrict__ q, half_t *__restrict__ k, const half_t *__restrict__ v,
@@ -215,18 +270,22 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(half_t *__restrict__ q, h
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
     const int t = blockIdx.x, tid = threadIdx.x, half_dim = head_dim / 2;
     float *cs = reinterpret_cast<float *>(smem_rk);                       // [half_dim][2]
-    half_t *krow = reinterpret_cast<half_t *>(cs + 2 * half_dim);         // [kv_heads * head_dim]
+    half_t *krow = reinterpret_cast<half_t *>(cs + 2 * half_dim);         // [this workgroup's kv heads][head_dim]
+    const size_t q_row = (size_t)heads * head_dim, kv_row = (size_t)kv_heads * head_dim;
+    // (gridDim.y workgroups share a token's heads)
+    heads /= (int)gridDim.y; kv_heads /= (int)gridDim.y;
     const int kv_dim = kv_heads * head_dim;
+    const size_t kv0 = (size_t)t * kv_row + (size_t)blockIdx.y * kv_dim, c0r = (size_t)t * cache_row_elems + (size_t)blockIdx.y * kv_dim;
     for (int c = tid; c < half_dim; c += 256) {
         float co = 1.0f, si = 0.0f;
         if (order != 2 || 2 * c < rope_cols) rope_angle(c, pos0 + t, theta, rope_dims, co, si);
         cs[2 * c] = co; cs[2 * c + 1] = si;
     }
-    const half_t *ksrc = k + (size_t)t * kv_dim;
+    const half_t *ksrc = k + kv0;
     for (int c = tid; c < kv_dim / 8; c += 256) reinterpret_cast<u4 *>(krow)[c] = reinterpret_cast<const u4 *>(ksrc)[c];
     if (vcache)
         for (int c = tid; c < kv_dim / 8; c += 256)
-            reinterpret_cast<u4 *>(vcache + (size_t)t * cache_row_elems)[c] = reinterpret_cast<const u4 *>(v + (size_t)t * kv_dim)[c];
+            reinterpret_cast<u4 *>(vcache + c0r)[c] = reinterpret_cast<const u4 *>(v + kv0)[c];
     __syncthreads();
     auto rotate = [&](half_t *row, int col) {                              // rope_rotate's expressions (ifa_math.h)
         if (order == 2 && 2 * col >= rope_cols) return;
@@ -237,7 +296,7 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(half_t *__restrict__ q, h
         row[i0] = f2h(a - bq);
         row[i1] = f2h(d + e);
     };
-    half_t *qrow = q + (size_t)t * heads * head_dim;
+    half_t *qrow = q + (size_t)t * q_row + (size_t)blockIdx.y * heads * head_dim;
     if (rope_cols == head_dim && head_dim % 16 == 0) {
         // eight pairs per thread through 16-byte accesses (the same expressions as `rotate`): a 128-token prompt spent 10 us per layer
         // here in 2-byte loads and stores (rocprofv3 r06), now one round trip
@@ -269,8 +328,8 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(half_t *__restrict__ q, h
     __syncthreads();
     for (int c = tid; c < kv_dim / 8; c += 256) {
         const u4 kv8 = reinterpret_cast<const u4 *>(krow)[c];
-        reinterpret_cast<u4 *>(k + (size_t)t * kv_dim)[c] = kv8;
-        if (kcache) reinterpret_cast<u4 *>(kcache + (size_t)t * cache_row_elems)[c] = kv8;
+        reinterpret_cast<u4 *>(k + kv0)[c] = kv8;
+        if (kcache) reinterpret_cast<u4 *>(kcache + c0r)[c] = kv8;
     }
 }
 
@@ -469,6 +528,22 @@ using namespace ifa;
 
 extern "C" {
 
+// whole 16-byte pieces, at most two a thread of eight waves
+static bool rmsnorm_rows_ok(size_t cols, const void *x, const void *w, const void *b, const void *y, const void *add, const void *sum_out)
+{
+    return cols % 8 == 0 && cols <= 8192 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)y | (uintptr_t)add | (uintptr_t)sum_out) & 15) == 0;
+}
+static void rmsnorm_rows(const void *x, size_t rows, size_t cols, const void *w, const void *b, float multi_base, float eps, void *y, const void *add, void *sum_out, hipStream_t s)
+{
+    const unsigned waves = (unsigned)((cols / 8 + 63) / 64);
+    const dim3 grid((unsigned)rows), block(64 * std::min(waves, 8u));
+#define IFA_RMS(NC, ADD) k_rmsnorm_rows<NC, ADD><<<grid, block, 0, s>>>((const half_t *)x, (int)cols, (const half_t *)w, (const half_t *)b, multi_base, eps, (half_t *)y, \
+                                                                        (const half_t *)add, (half_t *)sum_out)
+    if (waves <= 8) { if (add) IFA_RMS(1, true); else IFA_RMS(1, false); }
+    else { if (add) IFA_RMS(2, true); else IFA_RMS(2, false); }
+#undef IFA_RMS
+}
+
 // engine-internal: sum_out = a + addend (TensorOpr::Add, half rounding), y = LayerNormalization(sum_out) in one launch
 int ifa_add_layernorm(int kind, const void *a, const void *addend, size_t rows, size_t cols, const void *w, const void *b,
                       float multi_base, float eps, void *sum_out, void *y, ifa_stream stream)
@@ -479,7 +554,8 @@ int ifa_add_layernorm(int kind, const void *a, const void *addend, size_t rows, 
     if (rows == 0 || cols == 0) return IFA_OK;
     const size_t smem = (cols * 2 + 15) & ~(size_t)15;
     IFA_REQUIRE(smem <= 64 * 1024, "ifa_add_layernorm: %zu columns", cols);
-    if (kind == 0)
+    if (kind == 0 && rmsnorm_rows_ok(cols, a, w, b, y, addend, sum_out)) rmsnorm_rows(a, rows, cols, w, b, multi_base, eps, y, addend, sum_out, ifa_s(stream));
+    else if (kind == 0)
         k_layernorm<0><<<dim3((unsigned)rows), dim3(128), smem, ifa_s(stream)>>>((const half_t *)a, (int)cols, (const half_t *)w, (const half_t *)b, multi_base, eps,
                                                                                  (half_t *)y, (const half_t *)addend, (half_t *)sum_out);
     else
@@ -497,7 +573,8 @@ int ifa_layernorm(int kind, const void *x, size_t rows, size_t cols, const void 
     IFA_REQUIRE(b == nullptr || w != nullptr, "ifa_layernorm: bias without weight");
     if (rows == 0 || cols == 0) return IFA_OK;
     IFA_REQUIRE(cols <= 65536, "ifa_layernorm: %zu columns (limit 65536)", cols);
-    if (kind == 0)
+    if (kind == 0 && rmsnorm_rows_ok(cols, x, w, b, y, nullptr, nullptr)) rmsnorm_rows(x, rows, cols, w, b, multi_base, eps, y, nullptr, nullptr, ifa_s(stream));
+    else if (kind == 0)
         k_layernorm<0><<<dim3((unsigned)rows), dim3(128), 0, ifa_s(stream)>>>((const half_t *)x, (int)cols, (const half_t *)w, (const half_t *)b, multi_base, eps, (half_t *)y);
     else
         k_layernorm<1><<<dim3((unsigned)rows), dim3(128), (cols * 2 + 15) & ~(size_t)15, ifa_s(stream)>>>((const half_t *)x, (int)cols, (const half_t *)w, (const half_t *)b, multi_base, eps, (half_t *)y);
@@ -543,7 +620,10 @@ int ifa_rope_qk_store(void *q, void *k, const void *v, int head_dim, int heads, 
     const int rope_cols = (int)(head_dim * partial_rotary_factor + 0.5f);
     const size_t smem = (size_t)head_dim * 4 + (size_t)kv_dim * 2;
     if (smem > 64 * 1024 || (((uintptr_t)k | (uintptr_t)kcache_rows | (uintptr_t)vcache_rows | (uintptr_t)v) & 15) || (cache_row_elems % 8)) return IFA_ERR_STATE;
-    k_rope_qk_store<<<dim3((unsigned)tokens), dim3(256), smem, ifa_s(stream)>>>((half_t *)q, (half_t *)k, (const half_t *)v, head_dim, heads, kv_heads, pos0,
+    // a workgroup a token leaves a short prompt's launch waiting for one chain (angles, rows, LDS, rows): a token's heads shared by four -- 37 / 512 tokens of 32 heads 6.9 / 9.4
+    // -> 5.2 / 9.1 us; 2048 tokens are at the copy's rate with one (22 us for 100 MB)
+    const unsigned ny = tokens <= ROPE_SPLIT_TOKENS && heads % 4 == 0 && kv_heads % 4 == 0 && (kv_dim / 4) % 8 == 0 ? 4 : 1;
+    k_rope_qk_store<<<dim3((unsigned)tokens, ny), dim3(256), smem, ifa_s(stream)>>>((half_t *)q, (half_t *)k, (const half_t *)v, head_dim, heads, kv_heads, pos0,
                                                                                theta, order, rope_cols, rope_cols, (half_t *)kcache_rows,
                                                                                (half_t *)vcache_rows, cache_row_elems);
     IFA_LAUNCH_CHECK();

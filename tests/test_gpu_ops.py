@@ -488,3 +488,21 @@ def test_kv_store_rows(kvd):
     exp = rows.view(np.uint8).reshape(T, rb) if kvd == dt.F16 else o.quantize_act_q8(rows).reshape(T, rb)
     assert np.array_equal(got[row0:row0 + T], exp)
     assert (got[:row0] == 0xAB).all() and (got[row0 + T:] == 0xAB).all()
+
+
+@pytest.mark.parametrize("cols", [8, 504, 512, 520, 4096, 4104, 8184, 8192])
+@pytest.mark.parametrize("wb", ["none", "weight", "both"])
+def test_rms_rows_in_registers_give_the_bits_of_the_walking_kernel(cols, wb):
+    """rows of whole 16-byte pieces: one or two pieces a thread, whole and partial last groups; the same rows from an address off 16 bytes take the kernel that walks them"""
+    rng = np.random.default_rng(cols)
+    rows = 5
+    x, w, b = (rng.standard_normal(n).astype(np.float16) for n in ((rows, cols), (cols,), (cols,)))
+    L, xd, wd, bd = g.capi(), g.dev(x), g.dev(w), g.dev(b)
+    off = torch.zeros(rows * cols + 1, dtype=torch.float16, device="cuda")
+    off[1:] = torch.from_numpy(x).cuda().reshape(-1)
+    got, want = (torch.full((rows, cols), 7.0, dtype=torch.float16, device="cuda") for _ in range(2))
+    args = (g.p(wd) if wb != "none" else None, g.p(bd) if wb == "both" else None, 1.0 if wb == "weight" else 0.0, 1e-5)
+    ia.check(L.ifa_layernorm(0, g.p(xd), rows, cols, *args, g.p(got), g.stream()))
+    ia.check(L.ifa_layernorm(0, off.data_ptr() + 2, rows, cols, *args, g.p(want), g.stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)

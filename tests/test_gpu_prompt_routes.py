@@ -92,3 +92,20 @@ def test_short_prompt_routes_match_the_oracle(T):
         assert tok == int(t_or)
     print("T=%d worst row %.4f x std" % (T, worst))
     wk.close()
+
+
+@pytest.mark.parametrize("shape", ["llama2_7b", "test_gqa"])
+def test_short_prompts_leave_the_cache_rows_of_long_ones(shape):
+    """up to 768 tokens four workgroups share a token's rotation (head counts that four divide), above one holds it: the cache rows of the first layer have the same bits"""
+    wk, _, s = synth.build(shape, dt.Q4_B32T1A, dt.F16, max_ctx=832, layers=1, vocab=1000)
+    toks = np.random.default_rng(3).integers(3, s["vocab"], 800).astype(np.int32)
+    rows = {}
+    for T in (40, 800):
+        wk.reset()
+        wk.forward(toks[:T], 0)
+        rows[T] = [np.array(wk.read_buffer(n, 0, nbytes=40 * s["kv_heads"] * s["head_dim"] * 2)) for n in ("kcache", "vcache")]
+    for a, b in zip(rows[40], rows[800]):
+        a, b = a.view(np.float16).astype(np.float32), b.view(np.float16).astype(np.float32)
+        # (the products in front take other kernels by length: their sums' order, one rounding)
+        assert np.abs(a - b).max() <= 2.0 ** -9 * np.abs(b).max(), np.abs(a - b).max()
+    wk.close()
