@@ -332,6 +332,20 @@ def test_products_of_prompts_with_steps_under_way(T, N, K):
     assert np.all(np.abs(got[:, :N] - (orc.f64(A) @ orc.f64(Wm).T + orc.f64(b))) <= bound) and np.all(got[:, N:] == 7.0) and torch.equal(out, other)
 
 
+@pytest.mark.parametrize("K", [8, 504, 520, 2048, 2056, 4616])
+@pytest.mark.parametrize("T", [1, 2, 3, 5, 6, 7, 8])
+def test_products_of_a_few_rows_ask_for_2048_columns_of_the_weight_at_a_time(T, K):
+    """one and more passes of 512 and of 2048 columns, whole and not, every count of rows: 32-bit activations against 64 bits"""
+    N = 37
+    rng = np.random.default_rng(T * 10000 + K)
+    Wm, A, b = bf16_round(rng.standard_normal((N, K))), rng.standard_normal((T, K + 4)).astype(np.float32), bf16_round(rng.standard_normal(N))
+    out = torch.full((T, N + 2), 7.0, dtype=torch.float32, device="cuda")
+    ia.check(capi().ifa_linear_bf16w(p(devbf(Wm)), N, K, p(dev32(A)), K + 4, T, p(devbf(b)), None, 1.0, 0, 0, p(out), N + 2, 0, 0, None)); sync()
+    got = out.cpu().numpy()
+    bound = (K / 64 + 12) * 2.0 ** -24 * (np.abs(orc.f64(A[:, :K])) @ np.abs(orc.f64(Wm)).T + np.abs(orc.f64(b)))
+    assert np.all(np.abs(got[:, :N] - (orc.f64(A[:, :K]) @ orc.f64(Wm).T + orc.f64(b))) <= bound) and np.all(got[:, N:] == 7.0)
+
+
 def test_products_of_prompts_decline_bad_arguments():
     L = capi()
     z = torch.zeros(1 << 16, dtype=torch.float32, device="cuda")
