@@ -253,7 +253,9 @@ __global__ void __launch_bounds__(256) k_moe_up_rows(const float *__restrict__ h
 }
 
 // grid (width chunks, rows): y[t][c] (+)= sum_k wgt * (identity ? h[t][c] : W_down[e][c] . act[p]); a wave per c at a time.  The chosen
-// experts are walked eight at a time with their loads issued side by side (a step of one token is bound by requests in flight).
+// experts are walked NK at a time with their loads issued side by side (a step is bound by requests in flight: four experts take 130 registers, so that twice as many
+// waves are in flight as with eight), their weighted partial sums reduced once (six rows of four experts of 704 columns 21.6 -> 12.4 us).
+template <int NK>
 __global__ void __launch_bounds__(256) k_moe_down_rows(const float *__restrict__ h, size_t ldh, int W, int F, int experts, int top, const bf16_t *__restrict__ down,
                                                        const int *__restrict__ idx, const float *__restrict__ wgt, const float *__restrict__ act,
                                                        int accumulate, float *__restrict__ y, size_t ldy, int vec)
@@ -261,23 +263,23 @@ __global__ void __launch_bounds__(256) k_moe_down_rows(const float *__restrict__
     const int t = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), nwaves = gridDim.x * (blockDim.x >> 6);
     for (int c = wave; c < W; c += nwaves) {
-        float out = 0.0f;
-        for (int k0 = 0; k0 < top; k0 += 8) {
-            int e[8]; float acc[8];
+        float out = 0.0f, part = 0.0f;
+        for (int k0 = 0; k0 < top; k0 += NK) {
+            int e[NK]; float acc[NK];
 #pragma unroll
-            for (int k = 0; k < 8; k++) { e[k] = k0 + k < top ? idx[t * top + k0 + k] : experts; acc[k] = 0.0f; }
+            for (int k = 0; k < NK; k++) { e[k] = k0 + k < top ? idx[t * top + k0 + k] : experts; acc[k] = 0.0f; }
             if (vec) {
                 for (int j = lane * 8; j < F; j += 512) {
-                    u32x4m wv[8]; float4 a0[8], a1[8];
+                    u32x4m wv[NK]; float4 a0[NK], a1[NK];
 #pragma unroll
-                    for (int k = 0; k < 8; k++)
+                    for (int k = 0; k < NK; k++)
                         if (e[k] < experts) {
                             wv[k] = *reinterpret_cast<const u32x4m *>(down + ((size_t)e[k] * W + c) * F + j);
                             const float *a = act + (size_t)(t * top + k0 + k) * F + j;
                             a0[k] = *reinterpret_cast<const float4 *>(a); a1[k] = *reinterpret_cast<const float4 *>(a + 4);
                         }
 #pragma unroll
-                    for (int k = 0; k < 8; k++)
+                    for (int k = 0; k < NK; k++)
                         if (e[k] < experts) {
                             float s = acc[k];
                             s = fmaf(a0[k].x, __uint_as_float(wv[k][0] << 16), s); s = fmaf(a0[k].y, __uint_as_float(wv[k][0] & 0xFFFF0000u), s);
@@ -289,7 +291,7 @@ __global__ void __launch_bounds__(256) k_moe_down_rows(const float *__restrict__
                 }
             } else {
 #pragma unroll
-                for (int k = 0; k < 8; k++)
+                for (int k = 0; k < NK; k++)
                     if (e[k] < experts) {
                         const bf16_t *w = down + ((size_t)e[k] * W + c) * F;
                         const float *a = act + (size_t)(t * top + k0 + k) * F;
@@ -297,12 +299,14 @@ __global__ void __launch_bounds__(256) k_moe_down_rows(const float *__restrict__
                     }
             }
 #pragma unroll
-            for (int k = 0; k < 8; k++) {      // in the order of the row's choices
+            for (int k = 0; k < NK; k++) {      // in the order of the row's choices
                 if (k0 + k >= top) break;
                 const float wk = wgt[t * top + k0 + k];
-                out = fmaf(wk, e[k] < experts ? wave_sum(acc[k]) : h[(size_t)t * ldh + c], out);
+                if (e[k] < experts) part = fmaf(wk, acc[k], part);
+                else out = fmaf(wk, h[(size_t)t * ldh + c], out);
             }
         }
+        out += wave_sum(part);
         if (lane == 0) { float *d = y + (size_t)t * ldy + c; *d = accumulate ? *d + out : out; }
     }
 }
@@ -479,8 +483,11 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
         else if (experts > 0)
             hipLaunchKernelGGL((k_moe_up_rows<false, false>), dim3(std::min(512u, ifa_cdiv((size_t)ff, 4)), (unsigned)pairs), dim3(256), 0, s, h, ldh, width, ff, experts, top,
                                (const bf16_t *)up_bf16, idx_dev, actb, vec_u, 0, 0.0f, RouteSel());
-        hipLaunchKernelGGL(k_moe_down_rows, dim3(std::min(1024u, ifa_cdiv((size_t)width, 4)), (unsigned)rows), dim3(256), 0, s, h, ldh, width, ff, experts, top,
-                           (const bf16_t *)down_bf16, idx_dev, (const float *)wgt_f32, actb, accumulate ? 1 : 0, (float *)y_f32, ldy, vec_d);
+        const dim3 grid(std::min(1024u, ifa_cdiv((size_t)width, 4)), (unsigned)rows);
+        if (top <= 4) hipLaunchKernelGGL(k_moe_down_rows<4>, grid, dim3(256), 0, s, h, ldh, width, ff, experts, top, (const bf16_t *)down_bf16, idx_dev, (const float *)wgt_f32, actb,
+                                         accumulate ? 1 : 0, (float *)y_f32, ldy, vec_d);
+        else hipLaunchKernelGGL(k_moe_down_rows<8>, grid, dim3(256), 0, s, h, ldh, width, ff, experts, top, (const bf16_t *)down_bf16, idx_dev, (const float *)wgt_f32, actb,
+                                accumulate ? 1 : 0, (float *)y_f32, ldy, vec_d);
         IFA_LAUNCH_CHECK();
         return IFA_OK;
     }

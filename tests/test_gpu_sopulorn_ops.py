@@ -288,3 +288,27 @@ def test_gated_experts_over_bfloat16_rows(T, W, F, E, top):
     got = y.cpu().numpy()
     assert np.all(np.abs(got[:, :W] - want) <= bound) and np.all(got[:, W:] == 7.0)
 
+
+@pytest.mark.parametrize("T,F,top", [(1, 24, 1), (3, 520, 4), (6, 704, 4), (8, 72, 5), (2, 1032, 9)])
+def test_experts_of_a_few_rows_walked_four_and_eight_at_a_time(T, F, top):
+    """fewer, as many and more choices than are walked together; inner sizes of one and more passes of 512 columns: against 64 bits"""
+    W, E = 40, 12
+    rng = np.random.default_rng(F + top)
+    h = rng.standard_normal((T, W)).astype(np.float32)
+    gu = bf16_round(rng.standard_normal((E, 2 * F, W)) / np.sqrt(W)); dn = bf16_round(rng.standard_normal((E, W, F)) / np.sqrt(F))
+    idx = np.stack([rng.permutation(E)[:top] for _ in range(T)]).astype(np.int32)
+    wgt = rng.uniform(0.1, 1.0, (T, top)).astype(np.float32)
+    want, mag = np.zeros((T, W)), np.zeros((T, W))
+    for e in range(E):
+        g, u = h.astype(np.float64) @ gu[e, :F].astype(np.float64).T, h.astype(np.float64) @ gu[e, F:].astype(np.float64).T
+        a, d, w = g / (1 + np.exp(-g)) * u, dn[e].astype(np.float64).T, np.where(idx == e, wgt, 0).sum(1, keepdims=True)
+        want += w * (a @ d); mag += w * ((np.abs(a) + np.abs(g) + np.abs(u) + 1) @ np.abs(d))
+    L = capi()
+    nb = L.ifa_moe_workspace_bytes(T, top, W, 3 * F, E)
+    ws = torch.zeros((nb + 15) // 4, dtype=torch.float32, device="cuda")
+    y = torch.full((T, W + 1), 7.0, dtype=torch.float32, device="cuda")
+    ia.check(L.ifa_moe_experts_gated_f32(p(dev32(h)), W, T, W, F, E, top, p(devbf(gu.reshape(E * 2 * F, W))), p(devbf(dn.reshape(E * W, F))), p(devi(idx)),
+                                         p(dev32(wgt)), 1, p(ws), nb, p(y), W + 1, 0, None)); sync()
+    got = y.cpu().numpy()
+    # 32-bit sums of W and of F products: at most (W + F / 64 + 16) roundings of half a unit of the magnitudes each
+    assert np.all(np.abs(got[:, :W] - want) <= (W + F / 64 + 16) * 2.0 ** -23 * mag) and np.all(got[:, W:] == 7.0)
