@@ -535,7 +535,8 @@ int ifa_kv_store_f32(const void *k_f32, size_t ldk, const void *v_f32, size_t ld
  * Steps of at least tile_min_rows rows (head sizes 32 / 64 / 96 / 128) take the tiled kernel -- scores and weighted sums on the matrix cores, every
  * 32-bit operand as three bfloat16 parts -- which needs the step's sequences on the host too (seqs_host [n_seqs], the same
  * values as seqs_dev; NULL / n_seqs 0: always one workgroup per row) and shares long key ranges out to several workgroups where ws_f32 has the
- * bytes that ifa_attention_tile_workspace_bytes names (with less: in fewer shares).  Smaller steps: with a workspace (ws_f32, ws_bytes; nullable) and at most 512
+ * bytes that ifa_attention_tile_workspace_bytes names (with less: in fewer shares; a single row never: its launch depends on no position, so that it can be
+ * captured and replayed further on).  Smaller steps: with a workspace (ws_f32, ws_bytes; nullable) and at most 512
  * (row, head) pairs, the keys of a pair are shared out to up to 32 workgroups (64 keys each) and merged by a second launch (decode steps). */
 size_t ifa_attention_tile_workspace_bytes(const void *seqs_host, int n_seqs, int heads, int kv_heads, int dim, int vdim, int window /* <= 0: none */, int keep_first);
 int ifa_attention_window_f32(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int norm_q, float eps, float scale, float softcap,

@@ -1064,8 +1064,9 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
     P.seqs = (const SeqDesc *)seqs_dev; P.row_seq = row_seq_dev; P.slot_base = (float *const *)slot_base_dev;
     P.k_off = k_off; P.v_off = v_off; P.out = (float *)out_f32; P.ldo = ldo; P.ws = nullptr; P.nsplit = 1;
     // prompts: the tiled matrix-core kernels (heads of up to 128 dimensions, zero-padded to whole 32s); single tokens and other sizes: a workgroup per row.
-    // With a workspace the bfloat16 form, from the smallest tiled step on (8 heads of 128: 16 rows 15.5 against 17.8 us, 256 rows 33 against 71, 64 rows behind 3000 keys 49 against 719)
-    if (rows >= (size_t)tile_min_rows && n_seqs > 0 && dim <= 128 && vdim <= 128 && ws_f32 && (uintptr_t)ws_f32 % 16 == 0) {
+    // With a workspace the bfloat16 form, from the smallest tiled step on (8 heads of 128: 16 rows 15.5 against 17.8 us, 256 rows 33 against 71, 64 rows behind 3000 keys 49 against 719).
+    // Not for one row: its grids follow from the HOST's positions, and a step of one row is captured once and replayed while the position on the device goes on.
+    if (rows > 1 && rows >= (size_t)tile_min_rows && n_seqs > 0 && dim <= 128 && vdim <= 128 && ws_f32 && (uintptr_t)ws_f32 % 16 == 0) {
         const TilePlan t = tile_plan((const ifa_seq_desc *)seqs_host, n_seqs, heads, kv_heads, dim, vdim, window, keep_first, ws_bytes);
         IFA_REQUIRE(t.tiles < 65536 && t.groups < 65536 && t.blocks < 65536, "%s: %zu query tiles, %zu key blocks in one step", who, t.tiles, t.blocks);
         if (t.bytes <= ws_bytes) {

@@ -1416,7 +1416,7 @@ int lay_set_option(ifa_model *m, const char *name, int value)
     if (!strcmp(name, "scan_chunk_min")) { n->opt_scan_chunk_min = value; return IFA_OK; }
     if (!strcmp(name, "ssm_chunk_min")) { n->opt_ssm_chunk_min = value; return IFA_OK; }
     if (!strcmp(name, "a16_min")) { n->opt_a16_min = value; return IFA_OK; }
-    if (!strcmp(name, "attn_tile_min")) { n->opt_attn_tile_min = value; return IFA_OK; }
+    if (!strcmp(name, "attn_tile_min")) { n->opt_attn_tile_min = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "graph")) { n->opt_graph = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "ops32")) { IFA_HIP_CHECK(hipStreamSynchronize(m->stream)); n->cfg.ops32 = value ? 1 : 0; drop_step_graph(n); return IFA_OK; }
     return ifa_fail(IFA_ERR_ARG, "ifa_model_set_option: unknown option '%s' (layer-list model: tap_layers, graph, ops32, attn_tile_min, a16_min, fuse_rows, fuse_post, ssm_chunk_min, scan_chunk_min, fuse_step)", name);
@@ -1567,7 +1567,7 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
             }
         }
     }
-    if (T >= (size_t)std::max(n->opt_attn_tile_min, 1)) {
+    if (T >= (size_t)std::max(n->opt_attn_tile_min, 2)) {          // (a step of one row takes no tiles of the workspace's form, see attention_launch)
         size_t need = 0;
         for (const LLayer &L : n->layers) {
             const ifa_layer_spec &sp = L.spec;

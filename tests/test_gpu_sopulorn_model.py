@@ -347,6 +347,29 @@ def test_greedy_generation_through_the_engine(tmp_path):
     eng.close()
 
 
+@pytest.mark.parametrize("graph", [1, 0])
+def test_generation_over_key_block_edges_with_single_rows_sent_to_the_tiles(tmp_path, graph):
+    """attn_tile_min 1: the launches of a decode step are shaped once and the position then advances on the device, over the edges of blocks of 32 keys and of the
+    shares of a key range (127 -> 128), a longer prompt growing the prompts' workspace in between"""
+    import inferflow_amd as ia
+    w = fx.random_weights(MIXED, 21)
+    prompt, other = tokens_for(MIXED, 100, 22), tokens_for(MIXED, 300, 23)
+    eng = engine_for(tmp_path, MIXED, w)
+    for name, value in ((b"attn_tile_min", 1), (b"graph", graph)):
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), name, value))
+    for _ in range(2):
+        q = eng.add_query(prompt)
+        gen, _ = eng.generate(q, 70)
+        eng.remove_query(q)
+        want = oracle_logits(MIXED, w, prompt + gen)
+        for i, tok in enumerate(gen):
+            row = want[len(prompt) - 1 + i]
+            assert row[tok] > row.max() - 1e-3 * np.abs(row).max(), i
+        lg, _ = run_whole(eng, other)
+        assert fx.rel_err(lg, oracle_logits(MIXED, w, other)).max() < TOL32
+    eng.close()
+
+
 def test_ini_route_and_trace_replay_tool(tmp_path):
     from inferflow_amd.engine import InferenceEngine
     w = fx.random_weights(MIXED, 17)
