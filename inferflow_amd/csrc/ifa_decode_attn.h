@@ -847,9 +847,10 @@ __global__ void __launch_bounds__(256) k_dec_attn_scores(const DecAttnParams P, 
         half_t sv = f2h(alpha * c);
         if (P.alibi) { float a = (float)j * mk; sv = f2h(a + h2f(sv)); }
         ws.S[(size_t)h * P.max_ctx + j] = sv;
-        // the thread's own maximum and sum so far (a new maximum scales the sum: at most a key in 256 of a thread's)
+        // the thread's own maximum and sum so far (a new maximum scales the sum: at most a key in 256 of a thread's); a score of -inf -- the half's overflow -- adds
+        // nothing, whatever the maximum is (-inf - -inf would be NaN)
         const float sf = P.kq_scale * h2f(sv), mn = fmaxf(lmax, sf);
-        lsum = (lmax == mn ? lsum : lsum * expf(lmax - mn)) + expf(sf - mn);
+        lsum = (lmax == mn ? lsum : lsum * expf(lmax - mn)) + (sf == -INFINITY ? 0.0f : expf(sf - mn));
         lmax = mn;
     }
     const float wm = wave_max(lmax);
@@ -903,11 +904,11 @@ __global__ void __launch_bounds__(256) k_dec_attn_pv(const DecAttnParams P, cons
     };
     const int jv0 = vact ? j0 + sp : j1;
     if (jv0 < j1) load_v(vcur, qs_c, qc_c, jv0);
-    // the row's maximum and sum from its splits': lane s holds split s
+    // the row's maximum and sum from its splits': lane s holds split s (sum 0: no keys, or scores of -inf only; a NaN among the scores is in the sum, not in the maximum)
     const int ns = ws.nsplits;
     const float *ml = ws.ml + 2 * (size_t)(h * ns + min(lane, ns - 1));
     const float ms = ml[0], lsv = ml[1], mx = wave_max(ms);
-    const float inv = 1.0f / wave_sum(lane < ns && ms != -INFINITY ? expf(ms - mx) * lsv : 0.0f);
+    const float inv = 1.0f / wave_sum(lane < ns && lsv != 0.0f ? expf(ms - mx) * lsv : 0.0f);
     for (int j = j0 + tid; j < j1; j += 256) {
         const half_t eh = f2h(expf(P.kq_scale * h2f(Sg[j]) - mx));
         Pl[j - j0] = f2h(h2f(eh) * inv);

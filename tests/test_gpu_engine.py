@@ -404,6 +404,35 @@ def test_splits_of_a_heads_keys_are_added_up_by_the_last_workgroup(keys, splits,
     wk.close()
 
 
+@pytest.mark.parametrize("rows,value", [((0,), 65504.0), ((0, 3, 64, 299), 65504.0), (range(64), 65504.0), ((7,), float("nan")), (range(64, 128), float("nan"))],
+                         ids=["first", "some", "whole_split", "nan", "nan_split"])
+def test_scores_that_overflow_to_infinity_and_nan_keys_behind_split_keys(rows, value):
+    """cached keys of the last layer whose F16 scores overflow, with both signs over the heads, and NaN keys: the split launches leave what the one-workgroup kernel leaves (weight 0
+    for -inf, NaN for +inf and NaN); splits of 64 keys"""
+    wk, _, s = synth.build("test_gqa", dt.Q4_B32T1A, dt.F16, max_ctx=400, quant_threshold=0, std=0.06)
+    last, kvw = s["layers"] - 1, s["kv_heads"] * s["head_dim"]
+    prompt = np.random.default_rng(5).integers(3, s["vocab"], 300).astype(np.int32)
+    tok = wk.forward(prompt, 0)
+    wk.set_option("attn_nsplits", 32)
+    finite = 0
+    for seed in range(6):
+        key = (value * np.random.default_rng(seed).choice([-1.0, 1.0], kvw)).astype(np.float16)
+        out = []
+        for ctx in (0, 16):
+            wk.forward(prompt, 0)
+            for r in rows:
+                wk.write_buffer("kcache", key, layer=last, offset=2 * kvw * r)
+            wk.set_option("attn_split_ctx", ctx)
+            wk.decode(tok, len(prompt), 1)
+            out.append(wk.read_buffer("att").view(np.float16).astype(np.float32))
+        bad = np.isnan(out[0])
+        assert np.array_equal(bad, np.isnan(out[1])), (seed, bad.sum(), np.isnan(out[1]).sum())
+        assert np.abs(out[0] - out[1])[~bad].max(initial=0.0) < 2e-3 * max(1.0, np.abs(out[0][~bad]).max(initial=0.0)), seed
+        finite += int((~bad).sum())
+    assert finite > 0 or value != value
+    wk.close()
+
+
 @pytest.mark.parametrize("kvd", [dt.F16, dt.Q8_B32T2], ids=["kvf16", "kvq8"])
 def test_dynamic_batching_rows_are_independent_queries(kvd):
     """ifa_model_decode_batch: one new token for each of n queries, every query on its own KV cache slot.  Rows must
