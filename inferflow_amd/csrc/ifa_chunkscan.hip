@@ -8,9 +8,12 @@
 //     a triangular system whose solution is U = U0 - W S with U0, W the solutions for the right hand sides beta V and beta G K: both before S is known
 //   o_i = G_i S^T q_i + sum_{j <= i} (G_i / G_j)(q_i . k_j) u_j;     S' = G_last S + sum_j (G_last / G_j) k_j u_j^T
 // so three launches do it: what a chunk needs no state for (all chunks at once), the states from chunk to chunk, the outputs (all chunks at once).
-// Now 69 us (30 + 10 + 29) and 165 us (36 + 91 + 38) per 2048 tokens and layer of 16 heads; at 601 tokens of 8 heads 35 and 80 (were 159 and 312).  The first and
-// third launches wait for their operands (scalar requests, 128 bytes a row, no staging: each is read by one or two waves), the second for its chain.
-// The decays' logarithms are summed, and kind 0's powers formed, in double; sums are fp32 throughout.
+// Now 66 us (25 + 10 + 30) and 192 us (33 + 114 + 45) per 2048 tokens and layer of 16 heads; at 601 tokens of 8 heads 27 and 81 (were 159 and 312).  The first and
+// third launches wait for their operands (no staging: each is read by one or two waves), the second for its chain.
+// Keys of 64 and 128 have instances here; other sizes go token by token.
+// fp32 operands; a sum that would leave more error than the token-by-token form's few additions do is formed in 64 bits (scores, states of kind 1), from zero in short
+// pieces (the others), and decays are rounded to float once, from double.  Error against 64 bits, rms, 601 tokens: kind 0 1.8e-7 (token by token 3.5e-7), its state 1.7e-7
+// (4.2e-7); kind 1 7.8e-8 (1.08e-7), its state 6.0e-8 (8.1e-8).  With one fp32 chain per sum kind 1 had 2.6e-7 and 1.4e-7 (75 us).
 #include <utility>
 #include "ifa_host.h"
 #include "ifa_f32_common.h"
@@ -23,6 +26,7 @@ namespace {
 constexpr int CL = 64;          // tokens of a chunk
 typedef float f32x16c __attribute__((ext_vector_type(16)));
 typedef float f32x4c __attribute__((ext_vector_type(4)));
+typedef double f64x4c __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(3))) float lds_f32;
 typedef const __attribute__((address_space(3))) f32x4c lds_f32x4;
 
@@ -59,11 +63,15 @@ __device__ __forceinline__ double power(double d, int n)
     return r;
 }
 
-// e^x, x <= 0 from a difference of double sums: what the conversion to float leaves off is a factor
+// e^x for a difference of double sums, within a rounding of the float result (expf's own error, up to two of them, would be in every decay): e^r of the
+// remainder |r| <= ln 2 / 2 as its power series up to r^8 / 8! (the rest is below 2.1e-10), in double
 __device__ __forceinline__ float exp_of(double x)
 {
-    const float hi = (float)x, e = expf(hi);
-    return fmaf(e, (float)(x - (double)hi), e);
+    const double n = rint(x * 1.4426950408889634), r = fma(n, -0.6931471805599453, x);
+    double p = 1.0 / 40320.0;
+    p = fma(p, r, 1.0 / 5040.0); p = fma(p, r, 1.0 / 720.0); p = fma(p, r, 1.0 / 120.0); p = fma(p, r, 1.0 / 24.0);
+    p = fma(p, r, 1.0 / 6.0); p = fma(p, r, 0.5); p = fma(p, r, 1.0); p = fma(p, r, 1.0);
+    return ldexpf((float)p, (int)n);
 }
 
 // lane t: the logarithms of the decays of positions 0 .. t of the chunk, summed (none past its end; a decay that has underflowed counts as e^-200)
@@ -132,23 +140,29 @@ __global__ void __launch_bounds__(256) k_linear_pass(ChunkArgs A)
     *state = S;
 }
 
-// x_T -= sum_{j < T} A_Tj x_j, for T = 0, 1, ...: straight-line code, x in registers; `rows`: A's place in LDS
+// x_T = A_TT (x_T - sum_{j < T} A_Tj x_j), for T = 0, 1, ...: straight-line code, x in registers; `rows`: A's place in LDS
 template <int T>
 __device__ __forceinline__ void solve_row(float (&x)[CL], uint32_t &rows)
 {
     asm volatile("" : "+v"(rows));          // (A's rows are read one by one as they are needed, not all ahead of everything)
+    f32x4c s = {0.f, 0.f, 0.f, 0.f};          // (four sums from zero: one chain from x_T on rounded every term to the size of x_T)
+    float beta = 0.0f;
 #pragma unroll
-    for (int j = 0; j < T; j += 4) {
+    for (int j = 0; j <= T; j += 4) {
         const f32x4c a = *(lds_f32x4 *)(uintptr_t)(rows + (T * (CL + 4) + j) * 4);
 #pragma unroll
-        for (int e = 0; e < 4; e++) if (j + e < T) x[T] = fmaf(-a[e], x[j + e], x[T]);
+        for (int e = 0; e < 4; e++) {
+            if (j + e < T) s[e] = fmaf(a[e], x[j + e], s[e]);
+            if (j + e == T) beta = a[e];
+        }
     }
+    x[T] = beta * (x[T] - ((s[0] + s[1]) + (s[2] + s[3])));
 }
 template <int... T>
 __device__ __forceinline__ void solve_rows(float (&x)[CL], uint32_t rows, std::integer_sequence<int, T...>) { (solve_row<T>(x, rows), ...); }
 
-// ---- kind 1, first launch: U0 and W of a chunk.  grid (chunks, heads).  A_ij = beta_i (G_i / G_j)(k_i . k_j), j < i, in LDS; then a thread per column of
-// [beta V | beta G K] solves (I + A) x = its column forwards, x in registers, A's rows read by all threads alike (2016 multiply-adds per thread)
+// ---- kind 1, first launch: U0 and W of a chunk.  grid (chunks, heads).  A_ij = (G_i / G_j)(k_i . k_j), j < i, and A_ii = beta_i in LDS; then a thread per column of
+// [V | G K] solves x_i = beta_i (column_i - sum_{j < i} A_ij x_j) forwards, x in registers, A's rows read by all threads alike (2080 multiply-adds per thread)
 __global__ void __launch_bounds__(256) k_delta_chunk(ChunkArgs A)
 {
     __shared__ __attribute__((aligned(16))) float Am[CL][CL + 4];
@@ -169,7 +183,7 @@ __global__ void __launch_bounds__(256) k_delta_chunk(ChunkArgs A)
         if (lane == 0) dec[CL] = exp_of(all);
     }
     __syncthreads();
-    const int wi = wave >> 1, wj = wave & 1;          // a 32 x 32 tile of k_i . k_j per wave
+    const int wi = wave >> 1, wj = wave & 1;          // a 32 x 32 tile of k_i . k_j per wave, 16 columns summed by themselves at a time
     f32x16c acc;
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = 0.0f;
@@ -177,16 +191,24 @@ __global__ void __launch_bounds__(256) k_delta_chunk(ChunkArgs A)
         const float *ri = kp + (size_t)min(32 * wi + i, n - 1) * A.ldk + 4 * g, *rj = kp + (size_t)min(32 * wj + i, n - 1) * A.ldk + 4 * g;
         for (int s0 = 0; s0 < A.dk; s0 += 64)
 #pragma unroll
-            for (int s = s0; s < s0 + 64; s += 8) {
-                const f32x4c a = *(const f32x4c *)(ri + s), b = *(const f32x4c *)(rj + s);
+            for (int s = s0; s < s0 + 64; s += 16) {
+                f32x16c part;
 #pragma unroll
-                for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], acc, 0, 0, 0);
+                for (int r = 0; r < 16; r++) part[r] = 0.0f;
+#pragma unroll
+                for (int u = 0; u < 16; u += 8) {
+                    const f32x4c a = *(const f32x4c *)(ri + s + u), b = *(const f32x4c *)(rj + s + u);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) part = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], part, 0, 0, 0);
+                }
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[r] += part[r];
             }
     }
 #pragma unroll
     for (int r = 0; r < 16; r++) {
         const int row = 32 * wi + (r & 3) + 8 * (r >> 2) + 4 * g, col = 32 * wj + i;
-        Am[row][col] = col < row && row < n ? beta[row] * exp_of(L[row] - L[col]) * acc[r] : 0.0f;
+        Am[row][col] = col == row ? beta[row] : (col < row && row < n ? exp_of(L[row] - L[col]) * acc[r] : 0.0f);
     }
     __syncthreads();
     for (int col = tid; col < A.dv + A.dk; col += 256) {
@@ -198,7 +220,7 @@ __global__ void __launch_bounds__(256) k_delta_chunk(ChunkArgs A)
 #pragma unroll
         for (int t = 0; t < CL; t++) x[t] = src[(size_t)min(t, n - 1) * ld];
 #pragma unroll
-        for (int t = 0; t < CL; t++) x[t] = t < n ? x[t] * beta[t] * (is_v ? 1.0f : gam[t]) : 0.0f;
+        for (int t = 0; t < CL; t++) x[t] = t < n ? (is_v ? x[t] : x[t] * gam[t]) : 0.0f;
         solve_rows(x, rows, std::make_integer_sequence<int, CL>());
         const size_t at = (size_t)blockIdx.x * A.heads + h;
         float *dst = is_v ? A.u + at * CL * A.dv + col : A.w + at * CL * A.dk + col - A.dv;
@@ -236,7 +258,7 @@ __global__ void __launch_bounds__(256) k_delta_pass(ChunkArgs A)
 #pragma unroll
     for (int t = 0; t < TK; t++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) S[t][r] = sd.pos0 > 0 ? state[(size_t)((wave * TK + t) * 16 + 4 * g + r) * A.dv] : 0.0f;
+        for (int r = 0; r < 4; r++) S[t][r] = sd.pos0 > 0 ? state[(size_t)((wave * TK + t) * 16 + 4 * r + g) * A.dv] : 0.0f;
     f32x4c wr[DK / 16], dr[4];
     float kr[TK][16], ur[4], last;
     auto request_w = [&](int c) {
@@ -266,7 +288,7 @@ __global__ void __launch_bounds__(256) k_delta_pass(ChunkArgs A)
         for (int t = 0; t < TK; t++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int row = (wave * TK + t) * 16 + 4 * g + r;
+                const int row = (wave * TK + t) * 16 + 4 * r + g;
                 Sb[row * LS + i] = S[t][r];
                 snap[(size_t)row * A.dv] = S[t][r];
             }
@@ -288,34 +310,44 @@ __global__ void __launch_bounds__(256) k_delta_pass(ChunkArgs A)
         }
         if (c + 1 < nc) request_w(c + 1);
         lds_barrier();
+        f64x4c add[TK];          // (summed in 64 bits: in 32 the 64 additions left more in the state than the tokens' own updates do)
 #pragma unroll
-        for (int t = 0; t < TK; t++) {
+        for (int t = 0; t < TK; t++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) S[t][r] *= last;
+            for (int r = 0; r < 4; r++) add[t][r] = (double)S[t][r] * (double)last;
 #pragma unroll
-            for (int x = 0; x < 16; x++)
-                S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[t][x] * dr[x >> 2][x & 3], Ub[(16 * (x >> 2) + 4 * g + (x & 3)) * LS + i], S[t], 0, 0, 0);
+        for (int x = 0; x < 16; x++) {
+            const double u1 = (double)Ub[(16 * (x >> 2) + 4 * g + (x & 3)) * LS + i];
+#pragma unroll
+            for (int t = 0; t < TK; t++) add[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)(kr[t][x] * dr[x >> 2][x & 3]), u1, add[t], 0, 0, 0);
         }
+#pragma unroll
+        for (int t = 0; t < TK; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) S[t][r] = (float)add[t][r];
         if (c + 1 < nc) request_k(c + 1);
     }
 #pragma unroll
     for (int t = 0; t < TK; t++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) state[(size_t)((wave * TK + t) * 16 + 4 * g + r) * A.dv] = S[t][r];
+        for (int r = 0; r < 4; r++) state[(size_t)((wave * TK + t) * 16 + 4 * r + g) * A.dv] = S[t][r];
 }
 
-// ---- third launch: the outputs of a chunk.  grid (chunks, heads, 64 value columns), two waves of 32 positions.  The products are transposed: scores K Q^T and
-// outputs U^T P^T, so that a lane's accumulators hold 16 keys of its position and are the second product's operand as they are.
-template <int KIND, int DK>
-__global__ void __launch_bounds__(128) k_chunk_out(ChunkArgs A)
+// ---- third launch: the outputs of a chunk.  grid (chunks, heads, 64 value columns), four waves of 16 positions.  The products are transposed: scores K Q^T and
+// outputs U^T P^T, so that a lane's accumulators hold four keys of its position and are the second product's operand as they are.  A lane's 16 bytes of a row of S
+// or U are columns 4 i .. 4 i + 3: column e of each goes to tile e, so that its outputs are 16 bytes side by side again.
+// The scores are summed in 64 bits: q . k of unit vectors is small against its terms, and in 32 bits its rounding was most of the outputs' error.  Everything else
+// is summed 16 terms at a time.  (Error against 64 bits, rms, and time: see the top.)  VEC: rows of U or v of whole aligned 16 bytes.
+template <int KIND, int DK, bool VEC>
+__global__ void __launch_bounds__(256) k_chunk_out(ChunkArgs A)
 {
-    __shared__ double L[2][CL];
-    __shared__ float pw[2][CL + 1];
+    __shared__ double L[4][CL];
+    __shared__ float pw[4][CL + 1];
     SeqDesc sd; int c;
     if (!chunk_seq(A, blockIdx.x, sd, c)) return;
-    const int h = blockIdx.y, kh = h / (A.heads / A.qk_heads), lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 31, g = lane >> 5;
-    const int t0 = c * CL, n = min(CL, sd.n - t0), pos = 32 * wave + i, c0 = blockIdx.z * 64, NT = min(2, (A.dv - c0) / 32);
-    if (32 * wave >= n) return;
+    const int h = blockIdx.y, kh = h / (A.heads / A.qk_heads), lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15, g = lane >> 4;
+    const int t0 = c * CL, n = min(CL, sd.n - t0), pos = 16 * wave + i, c0 = blockIdx.z * 64, cl = min(c0 + 4 * i, A.dv - 4);
+    if (16 * wave >= n) return;
     // (a table per wave: nothing to wait for but its own writes)
     if (KIND == 0) {
         const double d = (double)A.decay_head[h];
@@ -325,63 +357,64 @@ __global__ void __launch_bounds__(128) k_chunk_out(ChunkArgs A)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     const float *qp = A.q + (size_t)(sd.row0 + t0 + min(pos, n - 1)) * A.ldq + (size_t)kh * DK + 4 * g, *kp = A.k + (size_t)(sd.row0 + t0) * A.ldk + (size_t)kh * DK + 4 * g;
     const size_t at = (size_t)blockIdx.x * A.heads + h;
-    const float *up = KIND == 0 ? A.v + (size_t)(sd.row0 + t0) * A.ldv + (size_t)h * A.dv + c0 + i : A.u + at * CL * A.dv + c0 + i;
+    const float *up = KIND == 0 ? A.v + (size_t)(sd.row0 + t0) * A.ldv + (size_t)h * A.dv + cl : A.u + at * CL * A.dv + cl;
     const size_t ldu = KIND == 0 ? A.ldv : (size_t)A.dv;
-    f32x4c q[DK / 8];
+    auto row4 = [&](const float *p) -> f32x4c {
+        if constexpr (VEC) return *(const f32x4c *)p;
+        else return f32x4c{p[0], p[1], p[2], p[3]};
+    };
+    f32x4c q[DK / 16], o[4];
 #pragma unroll
-    for (int s = 0; s < DK / 8; s++) q[s] = *(const f32x4c *)(qp + 8 * s);
-    f32x16c o[2];
-    const float *st = A.st + at * DK * A.dv + c0 + i;
+    for (int s = 0; s < DK / 16; s++) q[s] = *(const f32x4c *)(qp + 16 * s);
 #pragma unroll
-    for (int nt = 0; nt < 2; nt++) {
+    for (int t = 0; t < 4; t++) o[t] = f32x4c{0.f, 0.f, 0.f, 0.f};
+    auto add16 = [&](const f32x4c (&a)[4], const f32x4c &b) {          // o += 16 terms, four of them per product
+        f32x4c part[4];
 #pragma unroll
-        for (int r = 0; r < 16; r++) o[nt][r] = 0.0f;
-        if (nt < NT) {
+        for (int t = 0; t < 4; t++) part[t] = f32x4c{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int s = 0; s < DK / 8; s++)
+        for (int e = 0; e < 4; e++)
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    o[nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(st[(size_t)(8 * s + 4 * g + e) * A.dv + 32 * nt], q[s][e], o[nt], 0, 0, 0);
-        }
+            for (int t = 0; t < 4; t++) part[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e][t], b[e], part[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 4; t++) o[t] += part[t];
+    };
+    const float *st = A.st + at * DK * A.dv + cl;
+#pragma unroll
+    for (int s = 0; s < DK / 16; s++) {
+        f32x4c a[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) a[e] = *(const f32x4c *)(st + (size_t)(16 * s + 4 * g + e) * A.dv);
+        add16(a, q[s]);
     }
     const double Li = KIND == 1 ? L[wave][pos] : 0.0;
     const float gam = KIND == 0 ? pw[wave][pos + 1] : exp_of(Li);
 #pragma unroll
-    for (int nt = 0; nt < 2; nt++)
+    for (int t = 0; t < 4; t++) o[t] *= gam;
+    for (int kt = 0; kt <= wave; kt++) {
+        f64x4c p = {0.0, 0.0, 0.0, 0.0};          // keys 16 kt + 4 r + g of the lane's position
+        const float *kr = kp + (size_t)min(16 * kt + i, n - 1) * A.ldk;
+        f32x4c u[4], w;
 #pragma unroll
-        for (int r = 0; r < 16; r++) o[nt][r] *= gam;
-    for (int jt = 0; jt <= wave; jt++) {
-        f32x16c p;
+        for (int r = 0; r < 4; r++) u[r] = row4(up + (size_t)min(16 * kt + 4 * r + g, n - 1) * ldu);
 #pragma unroll
-        for (int r = 0; r < 16; r++) p[r] = 0.0f;
-        const float *kr = kp + (size_t)min(32 * jt + i, n - 1) * A.ldk;
+        for (int s = 0; s < DK / 16; s++) {
+            const f32x4c k = *(const f32x4c *)(kr + 16 * s);
 #pragma unroll
-        for (int s = 0; s < DK / 8; s++) {
-            const f32x4c k = *(const f32x4c *)(kr + 8 * s);
-#pragma unroll
-            for (int e = 0; e < 4; e++) p = __builtin_amdgcn_mfma_f32_32x32x2f32(k[e], q[s][e], p, 0, 0, 0);
+            for (int e = 0; e < 4; e++) p = __builtin_amdgcn_mfma_f64_16x16x4f64((double)k[e], (double)q[s][e], p, 0, 0, 0);
         }
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int j = 32 * jt + (r & 3) + 8 * (r >> 2) + 4 * g;
-            p[r] = j <= pos ? p[r] * (KIND == 0 ? pw[wave][max(pos - j, 0)] : exp_of(Li - L[wave][j])) : 0.0f;
+        for (int r = 0; r < 4; r++) {
+            const int j = 16 * kt + 4 * r + g;
+            w[r] = j <= pos ? (float)(p[r] * (double)(KIND == 0 ? pw[wave][max(pos - j, 0)] : exp_of(Li - L[wave][j]))) : 0.0f;
         }
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++)
-            if (nt < NT) {
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    o[nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(up[(size_t)min(32 * jt + (r & 3) + 8 * (r >> 2) + 4 * g, n - 1) * ldu + 32 * nt], p[r], o[nt], 0, 0, 0);
-            }
+        add16(u, w);
     }
     if (pos >= n) return;
-    float *dst = A.out + (size_t)(sd.row0 + t0 + pos) * A.ldo + (size_t)h * A.dv + c0 + 4 * g;
+    float *dst = A.out + (size_t)(sd.row0 + t0 + pos) * A.ldo + (size_t)h * A.dv + c0 + 16 * g;
 #pragma unroll
-    for (int nt = 0; nt < 2; nt++)
-        if (nt < NT) {
-#pragma unroll
-            for (int r = 0; r < 16; r += 4) *(f32x4c *)(dst + 32 * nt + 8 * (r >> 2)) = f32x4c{o[nt][r], o[nt][r + 1], o[nt][r + 2], o[nt][r + 3]};
-        }
+    for (int r = 0; r < 4; r++)
+        if (c0 + 16 * g + 4 * r < A.dv) *(f32x4c *)(dst + 4 * r) = f32x4c{o[0][r], o[1][r], o[2][r], o[3][r]};
 }
 
 size_t al16c(size_t n) { return (n + 15) & ~(size_t)15; }
@@ -433,13 +466,14 @@ int ifa_state_chunked_f32(int kind, const void *q_f32, size_t ldq, const void *k
     if (kind == 0) {
         hipLaunchKernelGGL(k_linear_chunk, per_chunk, dim3(256), 0, s, A);
         hipLaunchKernelGGL(k_linear_pass, dim3(ifa_cdiv((size_t)dk * dv, 256), (unsigned)heads, (unsigned)n_seqs), dim3(256), 0, s, A);
-        if (dk == 64) hipLaunchKernelGGL((k_chunk_out<0, 64>), per_chunk, dim3(128), 0, s, A);
-        else hipLaunchKernelGGL((k_chunk_out<0, 128>), per_chunk, dim3(128), 0, s, A);
+        const bool vec = ldv % 4 == 0 && ((uintptr_t)v_f32 & 15) == 0;
+        if (dk == 64) { if (vec) hipLaunchKernelGGL((k_chunk_out<0, 64, true>), per_chunk, dim3(256), 0, s, A); else hipLaunchKernelGGL((k_chunk_out<0, 64, false>), per_chunk, dim3(256), 0, s, A); }
+        else { if (vec) hipLaunchKernelGGL((k_chunk_out<0, 128, true>), per_chunk, dim3(256), 0, s, A); else hipLaunchKernelGGL((k_chunk_out<0, 128, false>), per_chunk, dim3(256), 0, s, A); }
     } else {
         const dim3 pass((unsigned)(heads * (dv / 16)), (unsigned)n_seqs);
         hipLaunchKernelGGL(k_delta_chunk, dim3((unsigned)chunks, (unsigned)heads), dim3(256), 0, s, A);
-        if (dk == 64) { hipLaunchKernelGGL(k_delta_pass<64>, pass, dim3(256), 0, s, A); hipLaunchKernelGGL((k_chunk_out<1, 64>), per_chunk, dim3(128), 0, s, A); }
-        else { hipLaunchKernelGGL(k_delta_pass<128>, pass, dim3(256), 0, s, A); hipLaunchKernelGGL((k_chunk_out<1, 128>), per_chunk, dim3(128), 0, s, A); }
+        if (dk == 64) { hipLaunchKernelGGL(k_delta_pass<64>, pass, dim3(256), 0, s, A); hipLaunchKernelGGL((k_chunk_out<1, 64, true>), per_chunk, dim3(256), 0, s, A); }
+        else { hipLaunchKernelGGL(k_delta_pass<128>, pass, dim3(256), 0, s, A); hipLaunchKernelGGL((k_chunk_out<1, 128, true>), per_chunk, dim3(256), 0, s, A); }
     }
     IFA_LAUNCH_CHECK();
     return IFA_OK;

@@ -305,10 +305,12 @@ def dense_attention_64(q, k, v, pos0, heads, kv_heads, scale, window, keep, cap=
 # chunks of 64: one token more or less than a chunk, several chunks, sequences that end inside one, continued states, shared q / k heads, one value tile and odd counts of them
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("heads,qk_heads,dk,dv,steps", [(2, 2, 64, 128, [[(0, 1)], [(0, 63)], [(0, 64)]]), (4, 2, 128, 32, [[(0, 65), (1, 200)], [(1, 64), (0, 1)]]),
-                                                        (3, 1, 64, 96, [[(0, 130), (1, 3), (2, 64)], [(2, 66)]]), (2, 1, 128, 160, [[(0, 257)], [(0, 31)]])])
+                                                        (3, 1, 64, 96, [[(0, 130), (1, 3), (2, 64)], [(2, 66)]]), (2, 1, 128, 160, [[(0, 257)], [(0, 31)]]),
+                                                        (4, 2, 64, 64, [[(0, 700)]])])
 def test_state_recurrences_in_chunks(kind, heads, qk_heads, dk, dv, steps):
-    """Against the float64 recurrence, beside the token-by-token kernel on the same states: fp32 sums of up to 64 + dk terms in another grouping (bound 1e-5 of the
-    largest value; measured 1e-7 .. 1e-6 on either side).  One head's decays reach 0.02 per token, another's are 1."""
+    """Against the float64 recurrence, beside the token-by-token kernel on the same states: no further from it than that kernel is, outputs and states, over all of a case's
+    values (a tenth is what the two scatter by; single short sequences by more), and no value off by more than 1e-5 of the largest.  One head's decays reach 0.02
+    per token, another's are 1."""
     rng = np.random.default_rng(heads * 10 + dk + kind)
     total = {s_: sum(n for st in steps for q_, n in st if q_ == s_) for s_ in range(3)}
     unit = lambda a: (a / np.linalg.norm(a.reshape(a.shape[0], -1, dk), axis=-1).repeat(dk, -1).reshape(a.shape)).astype(np.float32)
@@ -331,8 +333,8 @@ def test_state_recurrences_in_chunks(kind, heads, qk_heads, dk, dv, steps):
         else:
             rep = lambda a: a.reshape(-1, qk_heads, dk).repeat_interleave(heads // qk_heads, 1).reshape(a.shape[0], -1)
             want[s_] = orc.decayed_linear_attention(rep(q), rep(k), v, heads, dk, dv, orc.t64(dec)).numpy()
-    off = 8
-    slots = [Slots(3, off + heads * dk * dv + 4) for _ in range(2)]
+    s_off, off = 8, np.zeros(2)          # (off: squared errors, relative to each sequence's size)
+    slots = [Slots(3, s_off + heads * dk * dv + 4) for _ in range(2)]
     at = {0: 0, 1: 0, 2: 0}
     for st in steps:
         seqs = [(n, at[s_], s_) for s_, n in st]
@@ -349,19 +351,37 @@ def test_state_recurrences_in_chunks(kind, heads, qk_heads, dk, dv, steps):
         gates = (p(dev32(dec)), None, None) if kind == 0 else (None, p(g), p(b))
         assert capi().ifa_state_chunked_fits(kind, p(q), qk_heads * dk, p(k), qk_heads * dk, p(v), heads * dv, dk, dv, p(outs[0]), heads * dv + 4)
         ia.check(capi().ifa_state_chunked_f32(kind, p(q), qk_heads * dk, p(k), qk_heads * dk, p(v), heads * dv, heads, qk_heads, dk, dv, *gates, p(d), host, len(st),
-                                              p(slots[0].table), off, p(ws), nb, p(outs[0]), heads * dv + 4, None))
+                                              p(slots[0].table), s_off, p(ws), nb, p(outs[0]), heads * dv + 4, None))
         ia.check(capi().ifa_state_scan_f32(kind, 0, p(q), qk_heads * dk, p(k), qk_heads * dk, p(v), heads * dv, heads, qk_heads, dk, dv, *gates, p(d), len(st),
-                                           p(slots[1].table), off, p(outs[1]), heads * dv + 4, None))
+                                           p(slots[1].table), s_off, p(outs[1]), heads * dv + 4, None))
         sync()
         got, r = [o.cpu().numpy()[:, :heads * dv] for o in outs], 0
         for s_, n in st:
             w = want[s_][at[s_]:at[s_] + n]
             err = [np.abs(x[r:r + n] - w).max() / np.abs(w).max() for x in got]
-            rel = [np.linalg.norm(x[r:r + n] - w) / np.linalg.norm(w) for x in got]
-            print("state", kind, heads, dk, dv, n, "chunks %.2g tokens %.2g" % tuple(err), "rms %.2g %.2g" % tuple(rel))
-            assert err[0] < 1e-5 and rel[0] < 1.5 * rel[1] + 1e-7, (s_, at[s_], n)
+            assert err[0] < 1e-5, (s_, at[s_], n)
+            off += np.array([np.square((x[r:r + n] - w) / np.linalg.norm(w) * n ** 0.5).sum() for x in got])
             r += n; at[s_] += n
-        assert (slots[0].mem[st[0][0]][off + heads * dk * dv:] == 1e9).all() and (slots[0].mem[st[0][0]][:off] == 1e9).all()
+        assert (slots[0].mem[st[0][0]][s_off + heads * dk * dv:] == 1e9).all() and (slots[0].mem[st[0][0]][:s_off] == 1e9).all()
+    print("state", kind, heads, dk, dv, "chunks %.3g tokens %.3g" % tuple(np.sqrt(off / sum(total.values()))))
+    assert off[0] < 1.1 ** 2 * off[1], np.sqrt(off / sum(total.values()))
+    # the states: the recurrence's own, from the tokens
+    off = np.zeros(2)
+    for s_, d in data.items():
+        if d is None:
+            continue
+        q, k, v, g, b = (orc.t64(a) for a in d)
+        L = len(q)
+        kk, vv = k.reshape(L, qk_heads, dk).repeat_interleave(heads // qk_heads, 1), v.reshape(L, heads, dv)
+        S = torch.zeros(heads, dk, dv, dtype=torch.float64)
+        for t in range(L):
+            S = S * (g[t] if kind else orc.t64(dec))[:, None, None]
+            u = b[t][:, None] * (vv[t] - torch.einsum("hk,hkv->hv", kk[t], S)) if kind else vv[t]
+            S = S + kk[t][:, :, None] * u[:, None]
+        for f in range(2):
+            off[f] += float((slots[f].mem[s_][s_off:s_off + S.numel()].cpu().double() - S.reshape(-1)).norm() / S.norm()) ** 2 * L
+    print("state", kind, heads, dk, dv, "left behind: chunks %.3g tokens %.3g" % tuple(np.sqrt(off / sum(total.values()))))
+    assert off[0] < 1.1 ** 2 * off[1], np.sqrt(off / sum(total.values()))
 
 
 # edges of the tiled kernel with a workspace: query tiles of 64 / 128 / 256 (groups of 4, 2, 1 heads), key blocks of 32, windows and kept tokens that begin and end
