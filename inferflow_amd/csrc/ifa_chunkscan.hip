@@ -8,7 +8,7 @@
 //     a triangular system whose solution is U = U0 - W S with U0, W the solutions for the right hand sides beta V and beta G K: both before S is known
 //   o_i = G_i S^T q_i + sum_{j <= i} (G_i / G_j)(q_i . k_j) u_j;     S' = G_last S + sum_j (G_last / G_j) k_j u_j^T
 // so three launches do it: what a chunk needs no state for (all chunks at once), the states from chunk to chunk, the outputs (all chunks at once).
-// Now 66 us (25 + 10 + 30) and 192 us (33 + 114 + 45) per 2048 tokens and layer of 16 heads; at 601 tokens of 8 heads 27 and 81 (were 159 and 312).  The first and
+// Now 60 us (25 + 10 + 25) and 192 us (33 + 114 + 45) per 2048 tokens and layer of 16 heads; at 601 tokens of 8 heads 27 and 81 (were 159 and 312).  The first and
 // third launches wait for their operands (no staging: each is read by one or two waves), the second for its chain.
 // Keys of 64 and 128 have instances here; other sizes go token by token.
 // fp32 operands; a sum that would leave more error than the token-by-token form's few additions do is formed in 64 bits (scores, states of kind 1), from zero in short
@@ -74,10 +74,11 @@ __device__ __forceinline__ float exp_of(double x)
     return ldexpf((float)p, (int)n);
 }
 
-// lane t: the logarithms of the decays of positions 0 .. t of the chunk, summed (none past its end; a decay that has underflowed counts as e^-200)
+// lane t: the logarithms of the decays of positions 0 .. t of the chunk, summed (none past its end; a decay that has underflowed counts as e^-200, NaN stays)
 __device__ __forceinline__ double log_decay_upto(const ChunkArgs &A, const SeqDesc &sd, int t0, int n, int h, int lane)
 {
-    double l = lane < n ? fmax(log((double)A.decay_row[(size_t)(sd.row0 + t0 + lane) * A.heads + h]), -200.0) : 0.0;
+    double l = lane < n ? log((double)A.decay_row[(size_t)(sd.row0 + t0 + lane) * A.heads + h]) : 0.0;
+    l = l < -200.0 ? -200.0 : l;
 #pragma unroll
     for (int k = 1; k < 64; k <<= 1) { const double x = __shfl_up(l, k, 64); if (lane >= k) l += x; }
     return l;
@@ -97,7 +98,7 @@ __global__ void __launch_bounds__(256) k_linear_chunk(ChunkArgs A)
     const float *kp = A.k + (size_t)(sd.row0 + t0) * A.ldk + (size_t)kh * A.dk, *vp = A.v + (size_t)(sd.row0 + t0) * A.ldv + (size_t)h * A.dv + c0;
     float vr[CL / 2];
 #pragma unroll
-    for (int s = 0; s < CL / 2; s++) vr[s] = vp[(size_t)min(2 * s + g, n - 1) * A.ldv + i];
+    for (int s = 0; s < CL / 2; s++) { const float x = vp[(size_t)min(2 * s + g, n - 1) * A.ldv + i]; vr[s] = 2 * s + g < n ? x : 0.0f; }
     for (int kt = (wave >> 1) * 32; kt < A.dk; kt += 64) {
         f32x16c acc;
 #pragma unroll
@@ -337,9 +338,9 @@ __global__ void __launch_bounds__(256) k_delta_pass(ChunkArgs A)
 // outputs U^T P^T, so that a lane's accumulators hold four keys of its position and are the second product's operand as they are.  A lane's 16 bytes of a row of S
 // or U are columns 4 i .. 4 i + 3: column e of each goes to tile e, so that its outputs are 16 bytes side by side again.
 // The scores are summed in 64 bits: q . k of unit vectors is small against its terms, and in 32 bits its rounding was most of the outputs' error.  Everything else
-// is summed 16 terms at a time.  (Error against 64 bits, rms, and time: see the top.)  VEC: rows of U or v of whole aligned 16 bytes.
+// is summed 16 terms at a time.  (Three workgroups on a compute unit: 168 registers.  Error against 64 bits, rms, and time: see the top.)  VEC: rows of U or v of whole aligned 16 bytes.
 template <int KIND, int DK, bool VEC>
-__global__ void __launch_bounds__(256) k_chunk_out(ChunkArgs A)
+__global__ void __launch_bounds__(256, KIND == 0 && DK == 128 ? 2 : 3) k_chunk_out(ChunkArgs A)
 {
     __shared__ double L[4][CL];
     __shared__ float pw[4][CL + 1];
@@ -357,7 +358,7 @@ __global__ void __launch_bounds__(256) k_chunk_out(ChunkArgs A)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     const float *qp = A.q + (size_t)(sd.row0 + t0 + min(pos, n - 1)) * A.ldq + (size_t)kh * DK + 4 * g, *kp = A.k + (size_t)(sd.row0 + t0) * A.ldk + (size_t)kh * DK + 4 * g;
     const size_t at = (size_t)blockIdx.x * A.heads + h;
-    const float *up = KIND == 0 ? A.v + (size_t)(sd.row0 + t0) * A.ldv + (size_t)h * A.dv + cl : A.u + at * CL * A.dv + cl;
+    const float *up = KIND == 0 ? A.v + (size_t)(sd.row0 + t0) * A.ldv + (size_t)h * A.dv : A.u + at * CL * A.dv;
     const size_t ldu = KIND == 0 ? A.ldv : (size_t)A.dv;
     auto row4 = [&](const float *p) -> f32x4c {
         if constexpr (VEC) return *(const f32x4c *)p;
@@ -379,6 +380,12 @@ __global__ void __launch_bounds__(256) k_chunk_out(ChunkArgs A)
 #pragma unroll
         for (int t = 0; t < 4; t++) o[t] += part[t];
     };
+    auto not_finite = [&](const f32x4c (&a)[4]) {
+        float z = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; r++) z += (a[r][0] * 0.0f + a[r][1] * 0.0f) + (a[r][2] * 0.0f + a[r][3] * 0.0f);
+        return z != 0.0f;          // (0, or NaN from any of them)
+    };
     const float *st = A.st + at * DK * A.dv + cl;
 #pragma unroll
     for (int s = 0; s < DK / 16; s++) {
@@ -396,7 +403,7 @@ __global__ void __launch_bounds__(256) k_chunk_out(ChunkArgs A)
         const float *kr = kp + (size_t)min(16 * kt + i, n - 1) * A.ldk;
         f32x4c u[4], w;
 #pragma unroll
-        for (int r = 0; r < 4; r++) u[r] = row4(up + (size_t)min(16 * kt + 4 * r + g, n - 1) * ldu);
+        for (int r = 0; r < 4; r++) u[r] = row4(up + (size_t)min(16 * kt + 4 * r + g, n - 1) * ldu + cl);
 #pragma unroll
         for (int s = 0; s < DK / 16; s++) {
             const f32x4c k = *(const f32x4c *)(kr + 16 * s);
@@ -408,7 +415,20 @@ __global__ void __launch_bounds__(256) k_chunk_out(ChunkArgs A)
             const int j = 16 * kt + 4 * r + g;
             w[r] = j <= pos ? (float)(p[r] * (double)(KIND == 0 ? pw[wave][max(pos - j, 0)] : exp_of(Li - L[wave][j]))) : 0.0f;
         }
-        add16(u, w);
+        if (kt == wave && __builtin_amdgcn_ballot_w64(not_finite(u))) {
+            // among the wave's own positions a later row has weight 0, which would turn infinities and NaN in it into NaN here: the rows one by one, up to the position's own
+#pragma unroll 1
+            for (int j = 0; j < 16; j++) {
+                const float wj = __shfl(j < 8 ? (j < 4 ? w[0] : w[1]) : (j < 12 ? w[2] : w[3]), i + 16 * (j & 3), 64);
+                const float *v = up + (size_t)min(16 * kt + j, n - 1) * ldu;
+#pragma unroll
+                for (int y = 0; y < 4; y++) {
+                    const f32x4c x = row4(v + min(c0 + 16 * g + 4 * y, A.dv - 4));
+#pragma unroll
+                    for (int t = 0; t < 4; t++) o[t][y] = j <= i ? fmaf(wj, x[t], o[t][y]) : o[t][y];
+                }
+            }
+        } else add16(u, w);
     }
     if (pos >= n) return;
     float *dst = A.out + (size_t)(sd.row0 + t0 + pos) * A.ldo + (size_t)h * A.dv + c0 + 16 * g;

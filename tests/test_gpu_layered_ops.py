@@ -384,6 +384,34 @@ def test_state_recurrences_in_chunks(kind, heads, qk_heads, dk, dv, steps):
     assert off[0] < 1.1 ** 2 * off[1], np.sqrt(off / sum(total.values()))
 
 
+@pytest.mark.parametrize("kind,what,value", [(0, "v", np.inf), (0, "v", np.nan), (0, "k", np.nan), (1, "v", -np.inf), (1, "v", np.nan), (1, "k", np.nan), (1, "g", np.nan), (1, "b", np.nan)])
+def test_infinities_and_nan_in_chunks_reach_no_earlier_token_and_no_other_column(kind, what, value):
+    """one value of one token not finite, at the edges of chunks and of their 16 positions: finite outputs and states exactly where the token-by-token form has them"""
+    rng = np.random.default_rng(kind)
+    heads, dk, dv, n = 2, 64, 96, 130
+    unit = lambda a: (a / np.linalg.norm(a.reshape(n, heads, dk), axis=-1).repeat(dk, -1)).astype(np.float32)
+    base = {"q": unit(rng.standard_normal((n, heads * dk))), "k": unit(rng.standard_normal((n, heads * dk))), "v": rng.standard_normal((n, heads * dv)),
+            "g": np.exp(-rng.uniform(0, 0.3, (n, heads))), "b": rng.uniform(0.05, 1, (n, heads))}
+    d, rs, _ = seq_tables([(n, 0, 0)])
+    host = (C.c_int * 4)(0, n, 0, 0)
+    nb = capi().ifa_state_chunked_workspace_bytes(kind, 3, heads, dk, dv)
+    for at in (0, 6, 15, 16, 63, 64, 100, 129):
+        x = {name: np.array(a, np.float32) for name, a in base.items()}
+        x[what][at, x[what].shape[1] - 2] = value
+        x = {name: dev32(a) for name, a in x.items()}
+        gates = (p(dev32(np.array([0.9, 0.99]))), None, None) if kind == 0 else (None, p(x["g"]), p(x["b"]))
+        sl, outs = [Slots(1, heads * dk * dv) for _ in range(2)], [torch.zeros((n, heads * dv), dtype=torch.float32, device="cuda") for _ in range(2)]
+        ws = torch.full((nb // 4,), float("nan"), dtype=torch.float32, device="cuda")
+        a = (p(x["q"]), heads * dk, p(x["k"]), heads * dk, p(x["v"]), heads * dv)
+        ia.check(capi().ifa_state_chunked_f32(kind, *a, heads, heads, dk, dv, *gates, p(d), host, 1, p(sl[0].table), 0, p(ws), nb, p(outs[0]), heads * dv, None))
+        ia.check(capi().ifa_state_scan_f32(kind, 0, *a, heads, heads, dk, dv, *gates, p(d), 1, p(sl[1].table), 0, p(outs[1]), heads * dv, None))
+        sync()
+        for got, want in ((outs[0], outs[1]), (sl[0].mem[0], sl[1].mem[0])):
+            fin = torch.isfinite(want)
+            assert torch.equal(torch.isfinite(got), fin), (at, int(torch.isfinite(got).sum()), int(fin.sum()))
+            assert float((got - want)[fin].abs().max()) < 1e-5 * float(want[fin].abs().max()) if fin.any() else True
+
+
 # edges of the tiled kernel with a workspace: query tiles of 64 / 128 / 256 (groups of 4, 2, 1 heads), key blocks of 32, windows and kept tokens that begin and end
 # inside blocks and meet in one, one chunk and many (short and long key ranges beside each other), continued sequences, head sizes that are not whole 32s or 4s
 TILE_WS = [(4, 1, 128, 128, 1 << 30, 0, [(0, 16)], 1.0), (8, 2, 128, 128, 1 << 30, 0, [(0, 65)], 1.0), (8, 2, 64, 128, 1 << 30, 0, [(0, 700), (0, 3), (610, 90)], 1.0),
