@@ -1068,8 +1068,7 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
     // Not for one row: its grids follow from the HOST's positions, and a step of one row is captured once and replayed while the position on the device goes on.
     if (rows > 1 && rows >= (size_t)tile_min_rows && n_seqs > 0 && dim <= 128 && vdim <= 128 && ws_f32 && (uintptr_t)ws_f32 % 16 == 0) {
         const TilePlan t = tile_plan((const ifa_seq_desc *)seqs_host, n_seqs, heads, kv_heads, dim, vdim, window, keep_first, ws_bytes);
-        IFA_REQUIRE(t.tiles < 65536 && t.groups < 65536 && t.blocks < 65536, "%s: %zu query tiles, %zu key blocks in one step", who, t.tiles, t.blocks);
-        if (t.bytes <= ws_bytes) {
+        if (t.bytes <= ws_bytes && t.tiles < 65536 && t.groups < 65536 && t.blocks < 65536) {          // (a grid's limits; beyond them the tiles below, as without a workspace)
             const int NTK = (dim + 31) / 32, NTV = (vdim + 31) / 32;
             TileArgs A;
             A.n_seqs = n_seqs; A.hpw = t.hpw; A.cb = t.cb; A.tiles = (int)t.tiles; A.shares = t.op_bytes / 4;
@@ -1091,7 +1090,7 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
             return IFA_OK;
         }
     }
-    // prompts without a workspace (or with one that the operands do not fit)
+    // prompts without a workspace (or with one that the operands do not fit, or of more key blocks than a grid has)
     if (rows >= (size_t)tile_min_rows && n_seqs > 0 && dim <= 128 && vdim <= 128) {
         const ifa_seq_desc *sh = (const ifa_seq_desc *)seqs_host;
         size_t tiles = 0;

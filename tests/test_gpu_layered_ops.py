@@ -493,6 +493,27 @@ def test_tiled_attention_takes_fewer_chunks_where_the_workspace_is_small():
         assert np.abs(r - res[0]).max() < 2e-6 * np.abs(res[0]).max()
 
 
+def test_tiled_attention_of_more_key_blocks_than_a_grid_has():
+    """32 queries behind 65600 keys each (2.1 million keys, one slot read by all): the workspace form's launch has a workgroup per block of 32 keys, up to 65535 of
+    them; beyond that the step runs as it does without a workspace"""
+    rng = np.random.default_rng(4)
+    heads, dim, T, ctx = 1, 32, 32, 65600
+    sl = Slots(1, 2 * (ctx + 1) * dim)
+    sl.mem[0].copy_(dev32(rng.standard_normal(2 * (ctx + 1) * dim)))
+    d, rs, _ = seq_tables([(1, ctx, 0)] * T)
+    host = (C.c_int * (4 * T))(*sum([[t, 1, ctx, 0] for t in range(T)], []))
+    q = dev32(rng.standard_normal((T, dim)))
+    nb = capi().ifa_attention_tile_workspace_bytes(host, T, heads, 1, dim, dim, 0, 0)
+    assert nb > 65535 * 3 * 64 * 16 * 4
+    res = []
+    for ws_bytes in (0, nb):
+        ws, out = torch.empty(max(ws_bytes, 4), dtype=torch.uint8, device="cuda"), torch.full((T, dim), float("nan"), dtype=torch.float32, device="cuda")
+        ia.check(capi().ifa_attention_kv_f32(p(q), dim, heads, 1, dim, dim, dim ** -0.5, 0, 0, 0, 0.0, p(d), p(rs), T, p(sl.table), 0, (ctx + 1) * dim, p(out), dim, host, T, 16, 0,
+                                             p(ws) if ws_bytes else None, ws_bytes, None))
+        sync(); res.append(out)
+    assert torch.equal(res[0], res[1]) and bool(torch.isfinite(res[0]).all())
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 8])
 def test_row_products_with_the_norm_or_the_gated_gelu_folded_in(T):
     rng = np.random.default_rng(40 + T)
