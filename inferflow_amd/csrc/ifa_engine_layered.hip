@@ -113,8 +113,11 @@ struct LayeredNet {
     int opt_fuse_post = 1;                 // POSTNORM layers, steps of at most 8 rows: norm-add, depth average, next input convolution and its tail in one launch
                                            // SANDWICH layers, every step size: the norm behind a sub-layer and the norm in front of the next one in one launch
                                            // PRENORM layers: the start of a looped pass inside the norm's launch; steps of at most 8 rows: the norm inside the router's launch
-    float *tile_ws = nullptr; size_t tile_ws_bytes = 0;      // the same for prompts through the tiled attention (grown by the steps that need more)
     float *attn_ws = nullptr; size_t attn_ws_bytes = 0;      // partial results of the windowed attention when a (row, head)'s keys are shared out
+    // Workspaces of prompts through the tiled attention and the chunked recurrences: reserved for one prompt as long as the context when the model is finalized (up to
+    // RESERVE_BYTES each), grown by steps that need more up to opt_workspace_mb each.  A step beyond that, or whose workspace cannot be had, runs without (fp32 tiles, token by token).
+    float *tile_ws = nullptr; size_t tile_ws_bytes = 0;
+    int opt_workspace_mb = 4096; bool step_tile_ws = false;
     bf16_t *a16 = nullptr, *h16 = nullptr; size_t a16_cap = 0, h16_cap = 0; int opt_a16_min = 17;          // activations of a prompt's product rounded to bfloat16; steps of at least this many rows (0: never)
     int opt_fuse_step = 1;                  // single-token steps of PARALLEL layers: norm inside the input product, everything behind the mixers in one launch
     int opt_attn_tile_min = 16;            // steps of at least this many rows run the windowed attention through the tiled kernel
@@ -137,6 +140,54 @@ struct LayeredNet {
 namespace {
 
 int lay_free(void *p) { if (p) (void)hipFree(p); return 0; }
+
+// A workspace that only makes a step faster (the step has a form without it): at least `need` bytes behind p, or false and none.  It grows by half at least, so that a row of
+// longer and longer prompts does not pay for it each time, and never beyond most.  The caller's launches that read the old one have been waited for.
+bool grow_workspace(ifa_model *m, void **p, size_t *have, size_t need, size_t most)
+{
+    if (need > most) return false;
+    if (need <= *have) return true;
+    if (hipStreamSynchronize(m->stream) != hipSuccess) return false;
+    lay_free(*p); *p = nullptr;
+    const size_t sizes[2] = {std::min(most, std::max(need, *have + *have / 2)), need};
+    *have = 0;
+    for (size_t bytes : sizes) {
+        if (hipMalloc(p, bytes) == hipSuccess) { *have = bytes; return true; }
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return false;
+}
+
+size_t tile_workspace_bytes(const LayeredNet *n, const ifa_seq_desc *seqs, int nseq)
+{
+    size_t need = 0;
+    for (const LLayer &L : n->layers) {
+        const ifa_layer_spec &sp = L.spec;
+        if (sp.mixer == IFA_MIX_WINDOW_LINEAR || sp.mixer == IFA_MIX_ROTARY)
+            need = std::max(need, ifa_attention_tile_workspace_bytes(seqs, nseq, sp.a_heads, sp.a_kv_heads, sp.a_dim, sp.mixer == IFA_MIX_ROTARY ? sp.a_vdim : sp.a_dim, sp.a_window,
+                                                                     sp.a_keep_first));
+    }
+    return need;
+}
+
+// (of the layers whose sizes the chunks take)
+size_t scan_workspace_bytes(const LayeredNet *n, size_t chunks)
+{
+    size_t need = 0;
+    for (const LLayer &L : n->layers) {
+        const ifa_layer_spec &sp = L.spec;
+        if (sp.mixer == IFA_MIX_WINDOW_LINEAR && ifa_state_chunked_fits(0, nullptr, 0, nullptr, 0, nullptr, 0, sp.l_dim, sp.l_vdim, nullptr, 0))
+            need = std::max(need, ifa_state_chunked_workspace_bytes(0, chunks, sp.l_heads, sp.l_dim, sp.l_vdim));
+        else if (sp.mixer == IFA_MIX_GATED_DELTA && ifa_state_chunked_fits(1, nullptr, 0, nullptr, 0, nullptr, 0, sp.d_dim, sp.d_vdim, nullptr, 0))
+            need = std::max(need, ifa_state_chunked_workspace_bytes(1, chunks, sp.d_heads, sp.d_dim, sp.d_vdim));
+    }
+    return need;
+}
+
+// what an attention over the step's rows may use: the prompts' workspace, or that of single rows' shares
+struct Scratch { float *p; size_t bytes; };
+Scratch attn_scratch(const LayeredNet *n) { return n->step_tile_ws ? Scratch{n->tile_ws, n->tile_ws_bytes} : Scratch{n->attn_ws, n->attn_ws_bytes}; }
 
 void drop_step_graph(LayeredNet *n)
 {
@@ -598,7 +649,8 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
     else {
         const int H = sp.a_heads, G = sp.a_kv_heads, D = sp.a_dim, DV = sp.a_vdim;
         const size_t OV = (size_t)H * DV;
-        const bool own = sp.a_kv_layer == 0, tile = T >= (size_t)n->opt_attn_tile_min;
+        const bool own = sp.a_kv_layer == 0;
+        const Scratch ws = attn_scratch(n);
         const LLayer &KV = own ? L : n->layers[(size_t)sp.a_kv_layer - 1];
         if ((rc = linear_in(m, L.w_in, NI, W, n->h, h16, T, L.b_in, n->proj, NI))) return rc;
         if ((rc = ifa_qk_rope_store_f32(n->proj + L.c_aq, NI, H, own ? n->proj + L.c_ak : nullptr, NI, own ? n->proj + L.c_av : nullptr, NI, G, D, DV,
@@ -606,7 +658,7 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
                                         slots, KV.o_k, KV.o_v, s))) return rc;
         if ((rc = ifa_attention_kv_f32(n->proj + L.c_aq, NI, H, G, D, DV, sp.a_scale, sp.a_window, sp.a_keep_first, sp.a_sink, sp.a_sink_score, n->seqs_dev,
                                        n->row_seq_dev, T, slots, KV.o_k, KV.o_v, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min,
-                                       c.max_ctx, tile ? n->tile_ws : n->attn_ws, tile ? n->tile_ws_bytes : n->attn_ws_bytes, s))) return rc;
+                                       c.max_ctx, ws.p, ws.bytes, s))) return rc;
         if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, OV, n->m1, OV, T, nullptr, nullptr, 1.0f, 0, n->m2, W))) return rc;
     }
     if ((rc = close_sub(n->m2, L.T(IFA_LT_NORM1B).data, any_ffn ? L.T(IFA_LT_NORM2).data : next_norm, in16 && !(any_ffn && moe)))) return rc;
@@ -670,18 +722,18 @@ int run_prenorm_layer(ifa_model *m, LLayer &L, size_t T, int nseq, int pass, boo
     if (sp.mixer == IFA_MIX_ROTARY) {
         const int H = sp.a_heads, G = sp.a_kv_heads, D = sp.a_dim, DV = sp.a_vdim;
         const size_t OV = (size_t)H * DV;
-        const bool tile = T >= (size_t)n->opt_attn_tile_min;
+        const Scratch ws = attn_scratch(n);
         if ((rc = ifa_qkv_rope_store_f32(n->proj + L.c_aq, NI, H, n->proj + L.c_ak, NI, n->proj + L.c_av, NI, G, D, DV, L.T(IFA_LT_A_Q_NORM).data, L.T(IFA_LT_A_K_NORM).data,
                                          c.eps, sp.a_rot_dims, L.freq, sp.a_vnorm, sp.a_vrot ? L.freq_v : nullptr, n->seqs_dev, n->row_seq_dev, T, slots, L.o_k + po,
                                          L.o_v + po, s))) return rc;
         if (sp.a_sink == 2)
             rc = ifa_attention_kv_sinks_f32(n->proj + L.c_aq, NI, H, G, D, DV, sp.a_scale, sp.a_window, sp.a_keep_first, L.T(IFA_LT_A_SINK).data, n->seqs_dev, n->row_seq_dev, T,
-                                            slots, L.o_k + po, L.o_v + po, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, c.max_ctx, tile ? n->tile_ws : n->attn_ws,
-                                            tile ? n->tile_ws_bytes : n->attn_ws_bytes, s);
+                                            slots, L.o_k + po, L.o_v + po, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, c.max_ctx, ws.p,
+                                            ws.bytes, s);
         else
             rc = ifa_attention_kv_f32(n->proj + L.c_aq, NI, H, G, D, DV, sp.a_scale, sp.a_window, sp.a_keep_first, sp.a_sink, sp.a_sink_score, n->seqs_dev, n->row_seq_dev, T,
-                                      slots, L.o_k + po, L.o_v + po, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, c.max_ctx, tile ? n->tile_ws : n->attn_ws,
-                                      tile ? n->tile_ws_bytes : n->attn_ws_bytes, s);
+                                      slots, L.o_k + po, L.o_v + po, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, c.max_ctx, ws.p,
+                                      ws.bytes, s);
         if (rc) return rc;
         // the sum over values that entered the cache turned by their positions is turned back by the row's own position
         if (sp.a_vrot && (rc = ifa_rotate_heads_f32(n->m1, OV, H, DV, DV & ~1, L.freq_v, -1.0f, n->seqs_dev, n->row_seq_dev, T, s))) return rc;
@@ -973,13 +1025,13 @@ int run_layers(ifa_model *m, size_t T, int nseq)
         }
         if (sp.mixer == IFA_MIX_WINDOW_LINEAR) {
             const size_t AQ = (size_t)sp.a_heads * sp.a_dim, LV = (size_t)sp.l_heads * sp.l_vdim;
-            const bool tile = T >= (size_t)n->opt_attn_tile_min;
+            const Scratch ws = attn_scratch(n);
             // windowed attention: the values are the keys as projected; the cache's K rows hold the normed keys
             if ((rc = ifa_kv_store_f32(n->proj + L.c_ak, NI, n->proj + L.c_ak, NI, sp.a_kv_heads, sp.a_dim, 1, c.eps, n->seqs_dev, n->row_seq_dev, T, slots,
                                        L.o_k, L.o_v, s))) return rc;
             if ((rc = ifa_attention_window_f32(n->proj + L.c_aq, NI, sp.a_heads, sp.a_kv_heads, sp.a_dim, 1, c.eps, sp.a_scale, sp.a_softcap, sp.a_window,
                                                sp.a_keep_first, L.T(IFA_LT_A_REL).data, L.bucket_of, sp.a_buckets, L.T(IFA_LT_A_SINK).data, n->seqs_dev,
-                                               n->row_seq_dev, T, slots, L.o_k, L.o_v, n->m1, AQ, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, tile ? n->tile_ws : n->attn_ws, tile ? n->tile_ws_bytes : n->attn_ws_bytes, s))) return rc;
+                                               n->row_seq_dev, T, slots, L.o_k, L.o_v, n->m1, AQ, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, ws.p, ws.bytes, s))) return rc;
             if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, AQ, n->m1, AQ, T, nullptr, ls1, sp.a_out_scale, 1, n->x, W))) return rc;
             // decayed linear attention
             if ((rc = run_state(m, 0, n->proj + L.c_lq, NI, n->proj + L.c_lk, NI, n->proj + L.c_lv, NI, sp.l_heads, sp.l_heads, sp.l_dim, sp.l_vdim,
@@ -1383,6 +1435,12 @@ int lay_finalize(ifa_model *m)
         IFA_HIP_CHECK(hipMalloc((void **)&n->next_dev, sizeof(int) * ifa_model::RING));
         IFA_HIP_CHECK(hipMalloc((void **)&n->ring_dev, sizeof(int) * ifa_model::RING));
     }
+    {   // (no matter if there is no room: a step asks again)
+        constexpr size_t RESERVE_BYTES = (size_t)256 << 20;
+        const ifa_seq_desc whole{0, n->cfg.max_ctx, 0, 0};
+        (void)grow_workspace(m, (void **)&n->tile_ws, &n->tile_ws_bytes, std::min(RESERVE_BYTES, tile_workspace_bytes(n, &whole, 1)), RESERVE_BYTES);
+        (void)grow_workspace(m, &n->scan_ws, &n->scan_ws_bytes, std::min(RESERVE_BYTES, scan_workspace_bytes(n, ((size_t)n->cfg.max_ctx + 63) / 64)), RESERVE_BYTES);
+    }
     m->finalized = true;
     return IFA_OK;
 }
@@ -1417,9 +1475,10 @@ int lay_set_option(ifa_model *m, const char *name, int value)
     if (!strcmp(name, "ssm_chunk_min")) { n->opt_ssm_chunk_min = value; return IFA_OK; }
     if (!strcmp(name, "a16_min")) { n->opt_a16_min = value; return IFA_OK; }
     if (!strcmp(name, "attn_tile_min")) { n->opt_attn_tile_min = value; drop_step_graph(n); return IFA_OK; }
+    if (!strcmp(name, "workspace_mb")) { n->opt_workspace_mb = value; return IFA_OK; }
     if (!strcmp(name, "graph")) { n->opt_graph = value; drop_step_graph(n); return IFA_OK; }
     if (!strcmp(name, "ops32")) { IFA_HIP_CHECK(hipStreamSynchronize(m->stream)); n->cfg.ops32 = value ? 1 : 0; drop_step_graph(n); return IFA_OK; }
-    return ifa_fail(IFA_ERR_ARG, "ifa_model_set_option: unknown option '%s' (layer-list model: tap_layers, graph, ops32, attn_tile_min, a16_min, fuse_rows, fuse_post, ssm_chunk_min, scan_chunk_min, fuse_step)", name);
+    return ifa_fail(IFA_ERR_ARG, "ifa_model_set_option: unknown option '%s' (layer-list model: tap_layers, graph, ops32, attn_tile_min, a16_min, fuse_rows, fuse_post, ssm_chunk_min, scan_chunk_min, fuse_step, workspace_mb)", name);
 }
 
 int lay_set_excluded(ifa_model *m, const int *ids_host, int cnt)
@@ -1533,22 +1592,14 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
         IFA_HIP_CHECK(hipMalloc((void **)&n->vx, n->step_ctx_rows * n->vx_max * 4));
         n->expand_rows = n->step_ctx_rows;
     }
+    const size_t most = (size_t)std::max(n->opt_workspace_mb, 0) << 20;
     n->scan_chunks = 0;
     {
-        int longest = 0; size_t chunks = 0, need = 0;
+        int longest = 0; size_t chunks = 0;
         for (int q = 0; q < nseq; q++) { longest = std::max(longest, lens[q]); chunks += ((size_t)lens[q] + 63) / 64; }
-        if (longest >= std::max(n->opt_scan_chunk_min, 2))
-            for (const LLayer &L : n->layers) {
-                const ifa_layer_spec &sp = L.spec;
-                if (sp.mixer == IFA_MIX_WINDOW_LINEAR) need = std::max(need, ifa_state_chunked_workspace_bytes(0, chunks, sp.l_heads, sp.l_dim, sp.l_vdim));
-                else if (sp.mixer == IFA_MIX_GATED_DELTA) need = std::max(need, ifa_state_chunked_workspace_bytes(1, chunks, sp.d_heads, sp.d_dim, sp.d_vdim));
-            }
-        if (need) n->scan_chunks = chunks;
-        if (need > n->scan_ws_bytes) {
-            IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
-            lay_free(n->scan_ws); n->scan_ws = nullptr; n->scan_ws_bytes = 0;
-            IFA_HIP_CHECK(hipMalloc(&n->scan_ws, need));
-            n->scan_ws_bytes = need;
+        if (longest >= std::max(n->opt_scan_chunk_min, 2)) {
+            const size_t need = scan_workspace_bytes(n, chunks);
+            if (need && grow_workspace(m, &n->scan_ws, &n->scan_ws_bytes, need, most)) n->scan_chunks = chunks;
         }
     }
     n->ssm_chunks = 0;
@@ -1567,21 +1618,8 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
             }
         }
     }
-    if (T >= (size_t)std::max(n->opt_attn_tile_min, 2)) {          // (a step of one row takes no tiles of the workspace's form, see attention_launch)
-        size_t need = 0;
-        for (const LLayer &L : n->layers) {
-            const ifa_layer_spec &sp = L.spec;
-            if (sp.mixer == IFA_MIX_WINDOW_LINEAR || sp.mixer == IFA_MIX_ROTARY)
-                need = std::max(need, ifa_attention_tile_workspace_bytes(n->seqs_host.data(), nseq, sp.a_heads, sp.a_kv_heads, sp.a_dim,
-                                                                         sp.mixer == IFA_MIX_ROTARY ? sp.a_vdim : sp.a_dim, sp.a_window, sp.a_keep_first));
-        }
-        if (need > n->tile_ws_bytes) {
-            IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
-            lay_free(n->tile_ws); n->tile_ws = nullptr; n->tile_ws_bytes = 0;
-            IFA_HIP_CHECK(hipMalloc((void **)&n->tile_ws, need));
-            n->tile_ws_bytes = need;
-        }
-    }
+    n->step_tile_ws = T >= (size_t)std::max(n->opt_attn_tile_min, 2)          // (a step of one row takes no tiles of the workspace's form, see attention_launch)
+                      && grow_workspace(m, (void **)&n->tile_ws, &n->tile_ws_bytes, tile_workspace_bytes(n, n->seqs_host.data(), nseq), most);
     if ((rc = run_layers(m, T, nseq))) return rc;
     ifa_stream s = (ifa_stream)m->stream;
     if (all) {
@@ -1648,7 +1686,7 @@ int lay_decode(ifa_model *m, int first_token, int start_pos, int n_steps, int *o
     if ((rc = check_span(m, n_steps, start_pos, nullptr)) || (rc = ensure_slot(m, n->cur_slot)) || (rc = ensure_rows(m, 1, 1)) || (rc = ensure_logits(m, 1))) return rc;
     if (n->opt_graph && !n->opt_tap_layers && !n->step_exec) {      // (the slot is read from the device tables: one capture serves every slot)
         drop_step_graph(n);
-        n->step_expand = false; n->scan_chunks = 0;
+        n->step_expand = false; n->scan_chunks = 0; n->step_tile_ws = false;
         n->seqs_host.assign(1, ifa_seq_desc{0, 1, start_pos, n->cur_slot});      // (the launches are shaped by it: one sequence, one row)
         IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
         IFA_HIP_CHECK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
@@ -1667,7 +1705,7 @@ int lay_decode(ifa_model *m, int first_token, int start_pos, int n_steps, int *o
     std::vector<int> tok(1, first_token), pos(1, start_pos), rs(1, 0);
     std::vector<ifa_seq_desc> sq(1); sq[0] = ifa_seq_desc{0, 1, start_pos, n->cur_slot};
     if ((rc = upload_tables(m, tok, pos, rs, sq))) return rc;
-    n->step_expand = false; n->scan_chunks = 0;
+    n->step_expand = false; n->scan_chunks = 0; n->step_tile_ws = false;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (elapsed_ms) { IFA_HIP_CHECK(hipEventCreate(&e0)); IFA_HIP_CHECK(hipEventCreate(&e1)); IFA_HIP_CHECK(hipEventRecord(e0, m->stream)); }
     for (int st = 0; st < n_steps; st++) {

@@ -299,6 +299,25 @@ def test_ini_route_and_trace_replay_tool(tmp_path):
         assert fx.rel_err(g, np.stack(exp)).max() < TOL32, s
 
 
+CHUNKED = fx.config([fx.parallel_layer(heads=4, kv_heads=2, dim=64, window=200, keep_first=3, lin_heads=3, lin_dim=64, lin_vdim=96, ff=72),
+                     fx.delta_layer(heads=4, kv_heads=2, dim=64, vdim=32, conv=3, ff=40)], width=72, vocab=97)
+
+
+@pytest.mark.parametrize("limit", [4096, 0])
+def test_prompts_with_and_without_the_workspaces_of_tiles_and_chunks(tmp_path, limit):
+    """a workspace that may not be had (limit 0) costs time, not the step: prompts of growing length, portions on both sides of the chunked form's border"""
+    import inferflow_amd as ia
+    w = fx.random_weights(CHUNKED, 31)
+    toks = tokens_for(CHUNKED, 420, 32)
+    want = oracle_logits(CHUNKED, w, toks)
+    eng = engine_for(tmp_path, CHUNKED, w)
+    ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"workspace_mb", limit))
+    for n in (20, 130, 420):
+        assert fx.rel_err(run_whole(eng, toks[:n])[0], want[:n]).max() < TOL32, n
+    assert fx.rel_err(run_portions(eng, toks, [113, 20, 1, 150]), want).max() < TOL32
+    eng.close()
+
+
 @pytest.mark.parametrize("ctx", [340, 60])      # keys of a head by six workgroups whose shares the last launch joins / by one
 def test_single_token_steps_in_few_launches(tmp_path, ctx):
     """Steps of one token whose layers' sizes allow the norm inside the input product, both mixers in one launch and everything behind them in another: against the
