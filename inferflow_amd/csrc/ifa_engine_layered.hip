@@ -128,11 +128,11 @@ struct LayeredNet {
     int *moe_idx = nullptr, *ctx0_dev = nullptr; void *moe_ws = nullptr; size_t moe_ws_bytes = 0, expand_rows = 0, kx_max = 0, vx_max = 0, top_max = 0;
     bool any_depth_avg = false, any_latent = false, any_moe = false, latent_tile_ok = true, step_expand = false;
     std::vector<int> ctx0_host; size_t step_ctx_rows = 0;
-    // state-space layers: steps whose longest sequence brings at least opt_ssm_chunk_min tokens run in chunks (ssm_chunks > 0), their workspace
-    // the recurrences of WINDOW_LINEAR and GATED_DELTA layers: steps whose longest sequence brings at least this many tokens run in chunks of 64 (scan_chunks > 0).
+    // the recurrences of WINDOW_LINEAR and GATED_DELTA layers: steps whose longest sequence brings at least this many tokens run in chunks of 64 (scan_chunks > 0; 0: never).
     // Measured where the two meet (whole Gelarax prompts, chunks / token by token): 96 tokens 1494 / 1467 and 2198 / 2163 us (widths 1024 / 2048), 128 tokens
     // 1520 / 1560 and 2219 / 2269
     int opt_scan_chunk_min = 112; size_t scan_chunks = 0, scan_ws_bytes = 0; void *scan_ws = nullptr;
+    // state-space layers: steps whose longest sequence brings at least opt_ssm_chunk_min tokens run in chunks (ssm_chunks > 0), their workspace
     bool any_ssm = false; int opt_ssm_chunk_min = 48; size_t ssm_chunks = 0, ssm_ws_bytes = 0; void *ssm_ws = nullptr;
     hipGraphExec_t step_exec = nullptr; hipGraph_t step_graph = nullptr; int step_slot = -1;
 };
@@ -1597,7 +1597,7 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
     {
         int longest = 0; size_t chunks = 0;
         for (int q = 0; q < nseq; q++) { longest = std::max(longest, lens[q]); chunks += ((size_t)lens[q] + 63) / 64; }
-        if (longest >= std::max(n->opt_scan_chunk_min, 2)) {
+        if (n->opt_scan_chunk_min > 0 && longest >= std::max(n->opt_scan_chunk_min, 2)) {
             const size_t need = scan_workspace_bytes(n, chunks);
             if (need && grow_workspace(m, &n->scan_ws, &n->scan_ws_bytes, need, most)) n->scan_chunks = chunks;
         }

@@ -318,6 +318,18 @@ def test_prompts_with_and_without_the_workspaces_of_tiles_and_chunks(tmp_path, l
     eng.close()
 
 
+def test_chunked_recurrences_are_switched_off_by_0(tmp_path):
+    """the bits of the token-by-token form, which a border above every prompt has too; the chunks' differ"""
+    import inferflow_amd as ia
+    eng = engine_for(tmp_path, CHUNKED, fx.random_weights(CHUNKED, 33))
+    toks, out = tokens_for(CHUNKED, 200, 34), {}
+    for border in (0, 1 << 30, 112):
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"scan_chunk_min", border))
+        out[border] = run_whole(eng, toks)[0]
+    assert np.array_equal(out[0], out[1 << 30]) and not np.array_equal(out[0], out[112])
+    eng.close()
+
+
 @pytest.mark.parametrize("ctx", [340, 60])      # keys of a head by six workgroups whose shares the last launch joins / by one
 def test_single_token_steps_in_few_launches(tmp_path, ctx):
     """Steps of one token whose layers' sizes allow the norm inside the input product, both mixers in one launch and everything behind them in another: against the
