@@ -185,9 +185,13 @@ size_t scan_workspace_bytes(const LayeredNet *n, size_t chunks)
     return need;
 }
 
-// what an attention over the step's rows may use: the prompts' workspace, or that of single rows' shares
+// what an attention over the step's rows may use: the prompts' workspace where tiles take its heads, else that of single rows' shares (heads above 128 go row by row
+// in prompts too: 24 rows behind 700 keys, 4 heads of 256, 20 us with shares)
 struct Scratch { float *p; size_t bytes; };
-Scratch attn_scratch(const LayeredNet *n) { return n->step_tile_ws ? Scratch{n->tile_ws, n->tile_ws_bytes} : Scratch{n->attn_ws, n->attn_ws_bytes}; }
+Scratch attn_scratch(const LayeredNet *n, int dim, int vdim)
+{
+    return n->step_tile_ws && dim <= 128 && vdim <= 128 ? Scratch{n->tile_ws, n->tile_ws_bytes} : Scratch{n->attn_ws, n->attn_ws_bytes};
+}
 
 void drop_step_graph(LayeredNet *n)
 {
@@ -650,7 +654,7 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
         const int H = sp.a_heads, G = sp.a_kv_heads, D = sp.a_dim, DV = sp.a_vdim;
         const size_t OV = (size_t)H * DV;
         const bool own = sp.a_kv_layer == 0;
-        const Scratch ws = attn_scratch(n);
+        const Scratch ws = attn_scratch(n, D, DV);
         const LLayer &KV = own ? L : n->layers[(size_t)sp.a_kv_layer - 1];
         if ((rc = linear_in(m, L.w_in, NI, W, n->h, h16, T, L.b_in, n->proj, NI))) return rc;
         if ((rc = ifa_qk_rope_store_f32(n->proj + L.c_aq, NI, H, own ? n->proj + L.c_ak : nullptr, NI, own ? n->proj + L.c_av : nullptr, NI, G, D, DV,
@@ -722,7 +726,7 @@ int run_prenorm_layer(ifa_model *m, LLayer &L, size_t T, int nseq, int pass, boo
     if (sp.mixer == IFA_MIX_ROTARY) {
         const int H = sp.a_heads, G = sp.a_kv_heads, D = sp.a_dim, DV = sp.a_vdim;
         const size_t OV = (size_t)H * DV;
-        const Scratch ws = attn_scratch(n);
+        const Scratch ws = attn_scratch(n, D, DV);
         if ((rc = ifa_qkv_rope_store_f32(n->proj + L.c_aq, NI, H, n->proj + L.c_ak, NI, n->proj + L.c_av, NI, G, D, DV, L.T(IFA_LT_A_Q_NORM).data, L.T(IFA_LT_A_K_NORM).data,
                                          c.eps, sp.a_rot_dims, L.freq, sp.a_vnorm, sp.a_vrot ? L.freq_v : nullptr, n->seqs_dev, n->row_seq_dev, T, slots, L.o_k + po,
                                          L.o_v + po, s))) return rc;
@@ -1025,7 +1029,7 @@ int run_layers(ifa_model *m, size_t T, int nseq)
         }
         if (sp.mixer == IFA_MIX_WINDOW_LINEAR) {
             const size_t AQ = (size_t)sp.a_heads * sp.a_dim, LV = (size_t)sp.l_heads * sp.l_vdim;
-            const Scratch ws = attn_scratch(n);
+            const Scratch ws = attn_scratch(n, sp.a_dim, sp.a_dim);
             // windowed attention: the values are the keys as projected; the cache's K rows hold the normed keys
             if ((rc = ifa_kv_store_f32(n->proj + L.c_ak, NI, n->proj + L.c_ak, NI, sp.a_kv_heads, sp.a_dim, 1, c.eps, n->seqs_dev, n->row_seq_dev, T, slots,
                                        L.o_k, L.o_v, s))) return rc;

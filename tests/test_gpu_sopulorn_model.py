@@ -370,6 +370,19 @@ def test_generation_over_key_block_edges_with_single_rows_sent_to_the_tiles(tmp_
     eng.close()
 
 
+def test_heads_above_128_share_their_keys_out_in_steps_of_a_few_rows(tmp_path):
+    """heads that no tile takes go row by row, a few rows' keys shared out to several workgroups whatever border the tiles have: the same bits"""
+    import inferflow_amd as ia
+    cfg = fx.config([fx.attention_layer(heads=2, kv_heads=1, dim=160, vdim=144, rot_dims=32)], width=64, vocab=97)
+    eng = engine_for(tmp_path, cfg, fx.random_weights(cfg, 41))
+    toks, out = tokens_for(cfg, 420, 42), []
+    for border in (16, 1 << 30):
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"attn_tile_min", border))
+        out.append(run_portions(eng, toks, [400, 20]))
+    assert np.array_equal(out[0][400:], out[1][400:])
+    eng.close()
+
+
 def test_ini_route_and_trace_replay_tool(tmp_path):
     from inferflow_amd.engine import InferenceEngine
     w = fx.random_weights(MIXED, 17)
