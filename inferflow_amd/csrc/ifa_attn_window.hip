@@ -534,43 +534,75 @@ __host__ __device__ __forceinline__ TileBlocks tile_blocks(int p0, int nq, int w
 
 struct TileArgs { int n_seqs, hpw, cb, tiles; size_t shares; };      // shares: where the chunks' partial results begin in the workspace (floats), behind the operands
 
-// the sequence and the tile of it (tiles of qw queries, numbered over the sequences) and the operand blocks of the sequences before it, or false
-__device__ __forceinline__ bool tile_of(const WinAttnArgs &P, int n_seqs, int qw, int &tile, SeqDesc &sd, int &block0)
-{
-    block0 = 0;
-    for (int sq = 0; sq < n_seqs; sq++) {
-        sd = P.seqs[sq];
-        const int nt = (sd.n + qw - 1) / qw;
-        if (tile < nt) return true;
-        tile -= nt;
-        block0 += seq_blocks(sd.pos0, sd.n, P.window, P.keep_first).count;
-    }
-    return false;
-}
-
-// The id-th chunk of the step, the chunks numbered tile by tile from the last tile on: its tile and its number there.  A grid of tiles x chunks would do without
-// this, but its empty places leave some XCD with more chunks than compute units, and the launch takes twice as long (100 against 50 us at 2048 tokens).
-__device__ __forceinline__ bool chunk_of(const WinAttnArgs &P, const TileArgs &A, int qw, int id, int &tile_g, int &chunk)
+// The item (of n) that a number running over all items' counts falls into, or -1; id becomes the number inside it.  A wave looks at 64 items at a time (walked by one thread,
+// a step of 1024 sequences behind 100 keys each took 10.6 ms, now 0.37; 512 behind 200 2.0 ms, now 0.26).  count: called by all lanes, -1 for none.
+template <class Count>
+__device__ __forceinline__ int item_of(int n, int &id, Count count)
 {
     const int lane = threadIdx.x & 63;
-    for (int t0 = 0; t0 < A.tiles; t0 += 64) {
-        int n = 0, tile = A.tiles - 1 - t0 - lane, block0;
-        SeqDesc sd;
-        if (tile >= 0 && tile_of(P, A.n_seqs, qw, tile, sd, block0))
-            n = (tile_blocks(sd.pos0 + tile * qw, min(qw, sd.n - tile * qw), P.window, P.keep_first).nb + A.cb - 1) / A.cb;
-        int upto = n;
+    for (int s0 = 0; s0 < n; s0 += 64) {
+        const int c = count(s0 + lane < n ? s0 + lane : -1);
+        int upto = c;
 #pragma unroll
         for (int k = 1; k < 64; k <<= 1) { const int x = __shfl_up(upto, k, 64); if (lane >= k) upto += x; }
         const uint64_t past = __builtin_amdgcn_ballot_w64(upto > id);
         if (past) {
             const int at = __builtin_ctzll(past);
-            tile_g = A.tiles - 1 - t0 - at;
-            chunk = id - (__builtin_amdgcn_readlane(upto, at) - __builtin_amdgcn_readlane(n, at));
-            return true;
+            id -= __builtin_amdgcn_readlane(upto, at) - __builtin_amdgcn_readlane(c, at);
+            return s0 + at;
         }
         id -= __builtin_amdgcn_readlane(upto, 63);
     }
-    return false;
+    return -1;
+}
+__device__ __forceinline__ int wave_sum_i(int v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+// The id-th chunk of the step, the chunks numbered tile by tile from the last sequence's last tile on: its sequence, its tile there (of qw queries) and over the step, its number
+// in the tile, the operand blocks of the sequences before.  A grid of tiles x chunks would do without this, but its empty places leave some XCD with more chunks
+// than compute units, and the launch takes twice as long (100 against 50 us at 2048 tokens).
+struct ChunkPlace { SeqDesc sd; int tile, tile_g, chunk, block0; };
+__device__ __forceinline__ bool chunk_of(const WinAttnArgs &P, const TileArgs &A, int qw, int id, ChunkPlace &at)
+{
+    const int lane = threadIdx.x & 63;
+    auto chunks = [&](int pos0, int n, int tile) { return (tile_blocks(pos0 + tile * qw, min(qw, n - tile * qw), P.window, P.keep_first).nb + A.cb - 1) / A.cb; };
+    int sq = 0;
+    if (A.n_seqs > 1) {
+        const int back = item_of(A.n_seqs, id, [&](int x) {
+            int pos0 = 0, n = 0, c = 0;
+            if (x >= 0) { const SeqDesc &sd = P.seqs[A.n_seqs - 1 - x]; pos0 = sd.pos0; n = sd.n; }
+            const int nt = (n + qw - 1) / qw;
+            if (nt <= 4) for (int t = 0; t < nt; t++) c += chunks(pos0, n, t);
+            for (uint64_t many = __builtin_amdgcn_ballot_w64(nt > 4); many; many &= many - 1) {          // (sequences of many tiles: the wave counts them together)
+                const int l = __builtin_ctzll(many), p = __builtin_amdgcn_readlane(pos0, l), m = __builtin_amdgcn_readlane(n, l), mt = __builtin_amdgcn_readlane(nt, l);
+                int part = 0;
+                for (int t = lane; t < mt; t += 64) part += chunks(p, m, t);
+                part = wave_sum_i(part);
+                if (lane == l) c = part;
+            }
+            return c;
+        });
+        if (back < 0) return false;
+        sq = A.n_seqs - 1 - back;
+    }
+    const SeqDesc sd = P.seqs[sq];
+    const int nt = (sd.n + qw - 1) / qw, back = item_of(nt, id, [&](int x) { return x >= 0 ? chunks(sd.pos0, sd.n, nt - 1 - x) : 0; });
+    if (back < 0) return false;
+    int blocks = 0, tiles = 0;
+    for (int s = lane; s < sq; s += 64) {
+        const SeqDesc &b = P.seqs[s];
+        blocks += seq_blocks(b.pos0, b.n, P.window, P.keep_first).count;
+        tiles += (b.n + qw - 1) / qw;
+    }
+    if (sq > 0) { blocks = wave_sum_i(blocks); tiles = wave_sum_i(tiles); }
+    at.sd = sd; at.chunk = id; at.tile = nt - 1 - back;
+    at.block0 = __builtin_amdgcn_readfirstlane(blocks);
+    at.tile_g = __builtin_amdgcn_readfirstlane(tiles) + at.tile;
+    return true;
 }
 
 // Operands of one block of 32 keys as the matrix instructions take them, [part][16 columns][lane][8]: keys (lane = 32 g + key, columns 16 ks + 8 g ..), then
@@ -584,16 +616,11 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, int n_seqs)
 {
     constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK;
     const int tid = threadIdx.x, kvh = blockIdx.x, dk = P.dim, dv = P.vdim;
-    int at = blockIdx.y, sq = 0;
-    SeqDesc sd;
-    SeqBlocks sb;
-    for (; sq < n_seqs; sq++) {
-        sd = P.seqs[sq];
-        sb = seq_blocks(sd.pos0, sd.n, P.window, P.keep_first);
-        if (at < sb.count) break;
-        at -= sb.count;
-    }
-    if (sq >= n_seqs) return;
+    int at = blockIdx.y;
+    const int sq = item_of(n_seqs, at, [&](int x) { if (x < 0) return 0; const SeqDesc &b = P.seqs[x]; return seq_blocks(b.pos0, b.n, P.window, P.keep_first).count; });
+    if (sq < 0) return;
+    const SeqDesc sd = P.seqs[sq];
+    const SeqBlocks sb = seq_blocks(sd.pos0, sd.n, P.window, P.keep_first);
     const int kb0 = (at < sb.kept ? at : sb.first + at - sb.kept) * WT_K, last = sd.pos0 + sd.n - 1;
     const size_t kvd = (size_t)P.kv_heads * dk, vvd = (size_t)P.kv_heads * dv;
     gfloat *kc = (gfloat *)(P.slot_base[sd.slot] + P.k_off + (size_t)kvh * dk), *vc = (gfloat *)(P.slot_base[sd.slot] + P.v_off + (size_t)kvh * dv);
@@ -637,11 +664,10 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5;
     const int h = blockIdx.x * A.hpw + wave % A.hpw, qsub = wave / A.hpw, kvh = blockIdx.x * A.hpw / (P.heads / P.kv_heads), dk = P.dim, dv = P.vdim;
     const int qw = 32 * (WT_WAVES / A.hpw);
-    int tile_g, chunk, block0;
-    if (!chunk_of(P, A, qw, blockIdx.y, tile_g, chunk)) return;
-    int tile = tile_g;
-    SeqDesc sd;
-    if (!tile_of(P, A.n_seqs, qw, tile, sd, block0)) return;
+    ChunkPlace at;
+    if (!chunk_of(P, A, qw, blockIdx.y, at)) return;
+    const SeqDesc sd = at.sd;
+    const int tile = at.tile, tile_g = at.tile_g, chunk = at.chunk, block0 = at.block0;
     const int r0 = sd.row0 + tile * qw, nq = min(qw, sd.n - tile * qw), p0 = sd.pos0 + tile * qw;
     const SeqBlocks sb = seq_blocks(sd.pos0, sd.n, P.window, P.keep_first);
     const TileBlocks tb = tile_blocks(p0, nq, P.window, P.keep_first);
@@ -823,9 +849,10 @@ __global__ void __launch_bounds__(256) k_attn_tile_combine(WinAttnArgs P, TileAr
 {
     __shared__ float fs[WT_MAX_CHUNKS][32], rows[32][129];
     const int tid = threadIdx.x, wave = blockIdx.z, h = blockIdx.x * A.hpw + wave % A.hpw, qsub = wave / A.hpw, dv = P.vdim, qw = 32 * (WT_WAVES / A.hpw), tile_g = blockIdx.y;
-    int tile = tile_g, block0;
-    SeqDesc sd;
-    if (!tile_of(P, A.n_seqs, qw, tile, sd, block0)) return;
+    int tile = tile_g;
+    const int sq = item_of(A.n_seqs, tile, [&](int x) { return x >= 0 ? (P.seqs[x].n + qw - 1) / qw : 0; });
+    if (sq < 0) return;
+    const SeqDesc sd = P.seqs[sq];
     const int nq = min(qw, sd.n - tile * qw), nq_w = min(32, nq - 32 * qsub);
     const int nch = (tile_blocks(sd.pos0 + tile * qw, nq, P.window, P.keep_first).nb + A.cb - 1) / A.cb;
     if (nch <= 1 || nq_w <= 0) return;
@@ -893,7 +920,11 @@ TilePlan tile_plan(const ifa_seq_desc *sh, int n_seqs, int heads, int kv_heads, 
     size_t cb = std::max<size_t>({2, total * hx / WT_SLOTS, (most + WT_MAX_CHUNKS - 1) / WT_MAX_CHUNKS});
     auto chunks = [&]() { return (most + cb - 1) / cb; };
     auto groups = [&]() { size_t n = 0; for (int nb : nbs) n += ((size_t)nb + cb - 1) / cb; return n; };
-    while (chunks() > 1 && groups() * hx > WT_SLOTS) cb++;
+    if (chunks() > 1 && groups() * hx > WT_SLOTS) {          // the smallest that fits, or one chunk a tile (fewer groups the larger it is: found by halves)
+        size_t lo = cb, hi = most;
+        while (hi - lo > 1) { cb = lo + (hi - lo) / 2; (groups() * hx > WT_SLOTS ? lo : hi) = cb; }
+        cb = hi;
+    }
     while (chunks() > 1 && t.op_bytes + t.tiles * hx * chunks() * share > ws_bytes) cb = std::max(cb + 1, (most + chunks() - 2) / (chunks() - 1));
     t.cb = (int)cb; t.chunks = (int)chunks(); t.groups = groups();
     t.bytes = t.op_bytes + (t.chunks > 1 ? t.tiles * hx * (size_t)t.chunks * share : 0);

@@ -514,6 +514,31 @@ def test_tiled_attention_of_more_key_blocks_than_a_grid_has():
     assert torch.equal(res[0], res[1]) and bool(torch.isfinite(res[0]).all())
 
 
+@pytest.mark.parametrize("window,keep", [(1 << 30, 0), (90, 40)])
+def test_tiled_attention_over_many_sequences(window, keep):
+    """130 sequences, most of one row, some of several and of more than four query tiles, at places that a wave looks at together and one by one: the rows' kernel's
+    outputs within the fp32 roundings of 300 keys (the bound of the test above)"""
+    rng = np.random.default_rng(6)
+    heads, kv_heads, dim, ctx = 4, 1, 32, 420
+    seqs = [(1, int(rng.integers(0, 400))) for _ in range(130)]
+    for at, one in ((0, (270, 3)), (5, (33, 64)), (63, (330, 31)), (64, (257, 0)), (70, (64, 100)), (127, (300, 100)), (129, (400, 0))):
+        seqs[at] = one
+    sl = Slots(3, 2 * ctx * dim)
+    for m in sl.mem:
+        m.copy_(dev32(rng.standard_normal(2 * ctx * dim)))
+    d, rs, T = seq_tables([(n, pos0, i % 3) for i, (n, pos0) in enumerate(seqs)])
+    host = (C.c_int * (4 * len(seqs)))(*d.cpu().numpy().reshape(-1).tolist())
+    q = dev32(rng.standard_normal((T, heads * dim)))
+    nb = capi().ifa_attention_tile_workspace_bytes(host, len(seqs), heads, kv_heads, dim, dim, 0 if window == 1 << 30 else window, keep)
+    res = []
+    for tile_min in (1 << 30, 16):
+        ws, out = torch.full((nb // 4,), float("nan"), dtype=torch.float32, device="cuda"), torch.full((T, heads * dim), float("nan"), dtype=torch.float32, device="cuda")
+        ia.check(capi().ifa_attention_kv_f32(p(q), heads * dim, heads, kv_heads, dim, dim, dim ** -0.5, 0 if window == 1 << 30 else window, keep, 0, 0.0, p(d), p(rs), T, p(sl.table), 0,
+                                             ctx * dim, p(out), heads * dim, host, len(seqs), tile_min, ctx, p(ws) if tile_min == 16 else None, nb, None))
+        sync(); res.append(out)
+    assert float((res[0] - res[1]).abs().max()) < 2e-6 * float(res[0].abs().max())
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 8])
 def test_row_products_with_the_norm_or_the_gated_gelu_folded_in(T):
     rng = np.random.default_rng(40 + T)
