@@ -413,37 +413,50 @@ __global__ void __launch_bounds__(256) k_lin_rows(LinArgs P)
 #pragma unroll
         for (int t = 0; t < TT; t++) acc[t] = 0.0f;
         const bf16_t *w = P.W + (size_t)n * P.K;
-        if (P.vec && PRO == 2) {          // (gate, up and the weight are enough in flight, and the activations the longer part)
+        // (with a prologue its operands and the weight are enough in flight and the activations the longer part; up to four rows the waves are, of a large matrix: 32000 rows of 1024,
+        // 2 / 4 rows 14.2 / 20.9 us, pieces first 15.7 / 23.0)
+        if (P.vec && (PRO != 0 || TT <= 4)) {
             for (int k = lane * 8; k < P.K; k += 512) {
                 const u32x4v wv = *reinterpret_cast<const u32x4v *>(w + k);
-                float w8[8];
+                float w8[8], g8[8];
 #pragma unroll
                 for (int e = 0; e < 4; e++) { w8[2 * e] = __uint_as_float(wv[e] << 16); w8[2 * e + 1] = __uint_as_float(wv[e] & 0xFFFF0000u); }
+                if (PRO == 1) {
+                    const u32x4v gv = *reinterpret_cast<const u32x4v *>(P.norm_w + k);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) { g8[2 * e] = __uint_as_float(gv[e] << 16); g8[2 * e + 1] = __uint_as_float(gv[e] & 0xFFFF0000u); }
+                }
 #pragma unroll
                 for (int t = 0; t < TT; t++) {
                     const float *a = P.A + (size_t)min(t, P.T - 1) * P.lda + k;
                     const float4 v0 = *reinterpret_cast<const float4 *>(a), v1 = *reinterpret_cast<const float4 *>(a + 4);
-                    const float4 u0 = *reinterpret_cast<const float4 *>(a + P.K), u1 = *reinterpret_cast<const float4 *>(a + P.K + 4);
-                    const float x8[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w}, u8[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+                    float x8[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+                    if (PRO == 1) {
+#pragma unroll
+                        for (int e = 0; e < 8; e++) x8[e] = (x8[e] - mean[t]) * rstd[t] * g8[e];
+                    } else if (PRO == 2) {
+                        const float4 u0 = *reinterpret_cast<const float4 *>(a + P.K), u1 = *reinterpret_cast<const float4 *>(a + P.K + 4);
+                        const float u8[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+                        for (int e = 0; e < 8; e++) x8[e] = gelu_tanh_f(x8[e]) * u8[e];
+                    }
                     float sum = acc[t];
 #pragma unroll
-                    for (int e = 0; e < 8; e++) sum = fmaf(gelu_tanh_f(x8[e]) * u8[e], w8[e], sum);
+                    for (int e = 0; e < 8; e++) sum = fmaf(x8[e], w8[e], sum);
                     acc[t] = sum;
                 }
             }
         } else if (P.vec) {
             // the weight's pieces of up to 2048 columns first (they come from memory; the rows come from the caches), past its end a piece again that is not multiplied: a piece
-            // asked for behind the products of the one before, and eight rows formed for six, took 9.4 instead of 8.3 us (33 products of six rows a step)
-            for (int k0 = 0; k0 < P.K; k0 += 4 * 512) {
-                u32x4v wp[4], gp[PRO == 1 ? 4 : 1];
+            // asked for behind the products of the one before, and eight rows formed for six, took 9.4 instead of 8.3 us (33 products of six rows a step).  As many pieces
+            // as there are.
+            auto block = [&](int k0, auto pieces) {
+                constexpr int NP = decltype(pieces)::value;
+                u32x4v wp[NP];
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int k = min(k0 + 512 * j + lane * 8, P.K - 8);
-                    wp[j] = *reinterpret_cast<const u32x4v *>(w + k);
-                    if (PRO == 1) gp[j] = *reinterpret_cast<const u32x4v *>(P.norm_w + k);
-                }
+                for (int j = 0; j < NP; j++) wp[j] = *reinterpret_cast<const u32x4v *>(w + min(k0 + 512 * j + lane * 8, P.K - 8));
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
+                for (int j = 0; j < NP; j++) {
                     const int k = k0 + 512 * j + lane * 8;
                     if (k0 + 512 * j >= P.K) break;
                     float4 v[TT][2];
@@ -453,27 +466,23 @@ __global__ void __launch_bounds__(256) k_lin_rows(LinArgs P)
                         v[t][0] = *reinterpret_cast<const float4 *>(a); v[t][1] = *reinterpret_cast<const float4 *>(a + 4);
                     }
                     if (k >= P.K) continue;
-                    float w8[8], g8[8];
+                    float w8[8];
 #pragma unroll
                     for (int e = 0; e < 4; e++) { w8[2 * e] = __uint_as_float(wp[j][e] << 16); w8[2 * e + 1] = __uint_as_float(wp[j][e] & 0xFFFF0000u); }
-                    if (PRO == 1) {
-#pragma unroll
-                        for (int e = 0; e < 4; e++) { g8[2 * e] = __uint_as_float(gp[j][e] << 16); g8[2 * e + 1] = __uint_as_float(gp[j][e] & 0xFFFF0000u); }
-                    }
 #pragma unroll
                     for (int t = 0; t < TT; t++) {
-                        float x8[8] = {v[t][0].x, v[t][0].y, v[t][0].z, v[t][0].w, v[t][1].x, v[t][1].y, v[t][1].z, v[t][1].w};
-                        if (PRO == 1) {
-#pragma unroll
-                            for (int e = 0; e < 8; e++) x8[e] = (x8[e] - mean[t]) * rstd[t] * g8[e];
-                        }
+                        const float x8[8] = {v[t][0].x, v[t][0].y, v[t][0].z, v[t][0].w, v[t][1].x, v[t][1].y, v[t][1].z, v[t][1].w};
                         float sum = acc[t];
 #pragma unroll
                         for (int e = 0; e < 8; e++) sum = fmaf(x8[e], w8[e], sum);
                         acc[t] = sum;
                     }
                 }
-            }
+            };
+            int k0 = 0;
+            for (; P.K - k0 > 1024; k0 += 2048) block(k0, std::integral_constant<int, 4>());
+            if (P.K - k0 > 512) block(k0, std::integral_constant<int, 2>());
+            else if (P.K - k0 > 0) block(k0, std::integral_constant<int, 1>());
         } else {
             for (int k = lane; k < P.K; k += 64) {
                 const float wk = bf2f(w[k]);

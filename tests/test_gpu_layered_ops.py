@@ -539,6 +539,21 @@ def test_tiled_attention_over_many_sequences(window, keep):
     assert float((res[0] - res[1]).abs().max()) < 2e-6 * float(res[0].abs().max())
 
 
+@pytest.mark.parametrize("T", [2, 4, 5, 6, 8])
+@pytest.mark.parametrize("K", [504, 512, 520, 1024, 1032, 1536, 2048, 2056, 3080])
+def test_products_of_a_few_rows_at_the_edges_of_the_weights_pieces(T, K):
+    """512 columns a piece, one, two or four pieces asked for together: K fp32 multiply-adds of magnitudes ~1 and weights ~1 / sqrt(K) (bound 1e-5; measured 1e-6)"""
+    rng = np.random.default_rng(T + K)
+    N = 37
+    W, bias = orc.bf16_round(rng.standard_normal((N, K)) / K ** 0.5), orc.bf16_round(rng.standard_normal(N))
+    x = rng.standard_normal((T, K + 8)).astype(np.float32)
+    c = torch.full((T, N + 1), float("nan"), dtype=torch.float32, device="cuda")
+    ia.check(capi().ifa_linear_bf16w_rows(0, None, 0.0, p(devbf(W)), N, K, p(dev32(x)), K + 8, T, p(devbf(bias)), None, 1.0, 0, p(c), N + 1, 0, 0, stream()))
+    got = c.cpu().numpy()
+    want = (orc.t64(x[:, :K]) @ orc.t64(W).T + orc.t64(bias)).numpy()
+    assert np.abs(got[:, :N] - want).max() < 1e-5 * np.abs(want).max() and np.isnan(got[:, N:]).all()
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 8])
 def test_row_products_with_the_norm_or_the_gated_gelu_folded_in(T):
     rng = np.random.default_rng(40 + T)
