@@ -345,6 +345,7 @@ __global__ void __launch_bounds__(1024) k_argmax_f32(const float *__restrict__ l
             for (int u = 0; u < 4; u++) v[u] = *reinterpret_cast<const float4 *>(r + min(c0 + 4 * (int)(threadIdx.x + u * blockDim.x), n4 - 4));
 #pragma unroll
             for (int u = 0; u < 4; u++) {
+                if (c0 + 4 * u * (int)blockDim.x >= n4) break;
                 const int c = min(c0 + 4 * (int)(threadIdx.x + u * blockDim.x), n4 - 4);
                 take(v[u].x, c); take(v[u].y, c + 1); take(v[u].z, c + 2); take(v[u].w, c + 3);
             }

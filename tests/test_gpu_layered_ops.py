@@ -554,6 +554,25 @@ def test_products_of_a_few_rows_at_the_edges_of_the_weights_pieces(T, K):
     assert np.abs(got[:, :N] - want).max() < 1e-5 * np.abs(want).max() and np.isnan(got[:, N:]).all()
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 7, 255, 1024, 4096, 4099, 4100, 8192, 16380, 16384, 16388, 20001, 33000])
+def test_argmax_of_rows_of_any_length(n):
+    """the largest value first, last, at the edges of rounds of 4 and 16 values a thread, twice (the lower index counts), and excluded"""
+    rng = np.random.default_rng(n)
+    spots = sorted({0, n - 1, n // 2, (n & ~3) - 1, n & ~3, 4095, 4096, 16383, 16384, 4 * 256 - 1, 4 * 256} & set(range(n)))
+    lg = rng.standard_normal((2 * len(spots), (n + 3) // 4 * 4)).astype(np.float32)
+    for i, c in enumerate(spots):
+        lg[2 * i, c] = 9.0
+        lg[2 * i + 1, c] = lg[2 * i + 1, n - 1] = lg[2 * i + 1, n // 3] = 9.0
+    lg[:, n:] = 99.0
+    for ex in (-1, n - 1):
+        best = torch.empty(len(lg), dtype=torch.int32, device="cuda")
+        ia.check(capi().ifa_argmax_rows_f32(p(dev32(lg)), n, lg.shape[1], len(lg), p(devi([1, ex, -1, -1])), p(best), stream()))
+        masked = lg[:, :n].copy()
+        if ex >= 0:
+            masked[:, ex] = -np.inf
+        assert best.cpu().tolist() == [int(r.argmax()) for r in masked]
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 8])
 def test_row_products_with_the_norm_or_the_gated_gelu_folded_in(T):
     rng = np.random.default_rng(40 + T)
