@@ -179,15 +179,17 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
     int t0, n0, t_end = P.T;
     const bf16_t *Wg = P.W;
     {
+        // (grouped: of the tiles that there are, not of the most there can be -- the empty ones, dealt out like the others, left up to five of the XCDs idle: 36 pairs of 64
+        // experts of 1024 x 704 66 -> 46 us, 2400 pairs 127 -> 101)
+        if constexpr (GROUPED) tiles_m = *P.n_tiles;
         const int nwg = tiles_m * tiles_n, orig = blockIdx.x, xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
+        if (GROUPED && orig >= nwg) return;
         const int wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
         constexpr int GM = 1024 / BM;          // bands of 1024 rows of C, the row tiles of a band fastest
         const int band = wg / (GM * tiles_n), within = wg % (GM * tiles_n), band_m = min(GM, tiles_m - band * GM);
         t0 = (band * GM + within % band_m) * BM; n0 = (within / band_m) * BN;
         if constexpr (GROUPED) {
-            const int tile = t0 / BM;
-            if (tile >= *P.n_tiles) return;
-            const int *tm = P.tile_map + 3 * tile;
+            const int *tm = P.tile_map + 3 * (t0 / BM);
             Wg += (size_t)tm[0] * P.N * P.K; t0 = tm[1]; t_end = tm[1] + tm[2];
         }
     }

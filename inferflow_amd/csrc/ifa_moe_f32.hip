@@ -492,11 +492,13 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
         return IFA_OK;
     }
     // gated experts, products over bfloat16 rows where the activations are rounded anyway: h once (in the place of the down products' output, which is not there yet), the experts'
-    // activations by the launch that forms them; row tiles of 128 where an expert has several on average
+    // activations by the launch that forms them.  From 512 columns on, of both products together: below, the launch that rounds h costs more than the products gain (8 experts,
+    // us before / now: 128 x 128 18.7 / 21.6, 256 x 128 20.6 / 21.6, 256 x 256 22.6 / 21.6).  Row tiles of 128 where an expert has several on average and they still fill the
+    // chip (4000 pairs of 8 experts: 1408 x 2048 288 -> 197 us; 520 x 136 52, 46 with tiles of 64, 59 with tiles of 128)
     const size_t lda_h = ((size_t)width + 63) & ~(size_t)63, lda_f = ((size_t)ff + 63) & ~(size_t)63;
-    const bool in16 = gated && !ops32 && width % 8 == 0 && width >= 64 && ff % 8 == 0 && ff >= 64 && lda_f <= 2 * (size_t)ff && lda_h <= 2 * (size_t)width * top
+    const bool in16 = gated && !ops32 && width % 8 == 0 && width >= 64 && ff % 8 == 0 && ff >= 64 && width + ff >= 512 && lda_f <= 2 * (size_t)ff && lda_h <= 2 * (size_t)width * top
                       && (((uintptr_t)up_bf16 | (uintptr_t)down_bf16) & 15) == 0;
-    const int tile_rows = in16 && pairs >= (size_t)256 * experts ? 128 : 64;
+    const int tile_rows = in16 && pairs >= (size_t)256 * experts && pairs / 128 * (((size_t)width + 127) / 128) >= 256 ? 128 : 64;
     const size_t max_tiles = (pairs + tile_rows - 1) / tile_rows + (size_t)experts;
     IFA_REQUIRE(max_tiles < 65536, "%s: %zu rows x %d choices exceed one step", who, rows, top);
     hipLaunchKernelGGL(k_moe_sort, dim3(1), dim3(1024), (size_t)(2 * experts + 1) * 4, s, idx_dev, (const float *)wgt_f32, (int)pairs, experts, top, a_rows, pair_pos, w_sorted,

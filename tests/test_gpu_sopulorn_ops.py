@@ -264,9 +264,11 @@ def test_gated_experts_in_rows_and_grouped(T, W, F, E, top):
             assert np.abs(y.cpu().numpy()[:, :W] - ref).max() < t_ * max(1.0, np.abs(want).max()), (ops32, acc)
 
 
-@pytest.mark.parametrize("T,W,F,E,top", [(9, 64, 72, 6, 2), (40, 264, 320, 5, 2), (300, 136, 264, 2, 2), (700, 72, 64, 3, 1), (130, 328, 72, 1, 1)])
+@pytest.mark.parametrize("T,W,F,E,top", [(9, 64, 72, 6, 2), (40, 264, 320, 5, 2), (300, 136, 264, 2, 2), (700, 72, 64, 3, 1), (130, 328, 72, 1, 1),
+                                         (9, 64, 456, 6, 2), (300, 136, 384, 2, 2), (20, 264, 320, 40, 2), (11, 520, 72, 3, 1), (9000, 520, 72, 2, 1), (130, 440, 72, 1, 1)])
 def test_gated_experts_over_bfloat16_rows(T, W, F, E, top):
-    """row tiles of 64 and 128, few and many steps, inner sizes that are no multiple of a step: h and the activations rounded to bfloat16 once"""
+    """sizes above and below the form's border, row tiles of 64 and 128 (9000 rows), few and many steps, inner sizes that are no multiple of a step, many experts without a row
+    (fewer tiles than there may be): h and the activations rounded to bfloat16 once"""
     rng = np.random.default_rng(T + W + F)
     h = bf16_round(rng.standard_normal((T, W)))
     gu = bf16_round(rng.standard_normal((E, 2 * F, W)) / np.sqrt(W)); dn = bf16_round(rng.standard_normal((E, W, F)) / np.sqrt(F))
