@@ -444,7 +444,8 @@ __global__ void __launch_bounds__(256) k_attn_window_tile(WinAttnArgs P, int n_s
 // Arithmetic: every 32-bit operand is the sum of three bfloat16 values (24 bits: nothing is lost but the last rounding), and a product takes
 // the six of the nine partial products that reach 2^-24 of the largest: 6 x 32 matrix-core cycles per 16 columns where the fp32 instructions
 // take 512.  Error against 64 bits: no larger than the fp32 instructions' (test_tiled_attention_with_a_workspace_against_64_bits_and_the_fp32_tiles).
-// An infinite value in a V row gives NaN (0 x inf of a lower part) where fp32 gives inf.
+// In blocks with an infinity or NaN among the keys or values (k_attn_parts marks them) the queries' and weights' parts are formed so that no lower part of 0 meets an infinity.  (An
+// infinity in a query is not looked for: its scores are infinities of both signs, their weights NaN.)
 // The fp32 tiles above took 487 us for 2048 causal tokens of 8 heads of 128 (16 tiles x 8 heads on half of the compute units, the last tile alone walking 64 blocks)
 // and 420 us for 16 heads with a window of 1024, soft cap and bias; this form 83 and 146 us, of it 6 us for the operands and 14 us for joining the
 // shares.  Bound by matrix cores and vector instructions in turn (3072 and ~2500 cycles per wave and block; the waves of a SIMD do not drift apart enough to
@@ -466,13 +467,47 @@ __device__ __forceinline__ Parts parts_of(const float *v)
     for (int e = 0; e < 8; e++) big = fmaxf(big, __builtin_fabsf(v[e]));
 #pragma unroll
     for (int e = 0; e < 8; e++) { r.p[0][e] = (__bf16)v[e]; d[e] = v[e] - (float)r.p[0][e]; }
-    if (__builtin_amdgcn_ballot_w64(big > 3.38e38f)) {          // (infinities stay in the first part)
+    if (__builtin_amdgcn_ballot_w64(big > 3.38e38f)) {          // (the first part of what would round to infinity is cut off instead; infinities stay in it)
 #pragma unroll
-        for (int e = 0; e < 8; e++) d[e] = __builtin_fabsf(v[e]) > 3.38e38f ? 0.0f : d[e];
+        for (int e = 0; e < 8; e++)
+            if (__builtin_fabsf(v[e]) > 3.38e38f) {
+                const float cut = __uint_as_float(__float_as_uint(v[e]) & 0xFFFF0000u);
+                r.p[0][e] = (__bf16)cut; d[e] = __builtin_fabsf(v[e]) == INFINITY ? 0.0f : v[e] - cut;
+            }
     }
 #pragma unroll
     for (int e = 0; e < 8; e++) { r.p[1][e] = (__bf16)d[e]; r.p[2][e] = (__bf16)(d[e] - (float)r.p[1][e]); }
     return r;
+}
+
+// For products with an infinity: the same values (zero apart) in three parts of one sign, none of them zero, so that each partial product is an infinity of the sum's sign.
+// Cut off instead of rounded; where nothing is left the smallest normal number, which adds nothing to a finite product.
+__device__ __forceinline__ Parts one_sign(const Parts &t)
+{
+    Parts r;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const float x = (float)t.p[0][e] + ((float)t.p[1][e] + (float)t.p[2][e]), least = x == 0.0f ? 0.0f : __builtin_copysignf(1.17549435e-38f, x);
+        const float a = __uint_as_float(__float_as_uint(x) & 0xFFFF0000u), d = x - a, b = __uint_as_float(__float_as_uint(d) & 0xFFFF0000u), c = d - b;
+        r.p[0][e] = (__bf16)a; r.p[1][e] = (__bf16)(b == 0.0f ? least : b); r.p[2][e] = (__bf16)(c == 0.0f ? least : c);
+    }
+    return r;
+}
+// (back again)
+__device__ __forceinline__ Parts rounded(const Parts &t)
+{
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = (float)t.p[0][e] + ((float)t.p[1][e] + (float)t.p[2][e]);
+    return parts_of(v);
+}
+
+__device__ __forceinline__ bool not_finite(const float *v)
+{
+    float z = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) z = fmaf(v[e], 0.0f, z);
+    return z != 0.0f;          // (0, or NaN from any of them)
 }
 
 // the five partial products below the leading one, smallest first
@@ -532,7 +567,8 @@ __host__ __device__ __forceinline__ TileBlocks tile_blocks(int p0, int nq, int w
     return t;
 }
 
-struct TileArgs { int n_seqs, hpw, cb, tiles; size_t shares; };      // shares: where the chunks' partial results begin in the workspace (floats), behind the operands
+// marks, shares: where the blocks' marks and the chunks' partial results begin in the workspace (floats), behind the operands
+struct TileArgs { int n_seqs, hpw, cb, tiles; size_t marks, shares; };
 
 // The item (of n) that a number running over all items' counts falls into, or -1; id becomes the number inside it.  A wave looks at 64 items at a time (walked by one thread,
 // a step of 1024 sequences behind 100 keys each took 10.6 ms, now 0.37; 512 behind 200 2.0 ms, now 0.26).  count: called by all lanes, -1 for none.
@@ -612,7 +648,7 @@ template <int NTK, int NTV> constexpr int kBlockPieces = 3 * 64 * (2 * NTK + 2 *
 // grid (kv heads, blocks of the step): the cache rows of a block into its operands -- once per layer and step, not once per tile that reads the block.
 // Bound by its launch and one trip to memory (reads 4, writes 6 bytes per value).  Rows past the sequence's last: that row again (their scores are masked).
 template <int NTK, int NTV>
-__global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, int n_seqs)
+__global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, int n_seqs, uint32_t *__restrict__ marks)
 {
     constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK;
     const int tid = threadIdx.x, kvh = blockIdx.x, dk = P.dim, dv = P.vdim;
@@ -626,6 +662,7 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, int n_seqs)
     gfloat *kc = (gfloat *)(P.slot_base[sd.slot] + P.k_off + (size_t)kvh * dk), *vc = (gfloat *)(P.slot_base[sd.slot] + P.v_off + (size_t)kvh * dv);
     bf16x8w *dst = (bf16x8w *)P.ws + ((size_t)blockIdx.y * P.kv_heads + kvh) * kBlockPieces<NTK, NTV>;
     const bool vec = dk % 4 == 0 && P.k_off % 4 == 0;      // (arena bases are 256-byte aligned)
+    bool odd = false;          // an infinity or NaN among the thread's values
     for (int e = tid; e < WT_K * (DK / 8); e += 256) {
         const int key = e / (DK / 8), c8 = e % (DK / 8), c = 8 * c8;
         gfloat *row = kc + (size_t)min(kb0 + key, last) * kvd;
@@ -638,6 +675,7 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, int n_seqs)
 #pragma unroll
             for (int x = 0; x < 8; x++) { const float f = row[min(c + x, dk - 1)]; v[x] = c + x < dk ? f : 0.0f; }
         }
+        odd |= not_finite(v);
         const Parts t = parts_of(v);
 #pragma unroll
         for (int pl = 0; pl < 3; pl++) dst[(pl * KS + (c8 >> 1)) * 64 + 32 * (c8 & 1) + key] = t.p[pl];
@@ -648,10 +686,13 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, int n_seqs)
         float v[8];
 #pragma unroll
         for (int x = 0; x < 8; x++) { const float f = vc[(size_t)min(kb0 + k0 + 8 * (x >> 2) + (x & 3), last) * vvd + min(d, dv - 1)]; v[x] = d < dv ? f : 0.0f; }
+        odd |= not_finite(v);
         const Parts t = parts_of(v);
 #pragma unroll
         for (int pl = 0; pl < 3; pl++) dst[((pl * NTV + (d >> 5)) * 2 + (sg >> 1)) * 64 + 32 * (sg & 1) + (d & 31)] = t.p[pl];
     }
+    const int any = __syncthreads_or(odd);
+    if (tid == 0) marks[(size_t)blockIdx.y * P.kv_heads + kvh] = any ? 1u : 0u;
 }
 
 // Key rows of dim <= 32 NTK and value rows of vdim <= 32 NTV floats.  VEC: rows of whole, aligned 16-byte pieces in q and the output.
@@ -687,6 +728,13 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
                 __builtin_amdgcn_global_load_lds((wa_glb_t *)(src + (u + wave) * 64 + lane), (wa_lds_t *)(dst + (u + wave) * 64), 16, 0, 0);
     };
     fetch(b0);
+    // which of the chunk's blocks (64 at a time) have a mark
+    auto marked = [&](int b) -> uint64_t {
+        const int x = min(b + lane, b1 - 1), block = x < tb.kept ? x : tb.first + x - tb.kept, at = block < sb.kept ? block : sb.kept + block - sb.first;
+        const uint32_t m = ((const __attribute__((address_space(1))) uint32_t *)(P.ws + A.marks))[(size_t)(block0 + at) * P.kv_heads + kvh];
+        return __builtin_amdgcn_ballot_w64(m != 0 && b + lane < b1);
+    };
+    uint64_t odd = marked(b0);
     // the lane's query, normed, in three parts (queries past the tile's last: that one again, not stored)
     Parts q[KS];
     {
@@ -728,6 +776,8 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
 #pragma unroll
         for (int r = 0; r < 16; r++) o[nt][r] = 0.0f;
     for (int b = b0; b < b1; b++) {
+        if (((b - b0) & 63) == 0 && b > b0) odd = marked(b);
+        const bool infinite = odd >> ((b - b0) & 63) & 1;
         const int kb0 = (b < tb.kept ? b : tb.first + b - tb.kept) * WT_K;
         const bool active = nq_w > 0 && kb0 <= qhi && (kb0 + WT_K - 1 >= qlo - P.window + 1 || kb0 < P.keep_first);
         // this wave's share of the block has landed, and behind the barrier every wave's, and no wave reads the other buffer any more
@@ -739,6 +789,10 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
         f32x16w acc;
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+        if (infinite) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) q[ks] = one_sign(q[ks]);
+        }
         {
             Parts k[2];
             auto read_k = [&](int ks) {
@@ -753,6 +807,10 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k[ks & 1].p[0], q[ks].p[0], acc, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
+        }
+        if (infinite) {
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) q[ks] = rounded(q[ks]);
         }
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[r] *= P.scale;
@@ -790,7 +848,8 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
         for (int r = 0; r < 16; r++) { const float p = exp_neg(acc[r] - m_use); w[r >> 3][r & 7] = p; psum += p; }
         l = l * corr + psum;             // (the keys of this half of the wave; the halves are added at the end)
         m = m_new;
-        const Parts w0 = parts_of(w[0]), w1 = parts_of(w[1]);
+        Parts w0 = parts_of(w[0]), w1 = parts_of(w[1]);
+        if (infinite) { w0 = one_sign(w0); w1 = one_sign(w1); }
         __builtin_amdgcn_sched_barrier(0);
         Parts v[2];
         auto read_v = [&](int u) {
@@ -896,8 +955,8 @@ __global__ void __launch_bounds__(256) k_attn_tile_combine(WinAttnArgs P, TileAr
 
 // How a step's tiles are shared out: hpw query heads and qw queries per workgroup, cb key blocks per chunk, up to `chunks` chunks per tile, so that the
 // chunks just fill the compute units once (one workgroup each: registers and LDS); below two blocks a chunk the partial results cost more than
-// the wait they save.  op_bytes: workspace of the blocks' operands, bytes: with the chunks' shares (none with one chunk).
-struct TilePlan { int hpw, qw, cb, chunks; size_t tiles, groups, blocks, op_bytes, bytes; };
+// the wait they save.  op_bytes: workspace of the blocks' operands and marks (from mark_at on), bytes: with the chunks' shares (none with one chunk).
+struct TilePlan { int hpw, qw, cb, chunks; size_t tiles, groups, blocks, mark_at, op_bytes, bytes; };
 TilePlan tile_plan(const ifa_seq_desc *sh, int n_seqs, int heads, int kv_heads, int dim, int vdim, int window, int keep_first, size_t ws_bytes)
 {
     TilePlan t;
@@ -915,7 +974,8 @@ TilePlan tile_plan(const ifa_seq_desc *sh, int n_seqs, int heads, int kv_heads, 
         }
     }
     t.tiles = nbs.size();
-    t.op_bytes = t.blocks * (size_t)kv_heads * 3 * 64 * 16 * (size_t)(2 * NTK + 2 * NTV);
+    t.mark_at = t.blocks * (size_t)kv_heads * 3 * 64 * 16 * (size_t)(2 * NTK + 2 * NTV);
+    t.op_bytes = t.mark_at + (t.blocks * (size_t)kv_heads * 4 + 15) / 16 * 16;
     const size_t hx = (size_t)(heads / t.hpw), share = (size_t)WT_WAVES * 32 * ((size_t)vdim + 2) * 4;
     size_t cb = std::max<size_t>({2, total * hx / WT_SLOTS, (most + WT_MAX_CHUNKS - 1) / WT_MAX_CHUNKS});
     auto chunks = [&]() { return (most + cb - 1) / cb; };
@@ -1102,14 +1162,14 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
         if (t.bytes <= ws_bytes && t.tiles < 65536 && t.groups < 65536 && t.blocks < 65536) {          // (a grid's limits; beyond them the tiles below, as without a workspace)
             const int NTK = (dim + 31) / 32, NTV = (vdim + 31) / 32;
             TileArgs A;
-            A.n_seqs = n_seqs; A.hpw = t.hpw; A.cb = t.cb; A.tiles = (int)t.tiles; A.shares = t.op_bytes / 4;
+            A.n_seqs = n_seqs; A.hpw = t.hpw; A.cb = t.cb; A.tiles = (int)t.tiles; A.marks = t.mark_at / 4; A.shares = t.op_bytes / 4;
             P.ws = (float *)ws_f32; P.nsplit = t.chunks;
             const bool vec = dim % 4 == 0 && vdim % 4 == 0 && ldq % 4 == 0 && ldo % 4 == 0 && (uintptr_t)q_f32 % 16 == 0 && (uintptr_t)out_f32 % 16 == 0;
             const dim3 grid((unsigned)(heads / t.hpw), (unsigned)t.groups);
 #define IFA_WT(K, V) { const size_t smem_t = (size_t)2 * kBlockPieces<K, V> * 16 + WT_WAVES * 64 * 4; \
                        const void *fn = vec ? (const void *)k_attn_tile<K, V, true> : (const void *)k_attn_tile<K, V, false>; \
                        IFA_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_t)); \
-                       hipLaunchKernelGGL((k_attn_parts<K, V>), dim3((unsigned)kv_heads, (unsigned)t.blocks), dim3(256), 0, ifa_s(stream), P, n_seqs); \
+                       hipLaunchKernelGGL((k_attn_parts<K, V>), dim3((unsigned)kv_heads, (unsigned)t.blocks), dim3(256), 0, ifa_s(stream), P, n_seqs, (uint32_t *)(P.ws + A.marks)); \
                        if (vec) hipLaunchKernelGGL((k_attn_tile<K, V, true>), grid, dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A); \
                        else hipLaunchKernelGGL((k_attn_tile<K, V, false>), grid, dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A); }
 #define IFA_WTV(K) { if (NTV == 1) IFA_WT(K, 1) else if (NTV == 2) IFA_WT(K, 2) else if (NTV == 3) IFA_WT(K, 3) else IFA_WT(K, 4) }

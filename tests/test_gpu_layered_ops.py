@@ -482,7 +482,7 @@ def test_tiled_attention_takes_fewer_chunks_where_the_workspace_is_small():
     d, rs, _ = seq_tables([(T, 0, 0)])
     q = dev32(rng.standard_normal((T, heads * dim)))
     nb = capi().ifa_attention_tile_workspace_bytes(host, 1, heads, kv_heads, dim, dim, 0, 0)
-    ops = (T + 31) // 32 * 3 * 64 * 16 * 4
+    ops = (T + 31) // 32 * 3 * 64 * 16 * 4 + ((T + 31) // 32 * 4 + 15) // 16 * 16          # (a mark per block behind them)
     res = []
     for ws_bytes in (nb, nb - 4, ops + 64, ops - 4):          # (the last: the operands do not fit, the fp32 tiles)
         ws, out = torch.empty(nb, dtype=torch.uint8, device="cuda"), torch.empty((T, heads * dim), dtype=torch.float32, device="cuda")
@@ -512,6 +512,37 @@ def test_tiled_attention_of_more_key_blocks_than_a_grid_has():
                                              p(ws) if ws_bytes else None, ws_bytes, None))
         sync(); res.append(out)
     assert torch.equal(res[0], res[1]) and bool(torch.isfinite(res[0]).all())
+
+
+@pytest.mark.parametrize("where,value", [("k", np.inf), ("k", -np.inf), ("v", np.inf), ("v", -np.inf), ("v", np.nan), ("k", np.nan), ("v", 3.395e38), ("v", -3.402e38), ("k", 3.4e38)])
+def test_tiled_attention_with_infinite_and_very_large_keys_and_values(where, value):
+    """one element of a key or value that every query sees, in a block of its own and beside others: infinities, NaN and finite outputs where the fp32 tiles have them (an
+    infinite key's score is -inf for half of the queries: weight 0), finite ones within 2e-6.  Very large values round to no bfloat16."""
+    rng = np.random.default_rng(8)
+    heads, kv_heads, dim, pos0, n = 4, 2, 64, 70, 100
+    ctx = pos0 + n
+    host = (C.c_int * 4)(0, n, pos0, 0)
+    d, rs, _ = seq_tables([(n, pos0, 0)])
+    q = dev32(rng.standard_normal((n, heads * dim)))
+    nb = capi().ifa_attention_tile_workspace_bytes(host, 1, heads, kv_heads, dim, dim, 0, 0)
+    for rows in ((5,), (5, 40), (69,)):
+        kv = {"k": rng.standard_normal((ctx, kv_heads, dim)).astype(np.float32), "v": rng.standard_normal((ctx, kv_heads, dim)).astype(np.float32)}
+        for i, r in enumerate(rows):
+            kv[where][r, 1, 17 + i] = value
+        sl = Slots(1, 2 * ctx * kv_heads * dim)
+        sl.mem[0].copy_(dev32(np.concatenate([kv["k"].reshape(-1), kv["v"].reshape(-1)])))
+        out = []
+        for ws_bytes in (nb, 0):
+            ws, o = torch.full((nb // 4,), float("nan"), dtype=torch.float32, device="cuda"), torch.zeros((n, heads * dim), dtype=torch.float32, device="cuda")
+            ia.check(capi().ifa_attention_kv_f32(p(q), heads * dim, heads, kv_heads, dim, dim, dim ** -0.5, 0, 0, 0, 0.0, p(d), p(rs), n, p(sl.table), 0, ctx * kv_heads * dim, p(o),
+                                                 heads * dim, host, 1, 16, 0, p(ws) if ws_bytes else None, ws_bytes, None))
+            sync(); out.append(o.cpu().numpy())
+        got, want = out
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(got[np.isinf(got)], want[np.isinf(want)]), rows
+        fin = np.isfinite(want)
+        big = np.abs(want) > 1e30
+        for part in (fin & big, fin & ~big):
+            assert not part.any() or np.abs(got[part] / 2 - want[part] / 2).max() < 1e-6 * np.abs(want[part]).max(), rows
 
 
 @pytest.mark.parametrize("window,keep", [(1 << 30, 0), (90, 40)])
