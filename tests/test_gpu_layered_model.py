@@ -359,6 +359,31 @@ def test_single_token_steps_in_few_launches(tmp_path, ctx):
     assert fx.rel_err(rows[0][1:], rows[1][1:]).max() < TOL32
 
 
+@pytest.mark.parametrize("ctx", [400, 4200])      # (4200: the first layer may have more than 4096 keys in view, for which its steps keep a launch per mixer)
+def test_generation_replays_the_single_token_launches(tmp_path, ctx):
+    """The captured step (cache rows, states, shares of the keys from the capture on) over the edges of a window and of several shares of 64 keys, with the fused launches and
+    with one launch per operation: the oracle's tokens, a prompt in between"""
+    import inferflow_amd as ia
+    cfg = fx.config([fx.parallel_layer(heads=4, kv_heads=2, dim=64, window=5000, keep_first=0, lin_heads=3, lin_dim=64, lin_vdim=96, ff=72),
+                     fx.delta_layer(heads=4, kv_heads=2, dim=64, vdim=32, conv=3, ff=96),
+                     fx.parallel_layer(heads=3, kv_heads=1, dim=100, window=150, keep_first=5, lin_heads=2, lin_dim=128, lin_vdim=40, ff=0)], width=136, vocab=97)
+    w = fx.random_weights(cfg, 51)
+    prompt = tokens_for(cfg, 120, 52)
+    for fused in (1, 0):
+        eng = engine_for(tmp_path, cfg, w, ctx=ctx, queries=2)
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"fuse_step", fused))
+        for _ in range(2):
+            q = eng.add_query(prompt)
+            gen, _ = eng.generate(q, 40)
+            eng.remove_query(q)
+            want = oracle_logits(cfg, w, prompt + gen)
+            for i, tok in enumerate(gen):
+                row = want[len(prompt) - 1 + i]
+                assert row[tok] > row.max() - 1e-3 * np.abs(row).max(), (fused, i)
+            run_whole(eng, tokens_for(cfg, 200, 53))
+        eng.close()
+
+
 @pytest.mark.parametrize("K", [8, 120, 512, 520, 1024, 1032, 2048, 2056, 4096])
 @pytest.mark.parametrize("N", [1, 5, 4099])
 def test_one_row_product_with_the_norm_inside(K, N):

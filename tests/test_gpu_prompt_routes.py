@@ -96,7 +96,8 @@ def test_short_prompt_routes_match_the_oracle(T):
 
 @pytest.mark.parametrize("shape", ["llama2_7b", "test_gqa"])
 def test_short_prompts_leave_the_cache_rows_of_long_ones(shape):
-    """up to 768 tokens four workgroups share a token's rotation (head counts that four divide), above one holds it: the cache rows of the first layer have the same bits"""
+    """up to 768 tokens four workgroups share a token's rotation (head counts that four divide), above one holds it, and the products in front take other kernels: the cache
+    rows of the first layer agree to a rounding (the rotation's bits: the test below)"""
     wk, _, s = synth.build(shape, dt.Q4_B32T1A, dt.F16, max_ctx=832, layers=1, vocab=1000)
     toks = np.random.default_rng(3).integers(3, s["vocab"], 800).astype(np.int32)
     rows = {}
@@ -106,6 +107,33 @@ def test_short_prompts_leave_the_cache_rows_of_long_ones(shape):
         rows[T] = [np.array(wk.read_buffer(n, 0, nbytes=40 * s["kv_heads"] * s["head_dim"] * 2)) for n in ("kcache", "vcache")]
     for a, b in zip(rows[40], rows[800]):
         a, b = a.view(np.float16).astype(np.float32), b.view(np.float16).astype(np.float32)
-        # (the products in front take other kernels by length: their sums' order, one rounding)
         assert np.abs(a - b).max() <= 2.0 ** -9 * np.abs(b).max(), np.abs(a - b).max()
     wk.close()
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,order,part", [(32, 8, 128, 1, 1.0), (8, 4, 64, 2, 1.0), (12, 4, 48, 2, 0.5), (8, 8, 80, 1, 0.5), (6, 6, 48, 1, 1.0), (32, 2, 64, 1, 1.0)])
+def test_rotation_by_four_workgroups_a_token_and_by_one_leave_the_same_bits(heads, kv_heads, head_dim, order, part):
+    """768 tokens and one more over the same rows: q, k and both caches, head counts that four divides and others"""
+    import ctypes as C
+    import torch
+    import inferflow_amd as ia
+    from tests.gpu_util import capi, p
+    gen = torch.Generator(device="cuda"); gen.manual_seed(heads + head_dim)
+    T, kvd, row = 769, kv_heads * head_dim, kv_heads * head_dim + 8
+    rows = [torch.randn(T, n * head_dim, generator=gen, device="cuda").half() for n in (heads, kv_heads, kv_heads)]
+    f = capi().ifa_rope_qk_store
+    f.argtypes = [C.c_void_p] * 3 + [C.c_int] * 5 + [C.c_float, C.c_int, C.c_float, C.c_void_p, C.c_void_p, C.c_size_t, C.c_void_p]
+    out = []
+    for n in (T, T - 1):
+        q, k, v = (t.clone() for t in rows)
+        caches = [torch.zeros(T, row, dtype=torch.float16, device="cuda") for _ in range(2)]
+        ia.check(f(p(q), p(k), p(v), head_dim, heads, kv_heads, n, 5, 10000.0, order, part, p(caches[0]), p(caches[1]), row, None))
+        torch.cuda.synchronize()
+        out.append([q, k] + caches)
+    for a, b, src in zip(out[0], out[1], (rows[0], rows[1], None, None)):
+        assert torch.equal(a[:T - 1].view(torch.int16), b[:T - 1].view(torch.int16))
+        if src is not None:
+            assert torch.equal(b[T - 1], src[T - 1]) and not torch.equal(b[:T - 1], src[:T - 1])
+        else:
+            assert not b[T - 1].any() and not b[:, kvd:].any()
+    assert torch.equal(out[0][2][:, :kvd], out[0][1]) and torch.equal(out[0][3][:, :kvd], rows[2])
