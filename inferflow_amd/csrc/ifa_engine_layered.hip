@@ -1092,7 +1092,7 @@ int run_head(ifa_model *m, size_t r0, size_t nr)
     LayeredNet *n = m->lay;
     const size_t W = (size_t)n->cfg.width, V = (size_t)n->cfg.vocab;
     int rc;
-    if (((n->opt_fuse_rows & 1) || (n->opt_fuse_step && nr == 1)) && nr <= 8 && W % 8 == 0 && n->cfg.stem == 0) {
+    if (((n->opt_fuse_rows & 1) || (n->opt_fuse_step && nr == 1)) && nr <= 8 && W % 8 == 0 && n->cfg.stem == 0 && n->cfg.logit_softcap <= 0.0f) {
         if ((rc = ifa_linear_bf16w_rows(1, n->out_norm.data, n->cfg.eps, n->lm_head.data, V, W, n->x + r0 * W, W, nr, nullptr, nullptr, 1.0f, 0, n->logits, V, 0, 0,
                                         (ifa_stream)m->stream))) return rc;
         n->logits_rows = nr;

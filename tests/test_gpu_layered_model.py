@@ -384,6 +384,52 @@ def test_generation_replays_the_single_token_launches(tmp_path, ctx):
         eng.close()
 
 
+def test_capped_logits_of_a_single_row(tmp_path):
+    """A model made through the C API with position vectors (stem 0) and a soft cap on its logits: a step of one token, whose head has the norm inside, and the first row of a
+    step of three leave the same capped logits"""
+    import ctypes as C
+    import re
+    import inferflow_amd as ia
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "inferflow_amd.h")).read(), flags=re.S)
+
+    def struct(name):
+        body = re.findall(r"typedef struct \{([^}]*)\} %s;" % name, text)[0]
+        fields = [(f.strip(), {"int": C.c_int, "float": C.c_float}[t]) for t, names in re.findall(r"(int|float) ([^;]+);", body) for f in names.split(",")]
+        return type(name, (C.Structure,), {"_fields_": fields})()
+    names = [n.split("=")[0].strip() for n in re.findall(r"enum \{\s*(IFA_LT_NORM1 = 40[^}]*)\}", text)[0].split(",")]
+    ids = {n[len("IFA_LT_"):]: 40 + i for i, n in enumerate(names)}
+    cfg, L = fx.config([fx.delta_layer(heads=2, kv_heads=1, dim=16, vdim=16, conv=2, ff=0)], width=32, vocab=37), ia.lib()
+    w = fx.random_weights(cfg, 61)
+    c, sp = struct("ifa_layered_config"), struct("ifa_layer_spec")
+    c.width, c.vocab, c.max_ctx, c.n_layers, c.ops32, c.eps, c.pos_base, c.logit_softcap = 32, 37, 64, 1, 1, 1e-5, 10000.0, 0.25
+    sp.mixer, sp.d_heads, sp.d_kv_heads, sp.d_dim, sp.d_vdim, sp.d_conv = 2, 2, 1, 16, 16, 2
+    m = C.c_void_p()
+    ia.check(L.ifa_model_create_layered(C.byref(c), C.byref(sp), C.byref(m)))
+    tensors = {(-1, 0): "embed", (-1, 1): "final.norm", (-1, 3): "head"}
+    for tid, leaf in (("NORM1", "norm1"), ("LS1", "ls1"), ("D_Q", "mix.q"), ("D_K", "mix.k"), ("D_V", "mix.v"), ("D_QCONV", "mix.q.conv"), ("D_KCONV", "mix.k.conv"),
+                      ("D_VCONV", "mix.v.conv"), ("D_B", "mix.b"), ("D_A", "mix.a"), ("D_ALOG", "mix.A_log"), ("D_DTBIAS", "mix.dt_bias"), ("D_G", "mix.g"), ("D_NORM", "mix.norm"),
+                      ("D_O", "mix.o")):
+        tensors[(0, ids[tid])] = "l0." + leaf
+    bf16 = int(re.search(r"IFA_BF16 = (\d+)", text).group(1))
+    for (layer, tid), name in tensors.items():
+        a = np.atleast_2d(orc.bf16_bits(w[name]))
+        ia.check(L.ifa_model_set_tensor_host(m, layer, tid, bf16, a.ctypes.data_as(C.c_void_p), *a.shape))
+    ia.check(L.ifa_model_finalize(m))
+
+    def step(tokens):
+        ints = lambda *v: (C.c_int * len(v))(*v)
+        ia.check(L.ifa_model_step_seqs(m, 1, ints(*tokens), ints(len(tokens)), ints(0), ints(0), 1, ints(0)))
+        d, r, k = C.c_void_p(), C.c_size_t(), C.c_size_t()
+        ia.check(L.ifa_model_logits_f32(m, C.byref(d), C.byref(r), C.byref(k)))
+        out = np.empty((r.value, k.value), np.float32)
+        ia.check(L.ifa_memcpy_d2h(out.ctypes.data_as(C.c_void_p), d, out.nbytes, None)); ia.check(L.ifa_stream_sync(None))
+        return out
+    one, three = step([5]), step([5, 9, 2])
+    want = 0.25 * np.tanh(oracle_logits(cfg, w, [5, 9, 2]) / 0.25)
+    assert one.shape == (1, 37) and fx.rel_err(one, want[:1]).max() < TOL32 and fx.rel_err(three, want).max() < TOL32
+    L.ifa_model_destroy(m)
+
+
 @pytest.mark.parametrize("K", [8, 120, 512, 520, 1024, 1032, 2048, 2056, 4096])
 @pytest.mark.parametrize("N", [1, 5, 4099])
 def test_one_row_product_with_the_norm_inside(K, N):
