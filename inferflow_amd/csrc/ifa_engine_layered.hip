@@ -115,7 +115,8 @@ struct LayeredNet {
                                            // PRENORM layers: the start of a looped pass inside the norm's launch; steps of at most 8 rows: the norm inside the router's launch
     float *attn_ws = nullptr; size_t attn_ws_bytes = 0;      // partial results of the windowed attention when a (row, head)'s keys are shared out
     // Workspaces of prompts through the tiled attention and the chunked recurrences: reserved for one prompt as long as the context when the model is finalized (up to
-    // RESERVE_BYTES each), grown by steps that need more up to opt_workspace_mb each.  A step beyond that, or whose workspace cannot be had, runs without (fp32 tiles, token by token).
+    // RESERVE_BYTES each), grown by steps that need more -- several prompts, or a shorter one whose keys are shared out further: 960 tokens behind a window of 1024, 16 heads of
+    // 128, 67 MB where 4096 tokens take 24 -- up to opt_workspace_mb each.  A step beyond that, or whose workspace cannot be had, runs without (fp32 tiles, token by token).
     float *tile_ws = nullptr; size_t tile_ws_bytes = 0;
     int opt_workspace_mb = 4096; bool step_tile_ws = false;
     bf16_t *a16 = nullptr, *h16 = nullptr; size_t a16_cap = 0, h16_cap = 0; int opt_a16_min = 17;          // activations of a prompt's product rounded to bfloat16; steps of at least this many rows (0: never)
