@@ -15,7 +15,7 @@
 //   * every LDS read of the loop is inline assembly (the compiler sees no LDS access to protect), waited for with lgkmcnt where
 //     the values are used;
 //   * a wave owns 32 weight rows of the tile and ALL 128 tokens (4 accumulator tiles): it dequantises its rows' codes from the raw
-//     bytes straight into the B operand registers (15 VALU per 8 weights, ifa_dequant_q4.h) -- no dequantised tile in LDS, no
+//     bytes straight into the B operand registers (11 VALU per 8 weights, ifa_dequant_q4.h) -- no dequantised tile in LDS, no
 //     second barrier -- while the MFMAs of the previous 16-column group run;
 //   * one barrier per step (the activation tile is shared by the four waves); parts of K as in k_gemm_big.
 // Weights: the MO copy of the rows GEMM (ifa_gemm_rows_mfma.h; Q4_B32T1A / B and the 64-weight nibble formats): a 16-row tile's K range
@@ -157,7 +157,6 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
     // (the stage holds this wave's codes as [tile][block of the half][row] x 16 bytes, the words likewise x 4 bytes)
     const uint32_t wc_off = lds0 + (uint32_t)(MD_A_BYTES + wave * 1024 + ((i >> 4) * 32 + (i & 15)) * 16);
     const uint32_t ws_off = lds0 + (uint32_t)(MD_A_BYTES + MD_WC_BYTES + wave * 256 + ((i >> 4) * 32 + (i & 15)) * 4);
-    const float fp8_up = q4_fp8_up();
 
     md_f16v acc[TA];
 #pragma unroll
@@ -227,46 +226,18 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
             for (int a = 0; a < TA; a++) asm volatile("" : "+v"(fa[k][a]));
         };
         asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(cw[0]), "+v"(cw[1]), "+v"(sw) : "n"(TA * LEAD));
-        // this lane's 8 weights of group ks: chunk 2 (ks % 2) + g of block ks / 2 -- value half(fma(q, scale, base)), q4x8_dequant's
-        // arithmetic (ifa_dequant_q4.h) in four pieces
-        uint32_t d_lo = 0, d_hi = 0; q4_f2 d_s2 = {0, 0}, d_b2 = {0, 0}, d_e02 = {0, 0}, d_e46 = {0, 0}, d_o13 = {0, 0}, d_o57 = {0, 0};
+        // this lane's 8 weights of group ks: chunk 2 (ks % 2) + g of block ks / 2 -- q4x8_dequant_mo's arithmetic (ifa_dequant_q4.h) in four pieces
+        uint32_t d_lo = 0, d_hi = 0; q4_h2 d_s2 = {0, 0}, d_b2 = {0, 0}, d_w[4];
         auto dq_a = [&](int ks) {
             const int h = ks >> 1;
-            const uint32_t sbw = sw[h];
-            const float base = hbits2f((uint16_t)(sbw & 0xFFFFu)), scale = hbits2f((uint16_t)(sbw >> 16)) * fp8_up;
             const uint32_t c_lo = cw[h][2 * (ks & 1)], c_hi = cw[h][2 * (ks & 1) + 1];      // (scalars first: one select, not an indexed element read)
-            const uint32_t code = g ? c_hi : c_lo;
+            const uint32_t code = g ? c_hi : c_lo, sbw = sw[h];
             d_lo = code & 0x0F0F0F0Fu; d_hi = (code >> 4) & 0x0F0F0F0Fu;
-            d_s2 = q4_f2{scale, scale}; d_b2 = q4_f2{base, base};
+            d_s2 = q4_scale2(sbw); d_b2 = q4_base2(sbw);
         };
-#ifndef IFA_MID_SCALAR_FMA
-#define IFA_MID_SCALAR_FMA 0      // 1: the conversion's fused multiply-adds as scalar v_fma_f32 (the guide prices a packed f32 op beside MFMAs at +22 cycles)
-#endif
-        auto fma2 = [&](q4_f2 x) {
-#if IFA_MID_SCALAR_FMA
-            q4_f2 r;
-            float r0, r1;
-            asm("v_fma_f32 %0, %1, %2, %3" : "=v"(r0) : "v"(x[0]), "v"(d_s2[0]), "v"(d_b2[0]));
-            asm("v_fma_f32 %0, %1, %2, %3" : "=v"(r1) : "v"(x[1]), "v"(d_s2[0]), "v"(d_b2[0]));
-            r[0] = r0; r[1] = r1;
-            return r;
-#else
-            return __builtin_elementwise_fma(x, d_s2, d_b2);
-#endif
-        };
-        auto dq_b = [&]() {
-            d_e02 = fma2(__builtin_amdgcn_cvt_pk_f32_fp8((int)d_lo, false));
-            d_e46 = fma2(__builtin_amdgcn_cvt_pk_f32_fp8((int)d_lo, true));
-        };
-        auto dq_c = [&]() {
-            d_o13 = fma2(__builtin_amdgcn_cvt_pk_f32_fp8((int)d_hi, false));
-            d_o57 = fma2(__builtin_amdgcn_cvt_pk_f32_fp8((int)d_hi, true));
-        };
-        auto dq_d = [&]() {
-            const q4_h2 w0 = __builtin_convertvector(q4_f2{d_e02[0], d_o13[0]}, q4_h2), w1 = __builtin_convertvector(q4_f2{d_e02[1], d_o13[1]}, q4_h2);
-            const q4_h2 w2 = __builtin_convertvector(q4_f2{d_e46[0], d_o57[0]}, q4_h2), w3 = __builtin_convertvector(q4_f2{d_e46[1], d_o57[1]}, q4_h2);
-            return md_h8{w0[0], w0[1], w1[0], w1[1], w2[0], w2[1], w3[0], w3[1]};
-        };
+        auto dq_b = [&]() { d_w[0] = q4_value2<false>(d_lo, d_s2, d_b2); d_w[1] = q4_value2<true>(d_lo, d_s2, d_b2); };
+        auto dq_c = [&]() { d_w[2] = q4_value2<false>(d_hi, d_s2, d_b2); d_w[3] = q4_value2<true>(d_hi, d_s2, d_b2); };
+        auto dq_d = [&]() { return md_h8{d_w[0][0], d_w[0][1], d_w[1][0], d_w[1][1], d_w[2][0], d_w[2][1], d_w[3][0], d_w[3][1]}; };
         auto frag = [&](int ks, int a) { fa[ks][a] = md_lds_b128(a_off + sb + (uint32_t)(a * 32 * ROWB) + (uint32_t)(((2 * ks) ^ lc) << 4)); };
         md_h8 fbc, fbn;
         dq_a(0); dq_b(); dq_c(); fbc = dq_d();

@@ -45,7 +45,8 @@ struct GmArgs {
 
 // MO layout ("MFMA operand order") of a matrix [rows][cols] of 4-bit codes with value q * scale + base, cols % 128 == 0: per tile of 16 rows
 //   nsup = cols / 128 supersteps of 1024 bytes: lane l = 16 g + r of a wave owns bytes 16 l .. 16 l + 15 = the 16 code bytes of
-//   block 4 S + g of row 16 tile + r (exactly its A operands of the superstep's four MFMAs), then
+//   block 4 S + g of row 16 tile + r (exactly its A operands of the superstep's four MFMAs; byte b of a word of eight codes holds element b
+//   in its low and element 4 + b in its high nibble, the order in which ifa_dequant_q4.h needs no permutes), then
 //   ceil(nsup / 4) quads of 1024 bytes: lane l owns the (base, scale) words of its blocks in supersteps 4 Q .. 4 Q + 3.
 // Rows past the end and the pad of the last quad are zero.  Same size as the tiled copy (+ the pad).
 size_t gemm_rows_mo_bytes(size_t rows, size_t cols);

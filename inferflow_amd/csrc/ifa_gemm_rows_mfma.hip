@@ -59,6 +59,8 @@ __global__ void __launch_bounds__(256) k_gemm_rows_mo_build(const uint8_t *__res
                 c = *reinterpret_cast<const u32x4 *>(rp + (size_t)blk * 16);
                 w = *reinterpret_cast<const uint32_t *>(rp + (size_t)nblk * 16 + (size_t)blk * 4);
             }
+#pragma unroll
+            for (int k = 0; k < 4; k++) c[k] = q4_word_to_mo(c[k]);
         }
         uint8_t *tb = mo + (size_t)tile * mo_tile;
         if (S < nsup) *reinterpret_cast<u32x4 *>(tb + (size_t)S * 1024 + (size_t)lane * 16) = c;

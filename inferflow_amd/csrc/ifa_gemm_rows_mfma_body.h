@@ -142,7 +142,6 @@ __device__ __forceinline__ void gemm_rows_mfma_body(const GmArgs &P, char *smem)
     const size_t row_bytes = tiled_row_bytes(Q4_B32T1A, (size_t)nblk);
     const int nq4 = (nsup + 3) >> 2;                              // MO: header quads per tile
     const size_t mo_tile = (size_t)(nsup + nq4) * 1024;           // MO: bytes per 16-row tile
-    const float fp8_up = q4_fp8_up();                             // (ifa_dequant_q4.h)
     const int row_stride = WHOLE ? K * 2 + 16 : G::ROW_STRIDE;    // bytes per activation row in LDS
     const int trow = min(r, T - 1);                               // B operand: token of this lane (columns past T: duplicates, never stored)
     const int trow1 = min(r + 16, T - 1);                         // second column tile (NT == 2)
@@ -221,16 +220,16 @@ __device__ __forceinline__ void gemm_rows_mfma_body(const GmArgs &P, char *smem)
                 cw4 = *reinterpret_cast<const u32x4 *>(patch + (size_t)r * G::CSTRIDE + (size_t)(4 * j + g) * 16);
                 sbw = *reinterpret_cast<const uint32_t *>(patch + 16 * G::CSTRIDE + (size_t)r * G::SSTRIDE + (size_t)(4 * j + g) * 4);
             }
-            const float base = hbits2f((uint16_t)(sbw & 0xFFFFu)), scale_up = hbits2f((uint16_t)(sbw >> 16)) * fp8_up;
+            const q4_h2 base2 = q4_base2(sbw), scale2 = q4_scale2(sbw);
             const int xcol = (WHOLE ? chunk * G::CHUNK_COLS : 0) + (wave * G::BPW + 4 * j + g) * 32;
             const char *xrow = smem + (size_t)trow * row_stride + (size_t)xcol * 2;
             const char *xrow1 = smem + (size_t)trow1 * row_stride + (size_t)xcol * 2;
 #pragma unroll
             for (int s4 = 0; s4 < 4; s4++) {
-                // byte b of the word: low nibble = element 8 s4 + 2b, high nibble = the next one (ifa_gemm_rows.hip); the reference's
-                // dequantised halves, two codes per conversion (ifa_dequant_q4.h: 15 VALU instructions per 8 weights, was 19)
+                // the dequantised halves, two codes per instruction (ifa_dequant_q4.h); the two layouts differ in the order of a word's nibbles
                 q4_h2 wq[4];
-                q4x8_dequant(cw4[s4], scale_up, base, wq);
+                if constexpr (MO) q4x8_dequant_mo(cw4[s4], scale2, base2, wq);
+                else q4x8_dequant(cw4[s4], scale2, base2, wq);
                 const h8m a = {wq[0][0], wq[0][1], wq[1][0], wq[1][1], wq[2][0], wq[2][1], wq[3][0], wq[3][1]};
                 const h8m b = *reinterpret_cast<const h8m *>(xrow + s4 * 16);
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc, 0, 0, 0);

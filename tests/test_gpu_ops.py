@@ -435,6 +435,31 @@ def test_gemm_rows_streaming_kernel_matches_per_token_oracle(d, T, rows, cols):
             assert np.allclose(y[t].astype(np.float64), y64, rtol=2e-3, atol=2e-3 * float(np.abs(y64).mean() + 1))
 
 
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_rows_gemm_weights_are_rounded_once(seed):
+    """One-hot activations return the dequantised weights themselves: half(q * scale + base) with ONE rounding (csrc/ifa_dequant_q4.h), every code and lane
+    position, scales and bases up to 2^20 apart -- exactly the half nearest to the 64-bit value (which holds q * scale + base without rounding)."""
+    import ctypes as C
+    L = g.capi()
+    L.ifa_gemm_rows_q4.restype = C.c_int
+    L.ifa_gemm_rows_q4.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_void_p, C.c_size_t, C.c_void_p, C.c_void_p, C.c_void_p]
+    rows, cols, T = 80, 128, 16
+    rng = np.random.default_rng(seed)
+    n = rows * cols // 32
+    scale = (rng.uniform(1, 2, n) * 2.0 ** rng.integers(-10, 5, n)).astype(np.float16)
+    base = (rng.choice([-1.0, 1.0], n) * rng.uniform(1, 2, n) * 2.0 ** rng.integers(-14, 10, n)).astype(np.float16)
+    codes = rng.integers(0, 16, (n, 32)).astype(np.uint8)
+    blocks = np.concatenate([base.view(np.uint8).reshape(n, 2), scale.view(np.uint8).reshape(n, 2), codes[:, 0::2] | (codes[:, 1::2] << 4)], 1).reshape(rows, -1)
+    want = (codes * scale.astype(np.float64)[:, None] + base.astype(np.float64)[:, None]).astype(np.float16).reshape(rows, cols)
+    Wt = g.repack(dt.Q4_B32T1A, g.dev(blocks), rows, cols)
+    for c0 in range(0, cols, T):
+        x = np.zeros((T, cols), np.float16)
+        x[np.arange(T), c0 + np.arange(T)] = 1.0
+        y = g.empty_f16(T, rows)
+        assert L.ifa_gemm_rows_q4(g.p(Wt), rows, cols, g.p(g.dev(x)), T, None, g.p(y), g.stream()) == 0
+        assert np.array_equal(g.host(y).T, want[:, c0:c0 + T]), c0
+
+
 def test_add_by_row_index_is_a_half_fma_scatter():
     # AddByRowIdx_Kernel (binary_tensor_opr.h:80-125): B[idx[r]] = hfma(A[r], w[r], B[idx[r]])
     rng = np.random.default_rng(9)
