@@ -1,4 +1,4 @@
-// ifa_decode_attn.h -- the batch-1 / batched decode attention kernels (k_dec_attn and the keys-split-over-workgroups
+// ifa_decode_attn.h -- the batch-1 decode attention kernels (k_dec_attn and the keys-split-over-workgroups
 // variants), split from ifa_decode_kernels.h so that the per-format GEMV translation units do not depend on them.
 #pragma once
 #include "ifa_decode_kernels.h"
@@ -21,7 +21,7 @@ struct DecAttnParams {
     int max_ctx;
     int8_t *xq;                // optional XqImage of `out` (Q8_B32T2, the quantiser the Wo GEMV would run in its prologue)
     long long *trace;          // optional [heads][8] wall-clock stamps (100 MHz) for tuning
-    // batched step (k_dec_attn<.., BATCH = true>, grid (heads, queries)): query b reads q|k|v at q + b * q_stride, its cache
+    // batched step (k_dec_attn_keys, ifa_decode_attn_keys.h): query b reads q|k|v at q + b * q_stride, its cache
     // pointers and context from batch_rows[b], its RoPE pairs at rope_tab + b * head_dim, and writes out + b * heads * head_dim
     const void *batch_rows;    // DecAttnBatchRow[queries]
     int q_stride;
@@ -47,6 +47,10 @@ __device__ __forceinline__ void dec_attn_emit_q8(int8_t *xq, int cols, int h, in
         Q.xsum[blk] = (float)sum;
     }
 }
+
+// The cache rows are read through pointers whose address space is STATED: in the batched step they come from the table in memory, and the FLAT loads the compiler emits
+// for a pointer of unknown origin also count on lgkmcnt -- every LDS wait of the score / softmax phases then waited for the K / V requests in flight
+#define IFA_GP(T, p) ((const __attribute__((address_space(1))) T *)(p))
 
 // rotate one pair with a precomputed (cos, sin); same expressions as rope_rotate
 __device__ __forceinline__ void rope_apply(half_t *row, int col, float c, float s, int order, int rope_cols)
@@ -155,25 +159,15 @@ struct DecAttnRegs {
 };
 
 // PHASE 0: the whole kernel; 1: the entry requests only; 2: everything behind them (R filled by a PHASE 1 call)
-template <int HD, bool Q8, bool BATCH, int PB, bool KT, bool FUSED, int PHASE = 0>
+template <int HD, bool Q8, int PB, bool KT, bool FUSED, int PHASE = 0>
 __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, const uint8_t *pkc, const uint8_t *pvc, int pheads, int pkvh,
                                               const DecAttnParams &P, const int h_in, const DecAttnFusedIn &F, DecAttnRegs<HD, Q8, PB, KT> &R)
 {
     int pos_b = 0;
     if constexpr (FUSED) pos_b = F.pos;
-    if constexpr (BATCH) {      // the query's cache pointers and position come from the step's table (one scalar fetch)
-        const DecAttnBatchRow br = reinterpret_cast<const DecAttnBatchRow *>(P.batch_rows)[blockIdx.y];
-        pkc = br.kc; pvc = br.vc; pos_b = br.n_ctx - 1;
-        pq += (size_t)blockIdx.y * P.q_stride;
-    }
-    // The cache rows are read through pointers whose address space is STATED (IFA_GP): in the batched step they come from the
-    // table in memory, and the FLAT loads the compiler emits for a pointer of unknown origin also count on lgkmcnt -- every LDS
-    // wait of the score / softmax phases then waited for the K / V requests in flight
-#define IFA_GP(T, p) ((const __attribute__((address_space(1))) T *)(p))
-    uint8_t *const kcw = BATCH ? const_cast<uint8_t *>(pkc) : P.kcache;      // the cache rows this workgroup may write
-    uint8_t *const vcw = BATCH ? const_cast<uint8_t *>(pvc) : P.vcache;
-    const float *const rope_tab = BATCH ? P.rope_tab + (size_t)blockIdx.y * HD : P.rope_tab;
-    half_t *const outp = BATCH ? P.out + (size_t)blockIdx.y * pheads * HD : P.out;
+    uint8_t *const kcw = P.kcache, *const vcw = P.vcache;      // the cache rows this workgroup may write
+    const float *const rope_tab = P.rope_tab;
+    half_t *const outp = P.out;
     static_assert(HD % 8 == 0 && HD <= 128 && (!Q8 || HD % 32 == 0), "head size: multiples of 8 up to 128 (Q8 rows: whole 32-blocks)");
     constexpr int DG = HD / 8;            // threads covering one V row (8 dims each)
     constexpr int NSPLIT = 256 / DG;      // key residues handled in parallel (head sizes 48 / 80 / 96: the last 256 % DG threads idle)
@@ -182,8 +176,7 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
     half_t *vn = kn + HD;                                          // [HD] new v (Q8 round-tripped)
     float *red = reinterpret_cast<float *>(vn + HD);               // [16]
     float *opart = red + 16;                                       // [NSPLIT][HD]
-    static_assert(!KT || (!Q8 && !BATCH && (DG & (DG - 1)) == 0 && PB % NSPLIT == 0), "K tile through LDS: F16 rows, one query, power-of-two pieces per row");
-    static_assert(!(FUSED && BATCH), "the fused tail is a single-query kernel");
+    static_assert(!KT || (!Q8 && (DG & (DG - 1)) == 0 && PB % NSPLIT == 0), "K tile through LDS: F16 rows, one query, power-of-two pieces per row");
     static_assert(PB >= NSPLIT && PB <= DEC_ATTN_MIN_ROWS, "prefetch bucket");
     uint8_t *ktile = reinterpret_cast<uint8_t *>(opart + NSPLIT * HD);                         // KT: [PB][HD] halves, 16-byte pieces XOR-swizzled by key
     half_t *S = reinterpret_cast<half_t *>(ktile + (KT ? (size_t)PB * HD * 2 : 0));            // [n_ctx]
@@ -240,9 +233,7 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
     q_in = (half_t)0; k_in = (half_t)0; v_in = (half_t)0;
     if constexpr (!FUSED) { q_in = pq[(size_t)h * HD + dq]; k_in = pq[(size_t)(pheads + kvh) * HD + dq]; v_in = pq[(size_t)(pheads + pkvh + kvh) * HD + dq]; }
     }
-    // (tid < DEC_ATTN_MIN_ROWS <= rows of the cache.)  Batched step: the position arrived with the cache pointers, so rows past
-    // the context are clamped to the last one (duplicate addresses: one cache line) -- unclamped, every (head, query) workgroup
-    // pulled 2 x 64 KB of cache rows whatever its context: 134 MB per layer at 32 queries, the whole cost of that launch
+    // (tid < DEC_ATTN_MIN_ROWS <= rows of the cache.)
     const int dg = tid % DG, sp = tid / DG;
     const bool vact = (256 % DG == 0) || sp < NSPLIT;   // this thread takes part in P.V
     constexpr int VPRE = PB / NSPLIT;                   // prefetched V keys per thread: j = sp + NSPLIT*i (PB keys)
@@ -251,7 +242,7 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
 #pragma unroll
         for (int i = 0; i < PB / NSPLIT; i++) kt[i] = IFA_GP(u32x4, pkc + (size_t)min(sp + NSPLIT * i, FUSED ? min(pos_b, PB - 1) : PB - 1) * row_bytes + head_off)[dg];
     } else {
-        load_k((BATCH || FUSED) ? min(tid, min(pos_b, PB - 1)) : min(tid, PB - 1));
+        load_k(FUSED ? min(tid, min(pos_b, PB - 1)) : min(tid, PB - 1));
     }
     // this step's (cos, sin) pair of the thread that will rotate: requested BETWEEN the K and the V rows -- behind both it was the
     // newest request, and the rotation waited (vmcnt(0)) for the whole prefetch; unconditional (a valid dummy address without RoPE)
@@ -266,7 +257,7 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
     const size_t vq_off = head_off + (size_t)(dg / 4) * 34;
 #pragma unroll
     for (int i = 0; i < VPRE; i++) {
-        const int j = min(sp + NSPLIT * i, BATCH ? pos_b : (FUSED ? min(pos_b, PB - 1) : PB - 1));
+        const int j = min(sp + NSPLIT * i, FUSED ? min(pos_b, PB - 1) : PB - 1);
         if constexpr (!Q8) {
             vreg[i] = IFA_GP(u32x4, pvc + (size_t)j * row_bytes + head_off)[dg];
         } else {
@@ -288,7 +279,7 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
     if (tr) P.trace[h * 8 + 0] = wall_clock64();
     // (a SCALAR load through the constant address space: as a vector load it was the newest request of the wave, and waiting for it
     //  -- vmcnt(0) -- meant waiting for every K / V row requested above before the new token's values could even be staged)
-    const int pos = (BATCH || FUSED) ? pos_b : *(const __attribute__((address_space(4))) int *)(P.state + 1);
+    const int pos = FUSED ? pos_b : *(const __attribute__((address_space(4))) int *)(P.state + 1);
     const int n_ctx = pos + 1;
     if constexpr (FUSED) {
         // the new token's values: one granule per row, valid when its tag is this step's epoch.  The producers are the other
@@ -378,31 +369,8 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
     const float alpha = 1.0f / sqrtf((float)HD) / P.kq_scale;
     const float mk = P.alibi ? alibi_slope(h + P.alibi_base, P.alibi_total) : 0.0f;
     float lmax = -INFINITY;
-    // BATCH (round 6, second session): the key row of the NEXT iteration is requested (into a second register set, clamped, unconditional)
-    // before this iteration's products -- the loop asked for a row and waited for it, one round trip per 256 keys with one workgroup per
-    // (head, query) and CU.  Single-query kernels stay as they were (they hand contexts past 320 keys to the split kernels).
-    uint32_t kreg2[(BATCH && !Q8) ? HD / 2 : 1];
-    uint32_t kq32b[(BATCH && Q8 && KALIGN >= 4) ? KBYTES / 4 : 1];
-    constexpr bool KPRE = BATCH && (!Q8 || KALIGN >= 4);
-    bool have = false;                                   // (KPRE) kreg / kq32 already hold row j
     for (int j = tid; j < n_ctx; j += 256) {
         ScoreAcc acc;
-        if constexpr (KPRE) {
-            const uint8_t *rowp2 = pkc + (size_t)min(j + 256, n_ctx - 1) * row_bytes + head_off;
-            if constexpr (!Q8) {
-#pragma unroll
-                for (int i = 0; i < HD / 8; i++) {
-                    const u32x4 t = IFA_GP(u32x4, rowp2)[i];
-                    kreg2[4 * i] = t[0]; kreg2[4 * i + 1] = t[1]; kreg2[4 * i + 2] = t[2]; kreg2[4 * i + 3] = t[3];
-                }
-            } else if constexpr (KALIGN == 8) {
-#pragma unroll
-                for (int i = 0; i < KBYTES / 8; i++) { const u32x2 t = IFA_GP(u32x2, rowp2)[i]; kq32b[2 * i] = t[0]; kq32b[2 * i + 1] = t[1]; }
-            } else {
-#pragma unroll
-                for (int i = 0; i < KBYTES / 4; i++) kq32b[i] = IFA_GP(uint32_t, rowp2)[i];
-            }
-        }
         if (Q8 && j == pos) {
             // the new token's (round-tripped) key: wide LDS reads into registers, then the same chain -- a scalar loop
             // over LDS kept the whole workgroup waiting at the next barrier for ~0.7 us
@@ -424,8 +392,8 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
                         const u32x4 t = reinterpret_cast<const u32x4 *>(kn)[i];
                         kreg[4 * i] = t[0]; kreg[4 * i + 1] = t[1]; kreg[4 * i + 2] = t[2]; kreg[4 * i + 3] = t[3];
                     }
-                } else if (j >= PB && !have) load_k(j);       // rows past the prefetched bucket: load now
-            } else if (j >= PB && !have) load_k(j);
+                } else if (j >= PB) load_k(j);       // rows past the prefetched bucket: load now
+            } else if (j >= PB) load_k(j);
             if constexpr (Q8) {
 #pragma unroll
                 for (int b = 0; b < HD / 32; b++) {
@@ -464,16 +432,6 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
         if (P.alibi) { float a = (float)j * mk; s = f2h(a + h2f(s)); }
         S[j] = s;
         lmax = fmaxf(lmax, P.kq_scale * h2f(s));
-        if constexpr (KPRE) {                            // the next iteration's row moves into the working registers
-            if constexpr (!Q8) {
-#pragma unroll
-                for (int i = 0; i < HD / 2; i++) kreg[i] = kreg2[i];
-            } else {
-#pragma unroll
-                for (int i = 0; i < KBYTES / 4; i++) kq32[i] = kq32b[i];
-            }
-            have = true;
-        }
     }
     if (tr) P.trace[h * 8 + 3] = wall_clock64();
     lmax = wave_max(lmax);
@@ -603,7 +561,7 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
         for (int s2 = 1; s2 < NSPLIT; s2++) acc = acc + opart[s2 * HD + tid];
         const half_t yh = f2h(acc);
         outp[(size_t)h * HD + tid] = yh;
-        if constexpr (HD % 32 == 0 && !BATCH) { if (P.xq) dec_attn_emit_q8<HD>(P.xq, P.heads * HD, h, tid, yh); }
+        if constexpr (HD % 32 == 0) { if (P.xq) dec_attn_emit_q8<HD>(P.xq, P.heads * HD, h, tid, yh); }
         if constexpr (FUSED && HD % 32 == 0) {
             if (F.att_gran) {
                 // the Alg2 quantiser of dec_attn_emit_q8 (same expressions), published as granules: four codes per dword (the quad's
@@ -632,13 +590,13 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
     if (tr) P.trace[h * 8 + 7] = wall_clock64();
 }
 
-template <int HD, bool Q8, bool BATCH = false, int PB = DEC_ATTN_MIN_ROWS, bool KT = false>
+template <int HD, bool Q8, int PB = DEC_ATTN_MIN_ROWS, bool KT = false>
 __global__ void __launch_bounds__(256) k_dec_attn(const half_t *pq, const uint8_t *pkc, const uint8_t *pvc, int pheads, int pkvh,
                                                   const DecAttnParams P)
 {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     DecAttnRegs<HD, Q8, PB, KT> R;
-    dec_attn_body<HD, Q8, BATCH, PB, KT, false>(smem, pq, pkc, pvc, pheads, pkvh, P, (int)blockIdx.x, DecAttnFusedIn{}, R);
+    dec_attn_body<HD, Q8, PB, KT, false>(smem, pq, pkc, pvc, pheads, pkvh, P, (int)blockIdx.x, DecAttnFusedIn{}, R);
 }
 
 // ------------------------------------------------------------ long contexts: keys split over workgroups

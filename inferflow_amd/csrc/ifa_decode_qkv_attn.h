@@ -167,7 +167,7 @@ __global__ void __launch_bounds__(QA_THREADS) k_dec_qkv_attn(const half_t *px, c
                 return;
             }
             DecAttnRegs<HD, Q8, PB, KT> RU;
-            dec_attn_body<HD, Q8, false, PB, KT, true>(smem, nullptr, A.kcache, A.vcache, A.heads, A.kv_heads, A, head, F, RU);
+            dec_attn_body<HD, Q8, PB, KT, true>(smem, nullptr, A.kcache, A.vcache, A.heads, A.kv_heads, A, head, F, RU);
             return;
         }
     }
@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(QA_THREADS) k_dec_qkv_attn(const half_t *px, c
         pre.finish(P.norm_w, P.norm_b, P.multi_base, P.eps, P.cols, L, P.xn_out, nullptr);
         load_rows(0, RW);
 #if IFA_QA_EARLY_KV
-        if (attn_wg) dec_attn_body<HD, Q8, false, PB, KT, true, 1>(smem, nullptr, A.kcache, A.vcache, A.heads, A.kv_heads, A, head, F, R);
+        if (attn_wg) dec_attn_body<HD, Q8, PB, KT, true, 1>(smem, nullptr, A.kcache, A.vcache, A.heads, A.kv_heads, A, head, F, R);
 #endif
     }
     lds_counter_wait(L.part + 131, NP);
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(QA_THREADS) k_dec_qkv_attn(const half_t *px, c
     if (attn_wg) {
         __syncthreads();             // every wave of this workgroup is done with the activation image: the LDS is the attention's now
         if (wave >= 4) return;
-        dec_attn_body<HD, Q8, false, PB, KT, true, IFA_QA_EARLY_KV ? 2 : 0>(smem, nullptr, A.kcache, A.vcache, A.heads, A.kv_heads, A, head, F, R);
+        dec_attn_body<HD, Q8, PB, KT, true, IFA_QA_EARLY_KV ? 2 : 0>(smem, nullptr, A.kcache, A.vcache, A.heads, A.kv_heads, A, head, F, R);
         return;
     }
 }

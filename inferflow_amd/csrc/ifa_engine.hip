@@ -299,6 +299,9 @@ int ifa_model_destroy(ifa_model *m)
     if (m->attn_ws.ml) (void)hipFree(m->attn_ws.ml);
     if (m->attn_ws.count) (void)hipFree(m->attn_ws.count);
     if (m->attn_ws.opart) (void)hipFree(m->attn_ws.opart);
+    if (m->keys_ws.ml) (void)hipFree(m->keys_ws.ml);
+    if (m->keys_ws.opart) (void)hipFree(m->keys_ws.opart);
+    if (m->keys_ws.count) (void)hipFree(m->keys_ws.count);
     for (Tensor &t : m->g) free_tensor(t);
     half_t **bufs[] = {&m->x, &m->x2, &m->xn, &m->hn, &m->pn, &m->q, &m->k, &m->v, &m->dqkv, &m->bqkv, &m->att, &m->a, &m->f, &m->t1, &m->t2, &m->logits,
                        &m->moe_gate, &m->moe_out, &m->moe_in, &m->moe_wdev};
@@ -469,6 +472,15 @@ int ifa_model_finalize(ifa_model *m)
         IFA_HIP_CHECK(hipMalloc((void **)&m->attn_ws.count, (size_t)c.heads * 4));
         IFA_HIP_CHECK(hipMemsetAsync(m->attn_ws.count, 0, (size_t)c.heads * 4, m->stream));
         IFA_HIP_CHECK(hipMalloc((void **)&m->attn_ws.opart, (size_t)c.heads * DEC_ATTN_MAX_SPLITS * c.head_dim * 4));
+    }
+    if (!m->keys_ws.count) {          // (for every number of queries that a fused step takes)
+        size_t slots = 0;
+        for (int n = 1; n <= DEC_KEYS_MAX_QUERIES; n++) slots = std::max(slots, (size_t)n * dec_keys_splits(c.heads, n, c.max_ctx));
+        slots *= c.heads;
+        IFA_HIP_CHECK(hipMalloc((void **)&m->keys_ws.ml, slots * 8));
+        IFA_HIP_CHECK(hipMalloc((void **)&m->keys_ws.opart, slots * c.head_dim * 4));
+        IFA_HIP_CHECK(hipMalloc((void **)&m->keys_ws.count, (size_t)DEC_KEYS_MAX_QUERIES * c.heads * 4));
+        IFA_HIP_CHECK(hipMemsetAsync(m->keys_ws.count, 0, (size_t)DEC_KEYS_MAX_QUERIES * c.heads * 4, m->stream));
     }
     if (!m->state) {
         IFA_HIP_CHECK(hipMalloc((void **)&m->state, sizeof(int) * (8 + ifa_model::RING)));

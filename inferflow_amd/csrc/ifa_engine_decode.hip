@@ -391,7 +391,7 @@ int launch_attn(ifa_model *m, int l)
     const dim3 grid((unsigned)c.heads), block(256);
     // (attention_lds_ok() routed contexts whose score row does not fit the 160 KiB LDS to the split kernels above)
 #define IFA_ATTN_GO(HDV, Q8V, PBV, KTV) do { \
-        auto kern = k_dec_attn<HDV, Q8V, false, PBV, KTV>; \
+        auto kern = k_dec_attn<HDV, Q8V, PBV, KTV>; \
         if (asmem > 48 * 1024) IFA_HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)asmem)); \
         kern<<<grid, block, asmem, m->stream>>>(A.q, A.kcache, A.vcache, A.heads, A.kv_heads, A); } while (0)
 #define IFA_ATTN_PB(HDV, Q8V, KTV) do { if (pb == 64) IFA_ATTN_GO(HDV, Q8V, 64, KTV); else if (pb == 128) IFA_ATTN_GO(HDV, Q8V, 128, KTV); else IFA_ATTN_GO(HDV, Q8V, 256, KTV); } while (0)

@@ -444,7 +444,7 @@ __global__ void __launch_bounds__(256) k_kv_store_rows(const half_t *__restrict_
 }
 
 // ---- the batched step as five launches per layer (the structure of the batch-1 step: ifa_gemm_rows_mfma.hip with the norm
-// prologue / GLU / residual epilogues, k_dec_attn<.., BATCH>): dense models with the sequential RMS wiring, every linear in
+// prologue / GLU / residual epilogues, k_dec_attn_keys): dense models with the sequential RMS wiring, every linear in
 // tiled Q4_B32T1, 2..16 queries.  Everything else takes the op-by-op rows below.
 bool batch_fused_ok(const ifa_model *m, int n)
 {
@@ -526,22 +526,7 @@ int batch_fused_layer(ifa_model *m, int l, int n, const half_t *x, half_t *xnext
         A.rope_order = c.rope_order; A.rope_cols = rope_dims;
         A.alibi = c.use_alibi; A.alibi_base = c.tp_rank * c.heads; A.alibi_total = c.heads * std::max(1, c.tp_size);
         A.out = m->att; A.max_ctx = c.max_ctx; A.batch_rows = rows_l; A.q_stride = (int)(QD + 2 * KVD);
-        const size_t asmem = dec_attn_smem(c.head_dim, c.max_ctx);
-        const dim3 grid((unsigned)c.heads, (unsigned)n), block(256);
-#define IFA_BATTN(HDV, Q8V) { auto kern = k_dec_attn<HDV, Q8V, true>; \
-        if (asmem > 48 * 1024) IFA_HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)asmem)); \
-        kern<<<grid, block, asmem, m->stream>>>(A.q, nullptr, nullptr, A.heads, A.kv_heads, A); }
-        switch (c.head_dim) {
-        case 32: if (A.kv_q8) IFA_BATTN(32, true) else IFA_BATTN(32, false) break;
-        case 64: if (A.kv_q8) IFA_BATTN(64, true) else IFA_BATTN(64, false) break;
-        case 96: if (A.kv_q8) IFA_BATTN(96, true) else IFA_BATTN(96, false) break;
-        case 128: if (A.kv_q8) IFA_BATTN(128, true) else IFA_BATTN(128, false) break;
-        case 48: IFA_BATTN(48, false) break;
-        case 80: IFA_BATTN(80, false) break;
-        default: return ifa_fail(IFA_ERR_ARG, "fused batched attention: head_dim %d", c.head_dim);
-        }
-#undef IFA_BATTN
-        IFA_LAUNCH_CHECK();
+        if ((rc = launch_attn_keys(A, m->keys_ws, c.head_dim, dec_keys_splits(c.heads, n, c.max_ctx), n, m->stream))) return rc;
     }
     // 3. wo (+ bias) + residual
     clear();

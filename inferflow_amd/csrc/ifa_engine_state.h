@@ -17,6 +17,7 @@
 #include "ifa_host.h"
 #include "ifa_decode_kernels.h"
 #include "ifa_decode_attn.h"
+#include "ifa_decode_attn_keys.h"
 #include "ifa_decode_gemv.h"
 #include "ifa_moe.h"
 #include "ifa_gemm_rows_mfma.h"
@@ -138,6 +139,7 @@ struct ifa_model {
     std::map<int, hipGraphExec_t> batch_graphs;      // captured batched step per batch size (dense models)
     // long-context decode attention (keys split over workgroups): workspace, switch and the context it starts at
     DecAttnSplitWs attn_ws = {nullptr, nullptr, nullptr, nullptr, 8};
+    DecKeysWs keys_ws = {nullptr, nullptr, nullptr, 1};      // batched steps
     int opt_attn_unload = 1;       // 1 (default): in the 256-row bucket the heads' workgroups of the fused QKV + attention launch take no weight rows (UL kernels)
     int opt_attn_nsplits = 0;      // > 0: splits per head whatever the context (measurement)
     // attention as the tail of the QKV launch (ifa_decode_qkv_attn.h): granules [layers][(heads + 2 kv_heads) * head_dim], the

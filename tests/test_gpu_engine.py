@@ -540,6 +540,44 @@ def test_batched_step_at_contexts_past_the_prefetched_bucket(kvd):
     wk.close()
 
 
+KEYS_SHAPES = {"d32": dict(heads=8, kv_heads=8, head_dim=32), "d48": dict(heads=8, kv_heads=4, head_dim=48), "d64": dict(heads=4, kv_heads=2, head_dim=64),
+               "d80": dict(heads=8, kv_heads=8, head_dim=80), "d96": dict(heads=4, kv_heads=4, head_dim=96), "d128": dict(heads=4, kv_heads=1, head_dim=128),
+               "d32_64heads": dict(heads=64, kv_heads=8, head_dim=32)}
+
+
+@pytest.mark.parametrize("shape,kvd", [(n, k) for n in KEYS_SHAPES for k in (dt.F16, dt.Q8_B32T2) if k == dt.F16 or KEYS_SHAPES[n]["head_dim"] % 32 == 0],
+                         ids=lambda v: v if isinstance(v, str) else ("kvf16" if v == dt.F16 else "kvq8"))
+def test_batched_attention_at_the_edges_of_passes_and_splits(shape, kvd, monkeypatch):
+    """k_dec_attn_keys: rows around one pass of a workgroup (128 keys of 128 dims, 256 of 64, 512 of 32), around a split (256 keys) and over several, head sizes that leave
+    lanes idle, grouped queries, splits of 512 keys (64 heads, 13 queries: two splits); against the op-by-op rows with the bounds of the test above, row order, and the same
+    bits again (the counts are back at zero)"""
+    monkeypatch.setitem(synth.SHAPES, "keys_" + shape, dict(dim=256, layers=2, ffn=512, vocab=600, **KEYS_SHAPES[shape]))
+    wk, _, s = synth.build("keys_" + shape, dt.Q4_B32T1A, kvd, max_ctx=640, quant_threshold=0, std=0.06)
+    lens = [1, 2, 63, 64, 127, 128, 129, 255, 256, 300, 511, 513, 600]
+    n, V = len(lens), s["vocab"]
+    wk.kv_slots(n)
+    rng = np.random.default_rng(7)
+    for i, k in enumerate(lens):
+        wk.select_kv(i)
+        wk.forward(rng.integers(3, V, k).astype(np.int32), 0)
+    cur = [int(t) for t in rng.integers(3, V, n)]
+    lg, lgu, lgp = (torch.empty((n, V), dtype=torch.float16, device="cuda") for _ in range(3))
+    wk.set_option("batch_fused", 0)
+    wk.decode_batch(cur, lens, list(range(n)), lgu)
+    wk.set_option("batch_fused", 1)
+    toks = wk.decode_batch(cur, lens, list(range(n)), lg)
+    A, U = g.host(lg).astype(np.float32), g.host(lgu).astype(np.float32)
+    for i in range(n):
+        cos = float((A[i] * U[i]).sum() / (np.linalg.norm(A[i]) * np.linalg.norm(U[i])))
+        assert cos >= 0.9999 and np.abs(A[i] - U[i]).max() <= 0.02, (lens[i], cos, np.abs(A[i] - U[i]).max())
+    order = [int(v) for v in rng.permutation(n)]
+    wk.decode_batch([cur[i] for i in order], [lens[i] for i in order], order, lgp)
+    assert np.array_equal(g.host(lgp), g.host(lg)[order])
+    for _ in range(2):
+        assert [int(t) for t in wk.decode_batch(cur, lens, list(range(n)))] == [int(t) for t in toks]
+    wk.close()
+
+
 @pytest.mark.parametrize("n", [2, 5, 8, 11, 16, 20, 27, 32])
 @pytest.mark.parametrize("kvd,shape", [(dt.F16, "test_mha"), (dt.Q8_B32T2, "test_mha"), (dt.F16, "test_moe"), (dt.F16, "test_moe_longffn")],
                          ids=["kvf16", "kvq8", "moe", "moe_longffn"])
