@@ -119,7 +119,7 @@ struct LayeredNet {
     // 128, 67 MB where 4096 tokens take 24 -- up to opt_workspace_mb each.  A step beyond that, or whose workspace cannot be had, runs without (fp32 tiles, token by token).
     float *tile_ws = nullptr; size_t tile_ws_bytes = 0;
     int opt_workspace_mb = 4096; bool step_tile_ws = false;
-    bf16_t *a16 = nullptr, *h16 = nullptr; size_t a16_cap = 0, h16_cap = 0; int opt_a16_min = 17;          // activations of a prompt's product rounded to bfloat16; steps of at least this many rows (0: never)
+    bf16_t *a16 = nullptr, *h16 = nullptr, *g16 = nullptr; size_t a16_cap = 0, h16_cap = 0, g16_cap = 0; int opt_a16_min = 17;          // activations of a prompt's product rounded to bfloat16; steps of at least this many rows (0: never)
     int opt_fuse_step = 1;                  // single-token steps of PARALLEL layers: norm inside the input product, everything behind the mixers in one launch
     int opt_attn_tile_min = 16;            // steps of at least this many rows run the windowed attention through the tiled kernel
     std::vector<ifa_seq_desc> seqs_host;   // the current step's sequences (the tiled attention's grid is sized from them)
@@ -439,26 +439,48 @@ int linear(ifa_model *m, const bf16_t *W, size_t N, size_t K, const float *A, si
     return ifa_linear_bf16w(W, N, K, A, lda, T, bias, mul, alpha, accumulate, m->lay->cfg.ops32, C, ldc, silu0, silu1, (ifa_stream)m->stream);
 }
 
-// the product behind a gated feed-forward's activations: they leave gate | up in the form that the product reads
-int glu_linear(ifa_model *m, int kind, float limit, const float *gate_up, size_t ld, size_t F, const float *row_gate, size_t ldg, const bf16_t *W, size_t N, size_t T,
-               const bf16_t *bias, const bf16_t *mul, int accumulate, float *C)
+// product of what a norm has left: bfloat16 rows (h16) or 32-bit rows
+int linear_in(ifa_model *m, const bf16_t *W, size_t N, size_t K, const float *h, const bf16_t *h16, size_t T, const bf16_t *bias, float *C, size_t ldc)
+{
+    if (h16) return ifa_linear_bf16_both(W, N, K, h16, K, T, bias, nullptr, 1.0f, 0, 0, C, nullptr, ldc, 0, 0, (ifa_stream)m->stream);
+    return linear(m, W, N, K, h, K, T, bias, nullptr, 1.0f, 0, C, ldc);
+}
+
+// A product whose columns [c_glu, c_glu + 2 F) are gate | up of a gated feed-forward.  Where the down-projection reads bfloat16 rows, the activations leave it so (n->g16; the
+// columns themselves are not stored), otherwise gate | up stay in C; glu_down is told by *left16.
+int linear_glu(ifa_model *m, const bf16_t *W, size_t N, size_t K, const float *h, const bf16_t *h16, size_t T, const bf16_t *bias, float *C, size_t ldc, int silu0, int silu1,
+               size_t c_glu, size_t F, int kind, float limit, bool *left16)
 {
     LayeredNet *n = m->lay;
     ifa_stream s = (ifa_stream)m->stream;
     int rc;
+    *left16 = takes_a16(n, K, T) && takes_a16(n, F, T);
+    if (!*left16) {
+        if (h16) return ifa_linear_bf16_both(W, N, K, h16, K, T, bias, nullptr, 1.0f, 0, 0, C, nullptr, ldc, silu0, silu1, s);
+        return linear(m, W, N, K, h, K, T, bias, nullptr, 1.0f, 0, C, ldc, silu0, silu1);
+    }
+    if ((rc = ensure_halfs(m, n->g16, n->g16_cap, T * a16_stride(F)))) return rc;
+    if (!h16) {
+        if ((rc = ensure_a16(m, T, K)) || (rc = ifa_rows_to_bf16(h, K, T, K, n->a16, a16_stride(K), s))) return rc;
+        h16 = n->a16;
+    }
+    return ifa_linear_bf16_glu(W, N, K, h16, a16_stride(K), T, bias, C, ldc, silu0, silu1, c_glu, F, kind, limit, n->g16, a16_stride(F), s);
+}
+
+// the down-projection behind it; row_gate (where they have not left so): the activations of row t times sigmoid(row_gate[t * ldg])
+int glu_down(ifa_model *m, bool left16, int kind, float limit, const float *gate_up, size_t ld, size_t F, const float *row_gate, size_t ldg, const bf16_t *W, size_t N, size_t T,
+             const bf16_t *bias, const bf16_t *mul, int accumulate, float *C)
+{
+    LayeredNet *n = m->lay;
+    ifa_stream s = (ifa_stream)m->stream;
+    int rc;
+    if (left16) return ifa_linear_bf16_both(W, N, F, n->g16, a16_stride(F), T, bias, mul, 1.0f, accumulate, 0, C, nullptr, N, 0, 0, s);
     if (takes_a16(n, F, T)) {
         if ((rc = ensure_a16(m, T, F)) || (rc = ifa_glu_to_bf16(kind, limit, gate_up, ld, T, F, row_gate, ldg, n->a16, a16_stride(F), s))) return rc;
         return ifa_linear_bf16_both(W, N, F, n->a16, a16_stride(F), T, bias, mul, 1.0f, accumulate, 0, C, nullptr, N, 0, 0, s);
     }
     if ((rc = ifa_glu_ex_f32(kind, limit, gate_up, ld, T, F, row_gate, ldg, n->m3, F, s))) return rc;
     return linear(m, W, N, F, n->m3, F, T, bias, mul, 1.0f, accumulate, C, N);
-}
-
-// product of what a norm has left: bfloat16 rows (h16) or 32-bit rows
-int linear_in(ifa_model *m, const bf16_t *W, size_t N, size_t K, const float *h, const bf16_t *h16, size_t T, const bf16_t *bias, float *C, size_t ldc)
-{
-    if (h16) return ifa_linear_bf16_both(W, N, K, h16, K, T, bias, nullptr, 1.0f, 0, 0, C, nullptr, ldc, 0, 0, (ifa_stream)m->stream);
-    return linear(m, W, N, K, h, K, T, bias, nullptr, 1.0f, 0, C, ldc);
 }
 
 // What lies between two sub-layers of a POSTNORM block: x += gnorm(sub) * norm_w; [depth average]; [h = x + conv(x), tail advanced].
@@ -687,18 +709,20 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
         if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, F, n->proj, N2, T, nullptr, nullptr, 1.0f, 0, n->m2, W))) return rc;
         return close_sub(n->m2, L.T(IFA_LT_NORM2B).data, next_norm, in16);
     }
-    if ((rc = linear_in(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2))) return rc;
     if (!moe) {
         const size_t F = (size_t)sp.ffn;
-        if ((rc = glu_linear(m, 3, sp.f_limit, n->proj + L.c2_fg, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m2))) return rc;
+        bool left16 = false;
+        if ((rc = linear_glu(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2, 0, 0, L.c2_fg, F, 3, sp.f_limit, &left16))) return rc;
+        if ((rc = glu_down(m, left16, 3, sp.f_limit, n->proj + L.c2_fg, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m2))) return rc;
     } else {
+        if ((rc = linear_in(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2))) return rc;
         // the router's logits (bias added by the product) are columns of the second product; the chosen experts read norm2's output
         if ((rc = ifa_moe_route_top_f32(n->proj + L.c2_router, N2, T, sp.x_experts, sp.x_top, nullptr, n->moe_idx, n->moe_wgt, s))) return rc;
         if ((rc = ifa_moe_experts_gated_f32(n->h, W, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data, n->moe_idx, n->moe_wgt,
                                             c.ops32, n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, s))) return rc;
         if (sp.x_shared_ff > 0) {      // the shared expert: its gate sigmoid(w_sg . h) multiplies the activations in front of the down-projection
             const size_t SF = (size_t)sp.x_shared_ff;
-            if ((rc = glu_linear(m, 0, 0.0f, n->proj + L.c2_shg, N2, SF, n->proj + L.c2_sg, N2, (const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, W, T, nullptr, nullptr, 1, n->m2))) return rc;
+            if ((rc = glu_down(m, false, 0, 0.0f, n->proj + L.c2_shg, N2, SF, n->proj + L.c2_sg, N2, (const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, W, T, nullptr, nullptr, 1, n->m2))) return rc;
         }
     }
     return close_sub(n->m2, L.T(IFA_LT_NORM2B).data, next_norm, in16);
@@ -848,8 +872,9 @@ int run_streams_layer(ifa_model *m, LLayer &L, size_t T, int nseq, int pass, LLa
     if (!any_ffn) return IFA_OK;
     if (!moe) {
         const size_t F = (size_t)sp.ffn, N2 = L.n_in2;
-        if ((rc = linear(m, L.w_in2, N2, W, n->h, W, T, nullptr, nullptr, 1.0f, 0, n->proj, N2))) return rc;
-        if ((rc = glu_linear(m, 0, 0.0f, n->proj, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m1))) return rc;
+        bool left16 = false;
+        if ((rc = linear_glu(m, L.w_in2, N2, W, n->h, nullptr, T, nullptr, n->proj, N2, 0, 0, 0, F, 0, 0.0f, &left16))) return rc;
+        if ((rc = glu_down(m, left16, 0, 0.0f, n->proj, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m1))) return rc;
     } else {
         const int XA = sp.x_experts;
         if (T <= 8 && XA <= 256 && n->opt_fuse_post) {      // a few rows: the choice inside the experts' first launch
@@ -1021,12 +1046,16 @@ int run_layers(ifa_model *m, size_t T, int nseq)
         const bool lin = sp.mixer == IFA_MIX_WINDOW_LINEAR;
         // steps of a few rows: the norm is formed inside the product's read of the residual, the gated GELU inside the down-projection's
         const bool fuse = T <= 8 && W % 8 == 0;
+        bool left16 = false;
         if (fuse && (n->opt_fuse_rows & 1)) {
             if ((rc = ifa_linear_bf16w_rows(1, L.T(IFA_LT_NORM1).data, c.eps, L.w_in, NI, W, n->x, W, T, L.b_in, nullptr, 1.0f, 0, n->proj, NI,
                                             lin ? (int)L.c_lq : 0, lin ? (int)L.c_lg : 0, s))) return rc;
         } else {
             if ((rc = ifa_layernorm_f32(1, n->x, W, T, W, L.T(IFA_LT_NORM1).data, c.eps, n->h, W, s))) return rc;
-            if ((rc = linear(m, L.w_in, NI, W, n->h, W, T, L.b_in, nullptr, 1.0f, 0, n->proj, NI, lin ? (int)L.c_lq : 0, lin ? (int)L.c_lg : 0))) return rc;
+            const int silu0 = lin ? (int)L.c_lq : 0, silu1 = lin ? (int)L.c_lg : 0;
+            if (sp.ffn > 0) rc = linear_glu(m, L.w_in, NI, W, n->h, nullptr, T, L.b_in, n->proj, NI, silu0, silu1, L.c_fg, (size_t)sp.ffn, 1, 0.0f, &left16);
+            else rc = linear(m, L.w_in, NI, W, n->h, W, T, L.b_in, nullptr, 1.0f, 0, n->proj, NI, silu0, silu1);
+            if (rc) return rc;
         }
         if (sp.mixer == IFA_MIX_WINDOW_LINEAR) {
             const size_t AQ = (size_t)sp.a_heads * sp.a_dim, LV = (size_t)sp.l_heads * sp.l_vdim;
@@ -1061,7 +1090,7 @@ int run_layers(ifa_model *m, size_t T, int nseq)
                 if ((rc = ifa_linear_bf16w_rows(2, nullptr, 0.0f, L.T(IFA_LT_FFN_DOWN).data, W, F, n->proj + L.c_fg, NI, T, L.T(IFA_LT_FFN_DOWN_B).data,
                                                 L.T(IFA_LT_LS2).data, 1.0f, 1, n->x, W, 0, 0, s))) return rc;
             } else {
-                if ((rc = glu_linear(m, 1, 0.0f, n->proj + L.c_fg, NI, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T,
+                if ((rc = glu_down(m, left16, 1, 0.0f, n->proj + L.c_fg, NI, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T,
                                      (const bf16_t *)L.T(IFA_LT_FFN_DOWN_B).data, (const bf16_t *)L.T(IFA_LT_LS2).data, 1, n->x))) return rc;
             }
         }
@@ -1130,7 +1159,7 @@ int lay_destroy(ifa_model *m)
     for (float *p : n->slot_ptr) lay_free(p);
     lay_free(n->slot_base_dev);
     if (n->tab_pin) (void)hipHostFree(n->tab_pin);
-    lay_free(n->attn_ws); lay_free(n->tile_ws); lay_free(n->scan_ws); lay_free(n->a16); lay_free(n->h16);
+    lay_free(n->attn_ws); lay_free(n->tile_ws); lay_free(n->scan_ws); lay_free(n->a16); lay_free(n->h16); lay_free(n->g16);
     lay_free(n->tab_dev); lay_free(n->excl_dev); lay_free(n->next_dev); lay_free(n->ring_dev);
     float *bufs[] = {n->x, n->h, n->proj, n->m1, n->m2, n->m3, n->beta, n->decay, n->logits, n->taps};
     for (float *b : bufs) lay_free(b);

@@ -99,6 +99,15 @@ __device__ __forceinline__ float gelu_tanh_f(float z)
 {
     return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
+// gated activation: kind 0 silu(a) u, 1 gelu_tanh(a) u, 2 relu(a) u, 3 the clamped form a sigmoid(1.702 a) (u + 1)
+__device__ __forceinline__ float glu_of(int kind, float limit, float a, float u)
+{
+    if (kind == 3) {
+        const float gc = fminf(a, limit), uc = fminf(fmaxf(u, -limit), limit);
+        return gc * sigmoid_f(1.702f * gc) * (uc + 1.0f);
+    }
+    return (kind == 0 ? silu_exact(a) : (kind == 1 ? gelu_tanh_f(a) : fmaxf(a, 0.0f))) * u;
+}
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.0f ? z : log1pf(expf(z)); }
 
 // First key position that the query at position i sees: a sliding window (window <= 0: none) and / or chunks of `chunk` positions counted from

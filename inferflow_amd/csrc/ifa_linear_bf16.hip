@@ -39,6 +39,8 @@ struct LinArgs {
     const int *tile_map, *n_tiles, *a_rows; const float *row_scale;
     bf16_t *C16;                               // (k_lin_tile with act_kind 2: the output in bfloat16 instead of C)
     int act_kind;                              // every output after the bias passes 1: the exact (erf) GELU, 2: the square of relu
+    // (k_lin_tile, GLU) columns [glu_c0, glu_c0 + 2 glu_f) are gate | up: instead of them G16[t][c] = act(gate[c]) up[c] in bfloat16, glu_w columns (whole 64s, zero beyond glu_f)
+    bf16_t *G16; int ldg, glu_c0, glu_f, glu_w, glu_kind; float glu_limit;
 };
 
 __device__ __forceinline__ void lin_store(const LinArgs &P, int t, int n, float acc)
@@ -170,9 +172,15 @@ typedef const __attribute__((address_space(1))) void lt_glb_t;
 // NB > 2: NB buffers, a step asked for NB - 1 steps ahead.  For products whose tiles do not fill the chip, which wait for one step after the other (0.4 to 0.7 us a step
 // with two buffers, 0.25 with more: the requests' issue, the fragments' way from LDS and the chain of products).
 // GROUPED: row tiles and matrices from P.tile_map, the rows of A by P.a_rows (null: as they are), each output row times P.row_scale.
-template <int BM, int BN, int NB, bool GROUPED>
+// GLU: column tiles from P.glu_c0 on serve BN / 2 outputs of a gated feed-forward: of 32 columns of such a tile 16 are gates and 16 the ups of the same outputs, so that one
+// exchange between a wave's rows of 16 lanes brings the two together and the activation is formed here and rounded once (the same values as k_glu_to_bf16's).  The 32-bit gate | up
+// rows were written and read again by a launch of their own: 2048 rows of width 2048, 11264 of 19968 columns
+// gate | up, 237 + 23 us -> 243; 601 rows of width 1024 31.6 + 7.4 -> 32.
+constexpr int LT_GROUPED = 1, LT_GLU = 2;
+template <int BM, int BN, int NB, int MODE>
 __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_tile(LinArgs P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
 {
+    constexpr bool GROUPED = MODE & LT_GROUPED, GLU = MODE & LT_GLU;
     constexpr int WAVES = BM == 32 ? 1 : 4, TA = BM == 32 ? 1 : BM / 64, TB = BM == 32 ? 1 : BN / 64, AI = BM / (8 * WAVES), WI = BN / (8 * WAVES), ROWB = 2 * LT_BK, STEPB = (BM + BN) * ROWB;
     __shared__ __attribute__((aligned(16))) char smem[NB * STEPB];          // [NB steps][BM rows of A, BN rows of W]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5, wm = wave & 1, wn = wave >> 1;          // (BM = 32: one wave, one tile)
@@ -193,6 +201,10 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
             Wg += (size_t)tm[0] * P.N * P.K; t0 = tm[1]; t_end = tm[1] + tm[2];
         }
     }
+    // a tile of gates and ups: o0, its first output
+    const int n_tile = n0 / BN, n_plain = GLU ? (P.glu_c0 + BN - 1) / BN : 0;
+    const bool glu = GLU && n_tile >= n_plain;
+    const int o0 = (n_tile - n_plain) * (BN / 2), n_end = GLU ? P.glu_c0 : P.N;
     auto swz = [](int r) { return (r >> 1) & 7; };
     const bf16_t *asrc[AI], *wsrc[WI];
     int wlim[WI];          // furthest step offset of the lane's piece inside a row of W
@@ -206,7 +218,8 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
 #pragma unroll
     for (int j = 0; j < WI; j++) {
         const int row = (wave * WI + j) * 8 + (lane >> 3), c = (lane & 7) ^ swz(row);
-        wsrc[j] = Wg + (size_t)min(n0 + row, P.N - 1) * P.K + c * 8;
+        const int wr = glu ? P.glu_c0 + ((row & 16) ? P.glu_f : 0) + min(o0 + 16 * (row >> 5) + (row & 15), P.glu_f - 1) : min(n0 + row, n_end - 1);
+        wsrc[j] = Wg + (size_t)wr * P.K + c * 8;
         wlim[j] = P.K - 8 - c * 8;
     }
     const int nsteps = lda16 / LT_BK;
@@ -313,7 +326,7 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
 #pragma unroll
         for (int b = 0; b < TB; b++) {
             const int n = n0 + wn * (BN / 2) + 32 * b + i;
-            if (n >= P.N) continue;
+            if (n >= n_end) continue;
             const float bv = P.bias ? bf2f(P.bias[n]) : 0.0f, mv = P.alpha * (P.mul ? bf2f(P.mul[n]) : 1.0f);
 #pragma unroll
             for (int a = 0; a < TA; a++)
@@ -324,6 +337,27 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
                 }
         }
     };
+    if constexpr (GLU) {
+        if (glu) {
+            // lanes of a first row of 16 hold gates, those of a second one ups: after the exchange of a second row's r with a first row's r + 8 both hold both, rows r here, r + 8 there
+            const int hi = i >> 4;
+#pragma unroll
+            for (int b = 0; b < TB; b++) {
+                const int o = o0 + (BM == 32 ? 0 : wn * (BN / 4)) + 16 * b + (i & 15);
+                const float gb = P.bias && o < P.glu_f ? bf2f(P.bias[P.glu_c0 + o]) : 0.0f, ub = P.bias && o < P.glu_f ? bf2f(P.bias[P.glu_c0 + P.glu_f + o]) : 0.0f;
+#pragma unroll
+                for (int a = 0; a < TA; a++)
+#pragma unroll
+                    for (int r = 0; r < 8; r++) {
+                        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[a][b][r]), __float_as_uint(acc[a][b][r + 8]), false, false);
+                        const int t = t0 + wm * (BM / 2) + 32 * a + (r & 3) + 8 * (r >> 2) + 16 * hi + 4 * g;
+                        const float v = glu_of(P.glu_kind, P.glu_limit, __uint_as_float(x[0]) + gb, __uint_as_float(x[1]) + ub);
+                        if (t < t_end && o < P.glu_w) P.G16[(size_t)t * P.ldg + o] = __builtin_bit_cast(bf16_t, (__bf16)(o < P.glu_f ? v : 0.0f));
+                    }
+            }
+            return;
+        }
+    }
     if constexpr (GROUPED) {          // (the rows' scales take the place of the columns')
 #pragma unroll
         for (int a = 0; a < TA; a++)
@@ -355,13 +389,40 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
     }
 }
 
-template <int BM, int BN, int NB, bool GROUPED>
+// column tiles of a product (gate | up: with G16's padding)
+size_t lin_col_tiles(const LinArgs &P, int bn, bool glu) { return glu ? (P.glu_c0 + bn - 1) / bn + ((size_t)P.glu_w + bn / 2 - 1) / (bn / 2) : ((size_t)P.N + bn - 1) / bn; }
+
+template <int BM, int BN, int NB, int MODE>
 int launch_lin_tile(const LinArgs &P, const bf16_t *a16, size_t lda16, size_t row_tiles, hipStream_t s)
 {
-    const int tm = (int)row_tiles, tn = (P.N + BN - 1) / BN;
-    hipLaunchKernelGGL((k_lin_tile<BM, BN, NB, GROUPED>), dim3((unsigned)tm * (unsigned)tn), dim3(BM == 32 ? 64 : 256), 0, s, P, a16, (int)lda16, tm, tn);
+    const int tm = (int)row_tiles, tn = (int)lin_col_tiles(P, BN, MODE & LT_GLU);
+    hipLaunchKernelGGL((k_lin_tile<BM, BN, NB, MODE>), dim3((unsigned)tm * (unsigned)tn), dim3(BM == 32 ? 64 : 256), 0, s, P, a16, (int)lda16, tm, tn);
     IFA_LAUNCH_CHECK();
     return IFA_OK;
+}
+
+// the largest tile that still gives every compute unit its share of workgroups
+template <int MODE>
+int lin_tile_dispatch(const LinArgs &P, const bf16_t *a, size_t lda, hipStream_t s)
+{
+    constexpr bool GLU = MODE & LT_GLU;
+    const size_t T = (size_t)P.T, t128 = (T + 127) / 128, t64 = (T + 63) / 64, n128 = lin_col_tiles(P, 128, GLU), n64 = lin_col_tiles(P, 64, GLU);
+    IFA_REQUIRE(t64 * n64 < (1u << 31), "linear_bf16: too many tiles");
+    if (t128 * n128 >= 384) return launch_lin_tile<128, 128, 2, MODE>(P, a, lda, t128, s);
+    if (t128 * n64 >= 256) return launch_lin_tile<128, 64, 2, MODE>(P, a, lda, t128, s);
+    if (t64 * n64 > LT_DEEP || lda < 4 * LT_BK) return launch_lin_tile<64, 64, 2, MODE>(P, a, lda, t64, s);
+    if (t64 * n64 > LT_SMALL || lda < 8 * LT_BK) return launch_lin_tile<64, 64, 4, MODE>(P, a, lda, t64, s);
+    return launch_lin_tile<32, 32, 8, MODE>(P, a, lda, (T + 31) / 32, s);
+}
+
+template <int MODE>
+int lin_grouped_dispatch(const LinArgs &P, const bf16_t *a, size_t lda, size_t max_tiles, int tile_rows, hipStream_t s)
+{
+    const size_t n64 = lin_col_tiles(P, 64, MODE & LT_GLU);
+    IFA_REQUIRE(max_tiles * n64 < (1u << 31), "linear_bf16_grouped: too many tiles");
+    if (tile_rows == 128) return launch_lin_tile<128, 128, 2, MODE>(P, a, lda, max_tiles, s);
+    if (max_tiles * n64 > LT_DEEP || lda < 4 * LT_BK) return launch_lin_tile<64, 64, 2, MODE>(P, a, lda, max_tiles, s);
+    return launch_lin_tile<64, 64, 4, MODE>(P, a, lda, max_tiles, s);
 }
 
 // rows of 32-bit values to bfloat16, zero up to ldy (a multiple of 8)
@@ -658,23 +719,33 @@ extern "C" int ifa_linear_bf16_both(const void *w_bf16, size_t rows, size_t cols
     P.act_kind = act;
     hipStream_t s = ifa_s(stream);
     const bf16_t *a = (const bf16_t *)a_bf16;
-    // the largest tile that still gives every compute unit its share of workgroups
-    const size_t t128 = (tokens + 127) / 128, n128 = (rows + 127) / 128, n64 = (rows + 63) / 64;
-    IFA_REQUIRE(((tokens + 63) / 64) * n64 < (1u << 31), "ifa_linear_bf16_both: too many tiles");
-    const size_t t64 = (tokens + 63) / 64;
-    if (t128 * n128 >= 384) return launch_lin_tile<128, 128, 2, false>(P, a, lda, t128, s);
-    if (t128 * n64 >= 256) return launch_lin_tile<128, 64, 2, false>(P, a, lda, t128, s);
-    if (t64 * n64 > LT_DEEP || lda < 4 * LT_BK) return launch_lin_tile<64, 64, 2, false>(P, a, lda, t64, s);
-    if (t64 * n64 > LT_SMALL || lda < 8 * LT_BK) return launch_lin_tile<64, 64, 4, false>(P, a, lda, t64, s);
-    return launch_lin_tile<32, 32, 8, false>(P, a, lda, (tokens + 31) / 32, s);
+    return lin_tile_dispatch<0>(P, a, lda, s);
+}
+
+int ifa_linear_bf16_glu(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,
+                        int silu_col1, size_t glu_col0, size_t glu_cols, int glu_kind, float glu_limit, void *glu_bf16, size_t ldg, ifa_stream stream)
+{
+    IFA_REQUIRE(w_bf16 && a_bf16 && glu_bf16 && (c_f32 || glu_col0 == 0), "linear_bf16_glu: null pointer");
+    IFA_REQUIRE(rows > 0 && cols >= (size_t)LT_BK && cols % 8 == 0 && tokens > 0 && lda % 64 == 0 && lda >= cols && lda - cols < 64 && ldc >= glu_col0 && glu_cols > 0
+                && glu_col0 + 2 * glu_cols <= rows && ldg >= ((glu_cols + 63) & ~(size_t)63) && ldg < (1u << 30) && glu_kind >= 0 && glu_kind <= 3 && (glu_kind != 3 || glu_limit > 0.0f),
+                "linear_bf16_glu: bad shape (%zu x %zu, %zu tokens, lda %zu, gate | up %zu + 2 x %zu)", rows, cols, tokens, lda, glu_col0, glu_cols);
+    IFA_REQUIRE(rows < (1u << 30) && cols < (1u << 30) && tokens < (1u << 30) && (((uintptr_t)a_bf16 | (uintptr_t)w_bf16) & 15) == 0, "linear_bf16_glu: dimension too large or unaligned operand");
+    LinArgs P;
+    memset(&P, 0, sizeof(P));
+    P.W = (const bf16_t *)w_bf16; P.C = (float *)c_f32; P.bias = (const bf16_t *)bias_bf16; P.T = (int)tokens; P.N = (int)rows; P.K = (int)cols; P.ldc = (int)ldc; P.alpha = 1.0f;
+    P.act_c0 = silu_col0; P.act_c1 = silu_col1; P.G16 = (bf16_t *)glu_bf16; P.ldg = (int)ldg; P.glu_c0 = (int)glu_col0; P.glu_f = (int)glu_cols;
+    P.glu_w = (P.glu_f + 63) & ~63; P.glu_kind = glu_kind; P.glu_limit = glu_limit;
+    return lin_tile_dispatch<LT_GLU>(P, (const bf16_t *)a_bf16, lda, ifa_s(stream));
 }
 
 // ifa_linear_bf16w_grouped over bfloat16 rows (as ifa_linear_bf16_both reads them), tiles of at most tile_rows = 64 or 128 rows of one group
 int ifa_linear_bf16_grouped(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, const int *a_rows_dev, const int *tile_map_dev, const int *n_tiles_dev,
-                            size_t max_tiles, int tile_rows, const void *row_scale_f32, void *c_f32, size_t ldc, ifa_stream stream)
+                            size_t max_tiles, int tile_rows, const void *row_scale_f32, void *c_f32, size_t ldc, int glu_kind, float glu_limit, void *glu_bf16, ifa_stream stream)
 {
-    IFA_REQUIRE(w_bf16 && a_bf16 && c_f32 && tile_map_dev && n_tiles_dev, "linear_bf16_grouped: null pointer");
-    IFA_REQUIRE(rows > 0 && cols >= (size_t)LT_BK && cols % 8 == 0 && max_tiles > 0 && lda % 64 == 0 && lda >= cols && lda - cols < 64 && ldc >= rows
+    IFA_REQUIRE(w_bf16 && a_bf16 && (c_f32 || glu_bf16) && tile_map_dev && n_tiles_dev, "linear_bf16_grouped: null pointer");
+    IFA_REQUIRE(!glu_bf16 || (rows % 2 == 0 && ldc % 64 == 0 && ldc >= rows / 2 && ldc - rows / 2 < 64 && !row_scale_f32 && glu_kind >= 0 && glu_kind <= 3 && (glu_kind != 3 || glu_limit > 0.0f)),
+                "linear_bf16_grouped: bad gate | up (%zu rows, ldc %zu)", rows, ldc);
+    IFA_REQUIRE(rows > 0 && cols >= (size_t)LT_BK && cols % 8 == 0 && max_tiles > 0 && lda % 64 == 0 && lda >= cols && lda - cols < 64 && (glu_bf16 || ldc >= rows)
                 && (tile_rows == 64 || tile_rows == 128) && rows < (1u << 30) && cols < (1u << 30) && (((uintptr_t)a_bf16 | (uintptr_t)w_bf16) & 15) == 0,
                 "linear_bf16_grouped: bad shape (%zu x %zu, lda %zu)", rows, cols, lda);
     LinArgs P;
@@ -682,12 +753,12 @@ int ifa_linear_bf16_grouped(const void *w_bf16, size_t rows, size_t cols, const 
     P.W = (const bf16_t *)w_bf16; P.C = (float *)c_f32; P.N = (int)rows; P.K = (int)cols; P.ldc = (int)ldc; P.alpha = 1.0f;
     P.tile_map = tile_map_dev; P.n_tiles = n_tiles_dev; P.a_rows = a_rows_dev; P.row_scale = (const float *)row_scale_f32;
     const bf16_t *a = (const bf16_t *)a_bf16;
-    const size_t n64 = (rows + 63) / 64;
-    IFA_REQUIRE(max_tiles * n64 < (1u << 31), "linear_bf16_grouped: too many tiles");
     hipStream_t s = ifa_s(stream);
-    if (tile_rows == 128) return launch_lin_tile<128, 128, 2, true>(P, a, lda, max_tiles, s);
-    if (max_tiles * n64 > LT_DEEP || lda < 4 * LT_BK) return launch_lin_tile<64, 64, 2, true>(P, a, lda, max_tiles, s);
-    return launch_lin_tile<64, 64, 4, true>(P, a, lda, max_tiles, s);
+    if (glu_bf16) {          // (all columns are gate | up)
+        P.G16 = (bf16_t *)glu_bf16; P.ldg = P.glu_w = (int)ldc; P.glu_f = (int)(rows / 2); P.glu_kind = glu_kind; P.glu_limit = glu_limit;
+        return lin_grouped_dispatch<LT_GROUPED | LT_GLU>(P, a, lda, max_tiles, tile_rows, s);
+    }
+    return lin_grouped_dispatch<LT_GROUPED>(P, a, lda, max_tiles, tile_rows, s);
 }
 
 extern "C" int ifa_linear_bf16w_act(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *bias_bf16, int act,

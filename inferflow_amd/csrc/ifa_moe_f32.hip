@@ -508,9 +508,8 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
     if (in16) {
         bf16_t *h16 = (bf16_t *)yp, *a16 = (bf16_t *)actb;
         if ((rc = ifa_rows_to_bf16(h_f32, ldh, rows, (size_t)width, h16, lda_h, stream))) return rc;
-        if ((rc = ifa_linear_bf16_grouped(up_bf16, (size_t)2 * ff, (size_t)width, h16, lda_h, a_rows, tile_map, n_tiles, max_tiles, tile_rows, nullptr, gub, (size_t)2 * ff, stream))) return rc;
-        if ((rc = ifa_glu_to_bf16(glu_kind, limit, gub, (size_t)2 * ff, pairs, (size_t)ff, nullptr, 0, a16, lda_f, stream))) return rc;
-        if ((rc = ifa_linear_bf16_grouped(down_bf16, (size_t)width, (size_t)ff, a16, lda_f, nullptr, tile_map, n_tiles, max_tiles, tile_rows, w_sorted, yp, (size_t)width, stream))) return rc;
+        if ((rc = ifa_linear_bf16_grouped(up_bf16, (size_t)2 * ff, (size_t)width, h16, lda_h, a_rows, tile_map, n_tiles, max_tiles, tile_rows, nullptr, nullptr, lda_f, glu_kind, limit, a16, stream))) return rc;
+        if ((rc = ifa_linear_bf16_grouped(down_bf16, (size_t)width, (size_t)ff, a16, lda_f, nullptr, tile_map, n_tiles, max_tiles, tile_rows, w_sorted, yp, (size_t)width, 0, 0.0f, nullptr, stream))) return rc;
     } else if (gated) {
         if ((rc = ifa_linear_bf16w_grouped(up_bf16, (size_t)2 * ff, (size_t)width, experts, h_f32, ldh, a_rows, tile_map, n_tiles, max_tiles, nullptr, 0, ops32, gub, (size_t)2 * ff, stream))) return rc;
         if ((rc = ifa_glu_ex_f32(glu_kind, limit, gub, (size_t)2 * ff, pairs, (size_t)ff, nullptr, 0, actb, (size_t)ff, stream))) return rc;

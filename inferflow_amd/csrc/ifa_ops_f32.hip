@@ -276,16 +276,7 @@ __global__ void __launch_bounds__(256) k_softcap(float *__restrict__ x, size_t n
     if (i < n) x[i] = cap * tanhf(x[i] / cap);
 }
 
-// out[t][c] = act(gu[t][c]) * gu[t][F + c]  [* sigmoid(row_gate[t])];  kind 3: the clamped form g sigmoid(1.702 g) (u + 1)
-__device__ __forceinline__ float glu_of(int kind, float limit, float a, float u)
-{
-    if (kind == 3) {
-        const float gc = fminf(a, limit), uc = fminf(fmaxf(u, -limit), limit);
-        return gc * sigmoid_f(1.702f * gc) * (uc + 1.0f);
-    }
-    return (kind == 0 ? silu_exact(a) : (kind == 1 ? gelu_tanh_f(a) : fmaxf(a, 0.0f))) * u;
-}
-
+// out[t][c] = act(gu[t][c]) * gu[t][F + c]  [* sigmoid(row_gate[t])]
 __global__ void __launch_bounds__(256) k_glu_f32(int kind, float limit, const float *__restrict__ gu, size_t ld, int F, const float *__restrict__ row_gate, size_t ldg,
                                                  float *__restrict__ out, size_t ldo)
 {

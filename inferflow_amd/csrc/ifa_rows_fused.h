@@ -38,9 +38,14 @@ int ifa_delta_row_prep(const float *x, size_t ldx, int channels, int taps, const
                        size_t state_off, int norm_cols, int group_dim, float l2_eps, int scale_cols, float scale, float *y, size_t ldy, const float *b, const float *a, int heads,
                        const ifa32::bf16_t *a_log, const ifa32::bf16_t *dt_bias, float *beta, float *decay, ifa_stream stream);
 
-// grouped products over bfloat16 rows (csrc/ifa_linear_bf16.hip): see ifa_linear_bf16w_grouped
+// grouped products over bfloat16 rows (csrc/ifa_linear_bf16.hip): see ifa_linear_bf16w_grouped.  glu_bf16 not null: the matrices' rows are gate | up (rows / 2 each) and only
+// act(gate) up is left, in bfloat16 rows of ldc (whole 64s, zero beyond rows / 2)
 int ifa_linear_bf16_grouped(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, const int *a_rows_dev, const int *tile_map_dev, const int *n_tiles_dev,
-                            size_t max_tiles, int tile_rows, const void *row_scale_f32, void *c_f32, size_t ldc, ifa_stream stream);
+                            size_t max_tiles, int tile_rows, const void *row_scale_f32, void *c_f32, size_t ldc, int glu_kind, float glu_limit, void *glu_bf16, ifa_stream stream);
+// ifa_linear_bf16_both whose output columns [glu_col0, glu_col0 + 2 glu_cols) are gate | up of a gated feed-forward: glu_bf16[t][c] = act(gate[c]) up[c] in bfloat16 rows of ldg
+// (whole 64s, zero beyond glu_cols) in their place; the columns before them as ever, any behind them not at all
+int ifa_linear_bf16_glu(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,
+                        int silu_col1, size_t glu_col0, size_t glu_cols, int glu_kind, float glu_limit, void *glu_bf16, size_t ldg, ifa_stream stream);
 // ifa_glu_ex_f32 whose output only products read: bfloat16 rows, zero up to ldo (a multiple of 8; csrc/ifa_ops_f32.hip)
 int ifa_glu_to_bf16(int kind, float limit, const void *gate_up_f32, size_t ld, size_t rows, size_t cols, const void *row_gate_f32, size_t ldg, void *out_bf16, size_t ldo,
                     ifa_stream stream);

@@ -318,6 +318,22 @@ def test_prompts_with_and_without_the_workspaces_of_tiles_and_chunks(tmp_path, l
     eng.close()
 
 
+@pytest.mark.parametrize("T", [17, 130, 601, 1500, 3100])
+def test_activations_formed_behind_their_product(tmp_path, T):
+    """bfloat16 operands: the gated activations formed in the product's own tiles (every tile size, inner sizes of whole and of broken tiles) and left in bfloat16, against gate | up
+    stored, activated and rounded by launches of their own (a16_min 0): the same sums in the same order, so the same bits"""
+    import inferflow_amd as ia
+    cfg = fx.config([fx.delta_layer(heads=2, kv_heads=1, dim=16, vdim=16, conv=3, ff=ff) for ff in (72, 1032, 0)], width=520, vocab=97)
+    eng = engine_for(tmp_path, cfg, fx.random_weights(cfg, 35), "bfloat16", 3200, 1)
+    toks, out = tokens_for(cfg, T, 36), {}
+    for border in (0, 17):
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"a16_min", border))
+        out[border] = run_whole(eng, toks)[0]
+    eng.close()
+    assert out[17].shape == (T, 97) and np.isfinite(out[17]).all()
+    assert np.array_equal(out[0], out[17])
+
+
 def test_chunked_recurrences_are_switched_off_by_0(tmp_path):
     """the bits of the token-by-token form, which a border above every prompt has too; the chunks' differ"""
     import inferflow_amd as ia
