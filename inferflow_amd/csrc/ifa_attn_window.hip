@@ -57,6 +57,7 @@ struct WinAttnArgs {
     int sink_fixed; float sink_score;                            // sink_fixed != 0 (and sink null): every head's sink has this score
     const SeqDesc *seqs; const int *row_seq; float *const *slot_base; size_t k_off, v_off;
     float *out; size_t ldo;
+    bf16_t *out16; size_t ld16;      // (k_attn_tile, k_attn_tile_combine) not null: the output in bfloat16 instead, for the product behind
     float *ws; int nsplit;           // nsplit > 1: the keys of a (row, head) are shared out to nsplit workgroups; partial results in ws [rows][heads][nsplit][dim + 2]
 };
 
@@ -452,6 +453,7 @@ __global__ void __launch_bounds__(256) k_attn_window_tile(WinAttnArgs P, int n_s
 // overlap them).  Hence the operands are split and laid out once per layer by k_attn_parts, not by every tile that reads them (staged and split per
 // workgroup: 126 us), and the key blocks of long tiles go to several workgroups (chunks of cb blocks, joined by k_attn_tile_combine).
 typedef __bf16 bf16x8w __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4w __attribute__((ext_vector_type(4)));
 constexpr int WT_WAVES = 8, WT_MAX_CHUNKS = 32, WT_SLOTS = 256;
 
 typedef const __attribute__((address_space(1))) void wa_glb_t;
@@ -889,6 +891,24 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
     const float M = fmaxf(m, snk);
     const float f = expf(m - M);
     const float sc = f / (ls * f + (has_sink(P) ? expf(snk - M) : 0.0f));
+    if (P.out16) {
+        bf16_t *d16 = P.out16 + (size_t)(r0 + 32 * qsub + i) * P.ld16 + (size_t)h * dv;
+#pragma unroll
+        for (int nt = 0; nt < NTV; nt++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                const int c = 32 * nt + 8 * (r >> 2) + 4 * g;
+                bf16x4w v;
+#pragma unroll
+                for (int x = 0; x < 4; x++) v[x] = (__bf16)(o[nt][r + x] * sc);
+                if constexpr (VEC) { if (c < dv) *reinterpret_cast<bf16x4w *>(d16 + c) = v; }
+                else {
+#pragma unroll
+                    for (int x = 0; x < 4; x++) if (c + x < dv) d16[c + x] = __builtin_bit_cast(bf16_t, v[x]);
+                }
+            }
+        return;
+    }
     float *dst = P.out + (size_t)(r0 + 32 * qsub + i) * P.ldo + (size_t)h * dv;
 #pragma unroll
     for (int nt = 0; nt < NTV; nt++)
@@ -949,6 +969,11 @@ __global__ void __launch_bounds__(256) k_attn_tile_combine(WinAttnArgs P, TileAr
 #pragma unroll
     for (int k = 0; k < 16; k++) rows[q][(tid >> 5) + 8 * k] = o[k];
     __syncthreads();
+    if (P.out16) {
+        bf16_t *d16 = P.out16 + (size_t)(sd.row0 + tile * qw + 32 * qsub) * P.ld16 + (size_t)h * dv;
+        for (int e = tid; e < nq_w * dv; e += 256) d16[(size_t)(e / dv) * P.ld16 + e % dv] = __builtin_bit_cast(bf16_t, (__bf16)rows[e / dv][e % dv]);
+        return;
+    }
     float *dst = P.out + (size_t)(sd.row0 + tile * qw + 32 * qsub) * P.ldo + (size_t)h * dv;
     for (int e = tid; e < nq_w * dv; e += 256) dst[(size_t)(e / dv) * P.ldo + e % dv] = rows[e / dv][e % dv];
 }
@@ -1141,8 +1166,10 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
                             int window, int keep_first, const void *rel_bf16, const int *bucket_of_dev, int n_buckets, const void *sink_bf16, int sink_fixed,
                             float sink_score, const void *seqs_dev, const int *row_seq_dev, size_t rows, void *const *slot_base_dev, size_t k_off, size_t v_off,
                             void *out_f32, size_t ldo, const void *seqs_host, int n_seqs, int tile_min_rows, int max_keys, void *ws_f32, size_t ws_bytes,
-                            ifa_stream stream)
+                            ifa_stream stream, void *out_bf16 = nullptr, size_t ld16 = 0, bool *left16 = nullptr)
 {
+    if (left16) *left16 = false;
+    IFA_REQUIRE(!out_bf16 || (left16 && ld16 >= (size_t)heads * vdim), "%s: bad bfloat16 output", who);
     IFA_REQUIRE(q_f32 && seqs_dev && row_seq_dev && slot_base_dev && out_f32, "%s: null pointer", who);
     IFA_REQUIRE(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && dim > 0 && vdim > 0 && rows > 0 && window >= 1 && keep_first >= 0, "%s: bad shape", who);
     IFA_REQUIRE(dim <= 64 * WA_DPL_MAX && vdim <= 64 * WA_DPL_MAX, "%s: head size %d / %d above %d", who, dim, vdim, 64 * WA_DPL_MAX);
@@ -1153,7 +1180,7 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
     P.softcap = softcap; P.window = window; P.keep_first = keep_first; P.rel = (const bf16_t *)rel_bf16; P.bucket_of = bucket_of_dev; P.n_buckets = n_buckets;
     P.sink = (const bf16_t *)sink_bf16; P.sink_fixed = sink_fixed; P.sink_score = sink_score;
     P.seqs = (const SeqDesc *)seqs_dev; P.row_seq = row_seq_dev; P.slot_base = (float *const *)slot_base_dev;
-    P.k_off = k_off; P.v_off = v_off; P.out = (float *)out_f32; P.ldo = ldo; P.ws = nullptr; P.nsplit = 1;
+    P.k_off = k_off; P.v_off = v_off; P.out = (float *)out_f32; P.ldo = ldo; P.out16 = nullptr; P.ld16 = 0; P.ws = nullptr; P.nsplit = 1;
     // prompts: the tiled matrix-core kernels (heads of up to 128 dimensions, zero-padded to whole 32s); single tokens and other sizes: a workgroup per row.
     // With a workspace the bfloat16 form, from the smallest tiled step on (8 heads of 128: 16 rows 15.5 against 17.8 us, 256 rows 33 against 71, 64 rows behind 3000 keys 49 against 719).
     // Not for one row: its grids follow from the HOST's positions, and a step of one row is captured once and replayed while the position on the device goes on.
@@ -1164,7 +1191,9 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
             TileArgs A;
             A.n_seqs = n_seqs; A.hpw = t.hpw; A.cb = t.cb; A.tiles = (int)t.tiles; A.marks = t.mark_at / 4; A.shares = t.op_bytes / 4;
             P.ws = (float *)ws_f32; P.nsplit = t.chunks;
-            const bool vec = dim % 4 == 0 && vdim % 4 == 0 && ldq % 4 == 0 && ldo % 4 == 0 && (uintptr_t)q_f32 % 16 == 0 && (uintptr_t)out_f32 % 16 == 0;
+            if (out_bf16) { P.out16 = (bf16_t *)out_bf16; P.ld16 = ld16; *left16 = true; }
+            const bool vec = dim % 4 == 0 && vdim % 4 == 0 && ldq % 4 == 0 && ldo % 4 == 0 && (uintptr_t)q_f32 % 16 == 0 && (uintptr_t)out_f32 % 16 == 0
+                             && (!out_bf16 || (ld16 % 4 == 0 && (uintptr_t)out_bf16 % 8 == 0));
             const dim3 grid((unsigned)(heads / t.hpw), (unsigned)t.groups);
 #define IFA_WT(K, V) { const size_t smem_t = (size_t)2 * kBlockPieces<K, V> * 16 + WT_WAVES * 64 * 4; \
                        const void *fn = vec ? (const void *)k_attn_tile<K, V, true> : (const void *)k_attn_tile<K, V, false>; \
@@ -1324,6 +1353,27 @@ int ifa_attention_kv_sinks_f32(const void *q_f32, size_t ldq, int heads, int kv_
 
 } // extern "C"
 
+int ifa_attention_window_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int norm_q, float eps, float scale, float softcap, int window, int keep_first,
+                                 const void *rel_bf16, const int *bucket_of_dev, int n_buckets, const void *sink_bf16, const void *seqs_dev, const int *row_seq_dev, size_t rows,
+                                 void *const *slot_base_dev, size_t k_off, size_t v_off, void *out_f32, size_t ldo, void *out_bf16, size_t ld16, bool *left16, const void *seqs_host,
+                                 int n_seqs, int tile_min_rows, void *ws_f32, size_t ws_bytes, ifa_stream stream)
+{
+    const int tile_ok = dim % 32 == 0 && k_off % 4 == 0 && v_off % 4 == 0;          // (as ifa_attention_window_f32)
+    return attention_launch("attention_window_to_bf16", q_f32, ldq, heads, kv_heads, dim, dim, norm_q, eps, scale, softcap, window, keep_first, rel_bf16, bucket_of_dev, n_buckets,
+                            sink_bf16, 0, 0.0f, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, out_f32, ldo, seqs_host, tile_ok ? n_seqs : 0, tile_min_rows, 0, ws_f32,
+                            ws_bytes, stream, out_bf16, ld16, left16);
+}
+
+int ifa_attention_kv_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int vdim, float scale, int window, int keep_first, int sink, float sink_score,
+                             const void *seqs_dev, const int *row_seq_dev, size_t rows, void *const *slot_base_dev, size_t k_off, size_t v_off, void *out_f32, size_t ldo,
+                             void *out_bf16, size_t ld16, bool *left16, const void *seqs_host, int n_seqs, int tile_min_rows, int max_keys, void *ws_f32, size_t ws_bytes,
+                             ifa_stream stream)
+{
+    return attention_launch("attention_kv_to_bf16", q_f32, ldq, heads, kv_heads, dim, vdim, 0, 0.0f, scale, 0.0f, window > 0 ? window : (1 << 30), keep_first, nullptr, nullptr, 0,
+                            nullptr, sink ? 1 : 0, sink_score, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, out_f32, ldo, seqs_host, n_seqs, tile_min_rows, max_keys,
+                            ws_f32, ws_bytes, stream, out_bf16, ld16, left16);
+}
+
 int ifa_mix_row(const IfaMixRow &M, int *nsplit, ifa_stream stream)
 {
     IFA_REQUIRE(M.q && M.k && M.lq && M.lk && M.lv && M.decay && M.seqs && M.row_seq && M.slot_base && M.out && M.lin_out && nsplit, "mix_row: null pointer");
@@ -1333,7 +1383,7 @@ int ifa_mix_row(const IfaMixRow &M, int *nsplit, ifa_stream stream)
     P.q = M.q; P.heads = M.heads; P.kv_heads = M.kv_heads; P.dim = P.vdim = M.dim; P.norm_q = 1; P.eps = M.eps; P.scale = M.scale; P.softcap = M.softcap;
     P.window = M.window; P.keep_first = M.keep_first; P.rel = M.rel; P.bucket_of = M.bucket_of; P.n_buckets = M.n_buckets; P.sink = M.sink;
     P.seqs = (const SeqDesc *)M.seqs; P.row_seq = M.row_seq; P.slot_base = (float *const *)M.slot_base; P.k_off = M.k_off; P.v_off = M.v_off;
-    P.out = M.out; P.ldo = P.ldq = (size_t)M.heads * M.dim;
+    P.out = M.out; P.out16 = nullptr; P.ldo = P.ldq = (size_t)M.heads * M.dim;
     const size_t keys = std::min((size_t)M.window + (size_t)M.keep_first, (size_t)M.max_keys);
     int ns = (int)std::min<size_t>(IFA_ROW_OUT_SPLITS, (keys + 63) / 64);
     while (ns > 1 && (size_t)M.heads * ns * ((size_t)M.dim + 2) * 4 > M.ws_bytes) ns--;

@@ -653,8 +653,9 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
     const float w_off = norm_offset_of(n);
     const void *next_norm = fused && next && next->spec.block == IFA_BLOCK_SANDWICH ? next->T(IFA_LT_NORM1).data : nullptr;
     *next_h_ready = next_norm != nullptr;
-    // steps whose products read bfloat16 rows: the norms leave them so (n->h16), but where a mixture of experts reads the rows itself
+    // steps whose products read bfloat16 rows: the norms leave them so (n->h16), but where a mixture of experts needs them in 32 bits
     const bool in16 = fused && norms_leave_h16(n, T);
+    const bool moe16 = in16 && moe && ifa_moe_gated_reads_bf16(T, (int)W, sp.x_ff, sp.x_top, c.ops32, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data);
     if (in16) { const int r = ensure_halfs(m, n->h16, n->h16_cap, T * W); if (r) return r; }
     const bf16_t *h16 = in16 ? n->h16 : nullptr;
     // x += norm_after(sub); h = norm_before(x) for whatever comes next
@@ -683,13 +684,18 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
         if ((rc = ifa_qk_rope_store_f32(n->proj + L.c_aq, NI, H, own ? n->proj + L.c_ak : nullptr, NI, own ? n->proj + L.c_av : nullptr, NI, G, D, DV,
                                         L.T(IFA_LT_A_Q_NORM).data, own ? L.T(IFA_LT_A_K_NORM).data : nullptr, c.eps, sp.a_rot_dims, L.freq, n->seqs_dev, n->row_seq_dev, T,
                                         slots, KV.o_k, KV.o_v, s))) return rc;
-        if ((rc = ifa_attention_kv_f32(n->proj + L.c_aq, NI, H, G, D, DV, sp.a_scale, sp.a_window, sp.a_keep_first, sp.a_sink, sp.a_sink_score, n->seqs_dev,
-                                       n->row_seq_dev, T, slots, KV.o_k, KV.o_v, n->m1, OV, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min,
-                                       c.max_ctx, ws.p, ws.bytes, s))) return rc;
-        if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, OV, n->m1, OV, T, nullptr, nullptr, 1.0f, 0, n->m2, W))) return rc;
+        bf16_t *out16 = nullptr;          // the attention's output as the output product reads it
+        bool left16 = false;
+        if (takes_a16(n, OV, T) && OV % 64 == 0) { if ((rc = ensure_a16(m, T, OV))) return rc; out16 = n->a16; }
+        if ((rc = ifa_attention_kv_to_bf16(n->proj + L.c_aq, NI, H, G, D, DV, sp.a_scale, sp.a_window, sp.a_keep_first, sp.a_sink, sp.a_sink_score, n->seqs_dev,
+                                           n->row_seq_dev, T, slots, KV.o_k, KV.o_v, n->m1, OV, out16, OV, &left16, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min,
+                                           c.max_ctx, ws.p, ws.bytes, s))) return rc;
+        if (left16) rc = linear_in(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, OV, nullptr, out16, T, nullptr, n->m2, W);
+        else rc = linear(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, OV, n->m1, OV, T, nullptr, nullptr, 1.0f, 0, n->m2, W);
+        if (rc) return rc;
     }
-    if ((rc = close_sub(n->m2, L.T(IFA_LT_NORM1B).data, any_ffn ? L.T(IFA_LT_NORM2).data : next_norm, in16 && !(any_ffn && moe)))) return rc;
-    if (any_ffn && moe) h16 = nullptr;
+    if ((rc = close_sub(n->m2, L.T(IFA_LT_NORM1B).data, any_ffn ? L.T(IFA_LT_NORM2).data : next_norm, in16 && !(any_ffn && moe && !moe16)))) return rc;
+    if (any_ffn && moe && !moe16) h16 = nullptr;
     if (!any_ffn) return IFA_OK;
     const size_t N2 = L.n_in2;
     if (sp.ffn_kind == IFA_FFN_RELU2) {      // the square of relu in the epilogue of the up-projection
@@ -718,8 +724,11 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
         if ((rc = linear_in(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2))) return rc;
         // the router's logits (bias added by the product) are columns of the second product; the chosen experts read norm2's output
         if ((rc = ifa_moe_route_top_f32(n->proj + L.c2_router, N2, T, sp.x_experts, sp.x_top, nullptr, n->moe_idx, n->moe_wgt, s))) return rc;
-        if ((rc = ifa_moe_experts_gated_f32(n->h, W, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data, n->moe_idx, n->moe_wgt,
-                                            c.ops32, n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, s))) return rc;
+        rc = moe16 ? ifa_moe_experts_gated_bf16(n->h16, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data, n->moe_idx, n->moe_wgt, n->moe_ws,
+                                                n->moe_ws_bytes, n->m2, W, 0, s)
+                   : ifa_moe_experts_gated_f32(n->h, W, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data, n->moe_idx, n->moe_wgt, c.ops32,
+                                               n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, s);
+        if (rc) return rc;
         if (sp.x_shared_ff > 0) {      // the shared expert: its gate sigmoid(w_sg . h) multiplies the activations in front of the down-projection
             const size_t SF = (size_t)sp.x_shared_ff;
             if ((rc = glu_down(m, false, 0, 0.0f, n->proj + L.c2_shg, N2, SF, n->proj + L.c2_sg, N2, (const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, W, T, nullptr, nullptr, 1, n->m2))) return rc;
@@ -965,6 +974,80 @@ int run_parallel_row(ifa_model *m, LLayer &L, bool *done)
     return ifa_row_out(O, s);
 }
 
+// the gated delta rule of a GATED_DELTA layer over T rows: short convolution, gates, recurrence; the state's outputs in n->m2
+int run_delta_mixer(ifa_model *m, LLayer &L, size_t T, int nseq)
+{
+    LayeredNet *n = m->lay;
+    const ifa_layer_spec &sp = L.spec;
+    const size_t NI = L.n_in;
+    ifa_stream s = (ifa_stream)m->stream;
+    void *const *slots = (void *const *)n->slot_base_dev;
+    int rc;
+    const size_t QK = (size_t)sp.d_kv_heads * sp.d_dim, DV = (size_t)sp.d_heads * sp.d_vdim, C = (size_t)L.conv_ch;
+    if ((rc = ifa_shortconv_silu_f32(n->proj + L.c_dq, NI, (int)C, sp.d_conv, L.w_conv, n->seqs_dev, n->row_seq_dev, T, slots, L.o_conv, (int)(2 * QK),
+                                     sp.d_dim, 1e-6f, (int)QK, 1.0f / sqrtf((float)sp.d_dim), n->m1, C, s))) return rc;
+    if ((rc = ifa_shortconv_tail_f32(n->proj + L.c_dq, NI, (int)C, sp.d_conv, n->seqs_dev, nseq, slots, L.o_conv, s))) return rc;
+    if ((rc = ifa_delta_gates_f32(n->proj + L.c_db, NI, n->proj + L.c_da, NI, sp.d_heads, T, L.T(IFA_LT_D_ALOG).data, L.T(IFA_LT_D_DTBIAS).data,
+                                  n->beta, n->decay, s))) return rc;
+    if ((rc = run_state(m, 1, n->m1, C, n->m1 + QK, C, n->m1 + 2 * QK, C, sp.d_heads, sp.d_kv_heads, sp.d_dim, sp.d_vdim, nullptr, n->decay,
+                        n->beta, nseq, L.o_rec, n->m2, DV))) return rc;
+    return IFA_OK;
+}
+
+// A PARALLEL block of a prompt whose products read bfloat16 rows: x += ls1 (s0 W0 a0 + s1 W1 a1) + ls2 (W2 a2 + b2) as ONE product over the mixers' and the feed-forward's outputs side by
+// side in n->a16, where their producers leave them rounded (before: a product each, every operand written in 32 bits and rounded by a launch of its own: 17 launches a layer, now 11).
+int run_parallel_prompt(ifa_model *m, LLayer &L, size_t T, int nseq, bool *done)
+{
+    LayeredNet *n = m->lay;
+    const ifa_layered_config &c = n->cfg;
+    const ifa_layer_spec &sp = L.spec;
+    const size_t W = (size_t)c.width, NI = L.n_in, F = (size_t)std::max(sp.ffn, 0);
+    ifa_stream s = (ifa_stream)m->stream;
+    void *const *slots = (void *const *)n->slot_base_dev;
+    const bool lin = sp.mixer == IFA_MIX_WINDOW_LINEAR;
+    const size_t AQ = lin ? (size_t)sp.a_heads * sp.a_dim : 0, MV = lin ? (size_t)sp.l_heads * sp.l_vdim : (size_t)sp.d_heads * sp.d_vdim;
+    *done = takes_a16(n, W, T) && (!AQ || takes_a16(n, AQ, T)) && takes_a16(n, MV, T) && (!F || takes_a16(n, F, T)) && W <= 8192;
+    if (!*done) return IFA_OK;
+    const size_t at1 = AQ ? a16_stride(AQ) : 0, at2 = at1 + a16_stride(MV), ld = at2 + (F ? a16_stride(F) : 0), ldw = a16_stride(W);
+    const void *ls1 = L.T(IFA_LT_LS1).data;
+    int rc;
+    if ((rc = ensure_halfs(m, n->h16, n->h16_cap, T * ldw)) || (rc = ensure_halfs(m, n->a16, n->a16_cap, T * ld))) return rc;
+    if (!ifa_layernorm_to_bf16(1, n->x, W, T, W, L.T(IFA_LT_NORM1).data, c.eps, n->h16, ldw, ldw, s)
+        && ((rc = ifa_layernorm_f32(1, n->x, W, T, W, L.T(IFA_LT_NORM1).data, c.eps, n->h, W, s)) || (rc = ifa_rows_to_bf16(n->h, W, T, W, n->h16, ldw, s)))) return rc;
+    IFA_LAUNCH_CHECK();
+    const int silu0 = lin ? (int)L.c_lq : 0, silu1 = lin ? (int)L.c_lg : 0;
+    rc = F ? ifa_linear_bf16_glu(L.w_in, NI, W, n->h16, ldw, T, L.b_in, n->proj, NI, silu0, silu1, L.c_fg, F, 1, 0.0f, n->a16 + at2, ld, s)
+           : ifa_linear_bf16_both(L.w_in, NI, W, n->h16, ldw, T, L.b_in, nullptr, 1.0f, 0, 0, n->proj, nullptr, NI, silu0, silu1, s);
+    if (rc) return rc;
+    // o -> the mixer's part of n->a16
+    auto gated_norm = [&](int group, const void *w, size_t c_gate, int act) -> int {
+        if (ifa_gated_groupnorm_to_bf16(n->m2, MV, T, (int)MV, group, w, group, n->proj + c_gate, NI, act, c.eps, n->a16 + at1, at2 - at1, ld, s)) { IFA_LAUNCH_CHECK(); return IFA_OK; }
+        int r = ifa_gated_groupnorm_f32(n->m2, MV, T, (int)MV, group, w, group, n->proj + c_gate, NI, act, c.eps, n->m2, MV, s);
+        return r ? r : ifa_rows_to_bf16_part(n->m2, MV, T, MV, n->a16 + at1, at2 - at1, ld, s);
+    };
+    if (lin) {
+        const Scratch ws = attn_scratch(n, sp.a_dim, sp.a_dim);
+        bool left16 = false;
+        if ((rc = ifa_kv_store_f32(n->proj + L.c_ak, NI, n->proj + L.c_ak, NI, sp.a_kv_heads, sp.a_dim, 1, c.eps, n->seqs_dev, n->row_seq_dev, T, slots, L.o_k, L.o_v, s))) return rc;
+        if ((rc = ifa_attention_window_to_bf16(n->proj + L.c_aq, NI, sp.a_heads, sp.a_kv_heads, sp.a_dim, 1, c.eps, sp.a_scale, sp.a_softcap, sp.a_window, sp.a_keep_first,
+                                               L.T(IFA_LT_A_REL).data, L.bucket_of, sp.a_buckets, L.T(IFA_LT_A_SINK).data, n->seqs_dev, n->row_seq_dev, T, slots, L.o_k, L.o_v, n->m1, AQ,
+                                               AQ == at1 ? n->a16 : nullptr, ld, &left16, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, ws.p, ws.bytes, s))) return rc;
+        if (!left16 && (rc = ifa_rows_to_bf16_part(n->m1, AQ, T, AQ, n->a16, at1, ld, s))) return rc;
+        if ((rc = run_state(m, 0, n->proj + L.c_lq, NI, n->proj + L.c_lk, NI, n->proj + L.c_lv, NI, sp.l_heads, sp.l_heads, sp.l_dim, sp.l_vdim, L.T(IFA_LT_L_DECAY).data, nullptr, nullptr,
+                            nseq, L.o_lin, n->m2, MV))) return rc;
+        if ((rc = gated_norm((int)MV, L.T(IFA_LT_L_NORM).data, L.c_lg, 0))) return rc;
+    } else {
+        if ((rc = run_delta_mixer(m, L, T, nseq))) return rc;
+        if ((rc = gated_norm(sp.d_vdim, L.T(IFA_LT_D_NORM).data, L.c_dg, 1))) return rc;
+    }
+    IfaSumPart parts[IFA_SUM_PARTS];
+    int np = 0;
+    if (lin) parts[np++] = {L.T(IFA_LT_A_O).data, AQ, ls1, nullptr, sp.a_out_scale};
+    parts[np++] = {L.T(lin ? IFA_LT_L_O : IFA_LT_D_O).data, MV, ls1, nullptr, lin ? sp.l_out_scale : 1.0f};
+    if (F) parts[np++] = {L.T(IFA_LT_FFN_DOWN).data, F, L.T(IFA_LT_LS2).data, L.T(IFA_LT_FFN_DOWN_B).data, 1.0f};
+    return ifa_linear_bf16_sum(parts, np, W, n->a16, ld, T, n->x, W, s);
+}
+
 // the layers of one step over T rows / nseq sequences whose tables are already on the device; leaves the residual in n->x
 int run_layers(ifa_model *m, size_t T, int nseq)
 {
@@ -1040,6 +1123,13 @@ int run_layers(ifa_model *m, size_t T, int nseq)
                 continue;
             }
         }
+        bool done = false;
+        if ((rc = run_parallel_prompt(m, L, T, nseq, &done))) return rc;
+        if (done) {
+            if (n->opt_tap_layers && n->taps && T <= n->taps_rows)
+                IFA_HIP_CHECK(hipMemcpyAsync(n->taps + ri * n->taps_rows * W, n->x, T * W * 4, hipMemcpyDeviceToDevice, m->stream));
+            continue;
+        }
         const bf16_t *ls1 = (const bf16_t *)L.T(IFA_LT_LS1).data;
         const size_t NI = L.n_in;
         // (the linear attention's q | k | v leave the product through SiLU: contiguous columns [c_lq, c_lg))
@@ -1073,14 +1163,8 @@ int run_layers(ifa_model *m, size_t T, int nseq)
             if ((rc = ifa_gated_groupnorm_f32(n->m2, LV, T, (int)LV, (int)LV, L.T(IFA_LT_L_NORM).data, (int)LV, n->proj + L.c_lg, NI, 0, c.eps, n->m2, LV, s))) return rc;
             if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_L_O).data, W, LV, n->m2, LV, T, nullptr, ls1, sp.l_out_scale, 1, n->x, W))) return rc;
         } else {
-            const size_t QK = (size_t)sp.d_kv_heads * sp.d_dim, DV = (size_t)sp.d_heads * sp.d_vdim, C = (size_t)L.conv_ch;
-            if ((rc = ifa_shortconv_silu_f32(n->proj + L.c_dq, NI, (int)C, sp.d_conv, L.w_conv, n->seqs_dev, n->row_seq_dev, T, slots, L.o_conv, (int)(2 * QK),
-                                             sp.d_dim, 1e-6f, (int)QK, 1.0f / sqrtf((float)sp.d_dim), n->m1, C, s))) return rc;
-            if ((rc = ifa_shortconv_tail_f32(n->proj + L.c_dq, NI, (int)C, sp.d_conv, n->seqs_dev, nseq, slots, L.o_conv, s))) return rc;
-            if ((rc = ifa_delta_gates_f32(n->proj + L.c_db, NI, n->proj + L.c_da, NI, sp.d_heads, T, L.T(IFA_LT_D_ALOG).data, L.T(IFA_LT_D_DTBIAS).data,
-                                          n->beta, n->decay, s))) return rc;
-            if ((rc = run_state(m, 1, n->m1, C, n->m1 + QK, C, n->m1 + 2 * QK, C, sp.d_heads, sp.d_kv_heads, sp.d_dim, sp.d_vdim, nullptr, n->decay,
-                                n->beta, nseq, L.o_rec, n->m2, DV))) return rc;
+            const size_t DV = (size_t)sp.d_heads * sp.d_vdim;
+            if ((rc = run_delta_mixer(m, L, T, nseq))) return rc;
             if ((rc = ifa_gated_groupnorm_f32(n->m2, DV, T, (int)DV, sp.d_vdim, L.T(IFA_LT_D_NORM).data, sp.d_vdim, n->proj + L.c_dg, NI, 1, c.eps, n->m2, DV, s))) return rc;
             if ((rc = linear(m, (const bf16_t *)L.T(IFA_LT_D_O).data, W, DV, n->m2, DV, T, nullptr, ls1, 1.0f, 1, n->x, W))) return rc;
         }

@@ -41,6 +41,8 @@ struct LinArgs {
     int act_kind;                              // every output after the bias passes 1: the exact (erf) GELU, 2: the square of relu
     // (k_lin_tile, GLU) columns [glu_c0, glu_c0 + 2 glu_f) are gate | up: instead of them G16[t][c] = act(gate[c]) up[c] in bfloat16, glu_w columns (whole 64s, zero beyond glu_f)
     bf16_t *G16; int ldg, glu_c0, glu_f, glu_w, glu_kind; float glu_limit;
+    // (k_lin_tile, SUM) several products into the same columns: A's rows hold their operands side by side, each padded to whole steps; W, K, mul, bias, alpha of each here
+    struct Part { const bf16_t *W, *mul, *bias; int K, steps; float alpha; } part[IFA_SUM_PARTS];
 };
 
 __device__ __forceinline__ void lin_store(const LinArgs &P, int t, int n, float acc)
@@ -176,11 +178,14 @@ typedef const __attribute__((address_space(1))) void lt_glb_t;
 // exchange between a wave's rows of 16 lanes brings the two together and the activation is formed here and rounded once (the same values as k_glu_to_bf16's).  The 32-bit gate | up
 // rows were written and read again by a launch of their own: 2048 rows of width 2048, 11264 of 19968 columns
 // gate | up, 237 + 23 us -> 243; 601 rows of width 1024 31.6 + 7.4 -> 32.
-constexpr int LT_GROUPED = 1, LT_GLU = 2;
+// SUM: the parts of a sum of products one after the other in ONE pass over K: their requests run on without a break, the tile's rows of C are read and written once, and the launches
+// but one go.  At a part's last step its columns' scales and biases take it from the step's accumulators into the sum.  (22 products of
+// a Gelarax prompt in 8 launches: 2048 rows of width 2048 1268 -> 1202 us, 601 of width 1024 312 -> 309, and 14 launches less.)
+constexpr int LT_GROUPED = 1, LT_GLU = 2, LT_SUM = 4;
 template <int BM, int BN, int NB, int MODE>
 __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_tile(LinArgs P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
 {
-    constexpr bool GROUPED = MODE & LT_GROUPED, GLU = MODE & LT_GLU;
+    constexpr bool GROUPED = MODE & LT_GROUPED, GLU = MODE & LT_GLU, SUM = MODE & LT_SUM;
     constexpr int WAVES = BM == 32 ? 1 : 4, TA = BM == 32 ? 1 : BM / 64, TB = BM == 32 ? 1 : BN / 64, AI = BM / (8 * WAVES), WI = BN / (8 * WAVES), ROWB = 2 * LT_BK, STEPB = (BM + BN) * ROWB;
     __shared__ __attribute__((aligned(16))) char smem[NB * STEPB];          // [NB steps][BM rows of A, BN rows of W]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5, wm = wave & 1, wn = wave >> 1;          // (BM = 32: one wave, one tile)
@@ -219,17 +224,34 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
     for (int j = 0; j < WI; j++) {
         const int row = (wave * WI + j) * 8 + (lane >> 3), c = (lane & 7) ^ swz(row);
         const int wr = glu ? P.glu_c0 + ((row & 16) ? P.glu_f : 0) + min(o0 + 16 * (row >> 5) + (row & 15), P.glu_f - 1) : min(n0 + row, n_end - 1);
-        wsrc[j] = Wg + (size_t)wr * P.K + c * 8;
-        wlim[j] = P.K - 8 - c * 8;
+        const int K = SUM ? P.part[0].K : P.K;
+        wsrc[j] = (SUM ? P.part[0].W : Wg) + (size_t)wr * K + c * 8;
+        wlim[j] = K - 8 - c * 8;
     }
+    // (SUM) the part that the next requested step belongs to, from its first step to the one behind its last; likewise for the next step of products
+    int q_part = 0, q_from = 0, q_to = SUM ? P.part[0].steps : 0, c_part = 0, c_to = q_to;
+    auto enter = [&](int step) {
+        if constexpr (SUM) {
+            if (step != q_to) return;
+            q_part++; q_from = q_to; q_to += P.part[q_part].steps;
+            const int K = P.part[q_part].K;
+#pragma unroll
+            for (int j = 0; j < WI; j++) {
+                const int row = (wave * WI + j) * 8 + (lane >> 3), c = (lane & 7) ^ swz(row);
+                wsrc[j] = P.part[q_part].W + (size_t)min(n0 + row, n_end - 1) * K + c * 8;
+                wlim[j] = K - 8 - c * 8;
+            }
+        }
+    };
     const int nsteps = lda16 / LT_BK;
     auto stage_a = [&](int step, char *to, int j) {
         __builtin_amdgcn_global_load_lds((lt_glb_t *)(asrc[j] + step * LT_BK), (lt_lds_t *)(to + (wave * AI + j) * 1024), 16, 0, 0);
     };
     auto stage_w = [&](int step, char *to, int j) {
-        __builtin_amdgcn_global_load_lds((lt_glb_t *)(wsrc[j] + min(step * LT_BK, wlim[j])), (lt_lds_t *)(to + BM * ROWB + (wave * WI + j) * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((lt_glb_t *)(wsrc[j] + min((step - q_from) * LT_BK, wlim[j])), (lt_lds_t *)(to + BM * ROWB + (wave * WI + j) * 1024), 16, 0, 0);
     };
     auto stage = [&](int step, char *to) {
+        enter(step);
 #pragma unroll
         for (int j = 0; j < AI; j++) stage_a(step, to, j);
 #pragma unroll
@@ -243,6 +265,42 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
         for (int b = 0; b < TB; b++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
+    f32x16v tot[SUM ? TA : 1][SUM ? TB : 1];
+    if constexpr (SUM) {
+#pragma unroll
+        for (int a = 0; a < TA; a++)
+#pragma unroll
+            for (int b = 0; b < TB; b++) tot[a][b] = acc[a][b];
+    }
+    // (asked for here: a request behind those of the steps would wait for all of them)
+    float p_mul[SUM ? IFA_SUM_PARTS : 1][TB], p_bias[SUM ? IFA_SUM_PARTS : 1][TB];
+    if constexpr (SUM) {
+#pragma unroll
+        for (int k = 0; k < IFA_SUM_PARTS; k++)
+#pragma unroll
+            for (int b = 0; b < TB; b++) {
+                const auto &part = P.part[k];
+                const int n = min(n0 + wn * (BN / 2) + 32 * b + i, P.N - 1);
+                p_bias[k][b] = part.bias ? bf2f(part.bias[n]) : 0.0f; p_mul[k][b] = part.alpha * (part.mul ? bf2f(part.mul[n]) : 1.0f);
+            }
+    }
+    auto close = [&](int step) {          // (behind the step's products)
+        if constexpr (SUM) {
+            if (step + 1 != c_to) return;
+#pragma unroll
+            for (int b = 0; b < TB; b++) {
+                float bv = p_bias[0][b], mv = p_mul[0][b];
+#pragma unroll
+                for (int k = 1; k < IFA_SUM_PARTS; k++) if (c_part == k) { bv = p_bias[k][b]; mv = p_mul[k][b]; }
+#pragma unroll
+                for (int a = 0; a < TA; a++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) { tot[a][b][r] += (acc[a][b][r] + bv) * mv; acc[a][b][r] = 0.0f; }
+            }
+            c_part++;
+            if (step + 1 < nsteps) c_to += P.part[c_part].steps;
+        }
+    };
     bf16x8v af[2][TA], wf[2][TB];
     auto frags = [&](const char *base, int ks, bf16x8v (&fa)[TA], bf16x8v (&fw)[TB]) {
         const int so = ((2 * ks) ^ lc) << 4;
@@ -272,6 +330,7 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
             __syncthreads();
             frags(nxt, 0, af[0], wf[0]);
             mma(af[1], wf[1]);
+            close(step);
         }
         const char *cur = smem + ((nsteps - 1) & 1) * STEPB;
 #pragma unroll
@@ -280,6 +339,7 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
             mma(af[ks & 1], wf[ks & 1]);
         }
         mma(af[1], wf[1]);
+        close(nsteps - 1);
     } else {
         static_assert(TA == 1 && TB == 1, "a wave reads one tile of each operand");
         const unsigned lds0 = (unsigned)(uintptr_t)(lt_lds_t *)smem;
@@ -296,6 +356,7 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
             asm volatile("" ::: "memory");
             char *to = smem + (j == 0 ? NB - 1 : j - 1) * STEPB;
             if constexpr (decltype(more)::value && BM > 32) stage(step + NB - 1, to);
+            if constexpr (decltype(more)::value && BM == 32) enter(step + NB - 1);
             const unsigned oa = j * STEPB + a_off, ow = j * STEPB + w_off;
             bf16x8v fa[4], fw[4];
             asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %4, %12\n\tds_read_b128 %1, %9\n\tds_read_b128 %5, %13\n\tds_read_b128 %2, %10\n\tds_read_b128 %6, %14\n\t"
@@ -313,6 +374,7 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
+            close(step);
         };
         // (at least NB steps)
 #pragma unroll
@@ -337,6 +399,21 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
                 }
         }
     };
+    if constexpr (SUM) {
+#pragma unroll
+        for (int b = 0; b < TB; b++) {
+            const int n = n0 + wn * (BN / 2) + 32 * b + i;
+            if (n >= n_end) continue;
+#pragma unroll
+            for (int a = 0; a < TA; a++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int t = t0 + wm * (BM / 2) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
+                    if (t < t_end) P.C[(size_t)t * P.ldc + n] += tot[a][b][r];
+                }
+        }
+        return;
+    }
     if constexpr (GLU) {
         if (glu) {
             // lanes of a first row of 16 hold gates, those of a second one ups: after the exchange of a second row's r with a first row's r + 8 both hold both, rows r here, r + 8 there
@@ -425,12 +502,12 @@ int lin_grouped_dispatch(const LinArgs &P, const bf16_t *a, size_t lda, size_t m
     return launch_lin_tile<64, 64, 4, MODE>(P, a, lda, max_tiles, s);
 }
 
-// rows of 32-bit values to bfloat16, zero up to ldy (a multiple of 8)
-__global__ void __launch_bounds__(256) k_rows_to_bf16(const float *__restrict__ x, size_t ldx, int cols, bf16_t *__restrict__ y, int ldy, int vec)
+// rows of 32-bit values to bfloat16, zero up to `width` columns (a multiple of 8) of rows of ldy
+__global__ void __launch_bounds__(256) k_rows_to_bf16(const float *__restrict__ x, size_t ldx, int cols, bf16_t *__restrict__ y, int width, int ldy, int vec)
 {
     const float *xr = x + (size_t)blockIdx.y * ldx;
     const int c = (blockIdx.x * 256 + threadIdx.x) * 8;
-    if (c >= ldy) return;
+    if (c >= width) return;
     float v[8];
     if (vec && c + 8 <= cols) {
         const float4 a = *reinterpret_cast<const float4 *>(xr + c), b = *reinterpret_cast<const float4 *>(xr + c + 4);
@@ -690,18 +767,24 @@ extern "C" int ifa_linear_bf16w(const void *w_bf16, size_t rows, size_t cols, co
                          stream, "ifa_linear_bf16w");
 }
 
-extern "C" int ifa_rows_to_bf16(const void *x_f32, size_t ldx, size_t rows, size_t cols, void *y_bf16, size_t ldy, ifa_stream stream)
+int ifa_rows_to_bf16_part(const void *x_f32, size_t ldx, size_t rows, size_t cols, void *y_bf16, size_t width, size_t ldy, ifa_stream stream)
 {
     IFA_REQUIRE(x_f32 && y_bf16, "ifa_rows_to_bf16: null pointer");
-    IFA_REQUIRE(rows > 0 && rows < 65536u * 16u && cols > 0 && ldx >= cols && ldy >= cols && ldy % 8 == 0 && ldy < (1u << 30) && ((uintptr_t)y_bf16 & 15) == 0, "ifa_rows_to_bf16: bad shape");
+    IFA_REQUIRE(rows > 0 && rows < 65536u * 16u && cols > 0 && ldx >= cols && width >= cols && width % 8 == 0 && ldy >= width && ldy % 8 == 0 && ldy < (1u << 30)
+                && ((uintptr_t)y_bf16 & 15) == 0, "ifa_rows_to_bf16: bad shape");
     const int vec = ldx % 4 == 0 && ((uintptr_t)x_f32 & 15) == 0;
     for (size_t r0 = 0; r0 < rows; r0 += 65535) {
         const size_t n = std::min<size_t>(65535, rows - r0);
-        hipLaunchKernelGGL(k_rows_to_bf16, dim3(ifa_cdiv(ldy / 8, 256), (unsigned)n), dim3(256), 0, ifa_s(stream), (const float *)x_f32 + r0 * ldx, ldx, (int)cols,
-                           (bf16_t *)y_bf16 + r0 * ldy, (int)ldy, vec);
+        hipLaunchKernelGGL(k_rows_to_bf16, dim3(ifa_cdiv(width / 8, 256), (unsigned)n), dim3(256), 0, ifa_s(stream), (const float *)x_f32 + r0 * ldx, ldx, (int)cols,
+                           (bf16_t *)y_bf16 + r0 * ldy, (int)width, (int)ldy, vec);
     }
     IFA_LAUNCH_CHECK();
     return IFA_OK;
+}
+
+extern "C" int ifa_rows_to_bf16(const void *x_f32, size_t ldx, size_t rows, size_t cols, void *y_bf16, size_t ldy, ifa_stream stream)
+{
+    return ifa_rows_to_bf16_part(x_f32, ldx, rows, cols, y_bf16, ldy, ldy, stream);
 }
 
 extern "C" int ifa_linear_bf16_both(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, size_t tokens, const void *bias_bf16, const void *mul_bf16,
@@ -720,6 +803,25 @@ extern "C" int ifa_linear_bf16_both(const void *w_bf16, size_t rows, size_t cols
     hipStream_t s = ifa_s(stream);
     const bf16_t *a = (const bf16_t *)a_bf16;
     return lin_tile_dispatch<0>(P, a, lda, s);
+}
+
+int ifa_linear_bf16_sum(const IfaSumPart *parts, int n_parts, size_t rows, const void *a_bf16, size_t lda, size_t tokens, void *c_f32, size_t ldc, ifa_stream stream)
+{
+    IFA_REQUIRE(parts && a_bf16 && c_f32 && n_parts >= 1 && n_parts <= IFA_SUM_PARTS, "linear_bf16_sum: null pointer or %d parts", n_parts);
+    IFA_REQUIRE(rows > 0 && tokens > 0 && ldc >= rows && rows < (1u << 30) && tokens < (1u << 30) && lda < (1u << 30) && ((uintptr_t)a_bf16 & 15) == 0, "linear_bf16_sum: bad shape");
+    LinArgs P;
+    memset(&P, 0, sizeof(P));
+    P.C = (float *)c_f32; P.T = (int)tokens; P.N = (int)rows; P.ldc = (int)ldc;
+    size_t at = 0;
+    for (int k = 0; k < n_parts; k++) {
+        const IfaSumPart &p = parts[k];
+        IFA_REQUIRE(p.w && ((uintptr_t)p.w & 15) == 0 && p.cols >= (size_t)LT_BK && p.cols % 8 == 0, "linear_bf16_sum: part %d of %zu columns", k, p.cols);
+        P.part[k].W = (const bf16_t *)p.w; P.part[k].mul = (const bf16_t *)p.mul; P.part[k].bias = (const bf16_t *)p.bias; P.part[k].K = (int)p.cols;
+        P.part[k].steps = (int)((p.cols + LT_BK - 1) / LT_BK); P.part[k].alpha = p.alpha;
+        at += (size_t)P.part[k].steps * LT_BK;
+    }
+    IFA_REQUIRE(at == lda, "linear_bf16_sum: parts of %zu columns in rows of %zu", at, lda);
+    return lin_tile_dispatch<LT_SUM>(P, (const bf16_t *)a_bf16, lda, ifa_s(stream));
 }
 
 int ifa_linear_bf16_glu(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,

@@ -448,11 +448,19 @@ size_t ifa_moe_workspace_bytes(size_t rows, int top, int width, int ff, int expe
     return al16(pairs * ff * 4) + al16(pairs * width * 4) + 3 * al16(pairs * 4) + al16(moe_tiles_max(rows, top, experts) * 12) + 16;
 }
 
+// whether gated experts of more than eight rows run over bfloat16 rows (k_lin_tile): sizes and alignment, see moe_experts
+static bool moe_in16(size_t rows, int width, int ff, int top, int ops32, const void *up_bf16, const void *down_bf16)
+{
+    const size_t lda_h = ((size_t)width + 63) & ~(size_t)63, lda_f = ((size_t)ff + 63) & ~(size_t)63;
+    return rows > 8 && !ops32 && width % 8 == 0 && width >= 64 && ff % 8 == 0 && ff >= 64 && width + ff >= 512 && lda_f <= 2 * (size_t)ff && lda_h <= 2 * (size_t)width * top
+           && (((uintptr_t)up_bf16 | (uintptr_t)down_bf16) & 15) == 0;
+}
+
 static int moe_experts(const char *who, int gated, int glu_kind, float limit, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int identity, int top, int act,
                        const void *up_bf16, const void *down_bf16, const int *idx_dev, const void *wgt_f32, int ops32, void *ws, size_t ws_bytes,
-                       void *y_f32, size_t ldy, int accumulate, ifa_stream stream, const RouteSel *sel = nullptr)
+                       void *y_f32, size_t ldy, int accumulate, ifa_stream stream, const RouteSel *sel = nullptr, const void *h_bf16 = nullptr)
 {
-    IFA_REQUIRE(h_f32 && idx_dev && wgt_f32 && ws && y_f32 && (experts == 0 || (up_bf16 && down_bf16)), "%s: null pointer", who);
+    IFA_REQUIRE((h_f32 || h_bf16) && idx_dev && wgt_f32 && ws && y_f32 && (experts == 0 || (up_bf16 && down_bf16)), "%s: null pointer", who);
     IFA_REQUIRE(rows > 0 && rows < 65536 && width > 0 && ff > 0 && experts >= 0 && experts <= 4096 && identity >= 0 && top >= 1 && top <= experts + identity && act == 0
                 && ldh >= (size_t)width && ldy >= (size_t)width, "%s: bad shape", who);
     // gated experts: the first product leaves gate | up (2 ff values per pair) in front of the activations
@@ -496,8 +504,8 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
     // us before / now: 128 x 128 18.7 / 21.6, 256 x 128 20.6 / 21.6, 256 x 256 22.6 / 21.6).  Row tiles of 128 where an expert has several on average and they still fill the
     // chip (4000 pairs of 8 experts: 1408 x 2048 288 -> 197 us; 520 x 136 52, 46 with tiles of 64, 59 with tiles of 128)
     const size_t lda_h = ((size_t)width + 63) & ~(size_t)63, lda_f = ((size_t)ff + 63) & ~(size_t)63;
-    const bool in16 = gated && !ops32 && width % 8 == 0 && width >= 64 && ff % 8 == 0 && ff >= 64 && width + ff >= 512 && lda_f <= 2 * (size_t)ff && lda_h <= 2 * (size_t)width * top
-                      && (((uintptr_t)up_bf16 | (uintptr_t)down_bf16) & 15) == 0;
+    const bool in16 = gated && moe_in16(rows, width, ff, top, ops32, up_bf16, down_bf16);
+    IFA_REQUIRE(in16 || h_f32, "%s: rows in bfloat16 where the sizes need 32 bits", who);
     const int tile_rows = in16 && pairs >= (size_t)256 * experts && pairs / 128 * (((size_t)width + 127) / 128) >= 256 ? 128 : 64;
     const size_t max_tiles = (pairs + tile_rows - 1) / tile_rows + (size_t)experts;
     IFA_REQUIRE(max_tiles < 65536, "%s: %zu rows x %d choices exceed one step", who, rows, top);
@@ -507,8 +515,8 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
     int rc;
     if (in16) {
         bf16_t *h16 = (bf16_t *)yp, *a16 = (bf16_t *)actb;
-        if ((rc = ifa_rows_to_bf16(h_f32, ldh, rows, (size_t)width, h16, lda_h, stream))) return rc;
-        if ((rc = ifa_linear_bf16_grouped(up_bf16, (size_t)2 * ff, (size_t)width, h16, lda_h, a_rows, tile_map, n_tiles, max_tiles, tile_rows, nullptr, nullptr, lda_f, glu_kind, limit, a16, stream))) return rc;
+        if (!h_bf16 && (rc = ifa_rows_to_bf16(h_f32, ldh, rows, (size_t)width, h16, lda_h, stream))) return rc;
+        if ((rc = ifa_linear_bf16_grouped(up_bf16, (size_t)2 * ff, (size_t)width, h_bf16 ? h_bf16 : h16, lda_h, a_rows, tile_map, n_tiles, max_tiles, tile_rows, nullptr, nullptr, lda_f, glu_kind, limit, a16, stream))) return rc;
         if ((rc = ifa_linear_bf16_grouped(down_bf16, (size_t)width, (size_t)ff, a16, lda_f, nullptr, tile_map, n_tiles, max_tiles, tile_rows, w_sorted, yp, (size_t)width, 0, 0.0f, nullptr, stream))) return rc;
     } else if (gated) {
         if ((rc = ifa_linear_bf16w_grouped(up_bf16, (size_t)2 * ff, (size_t)width, experts, h_f32, ldh, a_rows, tile_map, n_tiles, max_tiles, nullptr, 0, ops32, gub, (size_t)2 * ff, stream))) return rc;
@@ -562,3 +570,16 @@ int ifa_moe_experts_routed_rows_f32(int score_kind, int renorm, float renorm_eps
 }
 
 } // extern "C"
+
+bool ifa_moe_gated_reads_bf16(size_t rows, int width, int ff, int top, int ops32, const void *gate_up_bf16, const void *down_bf16)
+{
+    return width % 64 == 0 && moe_in16(rows, width, ff, top, ops32, gate_up_bf16, down_bf16);
+}
+
+int ifa_moe_experts_gated_bf16(const void *h_bf16, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16, const void *down_bf16, const int *idx_dev,
+                               const void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream)
+{
+    IFA_REQUIRE(h_bf16 && ((uintptr_t)h_bf16 & 15) == 0 && experts > 0 && ifa_moe_gated_reads_bf16(rows, width, ff, top, 0, gate_up_bf16, down_bf16), "moe_experts_gated_bf16: bad shape");
+    return moe_experts("moe_experts_gated_bf16", 1, 0, 0.0f, nullptr, (size_t)width, rows, width, ff, experts, 0, top, 0, gate_up_bf16, down_bf16, idx_dev, wgt_f32, 0, ws, ws_bytes, y_f32,
+                       ldy, accumulate, stream, nullptr, h_bf16);
+}

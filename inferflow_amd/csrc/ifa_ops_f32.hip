@@ -10,6 +10,7 @@ using namespace ifa32;
 namespace {
 
 typedef __bf16 bf16x8o __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4o __attribute__((ext_vector_type(4)));
 
 // x[t][c] = embed[token_t][c] + pe(pos_t)[c];  pe[2i] = sin(p w_i), pe[2i + 1] = cos(p w_i), w_i = base^(-2i / width).
 // The angle of position p reaches hundreds of radians where one fp32 ulp is already 1e-4: it is formed in double.
@@ -47,6 +48,47 @@ __global__ void __launch_bounds__(256) k_norm_f32(int kind, const float *__restr
     for (int c = threadIdx.x; c < cols; c += blockDim.x) {
         const float v = (xr[c] - mean) * rinv;
         yr[c] = w ? v * bf2f(w[c]) : v;
+    }
+}
+
+// The same into bfloat16 rows, zero up to `width` columns, the row in registers: every thread holds PIECES pieces of four values and requests row and weight before the first sum.
+// (Read three times from the caches, written in 32 bits and rounded by a launch of its own: 2048 rows of 2048 13.2 + 5.6 -> 7.8 us, 601 of 1024 6.3 + 5.0 -> 4.5.)
+template <int PIECES>
+__global__ void __launch_bounds__(256) k_norm_to_bf16(int kind, const float *__restrict__ x, size_t ldx, int cols, const bf16_t *__restrict__ w, float eps, bf16_t *__restrict__ y,
+                                                      int width, size_t ldy)
+{
+    __shared__ float red[17];
+    const float *xr = x + (size_t)blockIdx.x * ldx;
+    bf16_t *yr = y + (size_t)blockIdx.x * ldy;
+    float v[PIECES][4], s = 0.0f, q = 0.0f;
+    uint2 wv[PIECES];
+#pragma unroll
+    for (int p = 0; p < PIECES; p++) {
+        const int c = 4 * (threadIdx.x + p * 256);
+        const float4 a = c < cols ? *reinterpret_cast<const float4 *>(xr + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        wv[p] = w && c < cols ? *reinterpret_cast<const uint2 *>(w + c) : make_uint2(0x3F803F80u, 0x3F803F80u);
+        v[p][0] = a.x; v[p][1] = a.y; v[p][2] = a.z; v[p][3] = a.w;
+        s += (a.x + a.y) + (a.z + a.w);
+    }
+    const float mean = kind == 1 ? block_sum(s, red) / (float)cols : 0.0f;
+#pragma unroll
+    for (int p = 0; p < PIECES; p++)
+        if (4 * (threadIdx.x + p * 256) < (unsigned)cols) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) { v[p][e] -= mean; q = fmaf(v[p][e], v[p][e], q); }
+        }
+    const float rinv = 1.0f / sqrtf(block_sum(q, red) / (float)cols + eps);
+#pragma unroll
+    for (int p = 0; p < PIECES; p++) {
+        const int c = 4 * (threadIdx.x + p * 256);
+        if (c >= width) continue;
+        bf16x4o h;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t u = e < 2 ? wv[p].x : wv[p].y;
+            h[e] = (__bf16)(c < cols ? v[p][e] * rinv * __uint_as_float((e & 1) ? (u & 0xFFFF0000u) : (u << 16)) : 0.0f);
+        }
+        *reinterpret_cast<bf16x4o *>(yr + c) = h;
     }
 }
 
@@ -608,6 +650,17 @@ int ifa_norm_add_norm_f32(void *x_f32, size_t ldx, size_t rows, size_t cols, con
 }
 
 } // extern "C"
+
+bool ifa_layernorm_to_bf16(int kind, const void *x_f32, size_t ldx, size_t rows, size_t cols, const void *w_bf16, float eps, void *y_bf16, size_t width, size_t ldy, ifa_stream stream)
+{
+    if (!x_f32 || !y_bf16 || (kind != 0 && kind != 1) || rows == 0 || rows >= (1u << 31) || cols == 0 || cols % 4 || ldx < cols || ldx % 4 || width < cols || width % 8 || width > 8192
+        || ldy < width || ldy % 8 || ((uintptr_t)x_f32 & 15) || ((uintptr_t)y_bf16 & 15) || ((uintptr_t)w_bf16 & 7)) return false;
+    const dim3 grid((unsigned)rows);
+#define IFA_NB(P) hipLaunchKernelGGL(k_norm_to_bf16<P>, grid, dim3(256), 0, ifa_s(stream), kind, (const float *)x_f32, ldx, (int)cols, (const bf16_t *)w_bf16, eps, (bf16_t *)y_bf16, (int)width, ldy)
+    if (width <= 1024) IFA_NB(1); else if (width <= 2048) IFA_NB(2); else if (width <= 4096) IFA_NB(4); else IFA_NB(8);
+#undef IFA_NB
+    return true;
+}
 
 int ifa_glu_to_bf16(int kind, float limit, const void *gate_up_f32, size_t ld, size_t rows, size_t cols, const void *row_gate_f32, size_t ldg, void *out_bf16, size_t ldo,
                     ifa_stream stream)

@@ -46,6 +46,33 @@ int ifa_linear_bf16_grouped(const void *w_bf16, size_t rows, size_t cols, const 
 // (whole 64s, zero beyond glu_cols) in their place; the columns before them as ever, any behind them not at all
 int ifa_linear_bf16_glu(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,
                         int silu_col1, size_t glu_col0, size_t glu_cols, int glu_kind, float glu_limit, void *glu_bf16, size_t ldg, ifa_stream stream);
+// C[t][n] += sum over the parts of alpha mul[n] (W[n] . a[t] + bias[n]): a_bf16's rows hold the parts' operands side by side, each zero-padded to whole 64s (lda: their sum);
+// cols: a multiple of 8, 64 and more
+constexpr int IFA_SUM_PARTS = 3;
+struct IfaSumPart { const void *w; size_t cols; const void *mul, *bias; float alpha; };
+int ifa_linear_bf16_sum(const IfaSumPart *parts, int n_parts, size_t rows, const void *a_bf16, size_t lda, size_t tokens, void *c_f32, size_t ldc, ifa_stream stream);
+// ifa_rows_to_bf16 into the first `width` columns (a multiple of 8) of rows of ldy
+int ifa_rows_to_bf16_part(const void *x_f32, size_t ldx, size_t rows, size_t cols, void *y_bf16, size_t width, size_t ldy, ifa_stream stream);
+// Producers that leave what only products read in bfloat16: rows of ldy, zero from the last column up to `width` (both multiples of 8).  The norms: false where the sizes or the
+// alignment don't allow it (nothing launched).
+// ifa_layernorm_f32
+bool ifa_layernorm_to_bf16(int kind, const void *x_f32, size_t ldx, size_t rows, size_t cols, const void *w_bf16, float eps, void *y_bf16, size_t width, size_t ldy, ifa_stream stream);
+// ifa_gated_groupnorm_f32 (w as long as a group or as the row)
+bool ifa_gated_groupnorm_to_bf16(const void *o_f32, size_t ldo, size_t rows, int channels, int group, const void *w_bf16, int wlen, const void *gate_f32, size_t ldg, int gate_act,
+                                 float eps, void *y_bf16, size_t width, size_t ldy, ifa_stream stream);
+// ifa_attention_window_f32 / ifa_attention_kv_f32: *left16 tells whether the output is in out_bf16 (rows of ld16, heads * vdim columns) or, where the step's form writes 32 bits, in out_f32
+int ifa_attention_window_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int norm_q, float eps, float scale, float softcap, int window, int keep_first,
+                                 const void *rel_bf16, const int *bucket_of_dev, int n_buckets, const void *sink_bf16, const void *seqs_dev, const int *row_seq_dev, size_t rows,
+                                 void *const *slot_base_dev, size_t k_off, size_t v_off, void *out_f32, size_t ldo, void *out_bf16, size_t ld16, bool *left16, const void *seqs_host,
+                                 int n_seqs, int tile_min_rows, void *ws_f32, size_t ws_bytes, ifa_stream stream);
+int ifa_attention_kv_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int vdim, float scale, int window, int keep_first, int sink, float sink_score,
+                             const void *seqs_dev, const int *row_seq_dev, size_t rows, void *const *slot_base_dev, size_t k_off, size_t v_off, void *out_f32, size_t ldo,
+                             void *out_bf16, size_t ld16, bool *left16, const void *seqs_host, int n_seqs, int tile_min_rows, int max_keys, void *ws_f32, size_t ws_bytes,
+                             ifa_stream stream);
+// ifa_moe_experts_gated_f32 of more than eight rows that a norm has left in bfloat16 (rows of `width`), where the first tells that the experts' products read them so
+bool ifa_moe_gated_reads_bf16(size_t rows, int width, int ff, int top, int ops32, const void *gate_up_bf16, const void *down_bf16);
+int ifa_moe_experts_gated_bf16(const void *h_bf16, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16, const void *down_bf16, const int *idx_dev,
+                               const void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream);
 // ifa_glu_ex_f32 whose output only products read: bfloat16 rows, zero up to ldo (a multiple of 8; csrc/ifa_ops_f32.hip)
 int ifa_glu_to_bf16(int kind, float limit, const void *gate_up_f32, size_t ld, size_t rows, size_t cols, const void *row_gate_f32, size_t ldg, void *out_bf16, size_t ldo,
                     ifa_stream stream);

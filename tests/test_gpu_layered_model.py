@@ -318,20 +318,26 @@ def test_prompts_with_and_without_the_workspaces_of_tiles_and_chunks(tmp_path, l
     eng.close()
 
 
-@pytest.mark.parametrize("T", [17, 130, 601, 1500, 3100])
-def test_activations_formed_behind_their_product(tmp_path, T):
-    """bfloat16 operands: the gated activations formed in the product's own tiles (every tile size, inner sizes of whole and of broken tiles) and left in bfloat16, against gate | up
-    stored, activated and rounded by launches of their own (a16_min 0): the same sums in the same order, so the same bits"""
+@pytest.mark.parametrize("T,width", [(17, 520), (130, 520), (601, 520), (1500, 520), (3100, 520), (70, 2056), (300, 72), (130, 128)])
+def test_prompts_whose_products_read_bfloat16_rows(tmp_path, T, width):
+    """Activations formed in the product's own tiles, outputs of norms and mixers left in bfloat16, a layer's output products in one pass over their columns -- every tile size, few and many
+    steps, inner sizes that are no whole step, layers without feed-forward, norm groups of a power of two and others, attention heads that leave 32 bits -- against every operand stored in
+    32 bits and rounded on the way into a product of its own (a16_min 0).  Both round the same operands; sums in another order flip such a rounding here and there, which is up to 2^-8 of
+    one element: one layer at a time, since flips in one flip more in the next, up to the noise of all roundings"""
     import inferflow_amd as ia
-    cfg = fx.config([fx.delta_layer(heads=2, kv_heads=1, dim=16, vdim=16, conv=3, ff=ff) for ff in (72, 1032, 0)], width=520, vocab=97)
-    eng = engine_for(tmp_path, cfg, fx.random_weights(cfg, 35), "bfloat16", 3200, 1)
-    toks, out = tokens_for(cfg, T, 36), {}
-    for border in (0, 17):
-        ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"a16_min", border))
-        out[border] = run_whole(eng, toks)[0]
-    eng.close()
-    assert out[17].shape == (T, 97) and np.isfinite(out[17]).all()
-    assert np.array_equal(out[0], out[17])
+    for layer in (fx.delta_layer(heads=4, kv_heads=2, dim=16, vdim=32, conv=3, ff=72),
+                  fx.parallel_layer(heads=2, kv_heads=1, dim=32, window=100, keep_first=0, lin_heads=2, lin_dim=16, lin_vdim=40, ff=1032),
+                  fx.parallel_layer(heads=3, kv_heads=1, dim=24, window=50, keep_first=2, lin_heads=2, lin_dim=16, lin_vdim=48, ff=0),
+                  fx.delta_layer(heads=2, kv_heads=1, dim=16, vdim=40, conv=3, ff=200)):
+        cfg = fx.config([layer], width=width, vocab=97)
+        eng = engine_for(tmp_path, cfg, fx.random_weights(cfg, 35), "bfloat16", 3200, 1)
+        toks, out = tokens_for(cfg, T, 36), {}
+        for border in (0, 17):
+            ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"a16_min", border))
+            out[border] = run_whole(eng, toks)[0]
+        eng.close()
+        assert out[17].shape == (T, 97) and np.isfinite(out[17]).all()
+        assert fx.rel_err(out[17], out[0]).max() < 2.0 ** -8, layer
 
 
 def test_chunked_recurrences_are_switched_off_by_0(tmp_path):
