@@ -156,23 +156,20 @@ __global__ void __launch_bounds__(256) k_lin_mfma(LinArgs P)
     }
 }
 
-// ---- prompts, both operands in bfloat16 already: BM x BN output tiles, K in steps of 64, double-buffered in LDS.  Both operands go from memory to LDS
-// directly (global_load_lds_dwordx4: a wave moves 8 rows x 128 bytes per instruction, a step ahead); both images are [rows][64 halfs] with the eight
+// ---- prompts, both operands in bfloat16 already: BM x BN output tiles, WM x WN waves, K in steps of 64 through NB buffers in LDS.  Both operands go from memory to LDS
+// directly (global_load_lds_dwordx4: a wave moves 8 rows x 128 bytes per instruction, NB - 1 steps ahead); both images are [rows][64 halfs] with the eight
 // 16-byte pieces of row r at slot c ^ ((r >> 1) & 7), so that the fragment reads of 16 consecutive lanes (16 rows, one piece) are free of bank conflicts; the
 // loads write LDS linearly, the permutation sits in their SOURCE addresses.  The step's barrier stands before its last group of products: every wave has read
 // its last fragments by then, and the first fragments of the next buffer land under that group.
 // Workgroups are dealt to the eight XCDs round-robin: the id is remapped so that an XCD works on a compact block of tiles whose operands its L2 shares.
 // A's rows are K rounded up to whole steps long, zero beyond K (what W's requests bring in there -- held inside the row -- does not count).
 constexpr int LT_BK = 64;
-// Up to so many 64 x 64 tiles: 32 x 32 tiles of one wave each, seven steps under way / 64 x 64 tiles, three steps under way.  us with two buffers of 64 x 64, four of 64 x 64,
-// eight of 32 x 32 -- 16 tiles of 4096 columns 30.7, 18.3, 15.4; 64 tiles of 4096 46.0, 19.1, 15.8; 128 of 1024 9.9, 7.1, 6.8; 192 of 1024 10.0, 7.1, 11.3; 400 of 2560
-// 21.7, 18.4, 31.1; 640 of 1024 12.2, 14.2, 26.8; 640 of 4096 50.7, 47.7, 80.9.  (Steps split over two or four groups of waves: 24.0 for 64 tiles of 4096, and other sums.)
-constexpr size_t LT_SMALL = 128, LT_DEEP = 512;
+// Up to so many 64 x 64 tiles: 32 x 32 tiles of one wave each, seven steps under way.  us with two buffers of 64 x 64, four of 64 x 64, eight of 32 x 32 -- 16 tiles of 4096 columns
+// 30.7, 18.3, 15.4; 64 tiles of 4096 46.0, 19.1, 15.8; 128 of 1024 9.9, 7.1, 6.8; 192 of 1024 10.0, 7.1, 11.3.
+constexpr size_t LT_SMALL = 128;
 typedef __attribute__((address_space(3))) void lt_lds_t;
 typedef const __attribute__((address_space(1))) void lt_glb_t;
 
-// NB > 2: NB buffers, a step asked for NB - 1 steps ahead.  For products whose tiles do not fill the chip, which wait for one step after the other (0.4 to 0.7 us a step
-// with two buffers, 0.25 with more: the requests' issue, the fragments' way from LDS and the chain of products).
 // GROUPED: row tiles and matrices from P.tile_map, the rows of A by P.a_rows (null: as they are), each output row times P.row_scale.
 // GLU: column tiles from P.glu_c0 on serve BN / 2 outputs of a gated feed-forward: of 32 columns of such a tile 16 are gates and 16 the ups of the same outputs, so that one
 // exchange between a wave's rows of 16 lanes brings the two together and the activation is formed here and rounded once (the same values as k_glu_to_bf16's).  The 32-bit gate | up
@@ -182,13 +179,16 @@ typedef const __attribute__((address_space(1))) void lt_glb_t;
 // but one go.  At a part's last step its columns' scales and biases take it from the step's accumulators into the sum.  (22 products of
 // a Gelarax prompt in 8 launches: 2048 rows of width 2048 1268 -> 1202 us, 601 of width 1024 312 -> 309, and 14 launches less.)
 constexpr int LT_GROUPED = 1, LT_GLU = 2, LT_SUM = 4;
-template <int BM, int BN, int NB, int MODE>
-__global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_tile(LinArgs P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
+template <int BM, int BN, int WM, int WN, int NB, int MODE>
+__global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(LinArgs P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
 {
     constexpr bool GROUPED = MODE & LT_GROUPED, GLU = MODE & LT_GLU, SUM = MODE & LT_SUM;
-    constexpr int WAVES = BM == 32 ? 1 : 4, TA = BM == 32 ? 1 : BM / 64, TB = BM == 32 ? 1 : BN / 64, AI = BM / (8 * WAVES), WI = BN / (8 * WAVES), ROWB = 2 * LT_BK, STEPB = (BM + BN) * ROWB;
-    __shared__ __attribute__((aligned(16))) char smem[NB * STEPB];          // [NB steps][BM rows of A, BN rows of W]
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5, wm = wave & 1, wn = wave >> 1;          // (BM = 32: one wave, one tile)
+    constexpr int WAVES = WM * WN, TA = BM / (32 * WM), TB = BN / (32 * WN), AI = BM / (8 * WAVES), WI = BN / (8 * WAVES), ROWB = 2 * LT_BK, STEPB = (BM + BN) * ROWB;
+    static_assert(AI * 8 * WAVES == BM && WI * 8 * WAVES == BN && TA * 32 * WM == BM && TB * 32 * WN == BN, "whole rows and tiles a wave");
+    static_assert((NB - 2) * (AI + WI) < 64, "requests that s_waitcnt can count");
+    extern __shared__ __attribute__((aligned(16))) char lt_smem[];          // [NB steps][BM rows of A, BN rows of W]
+    char *const smem = lt_smem;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5, wm = wave % WM, wn = wave / WM;
     int t0, n0, t_end = P.T;
     const bf16_t *Wg = P.W;
     {
@@ -257,7 +257,7 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
 #pragma unroll
         for (int j = 0; j < WI; j++) stage_w(step, to, j);
     };
-    const int lc = g ^ swz(i), a_off = (wm * (BM / 2) + i) * ROWB, w_off = (BM + wn * (BN / 2) + i) * ROWB;          // (tile rows start at multiples of 32)
+    const int lc = g ^ swz(i), a_off = (wm * (BM / WM) + i) * ROWB, w_off = (BM + wn * (BN / WN) + i) * ROWB;          // (tile rows start at multiples of 32)
     f32x16v acc[TA][TB];
 #pragma unroll
     for (int a = 0; a < TA; a++)
@@ -280,7 +280,7 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
 #pragma unroll
             for (int b = 0; b < TB; b++) {
                 const auto &part = P.part[k];
-                const int n = min(n0 + wn * (BN / 2) + 32 * b + i, P.N - 1);
+                const int n = min(n0 + wn * (BN / WN) + 32 * b + i, P.N - 1);
                 p_bias[k][b] = part.bias ? bf2f(part.bias[n]) : 0.0f; p_mul[k][b] = part.alpha * (part.mul ? bf2f(part.mul[n]) : 1.0f);
             }
     }
@@ -340,23 +340,58 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
         }
         mma(af[1], wf[1]);
         close(nsteps - 1);
+    } else if constexpr (BM > 32) {
+        // A step's own requests have arrived (those of the NB - 2 steps behind it may be under way), everybody's with the barrier, before which every wave has also read the
+        // step before: its buffer takes the step NB - 1 further on.
+        auto arrived = [&](auto more) {
+            if constexpr (decltype(more)::value) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((NB - 2) * (AI + WI)) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
+        auto one = [&](int step, int j, auto more, auto last) {
+            const char *cur = smem + j * STEPB, *nxt = smem + (j + 1 == NB ? 0 : j + 1) * STEPB;
+            if constexpr (decltype(more)::value) stage(step + NB - 1, smem + (j == 0 ? NB - 1 : j - 1) * STEPB);
+#pragma unroll
+            for (int ks = 0; ks < 3; ks++) {          // (the next fragments under this one's products)
+                frags(cur, ks + 1, af[(ks + 1) & 1], wf[(ks + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                mma(af[ks & 1], wf[ks & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (!decltype(last)::value) {
+                arrived(more);
+                frags(nxt, 0, af[0], wf[0]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            mma(af[1], wf[1]);
+            __builtin_amdgcn_sched_barrier(0);
+            close(step);
+        };
+        // (at least NB steps)
+#pragma unroll
+        for (int j = 0; j < NB - 1; j++) stage(j, smem + j * STEPB);
+        arrived(std::true_type());
+        frags(smem, 0, af[0], wf[0]);
+        int step = 0, j = 0;
+        for (; step + NB - 1 < nsteps; step++) { one(step, j, std::true_type(), std::false_type()); j = j + 1 == NB ? 0 : j + 1; }
+        for (; step + 1 < nsteps; step++) { one(step, j, std::false_type(), std::false_type()); j = j + 1 == NB ? 0 : j + 1; }
+        one(step, j, std::false_type(), std::true_type());
     } else {
-        static_assert(TA == 1 && TB == 1, "a wave reads one tile of each operand");
+        static_assert(TA == 1 && TB == 1 && AI == 4 && WI == 4, "one wave: one tile of each operand, its requests of a step spread over four products");
         const unsigned lds0 = (unsigned)(uintptr_t)(lt_lds_t *)smem;
         unsigned at[4];
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) at[ks] = lds0 + (((2 * ks) ^ lc) << 4);
-        // One step: its own requests have arrived (those of the NB - 2 steps behind it may be under way), everybody's with the barrier, before which every wave has
-        // also read the step before: its buffer takes the step NB - 1 further on.  (The reads and their wait are one block: reads that the compiler sees wait for every
-        // request into LDS, once a round of the buffers at the least.)
+        // One step: its requests have arrived (those of the NB - 2 steps behind it may be under way) and the step before has been read: its buffer takes the step NB - 1 further on.
+        // (The reads and their wait are one block: reads that the compiler sees wait for every request into LDS, once a round of the buffers at the least.)
         auto one = [&](int step, int j, auto more) {
             if constexpr (decltype(more)::value) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NB - 2) * (AI + WI)) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             char *to = smem + (j == 0 ? NB - 1 : j - 1) * STEPB;
-            if constexpr (decltype(more)::value && BM > 32) stage(step + NB - 1, to);
-            if constexpr (decltype(more)::value && BM == 32) enter(step + NB - 1);
+            if constexpr (decltype(more)::value) enter(step + NB - 1);
             const unsigned oa = j * STEPB + a_off, ow = j * STEPB + w_off;
             bf16x8v fa[4], fw[4];
             asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %4, %12\n\tds_read_b128 %1, %9\n\tds_read_b128 %5, %13\n\tds_read_b128 %2, %10\n\tds_read_b128 %6, %14\n\t"
@@ -366,8 +401,7 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
 #pragma unroll
             for (int ks = 0; ks < 4; ks++) {
                 acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks], fw[ks], acc[0][0], 0, 0, 0);
-                if constexpr (decltype(more)::value && BM == 32) {          // (the only wave: its requests go out under its products, 4096 columns 16.5 -> 15.4 us)
-                    static_assert(BM > 32 || (AI == 4 && WI == 4), "the requests of a step over its four products");
+                if constexpr (decltype(more)::value) {          // (the only wave: its requests go out under its products, 4096 columns 16.5 -> 15.4 us)
                     __builtin_amdgcn_sched_barrier(0);
                     stage_a(step + NB - 1, to, ks);
                     stage_w(step + NB - 1, to, ks);
@@ -387,14 +421,14 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
     auto each = [&](auto f) {
 #pragma unroll
         for (int b = 0; b < TB; b++) {
-            const int n = n0 + wn * (BN / 2) + 32 * b + i;
+            const int n = n0 + wn * (BN / WN) + 32 * b + i;
             if (n >= n_end) continue;
             const float bv = P.bias ? bf2f(P.bias[n]) : 0.0f, mv = P.alpha * (P.mul ? bf2f(P.mul[n]) : 1.0f);
 #pragma unroll
             for (int a = 0; a < TA; a++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    const int t = t0 + wm * (BM / 2) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
+                    const int t = t0 + wm * (BM / WM) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
                     if (t < t_end) f((size_t)t * P.ldc + n, n, acc[a][b][r] + bv, mv);
                 }
         }
@@ -402,13 +436,13 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
     if constexpr (SUM) {
 #pragma unroll
         for (int b = 0; b < TB; b++) {
-            const int n = n0 + wn * (BN / 2) + 32 * b + i;
+            const int n = n0 + wn * (BN / WN) + 32 * b + i;
             if (n >= n_end) continue;
 #pragma unroll
             for (int a = 0; a < TA; a++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    const int t = t0 + wm * (BM / 2) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
+                    const int t = t0 + wm * (BM / WM) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
                     if (t < t_end) P.C[(size_t)t * P.ldc + n] += tot[a][b][r];
                 }
         }
@@ -420,14 +454,14 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
             const int hi = i >> 4;
 #pragma unroll
             for (int b = 0; b < TB; b++) {
-                const int o = o0 + (BM == 32 ? 0 : wn * (BN / 4)) + 16 * b + (i & 15);
+                const int o = o0 + wn * (BN / (2 * WN)) + 16 * b + (i & 15);
                 const float gb = P.bias && o < P.glu_f ? bf2f(P.bias[P.glu_c0 + o]) : 0.0f, ub = P.bias && o < P.glu_f ? bf2f(P.bias[P.glu_c0 + P.glu_f + o]) : 0.0f;
 #pragma unroll
                 for (int a = 0; a < TA; a++)
 #pragma unroll
                     for (int r = 0; r < 8; r++) {
                         const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[a][b][r]), __float_as_uint(acc[a][b][r + 8]), false, false);
-                        const int t = t0 + wm * (BM / 2) + 32 * a + (r & 3) + 8 * (r >> 2) + 16 * hi + 4 * g;
+                        const int t = t0 + wm * (BM / WM) + 32 * a + (r & 3) + 8 * (r >> 2) + 16 * hi + 4 * g;
                         const float v = glu_of(P.glu_kind, P.glu_limit, __uint_as_float(x[0]) + gb, __uint_as_float(x[1]) + ub);
                         if (t < t_end && o < P.glu_w) P.G16[(size_t)t * P.ldg + o] = __builtin_bit_cast(bf16_t, (__bf16)(o < P.glu_f ? v : 0.0f));
                     }
@@ -440,12 +474,12 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
         for (int a = 0; a < TA; a++)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const int t = t0 + wm * (BM / 2) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
+                const int t = t0 + wm * (BM / WM) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
                 if (t >= t_end) continue;
                 const float sc = P.row_scale ? P.row_scale[t] : 1.0f;
 #pragma unroll
                 for (int b = 0; b < TB; b++) {
-                    const int n = n0 + wn * (BN / 2) + 32 * b + i;
+                    const int n = n0 + wn * (BN / WN) + 32 * b + i;
                     if (n < P.N) P.C[(size_t)t * P.ldc + n] = acc[a][b][r] * sc;
                 }
             }
@@ -469,37 +503,61 @@ __global__ void __launch_bounds__(BM == 32 ? 64 : 256, BM == 32 ? 1 : 2) k_lin_t
 // column tiles of a product (gate | up: with G16's padding)
 size_t lin_col_tiles(const LinArgs &P, int bn, bool glu) { return glu ? (P.glu_c0 + bn - 1) / bn + ((size_t)P.glu_w + bn / 2 - 1) / (bn / 2) : ((size_t)P.N + bn - 1) / bn; }
 
-template <int BM, int BN, int NB, int MODE>
+template <int BM, int BN, int WM, int WN, int NB, int MODE>
 int launch_lin_tile(const LinArgs &P, const bf16_t *a16, size_t lda16, size_t row_tiles, hipStream_t s)
 {
+    constexpr int smem = NB * (BM + BN) * 2 * LT_BK;
     const int tm = (int)row_tiles, tn = (int)lin_col_tiles(P, BN, MODE & LT_GLU);
-    hipLaunchKernelGGL((k_lin_tile<BM, BN, NB, MODE>), dim3((unsigned)tm * (unsigned)tn), dim3(BM == 32 ? 64 : 256), 0, s, P, a16, (int)lda16, tm, tn);
+    const auto fn = k_lin_tile<BM, BN, WM, WN, NB, MODE>;
+    if (smem > 64 * 1024) IFA_HIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, smem));
+    hipLaunchKernelGGL(fn, dim3((unsigned)tm * (unsigned)tn), dim3(64 * WM * WN), smem, s, P, a16, (int)lda16, tm, tn);
     IFA_LAUNCH_CHECK();
     return IFA_OK;
 }
 
-// the largest tile that still gives every compute unit its share of workgroups
+// Tile shapes by what a round of the chip's 256 compute units takes: us a step of 64 columns with one and with two workgroups on a compute unit, and beside the steps, measured with weights
+// from memory.  us before (128 x 128 and 128 x 64 of 4 waves with two buffers, 64 x 64 with four) / now, tokens x columns x K: 2048 x 2048 x 9728 123 / 90, 1000 x 2048 x 9728 117 / 62,
+// 2000 x 1024 x 4864 58 / 32, 2048 x 1024 x 1024 15.4 / 8.7, 730 x 2836 x 1024 16.1 / 12.5, 1024 x 4096 x 2048 29.9 / 22.5, 601 x 1024 x 4864 22.1 / 20.8; in a Gelarax layer 2048 rows' input
+// product (19968 columns, gated) 238 / 207, its output product 150 / 108.  (256 x 128 tiles of eight waves, one a compute unit, 225 to 235 there.)
+struct LinShape { int per_cu; double one, two, beside; };
+enum { LT_128x128_PAIR, LT_128x128, LT_128x64, LT_64x64, LT_N_SHAPES };
+constexpr LinShape LT_SHAPES[LT_N_SHAPES] = {{2, 0.80, 1.17, 4}, {1, 0.55, 0, 5}, {1, 0.36, 0, 4}, {2, 0.255, 0.44, 4}};
+double lin_cost(const LinShape &h, size_t tiles, size_t steps)
+{
+    const size_t cus = 256, slots = cus * h.per_cu, full = tiles / slots, rest = tiles % slots;
+    const double all = steps * (h.per_cu == 2 ? h.two : h.one) + h.beside;
+    return full * all + (rest == 0 ? 0.0 : rest <= cus ? steps * h.one + h.beside : all);
+}
+
 template <int MODE>
 int lin_tile_dispatch(const LinArgs &P, const bf16_t *a, size_t lda, hipStream_t s)
 {
     constexpr bool GLU = MODE & LT_GLU;
-    const size_t T = (size_t)P.T, t128 = (T + 127) / 128, t64 = (T + 63) / 64, n128 = lin_col_tiles(P, 128, GLU), n64 = lin_col_tiles(P, 64, GLU);
+    const size_t T = (size_t)P.T, t128 = (T + 127) / 128, t64 = (T + 63) / 64, n128 = lin_col_tiles(P, 128, GLU), n64 = lin_col_tiles(P, 64, GLU), steps = lda / LT_BK;
     IFA_REQUIRE(t64 * n64 < (1u << 31), "linear_bf16: too many tiles");
-    if (t128 * n128 >= 384) return launch_lin_tile<128, 128, 2, MODE>(P, a, lda, t128, s);
-    if (t128 * n64 >= 256) return launch_lin_tile<128, 64, 2, MODE>(P, a, lda, t128, s);
-    if (t64 * n64 > LT_DEEP || lda < 4 * LT_BK) return launch_lin_tile<64, 64, 2, MODE>(P, a, lda, t64, s);
-    if (t64 * n64 > LT_SMALL || lda < 8 * LT_BK) return launch_lin_tile<64, 64, 4, MODE>(P, a, lda, t64, s);
-    return launch_lin_tile<32, 32, 8, MODE>(P, a, lda, (T + 31) / 32, s);
+    if (steps < 5) return t128 * n128 >= 384 ? launch_lin_tile<128, 128, 2, 4, 2, MODE>(P, a, lda, t128, s) : launch_lin_tile<64, 64, 2, 2, 2, MODE>(P, a, lda, t64, s);
+    if (t64 * n64 <= LT_SMALL && steps >= 8) return launch_lin_tile<32, 32, 1, 1, 8, MODE>(P, a, lda, (T + 31) / 32, s);
+    const size_t tiles[LT_N_SHAPES] = {t128 * n128, t128 * n128, t128 * n64, t64 * n64};
+    int best = 0;
+    for (int k = 1; k < LT_N_SHAPES; k++)
+        if (lin_cost(LT_SHAPES[k], tiles[k], steps) < lin_cost(LT_SHAPES[best], tiles[best], steps)) best = k;
+    switch (best) {
+    case LT_128x128_PAIR: return launch_lin_tile<128, 128, 2, 4, 2, MODE>(P, a, lda, t128, s);
+    case LT_128x128: return launch_lin_tile<128, 128, 2, 4, 4, MODE>(P, a, lda, t128, s);
+    case LT_128x64: return launch_lin_tile<128, 64, 4, 2, 4, MODE>(P, a, lda, t128, s);
+    default: return launch_lin_tile<64, 64, 2, 2, 5, MODE>(P, a, lda, t64, s);
+    }
 }
 
 template <int MODE>
 int lin_grouped_dispatch(const LinArgs &P, const bf16_t *a, size_t lda, size_t max_tiles, int tile_rows, hipStream_t s)
 {
-    const size_t n64 = lin_col_tiles(P, 64, MODE & LT_GLU);
-    IFA_REQUIRE(max_tiles * n64 < (1u << 31), "linear_bf16_grouped: too many tiles");
-    if (tile_rows == 128) return launch_lin_tile<128, 128, 2, MODE>(P, a, lda, max_tiles, s);
-    if (max_tiles * n64 > LT_DEEP || lda < 4 * LT_BK) return launch_lin_tile<64, 64, 2, MODE>(P, a, lda, max_tiles, s);
-    return launch_lin_tile<64, 64, 4, MODE>(P, a, lda, max_tiles, s);
+    IFA_REQUIRE(max_tiles * lin_col_tiles(P, 64, MODE & LT_GLU) < (1u << 31), "linear_bf16_grouped: too many tiles");
+    // (8192 pairs of 16 experts, 1408 x 1024 gate | up and 1024 x 704, us: four waves a 128 x 128 tile 54.8 + 46.8, eight 47.9 + 40.4; 2900 pairs: 64 x 64 tiles 34.2 + 18.8, 64 x 128 of
+    // eight waves 27.0 + 17.0)
+    if (tile_rows == 128) return launch_lin_tile<128, 128, 2, 4, 2, MODE>(P, a, lda, max_tiles, s);
+    if (lda >= 3 * LT_BK) return launch_lin_tile<64, 128, 2, 4, 3, MODE>(P, a, lda, max_tiles, s);
+    return launch_lin_tile<64, 64, 2, 2, 2, MODE>(P, a, lda, max_tiles, s);
 }
 
 // rows of 32-bit values to bfloat16, zero up to `width` columns (a multiple of 8) of rows of ldy
