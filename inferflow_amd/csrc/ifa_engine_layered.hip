@@ -446,16 +446,22 @@ int linear_in(ifa_model *m, const bf16_t *W, size_t N, size_t K, const float *h,
     return linear(m, W, N, K, h, K, T, bias, nullptr, 1.0f, 0, C, ldc);
 }
 
-// A product whose columns [c_glu, c_glu + 2 F) are gate | up of a gated feed-forward.  Where the down-projection reads bfloat16 rows, the activations leave it so (n->g16; the
-// columns themselves are not stored), otherwise gate | up stay in C; glu_down is told by *left16.
+// A product whose columns [c_glu, c_glu + 2 F) are gate | up of a gated feed-forward.  Where the down-projection reads bfloat16 rows, the activations leave it so (n->g16), steps of a few
+// rows leave them in 32 bits (n->m3); the columns themselves are not stored then.  Otherwise gate | up stay in C.  glu_down is told by *left.
+enum { GLU_COLUMNS = 0, GLU_16, GLU_32 };
 int linear_glu(ifa_model *m, const bf16_t *W, size_t N, size_t K, const float *h, const bf16_t *h16, size_t T, const bf16_t *bias, float *C, size_t ldc, int silu0, int silu1,
-               size_t c_glu, size_t F, int kind, float limit, bool *left16)
+               size_t c_glu, size_t F, int kind, float limit, int *left)
 {
     LayeredNet *n = m->lay;
     ifa_stream s = (ifa_stream)m->stream;
     int rc;
-    *left16 = takes_a16(n, K, T) && takes_a16(n, F, T);
-    if (!*left16) {
+    *left = takes_a16(n, K, T) && takes_a16(n, F, T) ? GLU_16 : GLU_COLUMNS;
+    if (*left == GLU_COLUMNS) {
+        if (T <= 8 && !h16 && ifa_linear_bf16w_glu_rows(W, N, K, h, K, T, bias, C, ldc, silu0, silu1, c_glu, F, kind, limit, n->m3, F, s)) {
+            IFA_LAUNCH_CHECK();
+            *left = GLU_32;
+            return IFA_OK;
+        }
         if (h16) return ifa_linear_bf16_both(W, N, K, h16, K, T, bias, nullptr, 1.0f, 0, 0, C, nullptr, ldc, silu0, silu1, s);
         return linear(m, W, N, K, h, K, T, bias, nullptr, 1.0f, 0, C, ldc, silu0, silu1);
     }
@@ -467,14 +473,16 @@ int linear_glu(ifa_model *m, const bf16_t *W, size_t N, size_t K, const float *h
     return ifa_linear_bf16_glu(W, N, K, h16, a16_stride(K), T, bias, C, ldc, silu0, silu1, c_glu, F, kind, limit, n->g16, a16_stride(F), s);
 }
 
-// the down-projection behind it; row_gate (where they have not left so): the activations of row t times sigmoid(row_gate[t * ldg])
-int glu_down(ifa_model *m, bool left16, int kind, float limit, const float *gate_up, size_t ld, size_t F, const float *row_gate, size_t ldg, const bf16_t *W, size_t N, size_t T,
+// the down-projection behind it; row_gate (not with GLU_16): the activations, or the sums behind them, of row t times sigmoid(row_gate[t * ldg])
+int glu_down(ifa_model *m, int left, int kind, float limit, const float *gate_up, size_t ld, size_t F, const float *row_gate, size_t ldg, const bf16_t *W, size_t N, size_t T,
              const bf16_t *bias, const bf16_t *mul, int accumulate, float *C)
 {
     LayeredNet *n = m->lay;
     ifa_stream s = (ifa_stream)m->stream;
     int rc;
-    if (left16) return ifa_linear_bf16_both(W, N, F, n->g16, a16_stride(F), T, bias, mul, 1.0f, accumulate, 0, C, nullptr, N, 0, 0, s);
+    if (left == GLU_32 && row_gate) return ifa_linear_bf16w_gated_rows(W, N, F, n->m3, F, T, row_gate, ldg, accumulate, C, N, s);
+    if (left == GLU_32) return linear(m, W, N, F, n->m3, F, T, bias, mul, 1.0f, accumulate, C, N);
+    if (left == GLU_16) return ifa_linear_bf16_both(W, N, F, n->g16, a16_stride(F), T, bias, mul, 1.0f, accumulate, 0, C, nullptr, N, 0, 0, s);
     if (takes_a16(n, F, T)) {
         if ((rc = ensure_a16(m, T, F)) || (rc = ifa_glu_to_bf16(kind, limit, gate_up, ld, T, F, row_gate, ldg, n->a16, a16_stride(F), s))) return rc;
         return ifa_linear_bf16_both(W, N, F, n->a16, a16_stride(F), T, bias, mul, 1.0f, accumulate, 0, C, nullptr, N, 0, 0, s);
@@ -717,21 +725,27 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
     }
     if (!moe) {
         const size_t F = (size_t)sp.ffn;
-        bool left16 = false;
-        if ((rc = linear_glu(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2, 0, 0, L.c2_fg, F, 3, sp.f_limit, &left16))) return rc;
-        if ((rc = glu_down(m, left16, 3, sp.f_limit, n->proj + L.c2_fg, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m2))) return rc;
+        int left = GLU_COLUMNS;
+        if ((rc = linear_glu(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2, 0, 0, L.c2_fg, F, 3, sp.f_limit, &left))) return rc;
+        if ((rc = glu_down(m, left, 3, sp.f_limit, n->proj + L.c2_fg, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m2))) return rc;
     } else {
-        if ((rc = linear_in(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2))) return rc;
+        int left = GLU_COLUMNS;
+        if (T <= 8 && sp.x_shared_ff > 0 && !takes_a16(n, W, T)) rc = linear_glu(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2, 0, 0, L.c2_shg, (size_t)sp.x_shared_ff, 0, 0.0f, &left);
+        else rc = linear_in(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2);
+        if (rc) return rc;
         // the router's logits (bias added by the product) are columns of the second product; the chosen experts read norm2's output
-        if ((rc = ifa_moe_route_top_f32(n->proj + L.c2_router, N2, T, sp.x_experts, sp.x_top, nullptr, n->moe_idx, n->moe_wgt, s))) return rc;
-        rc = moe16 ? ifa_moe_experts_gated_bf16(n->h16, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data, n->moe_idx, n->moe_wgt, n->moe_ws,
+        const bool choose = !(fused && T <= 8 && sp.x_experts <= 256);          // (a few rows: the choice inside the experts' first launch)
+        if (choose && (rc = ifa_moe_route_top_f32(n->proj + L.c2_router, N2, T, sp.x_experts, sp.x_top, nullptr, n->moe_idx, n->moe_wgt, s))) return rc;
+        rc = !choose ? ifa_moe_experts_gated_top_rows(n->proj + L.c2_router, N2, n->h, W, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data,
+                                                      n->moe_idx, n->moe_wgt, n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, s)
+           : moe16 ? ifa_moe_experts_gated_bf16(n->h16, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data, n->moe_idx, n->moe_wgt, n->moe_ws,
                                                 n->moe_ws_bytes, n->m2, W, 0, s)
                    : ifa_moe_experts_gated_f32(n->h, W, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data, n->moe_idx, n->moe_wgt, c.ops32,
                                                n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, s);
         if (rc) return rc;
         if (sp.x_shared_ff > 0) {      // the shared expert: its gate sigmoid(w_sg . h) multiplies the activations in front of the down-projection
             const size_t SF = (size_t)sp.x_shared_ff;
-            if ((rc = glu_down(m, false, 0, 0.0f, n->proj + L.c2_shg, N2, SF, n->proj + L.c2_sg, N2, (const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, W, T, nullptr, nullptr, 1, n->m2))) return rc;
+            if ((rc = glu_down(m, left, 0, 0.0f, n->proj + L.c2_shg, N2, SF, n->proj + L.c2_sg, N2, (const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, W, T, nullptr, nullptr, 1, n->m2))) return rc;
         }
     }
     return close_sub(n->m2, L.T(IFA_LT_NORM2B).data, next_norm, in16);
@@ -881,9 +895,9 @@ int run_streams_layer(ifa_model *m, LLayer &L, size_t T, int nseq, int pass, LLa
     if (!any_ffn) return IFA_OK;
     if (!moe) {
         const size_t F = (size_t)sp.ffn, N2 = L.n_in2;
-        bool left16 = false;
-        if ((rc = linear_glu(m, L.w_in2, N2, W, n->h, nullptr, T, nullptr, n->proj, N2, 0, 0, 0, F, 0, 0.0f, &left16))) return rc;
-        if ((rc = glu_down(m, left16, 0, 0.0f, n->proj, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m1))) return rc;
+        int left = GLU_COLUMNS;
+        if ((rc = linear_glu(m, L.w_in2, N2, W, n->h, nullptr, T, nullptr, n->proj, N2, 0, 0, 0, F, 0, 0.0f, &left))) return rc;
+        if ((rc = glu_down(m, left, 0, 0.0f, n->proj, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m1))) return rc;
     } else {
         const int XA = sp.x_experts;
         if (T <= 8 && XA <= 256 && n->opt_fuse_post) {      // a few rows: the choice inside the experts' first launch
@@ -1136,14 +1150,14 @@ int run_layers(ifa_model *m, size_t T, int nseq)
         const bool lin = sp.mixer == IFA_MIX_WINDOW_LINEAR;
         // steps of a few rows: the norm is formed inside the product's read of the residual, the gated GELU inside the down-projection's
         const bool fuse = T <= 8 && W % 8 == 0;
-        bool left16 = false;
+        int left = GLU_COLUMNS;
         if (fuse && (n->opt_fuse_rows & 1)) {
             if ((rc = ifa_linear_bf16w_rows(1, L.T(IFA_LT_NORM1).data, c.eps, L.w_in, NI, W, n->x, W, T, L.b_in, nullptr, 1.0f, 0, n->proj, NI,
                                             lin ? (int)L.c_lq : 0, lin ? (int)L.c_lg : 0, s))) return rc;
         } else {
             if ((rc = ifa_layernorm_f32(1, n->x, W, T, W, L.T(IFA_LT_NORM1).data, c.eps, n->h, W, s))) return rc;
             const int silu0 = lin ? (int)L.c_lq : 0, silu1 = lin ? (int)L.c_lg : 0;
-            if (sp.ffn > 0) rc = linear_glu(m, L.w_in, NI, W, n->h, nullptr, T, L.b_in, n->proj, NI, silu0, silu1, L.c_fg, (size_t)sp.ffn, 1, 0.0f, &left16);
+            if (sp.ffn > 0) rc = linear_glu(m, L.w_in, NI, W, n->h, nullptr, T, L.b_in, n->proj, NI, silu0, silu1, L.c_fg, (size_t)sp.ffn, 1, 0.0f, &left);
             else rc = linear(m, L.w_in, NI, W, n->h, W, T, L.b_in, nullptr, 1.0f, 0, n->proj, NI, silu0, silu1);
             if (rc) return rc;
         }
@@ -1174,7 +1188,7 @@ int run_layers(ifa_model *m, size_t T, int nseq)
                 if ((rc = ifa_linear_bf16w_rows(2, nullptr, 0.0f, L.T(IFA_LT_FFN_DOWN).data, W, F, n->proj + L.c_fg, NI, T, L.T(IFA_LT_FFN_DOWN_B).data,
                                                 L.T(IFA_LT_LS2).data, 1.0f, 1, n->x, W, 0, 0, s))) return rc;
             } else {
-                if ((rc = glu_down(m, left16, 1, 0.0f, n->proj + L.c_fg, NI, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T,
+                if ((rc = glu_down(m, left, 1, 0.0f, n->proj + L.c_fg, NI, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T,
                                      (const bf16_t *)L.T(IFA_LT_FFN_DOWN_B).data, (const bf16_t *)L.T(IFA_LT_LS2).data, 1, n->x))) return rc;
             }
         }
@@ -1742,7 +1756,8 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
     ifa_stream s = (ifa_stream)m->stream;
     if (all) {
         if ((rc = run_head(m, 0, T))) return rc;
-        for (int q = 0; q < nseq; q++)
+        if (T == (size_t)nseq) { if ((rc = ifa_argmax_rows_f32(n->logits, V, V, T, n->excl_dev, n->next_dev, s))) return rc; }          // (a token each)
+        else for (int q = 0; q < nseq; q++)
             if ((rc = ifa_argmax_rows_f32(n->logits + (size_t)last[(size_t)q] * V, V, V, 1, n->excl_dev, n->next_dev + q, s))) return rc;
     } else {
         // the sequences' last rows, normed one by one into consecutive rows of h, then one product

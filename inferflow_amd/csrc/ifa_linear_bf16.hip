@@ -40,7 +40,10 @@ struct LinArgs {
     bf16_t *C16;                               // (k_lin_tile with act_kind 2: the output in bfloat16 instead of C)
     int act_kind;                              // every output after the bias passes 1: the exact (erf) GELU, 2: the square of relu
     // (k_lin_tile, GLU) columns [glu_c0, glu_c0 + 2 glu_f) are gate | up: instead of them G16[t][c] = act(gate[c]) up[c] in bfloat16, glu_w columns (whole 64s, zero beyond glu_f)
+    // (k_lin_rows_group: in 32 bits, G)
     bf16_t *G16; int ldg, glu_c0, glu_f, glu_w, glu_kind; float glu_limit;
+    float *G;
+    const float *row_gate; int ld_gate;        // (lin_store) row t times sigmoid(row_gate[t * ld_gate])
     // (k_lin_tile, SUM) several products into the same columns: A's rows hold their operands side by side, each padded to whole steps; W, K, mul, bias, alpha of each here
     struct Part { const bf16_t *W, *mul, *bias; int K, steps; float alpha; } part[IFA_SUM_PARTS];
 };
@@ -52,6 +55,7 @@ __device__ __forceinline__ void lin_store(const LinArgs &P, int t, int n, float 
     if (P.act_kind == 1) acc = 0.5f * acc * (1.0f + erff(acc * 0.70710678118654752f));
     if (P.act_kind == 2) { acc = fmaxf(acc, 0.0f); acc *= acc; }
     if (P.row_scale) acc *= P.row_scale[t];
+    if (P.row_gate) acc *= sigmoid_f(P.row_gate[(size_t)t * P.ld_gate]);
     if (P.mul) acc *= bf2f(P.mul[n]);
     acc *= P.alpha;
     float *c = P.C + (size_t)t * P.ldc + n;
@@ -696,6 +700,103 @@ __global__ void __launch_bounds__(256) k_lin_rows(LinArgs P)
     }
 }
 
+// T <= TT rows of many outputs, NR of them a wave at a time: k_lin_rows reads TT rows of activations (32 bytes of each beside 16 of the weight) for one output, and with six rows
+// the caches' bandwidth for them bounds large matrices (32000 x 1024, six rows: 38.9 -> 31.0 us, 8192 x 2048
+// 21.0 -> 16.7; four outputs 34.9 and 21.0).  GLU: from column glu_c0 on the NR are gates and ups by twos, and the activation leaves instead
+// of them (the launch that formed it took 3.7 us).
+template <int TT, int NR, bool GLU>
+__global__ void __launch_bounds__(256) k_lin_rows_group(LinArgs P)
+{
+    const int lane = threadIdx.x & 63, wave = blockIdx.x * 4 + (threadIdx.x >> 6), nwaves = gridDim.x * 4;
+    const int n_end = GLU ? P.glu_c0 : P.N, plain = (n_end + NR - 1) / NR, groups = plain + (GLU ? (P.glu_f + NR / 2 - 1) / (NR / 2) : 0);
+    for (int grp = wave; grp < groups; grp += nwaves) {
+        const bool glu = GLU && grp >= plain;
+        const int n0 = grp * NR, o0 = (grp - plain) * (NR / 2);
+        const bf16_t *w[NR];
+        int row[NR];
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            row[r] = glu ? P.glu_c0 + ((r & 1) ? P.glu_f : 0) + min(o0 + (r >> 1), P.glu_f - 1) : min(n0 + r, n_end - 1);
+            w[r] = P.W + (size_t)row[r] * P.K;
+        }
+        float acc[TT][NR];
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int r = 0; r < NR; r++) acc[t][r] = 0.0f;
+        // (pieces of the weights first, see k_lin_rows; past the end a piece again that is not multiplied)
+        auto block = [&](int k0, auto pieces) {
+            constexpr int NP = decltype(pieces)::value;
+            u32x4v wp[NP][NR];
+#pragma unroll
+            for (int j = 0; j < NP; j++)
+#pragma unroll
+                for (int r = 0; r < NR; r++) wp[j][r] = *reinterpret_cast<const u32x4v *>(w[r] + min(k0 + 512 * j + lane * 8, P.K - 8));
+#pragma unroll
+            for (int j = 0; j < NP; j++) {
+                const int k = k0 + 512 * j + lane * 8;
+                if (k0 + 512 * j >= P.K) break;
+                float4 v[TT][2];
+#pragma unroll
+                for (int t = 0; t < TT; t++) {
+                    const float *a = P.A + (size_t)min(t, P.T - 1) * P.lda + min(k, P.K - 8);
+                    v[t][0] = *reinterpret_cast<const float4 *>(a); v[t][1] = *reinterpret_cast<const float4 *>(a + 4);
+                }
+                if (k >= P.K) continue;
+#pragma unroll
+                for (int r = 0; r < NR; r++) {
+                    float w8[8];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) { w8[2 * e] = __uint_as_float(wp[j][r][e] << 16); w8[2 * e + 1] = __uint_as_float(wp[j][r][e] & 0xFFFF0000u); }
+#pragma unroll
+                    for (int t = 0; t < TT; t++) {
+                        const float x8[8] = {v[t][0].x, v[t][0].y, v[t][0].z, v[t][0].w, v[t][1].x, v[t][1].y, v[t][1].z, v[t][1].w};
+                        float sum = acc[t][r];
+#pragma unroll
+                        for (int e = 0; e < 8; e++) sum = fmaf(x8[e], w8[e], sum);
+                        acc[t][r] = sum;
+                    }
+                }
+            }
+        };
+        int k0 = 0;
+        if constexpr (NR <= 2) for (; P.K - k0 > 1024; k0 += 2048) block(k0, std::integral_constant<int, 4>());
+        for (; P.K - k0 > 512; k0 += 1024) block(k0, std::integral_constant<int, 2>());
+        if (P.K - k0 > 0) block(k0, std::integral_constant<int, 1>());
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int r = 0; r < NR; r++) acc[t][r] = wave_sum(acc[t][r]);
+#pragma unroll
+        for (int t = 0; t < TT; t++) {
+            if (lane != t || t >= P.T) continue;
+            if (glu) {
+#pragma unroll
+                for (int r = 0; r < NR; r += 2) {
+                    const float gb = P.bias ? bf2f(P.bias[row[r]]) : 0.0f, ub = P.bias ? bf2f(P.bias[row[r + 1]]) : 0.0f;
+                    if (o0 + (r >> 1) < P.glu_f) P.G[(size_t)t * P.ldg + o0 + (r >> 1)] = glu_of(P.glu_kind, P.glu_limit, acc[t][r] + gb, acc[t][r + 1] + ub);
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < NR; r++) if (n0 + r < n_end) lin_store(P, t, n0 + r, acc[t][r]);
+            }
+        }
+    }
+}
+
+// workgroups: a group of outputs a wave, up to 32 waves a compute unit
+template <int NR, bool GLU>
+void launch_lin_rows_group(const LinArgs &P, hipStream_t s)
+{
+    const size_t n_end = GLU ? P.glu_c0 : P.N, groups = (n_end + NR - 1) / NR + (GLU ? ((size_t)P.glu_f + NR / 2 - 1) / (NR / 2) : 0);
+    const dim3 grid((unsigned)std::min<size_t>((groups + 3) / 4, 8192));
+    if (P.T == 1) hipLaunchKernelGGL((k_lin_rows_group<1, NR, GLU>), grid, dim3(256), 0, s, P);
+    else if (P.T == 2) hipLaunchKernelGGL((k_lin_rows_group<2, NR, GLU>), grid, dim3(256), 0, s, P);
+    else if (P.T <= 4) hipLaunchKernelGGL((k_lin_rows_group<4, NR, GLU>), grid, dim3(256), 0, s, P);
+    else if (P.T <= 6) hipLaunchKernelGGL((k_lin_rows_group<6, NR, GLU>), grid, dim3(256), 0, s, P);
+    else hipLaunchKernelGGL((k_lin_rows_group<8, NR, GLU>), grid, dim3(256), 0, s, P);
+}
+
 // ONE row, layer-normed on the way in (k_lin_rows with prologue 1 formed the norm again for every output row of a wave): each wave forms mean and variance
 // once and keeps its lanes' normed values in registers, then walks output rows, the next row's weights asked for before this one's are summed.  The first
 // row's weights are on their way under the norm, so the norm's own launch (6 us) is saved for about 1 us more here (both 12.4 us, now 7.6, over a token's products of width 1024).
@@ -775,7 +876,7 @@ __global__ void __launch_bounds__(256) k_lin_row_norm(LinArgs P)
 
 static int linear_launch(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *bias_bf16,
                          const void *mul_bf16, float alpha, int accumulate, int ops32, void *c_f32, size_t ldc, int silu_col0, int silu_col1, int prologue,
-                         const void *norm_w_bf16, float norm_eps, ifa_stream stream, const char *who, int act = 0)
+                         const void *norm_w_bf16, float norm_eps, ifa_stream stream, const char *who, int act = 0, const float *row_gate = nullptr, size_t ld_gate = 0)
 {
     IFA_REQUIRE(w_bf16 && a_f32 && c_f32, "%s: null pointer", who);
     IFA_REQUIRE(rows > 0 && cols > 0 && tokens > 0 && lda >= cols * (prologue == 2 ? 2 : 1) && ldc >= rows, "%s: bad shape (%zu x %zu, %zu tokens, lda %zu, ldc %zu)", who, rows, cols, tokens, lda, ldc);
@@ -786,7 +887,7 @@ static int linear_launch(const void *w_bf16, size_t rows, size_t cols, const voi
     P.T = (int)tokens; P.N = (int)rows; P.K = (int)cols; P.lda = (int)lda; P.ldc = (int)ldc;
     P.alpha = alpha; P.accumulate = accumulate ? 1 : 0; P.act_c0 = silu_col0; P.act_c1 = silu_col1;
     P.norm_w = (const bf16_t *)norm_w_bf16; P.norm_eps = norm_eps;
-    P.tile_map = P.n_tiles = P.a_rows = nullptr; P.row_scale = nullptr; P.act_kind = act; P.C16 = nullptr;
+    P.tile_map = P.n_tiles = P.a_rows = nullptr; P.row_scale = nullptr; P.act_kind = act; P.C16 = nullptr; P.row_gate = row_gate; P.ld_gate = (int)ld_gate;
     // 16-byte requests need whole 8-element pieces in every row of both operands
     P.vec = (cols % 8 == 0 && lda % 4 == 0 && ((uintptr_t)a_f32 & 15) == 0 && ((uintptr_t)w_bf16 & 15) == 0) ? 1 : 0;
     hipStream_t s = ifa_s(stream);
@@ -801,6 +902,8 @@ static int linear_launch(const void *w_bf16, size_t rows, size_t cols, const voi
         if (cols <= 2 * 512) hipLaunchKernelGGL(k_lin_row_norm<2>, dim3(grid), dim3(256), 0, s, P);
         else if (cols <= 4 * 512) hipLaunchKernelGGL(k_lin_row_norm<4>, dim3(grid), dim3(256), 0, s, P);
         else hipLaunchKernelGGL(k_lin_row_norm<8>, dim3(grid), dim3(256), 0, s, P);
+    } else if (tokens > 1 && tokens <= 8 && !prologue && P.vec && rows * cols >= (size_t)8 << 20) {
+        launch_lin_rows_group<2, false>(P, s);
     } else if (tokens <= 8) {
         const unsigned grid = (unsigned)std::min<size_t>((rows + 3) / 4, 8192);
 #define IFA_LR(TT) { if (prologue == 1) hipLaunchKernelGGL((k_lin_rows<TT, 1>), dim3(grid), dim3(256), 0, s, P); \
@@ -815,6 +918,29 @@ static int linear_launch(const void *w_bf16, size_t rows, size_t cols, const voi
     }
     IFA_LAUNCH_CHECK();
     return IFA_OK;
+}
+
+int ifa_linear_bf16w_gated_rows(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *row_gate_f32, size_t ld_gate, int accumulate, void *c_f32,
+                                size_t ldc, ifa_stream stream)
+{
+    IFA_REQUIRE(row_gate_f32 && tokens <= 8 && ld_gate < (1u << 30), "linear_bf16w_gated_rows: %zu rows (at most 8), or no gate", tokens);
+    return linear_launch(w_bf16, rows, cols, a_f32, lda, tokens, nullptr, nullptr, 1.0f, accumulate, 1, c_f32, ldc, 0, 0, 0, nullptr, 0.0f, stream, "linear_bf16w_gated_rows", 0,
+                         (const float *)row_gate_f32, ld_gate);
+}
+
+bool ifa_linear_bf16w_glu_rows(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,
+                               int silu_col1, size_t glu_col0, size_t glu_cols, int glu_kind, float glu_limit, void *g_f32, size_t ldg, ifa_stream stream)
+{
+    if (!w_bf16 || !a_f32 || !g_f32 || (!c_f32 && glu_col0) || tokens == 0 || tokens > 8 || cols == 0 || cols % 8 || lda < cols || lda % 4 || ((uintptr_t)a_f32 & 15) || ((uintptr_t)w_bf16 & 15)
+        || ldc < glu_col0 || glu_cols == 0 || glu_col0 + 2 * glu_cols > rows || ldg < glu_cols || rows >= (1u << 30) || cols >= (1u << 30) || lda >= (1u << 30) || ldc >= (1u << 30)
+        || ldg >= (1u << 30) || glu_kind < 0 || glu_kind > 3 || (glu_kind == 3 && !(glu_limit > 0.0f))) return false;
+    LinArgs P;
+    memset(&P, 0, sizeof(P));
+    P.W = (const bf16_t *)w_bf16; P.A = (const float *)a_f32; P.C = (float *)c_f32; P.bias = (const bf16_t *)bias_bf16; P.T = (int)tokens; P.N = (int)rows; P.K = (int)cols; P.lda = (int)lda;
+    P.ldc = (int)ldc; P.alpha = 1.0f; P.vec = 1; P.act_c0 = silu_col0; P.act_c1 = silu_col1; P.G = (float *)g_f32; P.ldg = (int)ldg; P.glu_c0 = (int)glu_col0; P.glu_f = (int)glu_cols;
+    P.glu_kind = glu_kind; P.glu_limit = glu_limit;
+    launch_lin_rows_group<2, true>(P, ifa_s(stream));
+    return true;
 }
 
 extern "C" int ifa_linear_bf16w(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens,
@@ -951,7 +1077,7 @@ extern "C" int ifa_linear_bf16w_grouped(const void *w_bf16, size_t rows, size_t 
     P.W = (const bf16_t *)w_bf16; P.A = (const float *)a_f32; P.C = (float *)c_f32; P.bias = nullptr; P.mul = nullptr;
     P.T = 0; P.N = (int)rows; P.K = (int)cols; P.lda = (int)lda; P.ldc = (int)ldc; P.alpha = 1.0f; P.accumulate = 0; P.act_c0 = P.act_c1 = 0;
     P.norm_w = nullptr; P.norm_eps = 0.0f;
-    P.tile_map = tile_map_dev; P.n_tiles = n_tiles_dev; P.a_rows = a_rows_dev; P.row_scale = (const float *)row_scale_f32; P.act_kind = act; P.C16 = nullptr;
+    P.tile_map = tile_map_dev; P.n_tiles = n_tiles_dev; P.a_rows = a_rows_dev; P.row_scale = (const float *)row_scale_f32; P.act_kind = act; P.C16 = nullptr; P.row_gate = nullptr; P.ld_gate = 0;
     P.vec = (cols % 8 == 0 && lda % 4 == 0 && ((uintptr_t)a_f32 & 15) == 0 && ((uintptr_t)w_bf16 & 15) == 0 && (rows * cols) % 8 == 0) ? 1 : 0;
     const dim3 grid(ifa_cdiv(rows, LM_N), (unsigned)max_tiles);
     if (ops32) hipLaunchKernelGGL(k_lin_mfma<true>, grid, dim3(256), 0, ifa_s(stream), P);

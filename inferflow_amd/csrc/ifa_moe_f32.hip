@@ -11,6 +11,7 @@
 // the pair's weight in the second's) and k_moe_combine adds a row's pairs in the fixed order of its choices.  No atomics on values: a
 // row's result does not depend on what else is in the step.
 #include <algorithm>
+#include <cstring>
 #include "ifa_host.h"
 #include "ifa_f32_common.h"
 #include "inferflow_amd.h"
@@ -166,7 +167,8 @@ __device__ int route_pair(const RouteSel &R, int t, int k, int top, bool leave)
     const int e = threadIdx.x;
     const bool live = e < R.n_all;
     float s = live ? R.logits[(size_t)t * R.ld + e] : -INFINITY;
-    if (R.score_kind == 1) s = live ? sigmoid_f(s) : 0.0f;
+    if (R.score_kind == 2) s = s == s ? s : -INFINITY;          // (the logits themselves; one that is no number comes last)
+    else if (R.score_kind == 1) s = live ? sigmoid_f(s) : 0.0f;
     else {          // softmax: the maximum over the row, then the sum
         const float wm = wave_max(s);
         if ((e & 63) == 0) red[e >> 6] = wm;
@@ -185,6 +187,20 @@ __device__ int route_pair(const RouteSel &R, int t, int k, int top, bool leave)
         for (int j = 0; j < R.n_all; j++) { const float v = ch[j]; rank += (v > c || (v == c && j < e)) ? 1 : 0; }
     }
     if (live && rank == k) mine = e;
+    if (R.score_kind == 2) {          // weights: softmax over the chosen
+        if (leave) {
+            const float wm = wave_max(c);
+            __syncthreads();
+            if ((e & 63) == 0) red[e >> 6] = wm;
+            __syncthreads();
+            float mx = -INFINITY;
+            for (int w = 0; w < (int)(blockDim.x >> 6); w++) mx = fmaxf(mx, red[w]);
+            const float pe = live && rank < top ? expf(c - mx) : 0.0f, all = block_sum(pe, red);
+            if (live && rank == k) { R.idx[(size_t)t * top + k] = e; R.wgt[(size_t)t * top + k] = pe / all; }
+        }
+        __syncthreads();
+        return mine;
+    }
     float sum = 0.0f;
     if (leave && R.renorm) sum = block_sum(live && rank < top ? s : 0.0f, red);
     if (leave && live && rank == k) {
@@ -570,6 +586,17 @@ int ifa_moe_experts_routed_rows_f32(int score_kind, int renorm, float renorm_eps
 }
 
 } // extern "C"
+
+int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
+                                   const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream)
+{
+    IFA_REQUIRE(logits_f32 && rows <= 8 && experts > 0 && experts <= 256 && ldl >= (size_t)experts, "moe_experts_gated_top_rows: %zu rows (at most 8), %d experts (at most 256)", rows, experts);
+    RouteSel R;
+    memset(&R, 0, sizeof(R));
+    R.logits = (const float *)logits_f32; R.ld = ldl; R.n_all = experts; R.score_kind = 2; R.idx = idx_dev; R.wgt = (float *)wgt_f32;
+    return moe_experts("moe_experts_gated_top_rows", 1, 0, 0.0f, h_f32, ldh, rows, width, ff, experts, 0, top, 0, gate_up_bf16, down_bf16, idx_dev, wgt_f32, 1, ws, ws_bytes, y_f32, ldy,
+                       accumulate, stream, &R);
+}
 
 bool ifa_moe_gated_reads_bf16(size_t rows, int width, int ff, int top, int ops32, const void *gate_up_bf16, const void *down_bf16)
 {
