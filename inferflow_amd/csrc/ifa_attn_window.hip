@@ -82,20 +82,58 @@ __device__ __forceinline__ void attn_row(const WinAttnArgs &P, const FreshRow &F
     __shared__ float red[17];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int dim = P.dim, vdim = P.vdim, g = h / (P.heads / P.kv_heads);
+    // FRESH: the query first, then the first keys and values, whose places do not depend on it: they are on their way under its norm, and a chunk's values under the scores of its keys
+    // (the mixers' launch of a token 8.9 -> 8.15 us; with many rows the registers for it cost more: six rows 12.1 -> 13.9)
+    const float *qr = P.q + (size_t)t * P.ldq + (size_t)h * dim;
+    float qv[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) qv[e] = e == 0 || 256 * e < dim ? qr[min(tid + 256 * e, dim - 1)] : 0.0f;
     const SeqDesc sd = P.seqs[P.row_seq[t]];
     const int i = sd.pos0 + t - sd.row0;
+    gfloat *own_k = nullptr, *own_v = nullptr;
+    if constexpr (FRESH) { own_k = (gfloat *)F.k + (size_t)g * dim; own_v = (gfloat *)F.v + (size_t)g * vdim; }
+    const int lo = max(0, i - P.window + 1), nkeep = min(P.keep_first, lo), nk = nkeep + (i - lo + 1);
+    const size_t kvd = (size_t)P.kv_heads * dim, vvd = (size_t)P.kv_heads * vdim;
+    gfloat *kc = (gfloat *)(P.slot_base[sd.slot] + P.k_off + (size_t)g * dim), *vc = (gfloat *)(P.slot_base[sd.slot] + P.v_off + (size_t)g * vdim);
+    // 16 keys per wave and step, four lanes per key (each a quarter of the dot product in interleaved 16-byte pieces, finished by a quad sum)
+    const int nchunks = (nk + 15) / 16, sub = lane & 3;
+    const int nsplit = max(1, P.nsplit);
+    // (heads of whole 16s up to 128: the key's pieces are held; value rows VB at a time, asked for side by side -- keys past the last: the row's own, not counted)
+    constexpr int VB = WA_DPL <= 2 ? 16 : WA_DPL <= 4 ? 8 : 2;
+    const bool held = FRESH && (dim & 15) == 0 && dim <= 128;
+    f32x4w kq[8];
+    float v[VB][WA_DPL];
+    auto place = [&](int ch) { const int vi = ch * 16 + (lane >> 2); return vi < nk ? (vi < nkeep ? vi : lo + (vi - nkeep)) : i; };
+    auto key_row = [&](int j) { return FRESH && j == i ? own_k : kc + (size_t)j * kvd; };
+    auto ask_k = [&](int j) {
+        if (!held) return;
+        gfloat *kr = key_row(j);
+#pragma unroll
+        for (int u = 0; u < 8; u++) kq[u] = *(gf32x4 *)(kr + min(4 * sub + 16 * u, dim - 4));
+    };
+    auto ask_v = [&](int j, int j0) {
+#pragma unroll
+        for (int jj = 0; jj < VB; jj++) {
+            const int kj = __shfl(j, 4 * (j0 + jj), 64);
+            gfloat *vr = FRESH && kj == i ? own_v : vc + (size_t)kj * vvd;
+#pragma unroll
+            for (int e = 0; e < WA_DPL; e++) v[jj][e] = vr[min(lane + 64 * e, vdim - 1)];
+        }
+    };
+    int ch = split * 4 + wave, j = place(ch);
+    if (FRESH && ch < nchunks) { ask_k(j); __builtin_amdgcn_sched_barrier(0); ask_v(j, 0); }
+    if constexpr (FRESH) __builtin_amdgcn_sched_barrier(0);
     {
-        const float *qr = P.q + (size_t)t * P.ldq + (size_t)h * dim;
         float s = 0.0f;
-        for (int c = tid; c < dim; c += blockDim.x) s = fmaf(qr[c], qr[c], s);
+#pragma unroll
+        for (int e = 0; e < 4; e++) if (tid + 256 * e < dim) s = fmaf(qv[e], qv[e], s);
         const float r = P.norm_q ? 1.0f / sqrtf(block_sum(s, red) / (float)dim + P.eps) : 1.0f;
-        for (int c = tid; c < dim; c += blockDim.x) qn[c] = qr[c] * r;
+#pragma unroll
+        for (int e = 0; e < 4; e++) if (tid + 256 * e < dim) qn[tid + 256 * e] = qv[e] * r;
     }
     __syncthreads();
-    gfloat *own_k = nullptr, *own_v = nullptr;
     float own_r = 1.0f;
     if constexpr (FRESH) {
-        own_k = (gfloat *)F.k + (size_t)g * dim; own_v = (gfloat *)F.v + (size_t)g * vdim;
         if (F.norm_k) {
             float s = 0.0f;
             for (int c = tid; c < dim; c += blockDim.x) s = fmaf(own_k[c], own_k[c], s);
@@ -107,30 +145,33 @@ __device__ __forceinline__ void attn_row(const WinAttnArgs &P, const FreshRow &F
             for (int c = tid; c < vdim; c += blockDim.x) vd[c] = own_v[c];
         }
     }
-    const int lo = max(0, i - P.window + 1), nkeep = min(P.keep_first, lo), nk = nkeep + (i - lo + 1);
-    const size_t kvd = (size_t)P.kv_heads * dim, vvd = (size_t)P.kv_heads * vdim;
-    gfloat *kc = (gfloat *)(P.slot_base[sd.slot] + P.k_off + (size_t)g * dim), *vc = (gfloat *)(P.slot_base[sd.slot] + P.v_off + (size_t)g * vdim);
     float m = -INFINITY, l = 0.0f, acc[WA_DPL];
 #pragma unroll
     for (int e = 0; e < WA_DPL; e++) acc[e] = 0.0f;
-    // 16 keys per wave and step, four lanes per key (each a quarter of the dot product in interleaved 16-byte pieces, finished by a quad sum)
-    const int nchunks = (nk + 15) / 16, sub = lane & 3;
-    const int nsplit = max(1, P.nsplit);
-    for (int ch = split * 4 + wave; ch < nchunks; ch += 4 * nsplit) {
-        const int vi = ch * 16 + (lane >> 2);
-        const bool valid = vi < nk;
-        const int j = valid ? (vi < nkeep ? vi : lo + (vi - nkeep)) : i;
-        gfloat *kr = FRESH && j == i ? own_k : kc + (size_t)j * kvd;
+    while (ch < nchunks) {
+        const int next = ch + 4 * nsplit;
+        const bool valid = ch * 16 + (lane >> 2) < nk;
         float s = 0.0f;
-        if ((dim & 3) == 0) {
-#pragma unroll 8
-            for (int c = 4 * sub; c < dim; c += 16) {
-                const f32x4w kv = *(gf32x4 *)(kr + c);
-                s = fmaf(qn[c], kv.x, s); s = fmaf(qn[c + 1], kv.y, s); s = fmaf(qn[c + 2], kv.z, s); s = fmaf(qn[c + 3], kv.w, s);
+        if (held) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int c = 4 * sub + 16 * u;
+                if (c < dim) { s = fmaf(qn[c], kq[u].x, s); s = fmaf(qn[c + 1], kq[u].y, s); s = fmaf(qn[c + 2], kq[u].z, s); s = fmaf(qn[c + 3], kq[u].w, s); }
             }
         } else {
-            for (int c = sub; c < dim; c += 4) s = fmaf(qn[c], kr[c], s);
+            gfloat *kr = key_row(j);
+            if ((dim & 3) == 0) {
+#pragma unroll 8
+                for (int c = 4 * sub; c < dim; c += 16) {
+                    const f32x4w kv = *(gf32x4 *)(kr + c);
+                    s = fmaf(qn[c], kv.x, s); s = fmaf(qn[c + 1], kv.y, s); s = fmaf(qn[c + 2], kv.z, s); s = fmaf(qn[c + 3], kv.w, s);
+                }
+            } else {
+                for (int c = sub; c < dim; c += 4) s = fmaf(qn[c], kr[c], s);
+            }
         }
+        const int jn = place(next);
+        if (FRESH && next < nchunks) ask_k(jn);
         s = quad_sum(s) * P.scale;
         if (FRESH && j == i) s *= own_r;
         if (P.softcap > 0.0f) s = P.softcap * tanhf(s / P.softcap);
@@ -143,17 +184,8 @@ __device__ __forceinline__ void attn_row(const WinAttnArgs &P, const FreshRow &F
 #pragma unroll
         for (int e = 0; e < WA_DPL; e++) acc[e] *= corr;
         m = m_new;
-        // value rows VB at a time, asked for side by side (keys past the last: the row's own, not counted): one after the other they were 16 trips to memory
-        constexpr int VB = WA_DPL <= 2 ? 16 : WA_DPL <= 4 ? 8 : 2;
         for (int j0 = 0; j0 < 16; j0 += VB) {
-            float v[VB][WA_DPL];
-#pragma unroll
-            for (int jj = 0; jj < VB; jj++) {
-                const int kj = __shfl(j, 4 * (j0 + jj), 64);
-                gfloat *vr = FRESH && kj == i ? own_v : vc + (size_t)kj * vvd;
-#pragma unroll
-                for (int e = 0; e < WA_DPL; e++) v[jj][e] = vr[min(lane + 64 * e, vdim - 1)];
-            }
+            if (!FRESH || j0 > 0) ask_v(j, j0);
 #pragma unroll
             for (int jj = 0; jj < VB; jj++) {
                 const float pj = __shfl(p, 4 * (j0 + jj), 64);
@@ -161,6 +193,8 @@ __device__ __forceinline__ void attn_row(const WinAttnArgs &P, const FreshRow &F
                 for (int e = 0; e < WA_DPL; e++) acc[e] = ch * 16 + j0 + jj < nk ? fmaf(pj, v[jj][e], acc[e]) : acc[e];
             }
         }
+        if (FRESH && next < nchunks) ask_v(jn, 0);
+        ch = next; j = jn;
     }
     if (lane == 0) { wm[wave] = m; wl[wave] = l; }
 #pragma unroll

@@ -1,6 +1,7 @@
 // ifa_rows_fused.hip -- what follows the mixers in a layer of PARALLEL wiring, for a step of one token: the shares of the attention joined, the gated norm of
 // the recurrent mixer, the gated feed-forward's activation and the three products that add into the residual, in one launch.
-// Such a step is bound by its launches: one that does next to nothing takes 4-6 us here, and these were six of the eleven of a layer (33 us; this one 10 at width 1024, of them 2 for its 10 MB of weights).
+// Such a step is bound by its launches: one that does next to nothing takes 4-6 us here, and these were six of the eleven of a layer (33 us; this one 8.9 at width 1024, of them 2 for its 10 MB of weights; 9.8 with the gates, the shares and the residual asked for behind the
+// weights).
 // A workgroup forms the whole activation row for itself (10-40 KB of operands out of the L2, behind its own weight requests) and its four waves take an
 // output row each; a wave's weights (up to 24 KB a row) are asked for before anything else.
 #include "ifa_rows_fused.h"
@@ -35,6 +36,39 @@ __global__ void __launch_bounds__(256) k_row_out(IfaRowOut P)
             const int c = min(4 * tid + 1024 * j, P.k2 - 4);
             gt[j] = *reinterpret_cast<const float4 *>(P.gate_up + c); up[j] = *reinterpret_cast<const float4 *>(P.gate_up + P.k2 + c);
         }
+    // ... and so are the gates, the norm's weights, the residual and the first 1024 columns' shares: behind the weights each of them was a further trip to the cache
+    float4 gv4[4];
+    uint2 nw[4];
+    if (P.k1)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (1024 * j < P.k1) {
+                const int c = min(4 * tid + 1024 * j, P.k1 - 4);
+                gv4[j] = *reinterpret_cast<const float4 *>(P.gate + c);
+                if (P.wlen % 4 == 0) nw[j] = *reinterpret_cast<const uint2 *>(P.norm_w + c % P.wlen);
+                else {
+                    uint32_t u[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) u[e] = P.norm_w[(c + e) % P.wlen];
+                    nw[j] = make_uint2(u[0] | (u[1] << 16), u[2] | (u[3] << 16));
+                }
+            }
+    const bool joined = P.k0 && P.nsplit > 1 && P.vdim % 4 == 0;
+    float m8[IFA_ROW_OUT_SPLITS], l8[IFA_ROW_OUT_SPLITS], snk8 = -INFINITY;
+    float2 v8[IFA_ROW_OUT_SPLITS][2];
+    if (joined) {
+        const int c = min(4 * tid, P.k0 - 4), h = c / P.vdim;
+        const float *src = P.a0 + (size_t)h * P.nsplit * (P.vdim + 2);
+#pragma unroll
+        for (int s = 0; s < IFA_ROW_OUT_SPLITS; s++) {
+            const float *at = src + (size_t)min(s, P.nsplit - 1) * (P.vdim + 2);
+            const float2 ml = *reinterpret_cast<const float2 *>(at);
+            m8[s] = ml.x; l8[s] = ml.y;
+            v8[s][0] = *reinterpret_cast<const float2 *>(at + 2 + c % P.vdim); v8[s][1] = *reinterpret_cast<const float2 *>(at + 4 + c % P.vdim);
+        }
+        if (P.sink) snk8 = bf2f(P.sink[h]);
+    }
+    const float xn = P.x[n], l1 = bf2f(P.ls1[n]), l2 = P.k2 ? bf2f(P.ls2[n]) : 0.0f, b2 = P.k2 ? bf2f(P.bias2[n]) : 0.0f;
     __builtin_amdgcn_sched_barrier(0);
     u32x4r w[NP];
 #pragma unroll
@@ -44,12 +78,25 @@ __global__ void __launch_bounds__(256) k_row_out(IfaRowOut P)
         w[p] = *reinterpret_cast<const u32x4r *>(row);
     }
     __builtin_amdgcn_sched_barrier(0);
-    const float xn = P.x[n], l1 = bf2f(P.ls1[n]), l2 = P.k2 ? bf2f(P.ls2[n]) : 0.0f, b2 = P.k2 ? bf2f(P.bias2[n]) : 0.0f;
     if (P.k0 && P.nsplit <= 1) {
 #pragma unroll
         for (int j = 0; j < 4; j++) if (4 * tid + 1024 * j < P.k0) *reinterpret_cast<float4 *>(act + 4 * tid + 1024 * j) = a0[j];
     } else {
-        for (int c = tid; c < P.k0; c += 256) {
+        if (joined && 4 * tid < P.k0) {
+            float M = snk8;
+#pragma unroll
+            for (int s = 0; s < IFA_ROW_OUT_SPLITS; s++) M = fmaxf(M, m8[s]);
+            float L = P.sink ? expf(snk8 - M) : 0.0f, a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < IFA_ROW_OUT_SPLITS; s++)
+                if (s < P.nsplit) {
+                    const float f = m8[s] == -INFINITY ? 0.0f : expf(m8[s] - M);
+                    L = fmaf(l8[s], f, L);
+                    a[0] = fmaf(v8[s][0].x, f, a[0]); a[1] = fmaf(v8[s][0].y, f, a[1]); a[2] = fmaf(v8[s][1].x, f, a[2]); a[3] = fmaf(v8[s][1].y, f, a[3]);
+                }
+            *reinterpret_cast<float4 *>(act + 4 * tid) = make_float4(a[0] / L, a[1] / L, a[2] / L, a[3] / L);
+        }
+        for (int c = joined ? 1024 + tid : tid; c < P.k0; c += 256) {
             const int h = c / P.vdim, d = c % P.vdim;
             const float *src = P.a0 + (size_t)h * P.nsplit * (P.vdim + 2);
             float m[IFA_ROW_OUT_SPLITS], l[IFA_ROW_OUT_SPLITS], v[IFA_ROW_OUT_SPLITS];
@@ -93,10 +140,9 @@ __global__ void __launch_bounds__(256) k_row_out(IfaRowOut P)
             if (!whole) for (int x = P.group / 8; x > 0; x >>= 1) s += __shfl_xor(s, x, 64);          // (a group: group / 4 lanes side by side)
             if (c < P.k1) {
                 const float r = 1.0f / sqrtf((whole ? all : s) / (float)P.group + P.eps);
-                const float4 g = *reinterpret_cast<const float4 *>(P.gate + c);
-                const float gv[4] = {g.x, g.y, g.z, g.w}, ov[4] = {o[j].x, o[j].y, o[j].z, o[j].w};
+                const float gv[4] = {gv4[j].x, gv4[j].y, gv4[j].z, gv4[j].w}, ov[4] = {o[j].x, o[j].y, o[j].z, o[j].w};
 #pragma unroll
-                for (int e = 0; e < 4; e++) act[P.k0 + c + e] = ov[e] * r * bf2f(P.norm_w[(c + e) % P.wlen]) * (P.gate_act == 0 ? sigmoid_f(gv[e]) : silu_exact(gv[e]));
+                for (int e = 0; e < 4; e++) act[P.k0 + c + e] = ov[e] * r * bf2f((bf16_t)((e < 2 ? nw[j].x : nw[j].y) >> (16 * (e & 1)))) * (P.gate_act == 0 ? sigmoid_f(gv[e]) : silu_exact(gv[e]));
             }
         }
     }
@@ -130,7 +176,7 @@ bool ifa_row_out_fits(const IfaRowOut &P)
     if (P.k1 && P.group != P.k1 && !(P.group % 4 == 0 && g4 >= 1 && g4 <= 64 && (g4 & (g4 - 1)) == 0 && P.k1 % P.group == 0)) return false;
     uintptr_t al = 0;
     if (P.k0) al |= (uintptr_t)P.w0 | (uintptr_t)P.a0;
-    if (P.k1) al |= (uintptr_t)P.w1 | (uintptr_t)P.o | (uintptr_t)P.gate;
+    if (P.k1) al |= (uintptr_t)P.w1 | (uintptr_t)P.o | (uintptr_t)P.gate | 2 * (uintptr_t)P.norm_w;          // (8 bytes)
     if (P.k2) al |= (uintptr_t)P.w2 | (uintptr_t)P.gate_up;
     return (al & 15) == 0;
 }
