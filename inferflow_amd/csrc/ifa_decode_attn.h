@@ -610,6 +610,9 @@ __global__ void __launch_bounds__(256) k_dec_attn(const half_t *pq, const uint8_
 // Bound by the chains of a pass behind each launch, not by the bytes (8-bit cache of 2900 keys: 25 MB a layer, 5 us).  As three kernels -- every split summed the whole
 // row's exponentials again, the outputs were added up by a launch of their own -- 8.3 + 9.9 + 5.0 us a layer; a token at 600 / 2900 / 6000 keys 1591 -> 1573, 1896 -> 1831,
 // 2191 -> 2074 us (8-bit cache).  Twice the splits for the scores alone: 1858 at 2900.
+// Four 8-bit codes to halves at a time (one by one: a third of either launch's instructions), sums and scores asked for in front of the V rows, two batches of those under way: 8.8 + 11.1
+// -> 8.2 + 10.6 us a layer at 2900 keys (12 tokens 21650 -> 21220 us; F16 cache 1799 -> 1758 a token).  Sixteen lanes a key for the scores (whole rows a request, as in the batched
+// kernel): 11.2 with 8, 12.5 with 16 requests under way.
 constexpr int DEC_ATTN_MAX_SPLITS = 32;      // splits per head are chosen per decode call from the context it will reach
 
 struct DecAttnSplitWs {
@@ -767,17 +770,22 @@ __global__ void __launch_bounds__(256) k_dec_attn_scores(const DecAttnParams P, 
         } else {
             const uint8_t *rowp = P.kcache + (size_t)j * row_bytes + head_off;
             if constexpr (QW) {
-                // byte B (compile-time) of the slice held in registers; block b = bytes [34 b, 34 b + 34): scale (half), 32 codes
-                auto kb = [&](int B) -> uint32_t { return (kqc[B >> 2] >> (8 * (B & 3))) & 0xFFu; };
+                // the slice held in registers; block b = bytes [34 b, 34 b + 34): scale (half), 32 codes, four of them to halves at a time (q8x4_dequant_h)
 #pragma unroll
                 for (int b = 0; b < HD / 32; b++) {
-                    const float sc = hbits2f((uint16_t)(kb(34 * b) | (kb(34 * b + 1) << 8)));
+                    const half_t sch = __builtin_bit_cast(half_t, (uint16_t)(kqc[(34 * b) >> 2] >> (8 * ((34 * b) & 3))));
+                    const half2_t sc2 = {sch, sch};
 #pragma unroll
-                    for (int i = 0; i < 16; i++) {
-                        const uint32_t two = kb(34 * b + 2 + 2 * i) | (kb(34 * b + 3 + 2 * i) << 8);
-                        const float k0 = h2f(f2h((float)(int)(int8_t)(two & 0xFF) * sc)), k1 = h2f(f2h((float)(int)(int8_t)(two >> 8) * sc));
-                        c = __builtin_fmaf((float)qreg[(b * 32 + 2 * i) >> 3][(2 * i) & 7], k0, c);
-                        c = __builtin_fmaf((float)qreg[(b * 32 + 2 * i + 1) >> 3][(2 * i + 1) & 7], k1, c);
+                    for (int w4 = 0; w4 < 8; w4++) {
+                        constexpr int last = KBYTES / 4 - 1;
+                        const int B0 = 34 * b + 2 + 4 * w4, d = 32 * b + 4 * w4;
+                        const uint32_t cw = (B0 & 3) == 0 ? kqc[B0 >> 2] : __builtin_amdgcn_alignbyte(kqc[(B0 >> 2) + 1 < last ? (B0 >> 2) + 1 : last], kqc[B0 >> 2], B0 & 3);
+                        half2_t lo, hi;
+                        q8x4_dequant_h(cw, sc2, lo, hi);
+                        c = __builtin_fmaf((float)qreg[d >> 3][d & 7], (float)lo[0], c);
+                        c = __builtin_fmaf((float)qreg[d >> 3][(d & 7) + 1], (float)lo[1], c);
+                        c = __builtin_fmaf((float)qreg[d >> 3][(d & 7) + 2], (float)hi[0], c);
+                        c = __builtin_fmaf((float)qreg[d >> 3][(d & 7) + 3], (float)hi[1], c);
                     }
                 }
             } else if constexpr (Q8) {
@@ -860,14 +868,26 @@ __global__ void __launch_bounds__(256) k_dec_attn_pv(const DecAttnParams P, cons
             }
         }
     };
-    const int jv0 = vact ? j0 + sp : j1;
-    if (jv0 < j1) load_v(vcur, qs_c, qc_c, jv0);
-    // the row's maximum and sum from its splits': lane s holds split s (sum 0: no keys, or scores of -inf only; a NaN among the scores is in the sum, not in the maximum)
+    // (the splits' sums and this split's first scores in front of them: they come out of the caches, and requests return in order)
     const int ns = ws.nsplits;
     const float *ml = ws.ml + 2 * (size_t)(h * ns + min(lane, ns - 1));
-    const float ms = ml[0], lsv = ml[1], mx = wave_max(ms);
+    const float ms = ml[0], lsv = ml[1];
+    const int jlast = max(j1 - 1, 0);
+    const half_t s_in[2] = {Sg[min(j0 + tid, jlast)], Sg[min(j0 + tid + 256, jlast)]};
+    const int jv0 = vact ? j0 + sp : j1;
+    __builtin_amdgcn_sched_barrier(0);
+    load_v(vcur, qs_c, qc_c, min(jv0, jlast));
+    load_v(vnxt, qs_n, qc_n, min(jv0 + VB * step, jlast));
+    __builtin_amdgcn_sched_barrier(0);
+    // the row's maximum and sum from its splits': lane s holds split s (sum 0: no keys, or scores of -inf only; a NaN among the scores is in the sum, not in the maximum)
+    const float mx = wave_max(ms);
     const float inv = 1.0f / wave_sum(lane < ns && lsv != 0.0f ? expf(ms - mx) * lsv : 0.0f);
-    for (int j = j0 + tid; j < j1; j += 256) {
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+        const half_t eh = f2h(expf(P.kq_scale * h2f(s_in[x]) - mx));
+        if (j0 + tid + 256 * x < j1) Pl[tid + 256 * x] = f2h(h2f(eh) * inv);
+    }
+    for (int j = j0 + tid + 512; j < j1; j += 256) {
         const half_t eh = f2h(expf(P.kq_scale * h2f(Sg[j]) - mx));
         Pl[j - j0] = f2h(h2f(eh) * inv);
     }
@@ -875,36 +895,33 @@ __global__ void __launch_bounds__(256) k_dec_attn_pv(const DecAttnParams P, cons
     float o[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) o[i] = 0.0f;
-    // batches of VB keys of this thread's sequence (j, j + NSPLIT, ...): the next batch is requested before the current one is
-    // multiplied; rows past the split are clamped and skipped -- the order of accumulation is that of a plain loop
-    for (int j = jv0; j < j1; j += VB * step) {
-        const bool more = j + VB * step < j1;
-        if (more) load_v(vnxt, qs_n, qc_n, j + VB * step);
+    // batches of VB keys of this thread's sequence (j, j + NSPLIT, ...), two of them under way: a batch's registers take the one after the next; rows past the split are clamped and
+    // skipped -- the order of accumulation is that of a plain loop
+    auto batch = [&](u32x4 (&bv)[Q8 ? 1 : VB], uint32_t (&bs)[Q8 ? VB : 1], uint32_t (&bc)[Q8 ? VB : 1][2], int j) {
 #pragma unroll
         for (int u = 0; u < VB; u++) {
             if (j + u * step >= j1) break;
             const float pu = h2f(Pl[j + u * step - j0]);
             if constexpr (Q8) {
-                const float sc = hbits2f((uint16_t)qs_c[u]);
+                const half_t sc = __builtin_bit_cast(half_t, (uint16_t)bs[u]);
+                half2_t v[4];
+                q8x4_dequant_h(bc[u][0], half2_t{sc, sc}, v[0], v[1]); q8x4_dequant_h(bc[u][1], half2_t{sc, sc}, v[2], v[3]);
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const uint32_t two = (qc_c[u][e >> 1] >> (16 * (e & 1))) & 0xFFFFu;
-                    o[2 * e] = __builtin_fmaf(pu, h2f(f2h((float)(int)(int8_t)(two & 0xFF) * sc)), o[2 * e]);
-                    o[2 * e + 1] = __builtin_fmaf(pu, h2f(f2h((float)(int)(int8_t)(two >> 8) * sc)), o[2 * e + 1]);
+                    o[2 * e] = __builtin_fmaf(pu, (float)v[e][0], o[2 * e]);
+                    o[2 * e + 1] = __builtin_fmaf(pu, (float)v[e][1], o[2 * e + 1]);
                 }
             } else {
-                const half8_t v8 = __builtin_bit_cast(half8_t, vcur[u]);
+                const half8_t v8 = __builtin_bit_cast(half8_t, bv[u]);
 #pragma unroll
                 for (int e = 0; e < 8; e++) o[e] = __builtin_fmaf(pu, (float)v8[e], o[e]);
             }
         }
-        if (more) {
-#pragma unroll
-            for (int u = 0; u < VB; u++) {
-                if constexpr (Q8) { qs_c[u] = qs_n[u]; qc_c[u][0] = qc_n[u][0]; qc_c[u][1] = qc_n[u][1]; }
-                else vcur[u] = vnxt[u];
-            }
-        }
+        if (j + 2 * VB * step < j1) load_v(bv, bs, bc, j + 2 * VB * step);
+    };
+    for (int j = jv0; j < j1; j += 2 * VB * step) {
+        batch(vcur, qs_c, qc_c, j);
+        if (j + VB * step < j1) batch(vnxt, qs_n, qc_n, j + VB * step);
     }
     if (vact) {
 #pragma unroll
