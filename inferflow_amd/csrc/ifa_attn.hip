@@ -499,6 +499,8 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass(const half_t *__rest
     // scores of key block kb for this wave's 32 queries: x[r] = kq_scale * half(alpha * q.k (+ ALiBi)), key = 32 kb + row(r)
     // scores of key block kb for this wave's 32 queries:  x[r] = half(alpha * q.k (+ ALiBi)) as float,  key = 32 kb + row(r);
     // masked keys: -inf.  exp(kq_scale * x - max) is then exp2(fma(log2(e) * kq_scale, x, c)) with c = -log2(e) * kq_scale * max.
+    // (ALiBi is a template parameter: its test inside the unrolled loop was sixteen branches a block.  Scores and probabilities stay pairs of halves, converted and compared two at a time:
+    // 32 heads of 128, 2048 tokens 147 -> 125 -> 120 us, 512 tokens 26 -> 22, 512 behind 1500 82 -> 65)
     // (the kernel is VALU-bound -- ~10 instructions per score and pass against 16 MFMAs per 512 scores -- so the mask is
     // applied only in blocks that reach past the wave's first query, and the exponent is one fma + v_exp_f32)
     const float l2e_kq = 1.44269504088896341f * kq_scale;
@@ -612,11 +614,11 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass(const half_t *__rest
     }
 }
 
-template <int HD, bool Q8>
+template <int HD, bool Q8, bool ALIBI>
 __global__ void __launch_bounds__(256, 2) k_attention_2pass_ks(const half_t *__restrict__ q, const uint8_t *__restrict__ kc,
                                                          const uint8_t *__restrict__ vc, int n_ctx, int q_tokens,
                                                          int prefix_len, int heads, int kv_heads, float kq_scale,
-                                                         int alibi, int alibi_base, int alibi_total, half_t *__restrict__ out)
+                                                         int alibi_base, int alibi_total, half_t *__restrict__ out)
 {
     static_assert(HD == 128 || HD == 64, "two-pass attention: head_dim 64 / 128");
     constexpr int KS = HD / 16, NT = HD / 32, CHK = HD / 8;
@@ -649,7 +651,7 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass_ks(const half_t *__r
     const int wave_keys = tw < q_tokens ? min(n_ctx, prefix_len + min(tw + 32, q_tokens)) : 0;
     const int wave_nkb = (wave_keys + 31) / 32;                                   // blocks past it are fully masked for this wave
     const float alpha = 1.0f / sqrtf((float)HD) / kq_scale;
-    const float mk = alibi ? alibi_slope(h + alibi_base, alibi_total) : 0.0f;
+    const float mk = ALIBI ? alibi_slope(h + alibi_base, alibi_total) : 0.0f;
 
     half8v qf[KS];
     {
@@ -660,7 +662,20 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass_ks(const half_t *__r
     }
     // ---- staging: K block rows as they are (swizzled chunks), V block transposed with permuted key columns
     half8v kreg[2][NKC];
+    // A pair of whole blocks inside the context: the pair's place is a scalar, a lane's place in it does not change (F16 cache; row by row every request cost a multiplication of 16 cycles)
+    auto whole = [&](int itn) { return !Q8 && 64 * itn + 64 <= n_ctx && 2 * itn + 1 < nkb; };
+    auto load_at = [&](const uint8_t *base, int row, int c) {
+        return __builtin_bit_cast(half8v, *reinterpret_cast<const u32x4v *>(base + ((uint32_t)row * (uint32_t)row_bytes + (uint32_t)(2 * (hoff + 8 * c)))));
+    };
     auto kload = [&](int itn) {
+        if (whole(itn)) {
+            const uint8_t *base = kc + (size_t)(64 * itn) * row_bytes;
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int it = 0; it < NKC; it++) { const int idx = tid + it * 256; kreg[p][it] = load_at(base, 32 * p + idx / CHK, idx % CHK); }
+            return;
+        }
 #pragma unroll
         for (int p = 0; p < 2; p++) {
             const int kb = min(2 * itn + p, nkb - 1);
@@ -687,6 +702,14 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass_ks(const half_t *__r
     const int vch = ((tid >> 4) & 3) + 4 * ((tid >> 6) % (CHK / 4));
     const int vkey0 = 16 * ((tid >> 6) / (CHK / 4)) + 2 * vpair;                  // even key of the lane pair within a pass
     auto vload = [&](int itn) {
+        if (whole(itn)) {
+            const uint8_t *base = vc + (size_t)(64 * itn) * row_bytes;
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int it = 0; it < NIT; it++) vreg[p][it] = load_at(base, 32 * p + min(vkey0 + vpar + it * KPI, 31), vch);
+            return;
+        }
 #pragma unroll
         for (int p = 0; p < 2; p++) {
             const int kb = min(2 * itn + p, nkb - 1);
@@ -727,7 +750,10 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass_ks(const half_t *__r
     // applied only in blocks that reach past the wave's first query, and the exponent is one fma + v_exp_f32)
     const float l2e_kq = 1.44269504088896341f * kq_scale;
     const int full_keys = tw < q_tokens ? min(n_ctx, prefix_len + tw + 1) : 0;   // every query of the wave sees keys below this
-    auto scores = [&](int kb, int buf, float (&x)[16]) {
+    typedef _Float16 f16x2v __attribute__((ext_vector_type(2)));
+    typedef float f32x2v __attribute__((ext_vector_type(2)));
+    auto pair = [](float a, float b) { return __builtin_convertvector((f32x2v{a, b}), f16x2v); };      // (both rounded to nearest in one instruction)
+    auto scores = [&](int kb, int buf, f16x2v (&x)[8]) {
         const char *Ks = KsP(buf, kp);
         f32x16v acc;
 #pragma unroll
@@ -738,15 +764,17 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass_ks(const half_t *__r
             acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[s2], acc, 0, 0, 0);
         }
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            half_t sv = f2h(alpha * acc[r]);
-            if (alibi) sv = f2h((float)(32 * kb + (r & 3) + 8 * (r >> 2) + 4 * g) * mk + h2f(sv));
-            x[r] = h2f(sv);
+        for (int r = 0; r < 8; r++) {
+            x[r] = pair(alpha * acc[2 * r], alpha * acc[2 * r + 1]);
+            if constexpr (ALIBI) {
+                const int key = 32 * kb + ((2 * r) & 3) + 8 * (r >> 1) + 4 * g;
+                x[r] = pair((float)key * mk + (float)x[r][0], (float)(key + 1) * mk + (float)x[r][1]);
+            }
         }
         if (32 * kb + 32 > full_keys) {                   // (wave-uniform: only the blocks on the causal edge)
 #pragma unroll
             for (int r = 0; r < 16; r++)
-                if (32 * kb + (r & 3) + 8 * (r >> 2) + 4 * g >= n_valid) x[r] = -INFINITY;
+                if (32 * kb + (r & 3) + 8 * (r >> 2) + 4 * g >= n_valid) x[r >> 1][r & 1] = (_Float16)-INFINITY;
         }
     };
     auto exp2_fast = [](float v) { return __builtin_amdgcn_exp2f(v); };
@@ -762,16 +790,17 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass_ks(const half_t *__r
         kstage((itn + 1) & 1);               // (the next pair of blocks, or a harmless repeat of the last one)
         kload(min(itn + 2, nit - 1));
         if (kb < wave_nkb && kb < nkb) {
-            float x[16];
+            f16x2v x[8];
             scores(kb, itn & 1, x);
-            float bm = x[0];
+            f16x2v b2 = x[0];
 #pragma unroll
-            for (int r = 1; r < 16; r++) bm = fmaxf(bm, x[r]);
+            for (int r = 1; r < 8; r++) b2 = __builtin_elementwise_max(b2, x[r]);
+            const float bm = fmaxf((float)b2[0], (float)b2[1]);
             if (bm > m) { sum *= exp2_fast(l2e_kq * (m - bm)); m = bm; }             // (m = -inf: sum is 0 and stays 0)
             if (m > -INFINITY) {
                 const float c = -l2e_kq * m;
 #pragma unroll
-                for (int r = 0; r < 16; r++) sum += exp2_fast(__builtin_fmaf(l2e_kq, x[r], c));   // masked: 2^-inf = 0
+                for (int r = 0; r < 16; r++) sum += exp2_fast(__builtin_fmaf(l2e_kq, (float)x[r >> 1][r & 1], c));   // masked: 2^-inf = 0
             }
         }
         __syncthreads();
@@ -819,14 +848,15 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass_ks(const half_t *__r
         vload(min(itn + 2, nit - 1));
         if (kb < wave_nkb && kb < nkb) {
             const half_t *Vt = VtP(itn & 1, kp);
-            float x[16];
+            f16x2v x[8];
             scores(kb, itn & 1, x);
             half8v pb[2];
             const float c = M > -INFINITY ? -l2e_kq * M : 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const half_t e = f2h(exp2_fast(__builtin_fmaf(l2e_kq, x[r], c)));       // masked keys: 2^-inf = 0
-                pb[r >> 3][r & 7] = f2h(h2f(e) * inv);
+            for (int r = 0; r < 8; r++) {
+                const f16x2v e = pair(exp2_fast(__builtin_fmaf(l2e_kq, (float)x[r][0], c)), exp2_fast(__builtin_fmaf(l2e_kq, (float)x[r][1], c)));       // masked keys: 2^-inf = 0
+                const f16x2v w = pair((float)e[0] * inv, (float)e[1] * inv);
+                pb[r >> 2][2 * (r & 3)] = w[0]; pb[r >> 2][2 * (r & 3) + 1] = w[1];
             }
 #pragma unroll
             for (int s2 = 0; s2 < 2; s2++)
@@ -985,10 +1015,10 @@ extern "C" int ifa_attention(const void *q, const void *kcache, const void *vcac
         hipStream_t hs = ifa_s(stream);
         dim3 grid((unsigned)((q_tokens + 63) / 64), (unsigned)heads);
         const size_t smem = (size_t)4 * 32 * head_dim * 2 + (size_t)4 * head_dim * F2_VROW * 2;
-#define IFA_F2K(HDV, Q8V) { auto kern = k_attention_2pass_ks<HDV, Q8V>; \
+#define IFA_F2K(HDV, Q8V) { const auto kern = alibi ? k_attention_2pass_ks<HDV, Q8V, true> : k_attention_2pass_ks<HDV, Q8V, false>; \
         if (smem > 48 * 1024) IFA_HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem)); \
         kern<<<grid, dim3(256), smem, hs>>>((const half_t *)q, (const uint8_t *)kcache, (const uint8_t *)vcache, n_ctx, q_tokens, \
-                                            prefix_len, heads, kv_heads, kq_scale, alibi, alibi_base_head, total_heads, (half_t *)out); }
+                                            prefix_len, heads, kv_heads, kq_scale, alibi_base_head, total_heads, (half_t *)out); }
         if (head_dim == 128) { if (kv_dtype == Q8_B32T2) IFA_F2K(128, true) else IFA_F2K(128, false) }
         else { if (kv_dtype == Q8_B32T2) IFA_F2K(64, true) else IFA_F2K(64, false) }
 #undef IFA_F2K
