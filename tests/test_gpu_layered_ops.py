@@ -105,6 +105,38 @@ def test_embedding_with_sinusoid_norms_glu_argmax():
     assert list(b) == [int(r.argmax()) for r in masked] and b[2] == 250
 
 
+@pytest.mark.parametrize("C_,gdim,nq,nsc,lens", [(40, 8, 16, 8, [(70, 1, 33), (2, 64, 1), (65, 3, 90)]), (1100, 64, 640, 320, [(3, 90, 1), (61, 2, 2), (1, 1, 100)]),
+                                                 (2052, 256, 512, 256, [(1500, 700, 1), (1, 5, 2100)]), (72, 0, 0, 0, [(64, 1, 2)])])
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_short_convolution_of_prompts(taps, C_, gdim, nq, nsc, lens):
+    """steps of at least 64 rows: two and eight rows a workgroup, sequences that begin and end inside a workgroup's rows and are shorter than the taps, tails carried from step to step,
+    channels in several workgroups and past the last whole one, norm groups of 8 to 256 channels and none"""
+    rng = np.random.default_rng(taps + C_)
+    w = orc.bf16_round(0.5 * rng.standard_normal((C_, taps)))
+    full = {s: rng.standard_normal((sum(l[s] for l in lens), C_ + 4)).astype(np.float32) for s in (0, 1, 2)}
+    want = {}
+    for s, xs in full.items():
+        y = orc.silu(orc.short_conv(orc.t64(xs[:, :C_]), orc.t64(w)))
+        if nq:
+            y[:, :nq] = orc.unit_vectors(y[:, :nq].reshape(-1, nq // gdim, gdim)).reshape(-1, nq)
+        y[:, :nsc] *= 0.25
+        want[s] = y.numpy()
+    sl, at = Slots(3, (taps - 1) * C_), {0: 0, 1: 0, 2: 0}
+    for step in lens:
+        seqs = [(n, at[s], s) for s, n in ((2, step[2]), (0, step[0]), (1, step[1]))]
+        x = np.concatenate([full[s][at[s]:at[s] + n] for n, _, s in seqs], 0)
+        d, rs, T = seq_tables(seqs)
+        assert T >= 64
+        y, xd = torch.full((T, C_ + 4), 7.0, dtype=torch.float32, device="cuda"), dev32(x)
+        ia.check(capi().ifa_shortconv_silu_f32(p(xd), C_ + 4, C_, taps, p(devbf(w)), p(d), p(rs), T, p(sl.table), 0, nq, gdim, 1e-6, nsc, 0.25, p(y), C_ + 4, stream()))
+        ia.check(capi().ifa_shortconv_tail_f32(p(xd), C_ + 4, C_, taps, p(d), len(seqs), p(sl.table), 0, stream()))
+        sync()
+        got, r = y.cpu().numpy(), 0
+        for n, a, s in seqs:
+            assert np.abs(got[r:r + n, :C_] - want[s][a:a + n]).max() < 1e-5 and np.all(got[r:r + n, C_:] == 7.0), (step, s)
+            at[s] += n; r += n
+
+
 @pytest.mark.parametrize("C_,gdim,nq,nsc", [(40, 8, 16, 8), (1100, 100, 600, 300)])      # (the second: a row's channels in two workgroups)
 @pytest.mark.parametrize("taps", [1, 2, 4])
 def test_short_convolution_with_carried_tail(taps, C_, gdim, nq, nsc):
