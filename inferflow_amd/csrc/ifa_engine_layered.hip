@@ -119,7 +119,10 @@ struct LayeredNet {
     // 128, 67 MB where 4096 tokens take 24 -- up to opt_workspace_mb each.  A step beyond that, or whose workspace cannot be had, runs without (fp32 tiles, token by token).
     float *tile_ws = nullptr; size_t tile_ws_bytes = 0;
     int opt_workspace_mb = 4096; bool step_tile_ws = false;
-    bf16_t *a16 = nullptr, *h16 = nullptr, *g16 = nullptr; size_t a16_cap = 0, h16_cap = 0, g16_cap = 0; int opt_a16_min = 17;          // activations of a prompt's product rounded to bfloat16; steps of at least this many rows (0: never)
+    bf16_t *a16 = nullptr, *h16 = nullptr, *g16 = nullptr; size_t a16_cap = 0, h16_cap = 0, g16_cap = 0; 
+    // activations of a product rounded to bfloat16 beforehand: steps of at least this many rows (0: never).  Above the eight rows whose activations stay in 32 bits; k_lin_mfma rounds the
+    // same on its way (9 / 16 tokens of Sopulorn 1561 -> 801 us / 1808 -> 1010, of Gelarax 1564 -> 642 / 1784 -> 823, 12 prompt rows of width 2048 2713 -> 979)
+    int opt_a16_min = 9;
     int opt_fuse_step = 1;                  // single-token steps of PARALLEL layers: norm inside the input product, everything behind the mixers in one launch
     int opt_attn_tile_min = 16;            // steps of at least this many rows run the windowed attention through the tiled kernel
     std::vector<ifa_seq_desc> seqs_host;   // the current step's sequences (the tiled attention's grid is sized from them)
