@@ -5,11 +5,12 @@
 // (accumulate into the 32-bit residual stream with a per-channel layer scale and a branch scale).
 //
 //   T <= 8    k_lin_rows: one wave per output row, the weight row streamed once in 16-byte pieces, all T activation rows
-//             multiplied against it in fp32 (decode steps: bound by the weight stream)
+//             multiplied against it in fp32 (decode steps: bound by the weight stream); k_lin_rows_group: two outputs a wave
+//             (large matrices, gated activations)
 //   T  > 8    k_lin_mfma: 64 x 64 output tiles, K in steps of 32 through LDS, four waves of 32 x 32 sub-tiles;
 //             OPS32 = false: operands rounded to bfloat16, v_mfma_f32_32x32x16_bf16;
 //             OPS32 = true : operands stay 32-bit, v_mfma_f32_32x32x2_f32 (the exact mode of the worker)
-//   prompts   k_lin_tile<BM, BN> (ifa_linear_bf16_both: activations rounded to bfloat16 beforehand, by their producer or by k_rows_to_bf16): tiles of up to
+//   T  > 8    k_lin_tile (ifa_linear_bf16_both, where the caller has rounded the activations: by their producer or by k_rows_to_bf16): tiles of up to
 //             128 x 128 (32 x 32 where there are few), both operands straight to LDS; the same sums in the same order as k_lin_mfma<false>
 // Accumulation is fp32 in every path.  No atomics, no split K: a result does not depend on what else runs.
 #include <algorithm>
@@ -178,10 +179,11 @@ typedef const __attribute__((address_space(1))) void lt_glb_t;
 // GLU: column tiles from P.glu_c0 on serve BN / 2 outputs of a gated feed-forward: of 32 columns of such a tile 16 are gates and 16 the ups of the same outputs, so that one
 // exchange between a wave's rows of 16 lanes brings the two together and the activation is formed here and rounded once (the same values as k_glu_to_bf16's).  The 32-bit gate | up
 // rows were written and read again by a launch of their own: 2048 rows of width 2048, 11264 of 19968 columns
-// gate | up, 237 + 23 us -> 243; 601 rows of width 1024 31.6 + 7.4 -> 32.
+// gate | up, 237 + 23 us -> 243 (207 with the tiles as they are); 601 rows of width 1024 31.6 + 7.4 -> 32 (28).
 // SUM: the parts of a sum of products one after the other in ONE pass over K: their requests run on without a break, the tile's rows of C are read and written once, and the launches
 // but one go.  At a part's last step its columns' scales and biases take it from the step's accumulators into the sum.  (22 products of
-// a Gelarax prompt in 8 launches: 2048 rows of width 2048 1268 -> 1202 us, 601 of width 1024 312 -> 309, and 14 launches less.)
+// a Gelarax prompt in 8 launches: 2048 rows of width 2048 1268 -> 1202 us (866 with the tiles as they are), 601 of width 1024 312 -> 309 (240), and 14
+// launches less.)
 constexpr int LT_GROUPED = 1, LT_GLU = 2, LT_SUM = 4;
 template <int BM, int BN, int WM, int WN, int NB, int MODE>
 __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(LinArgs P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
