@@ -1151,8 +1151,10 @@ int run_layers(ifa_model *m, size_t T, int nseq)
         const size_t NI = L.n_in;
         // (the linear attention's q | k | v leave the product through SiLU: contiguous columns [c_lq, c_lg))
         const bool lin = sp.mixer == IFA_MIX_WINDOW_LINEAR;
-        // steps of a few rows: the norm is formed inside the product's read of the residual, the gated GELU inside the down-projection's
+        // steps of a few rows: the norm is formed inside the product's read of the residual, the gated GELU inside the down-projection's (which reads gate | up, so that the first
+        // product stores them)
         const bool fuse = T <= 8 && W % 8 == 0;
+        const bool glu_inside = fuse && (n->opt_fuse_rows & 2) && sp.ffn > 0 && sp.ffn % 8 == 0 && L.c_fg % 4 == 0;
         int left = GLU_COLUMNS;
         if (fuse && (n->opt_fuse_rows & 1)) {
             if ((rc = ifa_linear_bf16w_rows(1, L.T(IFA_LT_NORM1).data, c.eps, L.w_in, NI, W, n->x, W, T, L.b_in, nullptr, 1.0f, 0, n->proj, NI,
@@ -1160,7 +1162,7 @@ int run_layers(ifa_model *m, size_t T, int nseq)
         } else {
             if ((rc = ifa_layernorm_f32(1, n->x, W, T, W, L.T(IFA_LT_NORM1).data, c.eps, n->h, W, s))) return rc;
             const int silu0 = lin ? (int)L.c_lq : 0, silu1 = lin ? (int)L.c_lg : 0;
-            if (sp.ffn > 0) rc = linear_glu(m, L.w_in, NI, W, n->h, nullptr, T, L.b_in, n->proj, NI, silu0, silu1, L.c_fg, (size_t)sp.ffn, 1, 0.0f, &left);
+            if (sp.ffn > 0 && !glu_inside) rc = linear_glu(m, L.w_in, NI, W, n->h, nullptr, T, L.b_in, n->proj, NI, silu0, silu1, L.c_fg, (size_t)sp.ffn, 1, 0.0f, &left);
             else rc = linear(m, L.w_in, NI, W, n->h, W, T, L.b_in, nullptr, 1.0f, 0, n->proj, NI, silu0, silu1);
             if (rc) return rc;
         }
@@ -1187,7 +1189,7 @@ int run_layers(ifa_model *m, size_t T, int nseq)
         }
         if (sp.ffn > 0) {
             const size_t F = (size_t)sp.ffn;
-            if (fuse && (n->opt_fuse_rows & 2) && F % 8 == 0 && L.c_fg % 4 == 0) {
+            if (glu_inside) {
                 if ((rc = ifa_linear_bf16w_rows(2, nullptr, 0.0f, L.T(IFA_LT_FFN_DOWN).data, W, F, n->proj + L.c_fg, NI, T, L.T(IFA_LT_FFN_DOWN_B).data,
                                                 L.T(IFA_LT_LS2).data, 1.0f, 1, n->x, W, 0, 0, s))) return rc;
             } else {

@@ -352,6 +352,28 @@ def test_chunked_recurrences_are_switched_off_by_0(tmp_path):
     eng.close()
 
 
+@pytest.mark.parametrize("a16_min", [9, 1])      # (1: the products over bfloat16 rows take steps of a few rows too)
+@pytest.mark.parametrize("layer", [fx.parallel_layer(heads=2, kv_heads=1, dim=32, lin_heads=2, lin_dim=16, lin_vdim=40, ff=72), fx.delta_layer(heads=2, kv_heads=1, dim=16, vdim=20, ff=200)],
+                         ids=["parallel", "delta"])      # (mixers' outputs of 80 columns, and of 40: fewer than those products take)
+def test_norm_and_activation_inside_the_products_of_a_few_rows(tmp_path, layer, a16_min):
+    """Every combination of the two (fuse_rows), each operation in a launch of its own otherwise, after a step of other values in the same buffers: one row, two, eight and a step that is too
+    large for either, against the oracle"""
+    import inferflow_amd as ia
+    cfg = fx.config([layer, layer], width=72, vocab=97)
+    w, toks = fx.random_weights(cfg, 71), tokens_for(cfg, 40, 72)
+    want = oracle_logits(cfg, w, toks)
+    eng = engine_for(tmp_path, cfg, w, "bfloat16", 64, 2)
+    for name, value in ((b"fuse_step", 0), (b"a16_min", a16_min)):
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), name, value))
+    for fused in (0, 1, 2, 3):
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"fuse_rows", fused))
+        for n in (1, 2, 8, 11):
+            run_whole(eng, tokens_for(cfg, 12, 73))
+            lg = run_whole(eng, toks[:n])[0]
+            assert fx.rel_err(lg, want[:n]).max() < (TOL32 if n <= 8 < a16_min else TOL16), (fused, n)
+    eng.close()
+
+
 @pytest.mark.parametrize("ctx", [340, 60])      # keys of a head by six workgroups whose shares the last launch joins / by one
 def test_single_token_steps_in_few_launches(tmp_path, ctx):
     """Steps of one token whose layers' sizes allow the norm inside the input product, both mixers in one launch and everything behind them in another: against the
