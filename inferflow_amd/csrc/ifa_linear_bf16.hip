@@ -40,23 +40,27 @@ struct LinArgs {
     const int *tile_map, *n_tiles, *a_rows; const float *row_scale;
     bf16_t *C16;                               // (k_lin_tile with act_kind 2: the output in bfloat16 instead of C)
     int act_kind;                              // every output after the bias passes 1: the exact (erf) GELU, 2: the square of relu
-    // (k_lin_tile, GLU) columns [glu_c0, glu_c0 + 2 glu_f) are gate | up: instead of them G16[t][c] = act(gate[c]) up[c] in bfloat16, glu_w columns (whole 64s, zero beyond glu_f)
-    // (k_lin_rows_group: in 32 bits, G)
-    bf16_t *G16; int ldg, glu_c0, glu_f, glu_w, glu_kind; float glu_limit;
-    float *G;
-    const float *row_gate; int ld_gate;        // (lin_store) row t times sigmoid(row_gate[t * ld_gate])
-    // (k_lin_tile, SUM) several products into the same columns: A's rows hold their operands side by side, each padded to whole steps; W, K, mul, bias, alpha of each here
-    struct Part { const bf16_t *W, *mul, *bias; int K, steps; float alpha; } part[IFA_SUM_PARTS];
 };
 
-__device__ __forceinline__ void lin_store(const LinArgs &P, int t, int n, float acc)
+// What only some kernels read stands in arguments of their own.  (In one struct, with the gate tested at run time, every product of a few rows took 0.05 to 0.2 us more and one of four rows
+// 0.3: 1024 x 1024, 1 / 4 / 8 rows 3.56 / 5.14 / 7.47 us against 3.63 / 5.49 / 7.70.)
+// Columns [glu_c0, glu_c0 + 2 glu_f) are gate | up.  k_lin_tile: instead of them G16[t][c] = act(gate[c]) up[c] in bfloat16, glu_w columns (whole 64s, zero beyond glu_f); k_lin_rows_group: G in
+// 32 bits
+struct LinGluArgs : LinArgs { bf16_t *G16; float *G; int ldg, glu_c0, glu_f, glu_w, glu_kind; float glu_limit; };
+// Row t times sigmoid(row_gate[t * ld_gate]) (lin_store)
+struct LinGatedArgs : LinArgs { const float *row_gate; int ld_gate; };
+// Several products into the same columns (k_lin_tile): A's rows hold their operands side by side, each padded to whole steps; W, K, mul, bias, alpha of each here
+struct LinSumArgs : LinArgs { struct Part { const bf16_t *W, *mul, *bias; int K, steps; float alpha; } part[IFA_SUM_PARTS]; };
+
+template <class Args>
+__device__ __forceinline__ void lin_store(const Args &P, int t, int n, float acc)
 {
     if (P.bias) acc += bf2f(P.bias[n]);
     if (n >= P.act_c0 && n < P.act_c1) acc = silu_exact(acc);
     if (P.act_kind == 1) acc = 0.5f * acc * (1.0f + erff(acc * 0.70710678118654752f));
     if (P.act_kind == 2) { acc = fmaxf(acc, 0.0f); acc *= acc; }
     if (P.row_scale) acc *= P.row_scale[t];
-    if (P.row_gate) acc *= sigmoid_f(P.row_gate[(size_t)t * P.ld_gate]);
+    if constexpr (std::is_same_v<Args, LinGatedArgs>) acc *= sigmoid_f(P.row_gate[(size_t)t * P.ld_gate]);
     if (P.mul) acc *= bf2f(P.mul[n]);
     acc *= P.alpha;
     float *c = P.C + (size_t)t * P.ldc + n;
@@ -185,8 +189,10 @@ typedef const __attribute__((address_space(1))) void lt_glb_t;
 // a Gelarax prompt in 8 launches: 2048 rows of width 2048 1268 -> 1202 us (866 with the tiles as they are), 601 of width 1024 312 -> 309 (240), and 14
 // launches less.)
 constexpr int LT_GROUPED = 1, LT_GLU = 2, LT_SUM = 4;
+template <int MODE>
+using LinTileArgs = std::conditional_t<(MODE & LT_SUM) != 0, LinSumArgs, std::conditional_t<(MODE & LT_GLU) != 0, LinGluArgs, LinArgs>>;
 template <int BM, int BN, int WM, int WN, int NB, int MODE>
-__global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(LinArgs P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
+__global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(LinTileArgs<MODE> P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
 {
     constexpr bool GROUPED = MODE & LT_GROUPED, GLU = MODE & LT_GLU, SUM = MODE & LT_SUM;
     constexpr int WAVES = WM * WN, TA = BM / (32 * WM), TB = BN / (32 * WN), AI = BM / (8 * WAVES), WI = BN / (8 * WAVES), ROWB = 2 * LT_BK, STEPB = (BM + BN) * ROWB;
@@ -213,9 +219,13 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
         }
     }
     // a tile of gates and ups: o0, its first output
-    const int n_tile = n0 / BN, n_plain = GLU ? (P.glu_c0 + BN - 1) / BN : 0;
-    const bool glu = GLU && n_tile >= n_plain;
-    const int o0 = (n_tile - n_plain) * (BN / 2), n_end = GLU ? P.glu_c0 : P.N;
+    int o0 = 0, n_end = P.N, K0 = P.K;
+    bool glu = false;
+    if constexpr (GLU) {
+        const int n_tile = n0 / BN, n_plain = (P.glu_c0 + BN - 1) / BN;
+        glu = n_tile >= n_plain; o0 = (n_tile - n_plain) * (BN / 2); n_end = P.glu_c0;
+    }
+    if constexpr (SUM) { Wg = P.part[0].W; K0 = P.part[0].K; }
     auto swz = [](int r) { return (r >> 1) & 7; };
     const bf16_t *asrc[AI], *wsrc[WI];
     int wlim[WI];          // furthest step offset of the lane's piece inside a row of W
@@ -229,13 +239,14 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
 #pragma unroll
     for (int j = 0; j < WI; j++) {
         const int row = (wave * WI + j) * 8 + (lane >> 3), c = (lane & 7) ^ swz(row);
-        const int wr = glu ? P.glu_c0 + ((row & 16) ? P.glu_f : 0) + min(o0 + 16 * (row >> 5) + (row & 15), P.glu_f - 1) : min(n0 + row, n_end - 1);
-        const int K = SUM ? P.part[0].K : P.K;
-        wsrc[j] = (SUM ? P.part[0].W : Wg) + (size_t)wr * K + c * 8;
-        wlim[j] = K - 8 - c * 8;
+        int wr = min(n0 + row, n_end - 1);
+        if constexpr (GLU) if (glu) wr = P.glu_c0 + ((row & 16) ? P.glu_f : 0) + min(o0 + 16 * (row >> 5) + (row & 15), P.glu_f - 1);
+        wsrc[j] = Wg + (size_t)wr * K0 + c * 8;
+        wlim[j] = K0 - 8 - c * 8;
     }
     // (SUM) the part that the next requested step belongs to, from its first step to the one behind its last; likewise for the next step of products
-    int q_part = 0, q_from = 0, q_to = SUM ? P.part[0].steps : 0, c_part = 0, c_to = q_to;
+    int q_part = 0, q_from = 0, q_to = 0, c_part = 0, c_to = 0;
+    if constexpr (SUM) q_to = c_to = P.part[0].steps;
     auto enter = [&](int step) {
         if constexpr (SUM) {
             if (step != q_to) return;
@@ -507,13 +518,14 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
 }
 
 // column tiles of a product (gate | up: with G16's padding)
-size_t lin_col_tiles(const LinArgs &P, int bn, bool glu) { return glu ? (P.glu_c0 + bn - 1) / bn + ((size_t)P.glu_w + bn / 2 - 1) / (bn / 2) : ((size_t)P.N + bn - 1) / bn; }
+size_t lin_col_tiles(const LinArgs &P, int bn) { return ((size_t)P.N + bn - 1) / bn; }
+size_t lin_col_tiles(const LinGluArgs &P, int bn) { return (P.glu_c0 + bn - 1) / bn + ((size_t)P.glu_w + bn / 2 - 1) / (bn / 2); }
 
 template <int BM, int BN, int WM, int WN, int NB, int MODE>
-int launch_lin_tile(const LinArgs &P, const bf16_t *a16, size_t lda16, size_t row_tiles, hipStream_t s)
+int launch_lin_tile(const LinTileArgs<MODE> &P, const bf16_t *a16, size_t lda16, size_t row_tiles, hipStream_t s)
 {
     constexpr int smem = NB * (BM + BN) * 2 * LT_BK;
-    const int tm = (int)row_tiles, tn = (int)lin_col_tiles(P, BN, MODE & LT_GLU);
+    const int tm = (int)row_tiles, tn = (int)lin_col_tiles(P, BN);
     const auto fn = k_lin_tile<BM, BN, WM, WN, NB, MODE>;
     if (smem > 64 * 1024) IFA_HIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, smem));
     hipLaunchKernelGGL(fn, dim3((unsigned)tm * (unsigned)tn), dim3(64 * WM * WN), smem, s, P, a16, (int)lda16, tm, tn);
@@ -536,10 +548,9 @@ double lin_cost(const LinShape &h, size_t tiles, size_t steps)
 }
 
 template <int MODE>
-int lin_tile_dispatch(const LinArgs &P, const bf16_t *a, size_t lda, hipStream_t s)
+int lin_tile_dispatch(const LinTileArgs<MODE> &P, const bf16_t *a, size_t lda, hipStream_t s)
 {
-    constexpr bool GLU = MODE & LT_GLU;
-    const size_t T = (size_t)P.T, t128 = (T + 127) / 128, t64 = (T + 63) / 64, n128 = lin_col_tiles(P, 128, GLU), n64 = lin_col_tiles(P, 64, GLU), steps = lda / LT_BK;
+    const size_t T = (size_t)P.T, t128 = (T + 127) / 128, t64 = (T + 63) / 64, n128 = lin_col_tiles(P, 128), n64 = lin_col_tiles(P, 64), steps = lda / LT_BK;
     IFA_REQUIRE(t64 * n64 < (1u << 31), "linear_bf16: too many tiles");
     if (steps < 5) return t128 * n128 >= 384 ? launch_lin_tile<128, 128, 2, 4, 2, MODE>(P, a, lda, t128, s) : launch_lin_tile<64, 64, 2, 2, 2, MODE>(P, a, lda, t64, s);
     if (t64 * n64 <= LT_SMALL && steps >= 8) return launch_lin_tile<32, 32, 1, 1, 8, MODE>(P, a, lda, (T + 31) / 32, s);
@@ -556,9 +567,9 @@ int lin_tile_dispatch(const LinArgs &P, const bf16_t *a, size_t lda, hipStream_t
 }
 
 template <int MODE>
-int lin_grouped_dispatch(const LinArgs &P, const bf16_t *a, size_t lda, size_t max_tiles, int tile_rows, hipStream_t s)
+int lin_grouped_dispatch(const LinTileArgs<MODE> &P, const bf16_t *a, size_t lda, size_t max_tiles, int tile_rows, hipStream_t s)
 {
-    IFA_REQUIRE(max_tiles * lin_col_tiles(P, 64, MODE & LT_GLU) < (1u << 31), "linear_bf16_grouped: too many tiles");
+    IFA_REQUIRE(max_tiles * lin_col_tiles(P, 64) < (1u << 31), "linear_bf16_grouped: too many tiles");
     // (8192 pairs of 16 experts, 1408 x 1024 gate | up and 1024 x 704, us: four waves a 128 x 128 tile 54.8 + 46.8, eight 47.9 + 40.4; 2900 pairs: 64 x 64 tiles 34.2 + 18.8, 64 x 128 of
     // eight waves 27.0 + 17.0)
     if (tile_rows == 128) return launch_lin_tile<128, 128, 2, 4, 2, MODE>(P, a, lda, max_tiles, s);
@@ -590,8 +601,8 @@ __global__ void __launch_bounds__(256) k_rows_to_bf16(const float *__restrict__ 
 // by launches and dependent loads, not arithmetic, so the neighbouring element-wise launch is folded in here):
 //   1  layer norm without bias: a = (x - mean) / sqrt(var + eps) * w[k]   (every wave forms mean and variance of the T rows itself)
 //   2  gated GELU: the row holds gate | up (2 K values), a = gelu_tanh(gate[k]) * up[k]
-template <int TT, int PRO>
-__global__ void __launch_bounds__(256) k_lin_rows(LinArgs P)
+template <int TT, int PRO, class Args = LinArgs>
+__global__ void __launch_bounds__(256) k_lin_rows(Args P)
 {
     const int lane = threadIdx.x & 63;
     const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), nwaves = gridDim.x * (blockDim.x >> 6);
@@ -706,11 +717,14 @@ __global__ void __launch_bounds__(256) k_lin_rows(LinArgs P)
 // the caches' bandwidth for them bounds large matrices (32000 x 1024, six rows: 38.9 -> 31.0 us, 8192 x 2048
 // 21.0 -> 16.7; four outputs 34.9 and 21.0).  GLU: from column glu_c0 on the NR are gates and ups by twos, and the activation leaves instead
 // of them (the launch that formed it took 3.7 us).
-template <int TT, int NR, bool GLU>
-__global__ void __launch_bounds__(256) k_lin_rows_group(LinArgs P)
+template <int TT, int NR, class Args>
+__global__ void __launch_bounds__(256) k_lin_rows_group(Args P)
 {
+    constexpr bool GLU = std::is_same_v<Args, LinGluArgs>;
     const int lane = threadIdx.x & 63, wave = blockIdx.x * 4 + (threadIdx.x >> 6), nwaves = gridDim.x * 4;
-    const int n_end = GLU ? P.glu_c0 : P.N, plain = (n_end + NR - 1) / NR, groups = plain + (GLU ? (P.glu_f + NR / 2 - 1) / (NR / 2) : 0);
+    int n_end = P.N, more = 0;
+    if constexpr (GLU) { n_end = P.glu_c0; more = (P.glu_f + NR / 2 - 1) / (NR / 2); }
+    const int plain = (n_end + NR - 1) / NR, groups = plain + more;
     for (int grp = wave; grp < groups; grp += nwaves) {
         const bool glu = GLU && grp >= plain;
         const int n0 = grp * NR, o0 = (grp - plain) * (NR / 2);
@@ -718,7 +732,8 @@ __global__ void __launch_bounds__(256) k_lin_rows_group(LinArgs P)
         int row[NR];
 #pragma unroll
         for (int r = 0; r < NR; r++) {
-            row[r] = glu ? P.glu_c0 + ((r & 1) ? P.glu_f : 0) + min(o0 + (r >> 1), P.glu_f - 1) : min(n0 + r, n_end - 1);
+            row[r] = min(n0 + r, n_end - 1);
+            if constexpr (GLU) if (glu) row[r] = P.glu_c0 + ((r & 1) ? P.glu_f : 0) + min(o0 + (r >> 1), P.glu_f - 1);
             w[r] = P.W + (size_t)row[r] * P.K;
         }
         float acc[TT][NR];
@@ -772,13 +787,14 @@ __global__ void __launch_bounds__(256) k_lin_rows_group(LinArgs P)
 #pragma unroll
         for (int t = 0; t < TT; t++) {
             if (lane != t || t >= P.T) continue;
-            if (glu) {
+            if constexpr (GLU) if (glu) {
 #pragma unroll
                 for (int r = 0; r < NR; r += 2) {
                     const float gb = P.bias ? bf2f(P.bias[row[r]]) : 0.0f, ub = P.bias ? bf2f(P.bias[row[r + 1]]) : 0.0f;
                     if (o0 + (r >> 1) < P.glu_f) P.G[(size_t)t * P.ldg + o0 + (r >> 1)] = glu_of(P.glu_kind, P.glu_limit, acc[t][r] + gb, acc[t][r + 1] + ub);
                 }
-            } else {
+            }
+            if (!glu) {
 #pragma unroll
                 for (int r = 0; r < NR; r++) if (n0 + r < n_end) lin_store(P, t, n0 + r, acc[t][r]);
             }
@@ -787,16 +803,30 @@ __global__ void __launch_bounds__(256) k_lin_rows_group(LinArgs P)
 }
 
 // workgroups: a group of outputs a wave, up to 32 waves a compute unit
-template <int NR, bool GLU>
-void launch_lin_rows_group(const LinArgs &P, hipStream_t s)
+template <int NR, class Args>
+void launch_lin_rows_group(const Args &P, hipStream_t s)
 {
-    const size_t n_end = GLU ? P.glu_c0 : P.N, groups = (n_end + NR - 1) / NR + (GLU ? ((size_t)P.glu_f + NR / 2 - 1) / (NR / 2) : 0);
+    size_t groups = ((size_t)P.N + NR - 1) / NR;
+    if constexpr (std::is_same_v<Args, LinGluArgs>) groups = ((size_t)P.glu_c0 + NR - 1) / NR + ((size_t)P.glu_f + NR / 2 - 1) / (NR / 2);
     const dim3 grid((unsigned)std::min<size_t>((groups + 3) / 4, 8192));
-    if (P.T == 1) hipLaunchKernelGGL((k_lin_rows_group<1, NR, GLU>), grid, dim3(256), 0, s, P);
-    else if (P.T == 2) hipLaunchKernelGGL((k_lin_rows_group<2, NR, GLU>), grid, dim3(256), 0, s, P);
-    else if (P.T <= 4) hipLaunchKernelGGL((k_lin_rows_group<4, NR, GLU>), grid, dim3(256), 0, s, P);
-    else if (P.T <= 6) hipLaunchKernelGGL((k_lin_rows_group<6, NR, GLU>), grid, dim3(256), 0, s, P);
-    else hipLaunchKernelGGL((k_lin_rows_group<8, NR, GLU>), grid, dim3(256), 0, s, P);
+    if (P.T == 1) hipLaunchKernelGGL((k_lin_rows_group<1, NR, Args>), grid, dim3(256), 0, s, P);
+    else if (P.T == 2) hipLaunchKernelGGL((k_lin_rows_group<2, NR, Args>), grid, dim3(256), 0, s, P);
+    else if (P.T <= 4) hipLaunchKernelGGL((k_lin_rows_group<4, NR, Args>), grid, dim3(256), 0, s, P);
+    else if (P.T <= 6) hipLaunchKernelGGL((k_lin_rows_group<6, NR, Args>), grid, dim3(256), 0, s, P);
+    else hipLaunchKernelGGL((k_lin_rows_group<8, NR, Args>), grid, dim3(256), 0, s, P);
+}
+
+// products of at most eight rows without a prologue
+template <class Args>
+void launch_lin_rows(const Args &P, hipStream_t s)
+{
+    if (P.T > 1 && P.vec && (size_t)P.N * P.K >= (size_t)8 << 20) { launch_lin_rows_group<2>(P, s); return; }
+    const dim3 grid((unsigned)std::min<size_t>(((size_t)P.N + 3) / 4, 8192));
+    if (P.T == 1) hipLaunchKernelGGL((k_lin_rows<1, 0, Args>), grid, dim3(256), 0, s, P);
+    else if (P.T == 2) hipLaunchKernelGGL((k_lin_rows<2, 0, Args>), grid, dim3(256), 0, s, P);
+    else if (P.T <= 4) hipLaunchKernelGGL((k_lin_rows<4, 0, Args>), grid, dim3(256), 0, s, P);
+    else if (P.T <= 6) hipLaunchKernelGGL((k_lin_rows<6, 0, Args>), grid, dim3(256), 0, s, P);
+    else hipLaunchKernelGGL((k_lin_rows<8, 0, Args>), grid, dim3(256), 0, s, P);
 }
 
 // ONE row, layer-normed on the way in (k_lin_rows with prologue 1 formed the norm again for every output row of a wave): each wave forms mean and variance
@@ -889,7 +919,7 @@ static int linear_launch(const void *w_bf16, size_t rows, size_t cols, const voi
     P.T = (int)tokens; P.N = (int)rows; P.K = (int)cols; P.lda = (int)lda; P.ldc = (int)ldc;
     P.alpha = alpha; P.accumulate = accumulate ? 1 : 0; P.act_c0 = silu_col0; P.act_c1 = silu_col1;
     P.norm_w = (const bf16_t *)norm_w_bf16; P.norm_eps = norm_eps;
-    P.tile_map = P.n_tiles = P.a_rows = nullptr; P.row_scale = nullptr; P.act_kind = act; P.C16 = nullptr; P.row_gate = row_gate; P.ld_gate = (int)ld_gate;
+    P.tile_map = P.n_tiles = P.a_rows = nullptr; P.row_scale = nullptr; P.act_kind = act; P.C16 = nullptr;
     // 16-byte requests need whole 8-element pieces in every row of both operands
     P.vec = (cols % 8 == 0 && lda % 4 == 0 && ((uintptr_t)a_f32 & 15) == 0 && ((uintptr_t)w_bf16 & 15) == 0) ? 1 : 0;
     hipStream_t s = ifa_s(stream);
@@ -904,13 +934,17 @@ static int linear_launch(const void *w_bf16, size_t rows, size_t cols, const voi
         if (cols <= 2 * 512) hipLaunchKernelGGL(k_lin_row_norm<2>, dim3(grid), dim3(256), 0, s, P);
         else if (cols <= 4 * 512) hipLaunchKernelGGL(k_lin_row_norm<4>, dim3(grid), dim3(256), 0, s, P);
         else hipLaunchKernelGGL(k_lin_row_norm<8>, dim3(grid), dim3(256), 0, s, P);
-    } else if (tokens > 1 && tokens <= 8 && !prologue && P.vec && rows * cols >= (size_t)8 << 20) {
-        launch_lin_rows_group<2, false>(P, s);
+    } else if (row_gate) {
+        IFA_REQUIRE(tokens <= 8 && !prologue, "%s: %zu rows (at most 8) with a gate", who, tokens);
+        LinGatedArgs G;
+        static_cast<LinArgs &>(G) = P;
+        G.row_gate = row_gate; G.ld_gate = (int)ld_gate;
+        launch_lin_rows(G, s);
+    } else if (tokens <= 8 && !prologue) {
+        launch_lin_rows(P, s);
     } else if (tokens <= 8) {
         const unsigned grid = (unsigned)std::min<size_t>((rows + 3) / 4, 8192);
-#define IFA_LR(TT) { if (prologue == 1) hipLaunchKernelGGL((k_lin_rows<TT, 1>), dim3(grid), dim3(256), 0, s, P); \
-                     else if (prologue == 2) hipLaunchKernelGGL((k_lin_rows<TT, 2>), dim3(grid), dim3(256), 0, s, P); \
-                     else hipLaunchKernelGGL((k_lin_rows<TT, 0>), dim3(grid), dim3(256), 0, s, P); }
+#define IFA_LR(TT) { if (prologue == 1) hipLaunchKernelGGL((k_lin_rows<TT, 1>), dim3(grid), dim3(256), 0, s, P); else hipLaunchKernelGGL((k_lin_rows<TT, 2>), dim3(grid), dim3(256), 0, s, P); }
         if (tokens == 1) IFA_LR(1) else if (tokens == 2) IFA_LR(2) else if (tokens <= 4) IFA_LR(4) else if (tokens <= 6) IFA_LR(6) else IFA_LR(8)
 #undef IFA_LR
     } else {
@@ -936,12 +970,12 @@ bool ifa_linear_bf16w_glu_rows(const void *w_bf16, size_t rows, size_t cols, con
     if (!w_bf16 || !a_f32 || !g_f32 || (!c_f32 && glu_col0) || tokens == 0 || tokens > 8 || cols == 0 || cols % 8 || lda < cols || lda % 4 || ((uintptr_t)a_f32 & 15) || ((uintptr_t)w_bf16 & 15)
         || ldc < glu_col0 || glu_cols == 0 || glu_col0 + 2 * glu_cols > rows || ldg < glu_cols || rows >= (1u << 30) || cols >= (1u << 30) || lda >= (1u << 30) || ldc >= (1u << 30)
         || ldg >= (1u << 30) || glu_kind < 0 || glu_kind > 3 || (glu_kind == 3 && !(glu_limit > 0.0f))) return false;
-    LinArgs P;
+    LinGluArgs P;
     memset(&P, 0, sizeof(P));
     P.W = (const bf16_t *)w_bf16; P.A = (const float *)a_f32; P.C = (float *)c_f32; P.bias = (const bf16_t *)bias_bf16; P.T = (int)tokens; P.N = (int)rows; P.K = (int)cols; P.lda = (int)lda;
     P.ldc = (int)ldc; P.alpha = 1.0f; P.vec = 1; P.act_c0 = silu_col0; P.act_c1 = silu_col1; P.G = (float *)g_f32; P.ldg = (int)ldg; P.glu_c0 = (int)glu_col0; P.glu_f = (int)glu_cols;
     P.glu_kind = glu_kind; P.glu_limit = glu_limit;
-    launch_lin_rows_group<2, true>(P, ifa_s(stream));
+    launch_lin_rows_group<2>(P, ifa_s(stream));
     return true;
 }
 
@@ -995,7 +1029,7 @@ int ifa_linear_bf16_sum(const IfaSumPart *parts, int n_parts, size_t rows, const
 {
     IFA_REQUIRE(parts && a_bf16 && c_f32 && n_parts >= 1 && n_parts <= IFA_SUM_PARTS, "linear_bf16_sum: null pointer or %d parts", n_parts);
     IFA_REQUIRE(rows > 0 && tokens > 0 && ldc >= rows && rows < (1u << 30) && tokens < (1u << 30) && lda < (1u << 30) && ((uintptr_t)a_bf16 & 15) == 0, "linear_bf16_sum: bad shape");
-    LinArgs P;
+    LinSumArgs P;
     memset(&P, 0, sizeof(P));
     P.C = (float *)c_f32; P.T = (int)tokens; P.N = (int)rows; P.ldc = (int)ldc;
     size_t at = 0;
@@ -1018,7 +1052,7 @@ int ifa_linear_bf16_glu(const void *w_bf16, size_t rows, size_t cols, const void
                 && glu_col0 + 2 * glu_cols <= rows && ldg >= ((glu_cols + 63) & ~(size_t)63) && ldg < (1u << 30) && glu_kind >= 0 && glu_kind <= 3 && (glu_kind != 3 || glu_limit > 0.0f),
                 "linear_bf16_glu: bad shape (%zu x %zu, %zu tokens, lda %zu, gate | up %zu + 2 x %zu)", rows, cols, tokens, lda, glu_col0, glu_cols);
     IFA_REQUIRE(rows < (1u << 30) && cols < (1u << 30) && tokens < (1u << 30) && (((uintptr_t)a_bf16 | (uintptr_t)w_bf16) & 15) == 0, "linear_bf16_glu: dimension too large or unaligned operand");
-    LinArgs P;
+    LinGluArgs P;
     memset(&P, 0, sizeof(P));
     P.W = (const bf16_t *)w_bf16; P.C = (float *)c_f32; P.bias = (const bf16_t *)bias_bf16; P.T = (int)tokens; P.N = (int)rows; P.K = (int)cols; P.ldc = (int)ldc; P.alpha = 1.0f;
     P.act_c0 = silu_col0; P.act_c1 = silu_col1; P.G16 = (bf16_t *)glu_bf16; P.ldg = (int)ldg; P.glu_c0 = (int)glu_col0; P.glu_f = (int)glu_cols;
@@ -1036,7 +1070,7 @@ int ifa_linear_bf16_grouped(const void *w_bf16, size_t rows, size_t cols, const 
     IFA_REQUIRE(rows > 0 && cols >= (size_t)LT_BK && cols % 8 == 0 && max_tiles > 0 && lda % 64 == 0 && lda >= cols && lda - cols < 64 && (glu_bf16 || ldc >= rows)
                 && (tile_rows == 64 || tile_rows == 128) && rows < (1u << 30) && cols < (1u << 30) && (((uintptr_t)a_bf16 | (uintptr_t)w_bf16) & 15) == 0,
                 "linear_bf16_grouped: bad shape (%zu x %zu, lda %zu)", rows, cols, lda);
-    LinArgs P;
+    LinGluArgs P;
     memset(&P, 0, sizeof(P));
     P.W = (const bf16_t *)w_bf16; P.C = (float *)c_f32; P.N = (int)rows; P.K = (int)cols; P.ldc = (int)ldc; P.alpha = 1.0f;
     P.tile_map = tile_map_dev; P.n_tiles = n_tiles_dev; P.a_rows = a_rows_dev; P.row_scale = (const float *)row_scale_f32;
@@ -1079,7 +1113,7 @@ extern "C" int ifa_linear_bf16w_grouped(const void *w_bf16, size_t rows, size_t 
     P.W = (const bf16_t *)w_bf16; P.A = (const float *)a_f32; P.C = (float *)c_f32; P.bias = nullptr; P.mul = nullptr;
     P.T = 0; P.N = (int)rows; P.K = (int)cols; P.lda = (int)lda; P.ldc = (int)ldc; P.alpha = 1.0f; P.accumulate = 0; P.act_c0 = P.act_c1 = 0;
     P.norm_w = nullptr; P.norm_eps = 0.0f;
-    P.tile_map = tile_map_dev; P.n_tiles = n_tiles_dev; P.a_rows = a_rows_dev; P.row_scale = (const float *)row_scale_f32; P.act_kind = act; P.C16 = nullptr; P.row_gate = nullptr; P.ld_gate = 0;
+    P.tile_map = tile_map_dev; P.n_tiles = n_tiles_dev; P.a_rows = a_rows_dev; P.row_scale = (const float *)row_scale_f32; P.act_kind = act; P.C16 = nullptr;
     P.vec = (cols % 8 == 0 && lda % 4 == 0 && ((uintptr_t)a_f32 & 15) == 0 && ((uintptr_t)w_bf16 & 15) == 0 && (rows * cols) % 8 == 0) ? 1 : 0;
     const dim3 grid(ifa_cdiv(rows, LM_N), (unsigned)max_tiles);
     if (ops32) hipLaunchKernelGGL(k_lin_mfma<true>, grid, dim3(256), 0, ifa_s(stream), P);
