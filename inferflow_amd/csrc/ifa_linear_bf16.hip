@@ -816,11 +816,22 @@ void launch_lin_rows_group(const Args &P, hipStream_t s)
     else hipLaunchKernelGGL((k_lin_rows_group<8, NR, Args>), grid, dim3(256), 0, s, P);
 }
 
+// Whether two outputs a wave are faster: large matrices whose half as many waves still hide the weights' way from memory (the more rows a wave has to sum, the fewer waves that takes), and
+// whose rows are long enough for it.  us one by one / by twos, rows of the weight x columns: 8192 x 1024 with 2, 4, 6, 8 rows 7.5 / 7.3, 9.6 / 8.8, 12.5 / 11.3, 15.8 / 15.8; 32000 x 2048
+// 34.9 / 28.8, 58 / 39, 70 / 51, 95 / 62; 2816 x 4096 9.6 / 9.9, 14.3 / 12.9, 16.6 / 16.2, 20.1 / 18.9; 2048 x 8192 12.6 / 13.6, 14.9 / 15.3, 22.3 / 18.8, 27.1 / 22.7; 4096 x 2048
+// 7.3 / 7.5, 10.2 / 9.2; and beyond the borders 1024 x 8192 10.5 / 10.7, 12.3 / 12.8, 14.6 / 16.2, 17.3 / 21.1; 16384 x 512 7.3 / 7.6, 10.4 / 10.3, 15.6 / 13.8, 18.4 / 20.7; 65536 x 128
+// 16.7 / 18.3, 27.8 / 30.2, 48 / 41, 59 / 63.  One row: one by one (only the gated form below takes two, where that saves a launch: 2816 gates of 1024 columns 7.1 / 5.4 with the activation's)
+bool lin_rows_by_twos(const LinArgs &P)
+{
+    if (P.T < 2 || !P.vec || P.K < 1024 || (size_t)P.N * P.K < (size_t)8 << 20) return false;
+    return P.N >= (P.T >= 5 ? 2048 : P.T >= 3 ? 2560 : 5120);
+}
+
 // products of at most eight rows without a prologue
 template <class Args>
 void launch_lin_rows(const Args &P, hipStream_t s)
 {
-    if (P.T > 1 && P.vec && (size_t)P.N * P.K >= (size_t)8 << 20) { launch_lin_rows_group<2>(P, s); return; }
+    if (lin_rows_by_twos(P)) { launch_lin_rows_group<2>(P, s); return; }
     const dim3 grid((unsigned)std::min<size_t>(((size_t)P.N + 3) / 4, 8192));
     if (P.T == 1) hipLaunchKernelGGL((k_lin_rows<1, 0, Args>), grid, dim3(256), 0, s, P);
     else if (P.T == 2) hipLaunchKernelGGL((k_lin_rows<2, 0, Args>), grid, dim3(256), 0, s, P);

@@ -364,6 +364,32 @@ def test_products_of_a_few_rows_ask_for_2048_columns_of_the_weight_at_a_time(T, 
     assert np.all(np.abs(got[:, :N] - (orc.f64(A[:, :K]) @ orc.f64(Wm).T + orc.f64(b))) <= bound) and np.all(got[:, N:] == 7.0)
 
 
+@pytest.mark.parametrize("N,K", [(8195, 1032), (5121, 1640), (2051, 4104), (2049, 8200), (16411, 512)])
+@pytest.mark.parametrize("T", [2, 3, 5, 6, 7, 8])
+def test_products_of_a_few_rows_two_outputs_a_wave(T, N, K):
+    """matrices of 8 M elements and more, an odd number of outputs, one and more passes of 2048, 1024 and 512 columns and their rests, sizes on both sides of the form's borders; with everything
+    that an output passes: bias, SiLU on some columns, scale, the sum with what was there: 32-bit activations against 64 bits"""
+    rng = np.random.default_rng(T * 100003 + N + K)
+    Wm, A = bf16_round(rng.standard_normal((N, K)) / np.sqrt(K)), rng.standard_normal((T, K + 4)).astype(np.float32)
+    b, mul, c0 = bf16_round(rng.standard_normal(N)), bf16_round(rng.standard_normal(N)), rng.standard_normal((T, N + 2)).astype(np.float32)
+    out, plain = torch.from_numpy(c0).cuda(), torch.full((T, N + 2), 7.0, dtype=torch.float32, device="cuda")
+    wd, ad, L = devbf(Wm), dev32(A), capi()
+    ia.check(L.ifa_linear_bf16w(p(wd), N, K, p(ad), K + 4, T, p(devbf(b)), p(devbf(mul)), 0.5, 1, 0, p(out), N + 2, 11, 1003, None))
+    ia.check(L.ifa_linear_bf16w(p(wd), N, K, p(ad), K + 4, T, None, None, 1.0, 0, 0, p(plain), N + 2, 0, 0, None)); sync()
+    exact = orc.f64(A[:, :K]) @ orc.f64(Wm).T
+    err = (K / 64 + 12) * 2.0 ** -24 * (np.abs(orc.f64(A[:, :K])) @ np.abs(orc.f64(Wm)).T + np.abs(orc.f64(b)))          # (of the sum, as above)
+    z = exact + orc.f64(b)
+    got = plain.cpu().numpy()
+    assert np.all(np.abs(got[:, :N] - exact) <= err) and np.all(got[:, N:] == 7.0)
+    act = z.copy()
+    act[:, 11:1003] = z[:, 11:1003] / (1.0 + np.exp(-z[:, 11:1003]))
+    want = act * orc.f64(mul) * 0.5 + orc.f64(c0[:, :N])
+    # SiLU's slope is below 1.1; its own evaluation, the two factors and the last sum round once or a few times each
+    bound = (1.1 * err + 16 * 2.0 ** -24 * np.abs(z)) * np.abs(orc.f64(mul)) * 0.5 + 4 * 2.0 ** -24 * (np.abs(want) + np.abs(orc.f64(c0[:, :N])))
+    got = out.cpu().numpy()
+    assert np.all(np.abs(got[:, :N] - want) <= bound) and np.array_equal(got[:, N:], c0[:, N:])
+
+
 def test_products_of_prompts_decline_bad_arguments():
     L = capi()
     z = torch.zeros(1 << 16, dtype=torch.float32, device="cuda")
