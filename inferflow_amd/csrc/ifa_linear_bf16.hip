@@ -552,7 +552,16 @@ int lin_tile_dispatch(const LinTileArgs<MODE> &P, const bf16_t *a, size_t lda, h
 {
     const size_t T = (size_t)P.T, t128 = (T + 127) / 128, t64 = (T + 63) / 64, n128 = lin_col_tiles(P, 128), n64 = lin_col_tiles(P, 64), steps = lda / LT_BK;
     IFA_REQUIRE(t64 * n64 < (1u << 31), "linear_bf16: too many tiles");
-    if (steps < 5) return t128 * n128 >= 384 ? launch_lin_tile<128, 128, 2, 4, 2, MODE>(P, a, lda, t128, s) : launch_lin_tile<64, 64, 2, 2, 2, MODE>(P, a, lda, t64, s);
+    if (steps < 5) {
+        // Fewer steps than the buffers of the tiles below: two buffers, but 64 x 64 tiles that all have a place at once take four where there are four steps.  us with 64 x 64 of two buffers,
+        // 64 x 64 of four, 128 x 64 (four waves, three workgroups a compute unit), 128 x 128 -- four steps, tokens x columns: 16 x 4096 4.4, 3.8, 5.2, 5.6; 1000 x 1024 4.5, 4.2, 5.4, 5.8;
+        // 1000 x 2048 5.6, 5.2, 6.3, 6.7; 411 x 5632 6.0, 7.5, 6.8, 6.9; 411 x 11264 9.8, 10.6, 8.7, 9.4; 1233 x 4096 9.9, 10.6, 8.8, 9.3; 601 x 11264 11.2, 13.7, 13.1, 10.0; two steps,
+        // 1000 x 4096 6.7, -, 6.9, 7.0; 1000 x 5632 8.1, -, 7.3, 7.7; 1233 x 5632 8.9, -, 10.0, 8.3
+        if (t128 * n128 >= 384) return launch_lin_tile<128, 128, 2, 4, 2, MODE>(P, a, lda, t128, s);
+        if (t128 * n64 > 512) return launch_lin_tile<128, 64, 2, 2, 2, MODE>(P, a, lda, t128, s);
+        if (steps == 4 && t64 * n64 <= 512) return launch_lin_tile<64, 64, 2, 2, 4, MODE>(P, a, lda, t64, s);
+        return launch_lin_tile<64, 64, 2, 2, 2, MODE>(P, a, lda, t64, s);
+    }
     if (t64 * n64 <= LT_SMALL && steps >= 8) return launch_lin_tile<32, 32, 1, 1, 8, MODE>(P, a, lda, (T + 31) / 32, s);
     const size_t tiles[LT_N_SHAPES] = {t128 * n128, t128 * n128, t128 * n64, t64 * n64};
     int best = 0;

@@ -350,6 +350,24 @@ def test_products_of_prompts_in_tiles_of_eight_waves(T, N, K):
     assert np.all(np.abs(got[:, :N] - (orc.f64(A) @ orc.f64(Wm).T + orc.f64(b))) <= bound) and np.all(got[:, N:] == 7.0) and torch.equal(out, other)
 
 
+@pytest.mark.parametrize("K", [64, 72, 192, 200, 256])
+@pytest.mark.parametrize("T,N", [(9, 130), (501, 4090), (515, 4090), (1000, 4090), (1000, 4100), (1000, 6010), (1000, 6020)])
+def test_products_of_prompts_of_one_to_four_steps(T, N, K):
+    """up to four steps of 64 columns, whole and not: 64 x 64 tiles of four buffers (up to 512 of them, four steps) and of two, 128 x 64 and 128 x 128 tiles of two, on both sides of the borders
+    between them: the sums of the product that rounds its activations itself"""
+    rng = np.random.default_rng(T + N + K)
+    Wm, A, b = bf16_round(rng.standard_normal((N, K))), bf16_round(rng.standard_normal((T, K))), bf16_round(rng.standard_normal(N))
+    wd, ad, bd, L, ld = devbf(Wm), dev32(A), devbf(b), capi(), (K + 63) // 64 * 64
+    a16 = torch.full((T, ld), -1, dtype=torch.int16, device="cuda")
+    out, other = (torch.full((T, N + 2), 7.0, dtype=torch.float32, device="cuda") for _ in range(2))
+    ia.check(L.ifa_rows_to_bf16(p(ad), K, T, K, p(a16), ld, None))
+    ia.check(L.ifa_linear_bf16_both(p(wd), N, K, p(a16), ld, T, p(bd), None, 1.0, 0, 0, p(out), None, N + 2, 0, 0, None))
+    ia.check(L.ifa_linear_bf16w(p(wd), N, K, p(ad), K, T, p(bd), None, 1.0, 0, 0, p(other), N + 2, 0, 0, None)); sync()
+    got = out.cpu().numpy()
+    bound = (K + 2) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(Wm).T.astype(np.float64) + np.abs(orc.f64(b)))          # (as above)
+    assert np.all(np.abs(got[:, :N] - (orc.f64(A) @ orc.f64(Wm).T + orc.f64(b))) <= bound) and np.all(got[:, N:] == 7.0) and torch.equal(out, other)
+
+
 @pytest.mark.parametrize("K", [8, 504, 520, 2048, 2056, 4616])
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 6, 7, 8])
 def test_products_of_a_few_rows_ask_for_2048_columns_of_the_weight_at_a_time(T, K):
