@@ -533,18 +533,24 @@ int launch_lin_tile(const LinTileArgs<MODE> &P, const bf16_t *a16, size_t lda16,
     return IFA_OK;
 }
 
-// Tile shapes by what a round of the chip's 256 compute units takes: us a step of 64 columns with one and with two workgroups on a compute unit, and beside the steps, measured with weights
-// from memory.  us before (128 x 128 and 128 x 64 of 4 waves with two buffers, 64 x 64 with four) / now, tokens x columns x K: 2048 x 2048 x 9728 123 / 90, 1000 x 2048 x 9728 117 / 62,
+// Tile shapes by what a round of the chip's 256 compute units takes: us a step of 64 columns and beside the steps, measured with weights from memory.  A round that is not full takes less a
+// step, the chip's clock and its caches being shared: where a compute unit has one workgroup, from `one` (few of them) to `full`; where it has two, `one` up to 256 workgroups, then from `two`
+// to `full`.  (As if every round took what a full one of short rows does, rows of 5632 columns and more ran alone on a compute unit in two rounds: tokens x columns x K 1233 x 4096 x 5632 97 us,
+// by twos 85; 4096 x 4096 x 5632 214 and 198; 2048 x 4096 x 8192 156 and 143.  Against the fastest shape of each of 570 sizes from 16 to 4096 tokens, 256 to 11264 columns and 320 to 11008 K
+// 1.5 % behind on average and up to 17, now 0.7.)
+// us before (128 x 128 and 128 x 64 of 4 waves with two buffers, 64 x 64 with four) / now, tokens x columns x K: 2048 x 2048 x 9728 123 / 90, 1000 x 2048 x 9728 117 / 62,
 // 2000 x 1024 x 4864 58 / 32, 2048 x 1024 x 1024 15.4 / 8.7, 730 x 2836 x 1024 16.1 / 12.5, 1024 x 4096 x 2048 29.9 / 22.5, 601 x 1024 x 4864 22.1 / 20.8; in a Gelarax layer 2048 rows' input
 // product (19968 columns, gated) 238 / 207, its output product 150 / 108.  (256 x 128 tiles of eight waves, one a compute unit, 225 to 235 there.)
-struct LinShape { int per_cu; double one, two, beside; };
+struct LinShape { int per_cu; double one, two, full, beside; };
 enum { LT_128x128_PAIR, LT_128x128, LT_128x64, LT_64x64, LT_N_SHAPES };
-constexpr LinShape LT_SHAPES[LT_N_SHAPES] = {{2, 0.80, 1.17, 4}, {1, 0.55, 0, 5}, {1, 0.36, 0, 4}, {2, 0.255, 0.44, 4}};
+constexpr LinShape LT_SHAPES[LT_N_SHAPES] = {{2, 0.80, 0.87, 1.13, 4}, {1, 0.42, 0, 0.585, 5}, {1, 0.36, 0, 0.36, 4}, {2, 0.255, 0.44, 0.44, 4}};
 double lin_cost(const LinShape &h, size_t tiles, size_t steps)
 {
-    const size_t cus = 256, slots = cus * h.per_cu, full = tiles / slots, rest = tiles % slots;
-    const double all = steps * (h.per_cu == 2 ? h.two : h.one) + h.beside;
-    return full * all + (rest == 0 ? 0.0 : rest <= cus ? steps * h.one + h.beside : all);
+    const size_t cus = 256, slots = cus * h.per_cu, rounds = tiles / slots, rest = tiles % slots;
+    const double whole = rounds * (steps * h.full + h.beside);
+    if (rest == 0) return whole;
+    const double a_step = h.per_cu == 1 ? h.one + (h.full - h.one) * rest / cus : rest <= cus ? h.one : h.two + (h.full - h.two) * (rest - cus) / cus;
+    return whole + steps * a_step + h.beside;
 }
 
 template <int MODE>
