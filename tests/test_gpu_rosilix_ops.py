@@ -350,11 +350,11 @@ def test_products_of_prompts_in_tiles_of_eight_waves(T, N, K):
     assert np.all(np.abs(got[:, :N] - (orc.f64(A) @ orc.f64(Wm).T + orc.f64(b))) <= bound) and np.all(got[:, N:] == 7.0) and torch.equal(out, other)
 
 
-@pytest.mark.parametrize("K", [64, 72, 192, 200, 256])
+@pytest.mark.parametrize("K", [64, 72, 192, 200, 256, 328, 2048, 2056])
 @pytest.mark.parametrize("T,N", [(9, 130), (501, 4090), (515, 4090), (1000, 4090), (1000, 4100), (1000, 6010), (1000, 6020)])
-def test_products_of_prompts_of_one_to_four_steps(T, N, K):
+def test_products_of_prompts_of_few_steps(T, N, K):
     """up to four steps of 64 columns, whole and not: 64 x 64 tiles of four buffers (up to 512 of them, four steps) and of two, 128 x 64 and 128 x 128 tiles of two, on both sides of the borders
-    between them: the sums of the product that rounds its activations itself"""
+    between them; 5, 32 and 33 steps, up to 32 of which 128 x 64 tiles take: the sums of the product that rounds its activations itself"""
     rng = np.random.default_rng(T + N + K)
     Wm, A, b = bf16_round(rng.standard_normal((N, K))), bf16_round(rng.standard_normal((T, K))), bf16_round(rng.standard_normal(N))
     wd, ad, bd, L, ld = devbf(Wm), dev32(A), devbf(b), capi(), (K + 63) // 64 * 64
