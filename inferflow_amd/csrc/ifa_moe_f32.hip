@@ -178,7 +178,8 @@ __device__ int route_pair(const RouteSel &R, int t, int k, int top, bool leave)
         s = live ? expf(s - mx) : 0.0f;
         s /= block_sum(s, red);
     }
-    const float c = live ? s + (R.corr ? bf2f(R.corr[e]) : 0.0f) : -INFINITY;
+    float c = live ? s + (R.corr ? bf2f(R.corr[e]) : 0.0f) : -INFINITY;
+    if (c != c) c = -INFINITY;          // (no number: last, so that the ranks are a permutation and every pair has an expert; its weight stays what it is)
     ch[e] = c;
     __syncthreads();
     int rank = 0;

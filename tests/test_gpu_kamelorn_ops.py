@@ -103,6 +103,31 @@ def test_experts_with_the_choice_inside_their_first_launch(rows, W, F, E, top, k
         assert near(plain, orc.logistic(np.take_along_axis(orc.f64(logits), idx_w, -1)), 5e-6)
 
 
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("E,top", [(6, 2), (5, 5), (256, 3)])
+def test_experts_of_rows_whose_router_left_no_numbers(kind, E, top):
+    """a row of NaN and a row with one NaN among a few: every pair has an expert of its own, the rows beside them are what they are by themselves"""
+    rows, W, F = 4, 40, 16
+    rng = np.random.default_rng(E + kind)
+    h, logits = rng.standard_normal((rows, W)).astype(np.float32), rng.standard_normal((rows, E)).astype(np.float32)
+    logits[1] = np.nan; logits[2, 3] = np.nan
+    gu, dd = devbf(bf16_round(rng.standard_normal((E * 2 * F, W)) * 0.3)), devbf(bf16_round(rng.standard_normal((E * W, F)) * 0.3))
+    L = capi()
+
+    def run(keep):
+        n = len(keep)
+        nb = L.ifa_moe_workspace_bytes(n, top, W, 3 * F, E)
+        ws = torch.empty((nb,), dtype=torch.uint8, device="cuda")
+        idx, wgt = torch.full((n, top), -1, dtype=torch.int32, device="cuda"), torch.zeros((n, top), dtype=torch.float32, device="cuda")
+        y, dh, dl = torch.zeros((n, W), dtype=torch.float32, device="cuda"), dev32(h[keep]), dev32(logits[keep])
+        ia.check(L.ifa_moe_experts_routed_rows_f32(kind, 1, 1e-20, 1.7, p(dl), E, None, 0, 0.0, p(dh), W, n, W, F, E, top, p(gu), p(dd), p(idx), p(wgt), p(ws), nb, p(y), W, 0, None)); sync()
+        return idx.cpu().numpy(), y.cpu().numpy()
+    idx, y = run([0, 1, 2, 3])
+    assert idx.min() >= 0 and idx.max() < E and all(len(set(r)) == top for r in idx.tolist()) and np.isnan(y[1]).all()
+    idx2, y2 = run([0, 3])
+    assert np.array_equal(idx[[0, 3]], idx2) and np.array_equal(y[[0, 3]], y2) and np.isfinite(y2).all()
+
+
 @pytest.mark.parametrize("T,n_all,top,scale", [(9, 6, 2, 2.5), (70, 16, 1, 0.3), (5, 5, 5, 1.0), (12, 70, 8, 3.0)])
 def test_renormalized_router_in_both_forms(T, n_all, top, scale):
     rng = np.random.default_rng(n_all + top)
