@@ -420,6 +420,7 @@ int ensure_halfs(ifa_model *m, bf16_t *&buf, size_t &cap, size_t need)
 {
     if (need <= cap) return IFA_OK;
     IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
+    drop_step_graph(m->lay);          // (with a16_min 1 a captured step reads these)
     lay_free(buf); buf = nullptr; cap = 0;
     IFA_HIP_CHECK(hipMalloc((void **)&buf, need * 2));
     cap = need;

@@ -370,6 +370,24 @@ def test_generation_over_key_block_edges_with_single_rows_sent_to_the_tiles(tmp_
     eng.close()
 
 
+def test_generation_over_bfloat16_rows_of_single_tokens_beside_longer_and_longer_prompts(tmp_path):
+    """a16_min 1: the captured step reads the buffers of rounded activations, which a longer prompt allocates anew: the tokens of uncaptured steps"""
+    import inferflow_amd as ia
+    cfg = fx.config([fx.attention_layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=fx.dense(ff=136, limit=1.5)), fx.attention_layer(heads=4, kv_heads=2, dim=32, vdim=32, mlp=fx.dense(ff=72))],
+                    width=128, vocab=97)
+    w, seen = fx.random_weights(cfg, 25), {}
+    for graph in (1, 0):
+        eng = engine_for(tmp_path, cfg, w, "bfloat16")
+        for name, value in ((b"a16_min", 1), (b"graph", graph)):
+            ia.check(ia.lib().ifa_model_set_option(eng.worker(), name, value))
+        for n in (20, 90, 400):
+            q = eng.add_query(tokens_for(cfg, n, 26))
+            seen.setdefault(graph, []).append(eng.generate(q, 30)[0])
+            eng.remove_query(q)
+        eng.close()
+    assert seen[1] == seen[0] and all(len(set(t)) > 5 for t in seen[0])
+
+
 def test_heads_above_128_share_their_keys_out_in_steps_of_a_few_rows(tmp_path):
     """heads that no tile takes go row by row, a few rows' keys shared out to several workgroups whatever border the tiles have: the same bits"""
     import inferflow_amd as ia
