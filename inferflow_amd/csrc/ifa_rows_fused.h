@@ -44,19 +44,19 @@ int ifa_linear_bf16_grouped(const void *w_bf16, size_t rows, size_t cols, const 
                             size_t max_tiles, int tile_rows, const void *row_scale_f32, void *c_f32, size_t ldc, int glu_kind, float glu_limit, void *glu_bf16, ifa_stream stream);
 // ifa_linear_bf16_both whose output columns [glu_col0, glu_col0 + 2 glu_cols) are gate | up of a gated feed-forward: glu_bf16[t][c] = act(gate[c]) up[c] in bfloat16 rows of ldg
 // (whole 64s, zero beyond glu_cols) in their place; the columns before them as ever, any behind them not at all
-int ifa_linear_bf16_glu(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,
+extern "C" int ifa_linear_bf16_glu(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,
                         int silu_col1, size_t glu_col0, size_t glu_cols, int glu_kind, float glu_limit, void *glu_bf16, size_t ldg, ifa_stream stream);
 // At most eight rows of 32-bit activations.  ifa_linear_bf16w whose columns [glu_col0, glu_col0 + 2 glu_cols) are gate | up: g_f32[t][c] = act(gate[c]) up[c] in their place (false: sizes or
 // alignment don't allow it, nothing launched); and a product whose row t is multiplied by sigmoid(row_gate[t * ld_gate])
-bool ifa_linear_bf16w_glu_rows(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,
+extern "C" bool ifa_linear_bf16w_glu_rows(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,
                                int silu_col1, size_t glu_col0, size_t glu_cols, int glu_kind, float glu_limit, void *g_f32, size_t ldg, ifa_stream stream);
-int ifa_linear_bf16w_gated_rows(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *row_gate_f32, size_t ld_gate, int accumulate, void *c_f32,
+extern "C" int ifa_linear_bf16w_gated_rows(const void *w_bf16, size_t rows, size_t cols, const void *a_f32, size_t lda, size_t tokens, const void *row_gate_f32, size_t ld_gate, int accumulate, void *c_f32,
                                 size_t ldc, ifa_stream stream);
 // C[t][n] += sum over the parts of alpha mul[n] (W[n] . a[t] + bias[n]): a_bf16's rows hold the parts' operands side by side, each zero-padded to whole 64s (lda: their sum);
 // cols: a multiple of 8, 64 and more
 constexpr int IFA_SUM_PARTS = 3;
 struct IfaSumPart { const void *w; size_t cols; const void *mul, *bias; float alpha; };
-int ifa_linear_bf16_sum(const IfaSumPart *parts, int n_parts, size_t rows, const void *a_bf16, size_t lda, size_t tokens, void *c_f32, size_t ldc, ifa_stream stream);
+extern "C" int ifa_linear_bf16_sum(const IfaSumPart *parts, int n_parts, size_t rows, const void *a_bf16, size_t lda, size_t tokens, void *c_f32, size_t ldc, ifa_stream stream);
 // ifa_rows_to_bf16 into the first `width` columns (a multiple of 8) of rows of ldy
 int ifa_rows_to_bf16_part(const void *x_f32, size_t ldx, size_t rows, size_t cols, void *y_bf16, size_t width, size_t ldy, ifa_stream stream);
 // Producers that leave what only products read in bfloat16: rows of ldy, zero from the last column up to `width` (both multiples of 8).  The norms: false where the sizes or the
@@ -80,7 +80,7 @@ bool ifa_moe_gated_reads_bf16(size_t rows, int width, int ff, int top, int ops32
 int ifa_moe_experts_gated_bf16(const void *h_bf16, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16, const void *down_bf16, const int *idx_dev,
                                const void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream);
 // ifa_moe_route_top_f32 inside the first launch of ifa_moe_experts_gated_f32: at most eight rows, 256 experts
-int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
+extern "C" int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
                                    const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream);
 // ifa_glu_ex_f32 whose output only products read: bfloat16 rows, zero up to ldo (a multiple of 8; csrc/ifa_ops_f32.hip)
 int ifa_glu_to_bf16(int kind, float limit, const void *gate_up_f32, size_t ld, size_t rows, size_t cols, const void *row_gate_f32, size_t ldg, void *out_bf16, size_t ldo,

@@ -578,6 +578,72 @@ def test_batched_attention_at_the_edges_of_passes_and_splits(shape, kvd, monkeyp
     wk.close()
 
 
+@pytest.mark.parametrize("kvd", [dt.F16, dt.Q8_B32T2], ids=["kvf16", "kvq8"])
+def test_batched_attention_over_many_splits(kvd, monkeypatch):
+    """k_dec_attn_keys: 9, 16, 17, 32 splits of 256 keys and 17 of 512 (contexts up to 8700, as many splits as a workgroup adds up), a query of one split beside them; against the op-by-op rows
+    with the bounds of the tests above, row order, and the same bits again"""
+    monkeypatch.setitem(synth.SHAPES, "keys_long", dict(dim=256, layers=2, ffn=512, vocab=600, heads=4, kv_heads=2, head_dim=64))
+    wk, _, s = synth.build("keys_long", dt.Q4_B32T1A, kvd, max_ctx=8704, quant_threshold=0, std=0.06)
+    lens, V = [2049, 4095, 4096, 8191, 8200, 8690, 70], s["vocab"]
+    n = len(lens)
+    wk.kv_slots(n)
+    rng = np.random.default_rng(11)
+    for i, k in enumerate(lens):
+        wk.select_kv(i)
+        wk.forward(rng.integers(3, V, k).astype(np.int32), 0)
+    cur = [int(t) for t in rng.integers(3, V, n)]
+    lg, lgu, lgp = (torch.empty((n, V), dtype=torch.float16, device="cuda") for _ in range(3))
+    wk.set_option("batch_fused", 0)
+    wk.decode_batch(cur, lens, list(range(n)), lgu)
+    wk.set_option("batch_fused", 1)
+    toks = wk.decode_batch(cur, lens, list(range(n)), lg)
+    A, U = g.host(lg).astype(np.float32), g.host(lgu).astype(np.float32)
+    for i in range(n):
+        cos = float((A[i] * U[i]).sum() / (np.linalg.norm(A[i]) * np.linalg.norm(U[i])))
+        assert cos >= 0.9999 and np.abs(A[i] - U[i]).max() <= 0.02, (lens[i], cos, np.abs(A[i] - U[i]).max())
+    order = [int(v) for v in rng.permutation(n)]
+    wk.decode_batch([cur[i] for i in order], [lens[i] for i in order], order, lgp)
+    assert np.array_equal(g.host(lgp), g.host(lg)[order])
+    for _ in range(2):
+        assert [int(t) for t in wk.decode_batch(cur, lens, list(range(n)))] == [int(t) for t in toks]
+    wk.close()
+
+
+@pytest.mark.parametrize("ctx", [60, 300, 700])      # one pass of a workgroup, several, and several splits
+def test_batched_attention_over_infinite_scores(ctx, monkeypatch):
+    """k_dec_attn_keys: a key whose score leaves the half's range.  Below it weighs nothing, above it and where there is no number the row is NaN; in any order of the rows"""
+    monkeypatch.setitem(synth.SHAPES, "keys_one", dict(dim=256, layers=1, ffn=256, vocab=600, heads=2, kv_heads=1, head_dim=128))
+    wk, _, s = synth.build("keys_one", dt.Q4_B32T1A, dt.F16, max_ctx=768, quant_threshold=0, std=0.5)
+    V, rng = s["vocab"], np.random.default_rng(5)
+    prompt = rng.integers(3, V, ctx).astype(np.int32)
+    wk.kv_slots(4)
+    for slot, value in enumerate((None, 60000.0, -60000.0, np.nan)):
+        wk.select_kv(slot)
+        wk.forward(prompt, 0)
+        if value is not None:
+            wk.write_buffer("kcache", np.full(128, value, np.float16), 0, offset=(ctx // 3) * 256)
+    seen = set()
+    for tok in range(7, 600, 45):
+        out = {}
+        for fused in (0, 1):
+            wk.set_option("batch_fused", fused)
+            lg = torch.empty((4, V), dtype=torch.float16, device="cuda")
+            wk.decode_batch([tok] * 4, [ctx] * 4, [0, 1, 2, 3], lg)
+            out[fused] = g.host(lg).astype(np.float32)
+        nan = [bool(np.isnan(r).all()) for r in out[1]]
+        assert nan == [bool(np.isnan(r).all()) for r in out[0]] and nan[0] is False and nan[3] is True
+        assert all(np.isfinite(r).all() for r, bad in zip(out[1], nan) if not bad)
+        for r0, r1, bad in zip(out[0], out[1], nan):
+            if not bad:
+                cos = float((r0 * r1).sum() / (np.linalg.norm(r0) * np.linalg.norm(r1)))
+                assert cos >= 0.9999 and np.abs(r0 - r1).max() <= 0.02 * max(1.0, np.abs(r0).max()), (tok, cos)
+        wk.decode_batch([tok] * 4, [ctx] * 4, [3, 0, 2, 1], lg)
+        assert np.array_equal(g.host(lg)[[1, 3, 2, 0]].astype(np.float32), out[1], equal_nan=True)
+        seen |= {tuple(nan[1:3])}
+    assert seen & {(True, False), (False, True)}          # (both heads above the range in one slot, below it in the other)
+    wk.close()
+
+
 @pytest.mark.parametrize("n", [2, 5, 8, 11, 16, 20, 27, 32])
 @pytest.mark.parametrize("kvd,shape", [(dt.F16, "test_mha"), (dt.Q8_B32T2, "test_mha"), (dt.F16, "test_moe"), (dt.F16, "test_moe_longffn")],
                          ids=["kvf16", "kvq8", "moe", "moe_longffn"])

@@ -350,6 +350,118 @@ def test_products_of_prompts_in_tiles_of_eight_waves(T, N, K):
     assert np.all(np.abs(got[:, :N] - (orc.f64(A) @ orc.f64(Wm).T + orc.f64(b))) <= bound) and np.all(got[:, N:] == 7.0) and torch.equal(out, other)
 
 
+SIZES_OF_ALL_TILES = [(9, 34, 520), (33, 65, 512), (70, 97, 1000), (130, 2900, 72), (300, 520, 2048), (411, 11264, 328), (700, 1990, 320), (1000, 1985, 456), (1025, 2049, 648), (2500, 2600, 200),
+                      (2561, 4993, 320)]
+
+
+@pytest.mark.parametrize("T,N,K", SIZES_OF_ALL_TILES)
+@pytest.mark.parametrize("kind", [0, 1, 3])
+def test_gated_activations_in_the_tiles_of_their_product(T, N, K, kind):
+    """every tile shape, gate | up behind other columns (some through SiLU) that end inside a tile, inner sizes that are no whole tile, columns behind them that nobody stores: the bits of gate | up
+    stored, activated and rounded by launches of their own"""
+    F, c0 = N * 3 // 8, N // 4 & ~3
+    rng = np.random.default_rng(T + N + K + kind)
+    wd, bd = devbf(bf16_round(rng.standard_normal((N, K)) / np.sqrt(K))), devbf(bf16_round(rng.standard_normal(N)))
+    ad, L, ld, lg = dev32(bf16_round(rng.standard_normal((T, K)))), capi(), (K + 63) // 64 * 64, (F + 63) // 64 * 64
+    a16 = torch.full((T, ld), -1, dtype=torch.int16, device="cuda")
+    ia.check(L.ifa_rows_to_bf16(p(ad), K, T, K, p(a16), ld, None))
+    full, cut = (torch.full((T, N), 7.0, dtype=torch.float32, device="cuda") for _ in range(2))
+    g32, g16, want = torch.empty((T, F), dtype=torch.float32, device="cuda"), *(torch.full((T, lg), -1, dtype=torch.int16, device="cuda") for _ in range(2))
+    Z, F32 = C.c_size_t, C.c_float
+    ia.check(L.ifa_linear_bf16_both(p(wd), N, K, p(a16), ld, T, p(bd), None, 1.0, 0, 0, p(full), None, N, 4, c0 // 2, None))
+    ia.check(L.ifa_glu_ex_f32(kind, 0.75, C.c_void_p(full.data_ptr() + 4 * c0), N, T, F, None, 0, p(g32), F, None))
+    ia.check(L.ifa_rows_to_bf16(p(g32), F, T, F, p(want), lg, None))
+    ia.check(L.ifa_linear_bf16_glu(p(wd), Z(N), Z(K), p(a16), Z(ld), Z(T), p(bd), p(cut), Z(N), 4, c0 // 2, Z(c0), Z(F), kind, F32(0.75), p(g16), Z(lg), None)); sync()
+    assert torch.equal(g16, want) and torch.equal(cut[:, :c0], full[:, :c0]) and bool((cut[:, c0:] == 7.0).all())
+
+
+@pytest.mark.parametrize("T,N", [(t, n) for t, n, _ in SIZES_OF_ALL_TILES])
+@pytest.mark.parametrize("cols", [(64,), (64, 64, 64), (72, 64), (200, 64, 1032), (64, 520, 328)])
+def test_sums_of_products_in_one_pass(T, N, cols):
+    """one to three parts, parts of one step in a row (they end inside the requests' lead), parts that are no whole step, with and without scales and biases, every tile shape: against 64 bits"""
+    rng = np.random.default_rng(T + N + sum(cols))
+    ld = sum((k + 63) // 64 * 64 for k in cols)
+    a16, at, parts, keep = torch.full((T, ld), -1, dtype=torch.int16, device="cuda"), 0, [], []
+    c0 = rng.standard_normal((T, N + 2)).astype(np.float32)
+    want, bound = orc.f64(c0[:, :N]).copy(), 4 * 2.0 ** -24 * np.abs(orc.f64(c0[:, :N]))
+
+    class Part(C.Structure):
+        _fields_ = [("w", C.c_void_p), ("cols", C.c_size_t), ("mul", C.c_void_p), ("bias", C.c_void_p), ("alpha", C.c_float)]
+    L = capi()
+    for i, K in enumerate(cols):
+        A, Wm, b, m = bf16_round(rng.standard_normal((T, K))), bf16_round(rng.standard_normal((N, K)) / np.sqrt(K)), bf16_round(rng.standard_normal(N)), bf16_round(rng.standard_normal(N))
+        wide = (K + 63) // 64 * 64
+        a16[:, at:at + wide] = 0
+        a16[:, at:at + K] = devbf(A).view(torch.int16).reshape(T, K)
+        at += wide
+        wd, bd, md, alpha = devbf(Wm), devbf(b), devbf(m), (1.0, 0.7, -1.3)[i]
+        keep += [wd, bd, md]
+        parts.append(Part(wd.data_ptr(), K, md.data_ptr() if i != 1 else None, bd.data_ptr() if i != 0 else None, alpha))
+        s, mag = orc.f64(A) @ orc.f64(Wm).T, np.abs(orc.f64(A)) @ np.abs(orc.f64(Wm)).T
+        f = np.float32(alpha) * (orc.f64(m) if i != 1 else 1.0)
+        if i != 0:
+            s, mag = s + orc.f64(b), mag + np.abs(orc.f64(b))
+        want += f * s
+        bound += (K + 8) * 2.0 ** -24 * np.abs(f) * mag          # (at most K roundings of half a unit of the sum of the magnitudes, and those of the scale and of the sums behind)
+    out = torch.from_numpy(c0).cuda()
+    Z = C.c_size_t
+    ia.check(L.ifa_linear_bf16_sum((Part * len(parts))(*parts), len(parts), Z(N), p(a16), Z(ld), Z(T), p(out), Z(N + 2), None)); sync()
+    got = out.cpu().numpy()
+    assert np.all(np.abs(got[:, :N] - want) <= bound) and np.array_equal(got[:, N:], c0[:, N:])
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 5, 6, 8])
+@pytest.mark.parametrize("c0,F,K,kind", [(0, 1, 8, 0), (0, 37, 512, 1), (5, 40, 520, 3), (20, 1409, 1032, 0), (3, 300, 2056, 2), (1, 33, 4616, 1)])
+def test_gated_activations_behind_products_of_a_few_rows(T, c0, F, K, kind):
+    """an odd number of outputs, columns in front (some through SiLU) and behind, one and more passes of 2048, 1024 and 512 columns: 32-bit activations against 64 bits"""
+    N = c0 + 2 * F + 3
+    rng = np.random.default_rng(T * 1009 + F + K + kind)
+    Wm, A, b = bf16_round(rng.standard_normal((N, K)) / np.sqrt(K)), rng.standard_normal((T, K + 4)).astype(np.float32), bf16_round(rng.standard_normal(N))
+    out, act = (torch.full((T, n), 7.0, dtype=torch.float32, device="cuda") for n in (N, F + 1))
+    wd, ad, bd, L, Z = devbf(Wm), dev32(A), devbf(b), capi(), C.c_size_t
+    L.ifa_linear_bf16w_glu_rows.restype = C.c_bool
+    assert L.ifa_linear_bf16w_glu_rows(p(wd), Z(N), Z(K), p(ad), Z(K + 4), Z(T), p(bd), p(out), Z(N), 0, c0 // 2, Z(c0), Z(F), kind, C.c_float(0.75), p(act), Z(F + 1), None); sync()
+    z = orc.f64(A[:, :K]) @ orc.f64(Wm).T + orc.f64(b)
+    err = (K / 64 + 12) * 2.0 ** -24 * (np.abs(orc.f64(A[:, :K])) @ np.abs(orc.f64(Wm)).T + np.abs(orc.f64(b)))          # (of a sum, as above)
+    zg, zu, eg, eu = z[:, c0:c0 + F], z[:, c0 + F:c0 + 2 * F], err[:, c0:c0 + F], err[:, c0 + F:c0 + 2 * F]
+    if kind == 3:
+        zg, zu = np.minimum(zg, 0.75), np.clip(zu, -0.75, 0.75) + 1.0
+        g = zg / (1.0 + np.exp(-1.702 * zg))
+    elif kind == 2:
+        g = np.maximum(zg, 0.0)
+    elif kind == 1:
+        g = 0.5 * zg * (1.0 + np.tanh(0.7978845608028654 * (zg + 0.044715 * zg ** 3)))
+    else:
+        g = zg / (1.0 + np.exp(-zg))
+    # the activations' slopes are below 1.2; their own evaluation rounds a few times, the GELU's relative to its argument
+    bound = (1.2 * eg + 16 * 2.0 ** -24 * (np.abs(zg) + 1e-3)) * np.abs(zu) + np.abs(g) * (eu + 4 * 2.0 ** -24) + 4 * 2.0 ** -24 * np.abs(g * zu)
+    got, plain = act.cpu().numpy(), out.cpu().numpy()
+    assert np.all(np.abs(got[:, :F] - g * zu) <= bound) and np.all(got[:, F:] == 7.0) and np.all(plain[:, c0:] == 7.0)
+    want = z[:, :c0].copy()
+    want[:, :c0 // 2] = want[:, :c0 // 2] / (1.0 + np.exp(-want[:, :c0 // 2]))
+    assert np.all(np.abs(plain[:, :c0] - want) <= 1.1 * err[:, :c0] + 16 * 2.0 ** -24 * np.abs(z[:, :c0]))
+
+
+@pytest.mark.parametrize("T", [1, 2, 4, 5, 8])
+@pytest.mark.parametrize("N,K", [(37, 40), (37, 7), (130, 2056), (2051, 4104)])
+def test_products_of_a_few_rows_times_their_gates(T, N, K):
+    """row t times the logistic of its gate, one output and two a wave, stored and accumulated: against 64 bits"""
+    rng = np.random.default_rng(T * 31 + N + K)
+    Wm, A = bf16_round(rng.standard_normal((N, K)) / np.sqrt(K)), rng.standard_normal((T, K)).astype(np.float32)
+    gate, c0 = 3 * rng.standard_normal((T, 5)).astype(np.float32), rng.standard_normal((T, N + 2)).astype(np.float32)
+    s = 1.0 / (1.0 + np.exp(-orc.f64(gate[:, 2:3])))
+    exact, mag = orc.f64(A) @ orc.f64(Wm).T, np.abs(orc.f64(A)) @ np.abs(orc.f64(Wm)).T
+    L, Z, gd, wd, ad = capi(), C.c_size_t, dev32(gate), devbf(Wm), dev32(A)
+    for acc in (0, 1):
+        out = torch.from_numpy(c0).cuda()
+        ia.check(L.ifa_linear_bf16w_gated_rows(p(wd), Z(N), Z(K), p(ad), Z(K), Z(T), C.c_void_p(gd.data_ptr() + 8), Z(5), acc, p(out), Z(N + 2), None)); sync()
+        want = exact * s + (orc.f64(c0[:, :N]) if acc else 0.0)
+        bound = ((K / 64 + 12) * mag + 16 * np.abs(exact) + 2 * np.abs(want) + 64) * 2.0 ** -24 * np.maximum(s, 2.0 ** -6)
+        bound += 2 * 2.0 ** -24 * np.abs(orc.f64(c0[:, :N])) * acc
+        got = out.cpu().numpy()
+        assert np.all(np.abs(got[:, :N] - want) <= bound) and np.array_equal(got[:, N:], c0[:, N:])
+
+
 @pytest.mark.parametrize("K", [64, 72, 192, 200, 256, 328, 2048, 2056])
 @pytest.mark.parametrize("T,N", [(9, 130), (501, 4090), (515, 4090), (1000, 4090), (1000, 4100), (1000, 6010), (1000, 6020)])
 def test_products_of_prompts_of_few_steps(T, N, K):

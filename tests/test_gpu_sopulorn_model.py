@@ -370,6 +370,27 @@ def test_generation_over_key_block_edges_with_single_rows_sent_to_the_tiles(tmp_
     eng.close()
 
 
+@pytest.mark.parametrize("T", [9, 17, 130, 601, 1500])
+def test_experts_over_the_rows_that_the_norm_has_left_in_bfloat16(tmp_path, T):
+    """Prompts whose norms leave bfloat16 rows for experts and shared expert, between dense layers whose activations are formed in the tiles of their product, inner sizes of whole and of broken
+    steps: the bits of every operand stored in 32 bits and rounded on its way into a product (a16_min 0), and the oracle"""
+    import inferflow_amd as ia
+    cfg = fx.config([fx.attention_layer(heads=4, kv_heads=2, dim=32, vdim=32, mlp=fx.dense(ff=1032, limit=1.5)),
+                     fx.attention_layer(heads=4, kv_heads=2, dim=32, vdim=48, mlp=fx.moe(experts=5, top=2, ff=200, shared=72)),
+                     fx.attention_layer(heads=4, kv_heads=2, dim=32, vdim=48, kv_from=1, mlp=fx.moe(experts=3, top=1, ff=264, shared=0)),
+                     fx.attention_layer(heads=2, kv_heads=2, dim=32, vdim=40, mlp=fx.dense(ff=72))], width=320, vocab=97)
+    w, toks, out = fx.random_weights(cfg, 27), tokens_for(cfg, T, 28), {}
+    eng = engine_for(tmp_path, cfg, w, "bfloat16", 1536, 1)
+    for border in (0, 9):
+        run_whole(eng, tokens_for(cfg, 40, 29))          # (other values in the buffers)
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"a16_min", border))
+        out[border] = run_whole(eng, toks)[0]
+    eng.close()
+    assert np.array_equal(out[0], out[9])
+    if T <= 601:
+        assert_close(fx.rel_err(out[9], oracle_logits(cfg, w, toks)), "bfloat16", TOL16, T)
+
+
 def test_generation_over_bfloat16_rows_of_single_tokens_beside_longer_and_longer_prompts(tmp_path):
     """a16_min 1: the captured step reads the buffers of rounded activations, which a longer prompt allocates anew: the tokens of uncaptured steps"""
     import inferflow_amd as ia

@@ -239,6 +239,35 @@ def test_router_on_logits_with_ties_and_softmax_over_the_chosen(n_all, top):
         assert np.abs(wgt.cpu().numpy() - wgt_w).max() < 1e-6
 
 
+@pytest.mark.parametrize("T,W,F,E,top", [(1, 64, 24, 6, 2), (8, 40, 10, 3, 3), (8, 128, 64, 16, 4), (7, 64, 16, 256, 9), (2, 16, 8, 1, 1), (5, 14, 6, 70, 8)])
+def test_choice_by_the_largest_logits_inside_the_experts_first_launch(T, W, F, E, top):
+    """against the choice in a launch of its own and the experts behind it: ties, all equal, some at -inf; a row that has no numbers has experts nevertheless, and the rows beside it
+    what they have without it"""
+    rng = np.random.default_rng(T + W + E)
+    h, z = rng.standard_normal((T, W)).astype(np.float32), rng.standard_normal((T, E + 3)).astype(np.float32)
+    z[0, 1:3] = 2.5
+    for t, row in ((1, np.zeros(E)), (3, np.where(np.arange(E) % 2, -np.inf, 1.0)), (6, np.full(E, np.nan))):
+        if t < T:
+            z[t, :E] = row
+    gu, dd = devbf(bf16_round(rng.standard_normal((E * 2 * F, W)) / np.sqrt(W))), devbf(bf16_round(rng.standard_normal((E * W, F)) / np.sqrt(F)))
+    L, Z, dh, dz = capi(), C.c_size_t, dev32(h), dev32(z)
+    nb = L.ifa_moe_workspace_bytes(T, top, W, 3 * F, E)
+    ws = torch.zeros((nb + 15) // 4, dtype=torch.float32, device="cuda")
+    idx, idx_w = (torch.full((T, top), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    wgt, wgt_w = (torch.zeros((T, top), dtype=torch.float32, device="cuda") for _ in range(2))
+    y, y_w = (torch.full((T, W + 1), 0.5, dtype=torch.float32, device="cuda") for _ in range(2))
+    ia.check(L.ifa_moe_experts_gated_top_rows(p(dz), Z(E + 3), p(dh), Z(W), Z(T), W, F, E, top, p(gu), p(dd), p(idx), p(wgt), p(ws), Z(nb), p(y), Z(W + 1), 1, None)); sync()
+    some = [t for t in range(T) if t != 6]
+    ia.check(L.ifa_moe_route_top_f32(p(dz), E + 3, T, E, top, None, p(idx_w), p(wgt_w), None))
+    got, i, iw = y.cpu().numpy(), idx.cpu().numpy(), idx_w.cpu().numpy()
+    assert i.min() >= 0 and i.max() < E and all(len(set(r)) == top for r in i.tolist())
+    finite = [t for t in some if np.isfinite(np.take_along_axis(z[t], i[t], 0)).all()]
+    assert np.array_equal(i[finite], iw[finite]) and np.abs(wgt.cpu().numpy()[finite] - wgt_w.cpu().numpy()[finite]).max() < 1e-6
+    idx_w.copy_(idx); wgt_w.copy_(wgt)
+    ia.check(L.ifa_moe_experts_gated_f32(p(dh), W, T, W, F, E, top, p(gu), p(dd), p(idx_w), p(wgt_w), 1, p(ws), nb, p(y_w), W + 1, 1, None)); sync()
+    assert np.array_equal(got, y_w.cpu().numpy(), equal_nan=True) and np.isfinite(got[some]).all() and (T <= 6 or np.isnan(got[6, :W]).all())
+
+
 @pytest.mark.parametrize("T,W,F,E,top", [(1, 64, 24, 6, 2), (3, 40, 10, 3, 3), (8, 128, 64, 16, 4), (9, 64, 24, 6, 2), (70, 48, 20, 5, 1), (150, 64, 32, 20, 3), (5, 14, 6, 4, 2)])
 def test_gated_experts_in_rows_and_grouped(T, W, F, E, top):
     rng = np.random.default_rng(T + W + F)
