@@ -499,8 +499,6 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass(const half_t *__rest
     // scores of key block kb for this wave's 32 queries: x[r] = kq_scale * half(alpha * q.k (+ ALiBi)), key = 32 kb + row(r)
     // scores of key block kb for this wave's 32 queries:  x[r] = half(alpha * q.k (+ ALiBi)) as float,  key = 32 kb + row(r);
     // masked keys: -inf.  exp(kq_scale * x - max) is then exp2(fma(log2(e) * kq_scale, x, c)) with c = -log2(e) * kq_scale * max.
-    // (ALiBi is a template parameter: its test inside the unrolled loop was sixteen branches a block.  Scores and probabilities stay pairs of halves, converted and compared two at a time:
-    // 32 heads of 128, 2048 tokens 147 -> 125 -> 120 us, 512 tokens 26 -> 22, 512 behind 1500 82 -> 65)
     // (the kernel is VALU-bound -- ~10 instructions per score and pass against 16 MFMAs per 512 scores -- so the mask is
     // applied only in blocks that reach past the wave's first query, and the exponent is one fma + v_exp_f32)
     const float l2e_kq = 1.44269504088896341f * kq_scale;
@@ -746,6 +744,8 @@ __global__ void __launch_bounds__(256, 2) k_attention_2pass_ks(const half_t *__r
     // scores of key block kb for this wave's 32 queries: x[r] = kq_scale * half(alpha * q.k (+ ALiBi)), key = 32 kb + row(r)
     // scores of key block kb for this wave's 32 queries:  x[r] = half(alpha * q.k (+ ALiBi)) as float,  key = 32 kb + row(r);
     // masked keys: -inf.  exp(kq_scale * x - max) is then exp2(fma(log2(e) * kq_scale, x, c)) with c = -log2(e) * kq_scale * max.
+    // (ALiBi is a template parameter: its test inside the unrolled loop was sixteen branches a block.  Scores and probabilities stay pairs of halves, converted and compared two at a time:
+    // 32 heads of 128, 2048 tokens 147 -> 125 -> 120 us, 512 tokens 26 -> 22, 512 behind 1500 82 -> 65)
     // (the kernel is VALU-bound -- ~10 instructions per score and pass against 16 MFMAs per 512 scores -- so the mask is
     // applied only in blocks that reach past the wave's first query, and the exponent is one fma + v_exp_f32)
     const float l2e_kq = 1.44269504088896341f * kq_scale;

@@ -457,6 +457,7 @@ bool batch_fused_ok(const ifa_model *m, int n)
     if (D % 128 || QD % 128 || F % 128 || D > 4096 || KVD % 16 || D % 16 || F % 16) return false;
     if (c.head_dim != 32 && c.head_dim != 48 && c.head_dim != 64 && c.head_dim != 80 && c.head_dim != 96 && c.head_dim != 128) return false;
     if (c.kv_dtype == Q8_B32T2 && c.head_dim % 32 != 0) return false;
+    // (contexts of some 70 000 keys and more: the limit of a kernel that held the score row in LDS; k_dec_attn_keys holds none and has not been measured there)
     if (dec_attn_smem(c.head_dim, c.max_ctx) > IFA_LDS_LIMIT) return false;
     for (const Layer &L : m->layers) {
         const bool moe = c.experts > 0 && L.t[T_MOE_GATE].present();      // MoE layers: the attention half is fused, the FFN runs moe_ffn

@@ -589,7 +589,8 @@ int lin_grouped_dispatch(const LinTileArgs<MODE> &P, const bf16_t *a, size_t lda
 {
     IFA_REQUIRE(max_tiles * lin_col_tiles(P, 64) < (1u << 31), "linear_bf16_grouped: too many tiles");
     // (8192 pairs of 16 experts, 1408 x 1024 gate | up and 1024 x 704, us: four waves a 128 x 128 tile 54.8 + 46.8, eight 47.9 + 40.4; 2900 pairs: 64 x 64 tiles 34.2 + 18.8, 64 x 128 of
-    // eight waves 27.0 + 17.0)
+    // eight waves 27.0 + 17.0; whole experts, sort and sums with them, 36 pairs of these 28.7 -> 25.3, 64 pairs 29.5 -> 25.9, 54 pairs of 32 experts 2816 x 2048 and 2048 x 1408 132.6 -> 115.0,
+    // 18 pairs of 8 experts 512 x 512 and 512 x 256 19.2 -> 18.4)
     if (tile_rows == 128) return launch_lin_tile<128, 128, 2, 4, 2, MODE>(P, a, lda, max_tiles, s);
     if (lda >= 3 * LT_BK) return launch_lin_tile<64, 128, 2, 4, 3, MODE>(P, a, lda, max_tiles, s);
     return launch_lin_tile<64, 64, 2, 2, 2, MODE>(P, a, lda, max_tiles, s);

@@ -491,8 +491,8 @@ def test_dynamic_batching_rows_are_independent_queries(kvd):
 
 @pytest.mark.parametrize("kvd", [dt.F16, dt.Q8_B32T2], ids=["kvf16", "kvq8"])
 def test_batched_step_at_contexts_past_the_prefetched_bucket(kvd):
-    """Queries with several hundred cached keys in one batched step: k_dec_attn<.., BATCH> walks the keys past its 256-row entry prefetch
-    in 256-key iterations (K rows one iteration ahead) and the V rows in double-buffered batches of eight keys (round 6).  Every row
+    """Queries with several hundred cached keys in one batched step: k_dec_attn_keys shares a query's keys out to splits of 256, each
+    walked in passes of the rows that are requested together.  Every row
     against the same query decoded alone on a copy of its cache through the single-query step (at these contexts: the keys-split-over-
     workgroups kernels; Q8 activations alone vs F16 activations batched: the tolerance of test_dynamic_batching_rows_are_independent_queries),
     the fused step against the op-by-op rows, and row order must not matter (identical bits under permutation)."""

@@ -1,6 +1,6 @@
 // valu_rate_probe.hip -- issue cost (cycles per wave instruction) of the VALU instructions of the Q4 dequantisation on gfx950:
-// v_cvt_pk_f32_fp8, v_pk_fma_f32, v_cvt_pk_f16_f32, v_cvt_f32_ubyteN, v_dot2c_f32_f16, and the whole q4x8_dequant (15
-// instructions per 8 weights) -- one wave per SIMD and two, against a dependent v_add_f32 chain (4 cycles per instruction) that
+// v_cvt_pk_f32_fp8, v_pk_fma_f16, v_cvt_pk_f16_f32, v_cvt_f32_ubyteN, v_dot2c_f32_f16, and the whole q4x8_dequant (in the tiled
+// order: 15 instructions per 8 weights, 11 in the MFMA operand order) -- one wave per SIMD and two, against a dependent v_add_f32 chain (4 cycles per instruction) that
 // also gives the shader clock.   hipcc --offload-arch=gfx950 -O3 -I inferflow_amd/csrc -o valu_rate_probe valu_rate_probe.hip
 #include <hip/hip_runtime.h>
 #include <cstdio>
@@ -30,13 +30,13 @@ __global__ void k(int iters, float *out, long long *ticks, uint32_t seed)
                 asm volatile("v_cvt_pk_f32_fp8 %0, %1" : "=v"(p2) : "v"(w2));
                 asm volatile("v_cvt_pk_f32_fp8 %0, %1" : "=v"(p3) : "v"(w3));
             }
-        } else if constexpr (MODE == 2) {   // 16 independent v_pk_fma_f32
+        } else if constexpr (MODE == 2) {   // 16 independent v_pk_fma_f16
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                asm volatile("v_pk_fma_f32 %0, %1, %2, %0" : "+v"(p0) : "v"(p1), "v"(p2));
-                asm volatile("v_pk_fma_f32 %0, %1, %2, %0" : "+v"(p1) : "v"(p2), "v"(p3));
-                asm volatile("v_pk_fma_f32 %0, %1, %2, %0" : "+v"(p2) : "v"(p3), "v"(p0));
-                asm volatile("v_pk_fma_f32 %0, %1, %2, %0" : "+v"(p3) : "v"(p0), "v"(p1));
+                asm volatile("v_pk_fma_f16 %0, %1, %2, %0" : "+v"(w0) : "v"(w1), "v"(w2));
+                asm volatile("v_pk_fma_f16 %0, %1, %2, %0" : "+v"(w1) : "v"(w2), "v"(w3));
+                asm volatile("v_pk_fma_f16 %0, %1, %2, %0" : "+v"(w2) : "v"(w3), "v"(w0));
+                asm volatile("v_pk_fma_f16 %0, %1, %2, %0" : "+v"(w3) : "v"(w0), "v"(w1));
             }
         } else if constexpr (MODE == 3) {   // 16 v_cvt_pk_f16_f32
 #pragma unroll
@@ -62,12 +62,12 @@ __global__ void k(int iters, float *out, long long *ticks, uint32_t seed)
                 asm volatile("v_dot2c_f32_f16 %0, %1, %2" : "+v"(p2[0]) : "v"(w2), "v"(w3));
                 asm volatile("v_dot2c_f32_f16 %0, %1, %2" : "+v"(p3[0]) : "v"(w3), "v"(w0));
             }
-        } else {                             // MODE 6: two whole q4x8_dequant (30 instructions, 16 weights)
+        } else {                             // MODE 6: two whole q4x8_dequant (16 weights)
             q4_h2 w[4];
-            q4x8_dequant(w0, a, b, w);
+            q4x8_dequant(w0, q4_scale2(w2), q4_base2(w2), w);
             asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
             w0 ^= __builtin_bit_cast(uint32_t, w[0]);
-            q4x8_dequant(w1, b, a, w);
+            q4x8_dequant(w1, q4_scale2(w3), q4_base2(w3), w);
             asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
             w1 ^= __builtin_bit_cast(uint32_t, w[3]);
         }
@@ -108,7 +108,7 @@ int main()
     printf("dependent v_add_f32: %.3f ns each -> %.2f GHz if 4 cycles\n", ns_per_add, ghz);
     run<0>("v_add_f32 (dependent)", 16, out, ticks, ghz);
     run<1>("v_cvt_pk_f32_fp8", 16, out, ticks, ghz);
-    run<2>("v_pk_fma_f32", 16, out, ticks, ghz);
+    run<2>("v_pk_fma_f16", 16, out, ticks, ghz);
     run<3>("v_cvt_pk_f16_f32", 16, out, ticks, ghz);
     run<4>("v_cvt_f32_ubyteN", 16, out, ticks, ghz);
     run<5>("v_dot2c_f32_f16", 16, out, ticks, ghz);
