@@ -561,7 +561,8 @@ int lin_tile_dispatch(const LinTileArgs<MODE> &P, const bf16_t *a, size_t lda, h
     // 128 x 128 tiles would give some compute units one workgroup and some two, 128 x 64 tiles of four waves, three a compute unit, share out more evenly.  us 128 x 128 / 128 x 64 (as before the
     // shapes below), tokens x columns x K: 411 x 11264 x 256, 512, 1024, 2048 9.4 / 8.7, 13.4 / 12.7, 21.7 / 20.7, 37.5 / 35.4; 601 x 6700 x 1024 19.8 / 18.9, x 2048 33.8 / 31.7;
     // 1233 x 3500 x 704, 1408 15.3 / 14.8, 24.9 / 23.6; beyond 32 steps nothing (1000 x 5632 x 4096 68.2 / 68.4, 1233 x 4600 x 5632 90.9 / 95.6)
-    if (t128 * n64 > 512 && t128 * n128 < 384 && steps <= 32) return launch_lin_tile<128, 64, 2, 2, 2, MODE>(P, a, lda, t128, s);
+    // (few steps, below: where 64 x 64 tiles of two buffers would have no place at once, four a compute unit: gated, 800 x 4816 x 256 8.0 us with those, 10.0 with these; 1000 x 4816 11.2, 10.3)
+    if (t128 * n64 > 512 && t128 * n128 < 384 && steps <= 32 && (steps >= 5 || t64 * n64 > 1024)) return launch_lin_tile<128, 64, 2, 2, 2, MODE>(P, a, lda, t128, s);
     if (steps < 5) {
         // Fewer steps than the buffers of the tiles below: two buffers, but 64 x 64 tiles that all have a place at once take four where there are four steps.  us with 64 x 64 of two buffers,
         // 64 x 64 of four, 128 x 64 (four waves, three workgroups a compute unit), 128 x 128 -- four steps, tokens x columns: 16 x 4096 4.4, 3.8, 5.2, 5.6; 1000 x 1024 4.5, 4.2, 5.4, 5.8;
