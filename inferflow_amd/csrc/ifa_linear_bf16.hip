@@ -219,13 +219,8 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
         }
     }
     // a tile of gates and ups: o0, its first output
-    int o0 = 0, n_end = P.N, K0 = P.K;
-    bool glu = false;
-    if constexpr (GLU) {
-        const int n_tile = n0 / BN, n_plain = (P.glu_c0 + BN - 1) / BN;
-        glu = n_tile >= n_plain; o0 = (n_tile - n_plain) * (BN / 2); n_end = P.glu_c0;
-    }
-    if constexpr (SUM) { Wg = P.part[0].W; K0 = P.part[0].K; }
+    const int n_end = [&]() { if constexpr (GLU) return P.glu_c0; else return P.N; }(), n_plain = GLU ? (n_end + BN - 1) / BN : 0, o0 = (n0 / BN - n_plain) * (BN / 2);
+    const bool glu = GLU && n0 / BN >= n_plain;
     auto swz = [](int r) { return (r >> 1) & 7; };
     const bf16_t *asrc[AI], *wsrc[WI];
     int wlim[WI];          // furthest step offset of the lane's piece inside a row of W
@@ -241,12 +236,14 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
         const int row = (wave * WI + j) * 8 + (lane >> 3), c = (lane & 7) ^ swz(row);
         int wr = min(n0 + row, n_end - 1);
         if constexpr (GLU) if (glu) wr = P.glu_c0 + ((row & 16) ? P.glu_f : 0) + min(o0 + 16 * (row >> 5) + (row & 15), P.glu_f - 1);
-        wsrc[j] = Wg + (size_t)wr * K0 + c * 8;
-        wlim[j] = K0 - 8 - c * 8;
+        const bf16_t *W0 = Wg;
+        int K = P.K;
+        if constexpr (SUM) { W0 = P.part[0].W; K = P.part[0].K; }
+        wsrc[j] = W0 + (size_t)wr * K + c * 8;
+        wlim[j] = K - 8 - c * 8;
     }
     // (SUM) the part that the next requested step belongs to, from its first step to the one behind its last; likewise for the next step of products
-    int q_part = 0, q_from = 0, q_to = 0, c_part = 0, c_to = 0;
-    if constexpr (SUM) q_to = c_to = P.part[0].steps;
+    int q_part = 0, q_from = 0, q_to = [&]() { if constexpr (SUM) return P.part[0].steps; else return 0; }(), c_part = 0, c_to = q_to;
     auto enter = [&](int step) {
         if constexpr (SUM) {
             if (step != q_to) return;
