@@ -178,6 +178,77 @@ bool prefill_mid_ok(ifa_model *m, int T, bool any_length)
     return true;
 }
 
+// FEW_MIN .. FEW_MAX rows through gemm_few: dense layers with the sequential RMS wiring, every linear with its operand-order copy (built here on first use, like the workspace, whose
+// addresses captured steps hold: one size for every number of rows)
+bool rows_few_ok(ifa_model *m, int T)
+{
+    const ifa_model_config &c = m->cfg;
+    if (!m->opt_rows_few || !m->opt_rows_mo || T < FEW_MIN || T > FEW_MAX || c.experts != 0 || c.norm_kind != 0 || c.dim > 8192 || !prefill_big_ok(m)) return false;
+    const size_t D = c.dim, QD = (size_t)c.heads * c.head_dim, KVD = (size_t)c.kv_heads * c.head_dim, F = c.ffn;
+    if (!few_ok(QD, D) || !few_ok(KVD, D) || !few_ok(D, QD) || !few_ok(F, D) || !few_ok(D, F) || ensure_mo(m) != IFA_OK) return false;
+    for (const Layer &L : m->layers) {
+        const int ids[] = {T_WQ, T_WK, T_WV, T_WO, T_W1, T_W3, T_W2};
+        for (int id : ids) if (!L.t[id].present() || !L.t[id].mo) return false;
+    }
+    if (!m->few.x) {
+        const size_t nx = few_frag_bytes(FEW_MAX, D), nf = few_frag_bytes(FEW_MAX, F), ns = (size_t)FEW_PARTS * FEW_MAX * D * sizeof(float);
+        char *p = nullptr;
+        if (hipMalloc((void **)&p, nx + nf + ns) != hipSuccess) { (void)hipGetLastError(); m->opt_rows_few = 0; return false; }
+        m->few = {(half_t *)p, (half_t *)(p + nx), (float *)(p + nx + nf)};
+    }
+    return true;
+}
+
+static FewArgs few_args(const ifa_model *m, int T)
+{
+    FewArgs P; memset(&P, 0, sizeof(P));
+    P.T = T; P.nsets = 1; P.act_kind = m->cfg.act_kind;
+    return P;
+}
+
+// the norm in front of layer l (l == layers: none) of the sums of product W, or of x itself (W null); x_out: the rows that it is formed of
+static int few_norm(ifa_model *m, int l, int id, int T, const Tensor *W, const Tensor *bias, const half_t *x, half_t *x_out)
+{
+    const ifa_model_config &c = m->cfg;
+    const bool norm = l < c.layers;
+    const Layer *L = norm ? &m->layers[(size_t)l] : nullptr;
+    const int idb = id == T_ATTN_NORM ? T_ATTN_NORM_B : T_FFN_NORM_B;
+    return few_sum_norm(m->few.sums, W ? few_parts(W->rows, W->cols) : 0, bias ? (const half_t *)bias->data : nullptr, x, x_out, T, c.dim, norm ? (const half_t *)L->t[id].data : nullptr,
+                        norm ? (const half_t *)L->t[idb].data : nullptr, id == T_ATTN_NORM ? c.attn_norm_base : c.ffn_norm_base, c.eps, norm ? m->few.x : nullptr, m->stream);
+}
+
+// wq | wk | wv of the normed rows in m->few.x (few_norm)
+static int few_qkv(ifa_model *m, const Layer &L, int T, half_t *q, half_t *k, half_t *v, int ldq, int ldkv)
+{
+    const ifa_model_config &c = m->cfg;
+    FewArgs P = few_args(m, T);
+    const int ids[] = {T_WQ, T_WK, T_WV}, idb[] = {T_WQ_B, T_WK_B, T_WV_B};
+    for (int i = 0; i < 3; i++) { P.W[i] = (const uint8_t *)L.t[ids[i]].mo; P.bias[i] = (const half_t *)L.t[idb[i]].data; P.rows[i] = i == 0 ? c.heads * c.head_dim : c.kv_heads * c.head_dim; }
+    P.nsets = 3; P.K = c.dim; P.X = m->few.x;
+    P.Y[0] = q; P.Y[1] = k; P.Y[2] = v; P.ldy[0] = ldq; P.ldy[1] = P.ldy[2] = ldkv;
+    return gemm_few(P, FEW_ROWS, m->stream);
+}
+
+// the layer behind its attention (rows of m->att): wo + residual, norm, gated pair, w2 + residual -> xnext, the next layer's norm -> m->few.x
+static int few_tail(ifa_model *m, int l, int T, const half_t *x, half_t *xnext)
+{
+    const ifa_model_config &c = m->cfg;
+    const Layer &L = m->layers[(size_t)l];
+    int rc;
+    FewArgs P = few_args(m, T);
+    P.W[0] = (const uint8_t *)L.t[T_WO].mo; P.rows[0] = c.dim; P.K = P.ldx = c.heads * c.head_dim; P.X = m->att; P.sums = m->few.sums;
+    if ((rc = gemm_few(P, FEW_SUMS, m->stream))) return rc;
+    if ((rc = few_norm(m, l, T_FFN_NORM, T, &L.t[T_WO], &L.t[T_WO_B], x, m->a))) return rc;
+    P = few_args(m, T);
+    P.W[0] = (const uint8_t *)L.t[T_W1].mo; P.W1 = (const uint8_t *)L.t[T_W3].mo; P.bias[0] = (const half_t *)L.t[T_W1_B].data; P.bias1 = (const half_t *)L.t[T_W3_B].data;
+    P.rows[0] = c.ffn; P.K = c.dim; P.X = m->few.x; P.Y[0] = m->few.ff;
+    if ((rc = gemm_few(P, FEW_GLU, m->stream))) return rc;
+    P = few_args(m, T);
+    P.W[0] = (const uint8_t *)L.t[T_W2].mo; P.rows[0] = c.dim; P.K = c.ffn; P.X = m->few.ff; P.sums = m->few.sums;
+    if ((rc = gemm_few(P, FEW_SUMS, m->stream))) return rc;
+    return few_norm(m, l + 1, T_ATTN_NORM, T, &L.t[T_W2], &L.t[T_W2_B], m->a, xnext);
+}
+
 int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, void *logits_out, int *next_token, bool no_head)
 {
     const ifa_model_config &c = m->cfg;
@@ -214,18 +285,20 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
     // weights dequantised once per workgroup and step into LDS; reference-layout rows), norms as their own launches.
     // the mid-length kernel (33 .. prefill_mid_max tokens): every linear of every layer a 4-bit tensor with its operand-order copy, dense FFN
     const bool pstat = m->opt_perf_stat != 0;       // per-phase times: the op-by-op layer below (one launch per reference op), never the fused routes
-    const bool pf_mid = !tp && !pstat && prefill_mid_ok(m, T, false);
-    const bool pf_big = pf_mid || (!tp && !pstat && T > std::max(32, m->opt_prefill_big_min) && prefill_big_ok(m));
+    const bool pf_few = !tp && !pstat && (T <= 32 ? m->opt_batch_fused : m->opt_prefill_mid) && rows_few_ok(m, T);      // (FEW_MIN .. FEW_MAX tokens: gemm_few)
+    const bool pf_mid = !pf_few && !tp && !pstat && prefill_mid_ok(m, T, false);
+    const bool pf_big = pf_few || pf_mid || (!tp && !pstat && T > std::max(32, m->opt_prefill_big_min) && prefill_big_ok(m));
     bool pf_fused = pf_big || (!tp && !pstat && T >= 2 && T <= 32 && batch_fused_ok(m, T) && c.experts == 0);
     if (pf_fused && !pf_big) {
         if ((rc = ensure_mo(m))) return rc;
         pf_fused = batch_fused_ok(m, T);          // (ensure_mo may have switched the copies off: ask again, see forward_batch)
     }
-    if (pf_big && !pf_mid && (rc = ensure_x32(m))) return rc;
+    if (pf_big && !pf_mid && !pf_few && (rc = ensure_x32(m))) return rc;
     // above prefill_mid_max: wo and w2 (4096 output columns: 128 x 128 tiles whatever the kernel) still through k_gemm_mid -- at 1024 tokens
     // 41 / 102 us per launch against 51 / 143 for the split-K halves of the large-tile kernel, which keeps wq | wk | wv and the gated pair
     // (profiles/r06_prefill_mid_parts.log section 13: 1024 / 1536 / 2048 tokens 4.5 / 3 / 0.8 % faster, 4096 tokens 4.7 % slower: up to 2048)
-    const bool pf_res_mid = pf_big && !pf_mid && !tp && T <= m->opt_prefill_res_mid && prefill_mid_ok(m, T, true);
+    const bool pf_res_mid = pf_big && !pf_mid && !pf_few && !tp && T <= m->opt_prefill_res_mid && prefill_mid_ok(m, T, true);
+    if (pf_few && (rc = few_norm(m, 0, T_ATTN_NORM, T, nullptr, nullptr, x, nullptr))) return rc;
     for (int l = 0; l < c.layers && pf_fused; l++) {
         Layer &L = m->layers[l];
         const size_t F = c.ffn;
@@ -241,14 +314,15 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
         GmArgs P;
         auto clear = [&]() { memset(&P, 0, sizeof(P)); P.T = T; P.eps = c.eps; P.act_kind = c.act_kind; P.mo = mo_flag; P.no_waits = pf_big ? !m->opt_gemm_splitk : !m->opt_rows_kparts; };
         clear();
-        if (!norm_fused && (rc = norm_rows(m, x, T, L.t[T_ATTN_NORM], pf_big ? L.t[T_ATTN_NORM_B] : nob, m->xn, c.attn_norm_base))) return rc;
+        if (pf_few) { if ((rc = few_qkv(m, L, T, m->q, m->k, m->v, (int)QD, (int)KVD))) return rc; }
+        else if (!norm_fused && (rc = norm_rows(m, x, T, L.t[T_ATTN_NORM], pf_big ? L.t[T_ATTN_NORM_B] : nob, m->xn, c.attn_norm_base))) return rc;
         P.W[0] = wp(T_WQ); P.W[1] = wp(T_WK); P.W[2] = wp(T_WV);
         P.rows[0] = (int)QD; P.rows[1] = (int)KVD; P.rows[2] = (int)KVD; P.nsets = 3; P.nblk = (int)(D / 32);
         P.X = norm_fused ? x : m->xn; P.ldx = (int)D;
         if (norm_fused) { P.norm_w = (const half_t *)L.t[T_ATTN_NORM].data; P.multi_base = c.attn_norm_base; }
         P.bias[0] = (const half_t *)L.t[T_WQ_B].data; P.bias[1] = (const half_t *)L.t[T_WK_B].data; P.bias[2] = (const half_t *)L.t[T_WV_B].data;
         P.Yset[0] = m->q; P.Yset[1] = m->k; P.Yset[2] = m->v; P.ldyset[0] = (int)QD; P.ldyset[1] = (int)KVD; P.ldyset[2] = (int)KVD;
-        if ((rc = lin(P, T_WQ, GM_PLAIN, norm_fused ? 1 : 0))) return rc;
+        if (!pf_few && (rc = lin(P, T_WQ, GM_PLAIN, norm_fused ? 1 : 0))) return rc;
         uint8_t *kdst = (uint8_t *)L.kcache + (size_t)prefix_len * m->kv_row_bytes;
         uint8_t *vdst = (uint8_t *)L.vcache + (size_t)prefix_len * m->kv_row_bytes;
         const bool kv_f16 = c.kv_dtype != Q8_B32T2;
@@ -273,6 +347,12 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
         if ((rc = ifa_attention(m->q, L.kcache, L.vcache, c.kv_dtype, prefix_len + T, T, prefix_len, c.heads, c.kv_heads,
                                 c.head_dim, c.use_alibi ? 1.0f : c.kq_scale, c.use_alibi, c.tp_rank * c.heads,
                                 c.heads * std::max(1, c.tp_size), m->att, s))) return rc;
+        if (pf_few) {
+            if ((rc = few_tail(m, l, T, x, m->f))) return rc;
+            std::swap(m->x, m->f);
+            x = m->x;
+            continue;
+        }
         clear();
         P.W[0] = wp(T_WO); P.rows[0] = (int)D; P.nsets = 1; P.nblk = (int)(QD / 32);
         P.X = m->att; P.ldx = (int)QD; P.bias[0] = (const half_t *)L.t[T_WO_B].data;
@@ -509,14 +589,20 @@ int batch_fused_layer(ifa_model *m, int l, int n, const half_t *x, half_t *xnext
     P.W[0] = rows_w(m, L.t[T_WQ]); P.W[1] = rows_w(m, L.t[T_WK]); P.W[2] = rows_w(m, L.t[T_WV]); P.mo = rows_mo(m, L.t[T_WQ]);
     P.rows[0] = (int)QD; P.rows[1] = (int)KVD; P.rows[2] = (int)KVD; P.nsets = 3; P.nblk = (int)(D / 32);
     // (9..16 queries: the activation rows are staged in chunks of 2048 columns, so the norm runs as its own launch)
+    const bool few = n >= FEW_MIN && rows_few_ok(m, n);
+    if (few) {
+        if (l == 0 && (rc = few_norm(m, 0, T_ATTN_NORM, n, nullptr, nullptr, x, nullptr))) return rc;
+        const int ld = (int)(QD + 2 * KVD);
+        if ((rc = few_qkv(m, L, n, m->bqkv, m->bqkv + QD, m->bqkv + QD + KVD, ld, ld))) return rc;
+    }
     const bool norm_fused = (n <= 8 || rows_mo(m, L.t[T_WQ])) && n <= 16;      // (MO layout: 16 rows x 4096 columns are one chunk too; 17..32 rows: chunked)
     Tensor nob;
-    if (!norm_fused && (rc = norm_rows(m, x, n, L.t[T_ATTN_NORM], nob, m->xn, c.attn_norm_base))) return rc;
+    if (!few && !norm_fused && (rc = norm_rows(m, x, n, L.t[T_ATTN_NORM], nob, m->xn, c.attn_norm_base))) return rc;
     P.X = norm_fused ? x : m->xn; P.ldx = (int)D;
     if (norm_fused) { P.norm_w = (const half_t *)L.t[T_ATTN_NORM].data; P.multi_base = c.attn_norm_base; }
     P.bias[0] = (const half_t *)L.t[T_WQ_B].data; P.bias[1] = (const half_t *)L.t[T_WK_B].data; P.bias[2] = (const half_t *)L.t[T_WV_B].data;
     P.Y = m->bqkv; P.ldy = (int)(QD + 2 * KVD);
-    if ((rc = gemm_rows_mfma_launch(P, GM_PLAIN, norm_fused ? 1 : 0, m->stream))) return rc;
+    if (!few && (rc = gemm_rows_mfma_launch(P, GM_PLAIN, norm_fused ? 1 : 0, m->stream))) return rc;
     // 2. RoPE, KV store, attention of every query on its own cache
     {
         const int rope_dims = (int)(c.head_dim * c.partial_rotary + 0.5f);
@@ -529,6 +615,7 @@ int batch_fused_layer(ifa_model *m, int l, int n, const half_t *x, half_t *xnext
         A.out = m->att; A.max_ctx = c.max_ctx; A.batch_rows = rows_l; A.q_stride = (int)(QD + 2 * KVD);
         if ((rc = launch_attn_keys(A, m->keys_ws, c.head_dim, dec_keys_splits(c.heads, n, c.max_ctx), n, m->stream))) return rc;
     }
+    if (few) return few_tail(m, l, n, x, xnext);
     // 3. wo (+ bias) + residual
     clear();
     P.W[0] = rows_w(m, L.t[T_WO]); P.mo = rows_mo(m, L.t[T_WO]); P.rows[0] = (int)D; P.nsets = 1; P.nblk = (int)(QD / 32);
@@ -618,6 +705,7 @@ int forward_batch(ifa_model *m, int n, const int *tokens_host, const int *pos_ho
         // is chosen; a step the tiled kernels do not cover takes the op-by-op rows below
         fused = batch_fused_ok(m, n);
         if (fused && (rcm = gemm_rows_kparts_reserve(m->stream))) return rcm;
+        if (fused) (void)rows_few_ok(m, n);      // (its workspace, before a capture)
     }
     if (has_moe && m->opt_moe_overlap) { int rcs = ensure_side_stream(m); if (rcs) return rcs; }
     // (MoE layers of the fused step route on the device -- no host round trip -- so they are captured too)

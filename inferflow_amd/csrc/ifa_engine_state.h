@@ -22,6 +22,7 @@
 #include "ifa_moe.h"
 #include "ifa_gemm_rows_mfma.h"
 #include "ifa_gemm_big.h"
+#include "ifa_gemm_few.h"
 #include "ifa_decode_lmhead_tail.h"
 #include "ifa_decode_singles.h"
 #include "ifa_decode_qkv_attn.h"
@@ -213,6 +214,10 @@ struct ifa_model {
     // operand-order copy; 320..768 tokens 8-9 % faster than the large tiles, 1024 tokens a tie (profiles/r06_prefill_mid_parts.log)
     int opt_prefill_mid = 1, opt_prefill_mid_max = 768;
     int opt_prefill_res_mid = 2048;   // prefill_mid_max + 1 .. this many tokens: wo / w2 still through k_gemm_mid, the other products through the large tiles (0: never)
+    // prompts of FEW_MIN .. FEW_MAX tokens and steps of as many queries through gemm_few (ifa_gemm_few.hip); its workspace, one allocation: rows in fragment order (a layer's
+    // input, the gated pair's output), sums of the parts of K
+    int opt_rows_few = 1;
+    struct { half_t *x, *ff; float *sums; } few = {nullptr, nullptr, nullptr};
     int opt_rows_kparts = 1, opt_gemm_splitk = 1;   // 0: never the launches whose workgroups wait for partner workgroups (K parts of the 9..32-row GEMM, split-K halves of the large-tile GEMM)
     int opt_debug_mo_alloc_fail = 0;           // tests: ensure_mo_build fails like an exhausted allocator after its first copy
     static constexpr int RING = 1024;
@@ -356,6 +361,7 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
 bool batch_fused_ok(const ifa_model *m, int n);
 bool prefill_big_ok(const ifa_model *m);
 bool prefill_mid_ok(ifa_model *m, int T, bool any_length);
+bool rows_few_ok(ifa_model *m, int T);
 int batch_fused_layer(ifa_model *m, int l, int n, const half_t *x, half_t *xnext, const void *rows_l);
 int forward_batch(ifa_model *m, int n, const int *tokens_host, const int *pos_host, const int *slot_host, int *next_tokens,
                          void *logits_out);

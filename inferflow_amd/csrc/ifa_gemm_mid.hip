@@ -114,8 +114,8 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
     // contiguous KiB -- lane 16 g + r holds the 16 code bytes of block 4 S + g of row r -- so a tile's K range is one linear stream,
     // like a decode row; the tiled rows fetched 32 bytes per row and step measured 1 TB/s: 32 DRAM pages per request).  A step is
     // half a superstep: lane -> (tile l / 32, block (l / 16) % 2 of the half, row l % 16), 2 x 512 contiguous bytes per request.
-    const int nsup = nblk >> 2, nq4 = (nsup + 3) >> 2;
-    const size_t mo_tile = (size_t)(nsup + nq4) * 1024;
+    const int nsup = nblk >> 2;
+    const size_t mo_tile = mo_tile_bytes(nsup);
     const uint8_t *wsrc, *wsbs;
     {
         const int nl0 = wave * 32;
@@ -123,7 +123,7 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
         const int row0 = n0 + (GLU && nl0 >= BNE ? nl0 - BNE : nl0);
         const int tile16 = min((row0 >> 4) + (lane >> 5), ((N + 15) >> 4) - 1);
         wsrc = Wm + (size_t)tile16 * mo_tile + (size_t)(lane & 31) * 16;
-        wsbs = wsrc + (size_t)nsup * 1024;
+        wsbs = Wm + (size_t)tile16 * mo_tile + mo_words_at(nsup) + (size_t)(lane & 31) * 4;
     }
     // the six requests of a stage, one at a time (piece 0..3: activation rows, 4: codes, 5: (base, scale) words): the main loop places
     // them between its MFMAs
@@ -140,7 +140,7 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
         if (piece == XP)
             __builtin_amdgcn_global_load_lds((md_glb_t *)(wsrc + (size_t)S * 1024 + (size_t)half * 512), (md_lds_t *)(st + MD_A_BYTES + wave * 1024), 16, 0, IFA_MID_WAUX);
         else
-            __builtin_amdgcn_global_load_lds((md_glb_t *)(wsbs + (size_t)(S >> 2) * 1024 + (size_t)half * 512 + (size_t)(S & 3) * 4),
+            __builtin_amdgcn_global_load_lds((md_glb_t *)(wsbs + (size_t)S * 256 + (size_t)half * 128),
                                              (md_lds_t *)(st + MD_A_BYTES + MD_WC_BYTES + wave * 256), 4, 0, IFA_MID_WAUX);
 #endif
     };

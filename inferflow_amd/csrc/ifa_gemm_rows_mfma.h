@@ -47,8 +47,13 @@ struct GmArgs {
 //   nsup = cols / 128 supersteps of 1024 bytes: lane l = 16 g + r of a wave owns bytes 16 l .. 16 l + 15 = the 16 code bytes of
 //   block 4 S + g of row 16 tile + r (exactly its A operands of the superstep's four MFMAs; byte b of a word of eight codes holds element b
 //   in its low and element 4 + b in its high nibble, the order in which ifa_dequant_q4.h needs no permutes), then
-//   ceil(nsup / 4) quads of 1024 bytes: lane l owns the (base, scale) words of its blocks in supersteps 4 Q .. 4 Q + 3.
-// Rows past the end and the pad of the last quad are zero.  Same size as the tiled copy (+ the pad).
+//   ceil(nsup / 4) quads of 1024 bytes: lane l owns the (base, scale) words of its blocks in supersteps 4 Q .. 4 Q + 3, then
+//   the same words again by supersteps, 256 bytes each (padded to whole KiB): lane l owns bytes 4 l .. 4 l + 3.  (The kernels whose waves own four supersteps in a row read the quads,
+//   one request for four; those whose waves take supersteps by turns, or halves of them, fetched every line of the quads up to four times: w1 | w3 of 48 rows 22.6 -> 21.4 us.
+//   With words by supersteps only, the batched steps of 2..16 queries were 2 to 4 % slower.)
+// Rows past the end and the pads are zero.
+constexpr size_t mo_tile_bytes(int nsup) { return (size_t)(nsup + 2 * ((nsup + 3) >> 2)) * 1024; }
+constexpr size_t mo_words_at(int nsup) { return (size_t)(nsup + ((nsup + 3) >> 2)) * 1024; }      // the words by supersteps
 size_t gemm_rows_mo_bytes(size_t rows, size_t cols);
 // dtype: Q4_B32T1A / B, or the 64-weight nibble formats Q4_B64T1 / Q3H_B64T1 (one (base, scale) per 64 weights, written for both
 // 32-weight halves: the kernel then runs unchanged; cols % 128 == 0)

@@ -37,7 +37,7 @@ template <bool B64>
 __global__ void __launch_bounds__(256) k_gemm_rows_mo_build(const uint8_t *__restrict__ tiled, int rows, int nblk, size_t row_bytes, uint8_t *__restrict__ mo)
 {
     const int nsup = nblk >> 2, nq4 = (nsup + 3) >> 2;            // nblk: 32-weight blocks per row
-    const size_t mo_tile = (size_t)(nsup + nq4) * 1024;
+    const size_t mo_tile = mo_tile_bytes(nsup);
     const int ntiles = (rows + 15) >> 4;
     const size_t total = (size_t)ntiles * nq4 * 4 * 64;            // (supersteps padded to whole quads: the pad's words are zero)
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
@@ -65,6 +65,7 @@ __global__ void __launch_bounds__(256) k_gemm_rows_mo_build(const uint8_t *__res
         uint8_t *tb = mo + (size_t)tile * mo_tile;
         if (S < nsup) *reinterpret_cast<u32x4 *>(tb + (size_t)S * 1024 + (size_t)lane * 16) = c;
         *reinterpret_cast<uint32_t *>(tb + (size_t)(nsup + (S >> 2)) * 1024 + (size_t)lane * 16 + (size_t)(S & 3) * 4) = w;
+        *reinterpret_cast<uint32_t *>(tb + mo_words_at(nsup) + (size_t)S * 256 + (size_t)lane * 4) = w;
     }
 }
 
@@ -301,8 +302,7 @@ int expand_b64_to_q4b32(int dtype, const void *tiled, size_t rows, size_t cols, 
 
 size_t gemm_rows_mo_bytes(size_t rows, size_t cols)
 {
-    const size_t nsup = cols / 128, nq4 = (nsup + 3) / 4;
-    return (rows + 15) / 16 * (nsup + nq4) * 1024;
+    return (rows + 15) / 16 * mo_tile_bytes((int)(cols / 128));
 }
 
 int gemm_rows_mo_build(int dtype, const void *tiled, size_t rows, size_t cols, void *mo, hipStream_t s)

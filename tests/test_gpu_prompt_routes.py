@@ -137,3 +137,62 @@ def test_rotation_by_four_workgroups_a_token_and_by_one_leave_the_same_bits(head
         else:
             assert not b[T - 1].any() and not b[:, kvd:].any()
     assert torch.equal(out[0][2][:, :kvd], out[0][1]) and torch.equal(out[0][3][:, :kvd], rows[2])
+
+
+def _biased(kvd, wd, T, **shape):
+    """a worker of two layers whose products and norms have biases"""
+    from inferflow_amd import worker as W
+    wk, _, s = synth.build("llama2_7b", wd, kvd, max_ctx=T + 16, layers=2, vocab=600, quant_threshold=0, **shape)
+    gen = torch.Generator(device="cuda"); gen.manual_seed(1)
+    qd, kvdim = s["heads"] * s["head_dim"], s["kv_heads"] * s["head_dim"]
+    for l in range(2):
+        for tid, n in ((W.T_WQ_B, qd), (W.T_WK_B, kvdim), (W.T_WV_B, kvdim), (W.T_WO_B, s["dim"]), (W.T_W1_B, s["ffn"]), (W.T_W3_B, s["ffn"]), (W.T_W2_B, s["dim"])):
+            wk.set_tensor_f16(l, tid, dt.F16, (0.3 * torch.randn(n, generator=gen, device="cuda")).half(), 1, n)
+    return wk, s
+
+
+@pytest.mark.parametrize("T", [9, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97, 128, 129, 191, 192])
+@pytest.mark.parametrize("wd,shape", [(dt.Q4_B32T1A, {}), (dt.Q3H_B64T1, dict(dim=1024, heads=16, kv_heads=2, head_dim=64, ffn=1408)), (dt.Q4_B32T1B, dict(dim=2176, heads=9, kv_heads=3, ffn=3712))],
+                         ids=["7b", "w1024", "w2176"])
+def test_products_that_stream_their_weights_over_few_rows_agree_with_the_others(wd, shape, T):
+    """9..192 rows (gemm_few) at both ends of every number of 16-row tiles and groups, whole and partial workgroups of tiles, numbers of supersteps that eight waves and the parts of K do not
+    divide, biases everywhere: against the products before (rows_few = 0; same halves, other orders of the fp32 sums: the bound of the routes above), from the start and behind a prefix"""
+    wk, s = _biased(dt.F16, wd, T, **shape)
+    toks = np.random.default_rng(T).integers(3, s["vocab"], T + 5).astype(np.int32)
+    out = {}
+    for v in (1, 0):
+        wk.set_option("rows_few", v)
+        out[v] = [_rows(wk, toks[:T], s["vocab"])[1]]
+        wk.reset()
+        wk.forward(toks[:5], 0)
+        lg = torch.empty((T, s["vocab"]), dtype=torch.float16, device="cuda")
+        wk.forward(toks[5:], 5, lg)
+        out[v].append(g.host(lg).astype(np.float32))
+    for a, b in zip(out[1], out[0]):
+        ok, why = _agree(a, b)
+        assert ok, why
+    wk.close()
+
+
+@pytest.mark.parametrize("n", [9, 16, 17, 32])
+@pytest.mark.parametrize("kvd", [dt.F16, dt.Q8_B32T2], ids=["f16", "q8"])
+def test_batched_steps_of_many_queries_agree_with_the_rows_products_and_replay(kvd, n):
+    """the same products in a batched step: against rows_few = 0, and the captured step replayed with other work between the replays gives the eager step's tokens"""
+    wk, s = _biased(kvd, dt.Q4_B32T1A, 32, dim=1024, heads=8, kv_heads=8, head_dim=128, ffn=2816)
+    V = s["vocab"]
+    wk.kv_slots(n)
+    rng = np.random.default_rng(n)
+    for i in range(n):
+        wk.select_kv(i); wk.forward(rng.integers(3, V, 3 + i % 7).astype(np.int32), 0)
+    new, pos, slots = rng.integers(3, V, n).astype(np.int32), [3 + i % 7 for i in range(n)], list(range(n))
+    out, lg = {}, torch.empty((n, V), dtype=torch.float16, device="cuda")
+    for v in (0, 1):
+        wk.set_option("rows_few", v)
+        tok = wk.decode_batch(new, pos, slots, lg)
+        out[v] = g.host(lg).astype(np.float32)
+    ok, why = _agree(out[1], out[0])
+    assert ok, why
+    for _ in range(4):
+        assert [int(t) for t in wk.decode_batch(new, pos, slots)] == [int(t) for t in tok]
+        wk.decode_batch(new[:4], pos[:4], slots[:4]); torch.cuda.synchronize()
+    wk.close()
