@@ -119,7 +119,9 @@ struct LayeredNet {
     // 128, 67 MB where 4096 tokens take 24 -- up to opt_workspace_mb each.  A step beyond that, or whose workspace cannot be had, runs without (fp32 tiles, token by token).
     float *tile_ws = nullptr; size_t tile_ws_bytes = 0;
     int opt_workspace_mb = 4096; bool step_tile_ws = false;
-    bf16_t *a16 = nullptr, *h16 = nullptr, *g16 = nullptr; size_t a16_cap = 0, h16_cap = 0, g16_cap = 0; 
+    bf16_t *a16 = nullptr, *h16 = nullptr, *g16 = nullptr; size_t a16_cap = 0, h16_cap = 0, g16_cap = 0;
+    float *planes = nullptr; size_t planes_cap = 0;          // summands of x that the next layer adds (run_parallel_prompt)
+   
     // activations of a product rounded to bfloat16 beforehand: steps of at least this many rows (0: never).  Above the eight rows whose activations stay in 32 bits; k_lin_mfma rounds the
     // same on its way (9 / 16 tokens of Sopulorn 1561 -> 801 us / 1808 -> 1010, of Gelarax 1564 -> 642 / 1784 -> 823, 12 prompt rows of width 2048 2713 -> 979)
     int opt_a16_min = 9;
@@ -416,13 +418,14 @@ float norm_offset_of(const LayeredNet *n) { return n->cfg.norm_plain ? 0.0f : 1.
 bool takes_a16(const LayeredNet *n, size_t K, size_t T) { return !n->cfg.ops32 && n->opt_a16_min > 0 && T >= (size_t)n->opt_a16_min && K % 8 == 0 && K >= 64; }
 size_t a16_stride(size_t K) { return (K + 63) & ~(size_t)63; }
 
-int ensure_halfs(ifa_model *m, bf16_t *&buf, size_t &cap, size_t need)
+template <class V>
+int ensure_halfs(ifa_model *m, V *&buf, size_t &cap, size_t need)
 {
     if (need <= cap) return IFA_OK;
     IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
     drop_step_graph(m->lay);          // (with a16_min 1 a captured step reads these)
     lay_free(buf); buf = nullptr; cap = 0;
-    IFA_HIP_CHECK(hipMalloc((void **)&buf, need * 2));
+    IFA_HIP_CHECK(hipMalloc((void **)&buf, need * sizeof(V)));
     cap = need;
     return IFA_OK;
 }
@@ -1014,7 +1017,8 @@ int run_delta_mixer(ifa_model *m, LLayer &L, size_t T, int nseq)
 
 // A PARALLEL block of a prompt whose products read bfloat16 rows: x += ls1 (s0 W0 a0 + s1 W1 a1) + ls2 (W2 a2 + b2) as ONE product over the mixers' and the feed-forward's outputs side by
 // side in n->a16, where their producers leave them rounded (before: a product each, every operand written in 32 bits and rounded by a launch of its own: 17 launches a layer, now 11).
-int run_parallel_prompt(ifa_model *m, LLayer &L, size_t T, int nseq, bool *done)
+// *pending planes of x's summands are in n->planes on entry and on return
+int run_parallel_prompt(ifa_model *m, LLayer &L, size_t T, int nseq, bool *done, int *pending)
 {
     LayeredNet *n = m->lay;
     const ifa_layered_config &c = n->cfg;
@@ -1025,12 +1029,19 @@ int run_parallel_prompt(ifa_model *m, LLayer &L, size_t T, int nseq, bool *done)
     const bool lin = sp.mixer == IFA_MIX_WINDOW_LINEAR;
     const size_t AQ = lin ? (size_t)sp.a_heads * sp.a_dim : 0, MV = lin ? (size_t)sp.l_heads * sp.l_vdim : (size_t)sp.d_heads * sp.d_vdim;
     *done = takes_a16(n, W, T) && (!AQ || takes_a16(n, AQ, T)) && takes_a16(n, MV, T) && (!F || takes_a16(n, F, T)) && W <= 8192;
-    if (!*done) return IFA_OK;
+    if (!*done) {
+        const int left = *pending;
+        *pending = 0;
+        return left ? ifa_add_planes_f32(n->x, n->planes, left, T, W, s) : IFA_OK;
+    }
     const size_t at1 = AQ ? a16_stride(AQ) : 0, at2 = at1 + a16_stride(MV), ld = at2 + (F ? a16_stride(F) : 0), ldw = a16_stride(W);
     const void *ls1 = L.T(IFA_LT_LS1).data;
     int rc;
     if ((rc = ensure_halfs(m, n->h16, n->h16_cap, T * ldw)) || (rc = ensure_halfs(m, n->a16, n->a16_cap, T * ld))) return rc;
-    if (!ifa_layernorm_to_bf16(1, n->x, W, T, W, L.T(IFA_LT_NORM1).data, c.eps, n->h16, ldw, ldw, s)
+    const bool summed = *pending && ifa_layernorm_planes_to_bf16(1, n->x, n->planes, *pending, T, W, L.T(IFA_LT_NORM1).data, c.eps, n->h16, ldw, ldw, s);
+    if (*pending && !summed && (rc = ifa_add_planes_f32(n->x, n->planes, *pending, T, W, s))) return rc;
+    *pending = 0;
+    if (!summed && !ifa_layernorm_to_bf16(1, n->x, W, T, W, L.T(IFA_LT_NORM1).data, c.eps, n->h16, ldw, ldw, s)
         && ((rc = ifa_layernorm_f32(1, n->x, W, T, W, L.T(IFA_LT_NORM1).data, c.eps, n->h, W, s)) || (rc = ifa_rows_to_bf16(n->h, W, T, W, n->h16, ldw, s)))) return rc;
     IFA_LAUNCH_CHECK();
     const int silu0 = lin ? (int)L.c_lq : 0, silu1 = lin ? (int)L.c_lg : 0;
@@ -1063,7 +1074,11 @@ int run_parallel_prompt(ifa_model *m, LLayer &L, size_t T, int nseq, bool *done)
     if (lin) parts[np++] = {L.T(IFA_LT_A_O).data, AQ, ls1, nullptr, sp.a_out_scale};
     parts[np++] = {L.T(lin ? IFA_LT_L_O : IFA_LT_D_O).data, MV, ls1, nullptr, lin ? sp.l_out_scale : 1.0f};
     if (F) parts[np++] = {L.T(IFA_LT_FFN_DOWN).data, F, L.T(IFA_LT_LS2).data, L.T(IFA_LT_FFN_DOWN_B).data, 1.0f};
-    return ifa_linear_bf16_sum(parts, np, W, n->a16, ld, T, n->x, W, s);
+    const int planes = W % 4 == 0 ? ifa_linear_bf16_sum_plane_count(W, ld, T) : 0;
+    if (planes && (rc = ensure_halfs(m, n->planes, n->planes_cap, (size_t)planes * T * W))) return rc;
+    if ((rc = ifa_linear_bf16_sum_planes(parts, np, W, n->a16, ld, T, n->x, W, planes ? n->planes : nullptr, s))) return rc;
+    *pending = planes;
+    return IFA_OK;
 }
 
 // the layers of one step over T rows / nseq sequences whose tables are already on the device; leaves the residual in n->x
@@ -1101,6 +1116,7 @@ int run_layers(ifa_model *m, size_t T, int nseq)
         return IFA_OK;
     }
     bool h_ready = false;
+    int pending = 0;          // planes of x's summands in n->planes (PARALLEL blocks of a prompt, between two of them)
     for (size_t ri = 0; ri < n->runs.size(); ri++) {
         const size_t li = (size_t)n->runs[ri].first;
         const int pass = n->runs[ri].second;
@@ -1142,9 +1158,14 @@ int run_layers(ifa_model *m, size_t T, int nseq)
             }
         }
         bool done = false;
-        if ((rc = run_parallel_prompt(m, L, T, nseq, &done))) return rc;
+        if ((rc = run_parallel_prompt(m, L, T, nseq, &done, &pending))) return rc;
         if (done) {
-            if (n->opt_tap_layers && n->taps && T <= n->taps_rows)
+            const bool tap = n->opt_tap_layers && n->taps && T <= n->taps_rows;
+            if (pending && (tap || !next_layer || next_layer->spec.block != sp.block)) {
+                if ((rc = ifa_add_planes_f32(n->x, n->planes, pending, T, W, s))) return rc;
+                pending = 0;
+            }
+            if (tap)
                 IFA_HIP_CHECK(hipMemcpyAsync(n->taps + ri * n->taps_rows * W, n->x, T * W * 4, hipMemcpyDeviceToDevice, m->stream));
             continue;
         }
@@ -1263,7 +1284,7 @@ int lay_destroy(ifa_model *m)
     for (float *p : n->slot_ptr) lay_free(p);
     lay_free(n->slot_base_dev);
     if (n->tab_pin) (void)hipHostFree(n->tab_pin);
-    lay_free(n->attn_ws); lay_free(n->tile_ws); lay_free(n->scan_ws); lay_free(n->a16); lay_free(n->h16); lay_free(n->g16);
+    lay_free(n->attn_ws); lay_free(n->tile_ws); lay_free(n->scan_ws); lay_free(n->a16); lay_free(n->h16); lay_free(n->g16); lay_free(n->planes);
     lay_free(n->tab_dev); lay_free(n->excl_dev); lay_free(n->next_dev); lay_free(n->ring_dev);
     float *bufs[] = {n->x, n->h, n->proj, n->m1, n->m2, n->m3, n->beta, n->decay, n->logits, n->taps};
     for (float *b : bufs) lay_free(b);

@@ -12,7 +12,7 @@
 //             OPS32 = true : operands stay 32-bit, v_mfma_f32_32x32x2_f32 (the exact mode of the worker)
 //   T  > 8    k_lin_tile (ifa_linear_bf16_both, where the caller has rounded the activations: by their producer or by k_rows_to_bf16): tiles of up to
 //             128 x 128 (32 x 32 where there are few), both operands straight to LDS; the same sums in the same order as k_lin_mfma<false>
-// Accumulation is fp32 in every path.  No atomics, no split K: a result does not depend on what else runs.
+// Accumulation is fp32 in every path.  No atomics; K is shared out (sums of products) by sizes alone, its parts added in order: a result does not depend on what else runs.
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -50,7 +50,7 @@ struct LinGluArgs : LinArgs { bf16_t *G16; float *G; int ldg, glu_c0, glu_f, glu
 // Row t times sigmoid(row_gate[t * ld_gate]) (lin_store)
 struct LinGatedArgs : LinArgs { const float *row_gate; int ld_gate; };
 // Several products into the same columns (k_lin_tile): A's rows hold their operands side by side, each padded to whole steps; W, K, mul, bias, alpha of each here
-struct LinSumArgs : LinArgs { struct Part { const bf16_t *W, *mul, *bias; int K, steps; float alpha; } part[IFA_SUM_PARTS]; };
+struct LinSumArgs : LinArgs { struct Part { const bf16_t *W, *mul, *bias; int K, steps; float alpha; } part[IFA_SUM_PARTS]; float *planes; int ks; };
 
 template <class Args>
 __device__ __forceinline__ void lin_store(const Args &P, int t, int n, float acc)
@@ -188,26 +188,30 @@ typedef const __attribute__((address_space(1))) void lt_glb_t;
 // but one go.  At a part's last step its columns' scales and biases take it from the step's accumulators into the sum.  (22 products of
 // a Gelarax prompt in 8 launches: 2048 rows of width 2048 1268 -> 1202 us (866 with the tiles as they are), 601 of width 1024 312 -> 309 (240), and 14
 // launches less.)
-constexpr int LT_GROUPED = 1, LT_GLU = 2, LT_SUM = 4;
+// SPLIT (with SUM): the steps shared out over P.ks workgroups a tile (lin_sum_plan).  (As a test at run time it cost the sums that are not shared out 7 %: 2048 rows of width 2048 104 -> 111 us.)
+constexpr int LT_GROUPED = 1, LT_GLU = 2, LT_SUM = 4, LT_SPLIT = 8;
 template <int MODE>
 using LinTileArgs = std::conditional_t<(MODE & LT_SUM) != 0, LinSumArgs, std::conditional_t<(MODE & LT_GLU) != 0, LinGluArgs, LinArgs>>;
 template <int BM, int BN, int WM, int WN, int NB, int MODE>
 __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(LinTileArgs<MODE> P, const bf16_t *__restrict__ A16, int lda16, int tiles_m, int tiles_n)
 {
-    constexpr bool GROUPED = MODE & LT_GROUPED, GLU = MODE & LT_GLU, SUM = MODE & LT_SUM;
+    constexpr bool GROUPED = MODE & LT_GROUPED, GLU = MODE & LT_GLU, SUM = MODE & LT_SUM, SPLIT = MODE & LT_SPLIT;
     constexpr int WAVES = WM * WN, TA = BM / (32 * WM), TB = BN / (32 * WN), AI = BM / (8 * WAVES), WI = BN / (8 * WAVES), ROWB = 2 * LT_BK, STEPB = (BM + BN) * ROWB;
     static_assert(AI * 8 * WAVES == BM && WI * 8 * WAVES == BN && TA * 32 * WM == BM && TB * 32 * WN == BN, "whole rows and tiles a wave");
     static_assert((NB - 2) * (AI + WI) < 64, "requests that s_waitcnt can count");
     extern __shared__ __attribute__((aligned(16))) char lt_smem[];          // [NB steps][BM rows of A, BN rows of W]
     char *const smem = lt_smem;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5, wm = wave % WM, wn = wave / WM;
-    int t0, n0, t_end = P.T;
+    int t0, n0, t_end = P.T, kz = 0;
     const bf16_t *Wg = P.W;
     {
         // (grouped: of the tiles that there are, not of the most there can be -- the empty ones, dealt out like the others, left up to five of the XCDs idle: 36 pairs of 64
         // experts of 1024 x 704 66 -> 46 us, 2400 pairs 127 -> 101)
         if constexpr (GROUPED) tiles_m = *P.n_tiles;
-        const int nwg = tiles_m * tiles_n, orig = blockIdx.x, xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
+        const int nwg = tiles_m * tiles_n;
+        int orig = blockIdx.x;
+        if constexpr (SPLIT) { kz = orig / nwg; orig -= kz * nwg; }
+        const int xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
         if (GROUPED && orig >= nwg) return;
         const int wg = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
         constexpr int GM = 1024 / BM;          // bands of 1024 rows of C, the row tiles of a band fastest
@@ -222,6 +226,15 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
     const int n_end = [&]() { if constexpr (GLU) return P.glu_c0; else return P.N; }(), n_plain = GLU ? (n_end + BN - 1) / BN : 0, o0 = (n0 / BN - n_plain) * (BN / 2);
     const bool glu = GLU && n0 / BN >= n_plain;
     auto swz = [](int r) { return (r >> 1) & 7; };
+    // (SPLIT) this workgroup's steps, k0 in front of them; (SUM) counted from k0, the part that the next requested step belongs to, from its first step to the one behind its last; likewise for the
+    // next step of products
+    int k0 = 0, nsteps = lda16 / LT_BK, q_part = 0, q_from = 0, q_to = 0;
+    if constexpr (SUM) q_to = P.part[0].steps;
+    if constexpr (SPLIT) {
+        const int all = nsteps;
+        k0 = kz * all / P.ks; nsteps = (kz + 1) * all / P.ks - k0; q_from = -k0; q_to -= k0;
+        while (q_to <= 0) { q_part++; q_from = q_to; q_to += P.part[q_part].steps; }
+    }
     const bf16_t *asrc[AI], *wsrc[WI];
     int wlim[WI];          // furthest step offset of the lane's piece inside a row of W
 #pragma unroll
@@ -229,7 +242,7 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
         const int row = (wave * AI + j) * 8 + (lane >> 3), c = (lane & 7) ^ swz(row);
         int at = min(t0 + row, t_end - 1);          // (rows beyond the last: repeated, not stored)
         if (GROUPED && P.a_rows) at = P.a_rows[at];
-        asrc[j] = A16 + (size_t)at * lda16 + c * 8;
+        asrc[j] = A16 + (size_t)at * lda16 + (SPLIT ? k0 * LT_BK : 0) + c * 8;
     }
 #pragma unroll
     for (int j = 0; j < WI; j++) {
@@ -238,12 +251,11 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
         if constexpr (GLU) if (glu) wr = P.glu_c0 + ((row & 16) ? P.glu_f : 0) + min(o0 + 16 * (row >> 5) + (row & 15), P.glu_f - 1);
         const bf16_t *W0 = Wg;
         int K = P.K;
-        if constexpr (SUM) { W0 = P.part[0].W; K = P.part[0].K; }
+        if constexpr (SUM) { W0 = P.part[q_part].W; K = P.part[q_part].K; }
         wsrc[j] = W0 + (size_t)wr * K + c * 8;
         wlim[j] = K - 8 - c * 8;
     }
-    // (SUM) the part that the next requested step belongs to, from its first step to the one behind its last; likewise for the next step of products
-    int q_part = 0, q_from = 0, q_to = [&]() { if constexpr (SUM) return P.part[0].steps; else return 0; }(), c_part = 0, c_to = q_to;
+    int c_part = q_part, c_to = q_to;
     auto enter = [&](int step) {
         if constexpr (SUM) {
             if (step != q_to) return;
@@ -257,7 +269,6 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
             }
         }
     };
-    const int nsteps = lda16 / LT_BK;
     auto stage_a = [&](int step, char *to, int j) {
         __builtin_amdgcn_global_load_lds((lt_glb_t *)(asrc[j] + step * LT_BK), (lt_lds_t *)(to + (wave * AI + j) * 1024), 16, 0, 0);
     };
@@ -300,7 +311,8 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
     }
     auto close = [&](int step) {          // (behind the step's products)
         if constexpr (SUM) {
-            if (step + 1 != c_to) return;
+            const bool whole = step + 1 == c_to;          // (else: another workgroup has the rest of the part, and its bias)
+            if (!whole && (!SPLIT || step + 1 != nsteps)) return;
 #pragma unroll
             for (int b = 0; b < TB; b++) {
                 float bv = p_bias[0][b], mv = p_mul[0][b];
@@ -309,7 +321,7 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
 #pragma unroll
                 for (int a = 0; a < TA; a++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) { tot[a][b][r] += (acc[a][b][r] + bv) * mv; acc[a][b][r] = 0.0f; }
+                    for (int r = 0; r < 16; r++) { tot[a][b][r] += (acc[a][b][r] + (!SPLIT || whole ? bv : 0.0f)) * mv; acc[a][b][r] = 0.0f; }
             }
             c_part++;
             if (step + 1 < nsteps) c_to += P.part[c_part].steps;
@@ -457,7 +469,9 @@ __global__ void __launch_bounds__(64 * WM * WN, BM == 32 ? 1 : 2) k_lin_tile(Lin
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     const int t = t0 + wm * (BM / WM) + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * g;
-                    if (t < t_end) P.C[(size_t)t * P.ldc + n] += tot[a][b][r];
+                    if (t >= t_end) continue;
+                    if (!SPLIT || kz == 0) P.C[(size_t)t * P.ldc + n] += tot[a][b][r];
+                    else P.planes[((size_t)(kz - 1) * P.T + t) * P.N + n] = tot[a][b][r];
                 }
         }
         return;
@@ -525,7 +539,9 @@ int launch_lin_tile(const LinTileArgs<MODE> &P, const bf16_t *a16, size_t lda16,
     const int tm = (int)row_tiles, tn = (int)lin_col_tiles(P, BN);
     const auto fn = k_lin_tile<BM, BN, WM, WN, NB, MODE>;
     if (smem > 64 * 1024) IFA_HIP_CHECK(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-    hipLaunchKernelGGL(fn, dim3((unsigned)tm * (unsigned)tn), dim3(64 * WM * WN), smem, s, P, a16, (int)lda16, tm, tn);
+    unsigned ks = 1;
+    if constexpr ((MODE & LT_SPLIT) != 0) ks = (unsigned)P.ks;
+    hipLaunchKernelGGL(fn, dim3((unsigned)tm * (unsigned)tn * ks), dim3(64 * WM * WN), smem, s, P, a16, (int)lda16, tm, tn);
     IFA_LAUNCH_CHECK();
     return IFA_OK;
 }
@@ -1053,13 +1069,38 @@ extern "C" int ifa_linear_bf16_both(const void *w_bf16, size_t rows, size_t cols
     return lin_tile_dispatch<0>(P, a, lda, s);
 }
 
-int ifa_linear_bf16_sum(const IfaSumPart *parts, int n_parts, size_t rows, const void *a_bf16, size_t lda, size_t tokens, void *c_f32, size_t ldc, ifa_stream stream)
+// Few tiles of many steps leave most of the chip idle: the steps are shared out over KS workgroups a tile, the first of which adds into C while the others leave their sums in planes
+// [KS - 1][tokens][rows] for the launch that reads C next.  us a Gelarax layer's sum, one workgroup a tile / shared out, width 1024: 37 tokens 28.0 / 12.6 (32 x 32 tiles by eight), 200
+// tokens 28 / 16.6 (64 x 64 by eight), 601 29.8 / 22.0 (128 x 64 by two); whole prompts of 9, 37, 128, 411, 601 tokens 643, 817, 1071, 1228, 1267 -> 506, 690, 954, 1146, 1219, width 2048 977, 1139, 1416,
+// 1788, 2061 -> 728, 898, 1211, 1740, 1960.  (Of the choices tried at each of those lengths -- four shapes by three, four, six, eight -- the model's is within 3 % of the fastest prompt.)
+struct LinSumPlan { int shape, ks; };
+static LinSumPlan lin_sum_plan(size_t T, size_t N, size_t steps)
+{
+    const size_t t128 = (T + 127) / 128, t64 = (T + 63) / 64, t32 = (T + 31) / 32, n128 = (N + 127) / 128, n64 = (N + 63) / 64, n32 = (N + 31) / 32;
+    const struct { LinShape h; size_t tiles; int buffers; } shapes[] = {{LT_SHAPES[LT_128x128], t128 * n128, 4}, {LT_SHAPES[LT_128x64], t128 * n64, 4}, {LT_SHAPES[LT_64x64], t64 * n64, 5},
+                                                                        {{2, 0.20, 0.32, 0.32, 3.5}, t32 * n32, 8}};
+    LinSumPlan best = {-1, 1};
+    double cost = 0;
+    for (int k = 0; k < 4; k++)
+        for (int z = 1; z <= 1 + IFA_SUM_PLANES; z++) {
+            if (steps / z < (size_t)shapes[k].buffers || shapes[k].tiles * z >= (1u << 31)) continue;
+            // (a plane is written here and read by the next launch, 3 TB/s; not for less than 15 %, what the model is worth)
+            const double c = (lin_cost(shapes[k].h, shapes[k].tiles * z, (steps + z - 1) / z) + (z > 1 ? 0.5 : 0.0) + (z - 1) * (0.1 + T * N * 8 / 3.0e6)) / (z > 1 ? 0.85 : 1.0);
+            if (best.shape < 0 || c < cost) { best = {k, z}; cost = c; }
+        }
+    return best;
+}
+
+int ifa_linear_bf16_sum_plane_count(size_t rows, size_t lda, size_t tokens) { return rows && tokens && lda ? lin_sum_plan(tokens, rows, lda / LT_BK).ks - 1 : 0; }
+
+int ifa_linear_bf16_sum_planes(const IfaSumPart *parts, int n_parts, size_t rows, const void *a_bf16, size_t lda, size_t tokens, void *c_f32, size_t ldc, float *planes,
+                               ifa_stream stream)
 {
     IFA_REQUIRE(parts && a_bf16 && c_f32 && n_parts >= 1 && n_parts <= IFA_SUM_PARTS, "linear_bf16_sum: null pointer or %d parts", n_parts);
     IFA_REQUIRE(rows > 0 && tokens > 0 && ldc >= rows && rows < (1u << 30) && tokens < (1u << 30) && lda < (1u << 30) && ((uintptr_t)a_bf16 & 15) == 0, "linear_bf16_sum: bad shape");
     LinSumArgs P;
     memset(&P, 0, sizeof(P));
-    P.C = (float *)c_f32; P.T = (int)tokens; P.N = (int)rows; P.ldc = (int)ldc;
+    P.C = (float *)c_f32; P.T = (int)tokens; P.N = (int)rows; P.ldc = (int)ldc; P.planes = planes; P.ks = 1;
     size_t at = 0;
     for (int k = 0; k < n_parts; k++) {
         const IfaSumPart &p = parts[k];
@@ -1069,7 +1110,22 @@ int ifa_linear_bf16_sum(const IfaSumPart *parts, int n_parts, size_t rows, const
         at += (size_t)P.part[k].steps * LT_BK;
     }
     IFA_REQUIRE(at == lda, "linear_bf16_sum: parts of %zu columns in rows of %zu", at, lda);
-    return lin_tile_dispatch<LT_SUM>(P, (const bf16_t *)a_bf16, lda, ifa_s(stream));
+    const bf16_t *a = (const bf16_t *)a_bf16;
+    const LinSumPlan plan = planes ? lin_sum_plan(tokens, rows, lda / LT_BK) : LinSumPlan{0, 1};
+    if (plan.ks == 1) return lin_tile_dispatch<LT_SUM>(P, a, lda, ifa_s(stream));
+    P.ks = plan.ks;
+    const size_t t128 = (tokens + 127) / 128;
+    switch (plan.shape) {
+    case 0: return launch_lin_tile<128, 128, 2, 4, 4, LT_SUM | LT_SPLIT>(P, a, lda, t128, ifa_s(stream));
+    case 1: return launch_lin_tile<128, 64, 4, 2, 4, LT_SUM | LT_SPLIT>(P, a, lda, t128, ifa_s(stream));
+    case 2: return launch_lin_tile<64, 64, 2, 2, 5, LT_SUM | LT_SPLIT>(P, a, lda, (tokens + 63) / 64, ifa_s(stream));
+    default: return launch_lin_tile<32, 32, 1, 1, 8, LT_SUM | LT_SPLIT>(P, a, lda, (tokens + 31) / 32, ifa_s(stream));
+    }
+}
+
+int ifa_linear_bf16_sum(const IfaSumPart *parts, int n_parts, size_t rows, const void *a_bf16, size_t lda, size_t tokens, void *c_f32, size_t ldc, ifa_stream stream)
+{
+    return ifa_linear_bf16_sum_planes(parts, n_parts, rows, a_bf16, lda, tokens, c_f32, ldc, nullptr, stream);
 }
 
 int ifa_linear_bf16_glu(const void *w_bf16, size_t rows, size_t cols, const void *a_bf16, size_t lda, size_t tokens, const void *bias_bf16, void *c_f32, size_t ldc, int silu_col0,

@@ -3,6 +3,7 @@
 #include <algorithm>
 #include "ifa_host.h"
 #include "ifa_f32_common.h"
+#include "ifa_rows_fused.h"
 #include "ifa_streams.h"
 
 using namespace ifa32;
@@ -54,9 +55,10 @@ __global__ void __launch_bounds__(256) k_norm_f32(int kind, const float *__restr
 
 // The same into bfloat16 rows, zero up to `width` columns, the row in registers: every thread holds PIECES pieces of four values and requests row and weight before the first sum.
 // (Read three times from the caches, written in 32 bits and rounded by a launch of its own: 2048 rows of 2048 13.2 + 5.6 -> 7.8 us, 601 of 1024 6.3 + 5.0 -> 4.5.)
-template <int PIECES>
-__global__ void __launch_bounds__(256) k_norm_to_bf16(int kind, const float *__restrict__ x, size_t ldx, int cols, const bf16_t *__restrict__ w, float eps, bf16_t *__restrict__ y,
-                                                      int width, size_t ldy)
+// PLANES: further summands of x's rows (dense, like the planes), which x takes up on the way.
+template <int PIECES, bool PLANES = false>
+__global__ void __launch_bounds__(256) k_norm_to_bf16(int kind, const float *x, size_t ldx, int cols, const bf16_t *__restrict__ w, float eps, bf16_t *__restrict__ y,
+                                                      int width, size_t ldy, const float *__restrict__ planes = nullptr, int n_planes = 0, float *x_out = nullptr)
 {
     __shared__ float red[17];
     const float *xr = x + (size_t)blockIdx.x * ldx;
@@ -66,7 +68,16 @@ __global__ void __launch_bounds__(256) k_norm_to_bf16(int kind, const float *__r
 #pragma unroll
     for (int p = 0; p < PIECES; p++) {
         const int c = 4 * (threadIdx.x + p * 256);
-        const float4 a = c < cols ? *reinterpret_cast<const float4 *>(xr + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 a = c < cols ? *reinterpret_cast<const float4 *>(xr + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (PLANES) {
+            float4 d[IFA_SUM_PLANES];
+            const size_t plane = (size_t)gridDim.x * cols, at = (size_t)blockIdx.x * cols + min(c, cols - 4);
+#pragma unroll
+            for (int k = 0; k < IFA_SUM_PLANES; k++) if (k < n_planes) d[k] = *reinterpret_cast<const float4 *>(planes + k * plane + at);
+#pragma unroll
+            for (int k = 0; k < IFA_SUM_PLANES; k++) if (k < n_planes && c < cols) { a.x += d[k].x; a.y += d[k].y; a.z += d[k].z; a.w += d[k].w; }
+            if (c < cols) *reinterpret_cast<float4 *>(x_out + (size_t)blockIdx.x * ldx + c) = a;
+        }
         wv[p] = w && c < cols ? *reinterpret_cast<const uint2 *>(w + c) : make_uint2(0x3F803F80u, 0x3F803F80u);
         v[p][0] = a.x; v[p][1] = a.y; v[p][2] = a.z; v[p][3] = a.w;
         s += (a.x + a.y) + (a.z + a.w);
@@ -661,6 +672,41 @@ bool ifa_layernorm_to_bf16(int kind, const void *x_f32, size_t ldx, size_t rows,
     if (width <= 1024) IFA_NB(1); else if (width <= 2048) IFA_NB(2); else if (width <= 4096) IFA_NB(4); else IFA_NB(8);
 #undef IFA_NB
     return true;
+}
+
+bool ifa_layernorm_planes_to_bf16(int kind, void *x_f32, const float *planes, int n_planes, size_t rows, size_t cols, const void *w_bf16, float eps, void *y_bf16, size_t width, size_t ldy,
+                                  ifa_stream stream)
+{
+    if (!x_f32 || !y_bf16 || !planes || n_planes < 1 || n_planes > IFA_SUM_PLANES || (kind != 0 && kind != 1) || rows == 0 || rows >= (1u << 31) || cols == 0 || cols % 4 || width < cols
+        || width % 8 || width > 8192 || ldy < width || ldy % 8 || (((uintptr_t)x_f32 | (uintptr_t)planes) & 15) || ((uintptr_t)y_bf16 & 15) || ((uintptr_t)w_bf16 & 7)) return false;
+    const dim3 grid((unsigned)rows);
+#define IFA_NB(P) hipLaunchKernelGGL((k_norm_to_bf16<P, true>), grid, dim3(256), 0, ifa_s(stream), kind, (const float *)x_f32, cols, (int)cols, (const bf16_t *)w_bf16, eps, (bf16_t *)y_bf16, \
+                                     (int)width, ldy, planes, n_planes, (float *)x_f32)
+    if (width <= 1024) IFA_NB(1); else if (width <= 2048) IFA_NB(2); else if (width <= 4096) IFA_NB(4); else IFA_NB(8);
+#undef IFA_NB
+    return true;
+}
+
+__global__ void __launch_bounds__(256) k_add_planes(float *x, const float *__restrict__ planes, int n_planes, size_t n)
+{
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= n) return;
+    float4 a = *reinterpret_cast<const float4 *>(x + i), d[IFA_SUM_PLANES];
+#pragma unroll
+    for (int k = 0; k < IFA_SUM_PLANES; k++) if (k < n_planes) d[k] = *reinterpret_cast<const float4 *>(planes + k * n + i);
+#pragma unroll
+    for (int k = 0; k < IFA_SUM_PLANES; k++) if (k < n_planes) { a.x += d[k].x; a.y += d[k].y; a.z += d[k].z; a.w += d[k].w; }
+    *reinterpret_cast<float4 *>(x + i) = a;
+}
+
+int ifa_add_planes_f32(float *x_f32, const float *planes, int n_planes, size_t rows, size_t cols, ifa_stream stream)
+{
+    const size_t n = rows * cols;
+    IFA_REQUIRE(x_f32 && planes && n_planes >= 1 && n_planes <= IFA_SUM_PLANES && n > 0 && cols % 4 == 0 && (((uintptr_t)x_f32 | (uintptr_t)planes) & 15) == 0 && n / 1024 < (1u << 31) - 1,
+                "add_planes: %d planes of %zu x %zu", n_planes, rows, cols);
+    hipLaunchKernelGGL(k_add_planes, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, ifa_s(stream), x_f32, planes, n_planes, n);
+    IFA_LAUNCH_CHECK();
+    return IFA_OK;
 }
 
 int ifa_glu_to_bf16(int kind, float limit, const void *gate_up_f32, size_t ld, size_t rows, size_t cols, const void *row_gate_f32, size_t ldg, void *out_bf16, size_t ldo,

@@ -57,12 +57,21 @@ extern "C" int ifa_linear_bf16w_gated_rows(const void *w_bf16, size_t rows, size
 constexpr int IFA_SUM_PARTS = 3;
 struct IfaSumPart { const void *w; size_t cols; const void *mul, *bias; float alpha; };
 extern "C" int ifa_linear_bf16_sum(const IfaSumPart *parts, int n_parts, size_t rows, const void *a_bf16, size_t lda, size_t tokens, void *c_f32, size_t ldc, ifa_stream stream);
+// ... with K shared out where that leaves less of the chip idle: the count of planes [tokens][rows] of further summands of C that the second writes (planes null: none, all of them in C)
+// and the caller adds, in order, where it next reads C (ifa_layernorm_planes_to_bf16, ifa_add_planes_f32)
+constexpr int IFA_SUM_PLANES = 7;
+extern "C" int ifa_linear_bf16_sum_plane_count(size_t rows, size_t lda, size_t tokens);
+extern "C" int ifa_linear_bf16_sum_planes(const IfaSumPart *parts, int n_parts, size_t rows, const void *a_bf16, size_t lda, size_t tokens, void *c_f32, size_t ldc, float *planes, ifa_stream stream);
+extern "C" int ifa_add_planes_f32(float *x_f32, const float *planes, int n_planes, size_t rows, size_t cols, ifa_stream stream);      // rows and planes dense
 // ifa_rows_to_bf16 into the first `width` columns (a multiple of 8) of rows of ldy
 int ifa_rows_to_bf16_part(const void *x_f32, size_t ldx, size_t rows, size_t cols, void *y_bf16, size_t width, size_t ldy, ifa_stream stream);
 // Producers that leave what only products read in bfloat16: rows of ldy, zero from the last column up to `width` (both multiples of 8).  The norms: false where the sizes or the
 // alignment don't allow it (nothing launched).
 // ifa_layernorm_f32
 bool ifa_layernorm_to_bf16(int kind, const void *x_f32, size_t ldx, size_t rows, size_t cols, const void *w_bf16, float eps, void *y_bf16, size_t width, size_t ldy, ifa_stream stream);
+// ... of x (dense rows) + planes, which x takes up
+extern "C" bool ifa_layernorm_planes_to_bf16(int kind, void *x_f32, const float *planes, int n_planes, size_t rows, size_t cols, const void *w_bf16, float eps, void *y_bf16, size_t width, size_t ldy,
+                                  ifa_stream stream);
 // ifa_gated_groupnorm_f32 (w as long as a group or as the row)
 bool ifa_gated_groupnorm_to_bf16(const void *o_f32, size_t ldo, size_t rows, int channels, int group, const void *w_bf16, int wlen, const void *gate_f32, size_t ldg, int gate_act,
                                  float eps, void *y_bf16, size_t width, size_t ldy, ifa_stream stream);

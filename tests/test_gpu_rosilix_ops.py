@@ -410,6 +410,53 @@ def test_sums_of_products_in_one_pass(T, N, cols):
     assert np.all(np.abs(got[:, :N] - want) <= bound) and np.array_equal(got[:, N:], c0[:, N:])
 
 
+@pytest.mark.parametrize("T,N,cols", [(9, 1024, (1024, 1024, 2816)), (33, 1000, (2056, 512)), (64, 1024, (4352,)), (65, 516, (64, 72, 3000)), (129, 2048, (2048, 2048, 5632)), (601, 1024, (1024, 1024, 2816)),
+                                      (300, 68, (8200,)), (2048, 1024, (1024, 1024, 2816))])
+def test_sums_of_products_shared_out_over_k_and_what_adds_their_planes(T, N, cols):
+    """the ranges of K end inside a part, at its end and in its last, partial step; planes and C together against 64 bits (the bound above), and the norm that adds the planes against the
+    addition and the norm by themselves, bit for bit"""
+    rng = np.random.default_rng(T + N + sum(cols))
+    L, Z = capi(), C.c_size_t
+    ld = sum((k + 63) // 64 * 64 for k in cols)
+    n_planes = L.ifa_linear_bf16_sum_plane_count(Z(N), Z(ld), Z(T))
+    assert (n_planes > 0) == (T < 2000) and n_planes <= 7
+
+    class Part(C.Structure):
+        _fields_ = [("w", C.c_void_p), ("cols", C.c_size_t), ("mul", C.c_void_p), ("bias", C.c_void_p), ("alpha", C.c_float)]
+    a16, at, parts, keep = torch.zeros((T, ld), dtype=torch.int16, device="cuda"), 0, [], []
+    c0 = rng.standard_normal((T, N)).astype(np.float32)
+    want = torch.from_numpy(c0).cuda().double()
+    bound = 12 * 2.0 ** -24 * want.abs()
+    for i, K in enumerate(cols):
+        A, Wm, b, m = bf16_round(rng.standard_normal((T, K))), bf16_round(rng.standard_normal((N, K)) / np.sqrt(K)), bf16_round(rng.standard_normal(N)), bf16_round(rng.standard_normal(N))
+        a16[:, at:at + K] = devbf(A).view(torch.int16).reshape(T, K)
+        at += (K + 63) // 64 * 64
+        wd, bd, md, alpha = devbf(Wm), devbf(b), devbf(m), (1.0, 0.7, -1.3)[i]
+        keep += [wd, bd, md]
+        parts.append(Part(wd.data_ptr(), K, md.data_ptr() if i != 1 else None, bd.data_ptr() if i != 0 else None, alpha))
+        A, Wm, b, m = (torch.from_numpy(orc.f64(v)).cuda() for v in (A, Wm, b, m))
+        s, mag = A @ Wm.T, A.abs() @ Wm.abs().T
+        f = np.float32(alpha) * (m if i != 1 else 1.0)
+        if i != 0:
+            s, mag = s + b, mag + b.abs()
+        want += f * s
+        bound += (K + 24) * 2.0 ** -24 * abs(f) * mag
+    out, planes = torch.from_numpy(c0).cuda(), torch.full((max(n_planes, 1), T, N), float("nan"), device="cuda")
+    ia.check(L.ifa_linear_bf16_sum_planes((Part * len(parts))(*parts), len(parts), Z(N), p(a16), Z(ld), Z(T), p(out), Z(N), p(planes) if n_planes else None, None)); sync()
+    if not n_planes:
+        planes = torch.zeros_like(planes)
+        n_planes = 1
+    assert bool(((out.double() + planes.double().sum(0) - want).abs() <= bound).all())
+    x, y, width, w = out.clone(), [torch.zeros(T, (N + 63) // 64 * 64, dtype=torch.bfloat16, device="cuda") for _ in range(2)], (N + 63) // 64 * 64, devbf(bf16_round(rng.standard_normal(N)))
+    L.ifa_layernorm_planes_to_bf16.restype = C.c_bool
+    assert L.ifa_layernorm_planes_to_bf16(1, p(x), p(planes), n_planes, Z(T), Z(N), p(w), C.c_float(1e-5), p(y[0]), Z(width), Z(width), None)
+    ia.check(L.ifa_add_planes_f32(p(out), p(planes), n_planes, Z(T), Z(N), None))
+    zero = torch.zeros(1, T, N, device="cuda")
+    x1 = out.clone()
+    assert L.ifa_layernorm_planes_to_bf16(1, p(x1), p(zero), 1, Z(T), Z(N), p(w), C.c_float(1e-5), p(y[1]), Z(width), Z(width), None); sync()
+    assert torch.equal(x, out) and torch.equal(y[0].view(torch.int16), y[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 6, 8])
 @pytest.mark.parametrize("c0,F,K,kind", [(0, 1, 8, 0), (0, 37, 512, 1), (5, 40, 520, 3), (20, 1409, 1032, 0), (3, 300, 2056, 2), (1, 33, 4616, 1)])
 def test_gated_activations_behind_products_of_a_few_rows(T, c0, F, K, kind):
