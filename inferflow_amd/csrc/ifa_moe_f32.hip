@@ -23,6 +23,10 @@ namespace {
 
 typedef uint32_t u32x4m __attribute__((ext_vector_type(4)));
 
+// What a choice compares: a score that is no number comes last, with those of -inf, and an entry already taken (NaN from there on) compares with nothing.
+// So every pass finds an entry of the row, and no entry twice, whatever the scores are: the experts read their weights by these indices.
+__device__ __forceinline__ float choice_of(float v) { return v == v ? v : -INFINITY; }
+
 __device__ __forceinline__ float gelu_erf_f(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 
 // one wave per row: softmax over n_all logits, then `top` passes of argmax over score + correction (lowest index on ties)
@@ -35,7 +39,7 @@ __global__ void __launch_bounds__(64) k_moe_route(const float *__restrict__ logi
     const int t = blockIdx.x, lane = threadIdx.x;
     const float *z = logits + (size_t)t * ld;
     if (score_kind == 1) {
-        for (int e = lane; e < n_all; e += 64) { const float s = sigmoid_f(z[e]); sc[e] = s; ch[e] = s + (corr ? bf2f(corr[e]) : 0.0f); }
+        for (int e = lane; e < n_all; e += 64) { const float s = sigmoid_f(z[e]); sc[e] = s; ch[e] = choice_of(s + (corr ? bf2f(corr[e]) : 0.0f)); }
     } else {
         float mx = -INFINITY;
         for (int e = lane; e < n_all; e += 64) mx = fmaxf(mx, z[e]);
@@ -43,7 +47,7 @@ __global__ void __launch_bounds__(64) k_moe_route(const float *__restrict__ logi
         float sum = 0.0f;
         for (int e = lane; e < n_all; e += 64) { const float p = expf(z[e] - mx); sc[e] = p; sum += p; }
         sum = wave_sum(sum);
-        for (int e = lane; e < n_all; e += 64) { const float s = sc[e] / sum; sc[e] = s; ch[e] = s + (corr ? bf2f(corr[e]) : 0.0f); }
+        for (int e = lane; e < n_all; e += 64) { const float s = sc[e] / sum; sc[e] = s; ch[e] = choice_of(s + (corr ? bf2f(corr[e]) : 0.0f)); }
     }
     __syncthreads();
     float sum = 0.0f;          // (lane 0: of the chosen scores)
@@ -54,7 +58,7 @@ __global__ void __launch_bounds__(64) k_moe_route(const float *__restrict__ logi
             const float ov = __shfl_xor(best, o, 64); const int oi = __shfl_xor(bi, o, 64);
             if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
         }
-        if (lane == 0) { idx[(size_t)t * top + k] = bi; wgt[(size_t)t * top + k] = sc[bi]; ch[bi] = -INFINITY; sum += sc[bi]; }
+        if (lane == 0) { idx[(size_t)t * top + k] = bi; wgt[(size_t)t * top + k] = sc[bi]; ch[bi] = NAN; sum += sc[bi]; }
         __syncthreads();
     }
     if (renorm && lane == 0) { const float den = sum + renorm_eps; for (int k = 0; k < top; k++) wgt[(size_t)t * top + k] = wgt[(size_t)t * top + k] / den * wgt_scale; }
@@ -68,7 +72,7 @@ __global__ void __launch_bounds__(64) k_moe_route_top(const float *__restrict__ 
     float *pw = ch + n_all;
     const int t = blockIdx.x, lane = threadIdx.x;
     const float *z = logits + (size_t)t * ld;
-    for (int e = lane; e < n_all; e += 64) ch[e] = z[e] + (bias ? bf2f(bias[e]) : 0.0f);
+    for (int e = lane; e < n_all; e += 64) ch[e] = choice_of(z[e] + (bias ? bf2f(bias[e]) : 0.0f));
     __syncthreads();
     float first = 0.0f, sum = 0.0f;
     for (int k = 0; k < top; k++) {
@@ -81,7 +85,7 @@ __global__ void __launch_bounds__(64) k_moe_route_top(const float *__restrict__ 
         if (k == 0) first = best;                      // the largest of all: the softmax's reference
         const float p = expf(best - first);
         sum += p;
-        if (lane == 0) { idx[(size_t)t * top + k] = bi; pw[k] = p; ch[bi] = -INFINITY; }
+        if (lane == 0) { idx[(size_t)t * top + k] = bi; pw[k] = p; ch[bi] = NAN; }
         __syncthreads();
     }
     for (int k = lane; k < top; k += 64) wgt[(size_t)t * top + k] = pw[k] / sum;
@@ -125,7 +129,7 @@ __global__ void __launch_bounds__(1024) k_moe_route_rows(const float *h, size_t 
     }
     __syncthreads();
     if (wave == 0 && score_kind == 1) {
-        for (int e = lane; e < n_all; e += 64) { const float sv = sigmoid_f(sc[e]); sc[e] = sv; ch[e] = sv + (corr ? bf2f(corr[e]) : 0.0f); }
+        for (int e = lane; e < n_all; e += 64) { const float sv = sigmoid_f(sc[e]); sc[e] = sv; ch[e] = choice_of(sv + (corr ? bf2f(corr[e]) : 0.0f)); }
     } else if (wave == 0) {
         float mx = -INFINITY;
         for (int e = lane; e < n_all; e += 64) mx = fmaxf(mx, sc[e]);
@@ -133,7 +137,7 @@ __global__ void __launch_bounds__(1024) k_moe_route_rows(const float *h, size_t 
         float sum = 0.0f;
         for (int e = lane; e < n_all; e += 64) { const float pe = expf(sc[e] - mx); sc[e] = pe; sum += pe; }      // (each lane touches its own entries only)
         sum = wave_sum(sum);
-        for (int e = lane; e < n_all; e += 64) { const float sv = sc[e] / sum; sc[e] = sv; ch[e] = sv + (corr ? bf2f(corr[e]) : 0.0f); }
+        for (int e = lane; e < n_all; e += 64) { const float sv = sc[e] / sum; sc[e] = sv; ch[e] = choice_of(sv + (corr ? bf2f(corr[e]) : 0.0f)); }
     }
     __syncthreads();
     float chosen = 0.0f;          // (thread 0: the sum of the chosen scores)
@@ -145,7 +149,7 @@ __global__ void __launch_bounds__(1024) k_moe_route_rows(const float *h, size_t 
                 const float ov = __shfl_xor(best, o, 64); const int oi = __shfl_xor(bi, o, 64);
                 if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
             }
-            if (lane == 0) { idx[(size_t)t * top + k] = bi; wgt[(size_t)t * top + k] = sc[bi]; ch[bi] = -INFINITY; chosen += sc[bi]; }
+            if (lane == 0) { idx[(size_t)t * top + k] = bi; wgt[(size_t)t * top + k] = sc[bi]; ch[bi] = NAN; chosen += sc[bi]; }
         }
         __syncthreads();
     }

@@ -229,6 +229,28 @@ def test_router_scores_choices_and_ties(rows, n_all, top):
         assert gi[0].tolist() == list(range(top))
 
 
+@pytest.mark.parametrize("n_all,top", [(5, 5), (73, 8), (130, 2)])
+def test_choices_of_rows_without_numbers(n_all, top):
+    """every choice is an entry of the row, and none twice: scores that are no numbers, all at -inf (a correction of -inf), or some of each"""
+    W, rows = 16, 4
+    nan, inf = np.float32(np.nan), np.float32(np.inf)
+    z = np.zeros((rows, n_all), np.float32)
+    z[0], z[1], z[2, ::2], z[3, 0] = nan, -inf, nan, inf
+    h = np.zeros((rows, W), np.float32)
+    h[1], h[2, 0], h[3, 0] = nan, inf, 1.0                     # products of NaN, of inf and of numbers
+    R = bf16_round(np.random.default_rng(n_all).standard_normal((n_all, W)))
+    L = capi()
+    for corr in (np.zeros(n_all, np.float32), np.full(n_all, -inf, np.float32)):
+        outs = [torch.full((rows, top), -1, dtype=torch.int32, device="cuda") for _ in range(3)]
+        wgt = torch.zeros((rows, top), dtype=torch.float32, device="cuda")
+        ia.check(L.ifa_moe_route_f32(p(dev32(z)), n_all, rows, n_all, top, p(devbf(corr)), p(outs[0]), p(wgt), None))
+        ia.check(L.ifa_moe_route_top_f32(p(dev32(z)), n_all, rows, n_all, top, p(devbf(corr)), p(outs[1]), p(wgt), None))
+        ia.check(L.ifa_moe_route_rows_f32(p(dev32(h)), W, rows, W, p(devbf(R)), n_all, top, p(devbf(corr)), p(outs[2]), p(wgt), None)); sync()
+        for o in outs:
+            got = o.cpu().numpy()
+            assert got.min() >= 0 and got.max() < n_all and all(len(set(r)) == top for r in got.tolist()), got
+
+
 @pytest.mark.parametrize("rows,W,n_all,top", [(1, 64, 21, 4), (8, 30, 5, 5), (3, 256, 130, 6)])
 def test_router_with_its_product_inside(rows, W, n_all, top):
     rng = np.random.default_rng(rows + W)
