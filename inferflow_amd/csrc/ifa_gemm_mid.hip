@@ -1,4 +1,4 @@
-// ifa_gemm_mid.hip -- the linear layers of a 33..512-token prompt:  Y[T][N] = X[T][K] . W[N][K]^T  (+ bias, residual, GLU)
+// ifa_gemm_mid.hip -- the linear layers of a 193..768-token prompt, wo / w2 of one up to 2048:  Y[T][N] = X[T][K] . W[N][K]^T  (+ bias, residual, GLU)
 //
 // Reference: MatrixMultiplication (src/transformer/inference_worker.cc:2364-2432): Dequantize the weight tensor to F16, F16 x F16
 // product with fp32 accumulation (src/tensor/cublas_engine.cu:420-436).  Same values here: every weight is half(fma(q, scale,
@@ -10,14 +10,20 @@
 // 64-column step ends up waiting for the requests it has just issued: a step is one memory round trip (~1 us; rocprofv3 at 128
 // tokens: W1|W3 62 us for 64 steps, wq|wk|wv 35 us for 16) however little it multiplies.  Above ~512 tokens the step's MFMA work
 // covers that; below, a layer is 225 us for 126 MB of weights and 52 GFLOP.  Here:
-//   * EVERYTHING global goes through direct-to-LDS loads into a ring of NS stages (activations 128 x 64 halves + the RAW 20-byte
-//     weight blocks of the step: 21 KB per stage), requested NS - 1 steps ahead, waited for with a COUNTED vmcnt;
+//   * activations go through direct-to-LDS loads into a ring of four stages (128 x 64 halves), requested by four waves that do nothing else, waited for with a
+//     COUNTED vmcnt; the raw weight codes, which only one wave reads, go straight to its registers, two steps ahead;
 //   * every LDS read of the loop is inline assembly (the compiler sees no LDS access to protect), waited for with lgkmcnt where
 //     the values are used;
 //   * a wave owns 32 weight rows of the tile and ALL 128 tokens (4 accumulator tiles): it dequantises its rows' codes from the raw
 //     bytes straight into the B operand registers (11 VALU per 8 weights, ifa_dequant_q4.h) -- no dequantised tile in LDS, no
 //     second barrier -- while the MFMAs of the previous 16-column group run;
-//   * one barrier per step (the activation tile is shared by the four waves); parts of K as in k_gemm_big.
+//   * one barrier per step (the activation tile is shared by the four waves), and no start of a step: the first groups' fragments and codes of the next step are
+//     asked for in this one.  Codes through the ring and a step that began with 19 LDS reads (its conversion and first wait in front of its first product), 140
+//     instructions a step, two workgroups on a compute unit to hide that, against 100 instructions and one workgroup, ms a prompt of 193, 300, 512, 600, 768, 2048 tokens,
+//     Llama-2-7B: 6.13, 8.78, 9.81, 12.6, 15.0, 33.75 -> 5.74, 8.21, 9.32, 11.5, 13.8, 33.4.
+// What bounds it: power.  In the loop the clock falls to 1.55 - 1.8 GHz; a step takes 740 - 800 cycles, 512 of them products, 1.25 PFLOP/s in all.  So what converts a weight more often to
+// read LDS less or to keep a SIMD busier does not pay: waves of 64 rows x 64 tokens (half the fragment reads) took 3 - 7 % longer than the form before, eight computing waves of 32 x 64
+// 8 % longer than this one.
 // Weights: the MO copy of the rows GEMM (ifa_gemm_rows_mfma.h; Q4_B32T1A / B and the 64-weight nibble formats): a 16-row tile's K range
 // is one linear stream of 1 KiB supersteps.
 #include <algorithm>
@@ -25,6 +31,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <cstdio>
+#include <type_traits>
 #include <vector>
 #include "ifa_host.h"
 #include "ifa_math.h"
@@ -41,35 +48,25 @@ typedef uint32_t md_u2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void md_lds_t;
 typedef const __attribute__((address_space(1))) void md_glb_t;
 
-#ifndef IFA_MID_LOADERS
-#define IFA_MID_LOADERS 1   // 1: four more waves (one per SIMD) issue the direct-to-LDS requests; 0: the computing waves do, between their MFMAs
-#endif
 constexpr int MD_BN = 128, MD_BK = 64, MD_NW = 4, MD_NT = 256;      // (token rows of a tile: 32 TA, template parameter)
 constexpr int md_a_bytes(int ta) { return 32 * ta * MD_BK * 2; }       // activation tile of a step (TA = 4: 16 KB), rows of 128 bytes, 16-byte chunks swizzled
-constexpr int MD_WC_BYTES = MD_NW * 1024, MD_WS_BYTES = MD_NW * 256; // raw codes (32 rows x 2 blocks x 16 B per wave), (base, scale) words
-constexpr int md_stage(int ta) { return md_a_bytes(ta) + MD_WC_BYTES + MD_WS_BYTES; }    // 21 KB (TA = 4) / 37 KB (TA = 8)
-constexpr int MD_THREADS = IFA_MID_LOADERS ? 2 * MD_NT : MD_NT;     // launched threads (MD_NT of them compute and run the tails)
-// measurement builds (-DIFA_MID_ABL=n): 1 = no activation requests, 2 = no MFMA, 3 = no dequantisation, 4 = no barrier, 5 = no weight requests
-#ifndef IFA_MID_ABL
-#define IFA_MID_ABL 0
-#endif
-#ifndef IFA_MID_WAUX
-#define IFA_MID_WAUX 0       // cache policy of the weight requests (2 = non-temporal)
-#endif
-constexpr int md_vm(int ta) { return IFA_MID_ABL == 1 ? 2 : (IFA_MID_ABL == 5 ? ta : ta + 2); }      // direct-to-LDS requests per wave and stage: TA (activations) + 2 (weights)
+constexpr int MD_NS = 4;                                               // stages of the ring: one read, one landed, two on their way
+constexpr int MD_THREADS = 2 * MD_NT;                                  // launched threads: MD_NT compute and run the tails, as many request the activations
 
-__device__ __forceinline__ md_u4 md_lds_b128(uint32_t addr) { md_u4 v; asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr)); return v; }
-__device__ __forceinline__ uint32_t md_lds_b32(uint32_t addr) { uint32_t v; asm volatile("ds_read_b32 %0, %1" : "=v"(v) : "v"(addr)); return v; }
+template <int OFF>
+__device__ __forceinline__ md_u4 md_lds_b128(uint32_t addr) { md_u4 v; asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF)); return v; }
+template <int I, int N, class F>
+__device__ __forceinline__ void md_each(F f) { if constexpr (I < N) { f(std::integral_constant<int, I>()); md_each<I + 1, N>(f); } }
 
 // EPI: GM_PLAIN | GM_RESIDUAL | GM_GLU (a weight tile = 64 rows of w1 and the same 64 rows of w3).  KS: parts of K (workgroups per
-// tile).  NS: stages of the ring.  TA: 32-token accumulator tiles of a wave -- the tile is 32 TA tokens x 128 weight rows (TA = 2 up to 64 tokens:
-// half of the products, fragment reads, activation requests and exchanged sums of a 128-row tile whose lower half repeats a row -- 37 tokens 4.67 -> 3.83 ms,
-// the same bits; TA = 8: a measurement setting).  LEAD: 16-column groups that the fragments are requested ahead.
-template <int EPI, int KS, int NS, int TA, int LEAD>
-__global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_gemm_mid(const GmArgs P, const BigGeo G)
+// tile).  TA: 32-token accumulator tiles of a wave -- the tile is 32 TA tokens x 128 weight rows (TA = 2 up to 64 tokens: half of the products, fragment reads,
+// activation requests and exchanged sums of a 128-row tile whose lower half repeats a row -- 37 tokens 4.67 -> 3.83 ms, the same bits).
+template <int EPI, int KS, int TA>
+__global__ void __launch_bounds__(MD_THREADS, 2) k_gemm_mid(const GmArgs P, const BigGeo G)
 {
     constexpr int BM = 32 * TA, BN = MD_BN, BK = MD_BK, NW = MD_NW, NT = MD_NT, ROWB = BK * 2;
-    constexpr int MD_A_BYTES = md_a_bytes(TA), MD_STAGE = md_stage(TA), MD_VM = md_vm(TA), XP = TA;      // XP: activation pieces (8 token rows) a wave requests per stage
+    constexpr int NS = MD_NS, STAGE = md_a_bytes(TA), XP = TA, LEAD = 2;      // XP: activation pieces (8 token rows) a loader wave requests per stage; LEAD: 16-column groups that the fragments are requested ahead
+    static_assert((NS - 1) * STAGE + STAGE <= 65536, "stages that an LDS read's offset reaches");
     constexpr bool GLU = EPI == GM_GLU;
     constexpr int BNE = GLU ? BN / 2 : BN;
     auto swz = [](int r) { return (r >> 1) & 7; };
@@ -80,7 +77,7 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
     const half_t *__restrict__ X = P.X;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave = wave_all & (NW - 1);              // a loader wave (IFA_MID_LOADERS) requests the pieces of the computing wave on its SIMD
+    const int wave = wave_all & (NW - 1);
     const bool loader = wave_all >= NW;
     // XCD-aware tile order, bands of token tiles (k_gemm_big's mapping)
     int wg;
@@ -101,8 +98,8 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
     const int ksteps = G.K / BK;
     const int s0 = (int)((long long)kz * ksteps / KS), nsteps = (int)((long long)(kz + 1) * ksteps / KS) - s0;      // (parts of K may differ by one step)
 
-    // ---- sources of this wave's direct-to-LDS pieces
-    // activations: 4 pieces of 8 token rows x 128 bytes; lane -> (row, chunk), the swizzle applied to the SOURCE (the load writes LDS linearly)
+    // ---- sources
+    // activations (loader waves): TA pieces of 8 token rows x 128 bytes; lane -> (row, chunk), the swizzle applied to the SOURCE (the load writes LDS linearly)
     const half_t *xsrc[XP];
 #pragma unroll
     for (int j = 0; j < XP; j++) {
@@ -113,50 +110,36 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
     // weights: this wave's 32 rows = two 16-row tiles of the MO copy (ifa_gemm_rows_mfma.h: per tile, superstep S of 128 columns is ONE
     // contiguous KiB -- lane 16 g + r holds the 16 code bytes of block 4 S + g of row r -- so a tile's K range is one linear stream,
     // like a decode row; the tiled rows fetched 32 bytes per row and step measured 1 TB/s: 32 DRAM pages per request).  A step is
-    // half a superstep: lane -> (tile l / 32, block (l / 16) % 2 of the half, row l % 16), 2 x 512 contiguous bytes per request.
+    // half a superstep: lane -> (block l / 32 of the half, tile (l / 16) % 2, row l % 16), 2 x 512 contiguous bytes per request.
     const int nsup = nblk >> 2;
     const size_t mo_tile = mo_tile_bytes(nsup);
-    const uint8_t *wsrc, *wsbs;
+    __amdgpu_buffer_rsrc_t wres;
+    uint32_t woff;
     {
         const int nl0 = wave * 32;
         const uint8_t *Wm = (GLU && nl0 >= BNE) ? P.W1 : W;
-        const int row0 = n0 + (GLU && nl0 >= BNE ? nl0 - BNE : nl0);
-        const int tile16 = min((row0 >> 4) + (lane >> 5), ((N + 15) >> 4) - 1);
-        wsrc = Wm + (size_t)tile16 * mo_tile + (size_t)(lane & 31) * 16;
-        wsbs = Wm + (size_t)tile16 * mo_tile + mo_words_at(nsup) + (size_t)(lane & 31) * 4;
+        const int first = (n0 + (GLU && nl0 >= BNE ? nl0 - BNE : nl0)) >> 4, last = ((N + 15) >> 4) - 1;
+        const int tile0 = min(first, last), two = min(first + 1, last) - tile0;          // (a tile behind the rows: the last one again)
+        const uint64_t at = (uint64_t)(Wm + (size_t)tile0 * mo_tile);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)at), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32));
+        wres = __builtin_amdgcn_make_buffer_rsrc((void *)(((uint64_t)hi << 32) | lo), 0, (int)((1 + two) * mo_tile), 0x00020000);
+        woff = ((lane >> 4) & 1) && two ? (uint32_t)mo_tile : 0u;
     }
-    // the six requests of a stage, one at a time (piece 0..3: activation rows, 4: codes, 5: (base, scale) words): the main loop places
-    // them between its MFMAs
-    auto issue_piece = [&](int step, int slot, int piece) {
-        char *st = smem + (size_t)slot * MD_STAGE;
-        if (piece < XP) {
-#if IFA_MID_ABL != 1
-            __builtin_amdgcn_global_load_lds((md_glb_t *)(xsrc[piece] + (size_t)(s0 + step) * BK), (md_lds_t *)(st + (size_t)(wave * XP + piece) * 1024), 16, 0, 0);
-#endif
-            return;
-        }
-#if IFA_MID_ABL != 5
-        const int S = (s0 + step) >> 1, half = (s0 + step) & 1;
-        if (piece == XP)
-            __builtin_amdgcn_global_load_lds((md_glb_t *)(wsrc + (size_t)S * 1024 + (size_t)half * 512), (md_lds_t *)(st + MD_A_BYTES + wave * 1024), 16, 0, IFA_MID_WAUX);
-        else
-            __builtin_amdgcn_global_load_lds((md_glb_t *)(wsbs + (size_t)S * 256 + (size_t)half * 128),
-                                             (md_lds_t *)(st + MD_A_BYTES + MD_WC_BYTES + wave * 256), 4, 0, IFA_MID_WAUX);
-#endif
-    };
-    auto issue = [&](int step, int slot) {
+    const uint32_t wc_off = woff + (uint32_t)((lane >> 5) * 256 + (lane & 15) * 16), wb_off = woff + (uint32_t)(mo_words_at(nsup) + (lane >> 5) * 64 + (lane & 15) * 4);
+    auto issue = [&](int step, int slot) {          // a loader wave's requests of a stage
+        char *st = smem + (size_t)slot * STAGE;
 #pragma unroll
-        for (int pc = 0; pc < XP + 2; pc++) issue_piece(step, slot, pc);
+        for (int j = 0; j < XP; j++)
+            __builtin_amdgcn_global_load_lds((md_glb_t *)(xsrc[j] + (size_t)(s0 + step) * BK), (md_lds_t *)(st + (size_t)(wave * XP + j) * 1024), 16, 0, 0);
     };
 
     // ---- per-lane LDS offsets: lane (i, g) reads token row i of a 32-row tile, chunk 2 ks + g; weight row i of its wave
     const int i = lane & 31, g = lane >> 5;
     const int lc = g ^ swz(i);
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(md_lds_t *)smem;
-    const uint32_t a_off = lds0 + (uint32_t)(i * ROWB);
-    // (the stage holds this wave's codes as [tile][block of the half][row] x 16 bytes, the words likewise x 4 bytes)
-    const uint32_t wc_off = lds0 + (uint32_t)(MD_A_BYTES + wave * 1024 + ((i >> 4) * 32 + (i & 15)) * 16);
-    const uint32_t ws_off = lds0 + (uint32_t)(MD_A_BYTES + MD_WC_BYTES + wave * 256 + ((i >> 4) * 32 + (i & 15)) * 4);
+    const uint32_t a_off = (uint32_t)(uintptr_t)(md_lds_t *)smem + (uint32_t)(i * ROWB);
+    uint32_t a_at[4];          // by 16-column group; stage and token tile are the reads' offsets
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) a_at[ks] = a_off + (uint32_t)(((2 * ks) ^ lc) << 4);
 
     md_f16v acc[TA];
 #pragma unroll
@@ -164,127 +147,117 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[a][r] = 0.0f;
 
-    constexpr bool LD = IFA_MID_LOADERS != 0;
-    if (!LD || loader) {
+    if (loader) {
+        // the loader wave of a SIMD: a request takes ~70 cycles of the instruction stream that issues it; here they go out while the computing wave multiplies.  It waits
+        // for ITS requests of stage `step` + 1 (vmcnt is per wave), every wave meets at the barrier, and it requests stage `step` + 3 into the slot that the computing
+        // waves have just left.
 #pragma unroll
         for (int p = 0; p < NS - 1; p++) issue(min(p, nsteps - 1), p);
-    }
-    int slot = 0;
-    if constexpr (LD) {
-        // The loader wave of a SIMD (IFA_MID_LOADERS): the six requests of a stage took their issue slots (~70 cycles each, ablation
-        // builds: profiles/r06_prefill_mid_parts.log) out of the ONE instruction stream that also issues the MFMAs; a second wave on
-        // the SIMD issues them on the memory port while the computing wave multiplies.  Same ring protocol, same barrier: the loader
-        // waits for ITS requests of stage `step` (vmcnt is per wave), every wave meets at the barrier, the loader requests stage
-        // step + NS - 1 into the slot the computing waves have just left.
-        if (loader) {
-            for (int step = 0; step < nsteps; step++) {
-                asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NS - 2) * MD_VM) : "memory");
-                __builtin_amdgcn_s_barrier();
-                const int nslot = slot == 0 ? NS - 1 : slot - 1;
-                issue(min(step + NS - 1, nsteps - 1), nslot);
-                slot = slot + 1 == NS ? 0 : slot + 1;
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the repeats behind the last stage have landed before the ring is reused
-            __builtin_amdgcn_s_barrier();                          // (pairs with the computing waves' first barrier behind the loop)
-            return;
+        for (int step = 0, slot = NS - 1; step < nsteps; step++) {
+            asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NS - 3) * XP) : "memory");
+            __builtin_amdgcn_s_barrier();
+            issue(min(step + NS - 1, nsteps - 1), slot);
+            slot = slot + 1 == NS ? 0 : slot + 1;
         }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the repeats behind the last stage have landed before the ring is reused
+        __builtin_amdgcn_s_barrier();                          // (pairs with the computing waves' first barrier behind the loop)
+        return;
     }
     if (trc) trc[1] = wall_clock64();
-    for (int step = 0; step < nsteps; step++) {
-        // stage `step` has landed (the NS - 2 younger stages may still be in flight); the barrier makes every wave's pieces visible
-        // and says that every wave is done with the stage read last step, whose slot takes the request of stage step + NS - 1
-        // (the bare barrier: __syncthreads() is fence + barrier, and the fence waits vmcnt(0) -- for the stages just requested)
-        if constexpr (!LD) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NS - 2) * MD_VM) : "memory");
-#if IFA_MID_ABL != 4
-        __builtin_amdgcn_s_barrier();
-#endif
-        asm volatile("" ::: "memory");
-        const int nslot = slot == 0 ? NS - 1 : slot - 1, nstep = min(step + NS - 1, nsteps - 1);      // the stage requested during this step
-        const uint32_t sb = (uint32_t)(slot * MD_STAGE);
-        // A wave alone on its SIMD issues in order: request issue (6 x ~80 cycles), the 19 LDS reads and their latency, the conversion and
-        // the MFMAs ran one after the other (0.65 us per step, IFA_MID_TRACE; the MFMAs alone are 0.21).  Now only the raw weights and the
-        // first group's activation fragments are read in front of the MFMAs; the other groups' fragments, the next stage's requests and
-        // the next group's conversion go BETWEEN the MFMAs (sched_barrier pins the order).
-        md_u4 cw[2]; md_u2 sw; md_u4 fa[4][TA];
-        cw[0] = md_lds_b128(wc_off + sb);
-        cw[1] = md_lds_b128(wc_off + sb + 256);
-        sw[0] = md_lds_b32(ws_off + sb);
-        sw[1] = md_lds_b32(ws_off + sb + 64);
+    // The computing waves.  A wave alone on its SIMD issues one instruction in some 8 cycles and a 32 x 32 x 16 product occupies the matrix unit for 32: what is not between
+    // products is lost.  So a step has no start and no end: during group G's TA products the fragments of group G + LEAD are requested and the weights of group G + 1
+    // converted, whether or not these belong to the next step (whose stage has landed by then), and the codes of the step after next are on their way to registers.
+    // sched_barrier pins the order; the loop is unrolled by the ring, so that a read's address is a register of its group and an offset.
+    md_u4 raw_c[2], cw; uint32_t raw_b[2]; md_u2 sw;          // codes and (base, scale) words as they come: lane half g holds block g of the step; then by 16-column group / by block
+    auto request = [&](int step, int k) {
+        const int at = s0 + min(step, nsteps - 1);
+        raw_c[k] = __builtin_amdgcn_raw_buffer_load_b128(wres, (int)wc_off, at * 512, 0);
+        raw_b[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(wres, (int)wb_off, at * 128, 0);
+    };
+    auto arrange = [&](int k) {          // a lane's chunk of group ks is 2 (ks % 2) + g of block ks / 2
+        const uint32_t c0 = raw_c[k][0], c1 = raw_c[k][1], c2 = raw_c[k][2], c3 = raw_c[k][3], w = raw_b[k];
+        const auto p = __builtin_amdgcn_permlane32_swap(c0, c1, false, false), q = __builtin_amdgcn_permlane32_swap(c2, c3, false, false), r = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+        cw = md_u4{p[0], q[0], p[1], q[1]};
+        sw = md_u2{r[0], r[1]};
+    };
+    // this lane's 8 weights of group ks -- q4x8_dequant_mo's arithmetic (ifa_dequant_q4.h) in four pieces
+    uint32_t d_lo = 0, d_hi = 0; q4_h2 d_s2 = {0, 0}, d_b2 = {0, 0}, d_w[4];
+    auto dq_a = [&](int ks) {
+        const uint32_t code = cw[ks], sbw = sw[ks >> 1];
+        d_lo = code & 0x0F0F0F0Fu; d_hi = (code >> 4) & 0x0F0F0F0Fu;
+        d_s2 = q4_scale2(sbw); d_b2 = q4_base2(sbw);
+    };
+    auto dq_b = [&]() { d_w[0] = q4_value2<false>(d_lo, d_s2, d_b2); d_w[1] = q4_value2<true>(d_lo, d_s2, d_b2); };
+    auto dq_c = [&]() { d_w[2] = q4_value2<false>(d_hi, d_s2, d_b2); d_w[3] = q4_value2<true>(d_hi, d_s2, d_b2); };
+    auto dq_d = [&]() { return md_h8{d_w[0][0], d_w[0][1], d_w[1][0], d_w[1][1], d_w[2][0], d_w[2][1], d_w[3][0], d_w[3][1]}; };
+    md_u4 fa[4][TA];          // fragments by 16-column group
+    // (a counted wait names the registers it makes valid: later uses depend on the statement)
+    auto landed = [&](int k) {
 #pragma unroll
-        for (int a = 0; a < TA; a++) fa[0][a] = md_lds_b128(a_off + sb + (uint32_t)(a * 32 * ROWB) + (uint32_t)(((0) ^ lc) << 4));
-        // fragments are requested LEAD 16-column groups ahead (round 6, second pass): with one group of lead and TA = 4 the wave sat in
-        // lgkmcnt(0) at the end of every group -- four waves read 64 KB of LDS per step, 512 cycles of the LDS pipe, as long as the step's
-        // MFMAs -- so the waits are counted (LDS returns in order; nothing else of this loop counts on lgkmcnt; the counter holds 15) and
-        // the pipe never drains.  TA = 8: a group's eight MFMAs cover the next group's reads, one group of lead.
-        if constexpr (LEAD == 2) {
-#pragma unroll
-            for (int a = 0; a < TA; a++) fa[1][a] = md_lds_b128(a_off + sb + (uint32_t)(a * 32 * ROWB) + (uint32_t)(((2) ^ lc) << 4));
-        }
-        // (a counted wait names the registers it makes valid: later uses depend on the statement)
-        auto landed = [&](int k) {
-#pragma unroll
-            for (int a = 0; a < TA; a++) asm volatile("" : "+v"(fa[k][a]));
-        };
-        asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(cw[0]), "+v"(cw[1]), "+v"(sw) : "n"(TA * LEAD));
-        // this lane's 8 weights of group ks: chunk 2 (ks % 2) + g of block ks / 2 -- q4x8_dequant_mo's arithmetic (ifa_dequant_q4.h) in four pieces
-        uint32_t d_lo = 0, d_hi = 0; q4_h2 d_s2 = {0, 0}, d_b2 = {0, 0}, d_w[4];
-        auto dq_a = [&](int ks) {
-            const int h = ks >> 1;
-            const uint32_t c_lo = cw[h][2 * (ks & 1)], c_hi = cw[h][2 * (ks & 1) + 1];      // (scalars first: one select, not an indexed element read)
-            const uint32_t code = g ? c_hi : c_lo, sbw = sw[h];
-            d_lo = code & 0x0F0F0F0Fu; d_hi = (code >> 4) & 0x0F0F0F0Fu;
-            d_s2 = q4_scale2(sbw); d_b2 = q4_base2(sbw);
-        };
-        auto dq_b = [&]() { d_w[0] = q4_value2<false>(d_lo, d_s2, d_b2); d_w[1] = q4_value2<true>(d_lo, d_s2, d_b2); };
-        auto dq_c = [&]() { d_w[2] = q4_value2<false>(d_hi, d_s2, d_b2); d_w[3] = q4_value2<true>(d_hi, d_s2, d_b2); };
-        auto dq_d = [&]() { return md_h8{d_w[0][0], d_w[0][1], d_w[1][0], d_w[1][1], d_w[2][0], d_w[2][1], d_w[3][0], d_w[3][1]}; };
-        auto frag = [&](int ks, int a) { fa[ks][a] = md_lds_b128(a_off + sb + (uint32_t)(a * 32 * ROWB) + (uint32_t)(((2 * ks) ^ lc) << 4)); };
-        md_h8 fbc, fbn;
-        dq_a(0); dq_b(); dq_c(); fbc = dq_d();
-        asm volatile("s_waitcnt lgkmcnt(%0)" :: "n"(TA * (LEAD - 1)));
-        landed(0);
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-#if IFA_MID_ABL == 2
-#pragma unroll
-            for (int a = 0; a < TA; a++) acc[a][ks] += (float)fbc[a % 8] * (float)__builtin_bit_cast(md_h8, fa[ks][a])[0];
-            if (ks < 3) { dq_a(ks + 1); dq_b(); dq_c(); fbn = dq_d(); }
-            if (ks + LEAD < 4) for (int a = 0; a < TA; a++) frag(ks + LEAD, a);
-            if (ks < 3 && !LD) for (int pc = ks * TA; pc < (ks + 1) * TA && pc < XP + 2; pc++) issue_piece(nstep, nslot, pc);
-#else
-            // TA MFMAs; between them (sched_barrier pins the order): the fragment reads of group ks + LEAD two at a time, the four pieces of
-            // the next group's conversion, and -- without loader waves -- the next stage's requests
-#pragma unroll
-            for (int a = 0; a < TA; a++) {
+        for (int a = 0; a < TA; a++) asm volatile("" : "+v"(fa[k][a]));
+    };
+    md_h8 fbc, fbn;
+    request(0, 0); request(1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    // the bare barrier (__syncthreads() is fence + barrier): stages `step` and `step` + 1 have landed, the one read last step may be overwritten
+    auto enter = [&]() { __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); };
+    auto one = [&](int step, auto J) {          // step % NS == J
+        constexpr int j = decltype(J)::value;
+        md_each<0, 4>([&](auto K) {
+            constexpr int ks = K.value, kf = (ks + LEAD) & 3, jf = ks + LEAD < 4 ? j : (j + 1) % NS;          // the group requested now, its stage
+            md_each<0, TA>([&](auto A) {
+                constexpr int a = A.value;
                 __builtin_amdgcn_sched_barrier(0);
                 acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(md_h8, fa[ks][a]), fbc, acc[a], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
-                if (ks + LEAD < 4 && 2 * a + 1 < TA) { frag(ks + LEAD, 2 * a); frag(ks + LEAD, 2 * a + 1); }
-                if (ks < 3) {
-                    if (a == 0) dq_a(ks + 1);
-                    if (a == TA / 4) dq_b();
-                    if (a == TA / 2) dq_c();
-                    if (a == 3 * TA / 4) fbn = dq_d();
-                    if constexpr (!LD) { if (ks * TA + a < XP + 2) issue_piece(nstep, nslot, ks * TA + a); }
+                if constexpr (2 * a < TA) {
+                    fa[kf][2 * a] = md_lds_b128<jf * STAGE + 2 * a * 32 * ROWB>(a_at[kf]);
+                    fa[kf][2 * a + 1] = md_lds_b128<jf * STAGE + (2 * a + 1) * 32 * ROWB>(a_at[kf]);
                 }
-            }
-#endif
-            if (ks < 3) {
-                // group ks + 1 has landed; with two groups of lead the TA requests of group ks + 2 may still be in flight
-                if (LEAD == 2 && ks + 2 < 4) asm volatile("s_waitcnt lgkmcnt(%0)" :: "n"(TA));
-                else asm volatile("s_waitcnt lgkmcnt(0)");
-                landed(ks + 1);
-            }
+                if constexpr (a == 0) {
+                    if constexpr (ks == 3) { arrange((j + 1) & 1); request(step + 3, (j + 1) & 1); }
+                    dq_a((ks + 1) & 3);
+                }
+                if constexpr (a == TA / 4) dq_b();
+                if constexpr (a == TA / 2) dq_c();
+                if constexpr (a == 3 * TA / 4) fbn = dq_d();
+            });
+            // group ks + 1 has landed; with two groups of lead the TA requests of group ks + 2 may still be in flight
+            asm volatile("s_waitcnt lgkmcnt(%0)" :: "n"(TA * (LEAD - 1)));
+            landed((ks + 1) & 3);
             fbc = fbn;
-        }
-        slot = slot + 1 == NS ? 0 : slot + 1;
+        });
+        enter();          // (behind the last step: the loader waves' last barrier, their requests have landed; they end there)
+    };
+    enter();
+    md_each<0, LEAD>([&](auto K) { md_each<0, TA>([&](auto A) { fa[K.value][A.value] = md_lds_b128<A.value * 32 * ROWB>(a_at[K.value]); }); });
+    arrange(0); request(2, 0);
+    dq_a(0); dq_b(); dq_c(); fbc = dq_d();
+    asm volatile("s_waitcnt lgkmcnt(%0)" :: "n"(TA * (LEAD - 1)));
+    landed(0);
+    int step = 0;
+    for (; step + NS <= nsteps; step += NS) {
+        one(step, std::integral_constant<int, 0>());
+        one(step + 1, std::integral_constant<int, 1>());
+        one(step + 2, std::integral_constant<int, 2>());
+        one(step + 3, std::integral_constant<int, 3>());
     }
-    // the repeats requested behind the last stage must have landed before the ring's memory is used for anything else
+    if (step < nsteps) {
+        one(step, std::integral_constant<int, 0>());
+        if (step + 1 < nsteps) {
+            one(step + 1, std::integral_constant<int, 1>());
+            if (step + 2 < nsteps) one(step + 2, std::integral_constant<int, 2>());
+        }
+    }
+    static_assert(NS == 4, "the loop is unrolled by the ring");
+    // what was requested behind the last step: in, before its registers and the ring's memory are used for anything else
+    asm volatile("s_waitcnt lgkmcnt(0)");
+#pragma unroll
+    for (int k = 0; k < LEAD; k++) landed(k);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if constexpr (LD) __builtin_amdgcn_s_barrier();      // (the loader waves' last barrier: their requests have landed; they end there)
     if (trc) trc[2] = wall_clock64();
-    // ---- parts of K as a REDUCE-SCATTER (KS > 1).  A thread's 64 sums are 16 units of 16 bytes; unit u = 4 a + q holds the 8 token
-    // rows [8 u, 8 u + 8) of this lane's weight row.  Part kz OWNS units [kz UB, (kz + 1) UB), i.e. token rows [8 kz UB, 8 (kz + 1) UB) of the
+    // ---- parts of K as a REDUCE-SCATTER (KS > 1).  A thread's 16 TA sums are 4 TA units of 16 bytes; unit u = 4 a + q holds the 8 token
+    // rows of band u for this lane's weight row.  Part kz OWNS bands [kz UB, (kz + 1) UB), i.e. token rows [8 kz UB, 8 (kz + 1) UB) of the
     // tile: it stores its other units (write-through, 16 bytes per store), arrives at the tile's counter, waits for all KS
     // parts, adds the other parts' values of ITS units in K order (part 0 + part 1 + ... with its own at position kz: the same
     // sequence of additions whichever part performs it) and runs the epilogue for its rows.  k_gemm_big's form -- the last part
@@ -292,7 +265,7 @@ __global__ void __launch_bounds__(MD_THREADS, TA == 4 && LEAD == 1 ? 4 : 2) k_ge
     // (KS - 1) / KS x 64 KB per workgroup whatever KS is, so short products can be cut into enough parts to fill the chip twice.
     constexpr int NU = 4 * TA;                           // 8-token-row bands of the tile = 16-byte units of a thread's sums
     static_assert(NU % KS == 0, "parts of K must divide the tile's row bands");
-    constexpr int UB = NU / KS;                          // units (8-row bands) a part owns
+    constexpr int UB = NU / KS;                          // bands a part owns
     const int row_lo = KS == 1 ? 0 : kz * UB * 8, nrows_own = KS == 1 ? BM : UB * 8;
     constexpr int VEC = BNE / 8;
     constexpr int PIECES = (BM / KS * VEC + NT - 1) / NT;  // 16-byte output pieces per thread (its part's rows)
@@ -446,8 +419,8 @@ bool gemm_mid_ok(int w_dtype, const GmArgs &P, int epi)
     return true;
 }
 
-template <int EPI, int KS, int NS, int TA, int LEAD>
-static int md_run_lead(const GmArgs &P, BigGeo G, int tn_count, hipStream_t s)
+template <int EPI, int KS, int TA>
+static int md_run(const GmArgs &P, BigGeo G, int tn_count, hipStream_t s)
 {
     if constexpr (KS > 1) {
         G.err = wait_err_word();
@@ -457,8 +430,8 @@ static int md_run_lead(const GmArgs &P, BigGeo G, int tn_count, hipStream_t s)
         if (rcs) return rcs;
         G.flags = (unsigned *)scratch; G.part = (unsigned long long *)((char *)scratch + SPLITK_FLAG_BYTES_H);
     }
-    const size_t smem = std::max((size_t)NS * md_stage(TA), (size_t)(32 * TA) * (MD_BN * 2 + 64));
-    auto kern = k_gemm_mid<EPI, KS, NS, TA, LEAD>;
+    const size_t smem = std::max((size_t)MD_NS * md_a_bytes(TA), (size_t)(32 * TA) * (MD_BN * 2 + 64));
+    auto kern = k_gemm_mid<EPI, KS, TA>;
     static std::atomic<uint64_t> attr_set{0};
     int dev = 0;
     (void)hipGetDevice(&dev);
@@ -486,27 +459,13 @@ static int md_run_lead(const GmArgs &P, BigGeo G, int tn_count, hipStream_t s)
             for (long long b = 0; b < grid; b++) t0 = std::min(t0, h[(size_t)b * 8]);
             double mx[5] = {0, 0, 0, 0, 0}, sm[5] = {0, 0, 0, 0, 0};
             for (long long b = 0; b < grid; b++) for (int k = 0; k < 5; k++) { const double v = (h[(size_t)b * 8 + k] - t0) * 0.01; mx[k] = std::max(mx[k], v); sm[k] += v; }
-            fprintf(stderr, "k_gemm_mid<%d,%d,%d,%d> grid %lld steps %d | us after the first workgroup's start, mean (max): start %.2f (%.2f) loop begins %.2f (%.2f) loop ends %.2f (%.2f) parts summed %.2f (%.2f) end %.2f (%.2f)\n",
-                    EPI, KS, NS, TA, grid, G.K / MD_BK / KS, sm[0] / grid, mx[0], sm[1] / grid, mx[1], sm[2] / grid, mx[2], sm[3] / grid, mx[3], sm[4] / grid, mx[4]);
+            fprintf(stderr, "k_gemm_mid<%d,%d,%d> grid %lld steps %d | us after the first workgroup's start, mean (max): start %.2f (%.2f) loop begins %.2f (%.2f) loop ends %.2f (%.2f) parts summed %.2f (%.2f) end %.2f (%.2f)\n",
+                    EPI, KS, TA, grid, G.K / MD_BK / KS, sm[0] / grid, mx[0], sm[1] / grid, mx[1], sm[2] / grid, mx[2], sm[3] / grid, mx[3], sm[4] / grid, mx[4]);
             return IFA_OK;
         }
     }
     kern<<<dim3((unsigned)grid), dim3(MD_THREADS), smem, s>>>(P, G);
     return IFA_OK;
-}
-
-#ifndef IFA_MID_NS
-#define IFA_MID_NS 3
-#endif
-
-// 128-token tiles, two workgroups on a compute unit where there are that many: 120 registers with one group of lead; 136 with two, which keep the second workgroup out.  A step of
-// a lone workgroup takes 0.54 us, of two together 0.84: 384 / 512 / 768 tokens 9.83 -> 9.45, 10.70 -> 10.24, 15.81 -> 15.42 ms.  A lone one needs the lead (96 tokens 4.40 -> 4.49
-// without).
-template <int EPI, int KS, int NS, int TA>
-static int md_run(const GmArgs &P, const BigGeo &G, int tn_count, hipStream_t s)
-{
-    if constexpr (TA == 4) { if ((long long)G.tiles_m * tn_count * KS <= md_num_cus()) return md_run_lead<EPI, KS, NS, TA, 2>(P, G, tn_count, s); }
-    return md_run_lead<EPI, KS, NS, TA, TA == 2 ? 2 : 1>(P, G, tn_count, s);
 }
 
 template <int EPI, int TA>
@@ -521,11 +480,8 @@ static int md_launch(const GmArgs &P, hipStream_t s)
     for (int i = P.nsets; i < 3; i++) G.tile0[i] = 1 << 30;
     G.tiles_m = (P.T + MD_BM - 1) / MD_BM; G.K = P.nblk * 32; G.tn0 = 0;
     const int ksteps = G.K / MD_BK;
-    // parts of K: the most that still put ONE workgroup on a CU.  (Two fit, but parts cost: the exchange of their sums is 4.5 to 8 us of a launch, and with two workgroups on
-    // a CU it is longer than what the shorter loops give -- wo / w2 of 192 and 512 tokens as 512 workgroups: 6.21 -> 7.27 and 9.97 -> 10.5 ms in all; the gated pair of 96
-    // tokens as 344 instead of 172: 4.40 -> 4.64; 37 tokens: the same.)  Every part >= MINS steps
-    static const bool two_per_cu = getenv("IFA_MID_TWO_PER_CU") != nullptr;      // (measurement: the first form's limit)
-    const long long tiles = (long long)G.tiles_m * tn_count, cap = (two_per_cu ? 2ll : 1ll) * md_num_cus();
+    // parts of K: the most that still put ONE workgroup on a CU (150 registers and eight waves: two do not fit).  Every part >= MINS steps
+    const long long tiles = (long long)G.tiles_m * tn_count, cap = md_num_cus();
     static const bool no_glu_split = getenv("IFA_MID_NO_GLU_SPLIT") != nullptr;      // (measurement: the gated pair as ONE part of K, like k_gemm_big's -- bit-identical products)
     const bool may = !P.no_waits && waits_enabled() && !(EPI == GM_GLU && no_glu_split);
     int rc = 1;
@@ -535,12 +491,10 @@ static int md_launch(const GmArgs &P, hipStream_t s)
     const int force_ks = force_epi ? force_epi : force_all;
     static const int mins = getenv("IFA_MID_MINSTEPS") ? atoi(getenv("IFA_MID_MINSTEPS")) : 4;
     auto fits = [&](int ks) { return may && tiles * ks <= cap && ksteps / ks >= mins && (!force_ks || ks <= force_ks); };
-    // (16 parts: the exchanged sums grow with the part count -- 30 MB written and read for wo: 30 us against 17 at 8 -- a measurement setting)
-    if constexpr (TA == 4) { if (force_ks >= 16 && fits(16)) rc = md_run<EPI, 16, IFA_MID_NS, TA>(P, G, tn_count, s); }
-    if (rc == 1 && fits(8)) rc = md_run<EPI, 8, IFA_MID_NS, TA>(P, G, tn_count, s);
-    if (rc == 1 && fits(4)) rc = md_run<EPI, 4, IFA_MID_NS, TA>(P, G, tn_count, s);
-    if (rc == 1 && fits(2)) rc = md_run<EPI, 2, IFA_MID_NS, TA>(P, G, tn_count, s);
-    if (rc == 1) rc = md_run<EPI, 1, IFA_MID_NS, TA>(P, G, tn_count, s);
+    if (rc == 1 && fits(8)) rc = md_run<EPI, 8, TA>(P, G, tn_count, s);
+    if (rc == 1 && fits(4)) rc = md_run<EPI, 4, TA>(P, G, tn_count, s);
+    if (rc == 1 && fits(2)) rc = md_run<EPI, 2, TA>(P, G, tn_count, s);
+    if (rc == 1) rc = md_run<EPI, 1, TA>(P, G, tn_count, s);
     if (rc) return rc;
     IFA_LAUNCH_CHECK();
     return IFA_OK;
@@ -549,16 +503,7 @@ static int md_launch(const GmArgs &P, hipStream_t s)
 int gemm_mid(const GmArgs &P, int epi, hipStream_t s)
 {
     if (!gemm_mid_ok(Q4_B32T1A, P, epi)) return ifa_fail(IFA_ERR_ARG, "mid-length GEMM: %d blocks per row / epilogue %d", P.nblk, epi);
-    // 256-token tiles (TA = 8): the weight stream and its conversion serve twice the products per step
     static const int force_ta = getenv("IFA_MID_TA") ? atoi(getenv("IFA_MID_TA")) : 0;      // (measurement)
-    // (measured round 6: 512 / 768 tokens 10.96 / 16.48 ms with 128-token tiles, 11.37 / 17.50 with 256; 1024 tokens 19.57 / 19.25 -- the
-    //  wide tile pays only where the large-tile kernel already ties, so it stays a measurement setting)
-    const bool wide = force_ta == 8;
-    if (wide) {
-        if (epi == GM_PLAIN) return md_launch<GM_PLAIN, 8>(P, s);
-        if (epi == GM_RESIDUAL) return md_launch<GM_RESIDUAL, 8>(P, s);
-        return md_launch<GM_GLU, 8>(P, s);
-    }
     if (force_ta == 2 || (!force_ta && P.T <= 64)) {      // (65 .. 192 tokens: the same time either way)
         if (epi == GM_PLAIN) return md_launch<GM_PLAIN, 2>(P, s);
         if (epi == GM_RESIDUAL) return md_launch<GM_RESIDUAL, 2>(P, s);

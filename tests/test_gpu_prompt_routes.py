@@ -174,6 +174,23 @@ def test_products_that_stream_their_weights_over_few_rows_agree_with_the_others(
     wk.close()
 
 
+@pytest.mark.parametrize("T", [193, 257, 385])
+@pytest.mark.parametrize("wd,shape", [(dt.Q4_B32T1A, {}), (dt.Q3H_B64T1, dict(dim=1024, heads=16, kv_heads=2, head_dim=64, ffn=1408)), (dt.Q4_B32T1B, dict(dim=2176, heads=9, kv_heads=3, ffn=3712))],
+                         ids=["q4a", "q3h", "q4b"])
+def test_products_whose_steps_run_into_each_other_agree_with_the_large_tiles(wd, shape, T):
+    """rows that fill no tile, numbers of 64-column steps with every remainder by the ring's four stages (16, 22, 34, 58 steps, whole and in parts), biases everywhere"""
+    wk, s = _biased(dt.F16, wd, T, **shape)
+    toks = np.random.default_rng(T).integers(3, s["vocab"], T).astype(np.int32)
+    out = []
+    for v in (1, 0):
+        wk.set_option("prefill_mid", v)
+        out.append(_rows(wk, toks, s["vocab"])[1])
+        wk.reset()
+    ok, why = _agree(out[0], out[1])
+    assert ok, why
+    wk.close()
+
+
 @pytest.mark.parametrize("n", [9, 16, 17, 32])
 @pytest.mark.parametrize("kvd", [dt.F16, dt.Q8_B32T2], ids=["f16", "q8"])
 def test_batched_steps_of_many_queries_agree_with_the_rows_products_and_replay(kvd, n):
