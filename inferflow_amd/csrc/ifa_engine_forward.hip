@@ -294,9 +294,8 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
         pf_fused = batch_fused_ok(m, T);          // (ensure_mo may have switched the copies off: ask again, see forward_batch)
     }
     if (pf_big && !pf_mid && !pf_few && (rc = ensure_x32(m))) return rc;
-    // above prefill_mid_max: wo and w2 (4096 output columns: 128 x 128 tiles whatever the kernel) still through k_gemm_mid -- at 1024 tokens
-    // 41 / 102 us per launch against 51 / 143 for the split-K halves of the large-tile kernel, which keeps wq | wk | wv and the gated pair
-    // (profiles/r06_prefill_mid_parts.log section 13: 1024 / 1536 / 2048 tokens 4.5 / 3 / 0.8 % faster, 4096 tokens 4.7 % slower: up to 2048)
+    // above a lowered prefill_mid_max: wo and w2 (4096 output columns: 128 x 128 tiles whatever the kernel) still through k_gemm_mid -- at 1024 tokens
+    // 39 / 93 us per launch against 51 / 143 for the split-K halves of the large-tile kernel, which keeps wq | wk | wv and the gated pair
     const bool pf_res_mid = pf_big && !pf_mid && !pf_few && !tp && T <= m->opt_prefill_res_mid && prefill_mid_ok(m, T, true);
     if (pf_few && (rc = few_norm(m, 0, T_ATTN_NORM, T, nullptr, nullptr, x, nullptr))) return rc;
     for (int l = 0; l < c.layers && pf_fused; l++) {

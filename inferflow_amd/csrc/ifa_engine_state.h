@@ -211,9 +211,10 @@ struct ifa_model {
     int opt_prefill_chunk = 1;      // prompts of 34..48 tokens as two passes of <= 32 tokens (ifa_model_forward)
     // round 6: prompts of 33 .. prefill_mid_max tokens take the four launches per layer from k_gemm_mid (ifa_gemm_mid.hip: ring of
     // direct-to-LDS stages requested by loader waves, weights dequantised into the MFMA operand registers) when every linear has its
-    // operand-order copy; 320..768 tokens 8-9 % faster than the large tiles, 1024 tokens a tie (profiles/r06_prefill_mid_parts.log)
-    int opt_prefill_mid = 1, opt_prefill_mid_max = 768;
-    int opt_prefill_res_mid = 2048;   // prefill_mid_max + 1 .. this many tokens: wo / w2 still through k_gemm_mid, the other products through the large tiles (0: never)
+    // operand-order copy.  A layer's four products, Llama-2-7B, us, through the large tiles (wo / w2 of up to 2048 tokens already through k_gemm_mid) and here:
+    // 800 tokens 462 and 399, 1024 484 and 437, 1300 780 and 645, 1536 785 and 687, 2048 878 and 837, 3000 1362 and 1266, 4096 1642 and 1591, 6000 2622 and 2377, 8192 3161 and 3156
+    int opt_prefill_mid = 1, opt_prefill_mid_max = 8192;
+    int opt_prefill_res_mid = 2048;   // prefill_mid_max + 1 .. this many tokens (where prefill_mid_max was lowered): wo / w2 still through k_gemm_mid, the other products through the large tiles (0: never)
     // prompts of FEW_MIN .. FEW_MAX tokens and steps of as many queries through gemm_few (ifa_gemm_few.hip); its workspace, one allocation: rows in fragment order (a layer's
     // input, the gated pair's output), sums of the parts of K
     int opt_rows_few = 1;

@@ -1,4 +1,4 @@
-// ifa_gemm_mid.hip -- the linear layers of a 193..768-token prompt, wo / w2 of one up to 2048:  Y[T][N] = X[T][K] . W[N][K]^T  (+ bias, residual, GLU)
+// ifa_gemm_mid.hip -- the linear layers of prompts from 193 tokens on (shorter ones: ifa_gemm_few.hip):  Y[T][N] = X[T][K] . W[N][K]^T  (+ bias, residual, GLU)
 //
 // Reference: MatrixMultiplication (src/transformer/inference_worker.cc:2364-2432): Dequantize the weight tensor to F16, F16 x F16
 // product with fp32 accumulation (src/tensor/cublas_engine.cu:420-436).  Same values here: every weight is half(fma(q, scale,
@@ -60,13 +60,13 @@ __device__ __forceinline__ void md_each(F f) { if constexpr (I < N) { f(std::int
 
 // EPI: GM_PLAIN | GM_RESIDUAL | GM_GLU (a weight tile = 64 rows of w1 and the same 64 rows of w3).  KS: parts of K (workgroups per
 // tile).  TA: 32-token accumulator tiles of a wave -- the tile is 32 TA tokens x 128 weight rows (TA = 2 up to 64 tokens: half of the products, fragment reads,
-// activation requests and exchanged sums of a 128-row tile whose lower half repeats a row -- 37 tokens 4.67 -> 3.83 ms, the same bits).
+// activation requests and exchanged sums of a 128-row tile whose lower half repeats a row -- 37 tokens 4.67 -> 3.83 ms, the same bits; TA = 8: md_wide).
 template <int EPI, int KS, int TA>
 __global__ void __launch_bounds__(MD_THREADS, 2) k_gemm_mid(const GmArgs P, const BigGeo G)
 {
     constexpr int BM = 32 * TA, BN = MD_BN, BK = MD_BK, NW = MD_NW, NT = MD_NT, ROWB = BK * 2;
-    constexpr int NS = MD_NS, STAGE = md_a_bytes(TA), XP = TA, LEAD = 2;      // XP: activation pieces (8 token rows) a loader wave requests per stage; LEAD: 16-column groups that the fragments are requested ahead
-    static_assert((NS - 1) * STAGE + STAGE <= 65536, "stages that an LDS read's offset reaches");
+    constexpr int NS = MD_NS, STAGE = md_a_bytes(TA), XP = TA, LEAD = TA == 8 ? 1 : 2;      // XP: activation pieces (8 token rows) a loader wave requests per stage; LEAD: 16-column groups that the fragments are requested ahead
+    static_assert(NS * STAGE <= 2 * 65536, "stages that an LDS read's offset reaches from two addresses");
     constexpr bool GLU = EPI == GM_GLU;
     constexpr int BNE = GLU ? BN / 2 : BN;
     auto swz = [](int r) { return (r >> 1) & 7; };
@@ -137,9 +137,16 @@ __global__ void __launch_bounds__(MD_THREADS, 2) k_gemm_mid(const GmArgs P, cons
     const int i = lane & 31, g = lane >> 5;
     const int lc = g ^ swz(i);
     const uint32_t a_off = (uint32_t)(uintptr_t)(md_lds_t *)smem + (uint32_t)(i * ROWB);
-    uint32_t a_at[4];          // by 16-column group; stage and token tile are the reads' offsets
+    uint32_t a_at[NS * STAGE > 65536 ? 2 : 1][4];          // by 16-column group; stage and token tile are the reads' offsets
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++) a_at[ks] = a_off + (uint32_t)(((2 * ks) ^ lc) << 4);
+    for (int ks = 0; ks < 4; ks++) {
+        a_at[0][ks] = a_off + (uint32_t)(((2 * ks) ^ lc) << 4);
+        if constexpr (NS * STAGE > 65536) a_at[1][ks] = a_at[0][ks] + 65536;
+    }
+    auto frag = [&](auto K, auto J, auto A) {          // group, stage, token tile
+        constexpr int at = decltype(J)::value * STAGE + decltype(A)::value * 32 * ROWB;
+        return md_lds_b128<(at & 65535)>(a_at[at >> 16][decltype(K)::value]);
+    };
 
     md_f16v acc[TA];
 #pragma unroll
@@ -211,8 +218,9 @@ __global__ void __launch_bounds__(MD_THREADS, 2) k_gemm_mid(const GmArgs P, cons
                 acc[a] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(md_h8, fa[ks][a]), fbc, acc[a], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (2 * a < TA) {
-                    fa[kf][2 * a] = md_lds_b128<jf * STAGE + 2 * a * 32 * ROWB>(a_at[kf]);
-                    fa[kf][2 * a + 1] = md_lds_b128<jf * STAGE + (2 * a + 1) * 32 * ROWB>(a_at[kf]);
+                    const std::integral_constant<int, kf> kc; const std::integral_constant<int, jf> jc;
+                    fa[kf][2 * a] = frag(kc, jc, std::integral_constant<int, 2 * a>());
+                    fa[kf][2 * a + 1] = frag(kc, jc, std::integral_constant<int, 2 * a + 1>());
                 }
                 if constexpr (a == 0) {
                     if constexpr (ks == 3) { arrange((j + 1) & 1); request(step + 3, (j + 1) & 1); }
@@ -230,7 +238,7 @@ __global__ void __launch_bounds__(MD_THREADS, 2) k_gemm_mid(const GmArgs P, cons
         enter();          // (behind the last step: the loader waves' last barrier, their requests have landed; they end there)
     };
     enter();
-    md_each<0, LEAD>([&](auto K) { md_each<0, TA>([&](auto A) { fa[K.value][A.value] = md_lds_b128<A.value * 32 * ROWB>(a_at[K.value]); }); });
+    md_each<0, LEAD>([&](auto K) { md_each<0, TA>([&](auto A) { fa[K.value][A.value] = frag(K, std::integral_constant<int, 0>(), A); }); });
     arrange(0); request(2, 0);
     dq_a(0); dq_b(); dq_c(); fbc = dq_d();
     asm volatile("s_waitcnt lgkmcnt(%0)" :: "n"(TA * (LEAD - 1)));
@@ -491,13 +499,29 @@ static int md_launch(const GmArgs &P, hipStream_t s)
     const int force_ks = force_epi ? force_epi : force_all;
     static const int mins = getenv("IFA_MID_MINSTEPS") ? atoi(getenv("IFA_MID_MINSTEPS")) : 4;
     auto fits = [&](int ks) { return may && tiles * ks <= cap && ksteps / ks >= mins && (!force_ks || ks <= force_ks); };
-    if (rc == 1 && fits(8)) rc = md_run<EPI, 8, TA>(P, G, tn_count, s);
-    if (rc == 1 && fits(4)) rc = md_run<EPI, 4, TA>(P, G, tn_count, s);
-    if (rc == 1 && fits(2)) rc = md_run<EPI, 2, TA>(P, G, tn_count, s);
+    if constexpr (TA < 8) {
+        if (rc == 1 && fits(8)) rc = md_run<EPI, 8, TA>(P, G, tn_count, s);
+        if (rc == 1 && fits(4)) rc = md_run<EPI, 4, TA>(P, G, tn_count, s);
+        if (rc == 1 && fits(2)) rc = md_run<EPI, 2, TA>(P, G, tn_count, s);
+    }
     if (rc == 1) rc = md_run<EPI, 1, TA>(P, G, tn_count, s);
     if (rc) return rc;
     IFA_LAUNCH_CHECK();
     return IFA_OK;
+}
+
+// 256-token tiles: a weight is converted once for twice the products.  A round of one tile a compute unit takes 1.9 rounds of 128-token tiles (64 steps: 66 us against 34.5), a last
+// round that is not full 0.8 of a full one: the form with the shorter sum.  us a launch, Llama-2-7B, 128 -> 256 tokens a tile: wq | wk | wv of 512, 1536, 2048, 4096 tokens
+// 64.6, 162.5, 204.2, 401.3 -> 57.4, 177.3, 198.6, 385.8; the gated pair of 512, 1024, 1536, 4096 109.7, 215.6, 319.8, 784.6 -> 121.2, 198.8, 323.2, 729.8; wo of 1300, 2048, 3000
+// 61.7, 72.3, 105.7 -> 59.4, 70.8, 119.1.  No parts of K here: fewer tiles than three quarters of a round are better cut into 128-token tiles' parts (w2 of 1024 tokens 93.3 against 98.1).
+static bool md_wide(const GmArgs &P, int epi)
+{
+    const int bne = epi == GM_GLU ? MD_BN / 2 : MD_BN;
+    long long tn = 0;
+    for (int i = 0; i < P.nsets; i++) tn += (P.rows[i] + bne - 1) / bne;
+    const long long cu = md_num_cus(), n4 = (P.T + 127) / 128 * tn, n8 = (P.T + 255) / 256 * tn;
+    auto rounds = [&](long long n) { return (double)(n / cu) + (n % cu ? 0.8 : 0.0); };
+    return 4 * n8 >= 3 * cu && 1.9 * rounds(n8) < rounds(n4);
 }
 
 int gemm_mid(const GmArgs &P, int epi, hipStream_t s)
@@ -508,6 +532,11 @@ int gemm_mid(const GmArgs &P, int epi, hipStream_t s)
         if (epi == GM_PLAIN) return md_launch<GM_PLAIN, 2>(P, s);
         if (epi == GM_RESIDUAL) return md_launch<GM_RESIDUAL, 2>(P, s);
         return md_launch<GM_GLU, 2>(P, s);
+    }
+    if (force_ta ? force_ta == 8 : md_wide(P, epi)) {
+        if (epi == GM_PLAIN) return md_launch<GM_PLAIN, 8>(P, s);
+        if (epi == GM_RESIDUAL) return md_launch<GM_RESIDUAL, 8>(P, s);
+        return md_launch<GM_GLU, 8>(P, s);
     }
     if (epi == GM_PLAIN) return md_launch<GM_PLAIN, 4>(P, s);
     if (epi == GM_RESIDUAL) return md_launch<GM_RESIDUAL, 4>(P, s);

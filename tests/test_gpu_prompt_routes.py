@@ -174,11 +174,12 @@ def test_products_that_stream_their_weights_over_few_rows_agree_with_the_others(
     wk.close()
 
 
-@pytest.mark.parametrize("T", [193, 257, 385])
+@pytest.mark.parametrize("T", [193, 257, 385, 2048, 2600])
 @pytest.mark.parametrize("wd,shape", [(dt.Q4_B32T1A, {}), (dt.Q3H_B64T1, dict(dim=1024, heads=16, kv_heads=2, head_dim=64, ffn=1408)), (dt.Q4_B32T1B, dict(dim=2176, heads=9, kv_heads=3, ffn=3712))],
                          ids=["q4a", "q3h", "q4b"])
 def test_products_whose_steps_run_into_each_other_agree_with_the_large_tiles(wd, shape, T):
-    """rows that fill no tile, numbers of 64-column steps with every remainder by the ring's four stages (16, 22, 34, 58 steps, whole and in parts), biases everywhere"""
+    """rows that fill no tile, numbers of 64-column steps with every remainder by the ring's four stages (16, 22, 34, 58 steps, whole and in parts), biases everywhere; 256-token
+    tiles (three quarters of a tile a compute unit and more, fewer rounds) for wq | wk | wv of 385 and 2048 rows, wo / w2 of 2048 (q4a), the gated pair of 2600 (q3h) and of 2048 (q4b)"""
     wk, s = _biased(dt.F16, wd, T, **shape)
     toks = np.random.default_rng(T).integers(3, s["vocab"], T).astype(np.int32)
     out = []
