@@ -1074,8 +1074,8 @@ int run_parallel_prompt(ifa_model *m, LLayer &L, size_t T, int nseq, bool *done,
     if (lin) parts[np++] = {L.T(IFA_LT_A_O).data, AQ, ls1, nullptr, sp.a_out_scale};
     parts[np++] = {L.T(lin ? IFA_LT_L_O : IFA_LT_D_O).data, MV, ls1, nullptr, lin ? sp.l_out_scale : 1.0f};
     if (F) parts[np++] = {L.T(IFA_LT_FFN_DOWN).data, F, L.T(IFA_LT_LS2).data, L.T(IFA_LT_FFN_DOWN_B).data, 1.0f};
-    const int planes = W % 4 == 0 ? ifa_linear_bf16_sum_plane_count(W, ld, T) : 0;
-    if (planes && (rc = ensure_halfs(m, n->planes, n->planes_cap, (size_t)planes * T * W))) return rc;
+    int planes = W % 4 == 0 ? ifa_linear_bf16_sum_plane_count(W, ld, T) : 0;
+    if (planes && ensure_halfs(m, n->planes, n->planes_cap, (size_t)planes * T * W) != IFA_OK) { (void)hipGetLastError(); planes = 0; }          // (no memory for them: a workgroup a tile)
     if ((rc = ifa_linear_bf16_sum_planes(parts, np, W, n->a16, ld, T, n->x, W, planes ? n->planes : nullptr, s))) return rc;
     *pending = planes;
     return IFA_OK;
