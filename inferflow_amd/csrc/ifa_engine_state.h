@@ -209,7 +209,7 @@ struct ifa_model {
     // (7 products + 4 element-wise launches), 40 tokens the same (profiles/r05_prompt_lengths.log)
     int opt_prefill_big_min = 47;
     int opt_prefill_chunk = 1;      // prompts of 34..48 tokens as two passes of <= 32 tokens (ifa_model_forward)
-    // round 6: prompts of 33 .. prefill_mid_max tokens take the four launches per layer from k_gemm_mid (ifa_gemm_mid.hip: ring of
+    // prompts of 33 .. prefill_mid_max tokens take the four launches per layer from k_gemm_mid (ifa_gemm_mid.hip: ring of
     // direct-to-LDS stages requested by loader waves, weights dequantised into the MFMA operand registers) when every linear has its
     // operand-order copy.  A layer's four products, Llama-2-7B, us, through the large tiles (wo / w2 of up to 2048 tokens already through k_gemm_mid) and here:
     // 800 tokens 462 and 399, 1024 484 and 437, 1300 780 and 645, 1536 785 and 687, 2048 878 and 837, 3000 1362 and 1266, 4096 1642 and 1591, 6000 2622 and 2377, 8192 3161 and 3156

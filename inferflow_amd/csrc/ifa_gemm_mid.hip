@@ -5,7 +5,7 @@
 // base)) -- the reference's dequantised half -- products accumulate in fp32 in ascending 16-column groups of this workgroup's K
 // range, parts of K added in order, one F16 rounding, bias / residual / gate as half operations (k_gemm_big's arithmetic).
 //
-// Why a second kernel (round 6).  k_gemm_big stages the activation tile with direct-to-LDS loads and reads its MFMA operands with
+// Why a second kernel.  k_gemm_big stages the activation tile with direct-to-LDS loads and reads its MFMA operands with
 // ordinary LDS loads; hipcc puts `s_waitcnt vmcnt(0)` in front of every LDS read that follows a direct-to-LDS request, so every
 // 64-column step ends up waiting for the requests it has just issued: a step is one memory round trip (~1 us; rocprofv3 at 128
 // tokens: W1|W3 62 us for 64 steps, wq|wk|wv 35 us for 16) however little it multiplies.  Above ~512 tokens the step's MFMA work
