@@ -173,7 +173,7 @@ bool prefill_mid_ok(ifa_model *m, int T, bool any_length)
     if (ensure_mo(m) != IFA_OK) return false;
     for (int l = 0; l < c.layers; l++) {
         const int ids[] = {T_WQ, T_WK, T_WV, T_WO, T_W1, T_W3, T_W2};
-        for (int id : ids) { const Tensor &t = m->layers[(size_t)l].t[id]; if (!t.present() || !t.mo || t.cols % 128 != 0 || t.rows % 16 != 0) return false; }
+        for (int id : ids) { const Tensor &t = m->layers[(size_t)l].t[id]; if (!t.present() || !t.mo || t.cols % 128 != 0 || t.cols < MID_MIN_COLS || t.rows % 16 != 0) return false; }
     }
     return true;
 }

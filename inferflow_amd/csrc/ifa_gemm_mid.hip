@@ -419,7 +419,7 @@ static int md_num_cus()
 bool gemm_mid_ok(int w_dtype, const GmArgs &P, int epi)
 {
     (void)w_dtype;      // (any format the MO copy holds: 4-bit codes with value q * scale + base per 32 weights)
-    if (!P.mo || P.T < 1 || P.nsets < 1 || P.nsets > 3 || P.nblk < 8 || P.nblk % 4 != 0) return false;
+    if (!P.mo || P.T < 1 || P.nsets < 1 || P.nsets > 3 || P.nblk * 32 < (int)MID_MIN_COLS || P.nblk % 4 != 0) return false;
     for (int i = 0; i < P.nsets; i++) if (P.rows[i] % 16 != 0) return false;
     if (epi == GM_GLU && (P.nsets != 1 || !P.W1 || P.rows[0] % 8 != 0)) return false;
     for (int i = 0; i < P.nsets; i++) if (P.rows[i] % 8 != 0) return false;

@@ -192,6 +192,20 @@ def test_products_whose_steps_run_into_each_other_agree_with_the_large_tiles(wd,
     wk.close()
 
 
+@pytest.mark.parametrize("T", [33, 64, 200, 800, 2100])
+@pytest.mark.parametrize("shape", [dict(dim=512, heads=2, kv_heads=2, head_dim=64, ffn=1024), dict(dim=512, heads=8, kv_heads=4, head_dim=64, ffn=128)], ids=["wo", "w2"])
+def test_prompts_of_models_with_a_matrix_of_128_columns(shape, T):
+    """two steps of 64 columns are fewer than k_gemm_mid takes: such models keep the large tiles at every length, as against the op-by-op layer"""
+    wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=2112, layers=2, vocab=600, quant_threshold=0, **shape)
+    toks, out = np.random.default_rng(T).integers(3, s["vocab"], T).astype(np.int32), []
+    for v in (1, 0):
+        wk.set_option("prefill_big", v)
+        out.append(_rows(wk, toks, s["vocab"])[1])
+    ok, why = _agree(*out)
+    assert ok, why
+    wk.close()
+
+
 @pytest.mark.parametrize("n", [9, 16, 17, 32])
 @pytest.mark.parametrize("kvd", [dt.F16, dt.Q8_B32T2], ids=["f16", "q8"])
 def test_batched_steps_of_many_queries_agree_with_the_rows_products_and_replay(kvd, n):
