@@ -59,6 +59,8 @@ size_t gemm_rows_mo_bytes(size_t rows, size_t cols);
 // 32-weight halves: the kernel then runs unchanged; cols % 128 == 0)
 int gemm_rows_mo_build(int dtype, const void *tiled, size_t rows, size_t cols, void *mo, hipStream_t s);
 
+extern "C" int ifa_gemm_rows_offsets_fit(size_t rows, size_t cols, int mo);
+
 // rows of 16 per set when nsets > 1, cols % 128 == 0, 2 <= T <= 8; norm == 1 needs cols <= 4096
 // the per-stream scratch of the K-parts launches exists (call before capturing a step that may use them)
 int gemm_rows_kparts_reserve(hipStream_t s);

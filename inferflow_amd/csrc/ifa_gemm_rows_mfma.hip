@@ -150,14 +150,19 @@ static int gm_launch1(int wgs, size_t smem, const GmArgs &P, int epi, int norm, 
     return gm_launch2<MT, 16>(wgs, smem, P, epi, norm, s);
 }
 
+// the kernels' byte offsets inside a matrix have 32 bits (tiled rows: 20 bytes a block and padding; operand-order copies: whole tiles)
+extern "C" int ifa_gemm_rows_offsets_fit(size_t rows, size_t cols, int mo)
+{
+    return (mo ? gemm_rows_mo_bytes(rows, cols) : (rows + 16) * (cols / 32 + 16) * 20) < ((size_t)1 << 32);
+}
+
 bool gemm_rows_mfma_fused_ok(const GmArgs &P, int epi, int norm)
 {
     if (P.T < 2 || P.T > (P.mo ? 32 : 16) || P.nblk <= 0 || P.nblk % 4 != 0 || P.nsets < 1 || P.nsets > 3) return false;      // (17..32 rows: MO layout only)
     if (norm == 1 && (P.nblk * 32 > GmGeo<32>::CHUNK_COLS || P.T > (P.mo ? 16 : 8))) return false;      // the norm prologue: whole rows in one chunk (tiled layout: <= 8 rows)
     if (epi == GM_GLU && (P.nsets != 1 || !P.W1)) return false;
     for (int i = 0; i < P.nsets; i++) if (P.rows[i] <= 0 || (P.nsets > 1 && P.rows[i] % 16 != 0)) return false;
-    for (int i = 0; i < P.nsets; i++)      // 32-bit byte offsets inside a matrix (tiled and MO copies are 20 bytes per block + padding)
-        if (((size_t)P.rows[i] + 16) * ((size_t)P.nblk + 16) * 20 >= ((size_t)1 << 32)) return false;
+    for (int i = 0; i < P.nsets; i++) if (!ifa_gemm_rows_offsets_fit((size_t)P.rows[i], (size_t)P.nblk * 32, P.mo)) return false;
     return true;
 }
 
