@@ -178,12 +178,12 @@ bool prefill_mid_ok(ifa_model *m, int T, bool any_length)
     return true;
 }
 
-// FEW_MIN .. FEW_MAX rows through gemm_few: dense layers with the sequential RMS wiring, every linear with its operand-order copy (built here on first use, like the workspace, whose
+// FEW_MIN .. few_max_rows rows through gemm_few: dense layers with the sequential RMS wiring, every linear with its operand-order copy (built here on first use, like the workspace, whose
 // addresses captured steps hold: one size for every number of rows)
 bool rows_few_ok(ifa_model *m, int T)
 {
     const ifa_model_config &c = m->cfg;
-    if (!m->opt_rows_few || !m->opt_rows_mo || T < FEW_MIN || T > FEW_MAX || c.experts != 0 || c.norm_kind != 0 || c.dim > 8192 || !prefill_big_ok(m)) return false;
+    if (!m->opt_rows_few || !m->opt_rows_mo || T < FEW_MIN || T > few_max_rows((size_t)c.dim, (size_t)c.ffn) || c.experts != 0 || c.norm_kind != 0 || c.dim > 8192 || !prefill_big_ok(m)) return false;
     const size_t D = c.dim, QD = (size_t)c.heads * c.head_dim, KVD = (size_t)c.kv_heads * c.head_dim, F = c.ffn;
     if (!few_ok(QD, D) || !few_ok(KVD, D) || !few_ok(D, QD) || !few_ok(F, D) || !few_ok(D, F) || ensure_mo(m) != IFA_OK) return false;
     for (const Layer &L : m->layers) {
@@ -191,7 +191,8 @@ bool rows_few_ok(ifa_model *m, int T)
         for (int id : ids) if (!L.t[id].present() || !L.t[id].mo) return false;
     }
     if (!m->few.x) {
-        const size_t nx = few_frag_bytes(FEW_MAX, D), nf = few_frag_bytes(FEW_MAX, F), ns = (size_t)FEW_PARTS * FEW_MAX * D * sizeof(float);
+        const int most = few_max_rows(D, F);
+        const size_t nx = few_frag_bytes(most, D), nf = few_frag_bytes(most, F), ns = (size_t)FEW_PARTS * most * D * sizeof(float);
         char *p = nullptr;
         if (hipMalloc((void **)&p, nx + nf + ns) != hipSuccess) { (void)hipGetLastError(); m->opt_rows_few = 0; return false; }
         m->few = {(half_t *)p, (half_t *)(p + nx), (float *)(p + nx + nf)};
@@ -285,7 +286,7 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
     // weights dequantised once per workgroup and step into LDS; reference-layout rows), norms as their own launches.
     // the mid-length kernel (33 .. prefill_mid_max tokens): every linear of every layer a 4-bit tensor with its operand-order copy, dense FFN
     const bool pstat = m->opt_perf_stat != 0;       // per-phase times: the op-by-op layer below (one launch per reference op), never the fused routes
-    const bool pf_few = !tp && !pstat && (T <= 32 ? m->opt_batch_fused : m->opt_prefill_mid) && rows_few_ok(m, T);      // (FEW_MIN .. FEW_MAX tokens: gemm_few)
+    const bool pf_few = !tp && !pstat && (T <= 32 ? m->opt_batch_fused : m->opt_prefill_mid) && rows_few_ok(m, T);      // (FEW_MIN .. few_max_rows tokens: gemm_few)
     const bool pf_mid = !pf_few && !tp && !pstat && prefill_mid_ok(m, T, false);
     const bool pf_big = pf_few || pf_mid || (!tp && !pstat && T > std::max(32, m->opt_prefill_big_min) && prefill_big_ok(m));
     bool pf_fused = pf_big || (!tp && !pstat && T >= 2 && T <= 32 && batch_fused_ok(m, T) && c.experts == 0);

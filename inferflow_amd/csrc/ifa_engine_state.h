@@ -215,7 +215,7 @@ struct ifa_model {
     // 800 tokens 462 and 399, 1024 484 and 437, 1300 780 and 645, 1536 785 and 687, 2048 878 and 837, 3000 1362 and 1266, 4096 1642 and 1591, 6000 2622 and 2377, 8192 3161 and 3156
     int opt_prefill_mid = 1, opt_prefill_mid_max = 8192;
     int opt_prefill_res_mid = 2048;   // prefill_mid_max + 1 .. this many tokens (where prefill_mid_max was lowered): wo / w2 still through k_gemm_mid, the other products through the large tiles (0: never)
-    // prompts of FEW_MIN .. FEW_MAX tokens and steps of as many queries through gemm_few (ifa_gemm_few.hip); its workspace, one allocation: rows in fragment order (a layer's
+    // prompts of FEW_MIN .. few_max_rows tokens and steps of as many queries through gemm_few (ifa_gemm_few.hip); its workspace, one allocation: rows in fragment order (a layer's
     // input, the gated pair's output), sums of the parts of K
     int opt_rows_few = 1;
     struct { half_t *x, *ff; float *sums; } few = {nullptr, nullptr, nullptr};

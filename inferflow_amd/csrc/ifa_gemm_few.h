@@ -4,7 +4,7 @@
 
 namespace ifa {
 
-constexpr int FEW_MIN = 9, FEW_MAX = 192;       // rows
+constexpr int FEW_MIN = 9, FEW_MAX = 192;       // rows (few_max_rows: of a model's layers)
 constexpr int FEW_PARTS = 8;                    // parts of K at the most
 
 // Rows in FRAGMENT ORDER ([K / 128][tiles of 16 rows][4][64 lanes][8 halves]): lane 16 g + r of piece s holds columns 128 S + 32 g + 8 s .. + 7 of row
@@ -28,6 +28,7 @@ struct FewArgs {
 };
 enum FewOut { FEW_ROWS, FEW_GLU, FEW_SUMS };
 bool few_ok(size_t rows, size_t cols);                       // a matrix that these launches take
+int few_max_rows(size_t dim, size_t ffn);                    // up to how many rows a layer of these sizes goes this way
 int few_parts(size_t rows, size_t cols);                     // FEW_SUMS: parts of K of such a matrix
 int gemm_few(const FewArgs &P, FewOut out, hipStream_t s);
 // x_out[t] = res[t] + half(sum of the parts' rows, in order) (+ bias), parts = 0: x_out not written, res[t]; y (nullable) = its RMS norm in fragment order

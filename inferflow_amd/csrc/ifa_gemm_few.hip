@@ -228,6 +228,15 @@ bool few_ok(size_t rows, size_t cols)
     return rows > 0 && rows % 16 == 0 && rows < (1u << 24) && cols >= 1024 && cols % 128 == 0 && cols <= 65536;
 }
 
+int few_max_rows(size_t dim, size_t ffn)
+{
+    // Every workgroup fetches all rows of its range of K: behind 96 rows of wide models k_gemm_mid's 128-token tiles are faster.  Four layers, us, k_gemm_mid / here, 64, 96, 128, 160, 192 rows:
+    // 4096 x 11008 431, 513, 528, 694, 698 / 379, 470, 514, 633, 664; 4096 x 14336 432, 523, 529, 717, 719 / 415, 521, 584, 723, 754; 5120 x 13824 502, 619, 630, 915, 919 / 498, 633, 708, 908, 961;
+    // 6144 x 16384 546, 677, 687, 1039, 1049 / 556, 738, 828, 1085, 1145; 8192 x 28672 851, 1153, 1171, 1932, 1948 / 886, 1246, 1412, 1963, 2074; narrower ones as the first, 0.75 to 0.97 (3072 x 8192 of
+    // 144 to 192 rows 1.02 to 1.08)
+    return dim * ffn <= (size_t)4096 * 12288 ? FEW_MAX : 96;
+}
+
 // tiles of a workgroup where parts of K are summed
 static int few_sum_tiles(size_t rows) { return rows >= 16 * 256 ? 4 : 2; }
 
@@ -248,11 +257,14 @@ int gemm_few(const FewArgs &A, FewOut out, hipStream_t s)
     for (int i = 0; i < A.nsets && ok; i++) { ok = A.W[i] && few_ok((size_t)A.rows[i], (size_t)A.K) && (out == FEW_SUMS || A.Y[i]) && (out != FEW_ROWS || A.ldy[i] % 4 == 0); P.tiles += A.rows[i] / 16; }
     if (!ok || (out == FEW_GLU && (!A.W1 || A.rows[0] % 128 != 0)) || (out == FEW_SUMS ? A.ldx % 8 != 0 || (A.ldx && A.ldx < A.K) : A.ldx != 0))
         return ifa_fail(IFA_ERR_ARG, "rows of a prompt: shape not covered (%d rows, %d x %d)", A.T, A.rows[0], A.K);
-    // the tiles a workgroup takes: the fewest rounds of the 256 compute units times tiles, the larger of two that are alike (it reads the rows less often)
+    // the tiles a workgroup takes: the least rounds of the 256 compute units times what a workgroup fetches, its weights (a pair's 24 bytes a column, at a compute unit's share of
+    // the memory's rate) and its rows (at its share of the L2s').  By rounds of weights alone the pairs of 28672 outputs went one to a workgroup, each with all the rows: a layer of width 8192, 64, 128
+    // rows 258, 414 us, so 222, 353; of width 7168 and 20480 outputs 194, 304, so 167, 262; up to 4096 x 14336 the choices are the same.
+    const double rows_of = 0.0234 * 16 * P.x_tiles * (out == FEW_GLU ? 1 : 2);
     auto choose = [&](std::initializer_list<int> sizes) {
-        int best = 0; long cost = 0;
+        int best = 0; double cost = 0;
         for (int n : sizes) {
-            const long c = (((long)P.tiles + n - 1) / n + 255) / 256 * n;
+            const double c = (((long)P.tiles + n - 1) / n + 255) / 256 * (n + rows_of);
             if (!best || c <= cost) { best = n; cost = c; }
         }
         return best;

@@ -174,6 +174,21 @@ def test_products_that_stream_their_weights_over_few_rows_agree_with_the_others(
     wk.close()
 
 
+@pytest.mark.parametrize("ffn,most", [(12288, 192), (12416, 96)])
+def test_where_wide_models_leave_the_products_over_few_rows(ffn, most):
+    """gemm_few sums K in another order, so its rows differ from the other route's in some bits, up to its last row count and no further"""
+    wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=208, layers=1, vocab=600, ffn=ffn)
+    toks = np.random.default_rng(ffn).integers(3, s["vocab"], 193).astype(np.int32)
+    for T, same in ((most, False), (most + 1, True)):
+        out = []
+        for v in (1, 0):
+            wk.set_option("rows_few", v)
+            out.append(_rows(wk, toks[:T], s["vocab"])[1])
+        ok, why = _agree(*out)
+        assert ok and np.array_equal(*out) == same, (T, why)
+    wk.close()
+
+
 @pytest.mark.parametrize("T", [193, 257, 385, 2048, 2600])
 @pytest.mark.parametrize("wd,shape", [(dt.Q4_B32T1A, {}), (dt.Q3H_B64T1, dict(dim=1024, heads=16, kv_heads=2, head_dim=64, ffn=1408)), (dt.Q4_B32T1B, dict(dim=2176, heads=9, kv_heads=3, ffn=3712))],
                          ids=["q4a", "q3h", "q4b"])
