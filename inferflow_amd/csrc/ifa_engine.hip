@@ -140,30 +140,60 @@ void *kv_ptr(ifa_model *m, size_t layer, int slot, bool is_v)
     return is_v ? sl.v[layer] : sl.k[layer];
 }
 
-// (a failed allocation -- the copies are 4.3 GB for Llama-2-7B Q4 -- is not an error of the step that triggered it: every partial
-//  copy is dropped, opt_rows_mo goes off and the tiled kernels (<= 16 rows per launch) serve the batched steps)
-int ensure_mo(ifa_model *m)
+static void free_mo(ifa_model *m)
 {
-    if (!m->opt_rows_mo) return IFA_OK;
-    // (option "debug_mo_alloc_fail": the build reports an allocation failure after its first copy -- the tests' way to walk the downgrade)
-    const int rc = ensure_mo_build(m);
-    if (rc == IFA_OK) return IFA_OK;
-    (void)hipGetLastError();
+    m->mo_built = false;
     for (Layer &L : m->layers) {
         for (Tensor &t : L.t) if (t.mo) { (void)hipFree(t.mo); t.mo = nullptr; }
         for (Tensor &t : L.experts) if (t.mo) { (void)hipFree(t.mo); t.mo = nullptr; }
         if (L.moe_table_mo) { (void)hipFree(L.moe_table_mo); L.moe_table_mo = nullptr; }
     }
-    m->opt_rows_mo = 0;
     drop_graphs(m);
+}
+
+// the copies' kind: with the words by supersteps where prompts of such a model go through gemm_few and gemm_mid (whatever the options, which may change), and where the rows products'
+// offsets reach them
+static int mo_kind(const ifa_model *m)
+{
+    if (m->mo_no_words || m->cfg.experts > 0 || m->cfg.tp_size > 1 || !prefill_big_layers(m)) return MO_QUADS;
+    for (const Layer &L : m->layers) {
+        const int ids[] = {T_WQ, T_WK, T_WV, T_WO, T_W1, T_W3, T_W2};
+        for (int id : ids) {
+            const Tensor &t = L.t[id];
+            if (!t.tiled || t.cols % 128 != 0 || t.cols < MID_MIN_COLS || t.rows % 16 != 0 || !ifa_gemm_rows_offsets_fit(t.rows, t.cols, MO_WORDS)) return MO_QUADS;
+        }
+    }
+    return MO_WORDS;
+}
+
+// (a failed allocation -- the copies are 4.1 GB for Llama-2-7B Q4, 4.9 with the words by supersteps -- is not an error of the step that triggered it: every partial
+//  copy is dropped, and there are copies without these words, which the rows products read, or, if there is no room for them either, opt_rows_mo goes off and the tiled kernels
+//  (<= 16 rows per launch) serve the batched steps)
+int ensure_mo(ifa_model *m)
+{
+    if (!m->opt_rows_mo || m->mo_built) return IFA_OK;
+    // (option "debug_mo_alloc_fail": the build reports an allocation failure after its first copy -- the tests' way to walk the downgrade)
+    const int kind = mo_kind(m);
+    if (ensure_mo_build(m, kind) == IFA_OK) return IFA_OK;
+    (void)hipGetLastError();
+    free_mo(m);
+    if (kind == MO_WORDS) {
+        m->mo_no_words = true;
+        if (ensure_mo_build(m, MO_QUADS) == IFA_OK) return IFA_OK;
+        (void)hipGetLastError();
+        free_mo(m);
+    }
+    m->opt_rows_mo = 0;
     fprintf(stderr, "inferflow_amd: the rows GEMM's operand-order weight copies could not be built (%s); batched steps use the tiled kernels\n", ifa_last_error());
     return IFA_OK;
 }
 
-int ensure_mo_build(ifa_model *m)
+int ensure_mo_build(ifa_model *m, int kind)
 {
     const ifa_model_config &c = m->cfg;
-    bool built = false;
+    bool built = false, other = false;
+    for (const Layer &L : m->layers) for (const Tensor &t : L.t) other = other || (t.mo && t.mo_kind != kind);
+    if (other) { IFA_HIP_CHECK(hipStreamSynchronize(m->stream)); free_mo(m); }          // (a matrix was replaced since)
     for (Layer &L : m->layers) {
         const bool moe = c.experts > 0 && L.t[T_MOE_GATE].present();
         const int ids[] = {T_WQ, T_WK, T_WV, T_WO, T_W1, T_W3, T_W2};
@@ -171,9 +201,10 @@ int ensure_mo_build(ifa_model *m)
             Tensor &t = L.t[id];
             if (moe && (id == T_W1 || id == T_W3 || id == T_W2)) continue;
             if (t.mo || !t.present() || !t.tiled || !rows_mo_fmt(t.dtype) || t.cols % 128 != 0) continue;
-            if (m->opt_debug_mo_alloc_fail && built) return ifa_fail(IFA_ERR_HIP, "hipMalloc: out of memory (simulated: debug_mo_alloc_fail)");
-            IFA_HIP_CHECK(hipMalloc(&t.mo, gemm_rows_mo_bytes(t.rows, t.cols)));
-            int rc = gemm_rows_mo_build(t.dtype, t.tiled, t.rows, t.cols, t.mo, m->stream);
+            if (built && (m->opt_debug_mo_alloc_fail == 1 || (m->opt_debug_mo_alloc_fail == 2 && kind == MO_WORDS))) return ifa_fail(IFA_ERR_HIP, "hipMalloc: out of memory (simulated: debug_mo_alloc_fail)");
+            IFA_HIP_CHECK(hipMalloc(&t.mo, gemm_rows_mo_bytes(t.rows, t.cols, kind)));
+            t.mo_kind = kind;
+            int rc = gemm_rows_mo_build(t.dtype, t.tiled, t.rows, t.cols, kind, t.mo, m->stream);
             if (rc) return rc;
             built = true;
         }
@@ -191,8 +222,9 @@ int ensure_mo_build(ifa_model *m)
             for (int k = 0; k < 3; k++) {
                 Tensor &t = L.experts[(size_t)e * 3 + order[k]];
                 if (!t.mo) {
-                    IFA_HIP_CHECK(hipMalloc(&t.mo, gemm_rows_mo_bytes(t.rows, t.cols)));
-                    int rc = gemm_rows_mo_build(t.dtype, t.tiled, t.rows, t.cols, t.mo, m->stream);
+                    IFA_HIP_CHECK(hipMalloc(&t.mo, gemm_rows_mo_bytes(t.rows, t.cols, kind)));
+                    t.mo_kind = kind;
+                    int rc = gemm_rows_mo_build(t.dtype, t.tiled, t.rows, t.cols, kind, t.mo, m->stream);
                     if (rc) return rc;
                     built = true;
                 }
@@ -203,6 +235,7 @@ int ensure_mo_build(ifa_model *m)
         IFA_HIP_CHECK(hipMemcpy(L.moe_table_mo, tab.data(), tab.size() * sizeof(void *), hipMemcpyHostToDevice));
     }
     if (built) IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
+    m->mo_built = true;
     return IFA_OK;
 }
 
@@ -393,6 +426,7 @@ int ifa_model_set_tensor(ifa_model *m, int layer, int tensor_id, int expert, int
         } else t = &L.t[tensor_id];
     }
     free_tensor(*t);
+    m->mo_built = false;
     if (expert >= 0) {      // the layer's table of MO copies points into the copy just freed: ensure_mo rebuilds it
         Layer &Lx = m->layers[(size_t)layer];
         if (Lx.moe_table_mo) { (void)hipFree(Lx.moe_table_mo); Lx.moe_table_mo = nullptr; }
@@ -640,6 +674,10 @@ int ifa_model_get_buffer(ifa_model *m, const char *name, int layer, void **dptr,
         IFA_REQUIRE(layer >= 0 && layer < c.layers && m->finalized, "ifa_model_get_buffer: layer %d", layer);
         p = name[0] == 'k' ? m->layers[(size_t)layer].kcache : m->layers[(size_t)layer].vcache;
         b = m->kv_row_bytes * (size_t)c.max_ctx;
+    } else if (!strcmp(name, "rows_copy")) {          // the layer's wq in operand order, once there is such a copy
+        IFA_REQUIRE(layer >= 0 && layer < c.layers, "ifa_model_get_buffer: layer %d", layer);
+        const Tensor &t = m->layers[(size_t)layer].t[T_WQ];
+        p = t.mo; b = t.mo ? gemm_rows_mo_bytes(t.rows, t.cols, t.mo_kind) : 0;
     } else return ifa_fail(IFA_ERR_ARG, "ifa_model_get_buffer: unknown buffer '%s'", name);
     *dptr = p;
     if (bytes) *bytes = b;

@@ -173,7 +173,7 @@ bool prefill_mid_ok(ifa_model *m, int T, bool any_length)
     if (ensure_mo(m) != IFA_OK) return false;
     for (int l = 0; l < c.layers; l++) {
         const int ids[] = {T_WQ, T_WK, T_WV, T_WO, T_W1, T_W3, T_W2};
-        for (int id : ids) { const Tensor &t = m->layers[(size_t)l].t[id]; if (!t.present() || !t.mo || t.cols % 128 != 0 || t.cols < MID_MIN_COLS || t.rows % 16 != 0) return false; }
+        for (int id : ids) { const Tensor &t = m->layers[(size_t)l].t[id]; if (rows_mo(m, t) != MO_WORDS) return false; }
     }
     return true;
 }
@@ -188,7 +188,7 @@ bool rows_few_ok(ifa_model *m, int T)
     if (!few_ok(QD, D) || !few_ok(KVD, D) || !few_ok(D, QD) || !few_ok(F, D) || !few_ok(D, F) || ensure_mo(m) != IFA_OK) return false;
     for (const Layer &L : m->layers) {
         const int ids[] = {T_WQ, T_WK, T_WV, T_WO, T_W1, T_W3, T_W2};
-        for (int id : ids) if (!L.t[id].present() || !L.t[id].mo) return false;
+        for (int id : ids) if (rows_mo(m, L.t[id]) != MO_WORDS) return false;
     }
     if (!m->few.x) {
         const int most = few_max_rows(D, F);
@@ -304,7 +304,7 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
         const size_t F = c.ffn;
         const bool norm_fused = !pf_big && (T <= 8 || rows_mo(m, L.t[T_WQ])) && T <= 16;
         auto wp = [&](int id) { return pf_mid ? (const uint8_t *)L.t[id].mo : (pf_big ? (const uint8_t *)(L.t[id].x32 ? L.t[id].x32 : L.t[id].data) : rows_w(m, L.t[id])); };
-        const int mo_flag = pf_mid ? 1 : (pf_big ? 0 : rows_mo(m, L.t[T_WQ]));
+        const int mo_flag = pf_mid ? (int)MO_WORDS : (pf_big ? 0 : rows_mo(m, L.t[T_WQ]));
         auto lin = [&](const GmArgs &A, int id, int epi, int norm) {
             if (pf_mid && gemm_mid_ok(L.t[id].dtype, A, epi)) return gemm_mid(A, epi, m->stream);
             if (pf_mid) return ifa_fail(IFA_ERR_STATE, "mid-length GEMM declined a product of layer tensor %d", id);
@@ -357,7 +357,7 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
         P.W[0] = wp(T_WO); P.rows[0] = (int)D; P.nsets = 1; P.nblk = (int)(QD / 32);
         P.X = m->att; P.ldx = (int)QD; P.bias[0] = (const half_t *)L.t[T_WO_B].data;
         P.Y = m->a; P.ldy = (int)D; P.res = x; P.ldres = (int)D;
-        if (pf_res_mid) { P.W[0] = (const uint8_t *)L.t[T_WO].mo; P.mo = 1; P.no_waits = !m->opt_rows_kparts; }
+        if (pf_res_mid) { P.W[0] = (const uint8_t *)L.t[T_WO].mo; P.mo = MO_WORDS; P.no_waits = !m->opt_rows_kparts; }
         if (pf_res_mid && gemm_mid_ok(L.t[T_WO].dtype, P, GM_RESIDUAL)) { if ((rc = gemm_mid(P, GM_RESIDUAL, m->stream))) return rc; }
         else { if (pf_res_mid) { P.W[0] = wp(T_WO); P.mo = mo_flag; } if ((rc = lin(P, T_WO, GM_RESIDUAL, 0))) return rc; }
         clear();
@@ -379,7 +379,7 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
         P.W[0] = wp(T_W2); P.rows[0] = (int)D; P.nsets = 1; P.nblk = (int)(F / 32);
         P.X = m->t1; P.ldx = (int)F; P.bias[0] = (const half_t *)L.t[T_W2_B].data;
         P.Y = m->f; P.ldy = (int)D; P.res = m->a; P.ldres = (int)D;
-        if (pf_res_mid) { P.W[0] = (const uint8_t *)L.t[T_W2].mo; P.mo = 1; P.no_waits = !m->opt_rows_kparts; }
+        if (pf_res_mid) { P.W[0] = (const uint8_t *)L.t[T_W2].mo; P.mo = MO_WORDS; P.no_waits = !m->opt_rows_kparts; }
         if (pf_res_mid && gemm_mid_ok(L.t[T_W2].dtype, P, GM_RESIDUAL)) { if ((rc = gemm_mid(P, GM_RESIDUAL, m->stream))) return rc; }
         else { if (pf_res_mid) { P.W[0] = wp(T_W2); P.mo = mo_flag; } if ((rc = lin(P, T_W2, GM_RESIDUAL, 0))) return rc; }
         std::swap(m->x, m->f);
@@ -555,10 +555,12 @@ bool batch_fused_ok(const ifa_model *m, int n)
 
 // prompts above `prefill_big_min` tokens as four launches of the large-tile GEMM per layer (forward_ops, pf_big): dense layers with the
 // sequential wiring, every linear a 20-byte-block Q4 tensor (wq / wk / wv of one format), dims in multiples of 64
-bool prefill_big_ok(const ifa_model *m)
+bool prefill_big_ok(const ifa_model *m) { return m->opt_prefill_big && !m->topo && prefill_big_layers(m); }
+
+bool prefill_big_layers(const ifa_model *m)
 {
     const ifa_model_config &c = m->cfg;
-    if (!m->opt_prefill_big || m->topo || c.parallel_attn || c.share_input || has_post_norms(m)) return false;
+    if (c.parallel_attn || c.share_input || has_post_norms(m)) return false;
     if (scale_on(c.attn_out_scale) || scale_on(c.ffn_out_scale)) return false;
     const size_t D = c.dim, QD = (size_t)c.heads * c.head_dim, F = c.ffn;
     if (D % 64 || QD % 64 || F % 64) return false;

@@ -45,6 +45,7 @@ struct Tensor {
     void *data = nullptr;    // reference layout (AoS blocks / F16), engine-owned
     void *tiled = nullptr;   // row-local plane layout for the fused kernels (or null)
     void *mo = nullptr;      // MFMA-operand-order copy for the small-batch rows GEMM (ifa_gemm_rows_mfma.h), built on first use
+    int mo_kind = 0;         // MO_QUADS | MO_WORDS, the same for all of a model's copies
     void *q3hn = nullptr;    // Q3H_B64T1: the values at the format's native 32 bytes per block for the decode GEMVs (option q3h_native, built on first use)
     void *x32 = nullptr;     // 64-weight nibble formats: the same values as Q4_B32T1A reference-layout blocks, for the large-tile prefill GEMM
     size_t rows = 0, cols = 0;
@@ -220,7 +221,8 @@ struct ifa_model {
     int opt_rows_few = 1;
     struct { half_t *x, *ff; float *sums; } few = {nullptr, nullptr, nullptr};
     int opt_rows_kparts = 1, opt_gemm_splitk = 1;   // 0: never the launches whose workgroups wait for partner workgroups (K parts of the 9..32-row GEMM, split-K halves of the large-tile GEMM)
-    int opt_debug_mo_alloc_fail = 0;           // tests: ensure_mo_build fails like an exhausted allocator after its first copy
+    int opt_debug_mo_alloc_fail = 0;           // tests: ensure_mo_build fails like an exhausted allocator after its first copy (2: of copies with MO_WORDS only)
+    bool mo_built = false, mo_no_words = false;          // every matrix that has an operand-order copy has it; there was no memory for MO_WORDS copies
     static constexpr int RING = 1024;
 };
 
@@ -299,7 +301,7 @@ extern "C" int ifa_rope_rows(void *x, int head_dim, int heads, int tokens, const
 // weight pointer of a rows-GEMM launch: the MO copy when it exists (all sets of a launch alike: ensure_mo builds all or none)
 static inline const uint8_t *rows_w(const ifa_model *m, const Tensor &t) { return (const uint8_t *)(m->opt_rows_mo && t.mo ? t.mo : t.tiled); }
 
-static inline int rows_mo(const ifa_model *m, const Tensor &t) { return m->opt_rows_mo && t.mo ? 1 : 0; }
+static inline int rows_mo(const ifa_model *m, const Tensor &t) { return m->opt_rows_mo && t.mo ? t.mo_kind : 0; }
 
 namespace ifae {
 
@@ -318,7 +320,7 @@ struct PerfSpan {
 void free_tensor(Tensor &t);
 void *kv_ptr(ifa_model *m, size_t layer, int slot, bool is_v);
 int ensure_mo(ifa_model *m);
-int ensure_mo_build(ifa_model *m);
+int ensure_mo_build(ifa_model *m, int kind);
 int ensure_x32(ifa_model *m);
 int ensure_q3hn(ifa_model *m);
 int ensure_scratch(ifa_model *m, int T);
@@ -361,6 +363,7 @@ int layer_tail_ops(ifa_model *m, int l, int T, half_t *&x, const half_t *attn_in
 int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, void *logits_out, int *next_token, bool no_head = false);
 bool batch_fused_ok(const ifa_model *m, int n);
 bool prefill_big_ok(const ifa_model *m);
+bool prefill_big_layers(const ifa_model *m);      // ... of the layers alone, whatever the options
 bool prefill_mid_ok(ifa_model *m, int T, bool any_length);
 bool rows_few_ok(ifa_model *m, int T);
 int batch_fused_layer(ifa_model *m, int l, int n, const half_t *x, half_t *xnext, const void *rows_l);

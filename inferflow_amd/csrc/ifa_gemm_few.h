@@ -13,7 +13,7 @@ constexpr int FEW_PARTS = 8;                    // parts of K at the most
 inline size_t few_frag_bytes(int rows, size_t cols) { return (size_t)((rows + 15) / 16) * 16 * cols * 2; }
 
 struct FewArgs {
-    const uint8_t *W[3];           // MO copies; up to three matrices one after the other (rows of 16 each); gated pairs: W[0] with W1
+    const uint8_t *W[3];           // MO_WORDS copies; up to three matrices one after the other (rows of 16 each); gated pairs: W[0] with W1
     const uint8_t *W1;
     int rows[3];
     int nsets, K, T;

@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(512) k_gemm_few(const FewLaunch P)
     const int s_lo = kz * nsup / P.ks, s_hi = (kz + 1) * nsup / P.ks;
     const GmSets S = {P.W[0], P.W[1], P.W[2], P.bias[0], P.bias[1], P.bias[2], P.Y[0], P.Y[1], P.Y[2], P.rows[0], P.rows[1], P.rows[2], P.nsets, P.ldy[0], P.ldy[1], P.ldy[2]};
     auto tile_of = [&](int it) { return GLU ? wg * (MT / 2) + (it >> 1) : wg * MT + it; };
-    const int mo_tile = (int)mo_tile_bytes(nsup), words = (int)mo_words_at(nsup);
+    const int mo_tile = (int)mo_tile_bytes(nsup, MO_WORDS), words = (int)mo_words_at(nsup);
     __amdgpu_buffer_rsrc_t wr[MT];
 #pragma unroll
     for (int it = 0; it < MT; it++) {

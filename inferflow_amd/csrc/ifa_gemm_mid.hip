@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(MD_THREADS, 2) k_gemm_mid(const GmArgs P, cons
     // like a decode row; the tiled rows fetched 32 bytes per row and step measured 1 TB/s: 32 DRAM pages per request).  A step is
     // half a superstep: lane -> (block l / 32 of the half, tile (l / 16) % 2, row l % 16), 2 x 512 contiguous bytes per request.
     const int nsup = nblk >> 2;
-    const size_t mo_tile = mo_tile_bytes(nsup);
+    const size_t mo_tile = mo_tile_bytes(nsup, MO_WORDS);
     __amdgpu_buffer_rsrc_t wres;
     uint32_t woff;
     {
@@ -419,7 +419,7 @@ static int md_num_cus()
 bool gemm_mid_ok(int w_dtype, const GmArgs &P, int epi)
 {
     (void)w_dtype;      // (any format the MO copy holds: 4-bit codes with value q * scale + base per 32 weights)
-    if (!P.mo || P.T < 1 || P.nsets < 1 || P.nsets > 3 || P.nblk * 32 < (int)MID_MIN_COLS || P.nblk % 4 != 0) return false;
+    if (P.mo != MO_WORDS || P.T < 1 || P.nsets < 1 || P.nsets > 3 || P.nblk * 32 < (int)MID_MIN_COLS || P.nblk % 4 != 0) return false;
     for (int i = 0; i < P.nsets; i++) if (P.rows[i] % 16 != 0) return false;
     if (epi == GM_GLU && (P.nsets != 1 || !P.W1 || P.rows[0] % 8 != 0)) return false;
     for (int i = 0; i < P.nsets; i++) if (P.rows[i] % 8 != 0) return false;

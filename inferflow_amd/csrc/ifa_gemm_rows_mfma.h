@@ -28,7 +28,7 @@ struct GmArgs {
     int act_kind;
     half_t *Yset[3];               // optional: set i written to its own matrix Yset[i][t * ldyset[i] + row] (q, k, v of a prompt)
     int ldyset[3];
-    int mo;                        // W[] / W1 are MO-layout copies (below) instead of the tiled layout
+    int mo;                        // W[] / W1 are MO-layout copies (below: MO_QUADS or MO_WORDS) instead of the tiled layout
     long long *trace;              // optional [workgroups][16] wall-clock stamps (tuning: IFA_ROWS_TRACE=1 prints a timeline per launch)
     // K parts (round 4: chunked rows of 9..32 queries, kernels instantiated with KPM > 0): kparts consecutive workgroups share a
     // group of KPM * kparts tiles; each walks its own chunks of K for ALL of them, leaves the fp32 sums of the tiles it does not
@@ -48,16 +48,17 @@ struct GmArgs {
 //   block 4 S + g of row 16 tile + r (exactly its A operands of the superstep's four MFMAs; byte b of a word of eight codes holds element b
 //   in its low and element 4 + b in its high nibble, the order in which ifa_dequant_q4.h needs no permutes), then
 //   ceil(nsup / 4) quads of 1024 bytes: lane l owns the (base, scale) words of its blocks in supersteps 4 Q .. 4 Q + 3, then
-//   the same words again by supersteps, 256 bytes each (padded to whole KiB): lane l owns bytes 4 l .. 4 l + 3.  (The kernels whose waves own four supersteps in a row read the quads,
+//   (MO_WORDS) the same words again by supersteps, 256 bytes each (padded to whole KiB): lane l owns bytes 4 l .. 4 l + 3.  (The kernels whose waves own four supersteps in a row read the quads,
 //   one request for four; those whose waves take supersteps by turns, or halves of them, fetched every line of the quads up to four times: w1 | w3 of 48 rows 22.6 -> 21.4 us.
-//   With words by supersteps only, the batched steps of 2..16 queries were 2 to 4 % slower.)
+//   With words by supersteps only, the batched steps of 2..16 queries were 2 to 4 % slower.  A fifth more memory, so only copies that k_gemm_few and k_gemm_mid read have them: mo_kind.)
 // Rows past the end and the pads are zero.
-constexpr size_t mo_tile_bytes(int nsup) { return (size_t)(nsup + 2 * ((nsup + 3) >> 2)) * 1024; }
+enum { MO_QUADS = 1, MO_WORDS = 2 };
+constexpr size_t mo_tile_bytes(int nsup, int kind) { return (size_t)(nsup + (kind == MO_WORDS ? 2 : 1) * ((nsup + 3) >> 2)) * 1024; }
 constexpr size_t mo_words_at(int nsup) { return (size_t)(nsup + ((nsup + 3) >> 2)) * 1024; }      // the words by supersteps
-size_t gemm_rows_mo_bytes(size_t rows, size_t cols);
+size_t gemm_rows_mo_bytes(size_t rows, size_t cols, int kind);
 // dtype: Q4_B32T1A / B, or the 64-weight nibble formats Q4_B64T1 / Q3H_B64T1 (one (base, scale) per 64 weights, written for both
 // 32-weight halves: the kernel then runs unchanged; cols % 128 == 0)
-int gemm_rows_mo_build(int dtype, const void *tiled, size_t rows, size_t cols, void *mo, hipStream_t s);
+int gemm_rows_mo_build(int dtype, const void *tiled, size_t rows, size_t cols, int kind, void *mo, hipStream_t s);
 
 extern "C" int ifa_gemm_rows_offsets_fit(size_t rows, size_t cols, int mo);
 

@@ -34,10 +34,10 @@ namespace ifa {
 // (ifa_tiled.h: [32 B codes] x n, [base, scale] x n per row) -- whose value is q * scale + base like Q4_B32T1: the 64-block's
 // word is written for both of its halves, and the rows GEMM runs unchanged on 32-weight blocks.
 template <bool B64>
-__global__ void __launch_bounds__(256) k_gemm_rows_mo_build(const uint8_t *__restrict__ tiled, int rows, int nblk, size_t row_bytes, uint8_t *__restrict__ mo)
+__global__ void __launch_bounds__(256) k_gemm_rows_mo_build(const uint8_t *__restrict__ tiled, int rows, int nblk, size_t row_bytes, int kind, uint8_t *__restrict__ mo)
 {
     const int nsup = nblk >> 2, nq4 = (nsup + 3) >> 2;            // nblk: 32-weight blocks per row
-    const size_t mo_tile = mo_tile_bytes(nsup);
+    const size_t mo_tile = mo_tile_bytes(nsup, kind);
     const int ntiles = (rows + 15) >> 4;
     const size_t total = (size_t)ntiles * nq4 * 4 * 64;            // (supersteps padded to whole quads: the pad's words are zero)
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(256) k_gemm_rows_mo_build(const uint8_t *__res
         uint8_t *tb = mo + (size_t)tile * mo_tile;
         if (S < nsup) *reinterpret_cast<u32x4 *>(tb + (size_t)S * 1024 + (size_t)lane * 16) = c;
         *reinterpret_cast<uint32_t *>(tb + (size_t)(nsup + (S >> 2)) * 1024 + (size_t)lane * 16 + (size_t)(S & 3) * 4) = w;
-        *reinterpret_cast<uint32_t *>(tb + mo_words_at(nsup) + (size_t)S * 256 + (size_t)lane * 4) = w;
+        if (kind == MO_WORDS) *reinterpret_cast<uint32_t *>(tb + mo_words_at(nsup) + (size_t)S * 256 + (size_t)lane * 4) = w;
     }
 }
 
@@ -153,7 +153,7 @@ static int gm_launch1(int wgs, size_t smem, const GmArgs &P, int epi, int norm, 
 // the kernels' byte offsets inside a matrix have 32 bits (tiled rows: 20 bytes a block and padding; operand-order copies: whole tiles)
 extern "C" int ifa_gemm_rows_offsets_fit(size_t rows, size_t cols, int mo)
 {
-    return (mo ? gemm_rows_mo_bytes(rows, cols) : (rows + 16) * (cols / 32 + 16) * 20) < ((size_t)1 << 32);
+    return (mo ? gemm_rows_mo_bytes(rows, cols, mo) : (rows + 16) * (cols / 32 + 16) * 20) < ((size_t)1 << 32);
 }
 
 bool gemm_rows_mfma_fused_ok(const GmArgs &P, int epi, int norm)
@@ -249,11 +249,11 @@ int gemm_rows_mfma(const void *Wt_tiled, size_t rows, size_t cols, const void *x
         static std::map<std::pair<const void *, size_t>, void *> cache;      // (never freed: a tuning aid)
         void *&mo = cache[std::make_pair(Wt_tiled, rows * 65537 + cols)];
         if (!mo) {
-            IFA_HIP_CHECK(hipMalloc(&mo, gemm_rows_mo_bytes(rows, cols)));
-            int rc = gemm_rows_mo_build(Q4_B32T1A, Wt_tiled, rows, cols, mo, s);
+            IFA_HIP_CHECK(hipMalloc(&mo, gemm_rows_mo_bytes(rows, cols, MO_QUADS)));
+            int rc = gemm_rows_mo_build(Q4_B32T1A, Wt_tiled, rows, cols, MO_QUADS, mo, s);
             if (rc) return rc;
         }
-        P.W[0] = (const uint8_t *)mo; P.mo = 1;
+        P.W[0] = (const uint8_t *)mo; P.mo = MO_QUADS;
     }
     return gemm_rows_mfma_launch(P, GM_PLAIN, 0, s);
 }
@@ -305,20 +305,20 @@ int expand_b64_to_q4b32(int dtype, const void *tiled, size_t rows, size_t cols, 
     return IFA_OK;
 }
 
-size_t gemm_rows_mo_bytes(size_t rows, size_t cols)
+size_t gemm_rows_mo_bytes(size_t rows, size_t cols, int kind)
 {
-    return (rows + 15) / 16 * mo_tile_bytes((int)(cols / 128));
+    return (rows + 15) / 16 * mo_tile_bytes((int)(cols / 128), kind);
 }
 
-int gemm_rows_mo_build(int dtype, const void *tiled, size_t rows, size_t cols, void *mo, hipStream_t s)
+int gemm_rows_mo_build(int dtype, const void *tiled, size_t rows, size_t cols, int kind, void *mo, hipStream_t s)
 {
     IFA_REQUIRE(tiled && mo && rows > 0 && cols % 128 == 0, "gemm_rows_mo_build: %zu x %zu", rows, cols);
     const size_t items = (rows + 15) / 16 * ((cols / 128 + 3) / 4 * 4) * 64;
     const dim3 grid((unsigned)std::min<size_t>(65535, (items + 255) / 256)), block(256);
     if (dtype == Q4_B32T1A || dtype == Q4_B32T1B)
-        k_gemm_rows_mo_build<false><<<grid, block, 0, s>>>((const uint8_t *)tiled, (int)rows, (int)(cols / 32), tiled_row_bytes(dtype, cols / 32), (uint8_t *)mo);
+        k_gemm_rows_mo_build<false><<<grid, block, 0, s>>>((const uint8_t *)tiled, (int)rows, (int)(cols / 32), tiled_row_bytes(dtype, cols / 32), kind, (uint8_t *)mo);
     else if (dtype == Q4_B64T1 || dtype == Q3H_B64T1)
-        k_gemm_rows_mo_build<true><<<grid, block, 0, s>>>((const uint8_t *)tiled, (int)rows, (int)(cols / 32), tiled_row_bytes(dtype, cols / 64), (uint8_t *)mo);
+        k_gemm_rows_mo_build<true><<<grid, block, 0, s>>>((const uint8_t *)tiled, (int)rows, (int)(cols / 32), tiled_row_bytes(dtype, cols / 64), kind, (uint8_t *)mo);
     else return ifa_fail(IFA_ERR_ARG, "gemm_rows_mo_build: format %d has no MO layout (value = q * scale + base nibble formats only)", dtype);
     IFA_LAUNCH_CHECK();
     return IFA_OK;

@@ -141,7 +141,7 @@ __device__ __forceinline__ void gemm_rows_mfma_body(const GmArgs &P, char *smem)
     const int ntiles = (P.total_rows + 15) >> 4;                  // (several sets: every set is whole tiles)
     const size_t row_bytes = tiled_row_bytes(Q4_B32T1A, (size_t)nblk);
     const int nq4 = (nsup + 3) >> 2;                              // MO: header quads per tile
-    const size_t mo_tile = mo_tile_bytes(nsup);                   // MO: bytes per 16-row tile
+    const size_t mo_tile = mo_tile_bytes(nsup, P.mo);               // MO: bytes per 16-row tile
     const int row_stride = WHOLE ? K * 2 + 16 : G::ROW_STRIDE;    // bytes per activation row in LDS
     const int trow = min(r, T - 1);                               // B operand: token of this lane (columns past T: duplicates, never stored)
     const int trow1 = min(r + 16, T - 1);                         // second column tile (NT == 2)

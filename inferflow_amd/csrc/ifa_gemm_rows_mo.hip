@@ -226,7 +226,7 @@ __global__ void __launch_bounds__(GM_THREADS) k_gemm_rows_mo_grouped(const MoeSm
     P.bias[0] = nullptr; P.bias[1] = nullptr; P.bias[2] = nullptr; P.bias1 = nullptr;
     P.Y = Y + (size_t)gq.row0 * rows; P.res = nullptr; P.ldy = rows; P.ldres = 0; P.act_kind = act_kind;
     P.Yset[0] = nullptr; P.Yset[1] = nullptr; P.Yset[2] = nullptr; P.ldyset[0] = 0; P.ldyset[1] = 0; P.ldyset[2] = 0;
-    P.mo = 1; P.trace = nullptr; P.kparts = 0; P.kpart_sums = nullptr;
+    P.mo = MO_QUADS; P.trace = nullptr; P.kparts = 0; P.kpart_sums = nullptr;
     // groups of 2..4 rows (most of them: 16 entries over 8 experts): four rows staged instead of eight, and rows longer than a chunk
     // (w2) staged whole -- no re-staging, no barriers in the chunk loop
     if (gq.nrows <= 4 && (CH == 1 || (size_t)4 * ((size_t)nblk * 64 + 16) <= (size_t)whole_lds)) {

@@ -59,16 +59,17 @@ def test_dtype_names(name, expect):
 
 @pytest.mark.parametrize("cols", [128, 4096, 20480, 28672])
 def test_rows_products_decline_matrices_whose_copies_pass_32_bit_offsets(cols):
-    """the layouts' own sizes on both sides of 4 GiB: operand-order copies of 16 rows x 128 columns are a KiB of codes and, by four of them, a KiB of (base, scale) words -- twice --, tiled rows
-    20 bytes a block of 32 and room"""
+    """the layouts' own sizes on both sides of 4 GiB: operand-order copies of 16 rows x 128 columns are a KiB of codes and, by four of them, a KiB of (base, scale) words -- twice
+    where products of many rows read them (2) --, tiled rows (0) 20 bytes a block of 32 and room"""
     import ctypes as C
     f = ia.lib().ifa_gemm_rows_offsets_fit
     f.argtypes, f.restype = [C.c_size_t, C.c_size_t, C.c_int], C.c_int
     sup = cols // 128
-    tile = 1024 * (sup + 2 * ((sup + 3) // 4))
-    most = ((1 << 32) - 1) // tile * 16                      # rows of the largest copy below 4 GiB
-    assert f(most, cols, 1) == 1 and f(most + 1, cols, 1) == 0
-    assert f(16, cols, 1) == 1 and f(16, cols, 0) == 1
+    for kind in (1, 2):
+        tile = 1024 * (sup + kind * ((sup + 3) // 4))
+        most = ((1 << 32) - 1) // tile * 16                      # rows of the largest copy below 4 GiB
+        assert f(most, cols, kind) == 1 and f(most + 1, cols, kind) == 0
+        assert f(16, cols, kind) == 1
     room = ((1 << 32) - 1) // (20 * (cols // 32 + 16)) - 16
     assert f(room, cols, 0) == 1 and f(room + 1, cols, 0) == 0
 

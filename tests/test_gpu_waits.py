@@ -60,6 +60,45 @@ def test_failed_operand_order_copy_allocation_does_not_fail_the_step_that_asked_
     wk.close(); ref.close()
 
 
+def test_only_copies_that_products_of_many_rows_read_hold_their_words_twice():
+    """a KiB of (base, scale) words by four of codes in a mixture-of-experts model's copies, which only the rows products read; two in a dense model's"""
+    for shape, per in (("test_moe", 1), ("test_gqa", 2)):
+        wk, _, s = synth.build(shape, dt.Q4_B32T1A, dt.F16, max_ctx=48, quant_threshold=0)
+        assert wk.buffer("rows_copy")[1] == 0
+        wk.kv_slots(12)
+        cur, pos = _prefill_slots(wk, s["vocab"], 12, 3)
+        wk.decode_batch(cur, pos, list(range(12)))
+        sup = s["dim"] // 128
+        assert wk.buffer("rows_copy")[1] == s["heads"] * s["head_dim"] // 16 * 1024 * (sup + per * ((sup + 3) // 4)), shape
+        wk.close()
+
+
+@pytest.mark.parametrize("n", [12, 20])
+def test_without_memory_for_the_words_by_supersteps_the_rows_products_keep_their_copies(n):
+    """(simulated: debug_mo_alloc_fail 2) batched steps run as with rows_few 0, prompts as with prefill_mid 0, bit for bit: the copies without these words serve the rows products"""
+    shape = dict(dim=1024, heads=16, kv_heads=2, head_dim=64, ffn=1408)
+    wk, ref = (synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=256, layers=2, vocab=600, quant_threshold=0, **shape)[0] for _ in range(2))
+    wk.set_option("debug_mo_alloc_fail", 2)
+    ref.set_option("rows_few", 0); ref.set_option("prefill_mid", 0)
+    out = []
+    for w in (wk, ref):
+        w.kv_slots(n)
+        cur, pos = _prefill_slots(w, 600, n, 5)
+        lg = torch.empty((n, 600), dtype=torch.float16, device="cuda")
+        tok = [w.decode_batch(cur, pos, list(range(n)), lg), w.decode_batch(cur, pos, list(range(n)))]          # (eager, and captured)
+        rows = [g.host(lg).copy()]
+        for T in (20, 40, 200):
+            w.select_kv(0); w.reset()
+            pl = torch.empty((T, 600), dtype=torch.float16, device="cuda")
+            w.forward(np.arange(3, 3 + T).astype(np.int32), 0, pl)
+            rows.append(g.host(pl).copy())
+        out.append((tok, rows))
+    assert wk.buffer("rows_copy")[1] == 64 * 1024 * (8 + 2) and ref.buffer("rows_copy")[1] == 64 * 1024 * (8 + 2 * 2)
+    assert all(list(a) == list(b) for a, b in zip(out[0][0], out[1][0]))
+    assert all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
+    wk.close(); ref.close()
+
+
 @pytest.mark.parametrize("n", [12, 24])
 def test_rows_kparts_option_switches_the_waiting_launch_off(n):
     """w2 of test_longffn walks several chunks of K at 9..32 rows: K parts by default, plain chunk loop with rows_kparts = 0"""
