@@ -578,7 +578,8 @@ bool prefill_big_layers(const ifa_model *m)
     return true;
 }
 
-int batch_fused_layer(ifa_model *m, int l, int n, const half_t *x, half_t *xnext, const void *rows_l)
+// few: its products through gemm_few (rows_few_ok, asked once a step)
+int batch_fused_layer(ifa_model *m, int l, int n, bool few, const half_t *x, half_t *xnext, const void *rows_l)
 {
     const ifa_model_config &c = m->cfg;
     Layer &L = m->layers[(size_t)l];
@@ -590,13 +591,12 @@ int batch_fused_layer(ifa_model *m, int l, int n, const half_t *x, half_t *xnext
     clear();
     P.W[0] = rows_w(m, L.t[T_WQ]); P.W[1] = rows_w(m, L.t[T_WK]); P.W[2] = rows_w(m, L.t[T_WV]); P.mo = rows_mo(m, L.t[T_WQ]);
     P.rows[0] = (int)QD; P.rows[1] = (int)KVD; P.rows[2] = (int)KVD; P.nsets = 3; P.nblk = (int)(D / 32);
-    // (9..16 queries: the activation rows are staged in chunks of 2048 columns, so the norm runs as its own launch)
-    const bool few = n >= FEW_MIN && rows_few_ok(m, n);
     if (few) {
         if (l == 0 && (rc = few_norm(m, 0, T_ATTN_NORM, n, nullptr, nullptr, x, nullptr))) return rc;
         const int ld = (int)(QD + 2 * KVD);
         if ((rc = few_qkv(m, L, n, m->bqkv, m->bqkv + QD, m->bqkv + QD + KVD, ld, ld))) return rc;
     }
+    // (9..16 queries, tiled layout: the activation rows are staged in chunks of 2048 columns, so the norm runs as its own launch)
     const bool norm_fused = (n <= 8 || rows_mo(m, L.t[T_WQ])) && n <= 16;      // (MO layout: 16 rows x 4096 columns are one chunk too; 17..32 rows: chunked)
     Tensor nob;
     if (!few && !norm_fused && (rc = norm_rows(m, x, n, L.t[T_ATTN_NORM], nob, m->xn, c.attn_norm_base))) return rc;
@@ -699,7 +699,7 @@ int forward_batch(ifa_model *m, int n, const int *tokens_host, const int *pos_ho
     for (const Layer &Lc : m->layers) has_moe = has_moe || (c.experts > 0 && Lc.t[T_MOE_GATE].present());
     // (measured on Llama-2-7B Q4: the batched step is bound by the small-T GEMM kernels, ~6.7 ms with or without the
     //  graph, so replay is opt-in: set_option("batch_graph", 1))
-    bool fused = batch_fused_ok(m, n);          // five launches per layer: launch-bound without a graph, so it is replayed
+    bool few = false, fused = batch_fused_ok(m, n);          // five launches per layer: launch-bound without a graph, so it is replayed
     if (fused) {
         int rcm = ensure_mo(m); if (rcm) return rcm;
         // ensure_mo may have DOWNGRADED the model (the copies did not fit: opt_rows_mo = 0): what batch_fused_ok answered with the
@@ -707,7 +707,7 @@ int forward_batch(ifa_model *m, int n, const int *tokens_host, const int *pos_ho
         // is chosen; a step the tiled kernels do not cover takes the op-by-op rows below
         fused = batch_fused_ok(m, n);
         if (fused && (rcm = gemm_rows_kparts_reserve(m->stream))) return rcm;
-        if (fused) (void)rows_few_ok(m, n);      // (its workspace, before a capture)
+        few = fused && rows_few_ok(m, n);      // (and its workspace, before a capture)
     }
     if (has_moe && m->opt_moe_overlap) { int rcs = ensure_side_stream(m); if (rcs) return rcs; }
     // (MoE layers of the fused step route on the device -- no host round trip -- so they are captured too)
@@ -741,7 +741,7 @@ int forward_batch(ifa_model *m, int n, const int *tokens_host, const int *pos_ho
     bool xn_ready = false;           // see forward_ops: every residual Add is fused with the norm that follows it
     if (fused) {
         for (int l = 0; l < c.layers; l++) {
-            if ((rc = batch_fused_layer(m, l, n, x, m->f, rows_d + (size_t)l * (size_t)n))) return rc;
+            if ((rc = batch_fused_layer(m, l, n, few, x, m->f, rows_d + (size_t)l * (size_t)n))) return rc;
             std::swap(m->x, m->f);
             x = m->x;
         }

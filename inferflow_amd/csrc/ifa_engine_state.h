@@ -366,7 +366,7 @@ bool prefill_big_ok(const ifa_model *m);
 bool prefill_big_layers(const ifa_model *m);      // ... of the layers alone, whatever the options
 bool prefill_mid_ok(ifa_model *m, int T, bool any_length);
 bool rows_few_ok(ifa_model *m, int T);
-int batch_fused_layer(ifa_model *m, int l, int n, const half_t *x, half_t *xnext, const void *rows_l);
+int batch_fused_layer(ifa_model *m, int l, int n, bool few, const half_t *x, half_t *xnext, const void *rows_l);
 int forward_batch(ifa_model *m, int n, const int *tokens_host, const int *pos_host, const int *slot_host, int *next_tokens,
                          void *logits_out);
 // ---- ifa_engine_moe.hip
