@@ -286,7 +286,8 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
     // weights dequantised once per workgroup and step into LDS; reference-layout rows), norms as their own launches.
     // the mid-length kernel (33 .. prefill_mid_max tokens): every linear of every layer a 4-bit tensor with its operand-order copy, dense FFN
     const bool pstat = m->opt_perf_stat != 0;       // per-phase times: the op-by-op layer below (one launch per reference op), never the fused routes
-    const bool pf_few = !tp && !pstat && (T <= 32 ? m->opt_batch_fused : m->opt_prefill_mid) && rows_few_ok(m, T);      // (FEW_MIN .. few_max_rows tokens: gemm_few)
+    // FEW_MIN .. few_max_rows tokens: gemm_few, behind the switches of the products that it takes over
+    const bool pf_few = !tp && !pstat && (T <= 32 ? m->opt_batch_fused && m->opt_gemm_rows && gemm_rows_use_mfma() : m->opt_prefill_mid) && rows_few_ok(m, T);
     const bool pf_mid = !pf_few && !tp && !pstat && prefill_mid_ok(m, T, false);
     const bool pf_big = pf_few || pf_mid || (!tp && !pstat && T > std::max(32, m->opt_prefill_big_min) && prefill_big_ok(m));
     bool pf_fused = pf_big || (!tp && !pstat && T >= 2 && T <= 32 && batch_fused_ok(m, T) && c.experts == 0);

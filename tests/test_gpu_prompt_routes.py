@@ -174,6 +174,21 @@ def test_products_that_stream_their_weights_over_few_rows_agree_with_the_others(
     wk.close()
 
 
+@pytest.mark.parametrize("T", [9, 20, 32, 33, 60])
+@pytest.mark.parametrize("option", ["gemm_rows", "batch_fused", "prefill_mid"])
+def test_the_switches_of_the_products_over_few_rows_hold_for_all_that_serve_them(option, T):
+    """off, a prompt takes the bits that it has without gemm_few: up to 32 rows by gemm_rows and batch_fused, above by prefill_mid"""
+    wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=64, layers=2, vocab=600, quant_threshold=0, dim=1024, heads=16, kv_heads=2, head_dim=64, ffn=1408)
+    toks, out = np.random.default_rng(T).integers(3, s["vocab"], T).astype(np.int32), []
+    wk.set_option("prefill_chunk", 0)
+    for sw, few in ((1, 1), (0, 1), (0, 0)):
+        wk.set_option(option, sw); wk.set_option("rows_few", few)
+        out.append(_rows(wk, toks, s["vocab"])[1])
+    off = (T <= 32) != (option == "prefill_mid")
+    assert np.array_equal(out[1], out[2]) == off and np.array_equal(out[0], out[1]) != off
+    wk.close()
+
+
 @pytest.mark.parametrize("ffn,most", [(12288, 192), (12416, 96)])
 def test_where_wide_models_leave_the_products_over_few_rows(ffn, most):
     """gemm_few sums K in another order, so its rows differ from the other route's in some bits, up to its last row count and no further"""
