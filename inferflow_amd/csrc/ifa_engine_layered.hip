@@ -114,14 +114,14 @@ struct LayeredNet {
                                            // SANDWICH layers, every step size: the norm behind a sub-layer and the norm in front of the next one in one launch
                                            // PRENORM layers: the start of a looped pass inside the norm's launch; steps of at most 8 rows: the norm inside the router's launch
     float *attn_ws = nullptr; size_t attn_ws_bytes = 0;      // partial results of the windowed attention when a (row, head)'s keys are shared out
-    // Workspaces of prompts through the tiled attention and the chunked recurrences: reserved for one prompt as long as the context when the model is finalized (up to
+    // Workspaces of prompts through the tiled attention, the chunked recurrences and sums of products with K shared out (planes): reserved for one prompt as long as the context when the model is finalized (up to
     // RESERVE_BYTES each), grown by steps that need more -- several prompts, or a shorter one whose keys are shared out further: 960 tokens behind a window of 1024, 16 heads of
-    // 128, 67 MB where 4096 tokens take 24 -- up to opt_workspace_mb each.  A step beyond that, or whose workspace cannot be had, runs without (fp32 tiles, token by token).
+    // 128, 67 MB where 4096 tokens take 24 -- up to opt_workspace_mb each.  A step beyond that, or whose workspace cannot be had, runs without (fp32 tiles, token by token, a workgroup a
+    // tile of a sum).
     float *tile_ws = nullptr; size_t tile_ws_bytes = 0;
     int opt_workspace_mb = 4096; bool step_tile_ws = false;
     bf16_t *a16 = nullptr, *h16 = nullptr, *g16 = nullptr; size_t a16_cap = 0, h16_cap = 0, g16_cap = 0;
-    float *planes = nullptr; size_t planes_cap = 0;          // summands of x that the next layer adds (run_parallel_prompt)
-   
+    float *planes = nullptr; size_t planes_bytes = 0; bool step_planes = false;          // summands of x that the next layer adds (run_parallel_prompt)
     // activations of a product rounded to bfloat16 beforehand: steps of at least this many rows (0: never).  Above the eight rows whose activations stay in 32 bits; k_lin_mfma rounds the
     // same on its way (9 / 16 tokens of Sopulorn 1561 -> 801 us / 1808 -> 1010, of Gelarax 1564 -> 642 / 1784 -> 823, 12 prompt rows of width 2048 2713 -> 979)
     int opt_a16_min = 9;
@@ -418,14 +418,35 @@ float norm_offset_of(const LayeredNet *n) { return n->cfg.norm_plain ? 0.0f : 1.
 bool takes_a16(const LayeredNet *n, size_t K, size_t T) { return !n->cfg.ops32 && n->opt_a16_min > 0 && T >= (size_t)n->opt_a16_min && K % 8 == 0 && K >= 64; }
 size_t a16_stride(size_t K) { return (K + 63) & ~(size_t)63; }
 
-template <class V>
-int ensure_halfs(ifa_model *m, V *&buf, size_t &cap, size_t need)
+// where the operands of a PARALLEL block's output product lie in a row of n->a16: the mixers' (at 0 and at1), the feed-forward's (at2)
+struct SumColumns { size_t AQ, MV, F, at1, at2, ld; };
+SumColumns sum_columns(const ifa_layer_spec &sp)
+{
+    const bool lin = sp.mixer == IFA_MIX_WINDOW_LINEAR;
+    SumColumns c;
+    c.AQ = lin ? (size_t)sp.a_heads * sp.a_dim : 0; c.MV = lin ? (size_t)sp.l_heads * sp.l_vdim : (size_t)sp.d_heads * sp.d_vdim; c.F = (size_t)std::max(sp.ffn, 0);
+    c.at1 = c.AQ ? a16_stride(c.AQ) : 0; c.at2 = c.at1 + a16_stride(c.MV); c.ld = c.at2 + (c.F ? a16_stride(c.F) : 0);
+    return c;
+}
+
+// bytes of the planes that a step of T rows leaves between its PARALLEL blocks (0: none)
+size_t planes_workspace_bytes(const LayeredNet *n, size_t T)
+{
+    const size_t W = (size_t)n->cfg.width;
+    size_t most = 0;
+    if (!takes_a16(n, W, T) || W > 8192 || W % 4 != 0) return 0;
+    for (const LLayer &L : n->layers)
+        if (L.spec.block == IFA_BLOCK_PARALLEL) most = std::max(most, (size_t)ifa_linear_bf16_sum_plane_count(W, sum_columns(L.spec).ld, T));
+    return most * T * W * sizeof(float);
+}
+
+int ensure_halfs(ifa_model *m, bf16_t *&buf, size_t &cap, size_t need)
 {
     if (need <= cap) return IFA_OK;
     IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
     drop_step_graph(m->lay);          // (with a16_min 1 a captured step reads these)
     lay_free(buf); buf = nullptr; cap = 0;
-    IFA_HIP_CHECK(hipMalloc((void **)&buf, need * sizeof(V)));
+    IFA_HIP_CHECK(hipMalloc((void **)&buf, need * 2));
     cap = need;
     return IFA_OK;
 }
@@ -1023,18 +1044,17 @@ int run_parallel_prompt(ifa_model *m, LLayer &L, size_t T, int nseq, bool *done,
     LayeredNet *n = m->lay;
     const ifa_layered_config &c = n->cfg;
     const ifa_layer_spec &sp = L.spec;
-    const size_t W = (size_t)c.width, NI = L.n_in, F = (size_t)std::max(sp.ffn, 0);
+    const SumColumns at = sum_columns(sp);
+    const size_t W = (size_t)c.width, NI = L.n_in, AQ = at.AQ, MV = at.MV, F = at.F, at1 = at.at1, at2 = at.at2, ld = at.ld, ldw = a16_stride(W);
     ifa_stream s = (ifa_stream)m->stream;
     void *const *slots = (void *const *)n->slot_base_dev;
     const bool lin = sp.mixer == IFA_MIX_WINDOW_LINEAR;
-    const size_t AQ = lin ? (size_t)sp.a_heads * sp.a_dim : 0, MV = lin ? (size_t)sp.l_heads * sp.l_vdim : (size_t)sp.d_heads * sp.d_vdim;
     *done = takes_a16(n, W, T) && (!AQ || takes_a16(n, AQ, T)) && takes_a16(n, MV, T) && (!F || takes_a16(n, F, T)) && W <= 8192;
     if (!*done) {
         const int left = *pending;
         *pending = 0;
         return left ? ifa_add_planes_f32(n->x, n->planes, left, T, W, s) : IFA_OK;
     }
-    const size_t at1 = AQ ? a16_stride(AQ) : 0, at2 = at1 + a16_stride(MV), ld = at2 + (F ? a16_stride(F) : 0), ldw = a16_stride(W);
     const void *ls1 = L.T(IFA_LT_LS1).data;
     int rc;
     if ((rc = ensure_halfs(m, n->h16, n->h16_cap, T * ldw)) || (rc = ensure_halfs(m, n->a16, n->a16_cap, T * ld))) return rc;
@@ -1074,8 +1094,7 @@ int run_parallel_prompt(ifa_model *m, LLayer &L, size_t T, int nseq, bool *done,
     if (lin) parts[np++] = {L.T(IFA_LT_A_O).data, AQ, ls1, nullptr, sp.a_out_scale};
     parts[np++] = {L.T(lin ? IFA_LT_L_O : IFA_LT_D_O).data, MV, ls1, nullptr, lin ? sp.l_out_scale : 1.0f};
     if (F) parts[np++] = {L.T(IFA_LT_FFN_DOWN).data, F, L.T(IFA_LT_LS2).data, L.T(IFA_LT_FFN_DOWN_B).data, 1.0f};
-    int planes = W % 4 == 0 ? ifa_linear_bf16_sum_plane_count(W, ld, T) : 0;
-    if (planes && ensure_halfs(m, n->planes, n->planes_cap, (size_t)planes * T * W) != IFA_OK) { (void)hipGetLastError(); planes = 0; }          // (no memory for them: a workgroup a tile)
+    const int planes = n->step_planes ? ifa_linear_bf16_sum_plane_count(W, ld, T) : 0;
     if ((rc = ifa_linear_bf16_sum_planes(parts, np, W, n->a16, ld, T, n->x, W, planes ? n->planes : nullptr, s))) return rc;
     *pending = planes;
     return IFA_OK;
@@ -1599,6 +1618,9 @@ int lay_finalize(ifa_model *m)
         const ifa_seq_desc whole{0, n->cfg.max_ctx, 0, 0};
         (void)grow_workspace(m, (void **)&n->tile_ws, &n->tile_ws_bytes, std::min(RESERVE_BYTES, tile_workspace_bytes(n, &whole, 1)), RESERVE_BYTES);
         (void)grow_workspace(m, &n->scan_ws, &n->scan_ws_bytes, std::min(RESERVE_BYTES, scan_workspace_bytes(n, ((size_t)n->cfg.max_ctx + 63) / 64)), RESERVE_BYTES);
+        size_t planes = 0;          // (K is shared out between fewer workgroups the longer a prompt is: the most is at some length in between)
+        for (size_t T = 32; T < (size_t)n->cfg.max_ctx + 32; T += std::max<size_t>(32, T / 512 * 32)) planes = std::max(planes, planes_workspace_bytes(n, std::min(T, (size_t)n->cfg.max_ctx)));
+        if (planes) (void)grow_workspace(m, (void **)&n->planes, &n->planes_bytes, std::min(RESERVE_BYTES, planes), RESERVE_BYTES);
     }
     m->finalized = true;
     return IFA_OK;
@@ -1779,6 +1801,8 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
     }
     n->step_tile_ws = T >= (size_t)std::max(n->opt_attn_tile_min, 2)          // (a step of one row takes no tiles of the workspace's form, see attention_launch)
                       && grow_workspace(m, (void **)&n->tile_ws, &n->tile_ws_bytes, tile_workspace_bytes(n, n->seqs_host.data(), nseq), most);
+    const size_t planes = T >= 2 ? planes_workspace_bytes(n, T) : 0;
+    n->step_planes = planes && grow_workspace(m, (void **)&n->planes, &n->planes_bytes, planes, most);
     if ((rc = run_layers(m, T, nseq))) return rc;
     ifa_stream s = (ifa_stream)m->stream;
     if (all) {
@@ -1846,7 +1870,7 @@ int lay_decode(ifa_model *m, int first_token, int start_pos, int n_steps, int *o
     if ((rc = check_span(m, n_steps, start_pos, nullptr)) || (rc = ensure_slot(m, n->cur_slot)) || (rc = ensure_rows(m, 1, 1)) || (rc = ensure_logits(m, 1))) return rc;
     if (n->opt_graph && !n->opt_tap_layers && !n->step_exec) {      // (the slot is read from the device tables: one capture serves every slot)
         drop_step_graph(n);
-        n->step_expand = false; n->scan_chunks = 0; n->step_tile_ws = false;
+        n->step_expand = false; n->scan_chunks = 0; n->step_tile_ws = n->step_planes = false;
         n->seqs_host.assign(1, ifa_seq_desc{0, 1, start_pos, n->cur_slot});      // (the launches are shaped by it: one sequence, one row)
         IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
         IFA_HIP_CHECK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
@@ -1865,7 +1889,7 @@ int lay_decode(ifa_model *m, int first_token, int start_pos, int n_steps, int *o
     std::vector<int> tok(1, first_token), pos(1, start_pos), rs(1, 0);
     std::vector<ifa_seq_desc> sq(1); sq[0] = ifa_seq_desc{0, 1, start_pos, n->cur_slot};
     if ((rc = upload_tables(m, tok, pos, rs, sq))) return rc;
-    n->step_expand = false; n->scan_chunks = 0; n->step_tile_ws = false;
+    n->step_expand = false; n->scan_chunks = 0; n->step_tile_ws = n->step_planes = false;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (elapsed_ms) { IFA_HIP_CHECK(hipEventCreate(&e0)); IFA_HIP_CHECK(hipEventCreate(&e1)); IFA_HIP_CHECK(hipEventRecord(e0, m->stream)); }
     for (int st = 0; st < n_steps; st++) {

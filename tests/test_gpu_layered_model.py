@@ -318,6 +318,40 @@ def test_prompts_with_and_without_the_workspaces_of_tiles_and_chunks(tmp_path, l
     eng.close()
 
 
+@pytest.mark.parametrize("T", [9, 40, 300])
+def test_sums_of_products_with_and_without_the_workspace_of_their_planes(tmp_path, T):
+    """K shared out to workgroups, whose sums the next block's norm adds, the last block's an addition by itself; without the workspace (limit 0) a workgroup goes through all of K: sums in
+    another order, so some bits differ"""
+    import inferflow_amd as ia
+    cfg = fx.config([fx.parallel_layer(heads=4, kv_heads=2, dim=64, window=200, keep_first=3, lin_heads=4, lin_dim=64, lin_vdim=128, ff=2816),
+                     fx.delta_layer(heads=4, kv_heads=2, dim=64, vdim=64, conv=3, ff=2816)], width=512, vocab=97)
+    w, toks, out = fx.random_weights(cfg, 37), tokens_for(cfg, T, 38), []
+    for limit in (4096, 0):
+        eng = engine_for(tmp_path, cfg, w, "bfloat16", 400, 1)
+        for name, value in ((b"attn_tile_min", 1 << 20), (b"scan_chunk_min", 0), (b"workspace_mb", limit)):
+            ia.check(ia.lib().ifa_model_set_option(eng.worker(), name, value))
+        out.append(run_whole(eng, toks)[0])
+        eng.close()
+    want = oracle_logits(cfg, w, toks)
+    assert all(fx.rel_err(o, want).max() < TOL16 for o in out)
+    assert not np.array_equal(*out)
+
+
+def test_generation_over_bfloat16_rows_of_single_tokens_behind_a_prompt_without_planes(tmp_path):
+    """a16_min 1, a launch per operation: the captured step's sums take no planes, which no prompt may have left room for (2048 rows of width 1024: none)"""
+    import inferflow_amd as ia
+    cfg = fx.config([fx.parallel_layer(heads=8, kv_heads=2, dim=128, window=64, keep_first=0, lin_heads=8, lin_dim=64, lin_vdim=128, ff=2816)], width=1024, vocab=97)
+    w, seen = fx.random_weights(cfg, 39), {}
+    for graph in (1, 0):
+        eng = engine_for(tmp_path, cfg, w, "bfloat16", 2100, 1)
+        for name, value in ((b"a16_min", 1), (b"fuse_step", 0), (b"graph", graph)):
+            ia.check(ia.lib().ifa_model_set_option(eng.worker(), name, value))
+        q = eng.add_query(tokens_for(cfg, 2048, 40))
+        seen[graph] = eng.generate(q, 12)[0]
+        eng.close()
+    assert seen[1] == seen[0]
+
+
 @pytest.mark.parametrize("T,width", [(9, 520), (16, 520), (17, 520), (130, 520), (601, 520), (1500, 520), (3100, 520), (70, 2056), (300, 72), (130, 128)])
 def test_prompts_whose_products_read_bfloat16_rows(tmp_path, T, width):
     """Activations formed in the product's own tiles, outputs of norms and mixers left in bfloat16, a layer's output products in one pass over their columns -- every tile size, few and many
