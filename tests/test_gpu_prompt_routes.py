@@ -1,8 +1,5 @@
-"""-m gpu: the two prompt routes added in round 5 agree with the routes they replace (same rows, other kernels: agreement within the F16
-rounding of the summation order), on two layers of Llama-2-7B width:
-  * 34..48 tokens: two passes of the rows GEMM (32 + the rest; option prefill_chunk) against the op-by-op layer;
-  * 48..128 tokens: the four large-tile launches per layer (option prefill_big_min 47, with four parts of K for products of 32..96
-    tiles) against the op-by-op layer (prefill_big_min 128)."""
+"""-m gpu: routes of prompts against the routes that they replace (same rows, other kernels: agreement within the F16 rounding of the summation order), mostly on two layers.
+A test that compares two settings of an option turns off what would serve both of them alike, and says that their rows differ in some bit: sums of another order, so another route."""
 import numpy as np
 import pytest
 import torch
@@ -30,11 +27,12 @@ def test_two_pass_prompt_agrees_with_the_single_pass(T):
     wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=64, layers=2, vocab=2000)
     toks = np.random.default_rng(T).integers(3, s["vocab"], T).astype(np.int32)
     out = {}
+    wk.set_option("rows_few", 0); wk.set_option("prefill_mid", 0)
     for v in (1, 0):
         wk.set_option("prefill_chunk", v)
         out[v] = _rows(wk, toks, s["vocab"])
     ok, why = _agree(out[1][1], out[0][1])          # ALL rows: the first pass's logits land in rows 0..31, the second's behind them
-    assert ok, why
+    assert ok and not np.array_equal(out[1][1], out[0][1]), why
     wk.close()
 
 
@@ -43,40 +41,48 @@ def test_short_prompt_large_tile_route_agrees_with_the_op_by_op_layer(T):
     wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=160, layers=2, vocab=2000)
     toks = np.random.default_rng(T).integers(3, s["vocab"], T).astype(np.int32)
     out = {}
-    wk.set_option("prefill_chunk", 0)
+    for name in ("prefill_chunk", "rows_few", "prefill_mid"):
+        wk.set_option(name, 0)
     for v in (47, 128):
         wk.set_option("prefill_big_min", v)
         out[v] = _rows(wk, toks, s["vocab"])
     ok, why = _agree(out[47][1], out[128][1])
-    assert ok, why
+    assert ok and not np.array_equal(out[47][1], out[128][1]), why
     wk.close()
 
 
 @pytest.mark.parametrize("T", [33, 47, 63, 64])
 def test_prompts_in_64_token_tiles_agree_with_the_128_token_tiles(T):
-    """up to 64 tokens a tile of the mid-length products holds 64 rows: the products and their sums are those of the 128-row tile, which 65 tokens take, so a row is
-    off by no more than one that the other routes (attention and head by prompt length) leave"""
+    """up to 64 tokens a tile of k_gemm_mid holds 64 rows (rows_few 0: gemm_few serves such prompts otherwise): the products and their sums are those of the 128-row tile, which 65 tokens
+    take, so a row is off by no more than one that the other routes (attention and head by prompt length) leave"""
     wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=160, layers=2, vocab=2000)
-    wk.set_option("prefill_chunk", 0)
+    wk.set_option("prefill_chunk", 0); wk.set_option("rows_few", 0)
     toks = np.random.default_rng(T).integers(3, s["vocab"], 65).astype(np.int32)
+    wk.set_option("prefill_mid", 0)
+    other = [_rows(wk, toks[:n], s["vocab"])[1] for n in (T, 65)]
+    wk.set_option("prefill_mid", 1)
     short, long_ = _rows(wk, toks[:T], s["vocab"])[1], _rows(wk, toks, s["vocab"])[1][:T]
     for a, b in zip(short, long_):
         ok, why = _agree(a, b)
         assert ok, why
+    assert not np.array_equal(short, other[0]) and not np.array_equal(long_, other[1][:T])
     print("T=%d rows that differ in a bit: %d" % (T, sum(not np.array_equal(a, b) for a, b in zip(short, long_))))
     wk.close()
 
 
+@pytest.mark.parametrize("off", [(), ("rows_few",), ("rows_few", "prefill_mid")], ids=["few", "mid", "large"])
 @pytest.mark.parametrize("T", [40, 64, 128])
-def test_short_prompt_routes_match_the_oracle(T):
+def test_short_prompt_routes_match_the_oracle(T, off):
     """... and against the ORACLE (the reference's T > 1 rule: F16 activations x dequantised weights, fp32 sums), not only against each
-    other: two layers of Llama-2-7B width, the model read back from the worker, every row of the prompt.  40 tokens = two passes of
-    the rows GEMM, 64 / 128 = the large-tile launches with four parts of K.  Measured (r05): worst row 0.006-0.007 x std(logits) at 2 layers; bound 0.03 x std
+    other: two layers of Llama-2-7B width, the model read back from the worker, every row of the prompt.  gemm_few; without it k_gemm_mid; without that two passes of
+    the rows GEMM (40 tokens) and the large-tile launches with four parts of K (64, 128).  Measured: worst row 0.006-0.007 x std(logits) at 2 layers; bound 0.03 x std
     on every row (the whole-model law of test_gpu_fullsize_oracle would allow 0.08 sqrt(2) = 0.11), cosine >= 0.9999."""
     from tests import model_util as mu
     wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=160, layers=2, vocab=2000)
     om = mu.oracle_model_from_worker(wk, s, 160)
     toks = np.random.default_rng(100 + T).integers(3, s["vocab"], T).astype(np.int32)
+    for name in off:
+        wk.set_option(name, 0)
     tok, rows = _rows(wk, toks, s["vocab"])
     t_or, l_or = om.forward(toks, 0, nthreads=8)
     ref = l_or.astype(np.float32)
@@ -139,8 +145,8 @@ def test_rotation_by_four_workgroups_a_token_and_by_one_leave_the_same_bits(head
     assert torch.equal(out[0][2][:, :kvd], out[0][1]) and torch.equal(out[0][3][:, :kvd], rows[2])
 
 
-def _biased(kvd, wd, T, **shape):
-    """a worker of two layers whose products and norms have biases"""
+def _biased(kvd, wd, T, norms=True, **shape):
+    """a worker of two layers whose products, and norms, have biases, no two alike"""
     from inferflow_amd import worker as W
     wk, _, s = synth.build("llama2_7b", wd, kvd, max_ctx=T + 16, layers=2, vocab=600, quant_threshold=0, **shape)
     gen = torch.Generator(device="cuda"); gen.manual_seed(1)
@@ -148,6 +154,8 @@ def _biased(kvd, wd, T, **shape):
     for l in range(2):
         for tid, n in ((W.T_WQ_B, qd), (W.T_WK_B, kvdim), (W.T_WV_B, kvdim), (W.T_WO_B, s["dim"]), (W.T_W1_B, s["ffn"]), (W.T_W3_B, s["ffn"]), (W.T_W2_B, s["dim"])):
             wk.set_tensor_f16(l, tid, dt.F16, (0.3 * torch.randn(n, generator=gen, device="cuda")).half(), 1, n)
+        for tid in (W.T_ATTN_NORM_B, W.T_FFN_NORM_B) if norms else ():
+            wk.set_tensor_f16(l, tid, dt.F16, (0.3 * torch.randn(s["dim"], generator=gen, device="cuda")).half(), 1, s["dim"])
     return wk, s
 
 
@@ -156,7 +164,8 @@ def _biased(kvd, wd, T, **shape):
                          ids=["7b", "w1024", "w2176"])
 def test_products_that_stream_their_weights_over_few_rows_agree_with_the_others(wd, shape, T):
     """9..192 rows (gemm_few) at both ends of every number of 16-row tiles and groups, whole and partial workgroups of tiles, numbers of supersteps that eight waves and the parts of K do not
-    divide, biases everywhere: against the products before (rows_few = 0; same halves, other orders of the fp32 sums: the bound of the routes above), from the start and behind a prefix"""
+    divide, biases everywhere: against the products before (rows_few = 0; same halves, other orders of the fp32 sums: the bound of the routes above; up to 32 rows, which no other fused route
+    takes with norm biases, the op-by-op layer), from the start and behind a prefix"""
     wk, s = _biased(dt.F16, wd, T, **shape)
     toks = np.random.default_rng(T).integers(3, s["vocab"], T + 5).astype(np.int32)
     out = {}
@@ -170,7 +179,7 @@ def test_products_that_stream_their_weights_over_few_rows_agree_with_the_others(
         out[v].append(g.host(lg).astype(np.float32))
     for a, b in zip(out[1], out[0]):
         ok, why = _agree(a, b)
-        assert ok, why
+        assert ok and not np.array_equal(a, b), why
     wk.close()
 
 
@@ -204,12 +213,13 @@ def test_where_wide_models_leave_the_products_over_few_rows(ffn, most):
     wk.close()
 
 
-@pytest.mark.parametrize("T", [193, 257, 385, 2048, 2600])
+@pytest.mark.parametrize("T", [193, 257, 385, 2048, 2600, 5003, 8192])
 @pytest.mark.parametrize("wd,shape", [(dt.Q4_B32T1A, {}), (dt.Q3H_B64T1, dict(dim=1024, heads=16, kv_heads=2, head_dim=64, ffn=1408)), (dt.Q4_B32T1B, dict(dim=2176, heads=9, kv_heads=3, ffn=3712))],
                          ids=["q4a", "q3h", "q4b"])
 def test_products_whose_steps_run_into_each_other_agree_with_the_large_tiles(wd, shape, T):
     """rows that fill no tile, numbers of 64-column steps with every remainder by the ring's four stages (16, 22, 34, 58 steps, whole and in parts), biases everywhere; 256-token
-    tiles (three quarters of a tile a compute unit and more, fewer rounds) for wq | wk | wv of 385 and 2048 rows, wo / w2 of 2048 (q4a), the gated pair of 2600 (q3h) and of 2048 (q4b)"""
+    tiles (three quarters of a tile a compute unit and more, fewer rounds) for wq | wk | wv of 385 and 2048 rows, wo / w2 of 2048 (q4a), the gated pair of 2600 (q3h) and of 2048 (q4b);
+    up to the longest prompt that goes this way"""
     wk, s = _biased(dt.F16, wd, T, **shape)
     toks = np.random.default_rng(T).integers(3, s["vocab"], T).astype(np.int32)
     out = []
@@ -219,6 +229,21 @@ def test_products_whose_steps_run_into_each_other_agree_with_the_large_tiles(wd,
         wk.reset()
     ok, why = _agree(out[0], out[1])
     assert ok, why
+    wk.close()
+
+
+@pytest.mark.parametrize("T", [900, 2048, 2600])
+def test_a_lowered_border_of_the_mid_length_products_leaves_them_wo_and_w2(T):
+    """prefill_mid_max 768: above it the large tiles, wo and w2 of up to prefill_res_mid (2048) tokens through k_gemm_mid with its parts of K"""
+    wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=T + 16, layers=2, vocab=600, quant_threshold=0, dim=2048, heads=16, kv_heads=16, ffn=5632)
+    toks, out = np.random.default_rng(T).integers(3, s["vocab"], T).astype(np.int32), []
+    wk.set_option("prefill_mid_max", 768)
+    for v in (2048, 0):
+        wk.set_option("prefill_res_mid", v)
+        out.append(_rows(wk, toks, s["vocab"])[1])
+    ok, why = _agree(*out)
+    assert ok, why
+    print("T=%d the same bits: %s" % (T, np.array_equal(*out)))
     wk.close()
 
 
@@ -240,7 +265,7 @@ def test_prompts_of_models_with_a_matrix_of_128_columns(shape, T):
 @pytest.mark.parametrize("kvd", [dt.F16, dt.Q8_B32T2], ids=["f16", "q8"])
 def test_batched_steps_of_many_queries_agree_with_the_rows_products_and_replay(kvd, n):
     """the same products in a batched step: against rows_few = 0, and the captured step replayed with other work between the replays gives the eager step's tokens"""
-    wk, s = _biased(kvd, dt.Q4_B32T1A, 32, dim=1024, heads=8, kv_heads=8, head_dim=128, ffn=2816)
+    wk, s = _biased(kvd, dt.Q4_B32T1A, 32, norms=False, dim=1024, heads=8, kv_heads=8, head_dim=128, ffn=2816)
     V = s["vocab"]
     wk.kv_slots(n)
     rng = np.random.default_rng(n)
@@ -253,7 +278,7 @@ def test_batched_steps_of_many_queries_agree_with_the_rows_products_and_replay(k
         tok = wk.decode_batch(new, pos, slots, lg)
         out[v] = g.host(lg).astype(np.float32)
     ok, why = _agree(out[1], out[0])
-    assert ok, why
+    assert ok and not np.array_equal(out[1], out[0]), why
     for _ in range(4):
         assert [int(t) for t in wk.decode_batch(new, pos, slots)] == [int(t) for t in tok]
         wk.decode_batch(new[:4], pos[:4], slots[:4]); torch.cuda.synchronize()
