@@ -194,7 +194,7 @@ bool rows_few_ok(ifa_model *m, int T)
         const int most = few_max_rows(D, F);
         const size_t nx = few_frag_bytes(most, D), nf = few_frag_bytes(most, F), ns = (size_t)FEW_PARTS * most * D * sizeof(float);
         char *p = nullptr;
-        if (hipMalloc((void **)&p, nx + nf + ns) != hipSuccess) { (void)hipGetLastError(); m->opt_rows_few = 0; return false; }
+        if (m->opt_debug_mo_alloc_fail == 3 || hipMalloc((void **)&p, nx + nf + ns) != hipSuccess) { (void)hipGetLastError(); m->opt_rows_few = 0; return false; }
         m->few = {(half_t *)p, (half_t *)(p + nx), (float *)(p + nx + nf)};
     }
     return true;

@@ -221,7 +221,7 @@ struct ifa_model {
     int opt_rows_few = 1;
     struct { half_t *x, *ff; float *sums; } few = {nullptr, nullptr, nullptr};
     int opt_rows_kparts = 1, opt_gemm_splitk = 1;   // 0: never the launches whose workgroups wait for partner workgroups (K parts of the 9..32-row GEMM, split-K halves of the large-tile GEMM)
-    int opt_debug_mo_alloc_fail = 0;           // tests: ensure_mo_build fails like an exhausted allocator after its first copy (2: of copies with MO_WORDS only)
+    int opt_debug_mo_alloc_fail = 0;           // tests: ensure_mo_build fails like an exhausted allocator after its first copy (2: of copies with MO_WORDS only; 3: not there, but gemm_few's workspace)
     bool mo_built = false, mo_no_words = false;          // every matrix that has an operand-order copy has it; there was no memory for MO_WORDS copies
     static constexpr int RING = 1024;
 };

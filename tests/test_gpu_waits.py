@@ -73,13 +73,17 @@ def test_only_copies_that_products_of_many_rows_read_hold_their_words_twice():
         wk.close()
 
 
+@pytest.mark.parametrize("fail", [2, 3])
 @pytest.mark.parametrize("n", [12, 20])
-def test_without_memory_for_the_words_by_supersteps_the_rows_products_keep_their_copies(n):
-    """(simulated: debug_mo_alloc_fail 2) batched steps run as with rows_few 0, prompts as with prefill_mid 0, bit for bit: the copies without these words serve the rows products"""
+def test_without_memory_for_the_words_by_supersteps_or_the_workspace_the_other_products_serve(n, fail):
+    """(simulated: debug_mo_alloc_fail) 2, copies without the words by supersteps: batched steps run as with rows_few 0, prompts as with prefill_mid 0 beside it, bit for bit;
+    3, no workspace for gemm_few: as with rows_few 0"""
     shape = dict(dim=1024, heads=16, kv_heads=2, head_dim=64, ffn=1408)
     wk, ref = (synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=256, layers=2, vocab=600, quant_threshold=0, **shape)[0] for _ in range(2))
-    wk.set_option("debug_mo_alloc_fail", 2)
-    ref.set_option("rows_few", 0); ref.set_option("prefill_mid", 0)
+    wk.set_option("debug_mo_alloc_fail", fail)
+    ref.set_option("rows_few", 0)
+    if fail == 2:
+        ref.set_option("prefill_mid", 0)
     out = []
     for w in (wk, ref):
         w.kv_slots(n)
@@ -93,7 +97,7 @@ def test_without_memory_for_the_words_by_supersteps_the_rows_products_keep_their
             w.forward(np.arange(3, 3 + T).astype(np.int32), 0, pl)
             rows.append(g.host(pl).copy())
         out.append((tok, rows))
-    assert wk.buffer("rows_copy")[1] == 64 * 1024 * (8 + 2) and ref.buffer("rows_copy")[1] == 64 * 1024 * (8 + 2 * 2)
+    assert wk.buffer("rows_copy")[1] == 64 * 1024 * (8 + (2 if fail == 2 else 4)) and ref.buffer("rows_copy")[1] == 64 * 1024 * (8 + 2 * 2)
     assert all(list(a) == list(b) for a, b in zip(out[0][0], out[1][0]))
     assert all(np.array_equal(a, b) for a, b in zip(out[0][1], out[1][1]))
     wk.close(); ref.close()
