@@ -11,6 +11,8 @@ mins = [int(v) for v in os.environ.get("IFA_BIG_MINS", "128,47").split(",")]
 OPT = os.environ.get("IFA_AB_OPTION", "prefill_big_min")      # the option whose values IFA_BIG_MINS lists (e.g. prefill_chunk with 0,1)
 wk, _, s = synth.build(os.environ.get("IFA_SHAPE", "llama2_7b"), dt.Q4_B32T1A, dt.F16, max_ctx=max(lens) + 8)
 V = s["vocab"]
+if OPT in ("prefill_big_min", "prefill_chunk"):          # (what serves these lengths in front of them)
+    wk.set_option("rows_few", 0); wk.set_option("prefill_mid", 0)
 for T in lens:
     toks = np.random.default_rng(T).integers(3, V, T).astype(np.int32)
     out = {}

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Prompts of 33..64 tokens: two passes of the rows GEMM (prefill_chunk) against the mid-size GEMM route (prefill_big_min lowered), one box."""
+"""Prompts of 33..64 tokens: the products over few rows (default), the mid-size GEMM (rows_few 0), two passes of the rows GEMM or the large tiles (prefill_mid 0 beside it), one box."""
 import os, sys, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import numpy as np, torch
@@ -8,8 +8,8 @@ wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=128)
 for T in (33, 34, 40, 47, 48, 56, 64):
     toks = np.random.default_rng(T).integers(3, s["vocab"], T).astype(np.int32)
     res = []
-    for name, opts in (("default", {}), ("mid from 33", {"prefill_chunk": 0, "prefill_big_min": 32})):
-        wk.set_option("prefill_chunk", 1); wk.set_option("prefill_big_min", 47)
+    for name, opts in (("few", {}), ("mid", {"rows_few": 0}), ("two passes / large", {"rows_few": 0, "prefill_mid": 0})):
+        wk.set_option("rows_few", 1); wk.set_option("prefill_mid", 1)
         for k, v in opts.items(): wk.set_option(k, v)
         wk.reset(); tok = wk.forward(toks, 0)
         torch.cuda.synchronize(); t0 = time.perf_counter()
