@@ -163,9 +163,8 @@ int layer_tail_ops(ifa_model *m, int l, int T, half_t *&x, const half_t *attn_in
 }
 
 // no_head: a chunk of a longer prompt that is not its last one -- the layers only (KV cache rows written), no lm_head / argmax / sync
-// 33 .. prefill_mid_max tokens through k_gemm_mid (csrc/ifa_gemm_mid.hip): the large-tile route's conditions + an operand-order copy of
-// every linear (built here on first use).  From 33 tokens on: 5.3 ms for 33..48 tokens against 5.9-6.6 for two passes of the rows
-// GEMM (tools/short_prompt_routes.py, profiles/r06_prefill_mid_parts.log)
+// 33 .. prefill_mid_max tokens through k_gemm_mid (csrc/ifa_gemm_mid.hip), where gemm_few does not take them: the large-tile route's conditions + an operand-order copy
+// with the words by supersteps of every linear (built here on first use).  From 33 tokens on: faster than two passes of the rows GEMM (tools/short_prompt_routes.py)
 bool prefill_mid_ok(ifa_model *m, int T, bool any_length)
 {
     const ifa_model_config &c = m->cfg;
@@ -279,12 +278,13 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
     // prompts every one of them is a fixed ~5 us)
     const bool seq_wiring = !c.parallel_attn && !c.share_input;
     bool xn_ready = false;           // m->xn already holds the next norm's output (fused into the previous layer's last Add)
-    // prompts of 2..16 tokens on a dense Q4 model with the sequential RMS wiring: the linears of a layer as FOUR launches of
-    // the rows GEMM (ifa_gemm_rows_mfma.hip) -- norm prologue + wq | wk | wv into q / k / v, wo + residual, norm + w1 / w3 +
-    // GLU, w2 + residual -- instead of seven products and four element-wise launches (9..16 tokens: the norms stay launches)
-    // Prompts above `prefill_big_min` tokens (47; round 4: 128) take the same four launches per layer from the large-tile GEMM (ifa_gemm.hip, k_gemm_big: the
-    // weights dequantised once per workgroup and step into LDS; reference-layout rows), norms as their own launches.
-    // the mid-length kernel (33 .. prefill_mid_max tokens): every linear of every layer a 4-bit tensor with its operand-order copy, dense FFN
+    // Prompts on a dense Q4 model with the sequential RMS wiring: the linears of a layer as FOUR launches -- wq | wk | wv into q / k / v, wo + residual, w1 / w3 + GLU, w2 + residual --
+    // instead of seven products and four element-wise launches:
+    //   2..8 tokens (32 where gemm_few does not take them): the rows GEMM (ifa_gemm_rows_mfma.hip), up to 16 tokens with the norms inside;
+    //   FEW_MIN .. few_max_rows tokens: gemm_few (ifa_gemm_few.hip), the residuals added with the norm behind them;
+    //   beyond, to prefill_mid_max: k_gemm_mid (ifa_gemm_mid.hip), every linear of every layer a 4-bit tensor with its operand-order copy;
+    //   else above `prefill_big_min` tokens: the large-tile GEMM (ifa_gemm.hip, k_gemm_big: the weights dequantised once per workgroup and step into LDS; reference-layout rows).
+    // Norms that are not inside are launches of their own.
     const bool pstat = m->opt_perf_stat != 0;       // per-phase times: the op-by-op layer below (one launch per reference op), never the fused routes
     // FEW_MIN .. few_max_rows tokens: gemm_few, behind the switches of the products that it takes over
     const bool pf_few = !tp && !pstat && (T <= 32 ? m->opt_batch_fused && m->opt_gemm_rows && gemm_rows_use_mfma() : m->opt_prefill_mid) && rows_few_ok(m, T);
@@ -705,7 +705,7 @@ int forward_batch(ifa_model *m, int n, const int *tokens_host, const int *pos_ho
         int rcm = ensure_mo(m); if (rcm) return rcm;
         // ensure_mo may have DOWNGRADED the model (the copies did not fit: opt_rows_mo = 0): what batch_fused_ok answered with the
         // copies in view -- up to 32 rows, the 64-weight formats -- no longer holds, so it is asked again before a path or a graph
-        // is chosen; a step the tiled kernels do not cover takes the op-by-op rows below (ADVICE r4)
+        // is chosen; a step the tiled kernels do not cover takes the op-by-op rows below
         fused = batch_fused_ok(m, n);
         if (fused && (rcm = gemm_rows_kparts_reserve(m->stream))) return rcm;
         few = fused && rows_few_ok(m, n);      // (and its workspace, before a capture)
@@ -830,7 +830,7 @@ int ifa_model_forward(ifa_model *m, const int *tokens_host, int n_tokens, int pr
         }
         return IFA_OK;
     }
-    // Round 5: prompts of 34..48 tokens as TWO passes of the rows GEMM (32 tokens, then 2..16: the weights stream into registers five
+    // Prompts of 34..48 tokens that neither gemm_few nor k_gemm_mid takes, as TWO passes of the rows GEMM (32 tokens, then 2..16: the weights stream into registers five
     // groups deep) instead of one pass of the op-by-op layer: 40 tokens 7.08 -> 6.35 ms, 48 tokens 7.26 -> 6.67 (profiles/r05_prompt_lengths.log;
     // two passes of 17..32 rows each -- 49..64 tokens -- measured no faster than the tile kernels).  The second pass reads the first
     // one's K / V rows from the cache like any continued prompt; every row goes through the kernels of a prompt of <= 32 tokens.  Never

@@ -205,14 +205,16 @@ struct ifa_model {
     // debug_layers = N: layers [layer0, layer0 + N)) and, with debug_hidden_in, takes its input from the buffer "x" as the caller
     // left it instead of gathering the token's embedding row -- the SAME captured launches the bench times, fed the oracle's state
     int opt_debug_layer0 = 0, opt_debug_hidden_in = 0;
-    // prompts ABOVE this many tokens take the four large-tile launches per layer (forward_ops, pf_big).  Round 4: 128.  Round 5: 47 -- with
+    // prompts ABOVE this many tokens that nothing below takes go through the four large-tile launches per layer (forward_ops, pf_big): with
     // four parts of K for the products that offer 32..96 tiles, 64 / 96 / 128 tokens run 5 / 8 / 9 % faster than the op-by-op layer
     // (7 products + 4 element-wise launches), 40 tokens the same (profiles/r05_prompt_lengths.log)
     int opt_prefill_big_min = 47;
-    int opt_prefill_chunk = 1;      // prompts of 34..48 tokens as two passes of <= 32 tokens (ifa_model_forward)
-    // prompts of 33 .. prefill_mid_max tokens take the four launches per layer from k_gemm_mid (ifa_gemm_mid.hip: ring of
+    int opt_prefill_chunk = 1;      // prompts of 34..48 tokens that nothing below takes as two passes of <= 32 tokens (ifa_model_forward)
+    // prompts of 33 .. prefill_mid_max tokens that gemm_few does not take have the four launches per layer from k_gemm_mid (ifa_gemm_mid.hip: ring of
     // direct-to-LDS stages requested by loader waves, weights dequantised into the MFMA operand registers) when every linear has its
-    // operand-order copy.  A layer's four products, Llama-2-7B, us, through the large tiles (wo / w2 of up to 2048 tokens already through k_gemm_mid) and here:
+    // operand-order copy.  Of other widths, us, large tiles / through it, 1024, 2048, 4096, 8192 tokens: four layers of 256 351, 437, 648, 1255 / 345, 430, 660, 1281; of 512 389,
+    // 536, 845, 1517 / 390, 546, 822, 1575; of 768 432, 636, 1195, 2726 / 409, 661, 1184, 2830 (3000 tokens 558, 718, 916 / 541, 681, 828); two layers of 1024 258, 374, 686, 1525 / 250, 344, 652,
+    // 1471; of 4096 x 14336 1187, 2251, 4393, 9971 / 1092, 2163, 4324, 9878; of 8192 x 28672 3837, 7507, 14810, 32088 / 3505, 6976, 14387, 31941.  A layer's four products, Llama-2-7B, us, through the large tiles (wo / w2 of up to 2048 tokens already through k_gemm_mid) and here:
     // 800 tokens 462 and 399, 1024 484 and 437, 1300 780 and 645, 1536 785 and 687, 2048 878 and 837, 3000 1362 and 1266, 4096 1642 and 1591, 6000 2622 and 2377, 8192 3161 and 3156
     int opt_prefill_mid = 1, opt_prefill_mid_max = 8192;
     int opt_prefill_res_mid = 2048;   // prefill_mid_max + 1 .. this many tokens (where prefill_mid_max was lowered): wo / w2 still through k_gemm_mid, the other products through the large tiles (0: never)

@@ -17,8 +17,8 @@ int gemm_splitk_scratch(hipStream_t s, size_t part_bytes, size_t tiles, void **o
 bool gemm_big_ok(int w_dtype, const GmArgs &P, int epi);
 int gemm_big(int w_dtype, const GmArgs &P, int epi, hipStream_t s);
 
-// Prompts of 33..512 tokens (ifa_gemm_mid.hip, k_gemm_mid): 128 x 128 tiles, weights in the MO layout (Tensor::mo, P.mo = MO_WORDS),
-// everything global -> LDS through a ring of direct-to-LDS stages, the weights dequantised from their raw bytes straight into
+// Prompts of 33 tokens and more (ifa_gemm_mid.hip, k_gemm_mid): 128 x 128 tiles, weights in the MO layout (Tensor::mo, P.mo = MO_WORDS),
+// activations through a ring of direct-to-LDS stages, the weights dequantised from their raw bytes straight into
 // the MFMA operand registers.  Same products, summation order over K and epilogues as gemm_big's 128 x 128 tiles.
 constexpr size_t MID_MIN_COLS = 256;      // columns of every matrix (four steps)
 bool gemm_mid_ok(int w_dtype, const GmArgs &P, int epi);

@@ -1,4 +1,4 @@
-// ifa_gemm_mid.hip -- the linear layers of prompts from 193 tokens on (shorter ones: ifa_gemm_few.hip):  Y[T][N] = X[T][K] . W[N][K]^T  (+ bias, residual, GLU)
+// ifa_gemm_mid.hip -- the linear layers of prompts from 193 tokens on (97 in wide models, 33 where a matrix is not for ifa_gemm_few.hip, which takes the shorter ones):  Y[T][N] = X[T][K] . W[N][K]^T  (+ bias, residual, GLU)
 //
 // Reference: MatrixMultiplication (src/transformer/inference_worker.cc:2364-2432): Dequantize the weight tensor to F16, F16 x F16
 // product with fp32 accumulation (src/tensor/cublas_engine.cu:420-436).  Same values here: every weight is half(fma(q, scale,
@@ -7,9 +7,8 @@
 //
 // Why a second kernel.  k_gemm_big stages the activation tile with direct-to-LDS loads and reads its MFMA operands with
 // ordinary LDS loads; hipcc puts `s_waitcnt vmcnt(0)` in front of every LDS read that follows a direct-to-LDS request, so every
-// 64-column step ends up waiting for the requests it has just issued: a step is one memory round trip (~1 us; rocprofv3 at 128
-// tokens: W1|W3 62 us for 64 steps, wq|wk|wv 35 us for 16) however little it multiplies.  Above ~512 tokens the step's MFMA work
-// covers that; below, a layer is 225 us for 126 MB of weights and 52 GFLOP.  Here:
+// 64-column step ends up waiting for the requests it has just issued: a step is one memory round trip (~1 us; a 128-token prompt's
+// w1 | w3 62 us for 64 steps, wq | wk | wv 35 us for 16) however little it multiplies.  Here:
 //   * activations go through direct-to-LDS loads into a ring of four stages (128 x 64 halves), requested by four waves that do nothing else, waited for with a
 //     COUNTED vmcnt; the raw weight codes, which only one wave reads, go straight to its registers, two steps ahead;
 //   * every LDS read of the loop is inline assembly (the compiler sees no LDS access to protect), waited for with lgkmcnt where
@@ -21,9 +20,10 @@
 //     asked for in this one.  Codes through the ring and a step that began with 19 LDS reads (its conversion and first wait in front of its first product), 140
 //     instructions a step, two workgroups on a compute unit to hide that, against 100 instructions and one workgroup, ms a prompt of 193, 300, 512, 600, 768, 2048 tokens,
 //     Llama-2-7B: 6.13, 8.78, 9.81, 12.6, 15.0, 33.75 -> 5.74, 8.21, 9.32, 11.5, 13.8, 33.4.
-// What bounds it: power.  In the loop the clock falls to 1.55 - 1.8 GHz; a step takes 740 - 800 cycles, 512 of them products, 1.25 PFLOP/s in all.  So what converts a weight more often to
-// read LDS less or to keep a SIMD busier does not pay: waves of 64 rows x 64 tokens (half the fragment reads) took 3 - 7 % longer than the form before, eight computing waves of 32 x 64
-// 8 % longer than this one.
+// What bounds it: in the loop power, beside it the ends of the tiles.  Over whole launches the clock is 1.65 - 1.9 GHz (profiles/prompt_products_clock.txt; attention beside
+// them 2.2); a step takes 740 - 800 cycles, 512 of them products, 1.25 PFLOP/s in the loop.  So what converts a weight more often to read LDS less or to keep a SIMD busier does not pay: waves of
+// 64 rows x 64 tokens (half the fragment reads) took 3 - 7 % longer than the form before, eight computing waves of 32 x 64 8 % longer than this one.  With one workgroup on a compute unit nothing
+// runs under a tile's last sums and its output: the gated pair's 7 us an end are 75 of the 379 us of 2048 tokens (2752 tiles, 10.75 rounds) and 20 of the 109 of 512, 0.97 PFLOP/s in all.
 // Weights: the MO copy of the rows GEMM (ifa_gemm_rows_mfma.h; Q4_B32T1A / B and the 64-weight nibble formats): a 16-row tile's K range
 // is one linear stream of 1 KiB supersteps.
 #include <algorithm>
@@ -60,7 +60,7 @@ __device__ __forceinline__ void md_each(F f) { if constexpr (I < N) { f(std::int
 
 // EPI: GM_PLAIN | GM_RESIDUAL | GM_GLU (a weight tile = 64 rows of w1 and the same 64 rows of w3).  KS: parts of K (workgroups per
 // tile).  TA: 32-token accumulator tiles of a wave -- the tile is 32 TA tokens x 128 weight rows (TA = 2 up to 64 tokens: half of the products, fragment reads,
-// activation requests and exchanged sums of a 128-row tile whose lower half repeats a row -- 37 tokens 4.67 -> 3.83 ms, the same bits; TA = 8: md_wide).
+// activation requests and exchanged sums of a 128-row tile whose lower half repeats a row, the same bits -- where gemm_few does not take such prompts; TA = 8: md_wide).
 template <int EPI, int KS, int TA>
 __global__ void __launch_bounds__(MD_THREADS, 2) k_gemm_mid(const GmArgs P, const BigGeo G)
 {
