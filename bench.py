@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Headline benchmark: greedy batch-1 decode of a Llama-2-7B-shaped model with
-Q4_B32T1A weights (BASELINE.json configs[1]) on N MI355X GPUs.
+Q4_B32T1A weights on N MI355X GPUs.
 
     python bench.py --gpus N --steps K --warmup W
 
@@ -21,7 +21,7 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-HBM_PEAK_GBPS = 8000.0      # MI355X spec (MI355X_MICROARCH.md)
+HBM_PEAK_GBPS = 8000.0      # MI355X spec
 PROMPT_LEN = 16
 
 
@@ -130,7 +130,7 @@ def reference_cpu_baseline(n_tokens=128):
         gpu_tok_s = n_tokens / (time.perf_counter() - t0)
         eng.close()
         return {"value": ref_tok_s, "unit": "tokens/s", "cores": threads, "kind": "reference",
-                "sample": "the reference's CPU path (oracle/_ref/ifa_ref_engine) on a stories15M-shaped llama2.c checkpoint (configs[0]: "
+                "sample": "the reference's CPU path (oracle/_ref/ifa_ref_engine) on a stories15M-shaped llama2.c checkpoint ("
                           "d 288, 6 layers, vocab 32000, F32 weights), %d-token prompt + %d greedy tokens, cpu_threads %d; prefill %.1f ms"
                           % (PROMPT_LEN, n_tokens, threads, r["prefill_ms"]),
                 "gpu_same_checkpoint_tok_s": gpu_tok_s}
@@ -187,7 +187,7 @@ def pick_reference_layers(avail_gb=None, disk_gb=None):
 
 
 def reference_cpu_baseline_7b_width(n_tokens=16, layers=32, with_gpu=True):
-    """The reference's CPU path on the HEADLINE model (SURVEY 8d "C2-shaped weights, >= 16 tokens"): a Llama-2-7B
+    """The reference's CPU path on the HEADLINE model: a Llama-2-7B
     llama2.c checkpoint of `layers` layers (F32 weights: what its CPU side runs; all 32 layers = the headline model, a 27 GB file)
     with this engine on the same file (Q4 weights, F16 KV cache: the headline formats) next to it.  Machine-readable: "layers",
     "model_layers", "full_model", "bytes_per_token"."""
@@ -364,7 +364,7 @@ def loopback_line(args):
            "config": {"workload": "%s decode through the .ini surface, %d tensor-parallel ranks on ONE device" % (args.shape, R),
                       "parallelism": "tp%d loopback (one process, %d worker threads, in-process group instead of RCCL; partition_ranks = %d)" % (R, R, ranks),
                       "collectives": "loopback group (csrc/ifa_comm.hip LocalGroup): same slicing, merges and step logic as the RCCL path"},
-           "note": "functional check of the N > 1 path on a one-GPU box: R ranks share the device, so this is not a scaling number",
+           "note": "functional check of the N > 1 path on one GPU: R ranks share the device, so this is not a scaling number",
            "last_tokens": [int(t) for t in gen[-4:]]}
     os.dup2(saved, 1)
     print(json.dumps(out), flush=True)
@@ -597,7 +597,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=16)
     ap.add_argument("--shape", default="llama2_7b")
     ap.add_argument("--wdtype", default="q4", help="weight format: q4 (Q4_B32T1A, the headline config), q3h, q8, q4_b64, q5, q6")
-    ap.add_argument("--kv-dtype", default="f16", help="KV cache: f16 or q8 (configs[2] = --wdtype q3h --kv-dtype q8)")
+    ap.add_argument("--kv-dtype", default="f16", help="KV cache: f16 or q8 (--wdtype q3h --kv-dtype q8: 3.5-bit weights, 8-bit cache)")
     ap.add_argument("--groups", type=int, default=1, help="device groups (layer ranges) of the HYBRID partition; "
                     "gpus // groups ranks per group are tensor-parallel (default 1 = pure tensor parallelism)")
     ap.add_argument("--prefill-lens", default="128,1024", help="extra prompt lengths whose prefill rate is reported (N=1 only)")
@@ -605,7 +605,7 @@ def main():
                     "step (N=1 only; reported as batch_decode, never as value; 0 = skip)")
     ap.add_argument("--loopback", type=int, default=0, help="R > 1: run the tensor-parallel partition with R ranks on ONE device "
                     "(the C++ InferenceEngine with devices = 0&0..., in-process loopback group instead of RCCL) and print its line; "
-                    "a functional check of the N > 1 step logic on a one-GPU box, not a scaling number")
+                    "a functional check of the N > 1 step logic on one GPU, not a scaling number")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-tokens", type=int, default=0, help="CPU baseline sample size (0 = auto)")
     ap.add_argument("--arch", default="", help="'gelarax', 'muzopel', 'sopulorn', 'bogupel', 'kamelorn' or 'rosilix': instead of the headline workload, prefill / decode rates of models of that design beside the "
@@ -767,7 +767,7 @@ def main():
 
     tok_s = steps / wall
     n_avg = PROMPT_LEN + warmup + steps / 2.0
-    # ALGORITHMIC bytes (the reference's own block sizes -- Q3H_B64T1 is 32 B per 64 weights) are what every roofline
+    # ALGORITHMIC bytes (the reference's own block sizes: Q3H_B64T1 is 32 B per 64 weights) are what every roofline
     # figure of this line is computed on; the bytes the decode kernels actually stream are reported beside them (they differ for
     # Q3H_B64T1 only: its pair codes are expanded to nibbles at load time, 36 B per 64 weights -- 1.125x wasted traffic by construction)
     w_bytes = synth.weight_bytes(args.shape, wd, streamed=False)
@@ -828,7 +828,7 @@ def main():
             from inferflow_amd.build import source_hash
             import glob
             pmc_path = sorted(glob.glob(os.path.join(ROOT, "profiles", "r*_pmc_traffic.json")))[-1]        # the newest round's
-            if wd == dt.Q3H_B64T1:          # configs[2]: its own PMC pass (tools/profile_r05.sh)
+            if wd == dt.Q3H_B64T1:          # 3.5-bit weights: their own PMC pass (tools/profile_r05.sh)
                 q = sorted(glob.glob(os.path.join(ROOT, "profiles", "r*_pmc_q3h_q8_traffic.json")))
                 pmc_path = q[-1] if q else pmc_path
             pmc = json.load(open(pmc_path))
@@ -851,7 +851,7 @@ def main():
                            "frac": ffn13_bytes / us / 1e3 / HBM_PEAK_GBPS, "traffic": traffic, "traffic_note": traffic_note, "traffic_source": traffic_source,
                            "bytes_per_launch": ffn13_bytes, "streamed_bytes_per_launch": ffn13_streamed, "us_per_launch": us}
         out["kernels"] = per_kernel
-    # ---- prefill rate at longer prompts (16 / 128 / 1024-token prompts), outside the timed decode region
+    # ---- prefill rate at longer prompts, outside the timed decode region
     if world == 1 and hasattr(runner, "worker") and not os.environ.get("IFA_FORCE_TP"):
         pf = {}
         out["prefill_tok_s_first_call"] = PROMPT_LEN / prefill_s   # cold: code objects, scratch and KV pages touched for the first time
@@ -969,7 +969,7 @@ def main():
             out["cpu_baseline_port"] = {"value": None, "unit": "tokens/s", "cores": 0, "kind": "port",
                                         "sample": "failed: %r" % (e,)}
     # ---- the REFERENCE's own CPU path (oracle/_ref/ifa_ref_engine: /root/reference sources compiled by oracle/Makefile,
-    # travels prebuilt) on configs[0] -- the stories15M-shaped llama2.c checkpoint of bin/llm_inference.tiny.ini, the case
+    # travels prebuilt) on the stories15M-shaped llama2.c checkpoint of bin/llm_inference.tiny.ini, the case
     # the reference itself runs on CPU -- with this engine on the very same checkpoint next to it
     if world == 1 and not args.no_cpu_baseline and not os.environ.get("IFA_FORCE_TP"):
         try:
@@ -978,13 +978,13 @@ def main():
             out["cpu_baseline_reference"] = {"value": None, "unit": "tokens/s", "cores": 0, "kind": "reference", "sample": "failed: %r" % (e,)}
         if args.shape == "llama2_7b":
             # the reference on the HEADLINE model: all 32 layers when the host can hold the 27 GB F32 checkpoint (pick_reference_layers),
-            # else the largest slice that fits -- and the 8-layer slice of round 4 as its own line either way
+            # else the largest slice that fits -- and the 8-layer slice as its own line either way
             n_ref = int(os.environ.get("IFA_BENCH_REF_LAYERS", "-1"))
             forced = n_ref >= 0
             if n_ref < 0:
                 n_ref = pick_reference_layers()
             budget_s = float(os.environ.get("IFA_BENCH_REF_BUDGET_S", "240"))
-            # the 8-layer slice first (round 4's line, kept as its own key): what it took also says what all 32 layers will take on
+            # the 8-layer slice first (kept as its own key): what it took also says what all 32 layers will take on
             # this host (file write + load + decode scale with the layer count) -- the default run must stay inside a few minutes
             t8 = None
             if n_ref >= 8 and not os.environ.get("IFA_BENCH_SKIP_8_LAYERS"):
@@ -1012,8 +1012,8 @@ def main():
             else:
                 out["cpu_baseline_reference_7b"] = {"value": None, "unit": "tokens/s", "cores": 0, "kind": "reference", "layers": 0,
                                                     "sample": "not run: %.0f GB of host memory available, the 8-layer checkpoint needs ~15" % _host_avail_gb()}
-    # cpu_baseline (the contract's key) is ALWAYS on the headline workload -- all 32 layers of the model the GPU number is quoted on
-    # (ADVICE r4): the REFERENCE's own CPU path when the host could hold the full checkpoint (kind "reference", "full_model": true,
+    # cpu_baseline (the contract's key) is ALWAYS on the headline workload -- all 32 layers of the model the GPU number is quoted on:
+    # the REFERENCE's own CPU path when the host could hold the full checkpoint (kind "reference", "full_model": true,
     # F32 weights: what that path runs), else the oracle port of the quantised path on the whole model (kind "port").  A slice of
     # the model is never put under this key; slices keep their own keys with a machine-readable "layers" field.
     r7 = out.get("cpu_baseline_reference_7b") or {}

@@ -2,7 +2,7 @@
  * inferflow_amd.h -- C ABI of the MI355X-native quantized decode path.
  *
  * This is the drop-in boundary for the lower surface that Inferflow's
- * GpuInferenceWorker calls (SURVEY.md §8b):
+ * GpuInferenceWorker calls:
  *   TensorOpr::*      src/tensor/tensor_opr.h:33-131
  *   TensorMul::*      src/tensor/tensor_mul.h:14-57
  *   CublasEngine      src/tensor/cublas_engine.h:31-33
@@ -128,7 +128,7 @@ int ifa_inlaunch_waits_enabled(void);
 int ifa_gemm_release_stream(ifa_stream stream);
 
 /* Re-tile reference-layout rows into the row-local plane layout the fused
- * decode kernels stream (DESIGN.md "HBM layout"): same bytes per row, row stride
+ * decode kernels stream: same bytes per row, row stride
  * padded to a multiple of 16 (ifa_tiled_row_bytes; 0 for types without a tiled
  * layout).  Supported for the AX8-eligible types; src and dst must not alias;
  * dst holds rows * ifa_tiled_row_bytes(dtype, cols) bytes. */
@@ -355,7 +355,7 @@ int ifa_comm_init_rank(const void *id_128, int nranks, int rank, int device, ifa
 int ifa_comm_init_all(const int *device_ids, int n, ifa_comm **comms_out);
 /* a device list that names ONE device n times makes an in-process loopback group instead (RCCL refuses two ranks on a
  * device): kernels / copies on that device with a host rendezvous between the rank threads -- host-synchronous, not
- * capturable (ifa_comm_capturable() == 0); for exercising the multi-rank paths on a 1-GPU box */
+ * capturable (ifa_comm_capturable() == 0); for exercising the multi-rank paths on one GPU */
 int ifa_comm_capturable(const ifa_comm *c);
 /* identity of the communicator OBJECT (a new one at the same address gets a new serial): what a cached, captured step
  * is keyed on */
@@ -430,7 +430,7 @@ typedef struct {
     int stage, n_stages;   /* BY_LAYER / HYBRID: this worker's device group, number of groups (1 = BY_TENSOR only) */
     int prev_rank, next_rank, token_src;   /* ranks in `world`; -1 = none */
     int vocab_offset;      /* first vocabulary row of this rank's lm_head shard */
-    int force_collectives; /* issue the collectives even in a group of one (plumbing check on a 1-GPU box) */
+    int force_collectives; /* issue the collectives even in a group of one (plumbing check on one GPU) */
 } ifa_tp_topology;
 int ifa_model_tp_decode(ifa_model *m, const ifa_tp_topology *topo, int first_token, int start_pos, int n_steps,
                         int *out_tokens_host, float *elapsed_ms);

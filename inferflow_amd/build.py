@@ -1,7 +1,7 @@
 """Builds inferflow_amd/lib/libinferflow_amd.so (HIP kernels + C ABI) for gfx950.
 
 hipcc cross-compiles without a GPU, so this runs in the build container; the
-resulting .so is git-ignored but travels to the GPU box with the tree.
+resulting .so is git-ignored but travels to where the GPU is with the tree.
 """
 import glob
 import os
@@ -17,7 +17,7 @@ ARCH = "gfx950"
 
 HIPCC_FLAGS = [
     "--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC",
-    # exact-rounding parity with the host-compiled reference codecs (DESIGN.md)
+    # exact-rounding parity with the host-compiled reference codecs
     "-ffp-contract=off",
     # no packed fp32 instructions (v_pk_add / mul / fma_f32) from ordinary float code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -1,6 +1,6 @@
 // ifa_comm.hip -- collectives of the multi-GPU partitions behind the C ABI (RCCL over xGMI).
 //
-// What they replace in the reference (SURVEY.md 8a a17, 8b): the host-driven exchange of
+// What they replace in the reference: the host-driven exchange of
 // GpuInferenceWorker::DistributeAndMergeTensors / MergeTensors / DeviceCopy
 // (src/transformer/inference_worker.cc:2148-2335) over GpuInfGlobalData's mutex + 1 us sleeps
 // (src/transformer/gpu_inf_global_data.cu:25-199):
@@ -16,7 +16,7 @@
 //   * one process, one host thread per GPU (the C++ InferenceEngine, like the reference's one sslib::Thread per
 //     GPU, inference_engine.cc:1203-1206): ifa_comm_init_all creates the communicators of all ranks at once.
 //
-// Loopback groups: RCCL refuses a communicator with two ranks on one device, which is all a 1-GPU box can offer.  When
+// Loopback groups: RCCL refuses a communicator with two ranks on one device, which is all that one GPU can offer.  When
 // ifa_comm_init_all is given a device list with duplicates, the ranks become an in-process group whose collectives are
 // plain kernels / copies on that device with a host rendezvous between the rank threads (host-synchronous, not
 // capturable: ifa_comm_capturable() == 0).  Same results by construction (sums in half, rank order); it exists so that
@@ -239,7 +239,7 @@ int ifa_comm_init_rank(const void *id_128, int nranks, int rank, int device, ifa
 // One process per rank (ifa_comm_init_rank): the one-shot exchange needs the peers' inboxes and flags mapped into this process.
 // Inboxes, flags and counters are FINE-GRAINED device memory: kernels on different GPUs signal each other through them while
 // they run, and the HSA memory model only promises cross-agent visibility of coarse-grained (plain hipMalloc) memory at
-// dispatch boundaries -- a fresh flag next to a stale payload would be a silently wrong sum (ADVICE r3).
+// dispatch boundaries -- a fresh flag next to a stale payload would be a silently wrong sum.
 static hipError_t oneshot_alloc(void **p, size_t bytes)
 {
     return hipExtMallocWithFlags(p, bytes, hipDeviceMallocFinegrained);
@@ -247,7 +247,7 @@ static hipError_t oneshot_alloc(void **p, size_t bytes)
 
 // In-kernel visibility probe between two devices: the reader spins (bounded) on a word of ITS OWN device's flag area while the
 // writer, a kernel running on the OTHER device at the same time, stores the tag with system scope.  A host-side hipMemcpy
-// round trip (round 3's self-test) says nothing about what a running kernel sees.
+// round trip (as a first self-test had it) says nothing about what a running kernel sees.
 static __global__ void k_oneshot_probe_wait(const unsigned *word, unsigned tag, unsigned *seen, long long timeout_ticks)
 {
     const long long t_end = wall_clock64() + timeout_ticks;
@@ -396,7 +396,7 @@ int ifa_comm_init_all(const int *device_ids, int n, ifa_comm **comms_out)
     for (int i = 0; i < n; i++) {
         ifa_comm *c = new ifa_comm();
         c->comm = cs[(size_t)i]; c->rank = i; c->nranks = n; c->device = device_ids[i]; c->oneshot = os;
-        // The peer exchange has not run between two real devices yet (no multi-GPU box in four rounds): RCCL carries every
+        // The peer exchange has not run between two real devices yet (there was no machine with more than one): RCCL carries every
         // size until a caller switches it on (ifa_comm_set_oneshot) after checking a few steps against RCCL, as bench.py does
         c->no_oneshot = true;
         comms_out[i] = c;

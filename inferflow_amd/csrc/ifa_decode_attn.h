@@ -82,7 +82,7 @@ constexpr int DEC_ATTN_MIN_ROWS = 256;
 
 // Score chains per key.  The reference's Gemm_Alg2 adds a key's HD products as ONE fp32 chain in d order (gemm.h:83-178); this body
 // keeps that order by default (IFA_ATTN_NACC = 1): 128 dependent fma per key, the compiler pads the chain with a wait state per
-// step.  Round 5 measured the alternative SURVEY 8(c) allows (fp within tolerance): -DIFA_ATTN_NACC=4 sends the pairs
+// step.  Measured beside it, the same within tolerance only: -DIFA_ATTN_NACC=4 sends the pairs
 // (2 i, 2 i + 1) -- exactly as q and the key row hold them in memory -- through v_dot2_f32_f16 into four independent chains,
 // added as ((c0 + c1) + (c2 + c3)): 64 instructions per key instead of 128 + 128 wait states.  On MI355X the score phase of the
 // fused launch's attention tail went 0.76 -> 0.52 us (profiles/r05_attention_dot2_trace.log) -- 0.24 us of a 38 us layer,
@@ -122,7 +122,7 @@ struct ScoreAcc {
 // of 16-byte pieces): the K rows are requested like the V rows -- 16 bytes per lane, a wave instruction covers whole rows --
 // and transposed through an XOR-swizzled LDS tile into the one-key-per-lane registers of the score chain.  One key per lane
 // straight from memory is 64 different cache lines per wave instruction: the 256-row prefetch was 4096 line requests per
-// CU, ~1.7 us of the kernel before its first stamp (r04 trace: the score phase waited for K, the P.V phase for V).
+// CU, ~1.7 us of the kernel before its first stamp (trace: the score phase waited for K, the P.V phase for V).
 // FUSED (k_dec_qkv_attn, ifa_decode_qkv_attn.h): the body runs as the tail of the QKV launch on the first 256 threads of the
 // head's designated workgroup -- the new token's q | k | v values arrive as {epoch, half} granules written by the workgroups
 // that computed those rows (FusedIn), the position is already known (rows past it are not requested), head = `h_in`.
@@ -227,7 +227,7 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
         else return (kq16[B >> 1] >> (8 * (B & 1))) & 0xFFu;
     };
     // the new token's q / k / v values and this step's (cos, sin) pair FIRST: loads return in issue order, and behind the
-    // 128 KB of K / V rows below these few bytes arrived 1.5 us later than they had to (phase stamps, DESIGN.md)
+    // 128 KB of K / V rows below these few bytes arrived 1.5 us later than they had to (phase stamps)
     const int dq = min(tid, HD - 1);
     if constexpr (PHASE != 2) {
     q_in = (half_t)0; k_in = (half_t)0; v_in = (half_t)0;
@@ -508,7 +508,7 @@ __device__ __forceinline__ void dec_attn_body(char *smem, const half_t *pq, cons
             else acc_v(pj, vreg[i]);
         }
     }
-    // keys past the prefetched bucket (round 6, second session): batches of eight keys of this thread's sequence, the next batch
+    // keys past the prefetched bucket: batches of eight keys of this thread's sequence, the next batch
     // requested before the current one is multiplied (unconditional, clamped rows).  The loop asked for one V piece per iteration and
     // waited for it: a batched step at 2048 keys spent 96 us per layer in this kernel.  Same order of accumulation as the plain loop.
     {
@@ -645,7 +645,7 @@ __global__ void __launch_bounds__(256) k_dec_attn_scores(const DecAttnParams P, 
     const int kv_dim = P.kv_heads * HD;
     const size_t row_bytes = Q8 ? (size_t)(kv_dim / 32) * 34 : (size_t)kv_dim * 2;
     const size_t head_off = Q8 ? (size_t)((kvh * HD) / 32) * 34 : (size_t)kvh * HD * 2;
-    // Round 6 (second session): the key rows of the first pass are requested BEFORE the new token's values are staged, rotated and
+    // The key rows of the first pass are requested BEFORE the new token's values are staged, rotated and
     // stored (they depend on the split only; the new token's own row is never read from the cache), and the rows of the next pass before
     // the current one is multiplied: the kernel was a chain of ~6 dependent round trips for one or two passes of 256 keys.  Q8 rows come
     // as 4- / 8-byte requests of the head's slice (68 two-byte loads per key before).  Same products in the same order.

@@ -1,4 +1,4 @@
-// ifa_decode_chain.h -- round 6: consecutive GEMV ops of one decoder layer (batch 1) as ONE launch, with the NEXT op's weight
+// ifa_decode_chain.h -- consecutive GEMV ops of one decoder layer (batch 1) as ONE launch, with the NEXT op's weight
 // rows requested BEFORE the hand-off of the current op's output is waited for.
 //
 //   [Wo (+bias, +residual)] -> [RMS norm -> Q8 quantiser -> W1 | W3 -> activation -> gate] -> [Q8 quantiser -> W2 (+bias, +residual)]
@@ -8,7 +8,7 @@
 // launches (tests/test_gpu_chain.py).
 //
 // Why this and not the r3 / r4 forms.  A hand-off through memory costs ~3.3 us on this part (write-through store, visibility,
-// one load round trip behind the CU's own queue) against ~2.5 us for a kernel boundary + first load (DESIGN.md, r4 price list):
+// one load round trip behind the CU's own queue) against ~2.5 us for a kernel boundary + first load (measured):
 // a fused launch only wins through what STREAMS during the hand-off.  The r3 engine streamed into a 112 KiB LDS ring and paid
 // for it with issue-bound consumer waves; the r4 fusions split the waves (or the CUs) into a front part and loaders, so the
 // front part's round trips queued behind the loaders' requests.  Here every wave is both: the register file is the ring
@@ -17,7 +17,7 @@
 // the dependency chain sits behind more than one op's worth of its own requests.
 //
 // Hand-off: one 4-byte granule {tag16 << 16 | half} per output row, written by ONE agent-scope relaxed store (write-through,
-// MI355X_MICROARCH.md form R2: the data is the flag) and gathered 16 bytes (4 granules) per request with sc1 loads; a thread
+// the data is the flag) and gathered 16 bytes (4 granules) per request with sc1 loads; a thread
 // owns a chunk of 8 consecutive values -- the chunk of XPre's quantiser, so norm statistic and codes are the bits of the
 // separate launches -- and re-requests only the chunks whose tags are not this step's yet.  The gather is ONE pass in the
 // common case: every workgroup raises a flag (its last publishing wave, through an LDS counter) and ONE wave per CU polls the

@@ -337,7 +337,7 @@ struct WRowQ6B64 {
 
 // Q3H_B64T1 rows are streamed as nibble pairs (ifa_tiled.h: q3h_aos_to_nibbles), i.e. as WRowQ4B64 with codes 0..10.
 
-// Q3H_NATIVE: the same values at the format's own 32 bytes per block (engine option q3h_native; VERDICT r5 item 5: built to be
+// Q3H_NATIVE: the same values at the format's own 32 bytes per block (engine option q3h_native: built to be
 // measured against the 36-byte nibble form).  Streamed block = the 28 bytes D0..D6 of q3h_aos_to_tiled (ifa_tiled.h: byte b of
 // D[w] = pair code p[4w + b] in its low 7 bits, bit 7 = bit w of p[28 + b]) + (base, scale); row layout
 // [D0..D3: 16 B x n][D4, D5: 8 B x n][D6, (base, scale): 8 B x n].  A pair code is p = q0 + 11 q1 (q0 = element 2k, q1 = 2k + 1),

@@ -48,7 +48,7 @@ constexpr int dec_role(int epi, int norm) { return epi == EPI_GLU ? 2 : (epi == 
 template <int DT>
 constexpr int dec_rw(int epi, int norm, int nj, int nm, int th = DEC_THREADS)
 {
-    if (DT == Q4_B32T1A) {      // tuned on Llama-2-7B shapes (DESIGN.md "Kernel timeline")
+    if (DT == Q4_B32T1A) {      // tuned on Llama-2-7B shapes
         const int role = dec_role(epi, norm);
         const int forced = role == 0 ? IFA_T_RW_QKV : role == 1 ? IFA_T_RW_WO : role == 2 ? IFA_T_RW_GLU : role == 3 ? IFA_T_RW_W2 : 0;
         if (forced > 0) return forced;
@@ -62,8 +62,8 @@ constexpr int dec_rw(int epi, int norm, int nj, int nm, int th = DEC_THREADS)
         const int forced = role == 0 ? IFA_T_RW_QKV : role == 1 ? IFA_T_RW_WO : role == 2 ? IFA_T_RW_GLU : role == 3 ? IFA_T_RW_W2 : 0;
         if (forced > 0) return forced;
     }
-    // B64 formats (one block per lane at 4096 columns): sweep on Llama-2-7B Q3H + Q8 KV (configs[2];
-    // profiles/r02_sweep_q3h.log): 544 -> 601 tok/s; the same entries measured on Q4_B64T1 / Q5_B64T1 (Q6_B64T1: 1024 threads spill)
+    // B64 formats (one block per lane at 4096 columns): sweep on Llama-2-7B Q3H + Q8 KV
+    // (profiles/r02_sweep_q3h.log): 544 -> 601 tok/s; the same entries measured on Q4_B64T1 / Q5_B64T1 (Q6_B64T1: 1024 threads spill)
     if (DT == Q3H_B64T1 || DT == Q3H_NATIVE || DT == Q4_B64T1 || DT == Q5_B64T1 || DT == Q6_B64T1) {
         if (DT != Q6_B64T1 && epi == EPI_GLU && nj == 1 && th > DEC_THREADS) return 3;   // W1/W3 at 1024 threads: 16.7 -> 14.1 us (Q3H)
         if ((epi == EPI_RESIDUAL || epi == EPI_PLAIN) && norm == 2 && nj == 1) return 2; // Wo without a prologue: 6.3 -> 4.6 us
@@ -78,7 +78,7 @@ constexpr int dec_rw(int epi, int norm, int nj, int nm, int th = DEC_THREADS)
     return th > DEC_THREADS ? (rw + 1) / 2 : rw;           // 1024 threads: 128 registers per lane
 }
 
-// Workgroup size by kernel shape, measured on Llama-2-7B Q4 (DESIGN.md): the gated W1/W3 kernel and the short Wo kernel
+// Workgroup size by kernel shape, measured on Llama-2-7B Q4: the gated W1/W3 kernel and the short Wo kernel
 // (2 blocks per lane) gain from four waves per SIMD (issue stalls overlap), QKV and the long-row W2 kernel lose
 template <int DT>
 constexpr int dec_threads(int epi, int norm, int nj, bool xadd)
@@ -90,12 +90,12 @@ constexpr int dec_threads(int epi, int norm, int nj, bool xadd)
     }
     if ((DT == Q3H_B64T1 || DT == Q3H_NATIVE || DT == Q4_B64T1 || DT == Q5_B64T1) && nj == 1 && !xadd && epi == EPI_GLU) return 1024;          // (see dec_rw)
     if (DT == Q8_B32T2 && nj == 2 && !xadd && epi == EPI_GLU) return 1024;
-    if (DT == Q4_B32T1A && nj == 2 && !xadd && epi == EPI_PLAIN && norm == 1) return 1024;      // QKV with the wave-specialised prologue (r04 sweep: 8.8 -> 8.3 us)
+    if (DT == Q4_B32T1A && nj == 2 && !xadd && epi == EPI_PLAIN && norm == 1) return 1024;      // QKV with the wave-specialised prologue (sweep: 8.8 -> 8.3 us)
     return (DT == Q4_B32T1A && nj == 2 && !xadd && (epi == EPI_GLU || (epi == EPI_RESIDUAL && norm == 0))) ? 1024 : DEC_THREADS;
 }
 
 // waves that run the norm / quantiser prologue while the others already stream their rows (k_dec_gemv's NP; 0 = every wave
-// takes part in the prologue, the round 1-3 form).  Only the dense per-layer kernels with a prologue.
+// takes part in the prologue).  Only the dense per-layer kernels with a prologue.
 template <int DT>
 constexpr int dec_np(int epi, int norm, int nj, bool xadd, int th)
 {
@@ -103,7 +103,7 @@ constexpr int dec_np(int epi, int norm, int nj, bool xadd, int th)
     const int role = dec_role(epi, norm);
     const int forced = role == 0 ? IFA_T_NP_QKV : role == 2 ? IFA_T_NP_GLU : role == 3 ? IFA_T_NP_W2 : -1;
     if (forced >= 0) return forced < th / 64 ? forced : 0;
-    // round-4 sweep on Llama-2-7B Q4 (gpurun_out sweeps, DESIGN.md section 3 "wave-specialised prologue"): half of the waves
+    // sweep on Llama-2-7B Q4: half of the waves
     // run the prologue -- QKV 9.6 -> 8.2-8.5 us (1024 threads), W1/W3 13.1 -> 12.95, W2 9.05 -> 8.0-8.1 (512 threads);
     // a quarter or three quarters of the waves lose (the prologue's VALU time, or too few early requests)
     if (role == 0 || role == 2 || role == 3) return th / 128;
@@ -151,7 +151,7 @@ static int dec_gemv_launch_en(const DecGemvParams &P, int wgs_per_cu_opt, hipStr
     const size_t smem = xlds_bytes(P.cols);
     // the matrix pointer as a preloaded kernel argument when the launch has ONE matrix (pair) and no expert table (k_dec_gemv)
     const uint8_t *pw0 = (P.nsets == 1 && !epi_is_moe(EPI) && !P.w_table) ? P.W0[0] : nullptr;
-#ifdef IFA_NO_PRELOAD_W            // (A / B: the row addresses from the argument block, as before round 5)
+#ifdef IFA_NO_PRELOAD_W            // (A / B: the row addresses from the argument block, as before the preloaded ones)
     pw0 = nullptr;
 #endif
     // inputs that are normalised or feed an activation are [dim] vectors (dim <= 8192): <= 4 blocks per lane of a B32 format

@@ -1,7 +1,7 @@
 // ifa_decode_kernels.h -- fused batch-1 decode kernels (the hot path).
 //
 // One decoder layer at T=1 is 5 launches instead of the reference's ~30
-// launch+sync pairs (SURVEY.md appendix B):
+// launch+sync pairs:
 //   k_dec_gemv<QKV>   : [RMSNorm -> Q8 act-quant] prologue + Wq/Wk/Wv GEMV (+bias)
 //   k_dec_attn        : RoPE(q,k) + KV-cache write (F16 or Q8) + GQA attention
 //   k_dec_gemv<WO>    : [Q8 act-quant] + Wo GEMV + bias + residual add
@@ -561,7 +561,7 @@ __device__ __forceinline__ void dec_finish_row(const DecGemvParams &P, const Dec
 
 // RW = rows (EPI_GLU: row pairs) per wave and pass; rows are strided over the waves
 // (v = (pass*RW + i)*W + wave) so neighbouring waves stream neighbouring rows.
-// Order of memory traffic inside the kernel (measured, see DESIGN.md "Kernel timeline"):
+// Order of memory traffic inside the kernel (measured):
 //   1. activation (+norm weight) loads by all threads, then a barrier: the CU's memory
 //      pipeline is FIFO across waves, so these must be queued before any weight request;
 //   2. D1 rows of weights per wave (~40 KiB per CU: accepted without blocking);
@@ -571,7 +571,7 @@ __device__ __forceinline__ void dec_finish_row(const DecGemvParams &P, const Dec
 //      (bias / residual / activation) so the epilogue's loads overlap too.
 // TH = threads per workgroup: 512 (two waves per SIMD, 256 registers each) or 1024 (four waves per SIMD, 128 registers, half
 // the rows in flight per wave) -- chosen per kernel shape by the launcher (ifa_decode_gemv_impl.h)
-// NP > 0: WAVE-SPECIALISED prologue (round 4).  Waves [0, NP) request the activation, run the norm + quantiser among
+// NP > 0: WAVE-SPECIALISED prologue.  Waves [0, NP) request the activation, run the norm + quantiser among
 // themselves (LDS counters, XPre<.., NT>) and only then request their rows; waves [NP, TH/64) request ALL their rows right
 // after the first barrier and wait for the image behind them.  In the classic form every wave takes part in the prologue's
 // barriers, so at most D1 rows per wave (what the CU's memory queue accepts without blocking) can be in flight while the
@@ -584,10 +584,10 @@ __global__ void __launch_bounds__(TH) k_dec_gemv(const half_t *px, const half_t 
     // px / pnw / pnb / pcols repeat P.x / P.norm_w / P.norm_b / P.cols as leading scalar arguments: with
     // -amdgpu-kernarg-preload-count they arrive in SGPRs at wave launch, so the activation requests -- the head of
     // the kernel's critical path -- do not wait for the first scalar load of the argument block.
-    // pw0 / pw1 / pnblk / ptotal (round 5) do the same for the WEIGHT requests: pnblk = P.nblk and ptotal = P.total_rows for every
+    // pw0 / pw1 / pnblk / ptotal do the same for the WEIGHT requests: pnblk = P.nblk and ptotal = P.total_rows for every
     // launch; pw0 = P.W0[0], pw1 = P.W1 for the single-matrix launches (Wo, W1 / W3, W2), pw0 = null when there are several sets
     // or an expert table (the row addresses then come from the argument block as before).  Every row address of such a launch is then a function of preloaded scalars and
-    // the wave's own id: the stream's first request no longer waits ~0.4 us for the argument block's scalar load (r04 trace:
+    // the wave's own id: the stream's first request no longer waits ~0.4 us for the argument block's scalar load (trace:
     // "loads issued" at 0.9-1.0 us of the launch; the argument block is cold after every kernel boundary)
     extern __shared__ __attribute__((aligned(16))) char smem[];
     static_assert(NP == 0 || (NORM != 2 && !XADD && NP * 64 < TH), "wave-specialised prologue: a norm / quantiser prologue, some loader waves");

@@ -1,4 +1,4 @@
-// ifa_decode_lmhead_tail.h -- round 4: the END of a decode step as ONE launch: final norm + F16 lm_head GEMV (k_dec_lmhead_f16's
+// ifa_decode_lmhead_tail.h -- the END of a decode step as ONE launch: final norm + F16 lm_head GEMV (k_dec_lmhead_f16's
 // body) + greedy argmax + advance of the device state (k_dec_argmax_advance) + the NEXT step's embedding gather and RoPE table
 // (k_dec_gather).  Two launches less per token: both were pure latency chains (8.5 + 5.0 us for 64 KB of logits and an 8 KB row).
 //

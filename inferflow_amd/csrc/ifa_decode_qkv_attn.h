@@ -1,4 +1,4 @@
-// ifa_decode_qkv_attn.h -- round 4: the decode attention as the TAIL of the Wq|Wk|Wv launch (one kernel boundary per
+// ifa_decode_qkv_attn.h -- the decode attention as the TAIL of the Wq|Wk|Wv launch (one kernel boundary per
 // layer less: 5 -> 4 launches).
 //
 // Reference ops fused here (batch 1): RmsNorm -> Quantize -> Wq, Wk, Wv GEMV (+bias) (inference_worker.cc:1407-1621) and,
@@ -11,7 +11,7 @@
 // kv_heads sets of `gk` workgroups; set g computes exactly the rows of kv group g (k_dec_gemv deals rows round-robin over
 // all waves instead), so the attention of a head waits for gk workgroups -- 8 for Llama-2-7B -- not for the grid:
 //   * every finished row is published as ONE 8-byte {epoch, half} granule (agent-scope relaxed store: write-through,
-//     MI355X_MICROARCH.md "Persistent kernels" price list, form R2 -- no flag, no fence, valid iff the tag matches);
+//     no flag, no fence, valid iff the tag matches);
 //   * the head's designated workgroup (its own rows are part of the set, so it arrives with the others) requests the
 //     head's K / V rows -- now that the position is known, only rows that exist -- polls the 3 * HD granules while those
 //     are in flight, and runs dec_attn_body<FUSED>;
@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(QA_THREADS) k_dec_qkv_attn(const half_t *px, c
                                                              const uint8_t *pwq, const uint8_t *pwk, const uint8_t *pwv,
                                                              const DecGemvParams P, const DecAttnParams A, const DecQkvAttnExtra E)
 {
-    // pgeo / pwq / pwk / pwv (round 5): heads | kv_heads << 8 | gk << 16 and the three matrices as leading scalar arguments -- with
+    // pgeo / pwq / pwk / pwv: heads | kv_heads << 8 | gk << 16 and the three matrices as leading scalar arguments -- with
     // px / pnw / pnb / pcols they fill the 14 dwords the hardware preloads into SGPRs at wave launch, so that every q | k | v row
     // address is a function of preloaded scalars and the workgroup's id: the weight stream's first request does not wait for
     // the (cold) argument block (k_dec_gemv does the same: A / B on one box 808 vs 798-802 tok/s, profiles/r05_preload_ab.log)

@@ -1,7 +1,7 @@
-// ifa_decode_singles.h -- the single-row experts of a batched mixture-of-experts step (round 4).
+// ifa_decode_singles.h -- the single-row experts of a batched mixture-of-experts step.
 // A step of 8 queries x top-2 spreads 16 entries over 8 experts: two or three of them get exactly one row.  The reference
 // runs such a row through its T = 1 branch (TensorOpr::Quantize + Gemv_AX, inference_worker.cc:1772-1774: Q8 activations,
-// int8 dot, the arithmetic of the decode GEMV); round 3 ran them as three grouped launches over the reference-layout blocks
+// int8 dot, the arithmetic of the decode GEMV); before, they ran as three grouped launches over the reference-layout blocks
 // (k_gemv_ax8_grouped: 3.9 TB/s) behind two quantiser launches and an element-wise one.  Here they take the batch-1 decode
 // kernels' structure on the tiled rows those kernels stream: blockIdx.y is a slot of the device-built list (k_moe_build's
 // MoeSingle {expert, entry}); absent slots leave at once; the workgroup quantises its entry's row (XPre<0>: the same Q8_B32T2

@@ -427,7 +427,7 @@ int ifa_model_set_tensor(ifa_model *m, int layer, int tensor_id, int expert, int
     }
     free_tensor(*t);
     m->mo_built = false;
-    if (expert >= 0) {      // the layer's table of MO copies points into the copy just freed: ensure_mo rebuilds it (ADVICE r3)
+    if (expert >= 0) {      // the layer's table of MO copies points into the copy just freed: ensure_mo rebuilds it
         Layer &Lx = m->layers[(size_t)layer];
         if (Lx.moe_table_mo) { (void)hipFree(Lx.moe_table_mo); Lx.moe_table_mo = nullptr; }
     }

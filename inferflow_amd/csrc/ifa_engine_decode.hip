@@ -27,7 +27,7 @@ static int attn_split_threshold(const ifa_model *m)
 
 void choose_attn_split(ifa_model *m, int reach)
 {
-    // splits per head by the context the call reaches: 8 up to 8192 keys, 16 above (round 6, second session, after the kernels lost their
+    // splits per head by the context the call reaches: 8 up to 8192 keys, 16 above (after the kernels lost their
     // request chains: 2048 / 4096 / 8192 keys 563 / 484 / 404 tok/s with 8 splits against 535 / 483 / 400 with 16; 16384 keys 301 / 303 / 281
     // with 8 / 16 / 32; Q8 cache 4096 keys 487 against 465 -- profiles/r06_long_context_decode.log.  Was 8 / 16 / 32 from 512 / 2048 / 8192.)
     const int thr = attn_split_threshold(m);

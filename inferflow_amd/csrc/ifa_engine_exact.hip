@@ -2,7 +2,7 @@
 // summation order of the reference's CUDA kernels as the oracle restates them.  One token at a time, launch by launch, the layer of
 // GpuInferenceWorker::ProcessGpuLayer (inference_worker.cc:762-981) with every op boundary an F16 tensor: all of them, the int8 codes of
 // the re-quantised activations and of a Q8 KV cache, and the logits are then bit-identical to oracle.Model's
-// (tests/test_gpu_fullsize_oracle.py: 32 layers, configs[1] and configs[2]).  A parity instrument, ~50x slower than the timed path.
+// (tests/test_gpu_fullsize_oracle.py: 32 layers, 4-bit weights with the F16 cache and 3.5-bit ones with the 8-bit cache).  A parity instrument, ~50x slower than the timed path.
 #include <cmath>
 #include "ifa_engine_state.h"
 #include "ifa_exact.h"

@@ -355,7 +355,7 @@ int moe_ffn_device(ifa_model *m, Layer &L, const half_t *ff_n, int T, const half
     g.wtab = (const uint8_t *const *)L.moe_table_aos; g.on = 1;
     // (T <= small_max: no expert can collect more rows than the small groups take -- the tile list is empty, its launches are skipped)
     const int max_tiles = (small_max > 0 && T <= small_max) ? 0 : cap / tile_rows + E, max_singles = std::min(E, cap);
-    // Single-row experts (round 4): when no expert can collect a tile of rows (max_tiles == 0: a batched decode step) and the small
+    // Single-row experts: when no expert can collect a tile of rows (max_tiles == 0: a batched decode step) and the small
     // groups gate their own products (MO copies), the singles are the only rows the quantiser / element-wise launches below serve --
     // they then take two launches of the decode GEMV's structure on the tiled expert tables (ifa_decode_singles.h) instead of six
     if (m->opt_moe_singles && max_tiles == 0 && (smalls_mo || max_smalls == 0) && L.moe_table && dec_singles_supported(wdt, F, D, true)

@@ -394,7 +394,7 @@ int tp_check(ifa_model *m, const ifa_tp_topology *topo, const char *who)
 // token, [n_tokens][shard rows] F16 (return_output_tensors).
 // A bounded wait of the one-shot exchange that gave up (a peer that never arrived) left this rank without a sum -- and its epoch
 // one behind its peers'.  Every partition entry point checks after its stream sync: the call fails (the engine then aborts the
-// group), the captured steps are dropped and this communicator keeps RCCL for every size from now on (ADVICE r3).
+// group), the captured steps are dropped and this communicator keeps RCCL for every size from now on.
 int tp_oneshot_status(ifa_model *m, const ifa_tp_topology &t, const char *who)
 {
     if (!t.tp || !ifa_comm_oneshot(t.tp)) return IFA_OK;

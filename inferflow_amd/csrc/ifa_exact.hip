@@ -5,7 +5,7 @@
 // (Tensor_SoftMax_Alg2_Kernel, unary_tensor_opr.h:480-535).  Engine option `exact_order` routes single-token steps through these
 // kernels (csrc/ifa_engine_exact.hip): every F16 tensor and every int8 code of a step is then bit-identical to the oracle's, which
 // is what tests/test_gpu_fullsize_oracle.py asserts through 32 layers.  They are correctness instruments -- one half wave per row,
-// no layout tricks -- not the timed path; the timed kernels keep the same per-block terms in a wave64 order (DESIGN.md section 5).
+// no layout tricks -- not the timed path; the timed kernels keep the same per-block terms in a wave64 order.
 //
 // Transcendentals: the CPU side of the comparison calls libm, so (a) exp is restated here in the algorithm glibc's expf uses
 // (Szabolcs Nagy's exp2f-table form: N = 32 table of 2^(i/32), cubic in double; constants as published in glibc

@@ -365,7 +365,7 @@ typedef const __attribute__((address_space(1))) void pf_glb_t;
 // outputs, bias, residual, GLU pair; W[] / W1 are REFERENCE-layout rows here) + the tile geometry.
 // EPI: GM_PLAIN | GM_RESIDUAL (Y = half(res + y), TensorOpr::Add) | GM_GLU (a weight tile = BN / 2 rows of w1 and the
 // same BN / 2 rows of w3, both halves meet in the epilogue's LDS tile: Y = half(half(act(y1)) * y3)).
-// KS = 2 (round 4, 128 x 128 tiles of a product that offers no more tiles than CUs: wo and w2 of a 1024-token prompt are 256 tiles of
+// KS = 2 (128 x 128 tiles of a product that offers no more tiles than CUs: wo and w2 of a 1024-token prompt are 256 tiles of
 // four waves -- one workgroup per CU, the matrix pipe 25 % busy): two workgroups per tile, each walks half of K; the first half's
 // fp32 accumulators go through memory (write-through stores, one flag per tile) to the workgroup of the second half, which adds them
 // IN THAT ORDER (first half + second half: deterministic) and runs the epilogue.  The grid lists all first halves, then all second
@@ -399,7 +399,7 @@ __global__ void __launch_bounds__(WM * WN * 64) k_gemm_big(const GmArgs P, const
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid0 = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
-    // Stream-K schedule (KS = 0; round 6, 256 x 256 tiles of a product whose tile count is no multiple of the CU count: w1 | w3 of a
+    // Stream-K schedule (KS = 0; 256 x 256 tiles of a product whose tile count is no multiple of the CU count: w1 | w3 of a
     // 1024-token prompt are 344 tiles on 256 CUs, wq | wk | wv 192): ONE workgroup per CU; each first takes G.sk_full whole tiles,
     // then an equal share of the K steps of the G.sk_rem tiles that are left -- steps [b(w), b(w + 1)) of the remainder's linear
     // (tile, step) space, b(w) = w * sk_rem * S / grid -- which touches at most two tiles.  A share that does not END its tile leaves
@@ -894,14 +894,14 @@ static int launch_gemm_big(const GmArgs &P0, hipStream_t s)
     const bool split = full_n > 0 && rem_n > 0 && ifa_cdiv(T, (size_t)128) * rem_n <= cus && tm256 * rem_n < cus * 3 / 4;
     const size_t n128 = ifa_cdiv(T, (size_t)128) * ntiles(128);
     double c256 = CAP > 32 ? 1e30 : (split ? (double)(full_n / per_round) + 0.68 : rounds(256, 256, 1));   // (64-value blocks: the 256 x 256 variant would spill)
-    // Round 6, stream-K on the 256 x 256 tiles (k_gemm_big<.., KS = 0>; OPT-IN, bit 13 of ifa_gemm_big_tiles): every CU takes
+    // Stream-K on the 256 x 256 tiles (k_gemm_big<.., KS = 0>; OPT-IN, bit 13 of ifa_gemm_big_tiles): every CU takes
     // floor(tiles / CUs) whole tiles and then an equal share of the K steps of the rest.  Built, deterministic, within the F16 rounding of
     // the whole-tile kernel -- and measured SLOWER on the two products it was built for (1024-token prompt, Llama-2-7B Q4, one box,
     // rocprofv3 averages over 128 launches): w1 | w3 (344 tiles) 259.5 us against 144.3 + 84.2 for the round of whole tiles + the
     // 128-token-tile launch of the rest, wq | wk | wv (192 tiles) 135.6 against 117.5; prefill 20.4 against 18.6 ms (2048 tokens: 37.7
     // against 34.9).  The tail it removes is 35 / 29 us per layer; a share that does not end its tile sends 256 KB of fp32 sums through
-    // memory (write-through stores, 64 MB per launch) and the share that ends the tile reads up to three of them -- MI355X_MICROARCH.md
-    // prices that at ~12 us out + 4 us per slot in on an idle chip, here it costs 50-65.  Eligible when a share is >= 20 steps (<= 3
+    // memory (write-through stores, 64 MB per launch) and the share that ends the tile reads up to three of them: some
+    // 12 us out + 4 us per slot in on an idle chip, here 50-65.  Eligible when a share is >= 20 steps (<= 3
     // scratch slots per shared tile at K = 4096).  profiles/r06_stream_k_ab.log.
     bool sk = false;
     {
@@ -939,7 +939,7 @@ static int launch_gemm_big(const GmArgs &P0, hipStream_t s)
         const bool may_split = !force && EPI != GM_GLU && (g_gemm_big & (1 << 12)) == 0 && !P.no_waits && waits_enabled();
         const size_t ksteps = (size_t)P.nblk * CAP / PF_BK;
         const bool splitk = may_split && n128 <= cus && n128 * 2 >= cus && ksteps % 2 == 0 && P.nblk * CAP >= 2048;
-        // Round 5, prompts of 48..128 tokens (ONE token tile; the engine sends them here from `prefill_big_min` + 1 tokens on): wq | wk | wv
+        // Prompts of 48..128 tokens (ONE token tile; the engine sends them here from `prefill_big_min` + 1 tokens on): wq | wk | wv
         // are 96 tiles, wo and w2 32 -- a quarter or an eighth of the chip.  Four parts of K per tile when that still fits two
         // workgroups per CU and a part keeps >= 1024 columns: 64 tokens 7.46 -> 7.10 ms, 128 tokens 8.22 -> 7.46 (profiles/r05_prompt_lengths.log)
         const bool splitk4 = may_split && n128 * 2 < cus && n128 * 4 <= 2 * cus && ksteps % 4 == 0 && P.nblk * CAP >= 4096;
@@ -1083,7 +1083,7 @@ extern "C" int ifa_gemm(int w_dtype, const void *W, size_t rows, size_t cols, co
     IFA_REQUIRE(rows < (1u << 30) && cols < (1u << 30) && tokens <= 65535u * 64u, "ifa_gemm: shape too large");
     hipStream_t s = ifa_s(stream);
     // (every T runs the in-tree kernels: no vendor GEMM is linked or loaded by this library; the dequantise-once + hipBLASLt
-    //  comparison of rounds 1-3 is tools/bench_gemm_big.py, through torch.matmul on the dequantised operand)
+    //  comparison is tools/bench_gemm_big.py, through torch.matmul on the dequantised operand)
     if (w_dtype == F16) {
         launch_gemm<F16>(W, rows, cols, x_f16, tokens, bias_f16, y_f16, s);
     } else {

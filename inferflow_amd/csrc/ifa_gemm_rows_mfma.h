@@ -30,7 +30,7 @@ struct GmArgs {
     int ldyset[3];
     int mo;                        // W[] / W1 are MO-layout copies (below: MO_QUADS or MO_WORDS) instead of the tiled layout
     long long *trace;              // optional [workgroups][16] wall-clock stamps (tuning: IFA_ROWS_TRACE=1 prints a timeline per launch)
-    // K parts (round 4: chunked rows of 9..32 queries, kernels instantiated with KPM > 0): kparts consecutive workgroups share a
+    // K parts (chunked rows of 9..32 queries, kernels instantiated with KPM > 0): kparts consecutive workgroups share a
     // group of KPM * kparts tiles; each walks its own chunks of K for ALL of them, leaves the fp32 sums of the tiles it does not
     // finish in kpart_sums as 8-byte {1, value} granules (zero between launches) and finishes tiles [kp * KPM, (kp + 1) * KPM):
     // its own part from LDS, the others' granules polled, added in K order.  Filled by the launcher; 0 = off.

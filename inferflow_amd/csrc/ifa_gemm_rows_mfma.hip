@@ -23,7 +23,6 @@
 //     LDS with the same permutation, so the sum over k is the plain dot product in another (fixed) order;
 //   * the activation rows sit in LDS as F16, one chunk at a time (row stride + 16 B: conflict-free 16-byte reads); longer
 //     rows (w2) are walked in chunks with the accumulators kept in registers.
-// Measurements behind these choices and what bounds the kernel now: DESIGN.md section 3 "Dynamic batching", section 8.
 #include "ifa_gemm_rows_mfma_body.h"
 
 namespace ifa {

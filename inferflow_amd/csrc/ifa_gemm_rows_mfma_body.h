@@ -158,7 +158,7 @@ __device__ __forceinline__ void gemm_rows_mfma_body(const GmArgs &P, char *smem)
     // Weight requests are GLOBAL loads through an explicit address-space cast: the set pointers pass through integers
     // (readfirstlane, gm_sel), so the compiler no longer knows their address space and would emit FLAT loads -- which count
     // on lgkmcnt as well, so that every LDS wait in the compute phase (lgkmcnt(0)) also waited for all weight groups in flight:
-    // the kernel requested everything, waited, then computed (rows-trace timeline, DESIGN.md "Dynamic batching").
+    // the kernel requested everything, waited, then computed (rows-trace timeline).
     typedef const __attribute__((address_space(1))) u32x4 gu4;
     auto gload = [](const uint8_t *base, uint32_t off) { return __builtin_nontemporal_load((gu4 *)(base + off)); };
     auto fetch = [&](GmGrp &q, int it, int chunk, bool valid) {
@@ -373,7 +373,7 @@ __device__ __forceinline__ void gemm_rows_mfma_body(const GmArgs &P, char *smem)
         }
 #if IFA_ROWS_FETCH_EARLY
         if constexpr (NORM == 0) {
-            // Round 4: plain staging (wo, w2, all 17..32-row launches): the other PD - 1 groups are requested BEFORE the rows are
+            // Plain staging (wo, w2, all 17..32-row launches): the other PD - 1 groups are requested BEFORE the rows are
             // stored -- behind the rows' own requests in this CU's queue, so the rows still return first -- instead of behind the
             // staging barrier: 32 queries 3.69 -> 3.36 ms per step, 16 queries 2.28 -> 2.18 (2 queries: unchanged)
             if (first_chunk) {
@@ -429,7 +429,7 @@ __device__ __forceinline__ void gemm_rows_mfma_body(const GmArgs &P, char *smem)
         }
         xw_store();
     } else x_store(c_lo, true);
-    // The staging barrier FIRST, the other PD - 1 groups behind it (round 4): requested in front of the barrier, every wave sat in
+    // The staging barrier FIRST, the other PD - 1 groups behind it: requested in front of the barrier, every wave sat in
     // its load issue (4 x 5 KB per wave against a full memory queue) before it could arrive -- the rows were staged at 3.0 us and
     // the barrier passed at 4.8 (rows-trace: "other groups requested 3.22, x staged 4.77"); the first group is in flight since 0.8
 #if IFA_ROWS_FETCH_EARLY

@@ -7,7 +7,7 @@
 //    block, lanes own blocks l, l+64, ... and a DPP/bpermute tree sums the wave.
 //    The reference's 32-lane CUDA butterfly orders the fp32 adds differently;
 //    results agree to fp32 round-off and are compared after rounding to half
-//    with the tolerance stated in tests/ (DESIGN.md "Tolerances").
+//    with the tolerance stated in tests/.
 //  * fp16-activation path (gemv.h:469-1497): weights dequantised to half in
 //    registers, fp32 accumulate (the reference accumulates three variants in
 //    half, appendix A4; fp32 is at least as accurate).

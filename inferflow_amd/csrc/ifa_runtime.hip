@@ -41,7 +41,7 @@ unsigned *wait_err_word()
     auto it = g_wait_words.find(dev);
     if (it != g_wait_words.end() && it->second) return it->second;
     // (a failed allocation -- e.g. the first use fell inside a stream capture -- is NOT remembered: the next call tries again, and
-    //  the launchers below take their non-waiting kernels while the word is missing, ADVICE r5)
+    //  the launchers below take their non-waiting kernels while the word is missing)
     unsigned *p = nullptr;
     if (hipHostMalloc((void **)&p, 64, hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
     memset(p, 0, 64);

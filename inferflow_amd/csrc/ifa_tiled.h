@@ -1,5 +1,5 @@
 // ifa_tiled.h -- the "row-local plane" weight layout streamed by the fused
-// decode kernels (DESIGN.md "HBM layout").
+// decode kernels.
 //
 // A reference row is nblk AoS blocks {base, scale, bit-planes...}
 // (src/common/quant_types.h).  Block sizes of 20/34/36/44/52 B defeat aligned
@@ -62,8 +62,8 @@ IFA_TILED(Q5_B64T1, 3, IFA_ARR(32, 8, 4), IFA_ARR(12, 4, 0))
 // ---- Q3H_B64T1: the reference packs two 11-level codes into one 7-bit pair code p = q0 + 11 * q1 and splits p over
 // three bit planes (4 + 2 + 1 bits, quantization.h:823-851).  Decoding that in the GEMV is VALU work per weight
 // (re-assembling the planes: ~4 ops per element; with whole pair codes per byte and a multiply-shift division by 11:
-// ~1.6) and kept the 3.5-bit format BEHIND the 4-bit one on a part where the stream should be the only cost (round 2:
-// 607 tok/s vs 695 while reading 19 % fewer bytes).  The streaming layout is therefore chosen for decode cost: each
+// ~1.6) and kept the 3.5-bit format BEHIND the 4-bit one on a part where the stream should be the only cost
+// (607 tok/s vs 695 while reading 19 % fewer bytes).  The streaming layout is therefore chosen for decode cost: each
 // pair code is expanded ONCE, at load time, into the byte q0 | q1 << 4 -- exactly the Q4_B64T1 convention (byte i =
 // elements 2i low, 2i + 1 high) with codes 0..10 -- so the fused kernels decode it with two nibble masks and the
 // block is 36 bytes per 64 weights (4.5 bits) instead of 32 (4.0): still 10 % fewer streamed bytes than Q4_B32T1
@@ -84,7 +84,7 @@ __host__ __device__ inline void q3h_aos_to_nibbles(const uint8_t *aos, uint8_t *
     for (int k = 0; k < 32; k++) n32[k] = (uint8_t)((p[k] % 11) | ((p[k] / 11) << 4));
 }
 
-// Older byte-transposed form (round 1-2), kept for q3h_tiled_to_aos users:
+// Older byte-transposed form, kept for q3h_tiled_to_aos users:
 //   D[w] byte b (w = 0..6) = p[4w+b] | bit w of p[28+b] << 7        (p[k] = code of elements 2k, 2k+1)
 __host__ __device__ inline void q3h_pairs_from_aos(const uint8_t *aos, uint8_t *p)
 {

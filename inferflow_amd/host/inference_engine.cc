@@ -347,7 +347,7 @@ bool InferenceEngine::InitMulti(const std::vector<std::vector<int>> &groups)
             all_devices.push_back(w.device);
         }
     // a device named more than once: only as "every rank on ONE device" (loopback groups of the C ABI: the multi-rank
-    // paths on a 1-GPU box, tests); anything else is a configuration mistake
+    // paths on one GPU, tests); anything else is a configuration mistake
     bool dup = false, all_same = true;
     for (size_t i = 0; i < all_devices.size(); i++) {
         all_same = all_same && all_devices[i] == all_devices[0];

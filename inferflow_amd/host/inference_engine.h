@@ -6,7 +6,7 @@
 // (bool / query-id returns, a message through LogError -> ifa_engine_last_error(), never throws).
 // The host side is plain C++ and reaches the GPU only through the C ABI of include/inferflow_amd.h.
 //
-// Scope (SURVEY.md §8b/f1): token-id queries, one model per engine.  `devices` takes the reference's grammar
+// Scope: token-id queries, one model per engine.  `devices` takes the reference's grammar
 // (inference_engine.cc:1738-1783): "0" one GPU; "0&1" one device group, tensor parallel (BY_TENSOR); "0;1" two groups,
 // consecutive layer ranges (BY_LAYER); "0&1;2&3" HYBRID -- one worker and one host thread per GPU inside this process,
 // the exchanges through the C ABI collectives (RCCL).  Tokenizers, prompt templates and the HTTP service are outside
@@ -98,7 +98,7 @@ struct InferenceConfig {
     // layer) from this many on; below it each runs the fused single-query decode (Llama-2-7B Q4: 2 queries batched give
     // 825 aggregate tok/s against 690 for one after the other)
     int dynamic_batching_min_queries = 2;
-    // extension (tests on a 1-GPU box): run a single device through the partition path -- rank thread, communicator of
+    // extension (tests on one GPU): run a single device through the partition path -- rank thread, communicator of
     // one rank, the C-driven step with its collectives -- instead of the plain single-worker path
     bool force_partition_path = false;
     DebugOptions debug;

@@ -103,7 +103,7 @@ bool InferFlowServiceCore::InferOnce()
     if (engine_.QueryCount() == 0) { eg.unlock(); std::this_thread::sleep_for(std::chrono::milliseconds(1)); return true; }
     InferenceResult result;
     bool ok = engine_.Infer(result);
-    // One retry of a step that failed as a whole (ADVICE r5): the worker's bounded in-launch waits report a timeout as a FAILED call
+    // One retry of a step that failed as a whole: the worker's bounded in-launch waits report a timeout as a FAILED call
     // "repeat it: the waiting launches are off now" (IFA_ERR_STATE, include/inferflow_amd.h) -- recoverable by design, and a failed
     // Infer() commits nothing (Query::processed moves only behind a successful step), so the same step is simply run again; a second
     // failure ends the queries as before.

@@ -5,7 +5,7 @@
 // advances per step: the reference's dynamic batching, inferflow_service.cc:60-129); request handlers AddQuery and collect the
 // tokens of their query, whole or as a stream of chunks (:141-300); a URL containing "/chat/completions" switches the OpenAI-shaped
 // response (:477-500); "/stat" (or {"header": {"fn": "get_stat"}}) reports the engine state (:389-475).
-// Difference, by scope (SURVEY.md section 8: tokenizer and templates are out of scope): requests carry TOKEN IDS, responses too.
+// Difference, by scope (tokenizer and templates are out of scope): requests carry TOKEN IDS, responses too.
 //
 //   native  : {"prompt_token_ids": [1, 15043, ...], "max_output_len": 64, "decoding_alg": "sample.top_p", "random_seed": 1,
 //              "temperature": 0.8, "is_streaming_mode": false, "eos_token_id": 2}

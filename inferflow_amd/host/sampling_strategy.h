@@ -1,4 +1,4 @@
-// sampling_strategy.h -- the reference's standard decoding strategies on the host (SURVEY.md §8 f4):
+// sampling_strategy.h -- the reference's standard decoding strategies on the host:
 // Greedy, StdSampling ("sample.std"), TopK and TopP of StdSamplingStrategy
 // (src/transformer/sampling_strategy.cc:235-431): top-`pool_size` of the logits in TopKQueue order,
 // SoftMax with temperature over that pool, top_p / max_k cut, one draw with the engine's generator.

@@ -1,4 +1,4 @@
-"""Synthetic models for measurement and parity tests (SURVEY.md §8d):
+"""Synthetic models for measurement and parity tests:
 fp16 source tensors N(0, 0.02) from seed = 1000 + layer*16 + tensor_id, norm
 weights = 1, quantised on the device with the reference rule; tensors below
 tensor_quant_threshold stay F16 (src/transformer/network_builder.cc:1557-1562),
@@ -19,10 +19,10 @@ SHAPES = {
     "test_mha": dict(dim=256, layers=3, heads=8, kv_heads=8, head_dim=32, ffn=640, vocab=777),
     # w2 rows longer than one 4096-column chunk of the rows GEMM (chunk loop / whole-row staging)
     "test_longffn": dict(dim=256, layers=2, heads=4, kv_heads=4, head_dim=64, ffn=4352, vocab=500),
-    # data/models/yi_34b_chat (configs[3]) and a Llama-2-70B-shaped model: w2 rows of 20480 / 28672 columns
+    # data/models/yi_34b_chat and a Llama-2-70B-shaped model: w2 rows of 20480 / 28672 columns
     "yi_34b": dict(dim=7168, layers=60, heads=56, kv_heads=8, head_dim=128, ffn=20480, vocab=64000),
     "llama2_70b": dict(dim=8192, layers=80, heads=64, kv_heads=8, head_dim=128, ffn=28672, vocab=32000),
-    # data/models/falcon_40b_instruct (configs[3]): LayerNorm, GELU, plain (non-gated) MLP, attention and MLP both read
+    # data/models/falcon_40b_instruct: LayerNorm, GELU, plain (non-gated) MLP, attention and MLP both read
     # the layer input through their own norm (mlp_attn_share_input), 128 heads of 64 over 8 KV heads
     "falcon_40b": dict(dim=8192, layers=60, heads=128, kv_heads=8, head_dim=64, ffn=32768, vocab=65024,
                        norm_kind=1, act_kind=1, is_glu=0, share_input=1, rope_order=2),
@@ -104,7 +104,7 @@ def build(shape_name, wdtype=dt.Q4_B32T1A, kv_dtype=dt.F16, max_ctx=1024, quant_
 
 
 def weight_bytes(shape_name, wdtype=dt.Q4_B32T1A, quant_threshold=TENSOR_QUANT_THRESHOLD, streamed=False):
-    """Algorithmic weight bytes per decoded token (SURVEY.md §8d), excluding KV.  streamed=True: the bytes of the layout
+    """Algorithmic weight bytes per decoded token, excluding KV.  streamed=True: the bytes of the layout
     the decode kernels read (differs from the reference block bytes for Q3H_B64T1 only: 36 vs 32 per 64 weights)."""
     s = SHAPES[shape_name]
     per_layer = 0

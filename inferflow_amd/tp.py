@@ -9,7 +9,7 @@ Partition = the reference's BY_TENSOR strategy
   KV cache               : sharded by KV head
   lm_head                : sharded by vocabulary rows (the reference keeps it on the last
                            rank only; sharding it and doing a distributed argmax is the
-                           extension SURVEY.md §8e names)
+                           extension)
 Exchange = two sum all-reduces of one [dim] F16 vector per layer (after wo, after w2),
 exactly where the reference calls DistributeAndMergeTensors.  At batch-1 decode the
 payload is 8 KB, i.e. latency-bound.
@@ -151,7 +151,7 @@ class TPRunner:
             self.token_src = (groups - 1) * tp_size          # first rank of the last group announces the token
             world, rank, group = tp_size, tp_rank, my_group
         self.world, self.rank, self.group = world, rank, group
-        # IFA_FORCE_TP=1 with one rank: still issue the collectives (plumbing check on a 1-GPU box)
+        # IFA_FORCE_TP=1 with one rank: still issue the collectives (plumbing check on one GPU)
         self.force_collectives = bool(os.environ.get("IFA_FORCE_TP")) and dist.is_initialized()
         self.worker = None
         self.worker, self.shape, self.local_shape = build_tp_worker(

@@ -12,7 +12,7 @@
  *    (build with -ffp-contract=off); this matches the reference header as
  *    compiled for the host by g++ (the pin in tests/golden).  What nvcc's
  *    default -fmad=true would do on a CUDA device is not reproducible here and
- *    is stated as "unpinned" in DESIGN.md.
+ *    is stated as "unpinned".
  *  - fp16 <-> fp32 follows IEEE round-to-nearest-even, like CUDA __float2half_rn
  *    and half_float 2.2.0 (3rd_party/half/half.hpp:373-374).
  */
@@ -97,7 +97,7 @@ void orc_f2h_n(const float *src, orc_f16 *dst, size_t n)
 }
 
 /* ------------------------------------------------------- format registry */
-/* src/common/quant_types.h:11-174; sizes: SURVEY.md facts (sizeof checks).   */
+/* src/common/quant_types.h:11-174; sizes: sizeof checks.              */
 int orc_block_capacity(int dtype)
 {
     switch (dtype) {

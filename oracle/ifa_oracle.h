@@ -9,7 +9,7 @@
  * Parity pin: the block codecs are checked bit-for-bit against the reference's
  * own header (src/common/quantization.h) compiled on the host into
  * oracle/_ref/libifa_ref_quant.so (see oracle/Makefile, tests/golden/).
- * The reference ships no golden vectors or tests of its own (SURVEY.md §4).
+ * The reference ships no golden vectors or tests of its own.
  *
  * Every function cites the reference file:line it restates (paths relative
  * to the reference checkout).

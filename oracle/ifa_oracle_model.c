@@ -3,7 +3,7 @@
  *
  * Whole-model decoder forward with the reference's GPU-path semantics
  * (GpuInferenceWorker::Run, src/transformer/inference_worker.cc:234-340;
- * per-layer op order: SURVEY.md appendix B).  Every intermediate tensor is
+ * in the reference's per-layer op order).  Every intermediate tensor is
  * F16, activations are re-quantised to Q8_B32T2 before each eligible GEMV
  * (GetUseFullQuantGemv, inference_worker.cc:2707-2730), prefill rows go
  * through "dequantise the weight to half, fp32-accumulate" (MatrixMultiplication,

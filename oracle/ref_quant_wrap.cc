@@ -2,7 +2,7 @@
 // codecs, compiled from the sources where they lie (never copied):
 //   $(REF)/src/common/quantization.h, quant_types.h, data_types.h,
 //   $(REF)/3rd_party/half/half.hpp
-// Output: oracle/_ref/libifa_ref_quant.so (git-ignored; travels to the GPU box).
+// Output: oracle/_ref/libifa_ref_quant.so (git-ignored; travels to where the GPU is).
 // Test infrastructure only: pins oracle/ifa_oracle.c bit-for-bit and generates
 // tests/golden/*.npz (tests/golden/gen_golden.py).  Nothing in the product
 // path may load it.

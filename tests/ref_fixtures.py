@@ -1,7 +1,7 @@
 """Loader of the whole-model fixtures produced by the REFERENCE's CPU inference path (tests/golden/gen_model_fixtures.py,
 tests/golden/ref_model_*.npz) and the comparison rules shared by the CPU (oracle) and GPU (HIP engine) tests.
 
-Tolerance (SURVEY.md 8c): the reference CPU path runs F32 activations over the checkpoint's weights (ggml; RMS eps 1e-6),
+Tolerance: the reference CPU path runs F32 activations over the checkpoint's weights (ggml; RMS eps 1e-6),
 the GPU path rounds every op boundary to F16 (RMS eps 1e-5, appendix A5/A14), so logits are compared by cosine >= 0.999
 and max |delta| <= LOGIT_MAD (logits here reach |8|, where one F16 ulp is 0.0078), and a greedy id must equal the
 reference's whenever the reference's own top-2 gap exceeds LOGIT_TOL (a smaller gap is a tie at this precision); excused

@@ -1,4 +1,4 @@
-"""bench.py's watchdog (VERDICT r2 item 4a): a rank that makes no progress within a phase's limit ends the run with ONE
+"""bench.py's watchdog: a rank that makes no progress within a phase's limit ends the run with ONE
 JSON line carrying an "error" key on rank 0's stdout and a non-zero exit code -- a hang in communicator setup or in a
 collective must not cost the driver its whole scaling record."""
 import json
@@ -48,7 +48,7 @@ def test_disarmed_watchdog_lets_the_run_finish():
 
 def test_reference_cpu_baseline_picks_the_depth_the_host_can_hold():
     """bench.py's cpu_baseline is the reference's CPU path on ALL 32 layers when the host can hold the 26.4 GB F32 checkpoint twice
-    (file + the reference's heap), else the largest slice that fits -- and says which (VERDICT r4 item 7)"""
+    (file + the reference's heap), else the largest slice that fits -- and says which"""
     import importlib.util
     import os
     spec = importlib.util.spec_from_file_location("bench_mod", os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "bench.py"))

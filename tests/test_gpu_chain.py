@@ -59,7 +59,7 @@ def test_chained_launch_declines_shapes_it_has_no_kernel_for():
 
 
 def test_q3h_native_32_byte_stream_is_bit_identical_to_the_nibble_pair_stream():
-    """Option q3h_native (VERDICT r5 item 5): Wo / W1 / W3 / W2 of a Q3H_B64T1 model streamed at the format's own 32 bytes per 64
+    """Option q3h_native: Wo / W1 / W3 / W2 of a Q3H_B64T1 model streamed at the format's own 32 bytes per 64
     weights (pair codes decoded in the kernel: csrc/ifa_decode_formats.h WRowQ3HN) instead of the 36-byte nibble pairs: the same
     integer dots, so tokens, logits and KV rows must not change by a bit -- at Llama-2-7B widths (4096 / 11008 columns: one and
     three blocks per lane) and at a small GQA shape."""

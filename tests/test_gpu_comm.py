@@ -1,5 +1,5 @@
 """-m gpu: the collectives of the C ABI (csrc/ifa_comm.hip, RCCL) and the C-driven multi-GPU decode loop
-(ifa_model_tp_decode).  A 1-GPU box can only form a communicator of ONE rank (RCCL refuses two ranks on a device), which
+(ifa_model_tp_decode).  One GPU can only form a communicator of ONE rank (RCCL refuses two ranks on a device), which
 still runs every call through RCCL -- including inside the captured step; groups of 2+ ranks run where >= 2 GPUs are
 visible and skip cleanly otherwise.  The partition arithmetic of larger groups is covered on CPU (tests/test_tp_cpu.py)
 and with gloo ranks sharing one GPU (tests/test_gpu_tp.py)."""
@@ -60,7 +60,7 @@ def test_c_driven_tp_decode_equals_fused_decode_and_python_runner():
 
 def test_loopback_group_collectives_between_rank_threads():
     """ifa_comm_init_all with one device named n times: the in-process loopback group (what lets the multi-rank engine
-    paths run on a 1-GPU box).  Rank threads call the collectives concurrently, like the engine's rank threads."""
+    paths run on one GPU).  Rank threads call the collectives concurrently, like the engine's rank threads."""
     import ctypes as C
     import threading
     import inferflow_amd as ia
@@ -107,10 +107,10 @@ def test_loopback_group_collectives_between_rank_threads():
 
 @pytest.mark.parametrize("shape,tol", [("test_gqa", 0.03), ("test_moe", 0.05)], ids=["dense", "moe"])
 def test_batched_decode_over_a_tensor_parallel_group_matches_oracle(shape, tol):
-    """(moe: the Mixtral kind of step -- configs[4] -- experts sliced over the ranks like the dense FFN; the reference has no
-    tensor-parallel MoE to restate (SURVEY 8e): each rank accumulates its weighted expert products before the merge, the
+    """(moe: the Mixtral kind of step, experts sliced over the ranks like the dense FFN; the reference has no
+    tensor-parallel MoE to restate: each rank accumulates its weighted expert products before the merge, the
     oracle merges per expert, one more half rounding apart: stated bound 0.05.)
-    Dynamic batching under BY_TENSOR (configs[4] shape of work: several queries, one step, merges over [n][dim]): two
+    Dynamic batching under BY_TENSOR (several queries, one step, merges over [n][dim]): two
     rank threads on one GPU (loopback group), three queries on their own KV slots, every row against the oracle of its
     query with the merge restated and the T > 1 arithmetic (F16 activations) of a batched step."""
     import threading

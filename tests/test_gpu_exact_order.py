@@ -86,7 +86,7 @@ def test_exact_order_refuses_models_outside_the_step():
 def test_exact_order_mixture_of_experts_is_bit_identical_to_the_oracle(shape, wd, kvd, layers, steps):
     """Mixture-of-experts layers in the order-exact step: F16 router GEMV, 32-lane softmax, top-k by BuildRowsForMoE's rules, the
     selected experts' FFNs in ascending order, out x w + f accumulated as the oracle restates AddByRowIdx.  With both sides in ONE
-    summation order a router near tie is no longer a discontinuity between them (rounds 5's finding: at 32 random-init layers 55 of
+    summation order a router near tie is no longer a discontinuity between them (at 32 random-init layers 55 of
     56 rows ran different experts on the two sides): logits, ids and K / V rows are the oracle's bit for bit, free-running."""
     import oracle as o
     from inferflow_amd import synth

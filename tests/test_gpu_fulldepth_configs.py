@@ -1,5 +1,5 @@
-"""-m gpu: BASELINE configs[3] / configs[4] at FULL DEPTH against the oracle, in the form a one-GPU box allows,
-and SURVEY 8(c)'s own criterion -- identical greedy ids over >= 64 free-running steps -- on a model whose logits are well separated.
+"""-m gpu: Yi-34B, Falcon-40B and Mixtral-8x7B at FULL DEPTH against the oracle, in the form one GPU allows,
+and by identical greedy ids over >= 64 free-running steps, on a model whose logits are well separated.
 
   * Yi-34B Q4 (60 layers, 56 heads over 8 KV heads, ffn 20480, vocab 64000) through the PRODUCT surface with `devices = 0&0`: the C++
     InferenceEngine, two tensor-parallel workers on one device (in-process loopback group: the slicing, the two merges per layer, the
@@ -100,7 +100,7 @@ def test_yi_34b_all_60_layers_tensor_parallel_loopback_engine_matches_oracle(tmp
     if sep and tok != tok_o:
         id_fails.append("prompt")
     report = ["prompt: cos %.6f |dlogit| %.4f std" % (cos, mad)]
-    # the depth law with the constant THIS shape measures: 0.10 instead of the 7B model's 0.08 (r05 run, 60 layers: worst of six steps
+    # the depth law with the constant THIS shape measures: 0.10 instead of the 7B model's 0.08 (60 layers: worst of six steps
     # 0.636 std = 0.082 sqrt(60), the other five 0.35-0.55; rows of 7168 / 20480 values re-quantise 1.75x as many int8 blocks per
     # layer as the 7B widths and the maximum runs over 64000 logits instead of 32000)
     frac, cos_min = 0.10 * math.sqrt(N), 1.0 - 0.00005 - 0.00015 * N
@@ -124,7 +124,7 @@ def test_yi_34b_all_60_layers_tensor_parallel_loopback_engine_matches_oracle(tmp
 def test_mixtral_8x7b_width_eight_queries_tensor_parallel_loopback_engine_matches_oracle(tmp_path):
     """Mixtral-8x7B's widths through the product surface with `devices = 0&0` and EIGHT concurrent queries, FOUR layers deep: whole-model
     logits of a random-init mixture-of-experts model are comparable only while router near ties are rare -- at all 32 layers 55 of
-    56 rows met one (r05: profiles/r05_mixtral_routing_ties.log) and ran different experts on the two sides; at 4 layers most rows
+    56 rows met one (profiles/r05_mixtral_routing_ties.log) and ran different experts on the two sides; at 4 layers most rows
     are clean.  A row outside the law is excused only if the oracle's router margin of that row is a near tie (or an earlier row of the query
     already parted at one); at least half of the 56 rows must be inside the law.  The full DEPTH
     -- every one of the 32 layers against the oracle -- is tests/test_gpu_layerwise_oracle.py::...mixtral..."""
@@ -240,7 +240,7 @@ def test_falcon_40b_all_60_layers_fused_decode_matches_oracle():
 
 
 def test_peaky_llama2_7b_free_running_greedy_ids_are_identical_for_64_steps():
-    """"identical greedy tokens for >= 64 steps".  On the standard synthetic model the logits are flat (random lm_head:
+    """Identical greedy tokens for >= 64 steps.  On the standard synthetic model the logits are flat (random lm_head:
     top-2 gaps below the int8 re-quantisation noise), so ids part at near ties and the criterion cannot be shown.  Here the lm_head is
     TIED to a permutation of the embedding table and the embedding rows are large enough to carry through 32 random layers
     (synth.build embd_std / tied_lm_head): the one row aligned with the current token stands several logit-std above the other

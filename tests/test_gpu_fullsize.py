@@ -1,4 +1,4 @@
-"""-m gpu: BASELINE full-size checks (Llama-2-7B shapes, Q4_B32T1A) through
+"""-m gpu: full-size checks (Llama-2-7B shapes, Q4_B32T1A) through
 size-independent properties: fused == unfused bit for bit, decode is deterministic
 and idempotent w.r.t. the KV cache, the stream of tokens is identical with and
 without graph replay."""
@@ -64,7 +64,7 @@ def test_llama2_7b_width_other_formats_fused_equals_unfused(wd, kvd):
 def test_long_rows_fused_equals_unfused(shape, wd):
     """w2 rows of 20480 / 28672 / 32768 columns do not fit a lane's register image: the chunked, software-pipelined kernel
     (k_dec_gemv_long) must continue the same per-lane accumulation chain -> bit-identical to the op-level GEMV.
-    falcon_40b: full Falcon-40B widths (configs[3]): 8192 / 32768 columns, 128 heads of 64 over 8 KV heads, LayerNorm,
+    falcon_40b: full Falcon-40B widths: 8192 / 32768 columns, 128 heads of 64 over 8 KV heads, LayerNorm,
     GELU, plain MLP, shared MLP / attention input."""
     wk, _, s = synth.build(shape, wd, dt.F16, max_ctx=40, layers=2, vocab=8000)
     ok, why = wk.fused_supported()
@@ -81,7 +81,7 @@ def test_long_rows_fused_equals_unfused(shape, wd):
 
 
 def test_mixtral_8x7b_width_fused_equals_unfused_and_batched_rows_are_independent():
-    """configs[4] at its own widths: 8 experts of ffn 14336 (7 blocks per lane on w2's 14336 columns), top-2 routing, 32
+    """Mixtral-8x7B at its own widths: 8 experts of ffn 14336 (7 blocks per lane on w2's 14336 columns), top-2 routing, 32
     heads over 8 KV heads, 2 layers.  The fused MoE decode step == the op-by-op path bit for bit; a batched step of 8
     queries (the device-routed grouped path) gives every query the token its own single-query step gives."""
     wk, _, s = synth.build("mixtral_8x7b", dt.Q4_B32T1A, dt.F16, max_ctx=64, layers=2, vocab=8000)

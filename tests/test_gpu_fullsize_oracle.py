@@ -1,11 +1,11 @@
-"""-m gpu: the HEADLINE configurations against the oracle AT THEIR OWN SIZE (SURVEY.md section 8c "F4"
-and configs[2]): Llama-2-7B widths -- 32 x 128-wide heads, dim 4096, ffn 11008, the 32000 x 4096 lm_head --
+"""-m gpu: the HEADLINE configurations against the oracle AT THEIR OWN SIZE (4-bit weights with an F16 cache, 3.5-bit ones
+with an 8-bit cache): Llama-2-7B widths -- 32 x 128-wide heads, dim 4096, ffn 11008, the 32000 x 4096 lm_head --
   * Q4_B32T1A weights + F16 KV cache (the bench line's model), and
   * Q3H_B64T1 weights + Q8_B32T2 KV cache (the reference's 3.5-bit path),
 through the path bench.py times (graph replay of the wave-specialised GEMVs + the attention-tail launch), logits row AND greedy
 id of every step against oracle.Model on the SAME token history (the oracle's ids are fed to both sides).
 
-What can be promised at this depth, and why (tools/parity_depth.py prints the profile; DESIGN.md section 5):
+What can be promised at this depth, and why (tools/parity_depth.py prints the profile):
 the T = 1 path re-quantises its activations to int8 four times per layer (and, with a Q8 cache, the new K / V rows).  The two
 sides round the same values -- one layer, first tokens: |dlogit| <= 0.003 x std, cosine 1.000000 -- but they add fp32 terms in
 different orders (the oracle restates the reference's CUDA lane order, the kernels use wave64 orders; softmax and P.V sums grow
@@ -14,11 +14,11 @@ re-quantises that difference.  Measured (Q4 + F16 KV / Q3H + Q8 KV, worst of 7 s
 0.07 / 0.07 after 2, 0.09 / 0.13 after 4, 0.12 / 0.16 after 8, 0.17 / 0.20 after 16, 0.27 / 0.29 after 32 -- growth like
 sqrt(layers), no jump at any depth.  The test holds that law for the first N = 4 and N = 32 layers of the model,
     max |dlogit| <= 0.08 x sqrt(N) x std(oracle logits)      and      cosine >= 1 - 0.00005 - 0.00015 x N,
-and holds ONE layer (N = 1) to what one layer measures, not to the law's slack (VERDICT r4: 0.08 was 25x the figure of the first steps):
+and holds ONE layer (N = 1) to what one layer measures, not to the law's slack (0.08 was 25x the figure of the first steps):
     max |dlogit| <= 0.04 x std (F16 KV) / 0.06 x std (Q8 KV)      and      cosine >= 0.99995 / 0.9999.
 One layer measures 0.0015-0.003 x std on most steps and 0.028-0.03 on the steps where ONE int8 code of a re-quantised activation
 (the Wo or the W2 input: 127 levels per 32-value block) lands on the other side of a rounding tie -- step 7 of this very test with an
-F16 cache (r05 run: 0.0285), the third token with a Q8 cache (the cache row is one more int8 re-quantisation); 0.01 cannot be held by
+F16 cache (0.0285), the third token with a Q8 cache (the cache row is one more int8 re-quantisation); 0.01 cannot be held by
 two correct implementations that add fp32 terms in different orders, 0.04 / 0.06 is a single flip plus the usual figure;
 that every SINGLE layer of the 32 -- not only the first -- stays inside its one-layer figure is tests/test_gpu_layerwise_oracle.py,
 (std ~1.3: lm_head rows of std 0.02 over 4096 normalised values), and a greedy id must be the oracle's whenever the oracle's
@@ -118,11 +118,11 @@ def test_llama2_7b_widths_fused_decode_matches_oracle_at_depths_1_4_32(wd, kvd):
 
 @pytest.mark.parametrize("wd,kvd", [(dt.Q4_B32T1A, dt.F16), (dt.Q3H_B64T1, dt.Q8_B32T2)], ids=["q4_kvf16", "q3h_kvq8"])
 def test_llama2_7b_widths_order_exact_steps_are_bit_identical_to_the_oracle_through_32_layers(wd, kvd):
-    """SURVEY 8(c)'s bar for integer work, at the headline size: with option `exact_order` the worker runs every single-token step in the
+    """Integer work exactly, at the headline size: with option `exact_order` the worker runs every single-token step in the
     summation order of the reference's CUDA kernels (csrc/ifa_exact.hip: 32-lane int8 GEMV walk + xor butterfly, 128-chunk RMS norm,
     serial fp32 attention dots, 32-lane softmax; exp in glibc's algorithm, RoPE angles from the host libm) -- the order the oracle
-    restates.  Then nothing is left to a tolerance: through all 32 layers of configs[1] (Q4_B32T1A, F16 cache) and configs[2]
-    (Q3H_B64T1, Q8_B32T2 cache) the logits of every step, every greedy id, the last layer's output and the K / V rows of EVERY layer
+    restates.  Then nothing is left to a tolerance: through all 32 layers of Q4_B32T1A with an F16 cache and of
+    Q3H_B64T1 with a Q8_B32T2 cache the logits of every step, every greedy id, the last layer's output and the K / V rows of EVERY layer
     (for the Q8 cache: the int8 codes and scales of 4 re-quantisations per layer upstream of them) are the oracle's, bit for bit.
     This is what separates the depth law of the test above (half-ulp order differences of the timed kernels, compounding through
     the int8 re-quantisers) from an error: the same wiring, weights, quantisers and rounding points in the oracle's order have no
@@ -159,7 +159,7 @@ def test_llama2_7b_widths_order_exact_steps_are_bit_identical_to_the_oracle_thro
 
 
 def test_timed_ops_against_their_order_exact_forms_at_llama2_7b_size():
-    """The second link of the parity chain (VERDICT r5 item 6).  Link one: the worker's order-exact step equals the oracle bit for bit
+    """The second link of the parity chain.  Link one: the worker's order-exact step equals the oracle bit for bit
     through 32 layers (the test above).  Link two, here: every op of the timed path against its order-exact form (csrc/ifa_exact.hip,
     ifa_exact_*) on the SAME device inputs at Llama-2-7B size -- what one op's wave64 summation order costs, with nothing compounding:
       * RMS norm over 4096 values: <= 1 half ulp, <= 3 % of the values differ at all;
@@ -243,7 +243,7 @@ def test_timed_ops_against_their_order_exact_forms_at_llama2_7b_size():
 @pytest.mark.parametrize("wd", [dt.Q4_B32T1A, dt.Q3H_B64T1], ids=["q4", "q3h"])
 def test_llama2_7b_layer_blocks_on_the_device_equal_the_host_quantiser(wd):
     """The depth tests above multiply the blocks READ BACK from the worker (quantising 6.5 G weights on the host per case is half a
-    minute): a device quantiser or repack fault would then sit on both sides (ADVICE r5).  This closes that link at full width: the
+    minute): a device quantiser or repack fault would then sit on both sides.  This closes that link at full width: the
     seven matrices of two layers of the same synthetic model are generated again on the host side of the test (same seeds,
     inferflow_amd/synth.py), quantised by the ORACLE's quantiser (oracle.quantize: pinned to the reference header's bytes,
     tests/test_oracle_golden.py) and compared bit for bit with what ifa_model_get_tensor returns in the reference layout."""

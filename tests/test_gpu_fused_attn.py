@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     ("llama2_7b", dt.Q4_B32T1A, dt.F16, 4),        # headline widths (4 layers keep the test fast), 8 workgroups per head
-    ("llama2_7b", dt.Q3H_B64T1, dt.Q8_B32T2, 4),   # configs[2]: 3.5-bit weights, 8-bit KV cache
+    ("llama2_7b", dt.Q3H_B64T1, dt.Q8_B32T2, 4),   # 3.5-bit weights, 8-bit KV cache
     ("mixtral_dense_like", dt.Q4_B32T1A, dt.F16, 3),
 ]
 

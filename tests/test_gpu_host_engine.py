@@ -269,7 +269,7 @@ def test_per_tensor_weight_types_from_the_ini(tmp_path):
     eng.close()
 
 
-# ---- mixture of experts through the .ini surface (configs[4]; VERDICT r2 item 5)
+# ---- mixture of experts through the .ini surface
 @pytest.mark.parametrize("devices,tp_merge", [("0", 1), ("0&0", 2)], ids=["one_worker", "tensor_parallel_2"])
 def test_moe_safetensors_checkpoint_through_the_engine_matches_oracle(tmp_path, devices, tp_merge):
     """A Mixtral-named safetensors checkpoint (block_sparse_moe.gate / experts.{j}.w1|w2|w3, 4 experts, top-2) loaded by

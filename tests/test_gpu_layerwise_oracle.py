@@ -1,4 +1,4 @@
-"""-m gpu: LAYER-WISE, teacher-forced parity at Llama-2-7B size (VERDICT r4 "Next" 1a) -- a test where errors cannot compound.
+"""-m gpu: LAYER-WISE, teacher-forced parity at Llama-2-7B size -- a test where errors cannot compound.
 
 The whole-model comparisons (tests/test_gpu_fullsize_oracle.py) see the two sides only after 1, 4 or 32 layers have re-quantised
 each other's half-ulp differences; a fault that only shows in layers 2..32 would hide inside the depth law.  Here every one of the
@@ -42,9 +42,9 @@ def test_every_layer_of_llama2_7b_alone_on_the_oracles_state(wd, kvd, bound, per
 
 
 def test_every_layer_of_mixtral_8x7b_alone_on_the_oracles_state():
-    """configs[4]'s model at FULL depth (32 mixture-of-experts layers, 8 experts, top-2, 32 heads over 8 KV heads): whole-model logits
+    """Mixtral-8x7B at FULL depth (32 mixture-of-experts layers, 8 experts, top-2, 32 heads over 8 KV heads): whole-model logits
     cannot be compared at this depth -- with random-init routers 55 of 56 rows meet a router near tie in one of their 32 layers
-    and the two sides then run DIFFERENT experts (r05 run, profiles/r05_mixtral_routing_ties.log) -- but a layer alone has ONE
+    and the two sides then run DIFFERENT experts (profiles/r05_mixtral_routing_ties.log) -- but a layer alone has ONE
     routing decision per row: pairs whose oracle margin is a near tie are skipped (counted), every other layer must match."""
     try:
         import psutil

@@ -1,7 +1,7 @@
 """-m gpu: the one-shot all-reduce between PROCESSES (what `torchrun` ranks are): every rank exports the IPC handles of its inbox
 and flags (ifa_comm_oneshot_export), imports the peers' (hipIpcOpenMemHandle) and runs 30 all-reduces of decode-size vectors;
 results must equal the rank-order half sums bit for bit.  The ranks share device 0 -- cross-process mapping, epoch / parity
-protocol and arithmetic are what this covers; visibility between two DEVICES needs a multi-GPU box (bench.py compares the path
+protocol and arithmetic are what this covers; visibility between two DEVICES needs several GPUs (bench.py compares the path
 against RCCL there before using it)."""
 import os
 import subprocess

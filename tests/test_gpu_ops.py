@@ -147,7 +147,7 @@ def test_gemv_fp16_activation_path(d, rows, cols):
 # ------------------------------------------------- full-size property checks
 @pytest.mark.parametrize("rows,cols", [(4096, 4096), (11008, 4096), (4096, 11008)])
 def test_gemv_q4_full_size_against_dequantised_fp32(rows, cols):
-    """Llama-2-7B shapes (BASELINE configs[1]): the fused kernel must equal
+    """Llama-2-7B shapes: the fused kernel must equal
     dequant(W) @ dequant(x) computed in fp32 by torch on the same device."""
     torch.manual_seed(rows + cols)
     w = (torch.randn(rows, cols, device="cuda") * 0.02).half()

@@ -1,5 +1,5 @@
 """-m gpu: multi-GPU partitions INSIDE the C++ InferenceEngine (devices = 0&1 | 0;1 | 0&1;2&3: one worker + one host
-thread per GPU, the exchanges through the C ABI collectives), against the whole-model ORACLE.  A 1-GPU box runs the same
+thread per GPU, the exchanges through the C ABI collectives), against the whole-model ORACLE.  One GPU runs the same
 code path over a group of one (force_partition_path: rank thread, RCCL communicator of one rank, C-driven step with its
 collectives); the 2- and 4-GPU cases skip without the devices."""
 import numpy as np
@@ -133,7 +133,7 @@ def test_hybrid_2x2_matches_oracle(tmp_path):
 
 
 def test_query_batching_on_a_tensor_parallel_engine_matches_single_query_steps(tmp_path):
-    """Dynamic batching INSIDE a partitioned engine (VERDICT r2 item 5b; reference: query batching inside
+    """Dynamic batching INSIDE a partitioned engine (reference: query batching inside
     Infer_TensorParallelism, inference_engine.cc:1054-1124 + :1222-1296): three queries on "devices = 0&0" advance through
     ONE batched step per Infer() (ifa_model_tp_decode_batch on every rank) and reproduce what each gives alone."""
     ini, _ = fx.write_model_dir(str(tmp_path), fmt="llama2.c", wd="Q4", kvd="F16", ret="false", maxq=4, devices="0&0")

@@ -68,7 +68,7 @@ def test_perplexity_needs_output_tensors(tmp_path):
 
 
 def test_quantized_formats_rank_by_perplexity_on_the_f16_models_own_text(tmp_path):
-    """The tool's purpose (SURVEY §8 f2): compare formats.  Text = the F16 model's own greedy continuation, so the
+    """The tool's purpose: compare formats.  Text = the F16 model's own greedy continuation, so the
     F16 model scores it best and coarser formats score it no better than finer ones (up to noise)."""
     s = fx.SHAPE
     ini16, _ = fx.write_model_dir(str(tmp_path / "f16"), fmt="llama2.c", wd="F16", kvd="F16", ctx=128)

@@ -64,7 +64,7 @@ def test_service_shell_serves_token_id_queries(tmp_path):
             assert r["ret_code"] == "succ" and len(r["token_ids"]) == 12
         assert sum(r["token_ids"] == want for r in out) >= 3       # (a batched step runs T > 1 kernels: F16 activations may flip a near-tie)
         # more output than the context holds (prompt 9 + 500 > max_context_len 128): cut at what fits, the handler returns and
-        # the KV slot goes back -- asked maxq + 1 times, so a leaked slot would answer error.busy (ADVICE r4)
+        # the KV slot goes back -- asked maxq + 1 times, so a leaked slot would answer error.busy
         for _ in range(5):
             st, data = _post(port, "/", {"prompt_token_ids": prompt, "max_output_len": 500})
             r = json.loads(data)

@@ -143,7 +143,7 @@ def test_partitions_match_oracle(world, groups, shape, wd):
     lg_p, _, _, first = _run_ranks(world, groups=groups, shape=shape, wd=wd)
     lg_o, first_o, _, _ = _oracle_run(shape, n_decode=0, tp_merge=world // groups, wd=wd)
     if shape == "test_moe":
-        # the reference has no tensor-parallel MoE to restate (SURVEY 8e): each rank here accumulates its weighted expert
+        # the reference has no tensor-parallel MoE to restate: each rank here accumulates its weighted expert
         # products before the merge, the oracle merges per expert -- one more half rounding apart; stated bound 0.05
         cos = float((lg_p * lg_o).sum() / (np.linalg.norm(lg_p) * np.linalg.norm(lg_o)))
         assert cos >= 0.9995 and np.abs(lg_p - lg_o).max() <= 0.05

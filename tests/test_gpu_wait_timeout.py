@@ -1,4 +1,4 @@
-"""-m gpu: a bounded wait inside a launch that really times out on the device (ADVICE r5: codes 0x71 / 0x81 -> IFA_ERR_STATE ->
+"""-m gpu: a bounded wait inside a launch that really times out on the device (codes 0x71 / 0x81 -> IFA_ERR_STATE ->
 waits off -> the same call through the launches that do not wait).  Runs in a child process: the downgrade is process-wide."""
 import os
 import subprocess

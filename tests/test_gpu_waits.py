@@ -1,4 +1,4 @@
-"""-m gpu: the downgrade paths of ADVICE r4 / VERDICT r4 item 8 on the device.
+"""-m gpu: the downgrade paths on the device.
   * the MO-copy allocation fails inside the step that asked for it (simulated: option debug_mo_alloc_fail): the SAME step must
     still answer -- a 20-query step (which only the MO kernels serve as a fused step) falls to the op-by-op rows;
   * model options rows_kparts = 0 / gemm_splitk = 0: the launches whose workgroups wait for partner workgroups are never picked,
@@ -123,7 +123,7 @@ def test_rows_kparts_option_switches_the_waiting_launch_off(n):
 @pytest.mark.parametrize("n", [17, 24])
 def test_kparts_launches_inside_a_captured_batched_step(n):
     """The K-parts launches of a 17..32-query step under stream capture (no logits requested: the step is captured and replayed) --
-    found by tools/bench_batch.py in round 5: the launcher allocated its wait-error word (pinned host memory) at first use, which
+    found by tools/bench_batch.py: the launcher allocated its wait-error word (pinned host memory) at first use, which
     inside a thread-local capture fails and poisons the capture.  Captured and replayed steps must equal the eager step's ids."""
     wk, _, s = synth.build("test_longffn", dt.Q4_B32T1A, dt.F16, max_ctx=48, quant_threshold=0, std=0.06)
     V = s["vocab"]

@@ -60,7 +60,7 @@ def test_response_shapes():
     assert r["object"] == "chat.completion.chunk" and r["choices"][0]["delta"]["token_ids"] == [8] and r["choices"][0]["finish_reason"] is None
 
 
-# ---- the Infer / Commit loop over a host-only engine with InferenceEngine's query-table semantics (ADVICE r4: a query the
+# ---- the Infer / Commit loop over a host-only engine with InferenceEngine's query-table semantics (a query the
 # engine ends by itself -- context full -- produces no item; the handler used to wait for it forever and leak its KV slot)
 def _loop(max_ctx, prompt, max_output_len, eos=-1, n_requests=1, max_queries=2, fail_at=0, timeout_ms=3000):
     a = np.asarray(prompt, np.int32)
@@ -96,7 +96,7 @@ def test_eos_ends_with_finish_reason_stop():
 def test_prompt_that_leaves_no_room_is_refused():
     r = _loop(8, [1, 2, 3, 4, 5, 6, 7, 8], 4)[0]
     assert not r["ok"] and not r["hung"] and r["ret_code"] == "error.too_long_request" and r["active"] == 0
-    # a prompt of max_ctx - 1 tokens is what AddQuery still accepts: one token comes back (ADVICE r5: the shell used to refuse it)
+    # a prompt of max_ctx - 1 tokens is what AddQuery still accepts: one token comes back (the shell used to refuse it)
     r = _loop(8, [1, 2, 3, 4, 5, 6, 7], 4)[0]
     assert r["ok"] and not r["hung"] and r["ret_code"] == "succ" and r["token_ids"] == [8] and r["finish_reason"] == "length" and r["active"] == 0, r
 
@@ -112,7 +112,7 @@ def test_failed_engine_step_ends_the_query_with_an_error_and_frees_its_slot():
 
 def test_a_step_that_fails_once_is_run_again():
     # a recoverable failure (the worker's bounded in-launch wait gave up: "repeat it: the waiting launches are off now"): the loop runs
-    # the same step once more and no in-flight request is lost (ADVICE r5)
+    # the same step once more and no in-flight request is lost
     rs = _loop(64, [1, 2], 20, n_requests=3, max_queries=1, fail_at=3)
     for r in rs:
         assert r["ok"] and not r["hung"] and r["ret_code"] == "succ" and r["token_ids"] == list(range(3, 23)) and r["active"] == 0, r

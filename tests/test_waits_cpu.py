@@ -1,5 +1,5 @@
 """CPU: the residency rule behind every launch that waits for sibling workgroups INSIDE the launch (fused QKV + attention, split-K
-halves of the large-tile GEMM, K parts of the rows GEMM) -- VERDICT r4 item 8, ADVICE r4: such a launch is chosen only when its
+halves of the large-tile GEMM, K parts of the rows GEMM): such a launch is chosen only when its
 whole grid can be resident at once on the CUs this process may use; the CU count is mocked here (no device needed)."""
 import inferflow_amd as ia
 
@@ -29,7 +29,7 @@ def test_cu_masks_are_read():
     assert f(b"1:0-7", 0, 256) == 256                           # no entry for this device: everything
     assert f(b"garbage", 0, 256) == 256                         # unreadable: assume the device's own count
     assert f(b"0:0-511", 0, 256) == 256                         # never more than the device has
-    # a GPU LIST in front of the colon (ids and ranges): every listed device gets the mask (ADVICE r5)
+    # a GPU LIST in front of the colon (ids and ranges): every listed device gets the mask
     assert f(b"0,1:0-31", 1, 256) == 32 and f(b"0,2-3:0-15", 3, 256) == 16 and f(b"0,2-3:0-15", 1, 256) == 256
     # a mask that names GPUs in a form that cannot be read: conservative -- 0 CUs, so no launch that waits is chosen
     assert f(b"gpu0:0-31", 0, 256) == 0

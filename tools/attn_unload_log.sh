@@ -1,5 +1,5 @@
 #!/bin/bash
-# the measurements behind profiles/r06_attn_unload.log (GPU box, repo root)
+# the measurements behind profiles/r06_attn_unload.log (from the repository's root)
 OUT=gpurun_out/attn_unload; mkdir -p $OUT; L=$OUT/log; rm -f $L
 echo "# per-launch HIP-event averages (repeated launches: cache rows WARM) next to the rate of a real 16-step call (rows COLD), by context: tools/ctx_kernels.py (attn_unload 0)" >> $L
 IFA_CTXK_UNLOAD=0 timeout 300 python tools/ctx_kernels.py 2>&1 | grep context >> $L

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Prefill GEMM micro-benchmark (GPU box): TFLOP/s of ifa_gemm at Llama-2-7B shapes."""
+"""Prefill GEMM micro-benchmark: TFLOP/s of ifa_gemm at Llama-2-7B shapes."""
 import json, os, sys
 import torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))

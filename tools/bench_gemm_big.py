@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Large-T GEMM (GPU box): the in-tree large-tile MFMA kernel vs torch.matmul (hipBLASLt) on the dequantised operand -- a
+"""Large-T GEMM: the in-tree large-tile MFMA kernel vs torch.matmul (hipBLASLt) on the dequantised operand -- a
 measurement aid only, the library itself neither links nor loads a vendor GEMM -- with a correctness check of one against the
 other.  One JSON line per shape."""
 import json, os, sys

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Micro-benchmark of the GEMV kernels at Llama-2-7B shapes (GPU box only).
+"""Micro-benchmark of the GEMV kernels at Llama-2-7B shapes.
 Rotates over enough distinct weight copies to defeat the 256 MiB Infinity Cache.
 Prints one JSON line per variant: achieved algorithmic GB/s."""
 import json

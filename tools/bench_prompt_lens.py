@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Prefill rate by prompt length (Llama-2-7B Q4): the four large-tile launches per layer from `prefill_big_min` + 1 tokens on
-(option; 128 = round 4's rule) against the op-by-op layer below it.  IFA_PROMPT_LENS="48,64,96,128"  IFA_BIG_MINS="128,32" """
+(option; 128: an earlier rule) against the op-by-op layer below it.  IFA_PROMPT_LENS="48,64,96,128"  IFA_BIG_MINS="128,32" """
 import os, sys, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import numpy as np, torch

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Decode rate by context with the default options (16-step calls, best of 3): the table of DESIGN.md "Decode by context".
+"""Decode rate by context with the default options (16-step calls, best of 3).
     ctx_sweep.py [q8] [shape]"""
 import json, os, sys
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))

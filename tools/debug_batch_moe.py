@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Diagnosis aid (GPU box): the batched decode step of an MoE model at full width, option set by option set, every set run TWICE on a
+"""Diagnosis aid: the batched decode step of an MoE model at full width, option set by option set, every set run TWICE on a
 fixed (teacher-forced) token sequence: is the step deterministic, and which option removes an outlier row?
     python tools/debug_batch_moe.py [shape] [layers] [queries] [steps]"""
 import os

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Diagnosis aid (GPU box): MoE / GQA models at FULL WIDTH but few layers against the oracle, on one worker and through the
+"""Diagnosis aid: MoE / GQA models at FULL WIDTH but few layers against the oracle, on one worker and through the
 .ini engine with devices = 0&0, for prompts of 1..5 tokens -- which shape / path / prompt length parts from the oracle.
     python tools/debug_fulldepth.py [mixtral_8x7b|yi_34b] [layers]"""
 import json

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Diagnosis aid (GPU box): several queries registered BEFORE the first Infer() on an .ini engine (devices = 0 | 0&0), each checked
+"""Diagnosis aid: several queries registered BEFORE the first Infer() on an .ini engine (devices = 0 | 0&0), each checked
 against the oracle run on that query alone: prompt rows, then batched decode steps.
     python tools/debug_multiquery.py <shape> <layers> <nq>"""
 import json

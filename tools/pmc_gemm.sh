@@ -1,5 +1,5 @@
 #!/bin/bash
-# SQ counters of the prefill GEMM kernels (GPU box): bash tools/pmc_gemm.sh  -> gpurun_out/pmc_gemm.txt
+# SQ counters of the prefill GEMM kernels: bash tools/pmc_gemm.sh  -> gpurun_out/pmc_gemm.txt
 export TMPDIR=/tmp
 OUT=$PWD/gpurun_out/pmc_gemm
 rm -rf $OUT; mkdir -p $OUT

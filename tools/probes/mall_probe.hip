@@ -1,4 +1,4 @@
-// mall_probe.hip -- round 4: can the 256 MiB Infinity Cache hide a decode layer's weight stream behind the fixed
+// mall_probe.hip -- can the 256 MiB Infinity Cache hide a decode layer's weight stream behind the fixed
 // costs of its five dependent launches?
 //   A. bandwidth of a streaming read whose bytes were read once before (by default-policy or nt loads), by size and by
 //      how much other traffic came in between (retention);

@@ -1,5 +1,5 @@
 #!/bin/bash
-# per-kernel rocprofv3 averages of a short prompt's prefill (GPU box, repo root): LENS="64 128" MINS="128 32"
+# per-kernel rocprofv3 averages of a short prompt's prefill (from the repository's root): LENS="64 128" MINS="128 32"
 OUT=$PWD/gpurun_out/prof_prompt
 rm -rf $OUT; mkdir -p $OUT
 export TMPDIR=/tmp

@@ -1,5 +1,5 @@
 #!/bin/bash
-# per-kernel rocprofv3 averages of the batched step at a few batch sizes and of the Mixtral batch-8 step (GPU box, repo root)
+# per-kernel rocprofv3 averages of the batched step at a few batch sizes and of the Mixtral batch-8 step (from the repository's root)
 OUT=$PWD/gpurun_out/prof_batch
 rm -rf $OUT; mkdir -p $OUT
 export TMPDIR=/tmp

@@ -1,5 +1,5 @@
 #!/bin/bash
-# Round-2 profile set (run on the GPU box from the repo root; outputs under gpurun_out/prof_r02, copied to profiles/ by hand):
+# Profile set (from the repository's root; outputs under gpurun_out/prof_r02, copied to profiles/ by hand):
 #   1. rocprofv3 --kernel-trace --stats of the bench -> r02_rocprofv3_kernel_stats.csv
 #   2. PMC pass (own run, counters only): FETCH_SIZE -> r02_pmc_traffic.json (tools/pmc_summary.py)
 #   3. the bench line itself (after 2, so that it carries the traffic of THIS build) -> r02_bench_n1.json

@@ -1,5 +1,5 @@
 #!/bin/bash
-# Round-3 profile set (run on the GPU box from the repo root; outputs under gpurun_out/prof_r03, copied to profiles/ afterwards):
+# Profile set (from the repository's root; outputs under gpurun_out/prof_r03, copied to profiles/ afterwards):
 #   1. rocprofv3 --kernel-trace --stats of the bench                     -> r03_rocprofv3_kernel_stats.csv
 #   2. PMC pass (own run, counters only): FETCH_SIZE                     -> r03_pmc_traffic.json (tools/pmc_summary.py)
 #   3. the bench lines (after 2: they carry the traffic of THIS build)    -> r03_bench_n1.json, _q3h_q8, _q3h_f16, _mixtral

@@ -1,8 +1,8 @@
 #!/bin/bash
-# Round-6 profile set (GPU box, repo root; outputs under gpurun_out/prof_r06, the summaries are copied to profiles/ afterwards).
+# Profile set (from the repository's root; outputs under gpurun_out/prof_r06, the summaries are copied to profiles/ afterwards).
 # Run LAST: the PMC summary carries the hash of csrc/ (bench.py reports traffic: null for any other build).
 #   1. rocprofv3 --kernel-trace --stats of the bench (the driver's command: --steps 20 --warmup 5)  -> r06_rocprofv3_kernel_stats.csv
-#   2. PMC passes (own runs, counters only): FETCH_SIZE, headline config and configs[2]              -> r06_pmc_traffic.json, r06_pmc_q3h_q8_traffic.json
+#   2. PMC passes (own runs, counters only): FETCH_SIZE, headline config and 3.5-bit weights with an 8-bit cache              -> r06_pmc_traffic.json, r06_pmc_q3h_q8_traffic.json
 #   3. the bench lines (after 2: they carry the traffic of THIS build)                                -> r06_bench_n1.json (+ _steps128, _q3h_q8, _q3h_f16)
 #   4. per-phase traces of the fused launch and the four GEMVs                                        -> r06_fused_launch_phase_trace.log, r06_kernel_phase_trace.log
 #   5. A / B of the options that are still on the default path                                        -> r06_ab_options.log

@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """A / B of the native 32-byte Q3H_B64T1 stream (option q3h_native, csrc/ifa_decode_formats.h WRowQ3HN) against the 36-byte nibble-pair
-stream on configs[2] (Llama-2-7B widths, Q3H_B64T1 weights, Q8_B32T2 KV cache): HIP-event averages of the Wo / W1 | W3 / W2 launches
+stream on (Llama-2-7B widths, Q3H_B64T1 weights, Q8_B32T2 KV cache): HIP-event averages of the Wo / W1 | W3 / W2 launches
 (rotating over the 32 layers) and decode tokens/s, alternating on ONE box.
 
     python tools/q3h_native_ab.py [rounds]

@@ -1,6 +1,6 @@
 #!/bin/bash
 # Re-take the PMC traffic summary of the current build (it is tagged with the hash of the kernel sources: any csrc edit makes the
-# committed one stale and bench.py reports traffic: null) and the headline bench line.  GPU box, repo root; ~1 minute.
+# committed one stale and bench.py reports traffic: null) and the headline bench line.  From the repository's root; ~1 minute.
 set -x
 OUT=$PWD/gpurun_out/prof_r04
 mkdir -p $OUT; rm -rf $OUT/pmc

@@ -1,5 +1,5 @@
 #!/bin/bash
-# A / B of the preloaded weight pointers (round 5): the default library against lib_variants/gemvonly (k_dec_gemv preloads only, before k_dec_qkv_attn got them), alternating
+# A / B of the preloaded weight pointers: the default library against lib_variants/gemvonly (k_dec_gemv preloads only, before k_dec_qkv_attn got them), alternating
 for r in 1 2; do
   for v in default gemvonly; do
     if [ $v = default ]; then unset IFA_LIB; else export IFA_LIB=$PWD/lib_variants/$v/libinferflow_amd.so; fi

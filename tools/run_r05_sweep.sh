@@ -1,5 +1,5 @@
 #!/bin/bash
-# round-5 tuning run (GPU box): every library under lib_variants/ through the headline bench, the fused launch's phase stamps
+# tuning run: every library under lib_variants/ through the headline bench, the fused launch's phase stamps
 set -x
 mkdir -p gpurun_out
 rm -f gpurun_out/sweep.jsonl

@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Sweep workgroups-per-CU for the fused decode kernels (GPU box only)."""
+"""Sweep workgroups-per-CU for the fused decode kernels."""
 import json, os, sys
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import numpy as np
