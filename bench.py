@@ -275,7 +275,7 @@ def reference_cpu_baseline_7b_width(n_tokens=16, layers=32, with_gpu=True):
 
 class Watchdog:
     """A hang in communicator setup or in a collective must not cost the whole scaling record: every rank watches its own
-    progress and, when a phase overruns its limit, rank 0 prints ONE JSON line with an "error" key (the driver's contract)
+    progress and, when a phase overruns its limit, rank 0 prints ONE JSON line with an "error" key (what the caller of a run over several GPUs reads)
     and the process exits -- which makes the launcher tear the other ranks down.  Limits: IFA_BENCH_TIMEOUT_INIT /
     IFA_BENCH_TIMEOUT_STEP seconds."""
 

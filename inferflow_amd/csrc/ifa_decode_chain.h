@@ -7,10 +7,10 @@
 // with the row / prologue / epilogue code of k_dec_gemv (ifa_decode_kernels.h): the chain is bit-identical to the separate
 // launches (tests/test_gpu_chain.py).
 //
-// Why this and not the r3 / r4 forms.  A hand-off through memory costs ~3.3 us on this part (write-through store, visibility,
+// Why this and not the forms before it.  A hand-off through memory costs ~3.3 us on this part (write-through store, visibility,
 // one load round trip behind the CU's own queue) against ~2.5 us for a kernel boundary + first load (measured):
-// a fused launch only wins through what STREAMS during the hand-off.  The r3 engine streamed into a 112 KiB LDS ring and paid
-// for it with issue-bound consumer waves; the r4 fusions split the waves (or the CUs) into a front part and loaders, so the
+// a fused launch only wins through what STREAMS during the hand-off.  One streamed into a 112 KiB LDS ring and paid
+// for it with issue-bound consumer waves; others split the waves (or the CUs) into a front part and loaders, so the
 // front part's round trips queued behind the loaders' requests.  Here every wave is both: the register file is the ring
 // (512 KiB per CU; a wave keeps 6-17 KiB of the next op's rows in its own registers, the same registers and the same code
 // k_dec_gemv streams through at 7 TB/s), and a wave requests its next rows only after its own stores are out, so nothing of

@@ -470,7 +470,7 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
     if (logits_out) { if ((rc = matmul(m, hfin, T, lm, none, m->logits))) return rc; }
     else if (lm.dtype == F16 && D % 8 == 0 && D <= 8192) {
         // the last row only: the decode step's lm_head kernel on the normalised row (same per-row chain as the op-level GEMV --
-        // bit-identical logits -- at 6 TB/s instead of 1.1: 232 -> 45 us per prompt, rocprofv3 r06)
+        // bit-identical logits -- at 6 TB/s instead of 1.1: 232 -> 45 us per prompt, rocprofv3)
         DecLmHeadParams H2; memset(&H2, 0, sizeof(H2));
         H2.x = hfin + (size_t)t0 * D; H2.eps = c.eps; H2.cols = (int)D; H2.W = (const half_t *)lm.data; H2.logits = m->logits + (size_t)t0 * V; H2.rows = (int)V;
         if ((rc = launch_lmhead(H2, 0, m->opt_rpw_lm, m->stream))) return rc;

@@ -299,7 +299,7 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(half_t *__restrict__ q, h
     half_t *qrow = q + (size_t)t * q_row + (size_t)blockIdx.y * heads * head_dim;
     if (rope_cols == head_dim && head_dim % 16 == 0) {
         // eight pairs per thread through 16-byte accesses (the same expressions as `rotate`): a 128-token prompt spent 10 us per layer
-        // here in 2-byte loads and stores (rocprofv3 r06), now one round trip
+        // here in 2-byte loads and stores (rocprofv3), now one round trip
         typedef _Float16 h8 __attribute__((ext_vector_type(8)));
         const int per_head = half_dim / 8;
         for (int p = tid; p < heads * per_head; p += 256) {

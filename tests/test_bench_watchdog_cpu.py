@@ -1,6 +1,6 @@
 """bench.py's watchdog: a rank that makes no progress within a phase's limit ends the run with ONE
 JSON line carrying an "error" key on rank 0's stdout and a non-zero exit code -- a hang in communicator setup or in a
-collective must not cost the driver its whole scaling record."""
+collective must not cost a caller its whole scaling record."""
 import json
 import os
 import subprocess
