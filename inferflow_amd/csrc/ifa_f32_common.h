@@ -108,6 +108,33 @@ __device__ __forceinline__ float glu_of(int kind, float limit, float a, float u)
     }
     return (kind == 0 ? silu_exact(a) : (kind == 1 ? gelu_tanh_f(a) : fmaxf(a, 0.0f))) * u;
 }
+// one piece of eight columns of act(gate) up [* sigmoid(row_gate)] in bfloat16: gu's rows hold gate | up of F columns, out's are of ldo = 8 pieces, zero beyond F (VEC: both halves of gu's
+// rows on 16-byte boundaries)
+template <bool VEC>
+__device__ __forceinline__ void glu_piece(int kind, float limit, const float *__restrict__ gu, size_t ld, int F, const float *__restrict__ row_gate, size_t ldg, bf16_t *__restrict__ out,
+                                          int ldo, int pieces, size_t id)
+{
+    typedef __bf16 bf16x8g __attribute__((ext_vector_type(8)));
+    const size_t t = id / pieces;
+    const int c = (int)(id % pieces) * 8;
+    const float *g = gu + t * ld;
+    float a[8], u[8];
+    if (VEC && c + 8 <= F) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const float4 x = *reinterpret_cast<const float4 *>(g + c + 4 * h), y = *reinterpret_cast<const float4 *>(g + F + c + 4 * h);
+            a[4 * h] = x.x; a[4 * h + 1] = x.y; a[4 * h + 2] = x.z; a[4 * h + 3] = x.w; u[4 * h] = y.x; u[4 * h + 1] = y.y; u[4 * h + 2] = y.z; u[4 * h + 3] = y.w;
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) { a[e] = c + e < F ? g[c + e] : 0.0f; u[e] = c + e < F ? g[F + c + e] : 0.0f; }
+    }
+    const float rg = row_gate ? sigmoid_f(row_gate[t * ldg]) : 1.0f;
+    bf16x8g h;
+#pragma unroll
+    for (int e = 0; e < 8; e++) h[e] = (__bf16)(c + e < F ? glu_of(kind, limit, a[e], u[e]) * rg : 0.0f);
+    *reinterpret_cast<bf16x8g *>(out + t * ldo + c) = h;
+}
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.0f ? z : log1pf(expf(z)); }
 
 // First key position that the query at position i sees: a sliding window (window <= 0: none) and / or chunks of `chunk` positions counted from

@@ -365,6 +365,127 @@ __global__ void __launch_bounds__(1024) k_moe_sort(const int *__restrict__ idx, 
     }
 }
 
+// The same in two launches of many workgroups, for the choice by the largest logits (k_moe_route_top's, a wave a row): k_moe_route_count leaves, for each block of `rb` rows, how many of its
+// pairs chose each expert, k_moe_place adds these counts up and gives the pairs their places, in their order.  One workgroup took 7.8 us for 787 rows of 16 experts, top 4, and 13.6 for 2048:
+// the pairs come and go through one compute unit, and its threads' counters wait for each other.  At most 512 experts (LDS) and 256 blocks (a placing workgroup reads all their counts).
+constexpr int PLACE_EXPERTS = 512, PLACE_BLOCKS = 256, PLACE_WAVES = 16;
+size_t route_count_smem(int experts, int top) { return ((size_t)experts + PLACE_WAVES * (size_t)(experts + top)) * 4; }
+__global__ void __launch_bounds__(64 * PLACE_WAVES) k_moe_route_count(const float *__restrict__ logits, size_t ld, int experts, int top, int rows, int rb, int *__restrict__ idx,
+                                                                      float *__restrict__ wgt, int *__restrict__ counts)
+{
+    extern __shared__ int hist[];          // [experts] counts; per wave [experts] choice values, [top] weights before the division
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float *ch = (float *)(hist + experts) + wave * (experts + top), *pw = ch + experts;
+    auto in_order = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };          // (a wave's own LDS accesses)
+    for (int e = threadIdx.x; e < experts; e += 64 * PLACE_WAVES) hist[e] = 0;
+    __syncthreads();
+    for (int r = wave; r < rb; r += PLACE_WAVES) {
+        const int t = blockIdx.x * rb + r;
+        if (t >= rows) break;
+        const float *z = logits + (size_t)t * ld;
+        for (int e = lane; e < experts; e += 64) ch[e] = choice_of(z[e]);
+        in_order();
+        float first = 0.0f, sum = 0.0f;
+        for (int k = 0; k < top; k++) {
+            float best = -INFINITY; int bi = 0x7FFFFFFF;
+            for (int e = lane; e < experts; e += 64) { const float v = ch[e]; if (v > best || (v == best && e < bi)) { best = v; bi = e; } }
+            for (int o = 32; o > 0; o >>= 1) {
+                const float ov = __shfl_xor(best, o, 64); const int oi = __shfl_xor(bi, o, 64);
+                if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
+            }
+            if (k == 0) first = best;
+            const float p = expf(best - first);
+            sum += p;
+            if (lane == 0) { idx[(size_t)t * top + k] = bi; pw[k] = p; ch[bi] = NAN; atomicAdd(&hist[bi], 1); }
+            in_order();
+        }
+        for (int k = lane; k < top; k += 64) wgt[(size_t)t * top + k] = pw[k] / sum;
+        in_order();
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < experts; e += 64 * PLACE_WAVES) counts[(size_t)blockIdx.x * experts + e] = hist[e];
+}
+
+// what k_moe_sort leaves, and the counts of the blocks
+struct MoePlace { const int *idx; const float *wgt; int n_pairs, experts, top; int *a_rows, *pair_pos; float *w_sorted; int *tile_map, *n_tiles; int tile_rows; const int *counts; int blocks, rb; };
+size_t place_smem(int experts) { return (size_t)(2 + PLACE_WAVES) * experts * 4; }
+
+// workgroup `wg` places the pairs of PLACE_WAVES blocks, a block a wave; the first one leaves the tiles too
+__device__ void moe_place(const MoePlace &S, int wg, int *lds)
+{
+    const int E = S.experts, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b0 = wg * PLACE_WAVES, pad = E <= 1 ? 1 : 1 << (32 - __builtin_clz(E - 1));
+    int *all = lds, *before = lds + E, *mine = lds + (2 + wave) * E;
+    for (int e = tid; e < 2 * E; e += 64 * PLACE_WAVES) lds[e] = 0;
+    __syncthreads();
+    {
+        const int e = tid & (pad - 1);
+        int n = 0, f = 0;
+        if (e < E)
+            for (int b = tid / pad; b < S.blocks; b += 64 * PLACE_WAVES / pad) { const int c = S.counts[(size_t)b * E + e]; n += c; if (b < b0) f += c; }
+        if (n) atomicAdd(&all[e], n);
+        if (f) atomicAdd(&before[e], f);
+    }
+    __syncthreads();
+    if (wave == 0) {          // where an expert's range begins; its tiles
+        int from = 0, tiles = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + lane, n = e < E ? all[e] : 0, nt = (n + S.tile_rows - 1) / S.tile_rows;
+            int upto = n, t_upto = nt;
+#pragma unroll
+            for (int k = 1; k < 64; k <<= 1) {
+                const int x = __shfl_up(upto, k, 64), y = __shfl_up(t_upto, k, 64);
+                if (lane >= k) { upto += x; t_upto += y; }
+            }
+            const int o = from + upto - n;
+            if (e < E) before[e] += o;
+            if (wg == 0)
+                for (int k = 0; k < nt; k++) {
+                    int *tm = S.tile_map + 3 * (tiles + t_upto - nt + k);
+                    tm[0] = e; tm[1] = o + k * S.tile_rows; tm[2] = min(S.tile_rows, n - k * S.tile_rows);
+                }
+            from += __builtin_amdgcn_readlane(upto, 63); tiles += __builtin_amdgcn_readlane(t_upto, 63);
+        }
+        if (wg == 0 && lane == 0) *S.n_tiles = tiles;
+    }
+    __syncthreads();
+    for (int e = tid; e < E; e += 64 * PLACE_WAVES) {          // ... and each wave's part of it
+        int c[PLACE_WAVES], at = before[e];
+#pragma unroll
+        for (int w = 0; w < PLACE_WAVES; w++) c[w] = S.counts[(size_t)min(b0 + w, S.blocks - 1) * E + e];
+#pragma unroll
+        for (int w = 0; w < PLACE_WAVES; w++) { lds[(2 + w) * E + e] = at; at += c[w]; }
+    }
+    __syncthreads();
+    if (b0 + wave >= S.blocks) return;
+    const int p0 = (b0 + wave) * S.rb * S.top, p1 = min(S.n_pairs, p0 + S.rb * S.top), bits = 32 - __builtin_clz(E);          // (E itself stands for no pair)
+    for (int q = p0; q < p1; q += 64) {
+        const int p = q + lane, e = p < p1 ? S.idx[p] : E;
+        const float w = S.wgt[min(p, p1 - 1)];
+        uint64_t same = ~(uint64_t)0;          // the lanes of the same expert
+        for (int b = 0; b < bits; b++) { const uint64_t set = __builtin_amdgcn_ballot_w64(e >> b & 1); same &= e >> b & 1 ? set : ~set; }
+        const int earlier = __builtin_popcountll(same & (((uint64_t)1 << lane) - 1));
+        if (p < p1) {
+            const int pos = mine[e] + earlier;
+            S.a_rows[pos] = p / S.top; S.pair_pos[p] = pos; S.w_sorted[pos] = w;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (p < p1 && earlier == 0) mine[e] += __builtin_popcountll(same);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+}
+
+// ... beside the shared expert's activations (k_glu_to_bf16), which need as little of the choice: the first `placing` workgroups and the others
+struct MoeGlu { const float *gate_up; size_t ld; int F; const float *row_gate; size_t ldg; bf16_t *out; int ldo, pieces, vec; size_t total; };
+__global__ void __launch_bounds__(64 * PLACE_WAVES) k_moe_place_glu(MoePlace S, int placing, MoeGlu G)
+{
+    extern __shared__ int place_lds[];
+    if ((int)blockIdx.x < placing) { moe_place(S, blockIdx.x, place_lds); return; }
+    const size_t id = (size_t)(blockIdx.x - placing) * 1024 + threadIdx.x;
+    if (id >= G.total) return;
+    if (G.vec) glu_piece<true>(0, 0.0f, G.gate_up, G.ld, G.F, G.row_gate, G.ldg, G.out, G.ldo, G.pieces, id);
+    else glu_piece<false>(0, 0.0f, G.gate_up, G.ld, G.F, G.row_gate, G.ldg, G.out, G.ldo, G.pieces, id);
+}
+
 // y[t][c] (+)= sum_k (identity ? wgt h[t][c] : yp[pair_pos][c])  (the pair's weight is already inside yp)
 __global__ void __launch_bounds__(256) k_moe_combine(const float *__restrict__ h, size_t ldh, int W, int top, const int *__restrict__ pair_pos,
                                                      const float *__restrict__ wgt, const float *__restrict__ yp, int accumulate, float *__restrict__ y, size_t ldy)
@@ -477,6 +598,29 @@ static bool moe_in16(size_t rows, int width, int ff, int top, int ops32, const v
            && (((uintptr_t)up_bf16 | (uintptr_t)down_bf16) & 15) == 0;
 }
 
+// the workspace of a step's pairs (ff_ws: 3 ff of gated experts, whose first product leaves gate | up in front of the activations)
+struct MoeSpace { float *actb, *yp; int *a_rows, *pair_pos; float *w_sorted; int *tile_map, *n_tiles; };
+static MoeSpace moe_space(void *ws, size_t rows, int top, int width, int ff_ws, int experts)
+{
+    const size_t pairs = rows * (size_t)top;
+    char *b = (char *)ws;
+    MoeSpace s;
+    s.actb = (float *)b; b += al16(pairs * ff_ws * 4);
+    s.yp = (float *)b; b += al16(pairs * width * 4);
+    s.a_rows = (int *)b; b += al16(pairs * 4);
+    s.pair_pos = (int *)b; b += al16(pairs * 4);
+    s.w_sorted = (float *)b; b += al16(pairs * 4);
+    s.tile_map = (int *)b; b += al16(moe_tiles_max(rows, top, experts) * 12);
+    s.n_tiles = (int *)b;
+    return s;
+}
+
+// row tiles of bfloat16 experts' products, see moe_experts
+static int moe_tile_rows16(size_t pairs, int width, int experts)
+{
+    return pairs >= (size_t)256 * experts && pairs / 128 * (((size_t)width + 127) / 128) >= 256 ? 128 : 64;
+}
+
 static int moe_experts(const char *who, int gated, int glu_kind, float limit, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int identity, int top, int act,
                        const void *up_bf16, const void *down_bf16, const int *idx_dev, const void *wgt_f32, int ops32, void *ws, size_t ws_bytes,
                        void *y_f32, size_t ldy, int accumulate, ifa_stream stream, const RouteSel *sel = nullptr, const void *h_bf16 = nullptr)
@@ -489,15 +633,10 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
     IFA_REQUIRE(ws_bytes >= ifa_moe_workspace_bytes(rows, top, width, ff_ws, experts) && ((uintptr_t)ws & 15) == 0, "%s: workspace of %zu bytes, %zu needed", who, ws_bytes,
                 ifa_moe_workspace_bytes(rows, top, width, ff_ws, experts));
     const size_t pairs = rows * (size_t)top;
-    char *b = (char *)ws;
-    float *actb = (float *)b; b += al16(pairs * ff_ws * 4);
-    float *gub = actb + pairs * ff;                     // [pairs][2 ff] (gated experts, many rows)
-    float *yp = (float *)b; b += al16(pairs * width * 4);
-    int *a_rows = (int *)b; b += al16(pairs * 4);
-    int *pair_pos = (int *)b; b += al16(pairs * 4);
-    float *w_sorted = (float *)b; b += al16(pairs * 4);
-    int *tile_map = (int *)b; b += al16(moe_tiles_max(rows, top, experts) * 12);
-    int *n_tiles = (int *)b;
+    const MoeSpace at = moe_space(ws, rows, top, width, ff_ws, experts);
+    float *const actb = at.actb, *const gub = actb + pairs * ff;                     // gub: [pairs][2 ff] (gated experts, many rows)
+    float *const yp = at.yp, *const w_sorted = at.w_sorted;
+    int *const a_rows = at.a_rows, *const pair_pos = at.pair_pos, *const tile_map = at.tile_map, *const n_tiles = at.n_tiles;
     hipStream_t s = ifa_s(stream);
     const float *h = (const float *)h_f32;
     if (rows <= 8 || experts == 0) {
@@ -527,7 +666,7 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
     const size_t lda_h = ((size_t)width + 63) & ~(size_t)63, lda_f = ((size_t)ff + 63) & ~(size_t)63;
     const bool in16 = gated && moe_in16(rows, width, ff, top, ops32, up_bf16, down_bf16);
     IFA_REQUIRE(in16 || h_f32, "%s: rows in bfloat16 where the sizes need 32 bits", who);
-    const int tile_rows = in16 && pairs >= (size_t)256 * experts && pairs / 128 * (((size_t)width + 127) / 128) >= 256 ? 128 : 64;
+    const int tile_rows = in16 ? moe_tile_rows16(pairs, width, experts) : 64;
     const size_t max_tiles = (pairs + tile_rows - 1) / tile_rows + (size_t)experts;
     IFA_REQUIRE(max_tiles < 65536, "%s: %zu rows x %d choices exceed one step", who, rows, top);
     hipLaunchKernelGGL(k_moe_sort, dim3(1), dim3(1024), (size_t)(2 * experts + 1) * 4, s, idx_dev, (const float *)wgt_f32, (int)pairs, experts, top, a_rows, pair_pos, w_sorted,
@@ -614,4 +753,45 @@ int ifa_moe_experts_gated_bf16(const void *h_bf16, size_t rows, int width, int f
     IFA_REQUIRE(h_bf16 && ((uintptr_t)h_bf16 & 15) == 0 && experts > 0 && ifa_moe_gated_reads_bf16(rows, width, ff, top, 0, gate_up_bf16, down_bf16), "moe_experts_gated_bf16: bad shape");
     return moe_experts("moe_experts_gated_bf16", 1, 0, 0.0f, nullptr, (size_t)width, rows, width, ff, experts, 0, top, 0, gate_up_bf16, down_bf16, idx_dev, wgt_f32, 0, ws, ws_bytes, y_f32,
                        ldy, accumulate, stream, nullptr, h_bf16);
+}
+
+// Choice by the largest logits + the shared expert's activations + ifa_moe_experts_gated_bf16 without the sum of a row's pairs, which the norm behind it forms (ifa_norm_add_norm_moe): rows of
+// ifa_moe_gated_reads_bf16, at most 65535, of at most PLACE_EXPERTS experts.  us choice + sort + activations, before / now: 787 rows of 16 experts, top 4, 1408 shared columns
+// 4.7 + 7.8 + 5.5 / 5.9 + 5.5, 2048 rows 5.6 + 13.6 + 8.8 / 6.7 + 8.6
+int ifa_moe_prompt(const IfaMoePrompt &P, const int **pair_pos, const float **pair_rows, ifa_stream stream)
+{
+    const size_t pairs = P.rows * (size_t)P.top, lda_f = ((size_t)P.ff + 63) & ~(size_t)63;
+    IFA_REQUIRE(P.logits && P.h16 && P.idx && P.wgt && P.ws && P.gate_up && P.down && P.experts >= 1 && P.experts <= PLACE_EXPERTS && P.top >= 1 && P.top <= P.experts && P.rows > 0 && P.rows < 65536
+                && P.ldl >= (size_t)P.experts && ((uintptr_t)P.h16 & 15) == 0 && ifa_moe_gated_reads_bf16(P.rows, P.width, P.ff, P.top, 0, P.gate_up, P.down), "moe_prompt: bad arguments");
+    IFA_REQUIRE(!P.sh_ff || (P.sh_gate_up && P.sh_act && P.sh_ld >= 2 * (size_t)P.sh_ff && P.sh_ldo % 8 == 0 && P.sh_ldo >= (size_t)P.sh_ff && P.sh_ldo < (1u << 30) && ((uintptr_t)P.sh_act & 15) == 0),
+                "moe_prompt: bad shared expert");
+    IFA_REQUIRE(P.ws_bytes >= ifa_moe_workspace_bytes(P.rows, P.top, P.width, 3 * P.ff, P.experts) && ((uintptr_t)P.ws & 15) == 0, "moe_prompt: workspace of %zu bytes", P.ws_bytes);
+    const int tile_rows = moe_tile_rows16(pairs, P.width, P.experts);
+    const size_t max_tiles = (pairs + tile_rows - 1) / tile_rows + (size_t)P.experts;
+    IFA_REQUIRE(max_tiles < 65536, "moe_prompt: %zu rows x %d choices exceed one step", P.rows, P.top);
+    const MoeSpace at = moe_space(P.ws, P.rows, P.top, P.width, 3 * P.ff, P.experts);
+    // (the counts lie where experts of 32-bit rows have their gates and ups: 2 ff >= 128 values a pair, more than 32 a row and 512)
+    const int rb = PLACE_WAVES * (int)((P.rows + (size_t)PLACE_WAVES * PLACE_BLOCKS - 1) / ((size_t)PLACE_WAVES * PLACE_BLOCKS)), blocks = (int)((P.rows + rb - 1) / rb);
+    int *counts = (int *)(at.actb + pairs * P.ff);
+    const MoePlace S = {P.idx, P.wgt, (int)pairs, P.experts, P.top, at.a_rows, at.pair_pos, at.w_sorted, at.tile_map, at.n_tiles, tile_rows, counts, blocks, rb};
+    MoeGlu G;
+    memset(&G, 0, sizeof(G));
+    if (P.sh_ff) {
+        G.gate_up = P.sh_gate_up; G.ld = P.sh_ld; G.F = P.sh_ff; G.row_gate = P.sh_gate; G.ldg = P.sh_ldg; G.out = P.sh_act; G.ldo = (int)P.sh_ldo; G.pieces = (int)(P.sh_ldo / 8);
+        G.vec = P.sh_ld % 4 == 0 && P.sh_ff % 4 == 0 && ((uintptr_t)P.sh_gate_up & 15) == 0; G.total = P.rows * (size_t)G.pieces;
+    }
+    int rc;
+    const int placing = (blocks + PLACE_WAVES - 1) / PLACE_WAVES;
+    const size_t lds = route_count_smem(P.experts, P.top);
+    if (lds > 64 * 1024) IFA_HIP_CHECK(hipFuncSetAttribute((const void *)k_moe_route_count, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_moe_route_count, dim3((unsigned)blocks), dim3(64 * PLACE_WAVES), lds, ifa_s(stream), P.logits, P.ldl, P.experts, P.top, (int)P.rows, rb, P.idx, P.wgt, counts);
+    hipLaunchKernelGGL(k_moe_place_glu, dim3((unsigned)(placing + (G.total + 1023) / 1024)), dim3(64 * PLACE_WAVES), place_smem(P.experts), ifa_s(stream), S, placing, G);
+    IFA_LAUNCH_CHECK();
+    bf16_t *a16 = (bf16_t *)at.actb;
+    if ((rc = ifa_linear_bf16_grouped(P.gate_up, (size_t)2 * P.ff, (size_t)P.width, P.h16, (size_t)P.width, at.a_rows, at.tile_map, at.n_tiles, max_tiles, tile_rows, nullptr, nullptr, lda_f, 0,
+                                      0.0f, a16, stream))) return rc;
+    if ((rc = ifa_linear_bf16_grouped(P.down, (size_t)P.width, (size_t)P.ff, a16, lda_f, nullptr, at.tile_map, at.n_tiles, max_tiles, tile_rows, at.w_sorted, at.yp, (size_t)P.width, 0, 0.0f,
+                                      nullptr, stream))) return rc;
+    *pair_pos = at.pair_pos; *pair_rows = at.yp;
+    return IFA_OK;
 }

@@ -88,6 +88,16 @@ int ifa_attention_kv_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_he
 bool ifa_moe_gated_reads_bf16(size_t rows, int width, int ff, int top, int ops32, const void *gate_up_bf16, const void *down_bf16);
 int ifa_moe_experts_gated_bf16(const void *h_bf16, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16, const void *down_bf16, const int *idx_dev,
                                const void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream);
+// Prompts: choice by the largest logits, experts over bfloat16 rows (ifa_moe_gated_reads_bf16) without the sum of a row's pairs, and beside them the activations of a shared expert (sh_ff > 0):
+// sh_act[t] = silu(gate) up [* sigmoid(sh_gate[t * sh_ldg])] in bfloat16 rows of sh_ldo.  pair_pos [rows][top], pair_rows [pairs][width] (in ws): what ifa_norm_add_norm_moe adds up
+struct IfaMoePrompt {
+    const float *logits; size_t ldl, rows; int width, ff, experts, top; const ifa32::bf16_t *gate_up, *down, *h16; int *idx; float *wgt; void *ws; size_t ws_bytes;
+    const float *sh_gate_up; size_t sh_ld; int sh_ff; const float *sh_gate; size_t sh_ldg; ifa32::bf16_t *sh_act; size_t sh_ldo;
+};
+extern "C" int ifa_moe_prompt(const IfaMoePrompt &P, const int **pair_pos, const float **pair_rows, ifa_stream stream);
+// ifa_norm_add_norm_f32 / _to_bf16 (h_f32 or h_bf16) of the row  sum_k pair_rows[pair_pos[t][k]] (+ m[t])
+extern "C" int ifa_norm_add_norm_moe(void *x_f32, size_t ldx, size_t rows, size_t cols, const void *m_f32, size_t ldm, const int *pair_pos_dev, const void *pair_rows_f32, int top,
+                          const void *w_after_bf16, const void *w_before_bf16, float w_offset, float eps, void *h_f32, void *h_bf16, size_t ldh, ifa_stream stream);
 // ifa_moe_route_top_f32 inside the first launch of ifa_moe_experts_gated_f32: at most eight rows, 256 experts
 extern "C" int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
                                    const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream);
