@@ -16,6 +16,7 @@
 #include "ifa_f32_common.h"
 #include "inferflow_amd.h"
 #include "ifa_rows_fused.h"
+#include "ifa_chunkscan.h"
 
 using namespace ifa32;
 
@@ -604,7 +605,26 @@ __host__ __device__ __forceinline__ TileBlocks tile_blocks(int p0, int nq, int w
 }
 
 // marks, shares: where the blocks' marks and the chunks' partial results begin in the workspace (floats), behind the operands
-struct TileArgs { int n_seqs, hpw, cb, tiles; size_t marks, shares; };
+// few: a step's sequences, where there are up to FEW, and the chunks of those behind, the tiles and the operand blocks of those in front of each: tables in memory, each behind the other, were a
+// microsecond a trip in front of everything else
+constexpr int FEW = 4;
+struct FewSeq { SeqDesc sd; int chunk0, tile0, block0; };
+struct TileArgs { int n_seqs, hpw, cb, tiles; size_t marks, shares; int n_few; FewSeq few[FEW]; };
+// the sequence that holds an item, the first items of the sequences given by `at`
+template <class At>
+__device__ __forceinline__ FewSeq few_of(const TileArgs &A, int id, At at)
+{
+    FewSeq f = A.few[0];
+#pragma unroll
+    for (int s = 1; s < FEW; s++) if (s < A.n_few && id >= at(A.few[s])) f = A.few[s];
+    return f;
+}
+
+// The windowed attention's launches may bring the decayed linear attention's of the same layer with them (IfaLinearSide): chunk sums beside the keys' operands, the states from chunk to chunk
+// beside the tiles, the chunks' outputs beside the shares.  Alone, each of them left most of the chip idle: 601 rows of width 1024 (8 heads, 2 of keys) 4.6 + 6.3 + 15.2, 29.4 + 4.9 and
+// 9.2 + 12 us, together 16.0, 29.2 and 13.3; 2048 rows of width 2048 (16 heads, 4) 6.6 + 9.0 + 32, 140 + 10.6
+// and 13.4 + 27.4, together 42.7, 140.6 and 38.3
+struct SideArgs { ifachunk::ChunkArgs c; int chunks, zc, first, pass, per; };          // zc: pieces of 64 value columns; workgroups of the first and third launch, of the second (per: a head's)
 
 // The item (of n) that a number running over all items' counts falls into, or -1; id becomes the number inside it.  A wave looks at 64 items at a time (walked by one thread,
 // a step of 1024 sequences behind 100 keys each took 10.6 ms, now 0.37; 512 behind 200 2.0 ms, now 0.26).  count: called by all lanes, -1 for none.
@@ -642,8 +662,22 @@ __device__ __forceinline__ bool chunk_of(const WinAttnArgs &P, const TileArgs &A
 {
     const int lane = threadIdx.x & 63;
     auto chunks = [&](int pos0, int n, int tile) { return (tile_blocks(pos0 + tile * qw, min(qw, n - tile * qw), P.window, P.keep_first).nb + A.cb - 1) / A.cb; };
+    auto place = [&](const SeqDesc &sd) {          // (id: inside the sequence)
+        const int nt = (sd.n + qw - 1) / qw, back = item_of(nt, id, [&](int x) { return x >= 0 ? chunks(sd.pos0, sd.n, nt - 1 - x) : 0; });
+        at.sd = sd; at.chunk = id; at.tile = nt - 1 - back;
+        return back >= 0;
+    };
+    if (A.n_few) {
+        FewSeq f = A.few[0];          // (numbered from the last one on: its chunk0 is 0)
+#pragma unroll
+        for (int s = FEW - 1; s >= 0; s--) if (s < A.n_few && id >= A.few[s].chunk0) f = A.few[s];
+        id -= f.chunk0;
+        if (!place(f.sd)) return false;
+        at.block0 = f.block0; at.tile_g = f.tile0 + at.tile;
+        return true;
+    }
     int sq = 0;
-    if (A.n_seqs > 1) {
+    {
         const int back = item_of(A.n_seqs, id, [&](int x) {
             int pos0 = 0, n = 0, c = 0;
             if (x >= 0) { const SeqDesc &sd = P.seqs[A.n_seqs - 1 - x]; pos0 = sd.pos0; n = sd.n; }
@@ -661,9 +695,7 @@ __device__ __forceinline__ bool chunk_of(const WinAttnArgs &P, const TileArgs &A
         if (back < 0) return false;
         sq = A.n_seqs - 1 - back;
     }
-    const SeqDesc sd = P.seqs[sq];
-    const int nt = (sd.n + qw - 1) / qw, back = item_of(nt, id, [&](int x) { return x >= 0 ? chunks(sd.pos0, sd.n, nt - 1 - x) : 0; });
-    if (back < 0) return false;
+    if (!place(P.seqs[sq])) return false;
     int blocks = 0, tiles = 0;
     for (int s = lane; s < sq; s += 64) {
         const SeqDesc &b = P.seqs[s];
@@ -671,7 +703,6 @@ __device__ __forceinline__ bool chunk_of(const WinAttnArgs &P, const TileArgs &A
         tiles += (b.n + qw - 1) / qw;
     }
     if (sq > 0) { blocks = wave_sum_i(blocks); tiles = wave_sum_i(tiles); }
-    at.sd = sd; at.chunk = id; at.tile = nt - 1 - back;
     at.block0 = __builtin_amdgcn_readfirstlane(blocks);
     at.tile_g = __builtin_amdgcn_readfirstlane(tiles) + at.tile;
     return true;
@@ -681,68 +712,258 @@ __device__ __forceinline__ bool chunk_of(const WinAttnArgs &P, const TileArgs &A
 // values transposed (lane = 32 g + column, keys in the order in which the scores' accumulators hold them).  Columns beyond the rows' ends are zero.
 template <int NTK, int NTV> constexpr int kBlockPieces = 3 * 64 * (2 * NTK + 2 * NTV);
 
-// grid (kv heads, blocks of the step): the cache rows of a block into its operands -- once per layer and step, not once per tile that reads the block.
-// Bound by its launch and one trip to memory (reads 4, writes 6 bytes per value).  Rows past the sequence's last: that row again (their scores are masked).
-template <int NTK, int NTV>
-__global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, int n_seqs, uint32_t *__restrict__ marks)
+// One head of a row: its root mean square norm (with a weight), then the turn of its first rot_dims dimensions in pairs (see k_qk_rope_store); cs: [rot_dims / 2] cos, [rot_dims / 2] sin of
+// its position.  A wave; every lane reads both members of its pairs before anything is written, so that dst may be src (dim <= 64 CPL)
+template <int CPL>
+__device__ __forceinline__ void turn_head(const float *src, float *dst, int dim, bool norm, const bf16_t *nw_, float eps, int rot_dims, int pairing, const float *cs, int lane)
 {
-    constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK;
-    const int tid = threadIdx.x, kvh = blockIdx.x, dk = P.dim, dv = P.vdim;
-    int at = blockIdx.y;
-    const int sq = item_of(n_seqs, at, [&](int x) { if (x < 0) return 0; const SeqDesc &b = P.seqs[x]; return seq_blocks(b.pos0, b.n, P.window, P.keep_first).count; });
-    if (sq < 0) return;
-    const SeqDesc sd = P.seqs[sq];
-    const SeqBlocks sb = seq_blocks(sd.pos0, sd.n, P.window, P.keep_first);
-    const int kb0 = (at < sb.kept ? at : sb.first + at - sb.kept) * WT_K, last = sd.pos0 + sd.n - 1;
-    const size_t kvd = (size_t)P.kv_heads * dk, vvd = (size_t)P.kv_heads * dv;
-    gfloat *kc = (gfloat *)(P.slot_base[sd.slot] + P.k_off + (size_t)kvh * dk), *vc = (gfloat *)(P.slot_base[sd.slot] + P.v_off + (size_t)kvh * dv);
-    bf16x8w *dst = (bf16x8w *)P.ws + ((size_t)blockIdx.y * P.kv_heads + kvh) * kBlockPieces<NTK, NTV>;
-    const bool vec = dk % 4 == 0 && P.k_off % 4 == 0;      // (arena bases are 256-byte aligned)
-    bool odd = false;          // an infinity or NaN among the thread's values
-    for (int e = tid; e < WT_K * (DK / 8); e += 256) {
-        const int key = e / (DK / 8), c8 = e % (DK / 8), c = 8 * c8;
-        gfloat *row = kc + (size_t)min(kb0 + key, last) * kvd;
-        float v[8];
-        if (vec) {
-            const f32x4w lo = *(gf32x4 *)(row + min(c, dk - 4)), hi = *(gf32x4 *)(row + min(c + 4, dk - 4));
-#pragma unroll
-            for (int x = 0; x < 4; x++) { v[x] = c < dk ? lo[x] : 0.0f; v[4 + x] = c + 4 < dk ? hi[x] : 0.0f; }
-        } else {
-#pragma unroll
-            for (int x = 0; x < 8; x++) { const float f = row[min(c + x, dk - 1)]; v[x] = c + x < dk ? f : 0.0f; }
-        }
-        odd |= not_finite(v);
-        const Parts t = parts_of(v);
-#pragma unroll
-        for (int pl = 0; pl < 3; pl++) dst[(pl * KS + (c8 >> 1)) * 64 + 32 * (c8 & 1) + key] = t.p[pl];
+    const int half = rot_dims / 2;
+    float r = 1.0f;
+    if (norm) {
+        float s = 0.0f;
+        for (int c = lane; c < dim; c += 64) s = fmaf(src[c], src[c], s);
+        r = 1.0f / sqrtf(wave_sum(s) / (float)dim + eps);
     }
-    dst += 3 * KS * 64;
-    for (int e = tid; e < 4 * DV; e += 256) {
-        const int d = e % DV, sg = e / DV, k0 = 16 * (sg >> 1) + 4 * (sg & 1);
-        float v[8];
+    float val[CPL], oth[CPL];
 #pragma unroll
-        for (int x = 0; x < 8; x++) { const float f = vc[(size_t)min(kb0 + k0 + 8 * (x >> 2) + (x & 3), last) * vvd + min(d, dv - 1)]; v[x] = d < dv ? f : 0.0f; }
-        odd |= not_finite(v);
-        const Parts t = parts_of(v);
+    for (int e = 0; e < CPL; e++) {
+        const int c = lane + 64 * e;
+        val[e] = oth[e] = 0.0f;
+        if (c < dim) {
+            val[e] = src[c] * r * (nw_ ? bf2f(nw_[c]) : 1.0f);
+            if (c < rot_dims) { const int pc = pairing ? c ^ 1 : (c < half ? c + half : c - half); oth[e] = src[pc] * r * (nw_ ? bf2f(nw_[pc]) : 1.0f); }
+        }
+    }
 #pragma unroll
-        for (int pl = 0; pl < 3; pl++) dst[((pl * NTV + (d >> 5)) * 2 + (sg >> 1)) * 64 + 32 * (sg & 1) + (d & 31)] = t.p[pl];
+    for (int e = 0; e < CPL; e++) {
+        const int c = lane + 64 * e;
+        if (c >= dim) continue;
+        float out = val[e];
+        if (c < rot_dims) {
+            const bool first = pairing ? (c & 1) == 0 : c < half;          // first or second member of its pair
+            const int fi = pairing ? c >> 1 : (c < half ? c : c - half);
+            out = first ? val[e] * cs[fi] - oth[e] * cs[half + fi] : val[e] * cs[fi] + oth[e] * cs[half + fi];
+        }
+        dst[c] = out;
+    }
+}
+
+__device__ __forceinline__ void angle_of(int pos, const double *__restrict__ freq, int i, int half, float *cs)
+{
+    const double a = (double)pos * freq[i];
+    double sn, cn; sincos(a, &sn, &cn);          // (one argument reduction for both)
+    cs[i] = (float)cn; cs[half + i] = (float)sn;
+}
+
+// turn_head of a head of at most 128 that a wave holds, two values a lane (lane and lane + 64); w: the norm's weights (1: none), cs: the cosines and sines of the lane's pairs
+struct Turn { int half, from[2]; bool first[2]; float w[2]; };
+__device__ __forceinline__ Turn turn_of(int dim, int rot_dims, const bf16_t *nw_, int lane)
+{
+    Turn u;
+    u.half = rot_dims / 2;
+#pragma unroll
+    for (int e = 0; e < 2; e++) { const int c = lane + 64 * e; u.w[e] = nw_ ? bf2f(nw_[min(c, dim - 1)]) : 1.0f; u.first[e] = c < u.half; u.from[e] = c < u.half ? c + u.half : c - u.half; }
+    return u;
+}
+__device__ __forceinline__ void turn_held(float (&v)[2], const Turn &u, int dim, bool norm, float eps, int rot_dims, const float (&cv)[2], const float (&sv)[2], int lane)
+{
+    float r = 1.0f, val[2];
+    if (norm) {
+        float s = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 2; e++) if (lane + 64 * e < dim) s = fmaf(v[e], v[e], s);
+        r = 1.0f / sqrtf(wave_sum(s) / (float)dim + eps);
+    }
+#pragma unroll
+    for (int e = 0; e < 2; e++) val[e] = v[e] * r * u.w[e];
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const float a = __shfl(val[0], u.from[e] & 63, 64), b = __shfl(val[1], u.from[e] & 63, 64), oth = u.from[e] < 64 ? a : b;
+        v[e] = lane + 64 * e >= rot_dims ? val[e] : (u.first[e] ? val[e] * cv[e] - oth * sv[e] : val[e] * cv[e] + oth * sv[e]);
+    }
+}
+__device__ __forceinline__ void turn_angles(const float *cs, const Turn &u, int rot_dims, int lane, float (&cv)[2], float (&sv)[2])
+{
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const int c = lane + 64 * e, fi = u.first[e] ? c : c - u.half;
+        const bool in = c < rot_dims;
+        cv[e] = in ? cs[fi] : 1.0f; sv[e] = in ? cs[u.half + fi] : 0.0f;
+    }
+}
+
+// a row's heads in place, eight at a time, all their values asked for beside the row's place: a wave (cs: its own)
+template <class Pos>
+__device__ __forceinline__ void turn_row(float *q, int heads, int dim, const bf16_t *nw_, float eps, int rot_dims, const double *freq, float *cs, int lane, Pos position)
+{
+    constexpr int HB = 8;
+    const Turn u = turn_of(dim, rot_dims, nw_, lane);
+    float cv[2], sv[2];
+    for (int h0 = 0; h0 < heads; h0 += HB) {
+        float v[HB][2];
+#pragma unroll
+        for (int h = 0; h < HB; h++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) v[h][e] = q[(size_t)min(h0 + h, heads - 1) * dim + min(lane + 64 * e, dim - 1)];
+        if (h0 == 0) {
+            const int pos = position();
+            for (int i = lane; i < u.half; i += 64) angle_of(pos, freq, i, u.half, cs);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");          // (the wave's own)
+            turn_angles(cs, u, rot_dims, lane, cv, sv);
+        }
+#pragma unroll
+        for (int h = 0; h < HB; h++) {
+            turn_held(v[h], u, dim, nw_ != nullptr, eps, rot_dims, cv, sv, lane);
+#pragma unroll
+            for (int e = 0; e < 2; e++) if (h0 + h < heads && lane + 64 * e < dim) q[(size_t)(h0 + h) * dim + lane + 64 * e] = v[h][e];
+        }
+    }
+}
+
+// What a step brings to the cache (k null: nothing, or it is there already): keys as projected, normed and turned as k_kv_store_f32 and k_qk_rope_store do, and values; q_rows: the step's
+// queries are normed and turned in place, four rows a workgroup behind the blocks'.
+struct FreshKV { const float *k; size_t ldk; const float *v; size_t ldv; int norm; const bf16_t *norm_w; float eps; int rot_dims; const double *freq; int q_rows; const bf16_t *q_norm_w; float *q; };          // (q_rows 0: the queries are not turned)
+
+// A workgroup per (head of keys, block of the step, keys or values): the rows of a block into its operands -- once per layer and step, not once per tile that reads the block -- and those that the
+// step brings into the cache on their way: a position is in one of the step's blocks, and only there.  Keys go through LDS, all asked for at once.  Bound by its launch and its trips to
+// memory (reads 4, writes 6 bytes per value; fresh rows: 10).  Rows past the sequence's last: that row again (their scores are masked).
+// (A launch that stored the rows and one that read them back: 601 rows of 2 heads of 128 4.6 + 6.3 us; with 8 heads of queries turned 787 rows 8.4 + 6.6, 2048 11.6 + 7.1; now 11.2 and 13.7, the queries in the same launch.)
+template <int NTK, int NTV, bool SIDE>
+__global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, FreshKV F, int blocks, std::conditional_t<SIDE, SideArgs, int> side)
+{
+    constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK, KROW = DK + 4, VI = (4 * DV + 255) / 256;
+    int id = blockIdx.x;
+    if constexpr (SIDE) {
+        if (id < side.first) { ifachunk::linear_chunk(side.c, id % side.chunks, id / side.chunks % side.c.heads, id / side.chunks / side.c.heads); return; }
+        id -= side.first;
+    }
+    extern __shared__ __attribute__((aligned(16))) float part_lds[];          // [32][KROW], [32][rot_dims]
+    float *rows = part_lds, *cs = part_lds + WT_K * KROW;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = P.dim, dv = P.vdim, half = F.rot_dims / 2;
+    if constexpr (!SIDE)
+        if (id >= 2 * P.kv_heads * blocks) {          // queries, a row a wave
+            const int t = 4 * (id - 2 * P.kv_heads * blocks) + wave;
+            if (t < F.q_rows) turn_row(F.q + (size_t)t * P.ldq, P.heads, dk, F.q_norm_w, F.eps, F.rot_dims, F.freq, cs + wave * F.rot_dims, lane, [&]() {
+                    const SeqDesc sd = A.n_few ? few_of(A, t, [](const FewSeq &x) { return x.sd.row0; }).sd : P.seqs[P.row_seq[t]];
+                    return sd.pos0 + t - sd.row0;
+                });
+            return;
+        }
+    const bool keys = (id & 1) == 0;
+    const int kvh = (id >> 1) % P.kv_heads, place = (id >> 1) / P.kv_heads;
+    int at = place;
+    SeqDesc sd;
+    if (A.n_few) { const FewSeq f = few_of(A, place, [](const FewSeq &x) { return x.block0; }); sd = f.sd; at -= f.block0; }
+    else {
+        const int sq = item_of(A.n_seqs, at, [&](int x) { if (x < 0) return 0; const SeqDesc &b = P.seqs[x]; return seq_blocks(b.pos0, b.n, P.window, P.keep_first).count; });
+        if (sq < 0) return;
+        sd = P.seqs[sq];
+    }
+    const SeqBlocks sb = seq_blocks(sd.pos0, sd.n, P.window, P.keep_first);
+    const int kb0 = (at < sb.kept ? at : sb.first + at - sb.kept) * WT_K, last = sd.pos0 + sd.n - 1, fresh0 = F.k ? sd.pos0 : 0x7FFFFFFF;          // positions from fresh0 on are the step's
+    typedef __attribute__((address_space(1))) float gfloat_w;
+    bf16x8w *dst = (bf16x8w *)P.ws + ((size_t)place * P.kv_heads + kvh) * kBlockPieces<NTK, NTV>;
+    bool odd = false;          // an infinity or NaN among the thread's values
+    if (keys) {
+        const size_t kvd = (size_t)P.kv_heads * dk;
+        gfloat_w *kc = (gfloat_w *)(P.slot_base[sd.slot] + P.k_off + (size_t)kvh * dk);
+        constexpr int KW = WT_K / 4;          // keys a wave, two values of each a lane
+        float v[KW][2];
+#pragma unroll
+        for (int x = 0; x < KW; x++) {
+            const int j = min(kb0 + KW * wave + x, last);
+            gfloat *row = (gfloat *)F.k + (size_t)(sd.row0 + j - sd.pos0) * F.ldk + (size_t)kvh * dk;
+            if (kb0 < fresh0 && j < fresh0) row = (gfloat *)kc + (size_t)j * kvd;          // (blocks of the step alone do not wait for the slot's place)
+#pragma unroll
+            for (int e = 0; e < 2; e++) v[x][e] = row[min(lane + 64 * e, dk - 1)];
+        }
+        const Turn u = turn_of(dk, F.rot_dims, F.norm_w, lane);
+        if (kb0 + WT_K > fresh0) {
+            for (int e = lane; e < KW * half; e += 64) { const int key = KW * wave + e / half; angle_of(kb0 + key, F.freq, e % half, half, cs + key * F.rot_dims); }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");          // (the wave's own)
+        }
+#pragma unroll
+        for (int x = 0; x < KW; x++) {
+            const int key = KW * wave + x, j = kb0 + key;
+            if (min(j, last) >= fresh0) {          // (beyond the last: turned by another angle, masked like the row again)
+                float cv[2], sv[2];
+                turn_angles(cs + key * F.rot_dims, u, F.rot_dims, lane, cv, sv);
+                turn_held(v[x], u, dk, F.norm != 0, F.eps, F.rot_dims, cv, sv, lane);
+            }
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int c = lane + 64 * e;
+                if (c < DK) rows[key * KROW + c] = c < dk ? v[x][e] : 0.0f;
+                if (c < dk && j >= fresh0 && j <= last) kc[(size_t)j * kvd + c] = v[x][e];
+            }
+        }
+        __syncthreads();
+        for (int e = tid; e < WT_K * (DK / 8); e += 256) {
+            const int key = e / (DK / 8), c8 = e % (DK / 8);
+            const float *row = rows + key * KROW + 8 * c8;
+            float f[8];
+            const f32x4w lo = *(const f32x4w *)row, hi = *(const f32x4w *)(row + 4);
+#pragma unroll
+            for (int x = 0; x < 4; x++) { f[x] = lo[x]; f[4 + x] = hi[x]; }
+            odd |= not_finite(f);
+            const Parts t = parts_of(f);
+#pragma unroll
+            for (int pl = 0; pl < 3; pl++) dst[(pl * KS + (c8 >> 1)) * 64 + 32 * (c8 & 1) + key] = t.p[pl];
+        }
+    } else {
+        const size_t vvd = (size_t)P.kv_heads * dv;
+        gfloat_w *vc = (gfloat_w *)(P.slot_base[sd.slot] + P.v_off + (size_t)kvh * dv);
+        float v[VI][8];
+#pragma unroll
+        for (int u = 0; u < VI; u++) {
+            const int e = min(tid + 256 * u, 4 * DV - 1), d = e % DV, sg = e / DV, k0 = 16 * (sg >> 1) + 4 * (sg & 1);
+#pragma unroll
+            for (int x = 0; x < 8; x++) {
+                const int j = min(kb0 + k0 + 8 * (x >> 2) + (x & 3), last);
+                gfloat *row = (gfloat *)F.v + (size_t)(sd.row0 + j - sd.pos0) * F.ldv + (size_t)kvh * dv;
+                if (kb0 < fresh0 && j < fresh0) row = (gfloat *)vc + (size_t)j * vvd;
+                v[u][x] = row[min(d, dv - 1)];
+            }
+        }
+        dst += 3 * KS * 64;
+#pragma unroll
+        for (int u = 0; u < VI; u++) {
+            const int e = tid + 256 * u, d = e % DV, sg = e / DV, k0 = 16 * (sg >> 1) + 4 * (sg & 1);
+            if (e >= 4 * DV) break;
+#pragma unroll
+            for (int x = 0; x < 8; x++) {
+                const int j = kb0 + k0 + 8 * (x >> 2) + (x & 3);
+                if (j >= fresh0 && j <= last && d < dv) vc[(size_t)j * vvd + d] = v[u][x];
+                if (d >= dv) v[u][x] = 0.0f;
+            }
+            odd |= not_finite(v[u]);
+            const Parts t = parts_of(v[u]);
+#pragma unroll
+            for (int pl = 0; pl < 3; pl++) dst[((pl * NTV + (d >> 5)) * 2 + (sg >> 1)) * 64 + 32 * (sg & 1) + (d & 31)] = t.p[pl];
+        }
     }
     const int any = __syncthreads_or(odd);
-    if (tid == 0) marks[(size_t)blockIdx.y * P.kv_heads + kvh] = any ? 1u : 0u;
+    if (tid == 0) ((uint32_t *)(P.ws + A.marks))[2 * ((size_t)place * P.kv_heads + kvh) + (keys ? 0 : 1)] = any ? 1u : 0u;
 }
 
 // Key rows of dim <= 32 NTK and value rows of vdim <= 32 NTV floats.  VEC: rows of whole, aligned 16-byte pieces in q and the output.
 template <int NTK, int NTV, bool VEC>
-__global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, TileArgs A)
+__global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, TileArgs A, int hx, int groups, SideArgs side)
 {
     constexpr int KS = 2 * NTK, PIECES = kBlockPieces<NTK, NTV>;
+    const int bx = blockIdx.x % hx, by = blockIdx.x / hx;
+    if (by >= groups) {
+        const int id = blockIdx.x - hx * groups, e = id % side.per * (64 * WT_WAVES) + threadIdx.x;
+        if (e < side.c.dk * side.c.dv) ifachunk::linear_pass(side.c, e, id / side.per % side.c.heads, id / side.per / side.c.heads);
+        return;
+    }
     extern __shared__ bf16x8w ops[];                          // two blocks' operands, then a bias table per wave
     float *bias = (float *)(ops + 2 * PIECES) + 64 * (threadIdx.x >> 6);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 31, g = lane >> 5;
-    const int h = blockIdx.x * A.hpw + wave % A.hpw, qsub = wave / A.hpw, kvh = blockIdx.x * A.hpw / (P.heads / P.kv_heads), dk = P.dim, dv = P.vdim;
+    const int h = bx * A.hpw + wave % A.hpw, qsub = wave / A.hpw, kvh = bx * A.hpw / (P.heads / P.kv_heads), dk = P.dim, dv = P.vdim;
     const int qw = 32 * (WT_WAVES / A.hpw);
     ChunkPlace at;
-    if (!chunk_of(P, A, qw, blockIdx.y, at)) return;
+    if (!chunk_of(P, A, qw, by, at)) return;
     const SeqDesc sd = at.sd;
     const int tile = at.tile, tile_g = at.tile_g, chunk = at.chunk, block0 = at.block0;
     const int r0 = sd.row0 + tile * qw, nq = min(qw, sd.n - tile * qw), p0 = sd.pos0 + tile * qw;
@@ -767,8 +988,9 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
     // which of the chunk's blocks (64 at a time) have a mark
     auto marked = [&](int b) -> uint64_t {
         const int x = min(b + lane, b1 - 1), block = x < tb.kept ? x : tb.first + x - tb.kept, at = block < sb.kept ? block : sb.kept + block - sb.first;
-        const uint32_t m = ((const __attribute__((address_space(1))) uint32_t *)(P.ws + A.marks))[(size_t)(block0 + at) * P.kv_heads + kvh];
-        return __builtin_amdgcn_ballot_w64(m != 0 && b + lane < b1);
+        typedef uint32_t u32x2w __attribute__((ext_vector_type(2)));          // (its keys, its values)
+        const u32x2w m = ((const __attribute__((address_space(1))) u32x2w *)(P.ws + A.marks))[(size_t)(block0 + at) * P.kv_heads + kvh];
+        return __builtin_amdgcn_ballot_w64((m[0] | m[1]) != 0 && b + lane < b1);
     };
     uint64_t odd = marked(b0);
     // the lane's query, normed, in three parts (queries past the tile's last: that one again, not stored)
@@ -909,7 +1131,7 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
     // the lane holds value columns 32 nt + (r & 3) + 8 (r >> 2) + 4 g of its query
     const float ls = l + __shfl_xor(l, 32, 64);
     if (nch > 1) {                       // this chunk's share: [maximum][sum][columns] x 32 queries
-        float *dst = P.ws + A.shares + ((((size_t)tile_g * gridDim.x + blockIdx.x) * P.nsplit + chunk) * WT_WAVES + wave) * 32 * (dv + 2) + i;
+        float *dst = P.ws + A.shares + ((((size_t)tile_g * hx + bx) * P.nsplit + chunk) * WT_WAVES + wave) * 32 * (dv + 2) + i;
         if (g == 0) { dst[0] = m; dst[32] = ls; }
 #pragma unroll
         for (int nt = 0; nt < NTV; nt++)
@@ -957,26 +1179,30 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
         }
 }
 
-// the chunks' shares of 32 queries of a head and its sink into the output rows: grid (heads / hpw, tiles, waves of k_attn_tile x 4), 32 value columns a workgroup.
+// the chunks' shares of 32 queries of a head and its sink into the output rows: 256 threads for head group bx (of hx), tile tile_g and z (waves of k_attn_tile x 4), 32 value columns a workgroup.
 // A chain of requests (the sequence, the maxima, the shares), not their bytes: the shares of four chunks are asked for beside the maxima, which all threads fetch, and four workgroups do what one
 // did for all 128 columns, two chunks at a time.  us: Sopulorn 2048 tokens 13.7 -> 11.0, three prompts of 730 in all 10.4 -> 6.9; Gelarax 2048 of width 2048 13.7 -> 12.1, 601 of width 1024
 // 11.3 -> 9.0.  (The shares of all 32 possible chunks asked for at once: 208 registers, twice as long.)
 constexpr int WC_COLS = 32;
-__global__ void __launch_bounds__(256) k_attn_tile_combine(WinAttnArgs P, TileArgs A)
+__device__ __forceinline__ void tile_combine(const WinAttnArgs &P, const TileArgs &A, int hx, int bx, int tile_g, int z)
 {
     __shared__ float ms[WT_MAX_CHUNKS][32], ls[WT_MAX_CHUNKS][32], rows[32][WC_COLS + 1];
-    const int tid = threadIdx.x, wave = blockIdx.z % WT_WAVES, c0 = blockIdx.z / WT_WAVES * WC_COLS, h = blockIdx.x * A.hpw + wave % A.hpw, qsub = wave / A.hpw, dv = P.vdim;
-    const int qw = 32 * (WT_WAVES / A.hpw), tile_g = blockIdx.y, ncol = min(WC_COLS, dv - c0);
+    const int tid = threadIdx.x, wave = z % WT_WAVES, c0 = z / WT_WAVES * WC_COLS, h = bx * A.hpw + wave % A.hpw, qsub = wave / A.hpw, dv = P.vdim;
+    const int qw = 32 * (WT_WAVES / A.hpw), ncol = min(WC_COLS, dv - c0);
     int tile = tile_g;
-    const int sq = item_of(A.n_seqs, tile, [&](int x) { return x >= 0 ? (P.seqs[x].n + qw - 1) / qw : 0; });
-    if (sq < 0) return;
-    const SeqDesc sd = P.seqs[sq];
+    SeqDesc sd;
+    if (A.n_few) { const FewSeq f = few_of(A, tile_g, [](const FewSeq &x) { return x.tile0; }); sd = f.sd; tile -= f.tile0; }
+    else {
+        const int sq = item_of(A.n_seqs, tile, [&](int x) { return x >= 0 ? (P.seqs[x].n + qw - 1) / qw : 0; });
+        if (sq < 0) return;
+        sd = P.seqs[sq];
+    }
     const int nq = min(qw, sd.n - tile * qw), nq_w = min(32, nq - 32 * qsub);
     const int nch = (tile_blocks(sd.pos0 + tile * qw, nq, P.window, P.keep_first).nb + A.cb - 1) / A.cb;
     if (nch <= 1 || nq_w <= 0) return;
     const int share = WT_WAVES * 32 * (dv + 2), q = tid & 31, nowhere = nch * share * 4;
     // (requests behind the last chunk return zeros, without traffic)
-    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(P.ws + A.shares + (((size_t)tile_g * gridDim.x + blockIdx.x) * P.nsplit * WT_WAVES + wave) * 32 * (dv + 2), 0,
+    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(P.ws + A.shares + (((size_t)tile_g * hx + bx) * P.nsplit * WT_WAVES + wave) * 32 * (dv + 2), 0,
                                                                          nowhere, 0x00020000);
     auto at = [&](int c, int piece) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(src, c < nch ? (c * share + piece * 32 + q) * 4 : nowhere, 0, 0)); };
     // four chunks of shares beside the maxima and sums (thread: query q, chunks j, j + 8 ..), then four at a time
@@ -1023,6 +1249,18 @@ __global__ void __launch_bounds__(256) k_attn_tile_combine(WinAttnArgs P, TileAr
     }
 }
 
+__global__ void __launch_bounds__(256) k_attn_tile_combine(WinAttnArgs P, TileArgs A) { tile_combine(P, A, gridDim.x, blockIdx.x, blockIdx.y, blockIdx.z); }
+
+// ... behind the chunks' outputs of the linear attention beside it
+template <int DK, bool VEC>
+__global__ void __launch_bounds__(256, ifachunk::chunk_out_waves(0, DK)) k_attn_join_out(WinAttnArgs P, TileArgs A, SideArgs side, int hx)
+{
+    int id = blockIdx.x;
+    if (id < side.first) { ifachunk::chunk_out<0, DK, VEC>(side.c, id % side.chunks, id / side.chunks % side.c.heads, id / side.chunks / side.c.heads); return; }
+    id -= side.first;
+    tile_combine(P, A, hx, id % hx, id / hx % A.tiles, id / hx / A.tiles);
+}
+
 // How a step's tiles are shared out: hpw query heads and qw queries per workgroup, cb key blocks per chunk, up to `chunks` chunks per tile, so that the
 // chunks just fill the compute units once (one workgroup each: registers and LDS); below two blocks a chunk the partial results cost more than
 // the wait they save.  op_bytes: workspace of the blocks' operands and marks (from mark_at on), bytes: with the chunks' shares (none with one chunk).
@@ -1045,7 +1283,7 @@ TilePlan tile_plan(const ifa_seq_desc *sh, int n_seqs, int heads, int kv_heads, 
     }
     t.tiles = nbs.size();
     t.mark_at = t.blocks * (size_t)kv_heads * 3 * 64 * 16 * (size_t)(2 * NTK + 2 * NTV);
-    t.op_bytes = t.mark_at + (t.blocks * (size_t)kv_heads * 4 + 15) / 16 * 16;
+    t.op_bytes = t.mark_at + (t.blocks * (size_t)kv_heads * 8 + 15) / 16 * 16;
     const size_t hx = (size_t)(heads / t.hpw), share = (size_t)WT_WAVES * 32 * ((size_t)vdim + 2) * 4;
     size_t cb = std::max<size_t>({2, total * hx / WT_SLOTS, (most + WT_MAX_CHUNKS - 1) / WT_MAX_CHUNKS});
     auto chunks = [&]() { return (most + cb - 1) / cb; };
@@ -1059,6 +1297,27 @@ TilePlan tile_plan(const ifa_seq_desc *sh, int n_seqs, int heads, int kv_heads, 
     t.cb = (int)cb; t.chunks = (int)chunks(); t.groups = groups();
     t.bytes = t.op_bytes + (t.chunks > 1 ? t.tiles * hx * (size_t)t.chunks * share : 0);
     return t;
+}
+
+// (the rows of a step's sequences follow each other)
+void few_seqs(TileArgs &A, const ifa_seq_desc *sh, int n_seqs, const TilePlan &t, int window, int keep_first)
+{
+    A.n_few = 0;
+    memset(A.few, 0, sizeof(A.few));
+    if (n_seqs > FEW) return;
+    int tiles = 0, blocks = 0, row = sh[0].row0;
+    for (int q = 0; q < n_seqs; q++) {
+        if (sh[q].row0 != row || sh[q].n <= 0) return;
+        A.few[q].sd = {sh[q].row0, sh[q].n, sh[q].pos0, sh[q].slot};
+        A.few[q].tile0 = tiles; A.few[q].block0 = blocks;
+        tiles += (sh[q].n + t.qw - 1) / t.qw; blocks += seq_blocks(sh[q].pos0, sh[q].n, window, keep_first).count; row += sh[q].n;
+    }
+    int chunks = 0;
+    for (int q = n_seqs - 1; q >= 0; q--) {
+        A.few[q].chunk0 = chunks;
+        for (int at = 0; at < sh[q].n; at += t.qw) chunks += (tile_blocks(sh[q].pos0 + at, std::min(t.qw, sh[q].n - at), window, keep_first).nb + t.cb - 1) / t.cb;
+    }
+    A.n_few = n_seqs;
 }
 
 // ---- rotated queries and keys.  One workgroup per row, a wave per head at a time: RMS norm over the head's dim values with a weight
@@ -1083,11 +1342,7 @@ __global__ void __launch_bounds__(256) k_qk_rope_store(float *__restrict__ q, si
     // VX: two workgroups per row, blockIdx.y 0 for the queries and keys, 1 for the values (each forms only the angles it needs)
     const bool do_qk = !VX || blockIdx.y == 0, do_v = VX && blockIdx.y == 1;
     if (do_qk)
-    for (int i = tid; i < half; i += blockDim.x) {
-        const double a = (double)pos * freq[i];
-        double sn, cn; sincos(a, &sn, &cn);          // (one argument reduction for both)
-        cs[i] = (float)cn; cs[half + i] = (float)sn;
-    }
+    for (int i = tid; i < half; i += blockDim.x) angle_of(pos, freq, i, half, cs);
     float *vcs = cs + 2 * half;
     const int vhalf = vdim / 2;
     if (do_v && k && v_freq) {
@@ -1107,35 +1362,7 @@ __global__ void __launch_bounds__(256) k_qk_rope_store(float *__restrict__ q, si
         const float *src = is_q ? q + (size_t)t * ldq + (size_t)hd * dim : k + (size_t)t * ldk + (size_t)hd * dim;
         float *dst = is_q ? q + (size_t)t * ldq + (size_t)hd * dim : slot_base[sd.slot] + k_off + ((size_t)pos * kv_heads + hd) * dim;
         const bf16_t *nw_ = is_q ? q_norm_w : k_norm_w;
-        float r = 1.0f;
-        if (nw_) {
-            float s = 0.0f;
-            for (int c = lane; c < dim; c += 64) s = fmaf(src[c], src[c], s);
-            r = 1.0f / sqrtf(wave_sum(s) / (float)dim + eps);
-        }
-        // every lane reads both members of its pairs before anything of the head is written (q is rewritten in place); dim <= 64 RS_CPL
-        float val[RS_CPL], oth[RS_CPL];
-#pragma unroll
-        for (int e = 0; e < RS_CPL; e++) {
-            const int c = lane + 64 * e;
-            val[e] = oth[e] = 0.0f;
-            if (c < dim) {
-                val[e] = src[c] * r * (nw_ ? bf2f(nw_[c]) : 1.0f);
-                if (c < rot_dims) { const int pc = pairing ? c ^ 1 : (c < half ? c + half : c - half); oth[e] = src[pc] * r * (nw_ ? bf2f(nw_[pc]) : 1.0f); }
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < RS_CPL; e++) {
-            const int c = lane + 64 * e;
-            if (c >= dim) continue;
-            float out = val[e];
-            if (c < rot_dims) {
-                const bool first = pairing ? (c & 1) == 0 : c < half;          // first or second member of its pair
-                const int fi = pairing ? c >> 1 : (c < half ? c : c - half);
-                out = first ? val[e] * cs[fi] - oth[e] * cs[half + fi] : val[e] * cs[fi] + oth[e] * cs[half + fi];
-            }
-            dst[c] = out;
-        }
+        turn_head<RS_CPL>(src, dst, dim, nw_ != nullptr, nw_, eps, rot_dims, pairing, cs, lane);
     }
     if (VX) {
         if (!k || !do_v) return;
@@ -1211,9 +1438,11 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
                             int window, int keep_first, const void *rel_bf16, const int *bucket_of_dev, int n_buckets, const void *sink_bf16, int sink_fixed,
                             float sink_score, const void *seqs_dev, const int *row_seq_dev, size_t rows, void *const *slot_base_dev, size_t k_off, size_t v_off,
                             void *out_f32, size_t ldo, const void *seqs_host, int n_seqs, int tile_min_rows, int max_keys, void *ws_f32, size_t ws_bytes,
-                            ifa_stream stream, void *out_bf16 = nullptr, size_t ld16 = 0, bool *left16 = nullptr)
+                            ifa_stream stream, void *out_bf16 = nullptr, size_t ld16 = 0, bool *left16 = nullptr, const IfaFreshKV *fresh = nullptr, const IfaLinearSide *side = nullptr,
+                            bool *side_done = nullptr)
 {
     if (left16) *left16 = false;
+    if (side_done) *side_done = false;
     IFA_REQUIRE(!out_bf16 || (left16 && ld16 >= (size_t)heads * vdim), "%s: bad bfloat16 output", who);
     IFA_REQUIRE(q_f32 && seqs_dev && row_seq_dev && slot_base_dev && out_f32, "%s: null pointer", who);
     IFA_REQUIRE(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && dim > 0 && vdim > 0 && rows > 0 && window >= 1 && keep_first >= 0, "%s: bad shape", who);
@@ -1235,25 +1464,60 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
             const int NTK = (dim + 31) / 32, NTV = (vdim + 31) / 32;
             TileArgs A;
             A.n_seqs = n_seqs; A.hpw = t.hpw; A.cb = t.cb; A.tiles = (int)t.tiles; A.marks = t.mark_at / 4; A.shares = t.op_bytes / 4;
+            few_seqs(A, (const ifa_seq_desc *)seqs_host, n_seqs, t, window, keep_first);
             P.ws = (float *)ws_f32; P.nsplit = t.chunks;
             if (out_bf16) { P.out16 = (bf16_t *)out_bf16; P.ld16 = ld16; *left16 = true; }
             const bool vec = dim % 4 == 0 && vdim % 4 == 0 && ldq % 4 == 0 && ldo % 4 == 0 && (uintptr_t)q_f32 % 16 == 0 && (uintptr_t)out_f32 % 16 == 0
                              && (!out_bf16 || (ld16 % 4 == 0 && (uintptr_t)out_bf16 % 8 == 0));
-            const dim3 grid((unsigned)(heads / t.hpw), (unsigned)t.groups);
-#define IFA_WT(K, V) { const size_t smem_t = (size_t)2 * kBlockPieces<K, V> * 16 + WT_WAVES * 64 * 4; \
+            const int hx = heads / t.hpw;
+            FreshKV F;
+            memset(&F, 0, sizeof(F));
+            if (fresh) {
+                F.k = fresh->k; F.ldk = fresh->ldk; F.v = fresh->v; F.ldv = fresh->ldv; F.norm = fresh->norm; F.norm_w = fresh->norm_w; F.eps = fresh->eps; F.rot_dims = fresh->rot_dims;
+                F.freq = fresh->freq; F.q_rows = fresh->turn_q ? (int)rows : 0; F.q_norm_w = fresh->q_norm_w; F.q = (float *)q_f32;
+            }
+            SideArgs S;
+            memset(&S, 0, sizeof(S));
+            if (side) {
+                size_t chunks = 0;
+                const int rc = ifa_chunk_args(&S.c, &chunks, 0, side->q, side->ldq, side->k, side->ldk, side->v, side->ldv, side->heads, side->heads, side->dk, side->dv, side->decay, nullptr,
+                                              nullptr, seqs_dev, seqs_host, n_seqs, slot_base_dev, side->state_off, side->ws, side->ws_bytes, side->out, side->ldo);
+                if (rc) return rc;
+                S.chunks = (int)chunks; S.zc = (side->dv + 63) / 64; S.first = S.chunks * side->heads * S.zc; S.per = (side->dk * side->dv + 64 * WT_WAVES - 1) / (64 * WT_WAVES);
+                S.pass = S.per * side->heads * n_seqs;
+            }
+            const unsigned part_wgs = (unsigned)(S.first + 2 * kv_heads * t.blocks + ((size_t)F.q_rows + 3) / 4), tile_wgs = (unsigned)(hx * t.groups + S.pass);
+#define IFA_WT(K, V) { const size_t smem_p = (size_t)WT_K * (32 * K + 4 + F.rot_dims) * 4; \
+                       const size_t smem_t = (size_t)2 * kBlockPieces<K, V> * 16 + WT_WAVES * 64 * 4; \
                        const void *fn = vec ? (const void *)k_attn_tile<K, V, true> : (const void *)k_attn_tile<K, V, false>; \
                        IFA_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_t)); \
-                       hipLaunchKernelGGL((k_attn_parts<K, V>), dim3((unsigned)kv_heads, (unsigned)t.blocks), dim3(256), 0, ifa_s(stream), P, n_seqs, (uint32_t *)(P.ws + A.marks)); \
-                       if (vec) hipLaunchKernelGGL((k_attn_tile<K, V, true>), grid, dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A); \
-                       else hipLaunchKernelGGL((k_attn_tile<K, V, false>), grid, dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A); }
+                       if (side) hipLaunchKernelGGL((k_attn_parts<K, V, true>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, S); \
+                       else hipLaunchKernelGGL((k_attn_parts<K, V, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, 0); \
+                       if (vec) hipLaunchKernelGGL((k_attn_tile<K, V, true>), dim3(tile_wgs), dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A, hx, (int)t.groups, S); \
+                       else hipLaunchKernelGGL((k_attn_tile<K, V, false>), dim3(tile_wgs), dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A, hx, (int)t.groups, S); }
 #define IFA_WTV(K) { if (NTV == 1) IFA_WT(K, 1) else if (NTV == 2) IFA_WT(K, 2) else if (NTV == 3) IFA_WT(K, 3) else IFA_WT(K, 4) }
             if (NTK == 1) IFA_WTV(1) else if (NTK == 2) IFA_WTV(2) else if (NTK == 3) IFA_WTV(3) else IFA_WTV(4)
 #undef IFA_WTV
 #undef IFA_WT
-            if (t.chunks > 1) hipLaunchKernelGGL(k_attn_tile_combine, dim3(grid.x, (unsigned)t.tiles, (unsigned)(WT_WAVES * ((vdim + WC_COLS - 1) / WC_COLS))), dim3(256), 0, ifa_s(stream), P, A);
+            const unsigned joins = t.chunks > 1 ? (unsigned)(WT_WAVES * ((vdim + WC_COLS - 1) / WC_COLS)) : 0u;
+            if (side) {
+                const dim3 grid((unsigned)S.first + (unsigned)(hx * t.tiles) * joins);
+                const bool v16 = side->ldv % 4 == 0 && ((uintptr_t)side->v & 15) == 0;
+#define IFA_JO(D) { if (v16) hipLaunchKernelGGL((k_attn_join_out<D, true>), grid, dim3(256), 0, ifa_s(stream), P, A, S, hx); \
+                    else hipLaunchKernelGGL((k_attn_join_out<D, false>), grid, dim3(256), 0, ifa_s(stream), P, A, S, hx); }
+                if (side->dk == 64) IFA_JO(64) else IFA_JO(128)
+#undef IFA_JO
+                *side_done = true;
+            } else if (joins) hipLaunchKernelGGL(k_attn_tile_combine, dim3((unsigned)hx, (unsigned)t.tiles, joins), dim3(256), 0, ifa_s(stream), P, A);
             IFA_LAUNCH_CHECK();
             return IFA_OK;
         }
+    }
+    if (fresh) {
+        const int rc = fresh->turn_q ? ifa_qk_rope_store_f32((void *)q_f32, ldq, heads, fresh->k, fresh->ldk, fresh->v, fresh->ldv, kv_heads, dim, vdim, fresh->q_norm_w, fresh->norm_w, fresh->eps,
+                                                             fresh->rot_dims, fresh->freq, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, stream)
+                     : ifa_kv_store_f32(fresh->k, fresh->ldk, fresh->v, fresh->ldv, kv_heads, dim, fresh->norm, fresh->eps, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, stream);
+        if (rc) return rc;
     }
     // prompts without a workspace (or with one that the operands do not fit, or of more key blocks than a grid has)
     if (rows >= (size_t)tile_min_rows && n_seqs > 0 && dim <= 128 && vdim <= 128) {
@@ -1401,22 +1665,26 @@ int ifa_attention_kv_sinks_f32(const void *q_f32, size_t ldq, int heads, int kv_
 int ifa_attention_window_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int norm_q, float eps, float scale, float softcap, int window, int keep_first,
                                  const void *rel_bf16, const int *bucket_of_dev, int n_buckets, const void *sink_bf16, const void *seqs_dev, const int *row_seq_dev, size_t rows,
                                  void *const *slot_base_dev, size_t k_off, size_t v_off, void *out_f32, size_t ldo, void *out_bf16, size_t ld16, bool *left16, const void *seqs_host,
-                                 int n_seqs, int tile_min_rows, void *ws_f32, size_t ws_bytes, ifa_stream stream)
+                                 int n_seqs, int tile_min_rows, void *ws_f32, size_t ws_bytes, const IfaFreshKV &fresh, const IfaLinearSide *side, bool *side_done, ifa_stream stream)
 {
+    IFA_REQUIRE(fresh.k && fresh.v && !fresh.turn_q && !fresh.norm_w && fresh.rot_dims == 0 && fresh.ldk >= (size_t)kv_heads * dim && fresh.ldv >= (size_t)kv_heads * dim && (!side || side_done),
+                "attention_window_to_bf16: bad keys");
     const int tile_ok = dim % 32 == 0 && k_off % 4 == 0 && v_off % 4 == 0;          // (as ifa_attention_window_f32)
     return attention_launch("attention_window_to_bf16", q_f32, ldq, heads, kv_heads, dim, dim, norm_q, eps, scale, softcap, window, keep_first, rel_bf16, bucket_of_dev, n_buckets,
                             sink_bf16, 0, 0.0f, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, out_f32, ldo, seqs_host, tile_ok ? n_seqs : 0, tile_min_rows, 0, ws_f32,
-                            ws_bytes, stream, out_bf16, ld16, left16);
+                            ws_bytes, stream, out_bf16, ld16, left16, &fresh, side, side_done);
 }
 
 int ifa_attention_kv_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int vdim, float scale, int window, int keep_first, int sink, float sink_score,
                              const void *seqs_dev, const int *row_seq_dev, size_t rows, void *const *slot_base_dev, size_t k_off, size_t v_off, void *out_f32, size_t ldo,
                              void *out_bf16, size_t ld16, bool *left16, const void *seqs_host, int n_seqs, int tile_min_rows, int max_keys, void *ws_f32, size_t ws_bytes,
-                             ifa_stream stream)
+                             const IfaFreshKV &fresh, ifa_stream stream)
 {
+    IFA_REQUIRE(fresh.turn_q && (!fresh.k || (fresh.v && fresh.ldk >= (size_t)kv_heads * dim && fresh.ldv >= (size_t)kv_heads * vdim)) && fresh.norm == (fresh.norm_w != nullptr)
+                && fresh.rot_dims >= 0 && fresh.rot_dims <= dim && fresh.rot_dims % 2 == 0 && (fresh.rot_dims == 0 || fresh.freq), "attention_kv_to_bf16: bad keys");
     return attention_launch("attention_kv_to_bf16", q_f32, ldq, heads, kv_heads, dim, vdim, 0, 0.0f, scale, 0.0f, window > 0 ? window : (1 << 30), keep_first, nullptr, nullptr, 0,
                             nullptr, sink ? 1 : 0, sink_score, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, out_f32, ldo, seqs_host, n_seqs, tile_min_rows, max_keys,
-                            ws_f32, ws_bytes, stream, out_bf16, ld16, left16);
+                            ws_f32, ws_bytes, stream, out_bf16, ld16, left16, &fresh);
 }
 
 int ifa_mix_row(const IfaMixRow &M, int *nsplit, ifa_stream stream)

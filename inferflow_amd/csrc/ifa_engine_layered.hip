@@ -717,15 +717,15 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
         const Scratch ws = attn_scratch(n, D, DV);
         const LLayer &KV = own ? L : n->layers[(size_t)sp.a_kv_layer - 1];
         if ((rc = linear_in(m, L.w_in, NI, W, n->h, h16, T, L.b_in, n->proj, NI))) return rc;
-        if ((rc = ifa_qk_rope_store_f32(n->proj + L.c_aq, NI, H, own ? n->proj + L.c_ak : nullptr, NI, own ? n->proj + L.c_av : nullptr, NI, G, D, DV,
-                                        L.T(IFA_LT_A_Q_NORM).data, own ? L.T(IFA_LT_A_K_NORM).data : nullptr, c.eps, sp.a_rot_dims, L.freq, n->seqs_dev, n->row_seq_dev, T,
-                                        slots, KV.o_k, KV.o_v, s))) return rc;
+        const bf16_t *k_norm = own ? (const bf16_t *)L.T(IFA_LT_A_K_NORM).data : nullptr;
+        const IfaFreshKV fresh = {own ? n->proj + L.c_ak : nullptr, NI, own ? n->proj + L.c_av : nullptr, NI, k_norm != nullptr, k_norm, c.eps, sp.a_rot_dims, L.freq, 1,
+                                  (const bf16_t *)L.T(IFA_LT_A_Q_NORM).data};
         bf16_t *out16 = nullptr;          // the attention's output as the output product reads it
         bool left16 = false;
         if (takes_a16(n, OV, T) && OV % 64 == 0) { if ((rc = ensure_a16(m, T, OV))) return rc; out16 = n->a16; }
         if ((rc = ifa_attention_kv_to_bf16(n->proj + L.c_aq, NI, H, G, D, DV, sp.a_scale, sp.a_window, sp.a_keep_first, sp.a_sink, sp.a_sink_score, n->seqs_dev,
                                            n->row_seq_dev, T, slots, KV.o_k, KV.o_v, n->m1, OV, out16, OV, &left16, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min,
-                                           c.max_ctx, ws.p, ws.bytes, s))) return rc;
+                                           c.max_ctx, ws.p, ws.bytes, fresh, s))) return rc;
         if (left16) rc = linear_in(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, OV, nullptr, out16, T, nullptr, n->m2, W);
         else rc = linear(m, (const bf16_t *)L.T(IFA_LT_A_O).data, W, OV, n->m1, OV, T, nullptr, nullptr, 1.0f, 0, n->m2, W);
         if (rc) return rc;
@@ -1097,13 +1097,18 @@ int run_parallel_prompt(ifa_model *m, LLayer &L, size_t T, int nseq, bool *done,
     if (lin) {
         const Scratch ws = attn_scratch(n, sp.a_dim, sp.a_dim);
         bool left16 = false;
-        if ((rc = ifa_kv_store_f32(n->proj + L.c_ak, NI, n->proj + L.c_ak, NI, sp.a_kv_heads, sp.a_dim, 1, c.eps, n->seqs_dev, n->row_seq_dev, T, slots, L.o_k, L.o_v, s))) return rc;
+        // the keys stored and the chunked linear attention run in the windowed attention's launches
+        const IfaFreshKV fresh = {n->proj + L.c_ak, NI, n->proj + L.c_ak, NI, 1, nullptr, c.eps, 0, nullptr, 0, nullptr};
+        const IfaLinearSide side = {n->proj + L.c_lq, n->proj + L.c_lk, n->proj + L.c_lv, NI, NI, NI, sp.l_heads, sp.l_dim, sp.l_vdim, (const float *)L.T(IFA_LT_L_DECAY).data, L.o_lin,
+                                    n->scan_ws, n->scan_ws_bytes, n->m2, MV};
+        const bool chunked = n->scan_chunks && ifa_state_chunked_fits(0, side.q, NI, side.k, NI, side.v, NI, sp.l_dim, sp.l_vdim, n->m2, MV);
+        bool side_done = false;
         if ((rc = ifa_attention_window_to_bf16(n->proj + L.c_aq, NI, sp.a_heads, sp.a_kv_heads, sp.a_dim, 1, c.eps, sp.a_scale, sp.a_softcap, sp.a_window, sp.a_keep_first,
                                                L.T(IFA_LT_A_REL).data, L.bucket_of, sp.a_buckets, L.T(IFA_LT_A_SINK).data, n->seqs_dev, n->row_seq_dev, T, slots, L.o_k, L.o_v, n->m1, AQ,
-                                               AQ == at1 ? n->a16 : nullptr, ld, &left16, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, ws.p, ws.bytes, s))) return rc;
+                                               AQ == at1 ? n->a16 : nullptr, ld, &left16, n->seqs_host.data(), (int)n->seqs_host.size(), n->opt_attn_tile_min, ws.p, ws.bytes, fresh,
+                                               chunked ? &side : nullptr, &side_done, s))) return rc;
         if (!left16 && (rc = ifa_rows_to_bf16_part(n->m1, AQ, T, AQ, n->a16, at1, ld, s))) return rc;
-        if ((rc = run_state(m, 0, n->proj + L.c_lq, NI, n->proj + L.c_lk, NI, n->proj + L.c_lv, NI, sp.l_heads, sp.l_heads, sp.l_dim, sp.l_vdim, L.T(IFA_LT_L_DECAY).data, nullptr, nullptr,
-                            nseq, L.o_lin, n->m2, MV))) return rc;
+        if (!side_done && (rc = run_state(m, 0, side.q, NI, side.k, NI, side.v, NI, sp.l_heads, sp.l_heads, sp.l_dim, sp.l_vdim, side.decay, nullptr, nullptr, nseq, L.o_lin, n->m2, MV))) return rc;
         if ((rc = gated_norm((int)MV, L.T(IFA_LT_L_NORM).data, L.c_lg, 0))) return rc;
     } else {
         if ((rc = run_delta_mixer(m, L, T, nseq))) return rc;

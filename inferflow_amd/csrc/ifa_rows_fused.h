@@ -75,15 +75,20 @@ extern "C" bool ifa_layernorm_planes_to_bf16(int kind, void *x_f32, const float 
 // ifa_gated_groupnorm_f32 (w as long as a group or as the row)
 bool ifa_gated_groupnorm_to_bf16(const void *o_f32, size_t ldo, size_t rows, int channels, int group, const void *w_bf16, int wlen, const void *gate_f32, size_t ldg, int gate_act,
                                  float eps, void *y_bf16, size_t width, size_t ldy, ifa_stream stream);
-// ifa_attention_window_f32 / ifa_attention_kv_f32: *left16 tells whether the output is in out_bf16 (rows of ld16, heads * vdim columns) or, where the step's form writes 32 bits, in out_f32
-int ifa_attention_window_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int norm_q, float eps, float scale, float softcap, int window, int keep_first,
+// What a step brings to an attention's cache: keys and values as projected (k null: the layer reads rows that are there already).  norm: the keys by their root mean square (with norm_w or
+// without); rot_dims of them turned by pos * freq; turn_q: the queries (in place) like them, with q_norm_w.  As ifa_kv_store_f32 / ifa_qk_rope_store_f32, which these launches stand for
+struct IfaFreshKV { const float *k; size_t ldk; const float *v; size_t ldv; int norm; const ifa32::bf16_t *norm_w; float eps; int rot_dims; const double *freq; int turn_q; const ifa32::bf16_t *q_norm_w; };
+// The decayed linear attention of the same rows and slots (ifa_state_chunked_f32 of kind 0, its sizes): in the windowed attention's launches where *side_done says so
+struct IfaLinearSide { const float *q, *k, *v; size_t ldq, ldk, ldv; int heads, dk, dv; const float *decay; size_t state_off; void *ws; size_t ws_bytes; float *out; size_t ldo; };
+// ifa_kv_store_f32 / ifa_qk_rope_store_f32, then ifa_attention_window_f32 / ifa_attention_kv_f32: *left16 tells whether the output is in out_bf16 (rows of ld16, heads * vdim columns) or, where the step's form writes 32 bits, in out_f32
+extern "C" int ifa_attention_window_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int norm_q, float eps, float scale, float softcap, int window, int keep_first,
                                  const void *rel_bf16, const int *bucket_of_dev, int n_buckets, const void *sink_bf16, const void *seqs_dev, const int *row_seq_dev, size_t rows,
                                  void *const *slot_base_dev, size_t k_off, size_t v_off, void *out_f32, size_t ldo, void *out_bf16, size_t ld16, bool *left16, const void *seqs_host,
-                                 int n_seqs, int tile_min_rows, void *ws_f32, size_t ws_bytes, ifa_stream stream);
-int ifa_attention_kv_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int vdim, float scale, int window, int keep_first, int sink, float sink_score,
+                                 int n_seqs, int tile_min_rows, void *ws_f32, size_t ws_bytes, const IfaFreshKV &fresh, const IfaLinearSide *side, bool *side_done, ifa_stream stream);
+extern "C" int ifa_attention_kv_to_bf16(const void *q_f32, size_t ldq, int heads, int kv_heads, int dim, int vdim, float scale, int window, int keep_first, int sink, float sink_score,
                              const void *seqs_dev, const int *row_seq_dev, size_t rows, void *const *slot_base_dev, size_t k_off, size_t v_off, void *out_f32, size_t ldo,
                              void *out_bf16, size_t ld16, bool *left16, const void *seqs_host, int n_seqs, int tile_min_rows, int max_keys, void *ws_f32, size_t ws_bytes,
-                             ifa_stream stream);
+                             const IfaFreshKV &fresh, ifa_stream stream);
 // ifa_moe_experts_gated_f32 of more than eight rows that a norm has left in bfloat16 (rows of `width`), where the first tells that the experts' products read them so
 bool ifa_moe_gated_reads_bf16(size_t rows, int width, int ff, int top, int ops32, const void *gate_up_bf16, const void *down_bf16);
 int ifa_moe_experts_gated_bf16(const void *h_bf16, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16, const void *down_bf16, const int *idx_dev,
