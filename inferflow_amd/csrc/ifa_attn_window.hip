@@ -1160,7 +1160,7 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
                 if constexpr (VEC) { if (c < dv) *reinterpret_cast<bf16x4w *>(d16 + c) = v; }
                 else {
 #pragma unroll
-                    for (int x = 0; x < 4; x++) if (c + x < dv) d16[c + x] = __builtin_bit_cast(bf16_t, v[x]);
+                    for (int x = 0; x < 4; x++) if (c + x < dv) { const __bf16 one = v[x]; d16[c + x] = __builtin_bit_cast(bf16_t, one); }          // (the builtin of a vector element takes the first one)
                 }
             }
         return;

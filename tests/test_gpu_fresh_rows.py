@@ -50,7 +50,7 @@ ONE, PART, MANY = [[(70, 0, 0)], [(45, 70, 0)]], [[(33, 0, 1), (17, 0, 0), (40, 
 # behind kept tokens, up to four sequences and more, portions that begin inside a block, long enough for several chunks; the last: fewer rows than the tiled form takes
 @pytest.mark.parametrize("H,G,D,DV,rot,window,keep,steps,tile_min", [
     (8, 2, 128, 128, 64, 0, 0, ONE, 16), (4, 1, 128, 64, 128, 0, 0, PART, 16), (12, 3, 64, 96, 32, 40, 5, PART, 16), (6, 3, 96, 32, 0, 33, 70, ONE, 16), (5, 5, 40, 48, 10, 0, 0, PART, 16),
-    (20, 5, 32, 128, 32, 0, 0, MANY, 16), (2, 2, 128, 128, 126, 100, 40, [[(650, 0, 0)]], 16), (8, 2, 72, 100, 64, 0, 0, [[(9, 0, 0)], [(6, 9, 0)]], 16)])
+    (20, 5, 32, 128, 32, 0, 0, MANY, 16), (2, 2, 128, 128, 126, 100, 40, [[(650, 0, 0)]], 16), (8, 2, 72, 100, 64, 0, 0, [[(9, 0, 0)], [(6, 9, 0)]], 16), (3, 1, 30, 33, 30, 0, 0, PART, 16)])
 @pytest.mark.parametrize("own", [True, False])
 def test_rows_of_rotated_attention_stored_on_the_way(H, G, D, DV, rot, window, keep, steps, tile_min, own):
     rng = np.random.default_rng(H * D + rot)
