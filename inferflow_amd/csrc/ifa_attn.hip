@@ -388,6 +388,140 @@ __global__ void __launch_bounds__(256) k_attention_mfma(const half_t *__restrict
     }
 }
 
+// ---------------------------------------------------------------- short prompts from position 0 (4 .. 63 tokens, F16 cache, heads of 128 turned whole)
+// What k_rope_qk_store and k_attention_mfma do for such a step in one launch, a workgroup per (32-query tile, head): its queries, keys and values are in the step's own q / k / v rows, asked for
+// at once; the tile's own keys, turned, and values go into the cache on their way.  The cosines and sines come from a table of the step (tab [token][64] pairs, formed where the embedding rows
+// are gathered): the angles of every key again in every head's workgroup would be 8 us.  The same expressions in the same order, the same bits.
+// Bound by its launch and one chain (rows, LDS, scores, softmax, LDS, products): 37 tokens of 32 heads 4.8 + 10.9 -> 4.8 us a layer (a whole prompt of 37 2503 -> 2198).
+constexpr int FR_MAX = 64, FR_ROW = 128 + 8, FR_S = FR_MAX + 8;          // keys; halfs per row of queries / keys and of scores
+template <int ORDER>
+__global__ void __launch_bounds__(256) k_attention_fresh(const half_t *__restrict__ q, const half_t *__restrict__ k, const half_t *__restrict__ v, const float *__restrict__ tab, int T, int heads,
+                                                         int kv_heads, float kq_scale, half_t *__restrict__ kcache, half_t *__restrict__ vcache, size_t cache_row, half_t *__restrict__ out)
+{
+    constexpr int HD = 128, KS = HD / 16;
+    __shared__ __attribute__((aligned(16))) half_t Qs[32 * FR_ROW], Ks[FR_MAX * FR_ROW], S[32 * FR_S], Vt[2][HD * PF_VROW];
+    const int tile = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 31, g = lane >> 5, group = heads / kv_heads, kvh = h / group;
+    const int t0 = 32 * tile, nkb = tile + 1;
+    const bool stores = h % group == 0;          // (one head of those that share the keys)
+    const size_t q_row = (size_t)heads * HD, kv_row = (size_t)kv_heads * HD;
+    // a row's head in pieces of eight pairs: halfs a0 .. a0 + 7 and b0 .. b0 + 7
+    const int row = tid >> 3, c0 = 8 * (tid & 7), a0 = ORDER == 2 ? c0 : 2 * c0, b0 = ORDER == 2 ? c0 + HD / 2 : 2 * c0 + 8;
+    const int tq = min(t0 + row, T - 1);
+    auto pair_at = [&](const half_t *p, half8v (&x)[2]) { x[0] = *reinterpret_cast<const half8v *>(p + a0); x[1] = *reinterpret_cast<const half8v *>(p + b0); };
+    auto angles_at = [&](int t, float4 (&cs)[4]) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) cs[e] = *reinterpret_cast<const float4 *>(tab + ((size_t)t * (HD / 2) + c0) * 2 + 4 * e);
+    };
+    half8v qv[2], kv[2][2], va[2][2];
+    float4 cs[2][4];
+    pair_at(q + (size_t)tq * q_row + (size_t)h * HD, qv);
+    const int vpar = tid & 1, vpair = (tid >> 1) & 7, vch = ((tid >> 4) & 3) + 4 * wave, vkey0 = 2 * vpair;          // (as in k_attention_mfma)
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+        if (kb < nkb) {
+            const int t = min(32 * kb + row, T - 1);
+            pair_at(k + (size_t)t * kv_row + (size_t)kvh * HD, kv[kb]);
+            angles_at(t, cs[kb]);
+#pragma unroll
+            for (int it = 0; it < 2; it++) va[kb][it] = *reinterpret_cast<const half8v *>(v + (size_t)min(32 * kb + vkey0 + vpar + 16 * it, T - 1) * kv_row + (size_t)kvh * HD + 8 * vch);
+        }
+    auto turned = [&](const half8v (&x)[2], const float4 (&a)[4], half8v (&y)[2]) {          // rope_rotate's expressions (ifa_math.h)
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float x0 = ORDER == 2 ? h2f(x[0][e]) : h2f(e < 4 ? x[0][2 * e & 7] : x[1][(2 * e - 8) & 7]);
+            const float x1 = ORDER == 2 ? h2f(x[1][e]) : h2f(e < 4 ? x[0][(2 * e + 1) & 7] : x[1][(2 * e - 7) & 7]);
+            const float c = e & 1 ? a[e >> 1].z : a[e >> 1].x, sn = e & 1 ? a[e >> 1].w : a[e >> 1].y;
+            const float p0 = x0 * c, p1 = x1 * sn, p2 = x0 * sn, p3 = x1 * c;
+            const half_t r0 = f2h(p0 - p1), r1 = f2h(p2 + p3);
+            if (ORDER == 2) { y[0][e] = r0; y[1][e] = r1; }
+            else if (e < 4) { y[0][(2 * e) & 7] = r0; y[0][(2 * e + 1) & 7] = r1; }
+            else { y[1][(2 * e - 8) & 7] = r0; y[1][(2 * e - 7) & 7] = r1; }
+        }
+    };
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+        if (kb < nkb) {
+            half8v y[2];
+            turned(kv[kb], cs[kb], y);
+            half_t *dst = Ks + (size_t)(32 * kb + row) * FR_ROW;
+            *reinterpret_cast<half8v *>(dst + a0) = y[0]; *reinterpret_cast<half8v *>(dst + b0) = y[1];
+            if (kb == tile) {
+                half8v z[2];
+                turned(qv, cs[kb], z);
+                half_t *qd = Qs + (size_t)row * FR_ROW;
+                *reinterpret_cast<half8v *>(qd + a0) = z[0]; *reinterpret_cast<half8v *>(qd + b0) = z[1];
+                if (stores && t0 + row < T) {
+                    half_t *kd = kcache + (size_t)(t0 + row) * cache_row + (size_t)kvh * HD;
+                    *reinterpret_cast<half8v *>(kd + a0) = y[0]; *reinterpret_cast<half8v *>(kd + b0) = y[1];
+                }
+            }
+            // values: [dim][key], two keys a dword (as in k_attention_mfma)
+#pragma unroll
+            for (int it = 0; it < 2; it++) {
+                const int key = 32 * kb + vkey0 + vpar + 16 * it;
+                if (kb == tile && stores && key < T) *reinterpret_cast<half8v *>(vcache + (size_t)key * cache_row + (size_t)kvh * HD + 8 * vch) = va[kb][it];
+                const u32x4v w = __builtin_bit_cast(u32x4v, va[kb][it]);
+                const uint32_t m0 = vpar ? w[2] : w[0], m1 = vpar ? w[3] : w[1];
+                const uint32_t r0 = __shfl_xor(vpar ? w[0] : w[2], 1), r1 = __shfl_xor(vpar ? w[1] : w[3], 1);
+                const uint32_t e0 = vpar ? r0 : m0, e1 = vpar ? r1 : m1, o0 = vpar ? m0 : r0, o1 = vpar ? m1 : r1;
+                uint32_t *d = reinterpret_cast<uint32_t *>(Vt[kb] + (size_t)(8 * vch + 4 * vpar) * PF_VROW + vkey0 + 16 * it);
+                d[0 * PF_VROW / 2] = (e0 & 0xFFFFu) | (o0 << 16);
+                d[1 * PF_VROW / 2] = (e0 >> 16) | (o0 & 0xFFFF0000u);
+                d[2 * PF_VROW / 2] = (e1 & 0xFFFFu) | (o1 << 16);
+                d[3 * PF_VROW / 2] = (e1 >> 16) | (o1 & 0xFFFF0000u);
+            }
+        }
+    __syncthreads();
+    if (wave < nkb) {
+        const float alpha = 1.0f / sqrtf((float)HD) / kq_scale;
+        f32x16v acc;
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+#pragma unroll
+        for (int s2 = 0; s2 < KS; s2++)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8v *>(Qs + (size_t)i * FR_ROW + 16 * s2 + 8 * g),
+                                                         *reinterpret_cast<const half8v *>(Ks + (size_t)(32 * wave + i) * FR_ROW + 16 * s2 + 8 * g), acc, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; r++) S[(size_t)((r & 3) + 8 * (r >> 2) + 4 * g) * FR_S + 32 * wave + i] = f2h(alpha * acc[r]);
+    }
+    __syncthreads();
+    {   // softmax, a row eight lanes (wave_max and wave_sum over these)
+        const int r = 8 * wave + (lane >> 3), c = lane & 7, nch = 4 * nkb, nv = t0 + r < T && c < nch ? t0 + r + 1 : 0;
+        half8v p = *reinterpret_cast<const half8v *>(S + (size_t)r * FR_S + 8 * min(c, nch - 1));
+        float most = -INFINITY, sum = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) if (8 * c + e < nv) most = fmaxf(most, kq_scale * h2f(p[e]));
+        most = fmaxf(most, dpp_xor1(most)); most = fmaxf(most, dpp_xor2(most)); most = fmaxf(most, dpp_half_mirror(most));
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float ev = 8 * c + e < nv ? __expf(kq_scale * h2f(p[e]) - most) : 0.0f;
+            sum += ev;
+            p[e] = f2h(ev);
+        }
+        sum += dpp_xor1(sum); sum += dpp_xor2(sum); sum += dpp_half_mirror(sum);
+        const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+        if (8 * c < nv) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) p[e] = f2h(h2f(p[e]) * inv);
+        }
+        if (c < nch) *reinterpret_cast<half8v *>(S + (size_t)r * FR_S + 8 * c) = p;
+    }
+    __syncthreads();
+    f32x16v o;
+#pragma unroll
+    for (int r = 0; r < 16; r++) o[r] = 0.0f;
+    for (int kb = 0; kb < nkb; kb++)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; s2++)
+            o = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8v *>(S + (size_t)i * FR_S + 32 * kb + 16 * s2 + 8 * g),
+                                                       *reinterpret_cast<const half8v *>(Vt[kb] + (size_t)(32 * wave + i) * PF_VROW + 16 * s2 + 8 * g), o, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const int t = t0 + (r & 3) + 8 * (r >> 2) + 4 * g;
+        if (t < T) out[((size_t)t * heads + h) * HD + 32 * wave + i] = f2h(o[r]);
+    }
+}
+
 // ---------------------------------------------------------------- long prompts (q_tokens >= 128): two passes over the keys
 // One workgroup per (128-query tile, head), a wave per 32 queries.  The three-stage kernel above keeps a [32 x n_keys]
 // score tile (LDS, past ~2300 keys a global workspace) and re-reads a head's K / V once per 32 queries: at 4096 tokens it
@@ -956,6 +1090,12 @@ static int g_attn_2pass_min_keys = 1 << 30;      // contexts of at least this ma
                                                  // 128 / 256 / 512 / 1024 / 2048 / 4096 tokens: 64-query 11.9 / 16.9 / 27.4 / 60.2 / 165 / 492 us, staged kernel 15.6 / 18.9 / 32.7 / 77 / 334 / 1202,
                                                  // 128-query variant - / - / - / 75 / 175 / 519 -- Llama-2-7B heads, profiles/r02_attention_two_pass.log)
 
+// prompts that k_attention_fresh takes: those that k_attention_mfma would, with two blocks of keys at the most (fewer than four rows: a workgroup a row; 64 and more: the two-pass kernel)
+extern "C" bool attention_fresh_fits(int tokens, int head_dim, int rope_order, float partial_rotary_factor)
+{
+    return tokens >= 4 && tokens < g_attn_2pass_min && tokens <= FR_MAX && head_dim == 128 && (rope_order == 1 || rope_order == 2) && (partial_rotary_factor <= 0 || partial_rotary_factor == 1.0f);
+}
+
 extern "C" int ifa_attention_two_pass_min(int min_tokens)
 {
     const int prev = g_attn_2pass_min;
@@ -973,6 +1113,24 @@ extern "C" int ifa_attention_two_pass_min_keys(int min_keys)
 extern "C" int ifa_debug_attn_trace(unsigned long long *out8)
 {
     IFA_HIP_CHECK(hipMemcpyFromSymbol(out8, HIP_SYMBOL(ifa::g_attn_trace), 64));
+    return IFA_OK;
+}
+
+// engine-internal: ifa_rope_qk_store and ifa_attention of a prompt from position 0 in one launch (k_attention_fresh); tab: (cos, sin) of [token][head_dim / 2]; IFA_ERR_STATE where the two take
+// other kernels or the shape isn't covered (nothing launched)
+extern "C" int ifa_attention_fresh(const void *q, const void *k, const void *v, const float *tab, int tokens, int heads, int kv_heads, int head_dim, float kq_scale, int rope_order,
+                                   float partial_rotary_factor, void *kcache, void *vcache, size_t cache_row_elems, void *out, ifa_stream stream)
+{
+    IFA_REQUIRE(q && k && v && tab && kcache && vcache && out, "ifa_attention_fresh: null pointer");
+    IFA_REQUIRE(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && kq_scale > 0, "ifa_attention_fresh: heads %d kv_heads %d", heads, kv_heads);
+    if (!attention_fresh_fits(tokens, head_dim, rope_order, partial_rotary_factor) || cache_row_elems % 8
+        || (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)tab | (uintptr_t)kcache | (uintptr_t)vcache) & 15)) return IFA_ERR_STATE;
+    const dim3 grid((unsigned)((tokens + 31) / 32), (unsigned)heads);
+#define IFA_FRESH(O) k_attention_fresh<O><<<grid, dim3(256), 0, ifa_s(stream)>>>((const half_t *)q, (const half_t *)k, (const half_t *)v, tab, tokens, heads, kv_heads, kq_scale, (half_t *)kcache, \
+                                                                                 (half_t *)vcache, cache_row_elems, (half_t *)out)
+    if (rope_order == 2) IFA_FRESH(2); else IFA_FRESH(1);
+#undef IFA_FRESH
+    IFA_LAUNCH_CHECK();
     return IFA_OK;
 }
 

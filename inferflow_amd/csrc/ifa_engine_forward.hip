@@ -5,9 +5,17 @@
 namespace ifae {
 
 __global__ void __launch_bounds__(256) k_gather_rows(const half_t *__restrict__ embd, const int *__restrict__ tokens,
-                                                     int T, int dim, int vocab, half_t *__restrict__ x, float embd_scale)
+                                                     int T, int dim, int vocab, half_t *__restrict__ x, float embd_scale, float *__restrict__ rope_tab = nullptr,
+                                                     int head_dim = 0, int pos0 = 0, float theta = 0.0f)
 {
     const int t = blockIdx.y;
+    // (cos, sin) of the row's pairs (heads turned whole), for the launches that turn its queries and keys
+    if (rope_tab && blockIdx.x == 0)
+        for (int c = threadIdx.x; c < head_dim / 2; c += blockDim.x) {
+            float co, si;
+            rope_angle(c, pos0 + t, theta, head_dim, co, si);
+            rope_tab[(size_t)t * head_dim + 2 * c] = co; rope_tab[(size_t)t * head_dim + 2 * c + 1] = si;
+        }
     int tok = tokens[t];
     tok = min(max(tok, 0), vocab - 1);
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < dim; c += gridDim.x * blockDim.x) {
@@ -259,6 +267,9 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
     ifa_stream s = m->stream;
     const size_t D = c.dim, QD = (size_t)c.heads * c.head_dim, KVD = (size_t)c.kv_heads * c.head_dim;
     const ifa_tp_topology *tp = m->topo;            // multi-GPU partition (ifa_model_tp_prefill): merges + stage hand-over
+    // prompts of a few rows on the fused routes: rotation, cache rows and attention of a layer in one launch (the rows' angles come with the embedding rows)
+    const bool fresh = !tp && m->opt_attn_fresh && !m->opt_perf_stat && prefix_len == 0 && c.kv_dtype != Q8_B32T2 && !c.use_alibi
+                       && attention_fresh_fits(T, c.head_dim, c.rope_order, c.partial_rotary);
     const bool first_stage = !tp || tp->stage == 0, last_stage = !tp || tp->next_rank < 0 || tp->n_stages == 1;
     const bool merging = tp_merging(m);
     if (first_stage && (!m->g[T_EMBD].present() || m->g[T_EMBD].dtype != F16)) return ifa_fail(IFA_ERR_STATE, "F16 embeddings not set");
@@ -268,7 +279,7 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
         PerfSpan sp_embd(m, 1);          // (key 1: the embedding rows, InferenceEngine::Infer_Std, inference_engine.cc:1168-1176)
         IFA_HIP_CHECK(hipMemcpyAsync(m->tokens_dev, tokens_host, sizeof(int) * (size_t)T, hipMemcpyHostToDevice, m->stream));
         k_gather_rows<<<dim3(4, (unsigned)T), dim3(256), 0, m->stream>>>((const half_t *)m->g[T_EMBD].data, m->tokens_dev, T, (int)D,
-                                                                          (int)m->g[T_EMBD].rows, m->x, c.embd_scale);
+                                                                          (int)m->g[T_EMBD].rows, m->x, c.embd_scale, fresh ? m->prope : nullptr, c.head_dim, prefix_len, c.rope_theta);
         IFA_LAUNCH_CHECK();
     } else if ((rc = ifa_recv(tp->world, m->x, (size_t)T * D * 2, tp->prev_rank, s))) return rc;     // the previous group's [T][dim] output
     half_t *x = m->x;
@@ -327,8 +338,13 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
         uint8_t *kdst = (uint8_t *)L.kcache + (size_t)prefix_len * m->kv_row_bytes;
         uint8_t *vdst = (uint8_t *)L.vcache + (size_t)prefix_len * m->kv_row_bytes;
         const bool kv_f16 = c.kv_dtype != Q8_B32T2;
-        bool kv_stored = false;
-        if (c.rope_order != 0) {
+        bool kv_stored = false, attended = false;
+        if (fresh) {
+            rc = ifa_attention_fresh(m->q, m->k, m->v, m->prope, T, c.heads, c.kv_heads, c.head_dim, c.kq_scale, c.rope_order, c.partial_rotary, kdst, vdst, m->kv_row_bytes / 2, m->att, s);
+            if (rc == IFA_OK) kv_stored = attended = true;
+            else if (rc != IFA_ERR_STATE) return rc;
+        }
+        if (!attended && c.rope_order != 0) {
             rc = ifa_rope_qk_store(m->q, m->k, m->v, c.head_dim, c.heads, c.kv_heads, T, prefix_len, c.rope_theta, c.rope_order, c.partial_rotary,
                                    kv_f16 ? kdst : nullptr, kv_f16 ? vdst : nullptr, m->kv_row_bytes / 2, s);
             if (rc == IFA_OK) kv_stored = kv_f16;
@@ -345,7 +361,7 @@ int forward_ops(ifa_model *m, const int *tokens_host, int T, int prefix_len, voi
             IFA_HIP_CHECK(hipMemcpyAsync(kdst, m->k, (size_t)T * m->kv_row_bytes, hipMemcpyDeviceToDevice, m->stream));
             IFA_HIP_CHECK(hipMemcpyAsync(vdst, m->v, (size_t)T * m->kv_row_bytes, hipMemcpyDeviceToDevice, m->stream));
         }
-        if ((rc = ifa_attention(m->q, L.kcache, L.vcache, c.kv_dtype, prefix_len + T, T, prefix_len, c.heads, c.kv_heads,
+        if (!attended && (rc = ifa_attention(m->q, L.kcache, L.vcache, c.kv_dtype, prefix_len + T, T, prefix_len, c.heads, c.kv_heads,
                                 c.head_dim, c.use_alibi ? 1.0f : c.kq_scale, c.use_alibi, c.tp_rank * c.heads,
                                 c.heads * std::max(1, c.tp_size), m->att, s))) return rc;
         if (pf_few) {

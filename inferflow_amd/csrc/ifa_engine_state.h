@@ -102,6 +102,7 @@ struct ifa_model {
     half_t *dqkv = nullptr;     // the decode step's q | k | v vector as ONE buffer (k_dec_attn addresses k and v from q's pointer)
     half_t *bqkv = nullptr;     // fused batched step: [queries][q | k | v]
     float *brope = nullptr;     // fused batched step: [queries][head_dim] (cos, sin) pairs
+    float *prope = nullptr;     // prompts of few rows: [row][head_dim] (cos, sin) pairs (ifa_attention_fresh)
     size_t bqkv_rows = 0;
     half_t *att = nullptr, *a = nullptr, *f = nullptr, *t1 = nullptr, *t2 = nullptr, *logits = nullptr;
     uint8_t *xq = nullptr;
@@ -221,6 +222,7 @@ struct ifa_model {
     // prompts of FEW_MIN .. few_max_rows tokens and steps of as many queries through gemm_few (ifa_gemm_few.hip); its workspace, one allocation: rows in fragment order (a layer's
     // input, the gated pair's output), sums of the parts of K
     int opt_rows_few = 1;
+    int opt_attn_fresh = 1;
     struct { half_t *x, *ff; float *sums; } few = {nullptr, nullptr, nullptr};
     int opt_rows_kparts = 1, opt_gemm_splitk = 1;   // 0: never the launches whose workgroups wait for partner workgroups (K parts of the 9..32-row GEMM, split-K halves of the large-tile GEMM)
     int opt_debug_mo_alloc_fail = 0;           // tests: ensure_mo_build fails like an exhausted allocator after its first copy (2: of copies with MO_WORDS only; 3: not there, but gemm_few's workspace)
@@ -262,6 +264,10 @@ extern "C" int ifa_add_layernorm(int kind, const void *a, const void *addend, si
 extern "C" int ifa_rope_qk_store(void *q, void *k, const void *v, int head_dim, int heads, int kv_heads, int tokens, int pos0, float theta,
                                  int order, float partial_rotary_factor, void *kcache_rows, void *vcache_rows, size_t cache_row_elems,
                                  ifa_stream stream);
+
+extern "C" bool attention_fresh_fits(int tokens, int head_dim, int rope_order, float partial_rotary_factor);
+extern "C" int ifa_attention_fresh(const void *q, const void *k, const void *v, const float *tab, int tokens, int heads, int kv_heads, int head_dim, float kq_scale, int rope_order,
+                                   float partial_rotary_factor, void *kcache, void *vcache, size_t cache_row_elems, void *out, ifa_stream stream);
 
 extern "C" int ifa_activation_mul(int kind, const void *a, const void *b, size_t n, void *c, ifa_stream stream);
 

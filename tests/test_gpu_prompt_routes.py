@@ -283,3 +283,20 @@ def test_batched_steps_of_many_queries_agree_with_the_rows_products_and_replay(k
         assert [int(t) for t in wk.decode_batch(new, pos, slots)] == [int(t) for t in tok]
         wk.decode_batch(new[:4], pos[:4], slots[:4]); torch.cuda.synchronize()
     wk.close()
+
+
+@pytest.mark.parametrize("T", [4, 8, 9, 31, 32, 33, 62, 63])
+@pytest.mark.parametrize("order,shape", [(2, {}), (1, dict(kv_heads=8)), (2, dict(dim=1024, heads=8, kv_heads=2, head_dim=128, ffn=1408))], ids=["7b", "pairs_kv8", "w1024_kv2"])
+def test_rotation_and_attention_of_short_prompts_in_one_launch_leave_the_bits_of_two(order, shape, T):
+    """one tile of queries and two, whole and ragged; heads that share keys; both ways of pairing: every row's logits and the last layer's cache rows"""
+    wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=96, layers=2, vocab=600, rope_order=order, **shape)
+    toks = np.random.default_rng(T).integers(3, 600, T).astype(np.int32)
+    out = []
+    for on in (1, 0):
+        wk.set_option("attn_fresh", on)
+        tok, lg = _rows(wk, toks, 600)
+        out.append((tok, lg) + tuple(np.array(wk.read_buffer(n, 1, nbytes=96 * s["kv_heads"] * s["head_dim"] * 2)) for n in ("kcache", "vcache")))
+    wk.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    assert out[0][2].any() and np.isfinite(out[0][1]).all()
