@@ -100,6 +100,7 @@ struct LayeredNet {
     int *tab_pin = nullptr, *tab_dev = nullptr; size_t tab_rows = 0, tab_seqs = 0;
     int *tokens_dev = nullptr, *pos_dev = nullptr, *row_seq_dev = nullptr; ifa_seq_desc *seqs_dev = nullptr;
     int *excl_dev = nullptr, *next_dev = nullptr, *ring_dev = nullptr;
+    void *argmax_ws = nullptr;
     // activations (fp32), sized for scratch_rows
     size_t scratch_rows = 0, n_in_max = 0, mix_max = 0, ffn_max = 0, heads_max = 0;
     float *x = nullptr, *h = nullptr, *proj = nullptr, *m1 = nullptr, *m2 = nullptr, *m3 = nullptr, *beta = nullptr, *decay = nullptr, *logits = nullptr;
@@ -1305,11 +1306,6 @@ int run_head(ifa_model *m, size_t r0, size_t nr)
     return IFA_OK;
 }
 
-__global__ void k_lay_advance(int *tokens, int *pos, ifa_seq_desc *seqs, const int *next, int *ring, int step)
-{
-    tokens[0] = next[0]; pos[0] += 1; seqs[0].pos0 += 1; ring[step] = next[0];
-}
-
 // ---- the worker class
 int lay_destroy(ifa_model *m)
 {
@@ -1329,7 +1325,7 @@ int lay_destroy(ifa_model *m)
     lay_free(n->slot_base_dev);
     if (n->tab_pin) (void)hipHostFree(n->tab_pin);
     lay_free(n->attn_ws); lay_free(n->tile_ws); lay_free(n->scan_ws); lay_free(n->a16); lay_free(n->h16); lay_free(n->g16); lay_free(n->planes);
-    lay_free(n->tab_dev); lay_free(n->excl_dev); lay_free(n->next_dev); lay_free(n->ring_dev);
+    lay_free(n->tab_dev); lay_free(n->excl_dev); lay_free(n->next_dev); lay_free(n->ring_dev); lay_free(n->argmax_ws);
     float *bufs[] = {n->x, n->h, n->proj, n->m1, n->m2, n->m3, n->beta, n->decay, n->logits, n->taps};
     for (float *b : bufs) lay_free(b);
     if (m->stream && m->own_stream) (void)hipStreamDestroy(m->stream);
@@ -1637,6 +1633,7 @@ int lay_finalize(ifa_model *m)
         IFA_HIP_CHECK(hipMemset(n->excl_dev, 0, 4 * sizeof(int)));
         IFA_HIP_CHECK(hipMalloc((void **)&n->next_dev, sizeof(int) * ifa_model::RING));
         IFA_HIP_CHECK(hipMalloc((void **)&n->ring_dev, sizeof(int) * ifa_model::RING));
+        IFA_HIP_CHECK(hipMalloc(&n->argmax_ws, ifa_argmax_parts_bytes()));
     }
     {   // (no matter if there is no room: a step asks again)
         constexpr size_t RESERVE_BYTES = (size_t)256 << 20;
@@ -1832,9 +1829,9 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
     ifa_stream s = (ifa_stream)m->stream;
     if (all) {
         if ((rc = run_head(m, 0, T))) return rc;
-        if (T == (size_t)nseq) { if ((rc = ifa_argmax_rows_f32(n->logits, V, V, T, n->excl_dev, n->next_dev, s))) return rc; }          // (a token each)
+        if (T == (size_t)nseq) { if ((rc = ifa_argmax_parts_f32(n->logits, V, V, T, n->excl_dev, n->next_dev, n->argmax_ws, nullptr, s))) return rc; }          // (a token each)
         else for (int q = 0; q < nseq; q++)
-            if ((rc = ifa_argmax_rows_f32(n->logits + (size_t)last[(size_t)q] * V, V, V, 1, n->excl_dev, n->next_dev + q, s))) return rc;
+            if ((rc = ifa_argmax_parts_f32(n->logits + (size_t)last[(size_t)q] * V, V, V, 1, n->excl_dev, n->next_dev + q, n->argmax_ws, nullptr, s))) return rc;
     } else {
         // the sequences' last rows, normed one by one into consecutive rows of h, then one product
         for (int q = 0; q < nseq; q++)
@@ -1842,7 +1839,7 @@ int lay_step(ifa_model *m, int nseq, const int *tokens_host, const int *lens, co
         if ((rc = linear(m, (const bf16_t *)n->lm_head.data, V, W, n->h, W, (size_t)nseq, nullptr, nullptr, logit_scale_of(n), 0, n->logits, V))) return rc;
         if (n->cfg.logit_softcap > 0.0f && (rc = ifa_softcap_f32(n->logits, (size_t)nseq * V, n->cfg.logit_softcap, s))) return rc;
         n->logits_rows = (size_t)nseq;
-        if ((rc = ifa_argmax_rows_f32(n->logits, V, V, (size_t)nseq, n->excl_dev, n->next_dev, s))) return rc;
+        if ((rc = ifa_argmax_parts_f32(n->logits, V, V, (size_t)nseq, n->excl_dev, n->next_dev, n->argmax_ws, nullptr, s))) return rc;
     }
     std::vector<int> next((size_t)nseq, -1);
     IFA_HIP_CHECK(hipMemcpyAsync(next.data(), n->next_dev, (size_t)nseq * 4, hipMemcpyDeviceToHost, m->stream));
@@ -1875,14 +1872,15 @@ int lay_decode_batch(ifa_model *m, int cnt, const int *tokens_host, const int *p
     return IFA_OK;
 }
 
-// one token of the current slot's sequence, everything it depends on in device memory: capturable
+// one token of the current slot's sequence, everything it depends on in device memory, and on to the next one: capturable
 int enqueue_decode_step(ifa_model *m)
 {
     LayeredNet *n = m->lay;
     const size_t V = (size_t)n->cfg.vocab;
     int rc;
     if ((rc = run_layers(m, 1, 1)) || (rc = run_head(m, 0, 1))) return rc;
-    return ifa_argmax_rows_f32(n->logits, V, V, 1, n->excl_dev, n->next_dev, (ifa_stream)m->stream);
+    const IfaStepAdvance next = {n->tokens_dev, n->pos_dev, n->seqs_dev, n->ring_dev, ifa_model::RING};
+    return ifa_argmax_parts_f32(n->logits, V, V, 1, n->excl_dev, n->next_dev, n->argmax_ws, &next, (ifa_stream)m->stream);
 }
 
 int lay_decode(ifa_model *m, int first_token, int start_pos, int n_steps, int *out_tokens_host, float *elapsed_ms, bool prepare_only)
@@ -1920,11 +1918,12 @@ int lay_decode(ifa_model *m, int first_token, int start_pos, int n_steps, int *o
     for (int st = 0; st < n_steps; st++) {
         if (n->step_exec && n->opt_graph && !n->opt_tap_layers) IFA_HIP_CHECK(hipGraphLaunch(n->step_exec, m->stream));
         else if ((rc = enqueue_decode_step(m))) return rc;
-        hipLaunchKernelGGL(k_lay_advance, dim3(1), dim3(1), 0, m->stream, n->tokens_dev, n->pos_dev, n->seqs_dev, n->next_dev, n->ring_dev, st);
-        IFA_LAUNCH_CHECK();
     }
     if (elapsed_ms) IFA_HIP_CHECK(hipEventRecord(e1, m->stream));
-    IFA_HIP_CHECK(hipMemcpyAsync(out_tokens_host, n->ring_dev, (size_t)n_steps * 4, hipMemcpyDeviceToHost, m->stream));
+    // (the ring is kept by position)
+    const int at = start_pos % ifa_model::RING, head = std::min(n_steps, ifa_model::RING - at);
+    IFA_HIP_CHECK(hipMemcpyAsync(out_tokens_host, n->ring_dev + at, (size_t)head * 4, hipMemcpyDeviceToHost, m->stream));
+    if (n_steps > head) IFA_HIP_CHECK(hipMemcpyAsync(out_tokens_host + head, n->ring_dev, (size_t)(n_steps - head) * 4, hipMemcpyDeviceToHost, m->stream));
     IFA_HIP_CHECK(hipStreamSynchronize(m->stream));
     if (elapsed_ms) { IFA_HIP_CHECK(hipEventElapsedTime(elapsed_ms, e0, e1)); (void)hipEventDestroy(e0); (void)hipEventDestroy(e1); }
     return IFA_OK;

@@ -411,6 +411,64 @@ __global__ void __launch_bounds__(1024) k_argmax_f32(const float *__restrict__ l
     }
 }
 
+// The same for one row of many columns in two launches: a workgroup per part of the row (one compute unit takes a row of 32000, 128 KB, no faster than 7.9 us), then a wave over the parts.  step:
+// the row is a decode step's: its token goes on to be the next one's, inside the step's graph (a launch of its own behind it before: 235.3 -> 230.6 us a token of a Gelarax model of width 1024).
+constexpr int AM_PART = 1024, AM_PARTS = 64;          // columns a part (more where a row has more of them), most parts
+struct AmBest { float v; int i; };
+__device__ __forceinline__ void am_wave(AmBest &b)
+{
+    for (int o = 32; o > 0; o >>= 1) {
+        const float ov = __shfl_xor(b.v, o, 64); const int oi = __shfl_xor(b.i, o, 64);
+        if (ov > b.v || (ov == b.v && oi < b.i)) { b.v = ov; b.i = oi; }
+    }
+}
+__global__ void __launch_bounds__(256) k_argmax_parts(const float *__restrict__ r, int n, int part, const int *__restrict__ excluded, AmBest *__restrict__ best_of)
+{
+    __shared__ AmBest bs[4];
+    const int from = blockIdx.x * part, to = min(n, from + part);
+    const bool vec = ((uintptr_t)r & 15) == 0;          // (parts are whole pieces of four)
+    float v[4];
+    const int c0 = from + 4 * threadIdx.x;
+    auto fetch = [&](int c) {
+        if (vec && c + 4 <= to) { const float4 x = *reinterpret_cast<const float4 *>(r + c); v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w; }
+        else {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = c + e < to ? r[c + e] : 0.0f;
+        }
+    };
+    fetch(c0);          // (beside the excluded ones)
+    int ex[3] = {-1, -1, -1};
+    if (excluded) { const int e0 = excluded[0], e1 = excluded[1], e2 = excluded[2], e3 = excluded[3]; if (e0 > 0) ex[0] = e1; if (e0 > 1) ex[1] = e2; if (e0 > 2) ex[2] = e3; }
+    AmBest b = {-INFINITY, 0x7FFFFFFF};
+    for (int c = c0; c < to; c += 1024) {
+        if (c != c0) fetch(c);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int i = c + e;
+            if (i < to && i != ex[0] && i != ex[1] && i != ex[2] && (v[e] > b.v || (v[e] == b.v && i < b.i))) { b.v = v[e]; b.i = i; }
+        }
+    }
+    am_wave(b);
+    if ((threadIdx.x & 63) == 0) bs[threadIdx.x >> 6] = b;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; w++) if (bs[w].v > b.v || (bs[w].v == b.v && bs[w].i < b.i)) b = bs[w];
+        best_of[blockIdx.x] = b;
+    }
+}
+__global__ void __launch_bounds__(64) k_argmax_join(const AmBest *__restrict__ best_of, int parts, int *__restrict__ out, IfaStepAdvance step)
+{
+    AmBest b = {-INFINITY, 0x7FFFFFFF};
+    if ((int)threadIdx.x < parts) b = best_of[threadIdx.x];
+    int pos = 0;
+    if (step.tokens) pos = step.pos[0];
+    am_wave(b);
+    if (threadIdx.x != 0) return;
+    const int best = b.i == 0x7FFFFFFF ? 0 : b.i;
+    out[0] = best;
+    if (step.tokens) { step.tokens[0] = best; step.pos[0] = pos + 1; step.seqs[0].pos0 += 1; step.ring[pos % step.ring_size] = best; }
+}
+
 __global__ void __launch_bounds__(256) k_f32_to_f16(const float *__restrict__ src, size_t n, _Float16 *__restrict__ dst)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -603,6 +661,21 @@ int ifa_argmax_rows_f32(const void *logits_f32, size_t n, size_t row_stride, siz
 {
     IFA_REQUIRE(logits_f32 && out_dev && n > 0 && rows > 0 && n < (1u << 30), "ifa_argmax_rows_f32: bad arguments");
     hipLaunchKernelGGL(k_argmax_f32, dim3((unsigned)rows), dim3(n >= 4096 ? 1024 : 256), 0, ifa_s(stream), (const float *)logits_f32, (int)n, row_stride, excluded_dev, out_dev);
+    IFA_LAUNCH_CHECK();
+    return IFA_OK;
+}
+
+size_t ifa_argmax_parts_bytes() { return AM_PARTS * sizeof(AmBest); }
+
+int ifa_argmax_parts_f32(const float *logits, size_t n, size_t row_stride, size_t rows, const int *excluded_dev, int *out_dev, void *ws, const IfaStepAdvance *step, ifa_stream stream)
+{
+    IFA_REQUIRE(logits && out_dev && ws && n > 0 && rows > 0 && n < (1u << 30) && (!step || rows == 1), "ifa_argmax_parts_f32: bad arguments");
+    // (more rows: a workgroup each, side by side -- six rows of 32000 9.2 us in one launch, no more than the two)
+    if (rows > 1) return ifa_argmax_rows_f32(logits, n, row_stride, rows, excluded_dev, out_dev, stream);
+    const size_t part = std::max<size_t>(AM_PART, ((n + AM_PARTS - 1) / AM_PARTS + 3) / 4 * 4), parts = (n + part - 1) / part;
+    const IfaStepAdvance st = step ? *step : IfaStepAdvance{};
+    hipLaunchKernelGGL(k_argmax_parts, dim3((unsigned)parts), dim3(256), 0, ifa_s(stream), logits, (int)n, (int)part, excluded_dev, (AmBest *)ws);
+    hipLaunchKernelGGL(k_argmax_join, dim3(1), dim3(64), 0, ifa_s(stream), (const AmBest *)ws, (int)parts, out_dev, st);
     IFA_LAUNCH_CHECK();
     return IFA_OK;
 }

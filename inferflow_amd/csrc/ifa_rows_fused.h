@@ -21,6 +21,12 @@ constexpr int IFA_ROW_OUT_SPLITS = 8;
 bool ifa_row_out_fits(const IfaRowOut &P);
 int ifa_row_out(const IfaRowOut &P, ifa_stream stream);
 
+// ifa_argmax_rows_f32, one row in two launches (csrc/ifa_ops_f32.hip; ws of ifa_argmax_parts_bytes); step: a decode step's row, whose token becomes the next step's: tokens[0], ring[pos]
+// (modulo its size), position and the sequence's place one further on
+struct IfaStepAdvance { int *tokens, *pos; ifa_seq_desc *seqs; int *ring; int ring_size; };
+extern "C" size_t ifa_argmax_parts_bytes();
+extern "C" int ifa_argmax_parts_f32(const float *logits, size_t n, size_t row_stride, size_t rows, const int *excluded_dev, int *out_dev, void *ws, const IfaStepAdvance *step, ifa_stream stream);
+
 // the mixers of a WINDOW_LINEAR layer for ONE row: ifa_kv_store_f32 (keys normed, values the keys as projected) + ifa_attention_window_f32 + the decayed linear
 // attention of ifa_state_scan_f32.  *nsplit workgroups per head share the keys and nobody joins their shares (in ws; at most IFA_ROW_OUT_SPLITS; 1: out holds the row)
 struct IfaMixRow {

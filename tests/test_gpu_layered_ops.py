@@ -636,6 +636,42 @@ def test_argmax_of_rows_of_any_length(n):
         assert best.cpu().tolist() == [int(r.argmax()) for r in masked]
 
 
+@pytest.mark.parametrize("n", [1, 3, 1023, 1024, 1025, 4099, 32000, 65535, 65536, 65537, 70001])
+def test_argmax_in_parts_takes_what_the_argmax_of_a_row_does(n):
+    """the largest value at the edges of parts, twice (the lower index counts), excluded, beside NaN and among infinities; rows that start at odd places; and a decode step's move to its next token"""
+    lib = capi()
+    lib.ifa_argmax_parts_bytes.restype = C.c_size_t
+    f = lib.ifa_argmax_parts_f32
+    f.argtypes = [C.c_void_p, C.c_size_t, C.c_size_t, C.c_size_t] + [C.c_void_p] * 5
+    part = max(1024, ((n + 63) // 64 + 3) // 4 * 4)
+    spots = sorted({0, 3, n - 1, n // 2, part - 1, part, 2 * part - 1, (n - 1) // part * part} & set(range(n)))
+    rng = np.random.default_rng(n)
+    lg = rng.standard_normal((2 * len(spots) + 2, n + 1)).astype(np.float32)
+    for i, c in enumerate(spots):
+        lg[2 * i, c] = 9.0
+        lg[2 * i + 1, c] = lg[2 * i + 1, n - 1] = lg[2 * i + 1, n // 3] = 9.0
+        lg[2 * i, (c + 1) % n] = np.nan if n > 1 else 9.0
+    lg[-2] = -np.inf
+    lg[-1] = np.nan
+    lg[:, n:] = 99.0
+    x, ws = dev32(lg), torch.empty(lib.ifa_argmax_parts_bytes(), dtype=torch.uint8, device="cuda")
+    for ex in ([0, -1, -1, -1], [1, n - 1, -1, -1], [3, n - 1, 0, n // 3]):
+        got, want, rows = (torch.empty(len(lg), dtype=torch.int32, device="cuda") for _ in range(3))
+        ia.check(lib.ifa_argmax_rows_f32(p(x), n, lg.shape[1], len(lg), p(devi(ex)), p(want), stream()))
+        ia.check(f(p(x), n, lg.shape[1], len(lg), p(devi(ex)), p(rows), p(ws), None, stream()))
+        for r in range(len(lg)):
+            ia.check(f(C.c_void_p(x.data_ptr() + 4 * r * lg.shape[1]), n, lg.shape[1], 1, p(devi(ex)), C.c_void_p(got.data_ptr() + 4 * r), p(ws), None, stream()))
+        assert torch.equal(got, want) and torch.equal(rows, want)
+
+    class Advance(C.Structure):
+        _fields_ = [("tokens", C.c_void_p), ("pos", C.c_void_p), ("seqs", C.c_void_p), ("ring", C.c_void_p), ("ring_size", C.c_int)]
+    tokens, pos, seqs, ring, best = devi([7]), devi([1030]), devi([0, 1, 1030, 5]), torch.full((8,), -1, dtype=torch.int32, device="cuda"), devi([-1])
+    step = Advance(tokens.data_ptr(), pos.data_ptr(), seqs.data_ptr(), ring.data_ptr(), 8)
+    ia.check(f(p(x), n, lg.shape[1], 1, None, p(best), p(ws), C.byref(step), stream()))
+    at = int(best.cpu()[0])
+    assert tokens.tolist() == [at] and pos.tolist() == [1031] and seqs.tolist() == [0, 1, 1031, 5] and ring.tolist() == [-1] * 6 + [at, -1]
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 5, 8])
 def test_row_products_with_the_norm_or_the_gated_gelu_folded_in(T):
     rng = np.random.default_rng(40 + T)
