@@ -784,14 +784,22 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
         if (rc) return rc;
         // the router's logits (bias added by the product) are columns of the second product; the chosen experts read norm2's output
         const bool choose = !(fused && T <= 8 && sp.x_experts <= 256);          // (a few rows: the choice inside the experts' first launch)
+        const IfaMoeShared shared = {(const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, n->m3, SFP, (int)SFP, n->proj + L.c2_sg, N2, n->m1, W};
+        // (its activations are there; its rows go beside the experts', added up by the norm behind them, which takes such rows)
+        const bool with_shared = !choose && SFP > 0 && left == GLU_32 && n->mix_max >= W && W % 4 == 0 && W <= 8192
+                                 && (((uintptr_t)L.T(IFA_LT_NORM2B).data | (uintptr_t)next_norm) & 7) == 0 && ifa_moe_shared_fits(shared);
         if (choose && (rc = ifa_moe_route_top_f32(n->proj + L.c2_router, N2, T, sp.x_experts, sp.x_top, nullptr, n->moe_idx, n->moe_wgt, s))) return rc;
-        rc = !choose ? ifa_moe_experts_gated_top_rows(n->proj + L.c2_router, N2, n->h, W, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data,
-                                                      n->moe_idx, n->moe_wgt, n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, s)
+        rc = !choose ? ifa_moe_experts_gated_top_rows_shared(n->proj + L.c2_router, N2, n->h, W, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data,
+                                                      n->moe_idx, n->moe_wgt, n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, with_shared ? &shared : nullptr, s)
            : moe16 ? ifa_moe_experts_gated_bf16(n->h16, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data, n->moe_idx, n->moe_wgt, n->moe_ws,
                                                 n->moe_ws_bytes, n->m2, W, 0, s)
                    : ifa_moe_experts_gated_f32(n->h, W, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data, n->moe_idx, n->moe_wgt, c.ops32,
                                                n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, s);
         if (rc) return rc;
+        if (with_shared) {
+            if (ifa_norm_add_two_norm_f32(n->x, W, T, W, n->m2, n->m1, W, L.T(IFA_LT_NORM2B).data, next_norm, w_off, c.eps, n->h, W, s)) { IFA_LAUNCH_CHECK(); return IFA_OK; }
+            return ifa_fail(IFA_ERR_STATE, "rows of %zu columns that the norm behind the experts does not take", W);
+        }
         if (sp.x_shared_ff > 0) {      // the shared expert: its gate sigmoid(w_sg . h) multiplies the activations in front of the down-projection
             const size_t SF = (size_t)sp.x_shared_ff;
             if ((rc = glu_down(m, left, 0, 0.0f, n->proj + L.c2_shg, N2, SF, n->proj + L.c2_sg, N2, (const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, W, T, nullptr, nullptr, 1, n->m2))) return rc;

@@ -276,13 +276,60 @@ __global__ void __launch_bounds__(256) k_moe_up_rows(const float *__restrict__ h
 // grid (width chunks, rows): y[t][c] (+)= sum_k wgt * (identity ? h[t][c] : W_down[e][c] . act[p]); a wave per c at a time.  The chosen
 // experts are walked NK at a time with their loads issued side by side (a step is bound by requests in flight: four experts take 130 registers, so that twice as many
 // waves are in flight as with eight), their weighted partial sums reduced once (six rows of four experts of 704 columns 21.6 -> 12.4 us).
-template <int NK>
+// SHARED: the first of the rows' workgroups (one more than rows) are the shared expert's output product of all rows (k_lin_rows' sums, times sigmoid of a row's gate) into rows of their own, which
+// the norm behind adds: six rows of four experts of 704 and a shared one of 1408 to 1024 columns 13.0 + 9.8 -> 17.9 us.  (Added by the wave that has the row's sum, which reads the shared weights
+// once a row: 19.9; the shared expert's workgroups behind the others: 19.7.)
+constexpr int SH_ROWS = 8;
+__device__ __forceinline__ void shared_down(const IfaMoeShared &S, int rows, int W, int wave, int nwaves)
+{
+    constexpr int SP = 4;          // (pieces of 512 columns asked for ahead)
+    const int lane = threadIdx.x & 63;
+    for (int c = wave; c < W; c += nwaves) {
+        const bf16_t *w = S.down + (size_t)c * S.ff;
+        float acc[SH_ROWS];
+#pragma unroll
+        for (int t = 0; t < SH_ROWS; t++) acc[t] = 0.0f;
+        for (int k0 = 0; k0 < S.ff; k0 += 512 * SP) {
+            u32x4m wv[SP];
+#pragma unroll
+            for (int j = 0; j < SP; j++) wv[j] = *reinterpret_cast<const u32x4m *>(w + min(k0 + 512 * j + lane * 8, S.ff - 8));
+#pragma unroll
+            for (int j = 0; j < SP; j++) {
+                if (k0 + 512 * j >= S.ff) break;
+                const int k = k0 + 512 * j + lane * 8;
+                float4 a[SH_ROWS][2];
+#pragma unroll
+                for (int t = 0; t < SH_ROWS; t++) {
+                    const float *r = S.act + (size_t)min(t, rows - 1) * S.lda + min(k, S.ff - 8);
+                    a[t][0] = *reinterpret_cast<const float4 *>(r); a[t][1] = *reinterpret_cast<const float4 *>(r + 4);
+                }
+                if (k >= S.ff) continue;
+#pragma unroll
+                for (int t = 0; t < SH_ROWS; t++) {
+                    const float v[8] = {a[t][0].x, a[t][0].y, a[t][0].z, a[t][0].w, a[t][1].x, a[t][1].y, a[t][1].z, a[t][1].w};
+#pragma unroll
+                    for (int e = 0; e < 8; e++) acc[t] = fmaf(v[e], __uint_as_float((e & 1) ? (wv[j][e >> 1] & 0xFFFF0000u) : (wv[j][e >> 1] << 16)), acc[t]);
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < SH_ROWS; t++) acc[t] = wave_sum(acc[t]);
+#pragma unroll
+        for (int t = 0; t < SH_ROWS; t++)
+            if (lane == t && t < rows) S.out[(size_t)t * S.ldo + c] = acc[t] * sigmoid_f(S.gate[(size_t)t * S.ldg]);
+    }
+}
+template <int NK, bool SHARED>
 __global__ void __launch_bounds__(256) k_moe_down_rows(const float *__restrict__ h, size_t ldh, int W, int F, int experts, int top, const bf16_t *__restrict__ down,
                                                        const int *__restrict__ idx, const float *__restrict__ wgt, const float *__restrict__ act,
-                                                       int accumulate, float *__restrict__ y, size_t ldy, int vec)
+                                                       int accumulate, float *__restrict__ y, size_t ldy, int vec, std::conditional_t<SHARED, IfaMoeShared, int> S)
 {
-    const int t = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), nwaves = gridDim.x * (blockDim.x >> 6);
+    int t = blockIdx.y;
+    if constexpr (SHARED) {
+        if (t == 0) { shared_down(S, (int)gridDim.y - 1, W, wave, nwaves); return; }
+        t--;
+    }
     for (int c = wave; c < W; c += nwaves) {
         float out = 0.0f, part = 0.0f;
         for (int k0 = 0; k0 < top; k0 += NK) {
@@ -623,7 +670,7 @@ static int moe_tile_rows16(size_t pairs, int width, int experts)
 
 static int moe_experts(const char *who, int gated, int glu_kind, float limit, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int identity, int top, int act,
                        const void *up_bf16, const void *down_bf16, const int *idx_dev, const void *wgt_f32, int ops32, void *ws, size_t ws_bytes,
-                       void *y_f32, size_t ldy, int accumulate, ifa_stream stream, const RouteSel *sel = nullptr, const void *h_bf16 = nullptr)
+                       void *y_f32, size_t ldy, int accumulate, ifa_stream stream, const RouteSel *sel = nullptr, const void *h_bf16 = nullptr, const IfaMoeShared *shared = nullptr)
 {
     IFA_REQUIRE((h_f32 || h_bf16) && idx_dev && wgt_f32 && ws && y_f32 && (experts == 0 || (up_bf16 && down_bf16)), "%s: null pointer", who);
     IFA_REQUIRE(rows > 0 && rows < 65536 && width > 0 && ff > 0 && experts >= 0 && experts <= 4096 && identity >= 0 && top >= 1 && top <= experts + identity && act == 0
@@ -651,11 +698,12 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
         else if (experts > 0)
             hipLaunchKernelGGL((k_moe_up_rows<false, false>), dim3(std::min(512u, ifa_cdiv((size_t)ff, 4)), (unsigned)pairs), dim3(256), 0, s, h, ldh, width, ff, experts, top,
                                (const bf16_t *)up_bf16, idx_dev, actb, vec_u, 0, 0.0f, RouteSel());
-        const dim3 grid(std::min(1024u, ifa_cdiv((size_t)width, 4)), (unsigned)rows);
-        if (top <= 4) hipLaunchKernelGGL(k_moe_down_rows<4>, grid, dim3(256), 0, s, h, ldh, width, ff, experts, top, (const bf16_t *)down_bf16, idx_dev, (const float *)wgt_f32, actb,
-                                         accumulate ? 1 : 0, (float *)y_f32, ldy, vec_d);
-        else hipLaunchKernelGGL(k_moe_down_rows<8>, grid, dim3(256), 0, s, h, ldh, width, ff, experts, top, (const bf16_t *)down_bf16, idx_dev, (const float *)wgt_f32, actb,
-                                accumulate ? 1 : 0, (float *)y_f32, ldy, vec_d);
+        const dim3 grid(std::min(1024u, ifa_cdiv((size_t)width, 4)), (unsigned)rows + (shared ? 1u : 0u));
+#define IFA_DOWN(NK, SH, S) hipLaunchKernelGGL((k_moe_down_rows<NK, SH>), grid, dim3(256), 0, s, h, ldh, width, ff, experts, top, (const bf16_t *)down_bf16, idx_dev, (const float *)wgt_f32, \
+                                               actb, accumulate ? 1 : 0, (float *)y_f32, ldy, vec_d, S)
+        if (top <= 4) { if (shared) IFA_DOWN(4, true, *shared); else IFA_DOWN(4, false, 0); }
+        else { if (shared) IFA_DOWN(8, true, *shared); else IFA_DOWN(8, false, 0); }
+#undef IFA_DOWN
         IFA_LAUNCH_CHECK();
         return IFA_OK;
     }
@@ -731,15 +779,29 @@ int ifa_moe_experts_routed_rows_f32(int score_kind, int renorm, float renorm_eps
 
 } // extern "C"
 
-int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
-                                   const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream)
+int ifa_moe_experts_gated_top_rows_shared(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
+                                   const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, const IfaMoeShared *shared,
+                                   ifa_stream stream)
 {
+    IFA_REQUIRE(!shared || (shared->down && shared->act && shared->gate && shared->out && shared->ldo >= (size_t)width && ifa_moe_shared_fits(*shared)), "moe_experts_gated_top_rows: shared expert of %d columns", shared ? shared->ff : 0);
     IFA_REQUIRE(logits_f32 && rows <= 8 && experts > 0 && experts <= 256 && ldl >= (size_t)experts, "moe_experts_gated_top_rows: %zu rows (at most 8), %d experts (at most 256)", rows, experts);
     RouteSel R;
     memset(&R, 0, sizeof(R));
     R.logits = (const float *)logits_f32; R.ld = ldl; R.n_all = experts; R.score_kind = 2; R.idx = idx_dev; R.wgt = (float *)wgt_f32;
     return moe_experts("moe_experts_gated_top_rows", 1, 0, 0.0f, h_f32, ldh, rows, width, ff, experts, 0, top, 0, gate_up_bf16, down_bf16, idx_dev, wgt_f32, 1, ws, ws_bytes, y_f32, ldy,
-                       accumulate, stream, &R);
+                       accumulate, stream, &R, nullptr, shared);
+}
+
+int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
+                                   const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream)
+{
+    return ifa_moe_experts_gated_top_rows_shared(logits_f32, ldl, h_f32, ldh, rows, width, ff, experts, top, gate_up_bf16, down_bf16, idx_dev, wgt_f32, ws, ws_bytes, y_f32, ldy, accumulate,
+                                                 nullptr, stream);
+}
+
+bool ifa_moe_shared_fits(const IfaMoeShared &S)
+{
+    return S.ff >= 8 && S.ff % 8 == 0 && S.lda >= (size_t)S.ff && S.lda % 4 == 0 && (((uintptr_t)S.down | (uintptr_t)S.act) & 15) == 0;
 }
 
 bool ifa_moe_gated_reads_bf16(size_t rows, int width, int ff, int top, int ops32, const void *gate_up_bf16, const void *down_bf16)

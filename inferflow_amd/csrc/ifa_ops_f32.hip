@@ -254,7 +254,7 @@ struct MoePairs { const int *pos; const float *rows; int top, has_m; };
 template <int PIECES, bool MOE>
 __global__ void __launch_bounds__(1024) k_norm_add_norm_reg(float *__restrict__ x, size_t ldx, int cols, const float *__restrict__ m, size_t ldm,
                                                             const bf16_t *__restrict__ w_after, const bf16_t *__restrict__ w_before, float w_off, float eps,
-                                                            float *__restrict__ h, bf16_t *__restrict__ h16, size_t ldh, std::conditional_t<MOE, MoePairs, int> M)
+                                                            float *__restrict__ h, bf16_t *__restrict__ h16, size_t ldh, std::conditional_t<MOE, MoePairs, const float *> M)
 {
     __shared__ float red[17];
     float *xr = x + (size_t)blockIdx.x * ldx;
@@ -287,6 +287,8 @@ __global__ void __launch_bounds__(1024) k_norm_add_norm_reg(float *__restrict__ 
             if (M.has_m) { a.x += own.x; a.y += own.y; a.z += own.z; a.w += own.w; }
             if (c >= cols) a = make_float4(0.f, 0.f, 0.f, 0.f);
         }
+        if constexpr (!MOE)          // (M: rows that m's are added up with, or null)
+            if (M && c < cols) { const float4 v = *reinterpret_cast<const float4 *>(M + (size_t)blockIdx.x * ldm + c); a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w; }
         mv[p][0] = a.x; mv[p][1] = a.y; mv[p][2] = a.z; mv[p][3] = a.w; xv[p][0] = b.x; xv[p][1] = b.y; xv[p][2] = b.z; xv[p][3] = b.w;
     }
 #pragma unroll
@@ -624,10 +626,10 @@ int ifa_add_rows_vec_f32(void *x_f32, size_t ldx, size_t rows, size_t cols, cons
 
 // launches k_norm_add_norm_reg where the row fits the registers and every access is aligned; false: nothing launched
 static bool norm_add_norm_reg(void *x, size_t ldx, size_t rows, size_t cols, const void *m, size_t ldm, const void *w_after, const void *w_before, float w_offset, float eps,
-                              void *h, void *h16, size_t ldh, ifa_stream stream, const MoePairs *moe = nullptr)
+                              void *h, void *h16, size_t ldh, ifa_stream stream, const MoePairs *moe = nullptr, const float *m2 = nullptr)
 {
     const size_t quads = cols / 4;
-    const bool vec = cols % 4 == 0 && ldx % 4 == 0 && (!m || ldm % 4 == 0) && (((uintptr_t)x | (uintptr_t)m) & 15) == 0 && ((uintptr_t)w_after & 7) == 0
+    const bool vec = cols % 4 == 0 && ldx % 4 == 0 && (!m || ldm % 4 == 0) && (((uintptr_t)x | (uintptr_t)m | (uintptr_t)m2) & 15) == 0 && ((uintptr_t)w_after & 7) == 0
                      && (!w_before || (ldh % 4 == 0 && (((uintptr_t)h | (uintptr_t)h16) & 15) == 0 && ((uintptr_t)w_before & 7) == 0));
     if (!vec || quads > 2048) return false;
     const int pieces = quads <= 1024 ? 1 : 2;          // one piece of four values per thread up to 4096 columns, two beyond
@@ -635,8 +637,8 @@ static bool norm_add_norm_reg(void *x, size_t ldx, size_t rows, size_t cols, con
 #define IFA_NAN(P, MOE, M) hipLaunchKernelGGL((k_norm_add_norm_reg<P, MOE>), dim3((unsigned)rows), dim3(threads), 0, ifa_s(stream), (float *)x, ldx, (int)cols, (const float *)m, ldm, \
                                               (const bf16_t *)w_after, (const bf16_t *)w_before, w_offset, eps, (float *)h, (bf16_t *)h16, ldh, M)
     if (moe) { if (pieces == 1) IFA_NAN(1, true, *moe); else IFA_NAN(2, true, *moe); }
-    else if (pieces == 1) IFA_NAN(1, false, 0);
-    else IFA_NAN(2, false, 0);
+    else if (pieces == 1) IFA_NAN(1, false, m2);
+    else IFA_NAN(2, false, m2);
 #undef IFA_NAN
     return true;
 }
@@ -734,6 +736,13 @@ int ifa_norm_add_norm_moe(void *x_f32, size_t ldx, size_t rows, size_t cols, con
                 "norm_add_norm_moe: rows of %zu columns (at most 8192, whole 16-byte pieces, aligned)", cols);
     IFA_LAUNCH_CHECK();
     return IFA_OK;
+}
+
+bool ifa_norm_add_two_norm_f32(void *x_f32, size_t ldx, size_t rows, size_t cols, const void *m_f32, const void *m2_f32, size_t ldm, const void *w_after_bf16, const void *w_before_bf16,
+                              float w_offset, float eps, void *h_f32, size_t ldh, ifa_stream stream)
+{
+    if (!x_f32 || !m_f32 || !m2_f32 || !w_after_bf16 || (w_before_bf16 && !h_f32) || rows == 0 || cols == 0 || ldx < cols || ldm < cols || (w_before_bf16 && ldh < cols)) return false;
+    return norm_add_norm_reg(x_f32, ldx, rows, cols, m_f32, ldm, w_after_bf16, w_before_bf16, w_offset, eps, h_f32, nullptr, ldh, stream, nullptr, (const float *)m2_f32);
 }
 
 int ifa_norm_add_norm_f32(void *x_f32, size_t ldx, size_t rows, size_t cols, const void *m_f32, size_t ldm, const void *w_after_bf16,

@@ -106,12 +106,21 @@ struct IfaMoePrompt {
     const float *sh_gate_up; size_t sh_ld; int sh_ff; const float *sh_gate; size_t sh_ldg; ifa32::bf16_t *sh_act; size_t sh_ldo;
 };
 extern "C" int ifa_moe_prompt(const IfaMoePrompt &P, const int **pair_pos, const float **pair_rows, ifa_stream stream);
+// ifa_norm_add_norm_f32 of the row m[t] + m2[t] (rows of ldm; false: sizes or alignment don't allow it, nothing launched)
+extern "C" bool ifa_norm_add_two_norm_f32(void *x_f32, size_t ldx, size_t rows, size_t cols, const void *m_f32, const void *m2_f32, size_t ldm, const void *w_after_bf16, const void *w_before_bf16,
+                              float w_offset, float eps, void *h_f32, size_t ldh, ifa_stream stream);
 // ifa_norm_add_norm_f32 / _to_bf16 (h_f32 or h_bf16) of the row  sum_k pair_rows[pair_pos[t][k]] (+ m[t])
 extern "C" int ifa_norm_add_norm_moe(void *x_f32, size_t ldx, size_t rows, size_t cols, const void *m_f32, size_t ldm, const int *pair_pos_dev, const void *pair_rows_f32, int top,
                           const void *w_after_bf16, const void *w_before_bf16, float w_offset, float eps, void *h_f32, void *h_bf16, size_t ldh, ifa_stream stream);
-// ifa_moe_route_top_f32 inside the first launch of ifa_moe_experts_gated_f32: at most eight rows, 256 experts
+// ifa_moe_route_top_f32 inside the first launch of ifa_moe_experts_gated_f32: at most eight rows, 256 experts.  shared: the shared expert's output product beside the experts' in their launch,
+// out[t] = sigmoid(gate[t * ldg]) down . act[t] (ifa_linear_bf16w_gated_rows; rows that ifa_moe_shared_fits allows)
+struct IfaMoeShared { const ifa32::bf16_t *down; const float *act; size_t lda; int ff; const float *gate; size_t ldg; float *out; size_t ldo; };
+extern "C" bool ifa_moe_shared_fits(const IfaMoeShared &S);
 extern "C" int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
                                    const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream);
+extern "C" int ifa_moe_experts_gated_top_rows_shared(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
+                                          const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, const IfaMoeShared *shared,
+                                          ifa_stream stream);
 // ifa_glu_ex_f32 whose output only products read: bfloat16 rows, zero up to ldo (a multiple of 8; csrc/ifa_ops_f32.hip)
 int ifa_glu_to_bf16(int kind, float limit, const void *gate_up_f32, size_t ld, size_t rows, size_t cols, const void *row_gate_f32, size_t ldg, void *out_bf16, size_t ldo,
                     ifa_stream stream);

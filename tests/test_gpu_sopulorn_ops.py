@@ -268,6 +268,41 @@ def test_choice_by_the_largest_logits_inside_the_experts_first_launch(T, W, F, E
     assert np.array_equal(got, y_w.cpu().numpy(), equal_nan=True) and np.isfinite(got[some]).all() and (T <= 6 or np.isnan(got[6, :W]).all())
 
 
+@pytest.mark.parametrize("T,W,F,SF,E,top", [(1, 64, 24, 8, 6, 2), (6, 128, 64, 1408, 16, 4), (8, 40, 10, 520, 3, 3), (5, 14, 6, 2048, 70, 8), (7, 64, 16, 2056, 16, 9), (2, 16, 8, 4104, 1, 1)])
+def test_shared_expert_in_the_experts_last_launch_leaves_the_bits_of_its_own(T, W, F, SF, E, top):
+    """the output product beside the sum over the experts, in one launch and in two: pieces of 512 columns whole and ragged, more of them than are asked for ahead, rows of activations, gates and
+    outputs with strides; the experts' rows onto what is there and in its place; and the norm behind both, which adds them up"""
+    class Shared(C.Structure):
+        _fields_ = [("down", C.c_void_p), ("act", C.c_void_p), ("lda", C.c_size_t), ("ff", C.c_int), ("gate", C.c_void_p), ("ldg", C.c_size_t), ("out", C.c_void_p), ("ldo", C.c_size_t)]
+    rng = np.random.default_rng(T + W + SF)
+    L, Z = capi(), C.c_size_t
+    dh, dz = dev32(rng.standard_normal((T, W))), dev32(rng.standard_normal((T, E)))
+    gu, dd = devbf(bf16_round(rng.standard_normal((E * 2 * F, W)) / np.sqrt(W))), devbf(bf16_round(rng.standard_normal((E * W, F)) / np.sqrt(F)))
+    sd, act, gate = devbf(bf16_round(rng.standard_normal((W, SF)) / np.sqrt(SF))), dev32(rng.standard_normal((T, SF + 4))), dev32(rng.standard_normal((T, 3)))
+    nb = L.ifa_moe_workspace_bytes(T, top, W, 3 * F, E)
+    ws = torch.zeros((nb + 15) // 4, dtype=torch.float32, device="cuda")
+    idx, wgt = torch.zeros((T, top), dtype=torch.int32, device="cuda"), torch.zeros((T, top), dtype=torch.float32, device="cuda")
+    out, out_w = (torch.full((T, W + 2), 0.25, dtype=torch.float32, device="cuda") for _ in range(2))
+    shared = Shared(sd.data_ptr(), act.data_ptr(), SF + 4, SF, gate.data_ptr() + 4, 3, out.data_ptr(), W + 2)
+    for acc in (0, 1):
+        y, y_w = (torch.full((T, W + 1), 0.5, dtype=torch.float32, device="cuda") for _ in range(2))
+        args = [p(dz), Z(E), p(dh), Z(W), Z(T), W, F, E, top, p(gu), p(dd), p(idx), p(wgt), p(ws), Z(nb)]
+        ia.check(L.ifa_moe_experts_gated_top_rows_shared(*args, p(y), Z(W + 1), acc, C.byref(shared), None))
+        ia.check(L.ifa_moe_experts_gated_top_rows(*args, p(y_w), Z(W + 1), acc, None))
+        ia.check(L.ifa_linear_bf16w_gated_rows(p(sd), Z(W), Z(SF), p(act), Z(SF + 4), Z(T), C.c_void_p(gate.data_ptr() + 4), Z(3), 0, p(out_w), Z(W + 2), None)); sync()
+        assert torch.equal(y, y_w) and torch.equal(out, out_w) and torch.isfinite(y).all() and torch.isfinite(out).all()
+    if W % 4:
+        return
+    L.ifa_norm_add_two_norm_f32.restype = C.c_bool
+    a, b = y[:, :W].contiguous(), out[:, :W].contiguous()
+    wa, wb, x = devbf(bf16_round(rng.standard_normal(W))), devbf(bf16_round(rng.standard_normal(W))), dev32(rng.standard_normal((T, W)))
+    x_w, h, h_w = x.clone(), torch.zeros_like(x), torch.zeros_like(x)
+    f1 = C.c_float
+    assert L.ifa_norm_add_two_norm_f32(p(x), Z(W), Z(T), Z(W), p(a), p(b), Z(W), p(wa), p(wb), f1(1.0), f1(1e-6), p(h), Z(W), None)
+    ia.check(L.ifa_norm_add_norm_f32(p(x_w), W, T, W, p(a + b), W, p(wa), p(wb), 1.0, 1e-6, p(h_w), W, None)); sync()
+    assert torch.equal(x, x_w) and torch.equal(h, h_w)
+
+
 @pytest.mark.parametrize("T,W,F,E,top", [(1, 64, 24, 6, 2), (3, 40, 10, 3, 3), (8, 128, 64, 16, 4), (9, 64, 24, 6, 2), (70, 48, 20, 5, 1), (150, 64, 32, 20, 3), (5, 14, 6, 4, 2)])
 def test_gated_experts_in_rows_and_grouped(T, W, F, E, top):
     rng = np.random.default_rng(T + W + F)
