@@ -577,6 +577,33 @@ def test_tiled_attention_with_infinite_and_very_large_keys_and_values(where, val
             assert not part.any() or np.abs(got[part] / 2 - want[part] / 2).max() < 1e-6 * np.abs(want[part]).max(), rows
 
 
+@pytest.mark.parametrize("value", [3.395e38, -3.402e38, 3.3e38])
+def test_tiled_attention_with_very_large_queries(value):
+    """one value of two queries that rounds to no bfloat16, or just does, beside ordinary ones, on keys whose column is as small: the fp32 tiles' outputs within 2e-6 (the bound of the test above)"""
+    rng = np.random.default_rng(9)
+    heads, kv_heads, dim, n = 4, 2, 128, 100
+    host = (C.c_int * 4)(0, n, 0, 0)
+    d, rs, _ = seq_tables([(n, 0, 0)])
+    q = rng.standard_normal((n, heads, dim)).astype(np.float32)
+    q[40, 1, 77] = q[99, 3, 77] = value
+    k, v = (rng.standard_normal((n, kv_heads, dim)).astype(np.float32) for _ in range(2))
+    k[:, :, 77] *= 1e-30
+    sl = Slots(1, 2 * n * kv_heads * dim)
+    sl.mem[0].copy_(dev32(np.concatenate([k.reshape(-1), v.reshape(-1)])))
+    qd = dev32(q.reshape(n, -1))
+    nb = capi().ifa_attention_tile_workspace_bytes(host, 1, heads, kv_heads, dim, dim, 0, 0)
+    out = []
+    for ws_bytes in (nb, 0):
+        ws, o = torch.full((nb // 4,), float("nan"), dtype=torch.float32, device="cuda"), torch.zeros((n, heads * dim), dtype=torch.float32, device="cuda")
+        ia.check(capi().ifa_attention_kv_f32(p(qd), heads * dim, heads, kv_heads, dim, dim, 1e-8, 0, 0, 0, 0.0, p(d), p(rs), n, p(sl.table), 0, n * kv_heads * dim, p(o), heads * dim, host, 1, 16, 0,
+                                             p(ws) if ws_bytes else None, ws_bytes, None))
+        sync(); out.append(o.cpu().numpy())
+    got, want = out
+    assert np.isfinite(want).all() and np.abs(got - want).max() < 2e-6 * np.abs(want).max()
+    flat = v[:41, 0].mean(axis=0)          # (the large value counts: its query's weights are not all alike)
+    assert np.abs(want[40].reshape(heads, dim)[1] - flat).max() > 0.1
+
+
 @pytest.mark.parametrize("window,keep", [(1 << 30, 0), (90, 40)])
 def test_tiled_attention_over_many_sequences(window, keep):
     """130 sequences, most of one row, some of several and of more than four query tiles, at places that a wave looks at together and one by one: the rows' kernel's
