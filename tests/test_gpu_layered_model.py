@@ -523,3 +523,23 @@ def test_one_row_product_with_the_norm_inside(K, N):
     want[2:4] = orc.silu(want[2:4])
     got = c.cpu().numpy()
     assert np.abs(got[:N] - want.numpy()).max() < 1e-5 * max(1.0, float(want.abs().max())) and np.isnan(got[N:]).all()
+
+
+@pytest.mark.parametrize("start,steps", [(1010, 40), (1000, 25), (1024, 9)])
+def test_generation_across_the_end_of_the_ring_of_tokens(tmp_path, start, steps):
+    """the ring holds 1024 tokens by position: a call that ends at its last place, one that runs on from its first and one that starts there give the tokens that single steps do"""
+    cfg = fx.config([fx.parallel_layer(), fx.delta_layer()])
+    eng = engine_for(tmp_path, cfg, fx.random_weights(cfg, 61), ctx=1100, queries=1)
+    prompt = tokens_for(cfg, start, 7)
+    q = eng.add_query(prompt)
+    gen, _ = eng.generate(q, steps)
+    eng.remove_query(q)
+    q = eng.add_query(prompt)
+    one = []
+    for _ in range(steps):
+        t = eng.infer()[0][1]
+        one.append(t)
+        assert eng.commit({q: t})
+    eng.remove_query(q)
+    assert list(gen) == one
+    eng.close()
