@@ -137,31 +137,56 @@ __global__ void __launch_bounds__(256) k_group_rmsnorm(const float *__restrict__
 // x[t] = embed[token_t] + pair[row_t]; row_t = (prev_t * mul_prev + token_t * mul_cur) mod buckets, or `buckets` at position 0.  The
 // workgroup of a sequence's first row is the only one that reads the token the slot holds, and it leaves the sequence's last token
 // of this step there: no other workgroup touches that cell.
+// VEC: pieces of four columns, the first one of the row's embedding asked for beside the row's place, and the slot's cell by a sequence's first row alone: one by one behind the place and the slot a
+// launch took 8.4 / 17.0 us for 6 / 2048 rows of 1024, now 6.7 / 7.2
+template <bool VEC>
 __global__ void __launch_bounds__(256) k_embed_pair(const bf16_t *__restrict__ embed, int vocab, int width, const bf16_t *__restrict__ pair, int buckets,
                                                     int mul_prev, int mul_cur, const int *__restrict__ tokens, const SeqDesc *__restrict__ seqs,
                                                     const int *__restrict__ row_seq, float *const *__restrict__ slot_base, size_t state_off,
                                                     float *__restrict__ x, float embed_scale, float *__restrict__ x_copy)
 {
     const int t = blockIdx.x;
+    const int tok = min(max(tokens[t], 0), vocab - 1), before = tokens[max(t - 1, 0)];
     const SeqDesc sd = seqs[row_seq[t]];
-    const int tok = min(max(tokens[t], 0), vocab - 1);
-    int *cell = reinterpret_cast<int *>(slot_base[sd.slot] + state_off);
+    const bf16_t *er = embed + (size_t)tok * width;
+    uint2 first = make_uint2(0u, 0u);
+    if constexpr (VEC) if (4 * (int)threadIdx.x < width) first = *reinterpret_cast<const uint2 *>(er + 4 * threadIdx.x);
+    int *cell = nullptr;
+    if (t == sd.row0) cell = reinterpret_cast<int *>(slot_base[sd.slot] + state_off);
     int prow = buckets;
     if (pair) {
         const int pos = sd.pos0 + t - sd.row0;
         if (pos > 0) {
-            const int prev = t > sd.row0 ? tokens[t - 1] : *cell;
+            const int prev = t > sd.row0 ? before : *cell;
             prow = (int)(((long long)prev * mul_prev + (long long)tok * mul_cur) % (long long)buckets);
             if (prow < 0) prow += buckets;
         }
     }
     __syncthreads();      // (the read of the cell above is done in every thread before thread 0 rewrites it)
     if (t == sd.row0 && threadIdx.x == 0) *cell = tokens[sd.row0 + sd.n - 1];
-    for (int c = threadIdx.x; c < width; c += blockDim.x) {
-        float v = bf2f(embed[(size_t)tok * width + c]) * embed_scale;
-        if (pair) v += bf2f(pair[(size_t)prow * width + c]);
-        x[(size_t)t * width + c] = v;
-        if (x_copy) x_copy[(size_t)t * width + c] = v;
+    float *xr = x + (size_t)t * width, *xc = x_copy ? x_copy + (size_t)t * width : nullptr;
+    const bf16_t *pr = pair ? pair + (size_t)prow * width : nullptr;
+    if constexpr (VEC) {
+        for (int c = 4 * threadIdx.x; c < width; c += 4 * blockDim.x) {
+            const uint2 e = c < 4 * (int)blockDim.x ? first : *reinterpret_cast<const uint2 *>(er + c);
+            float v[4] = {__uint_as_float(e.x << 16), __uint_as_float(e.x & 0xFFFF0000u), __uint_as_float(e.y << 16), __uint_as_float(e.y & 0xFFFF0000u)};
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] *= embed_scale;
+            if (pr) {
+                const uint2 q = *reinterpret_cast<const uint2 *>(pr + c);
+                v[0] += __uint_as_float(q.x << 16); v[1] += __uint_as_float(q.x & 0xFFFF0000u); v[2] += __uint_as_float(q.y << 16); v[3] += __uint_as_float(q.y & 0xFFFF0000u);
+            }
+            const float4 o = make_float4(v[0], v[1], v[2], v[3]);
+            *reinterpret_cast<float4 *>(xr + c) = o;
+            if (xc) *reinterpret_cast<float4 *>(xc + c) = o;
+        }
+    } else {
+        for (int c = threadIdx.x; c < width; c += blockDim.x) {
+            float v = bf2f(er[c]) * embed_scale;
+            if (pr) v += bf2f(pr[c]);
+            xr[c] = v;
+            if (xc) xc[c] = v;
+        }
     }
 }
 
@@ -569,11 +594,7 @@ int ifa_embed_pair_f32(const void *embed_bf16, int vocab, int width, const void 
 {
     IFA_REQUIRE(embed_bf16 && tokens_dev && seqs_dev && row_seq_dev && slot_base_dev && x_f32, "ifa_embed_pair_f32: null pointer");
     IFA_REQUIRE(vocab > 0 && width > 0 && rows > 0 && (!pair_bf16 || buckets > 0), "ifa_embed_pair_f32: bad shape");
-    hipLaunchKernelGGL(k_embed_pair, dim3((unsigned)rows), dim3(256), 0, ifa_s(stream), (const bf16_t *)embed_bf16, vocab, width, (const bf16_t *)pair_bf16, buckets,
-                       mul_prev, mul_cur, tokens_dev, (const SeqDesc *)seqs_dev, row_seq_dev, (float *const *)slot_base_dev, state_off, (float *)x_f32, 1.0f,
-                       (float *)nullptr);
-    IFA_LAUNCH_CHECK();
-    return IFA_OK;
+    return ifa_embed_pair_scaled_f32(embed_bf16, vocab, width, 1.0f, pair_bf16, buckets, mul_prev, mul_cur, tokens_dev, seqs_dev, row_seq_dev, rows, slot_base_dev, state_off, x_f32, nullptr, stream);
 }
 
 int ifa_embed_pair_scaled_f32(const void *embed_bf16, int vocab, int width, float embed_scale, const void *pair_bf16, int buckets, int mul_prev, int mul_cur,
@@ -582,9 +603,12 @@ int ifa_embed_pair_scaled_f32(const void *embed_bf16, int vocab, int width, floa
 {
     IFA_REQUIRE(embed_bf16 && tokens_dev && seqs_dev && row_seq_dev && slot_base_dev && x_f32, "ifa_embed_pair_scaled_f32: null pointer");
     IFA_REQUIRE(vocab > 0 && width > 0 && rows > 0 && (!pair_bf16 || buckets > 0), "ifa_embed_pair_scaled_f32: bad shape");
-    hipLaunchKernelGGL(k_embed_pair, dim3((unsigned)rows), dim3(256), 0, ifa_s(stream), (const bf16_t *)embed_bf16, vocab, width, (const bf16_t *)pair_bf16, buckets,
-                       mul_prev, mul_cur, tokens_dev, (const SeqDesc *)seqs_dev, row_seq_dev, (float *const *)slot_base_dev, state_off, (float *)x_f32, embed_scale,
-                       (float *)x_copy_f32);
+    const bool vec = width % 4 == 0 && (((uintptr_t)embed_bf16 | (uintptr_t)pair_bf16) & 7) == 0 && (((uintptr_t)x_f32 | (uintptr_t)x_copy_f32) & 15) == 0;
+#define IFA_EP(V) hipLaunchKernelGGL(k_embed_pair<V>, dim3((unsigned)rows), dim3(256), 0, ifa_s(stream), (const bf16_t *)embed_bf16, vocab, width, (const bf16_t *)pair_bf16, buckets, \
+                                     mul_prev, mul_cur, tokens_dev, (const SeqDesc *)seqs_dev, row_seq_dev, (float *const *)slot_base_dev, state_off, (float *)x_f32, embed_scale, \
+                                     (float *)x_copy_f32)
+    if (vec) IFA_EP(true); else IFA_EP(false);
+#undef IFA_EP
     IFA_LAUNCH_CHECK();
     return IFA_OK;
 }

@@ -268,6 +268,31 @@ def test_choice_by_the_largest_logits_inside_the_experts_first_launch(T, W, F, E
     assert np.array_equal(got, y_w.cpu().numpy(), equal_nan=True) and np.isfinite(got[some]).all() and (T <= 6 or np.isnan(got[6, :W]).all())
 
 
+@pytest.mark.parametrize("W", [1, 4, 7, 1020, 1024, 1028, 1030, 2052])
+def test_embedding_rows_in_pieces_of_four_columns_and_one_by_one(W):
+    """widths within a round of the threads' pieces and beyond, whole pieces and not; two sequences, one from the start and one behind a token kept in its slot; with a pair table, without, and the
+    rows a second time: the values exactly"""
+    rng = np.random.default_rng(W)
+    V, B, mp, mc, scale = 50, 11, 36313, 27191, 1.7
+    E, P = bf16_round(rng.standard_normal((V, W))), bf16_round(rng.standard_normal((B + 1, W)))
+    slots = Slots(2, 64)
+    toks, L = np.array([3, 49, 0, 7, 8, 60, 12], np.int32), capi()
+    sd, rs, rows = seq_tables([(4, 0, 0), (3, 5, 1)])
+    for pair in (True, False):
+        slots.mem[1].view(torch.int32)[4] = 21
+        x, xc = (torch.full((rows, W), float("nan"), dtype=torch.float32, device="cuda") for _ in range(2))
+        ia.check(L.ifa_embed_pair_scaled_f32(p(devbf(E)), V, W, scale, p(devbf(P)) if pair else None, B, mp, mc, p(devi(toks)), p(sd), p(rs), rows, p(slots.table), 4, p(x), p(xc), None)); sync()
+        prev = [None, 3, 49, 0, 21, 8, 60]
+        want = np.zeros((rows, W), np.float32)
+        for t in range(rows):
+            tok = min(int(toks[t]), V - 1)
+            want[t] = E[tok].astype(np.float32) * np.float32(scale)
+            if pair:
+                want[t] += P[B if prev[t] is None else (prev[t] * mp + tok * mc) % B].astype(np.float32)
+        assert np.array_equal(x.cpu().numpy(), want) and torch.equal(x, xc)
+        assert int(slots.mem[0].view(torch.int32)[4]) == 7 and int(slots.mem[1].view(torch.int32)[4]) == 12
+
+
 @pytest.mark.parametrize("T,W,F,SF,E,top", [(1, 64, 24, 8, 6, 2), (6, 128, 64, 1408, 16, 4), (8, 40, 10, 520, 3, 3), (5, 14, 6, 2048, 70, 8), (7, 64, 16, 2056, 16, 9), (2, 16, 8, 4104, 1, 1)])
 def test_shared_expert_in_the_experts_last_launch_leaves_the_bits_of_its_own(T, W, F, SF, E, top):
     """the output product beside the sum over the experts, in one launch and in two: pieces of 512 columns whole and ragged, more of them than are asked for ahead, rows of activations, gates and
