@@ -769,15 +769,18 @@ __device__ __forceinline__ Turn turn_of(int dim, int rot_dims, const bf16_t *nw_
     for (int e = 0; e < 2; e++) { const int c = lane + 64 * e; u.w[e] = nw_ ? bf2f(nw_[min(c, dim - 1)]) : 1.0f; u.first[e] = c < u.half; u.from[e] = c < u.half ? c + u.half : c - u.half; }
     return u;
 }
+// the factor of a held head's root mean square norm
+__device__ __forceinline__ float norm_held(const float (&v)[2], int dim, float eps, int lane)
+{
+    float s = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 2; e++) if (lane + 64 * e < dim) s = fmaf(v[e], v[e], s);
+    return 1.0f / sqrtf(wave_sum(s) / (float)dim + eps);
+}
 __device__ __forceinline__ void turn_held(float (&v)[2], const Turn &u, int dim, bool norm, float eps, int rot_dims, const float (&cv)[2], const float (&sv)[2], int lane)
 {
     float r = 1.0f, val[2];
-    if (norm) {
-        float s = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 2; e++) if (lane + 64 * e < dim) s = fmaf(v[e], v[e], s);
-        r = 1.0f / sqrtf(wave_sum(s) / (float)dim + eps);
-    }
+    if (norm) r = norm_held(v, dim, eps, lane);
 #pragma unroll
     for (int e = 0; e < 2; e++) val[e] = v[e] * r * u.w[e];
 #pragma unroll
@@ -832,7 +835,9 @@ struct FreshKV { const float *k; size_t ldk; const float *v; size_t ldv; int nor
 // step brings into the cache on their way: a position is in one of the step's blocks, and only there.  Keys go through LDS, all asked for at once.  Bound by its launch and its trips to
 // memory (reads 4, writes 6 bytes per value; fresh rows: 10).  Rows past the sequence's last: that row again (their scores are masked).
 // (A launch that stored the rows and one that read them back: 601 rows of 2 heads of 128 4.6 + 6.3 us; with 8 heads of queries turned 787 rows 8.4 + 6.6, 2048 11.6 + 7.1; now 11.2 and 13.7, the queries in the same launch.)
-template <int NTK, int NTV, bool SIDE>
+// TURN: something is turned, or normed with a weight.  Without it (keys that are normed at most) the angles' and the turns' code is not there: steps of a few rows walk through the kernel's code once,
+// and 17 KB of it take 8.1 us for 19 rows of 2 heads of 128, 32 KB with both 9.9 (two launches, as above, 3.3 + 5.4 and the gap between them).
+template <int NTK, int NTV, bool TURN, bool SIDE>
 __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, FreshKV F, int blocks, std::conditional_t<SIDE, SideArgs, int> side)
 {
     constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK, KROW = DK + 4, VI = (4 * DV + 255) / 256;
@@ -844,7 +849,7 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, F
     extern __shared__ __attribute__((aligned(16))) float part_lds[];          // [32][KROW], [32][rot_dims]
     float *rows = part_lds, *cs = part_lds + WT_K * KROW;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = P.dim, dv = P.vdim, half = F.rot_dims / 2;
-    if constexpr (!SIDE)
+    if constexpr (TURN)
         if (id >= 2 * P.kv_heads * blocks) {          // queries, a row a wave
             const int t = 4 * (id - 2 * P.kv_heads * blocks) + wave;
             if (t < F.q_rows) turn_row(F.q + (size_t)t * P.ldq, P.heads, dk, F.q_norm_w, F.eps, F.rot_dims, F.freq, cs + wave * F.rot_dims, lane, [&]() {
@@ -881,18 +886,26 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, F
 #pragma unroll
             for (int e = 0; e < 2; e++) v[x][e] = row[min(lane + 64 * e, dk - 1)];
         }
-        const Turn u = turn_of(dk, F.rot_dims, F.norm_w, lane);
-        if (kb0 + WT_K > fresh0) {
-            for (int e = lane; e < KW * half; e += 64) { const int key = KW * wave + e / half; angle_of(kb0 + key, F.freq, e % half, half, cs + key * F.rot_dims); }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");          // (the wave's own)
+        Turn u;
+        if constexpr (TURN) {
+            u = turn_of(dk, F.rot_dims, F.norm_w, lane);
+            if (kb0 + WT_K > fresh0) {
+                for (int e = lane; e < KW * half; e += 64) { const int key = KW * wave + e / half; angle_of(kb0 + key, F.freq, e % half, half, cs + key * F.rot_dims); }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");          // (the wave's own)
+            }
         }
 #pragma unroll
         for (int x = 0; x < KW; x++) {
             const int key = KW * wave + x, j = kb0 + key;
             if (min(j, last) >= fresh0) {          // (beyond the last: turned by another angle, masked like the row again)
-                float cv[2], sv[2];
-                turn_angles(cs + key * F.rot_dims, u, F.rot_dims, lane, cv, sv);
-                turn_held(v[x], u, dk, F.norm != 0, F.eps, F.rot_dims, cv, sv, lane);
+                if constexpr (TURN) {
+                    float cv[2], sv[2];
+                    turn_angles(cs + key * F.rot_dims, u, F.rot_dims, lane, cv, sv);
+                    turn_held(v[x], u, dk, F.norm != 0, F.eps, F.rot_dims, cv, sv, lane);
+                } else if (F.norm) {
+                    const float r = norm_held(v[x], dk, F.eps, lane);
+                    v[x][0] *= r; v[x][1] *= r;
+                }
             }
 #pragma unroll
             for (int e = 0; e < 2; e++) {
@@ -1508,13 +1521,16 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
                 S.chunks = (int)chunks; S.zc = (side->dv + 63) / 64; S.first = S.chunks * side->heads * S.zc; S.per = (side->dk * side->dv + 64 * WT_WAVES - 1) / (64 * WT_WAVES);
                 S.pass = S.per * side->heads * n_seqs;
             }
+            const bool turn = F.rot_dims > 0 || F.q_rows > 0 || F.norm_w;
+            IFA_REQUIRE(!side || !turn, "%s: the linear attention goes beside keys that are not turned", who);
             const unsigned part_wgs = (unsigned)(S.first + 2 * kv_heads * t.blocks + ((size_t)F.q_rows + 3) / 4), tile_wgs = (unsigned)(hx * t.groups + S.pass);
 #define IFA_WT(K, V) { const size_t smem_p = (size_t)WT_K * (32 * K + 4 + F.rot_dims) * 4; \
                        const size_t smem_t = (size_t)2 * kBlockPieces<K, V> * 16 + WT_WAVES * 64 * 4; \
                        const void *fn = vec ? (const void *)k_attn_tile<K, V, true> : (const void *)k_attn_tile<K, V, false>; \
                        IFA_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_t)); \
-                       if (side) hipLaunchKernelGGL((k_attn_parts<K, V, true>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, S); \
-                       else hipLaunchKernelGGL((k_attn_parts<K, V, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, 0); \
+                       if (side) hipLaunchKernelGGL((k_attn_parts<K, V, false, true>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, S); \
+                       else if (turn) hipLaunchKernelGGL((k_attn_parts<K, V, true, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, 0); \
+                       else hipLaunchKernelGGL((k_attn_parts<K, V, false, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, 0); \
                        if (vec) hipLaunchKernelGGL((k_attn_tile<K, V, true>), dim3(tile_wgs), dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A, hx, (int)t.groups, S); \
                        else hipLaunchKernelGGL((k_attn_tile<K, V, false>), dim3(tile_wgs), dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A, hx, (int)t.groups, S); }
 #define IFA_WTV(K) { if (NTV == 1) IFA_WT(K, 1) else if (NTV == 2) IFA_WT(K, 2) else if (NTV == 3) IFA_WT(K, 3) else IFA_WT(K, 4) }

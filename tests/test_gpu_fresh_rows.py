@@ -140,3 +140,41 @@ def test_linear_attention_in_the_windowed_attentions_launches(H, G, D, LH, dk, d
         if done.value:
             assert same(lin[1], lin[0])
             assert all(same(a, b) for a, b in zip(slots[0].mem, slots[1].mem))
+
+
+# no linear attention beside it: rows normed and as they are, heads of one, two and four 32s, portions that begin inside a block, one key block and many, kept tokens, six sequences
+@pytest.mark.parametrize("H,G,D,norm,window,keep,steps,tile_min", [
+    (8, 2, 128, 1, 200, 4, [[(19, 0, 0)], [(65, 19, 0)]], 16), (4, 4, 64, 0, 90, 0, PART, 16), (2, 1, 32, 1, 1 << 20, 0, MANY, 16), (4, 2, 96, 0, 50, 40, [[(333, 0, 0)]], 16),
+    (8, 2, 128, 1, 64, 2, [[(12, 0, 1), (2, 0, 0)]], 2)])
+def test_rows_of_windowed_attention_stored_on_the_way(H, G, D, norm, window, keep, steps, tile_min):
+    rng = np.random.default_rng(H * D + window % 97)
+    NB, k_off = 12, 8
+    v_off = k_off + MAX * G * D
+    L = capi()
+    rel, sink = devbf(bf16_round(rng.standard_normal((NB, H)))), devbf(bf16_round(rng.standard_normal(H)))
+    bucket = devi(np.minimum(np.arange(MAX), NB - 1))
+    slots = [Slots(6, v_off + MAX * G * D) for _ in range(2)]
+    for step in steps:
+        sd, rs, T, hs = tables(step)
+        ck, cv = H * D, H * D + G * D
+        N = cv + G * D
+        proj = dev32(rng.standard_normal((T, N)))
+        proj[T // 2, ck + 3], proj[T - 1, cv + D - 1] = 1e30, -1e30
+        nb = L.ifa_attention_tile_workspace_bytes(hs, len(step), H, G, D, D, window, keep)
+        ws = torch.zeros(nb // 4 + 4, dtype=torch.float32, device="cuda")
+        out = [torch.zeros((T, H * D), dtype=torch.float32, device="cuda") for _ in range(2)]
+        out16 = torch.zeros((T, H * D), dtype=torch.bfloat16, device="cuda")
+        where = [(p(s.table), Z(k_off), Z(v_off)) for s in slots]
+        ia.check(L.ifa_kv_store_f32(at(proj, ck), Z(N), at(proj, cv), Z(N), G, D, norm, F32(1e-5), p(sd), p(rs), Z(T), *where[0], None))
+        ia.check(L.ifa_attention_window_f32(p(proj), Z(N), H, G, D, 1, F32(1e-5), F32(8.0), F32(20.0), window, keep, p(rel), p(bucket), NB, p(sink), p(sd), p(rs), Z(T), *where[0], p(out[0]),
+                                            Z(H * D), hs, len(step), tile_min, p(ws), Z(nb), None)); sync()
+        ws.fill_(7.0)
+        fresh = Fresh(at(proj, ck), N, at(proj, cv), N, norm, None, 1e-5, 0, None, 0, None)
+        left, done = C.c_bool(False), C.c_bool(True)
+        ia.check(L.ifa_attention_window_to_bf16(p(proj), Z(N), H, G, D, 1, F32(1e-5), F32(8.0), F32(20.0), window, keep, p(rel), p(bucket), NB, p(sink), p(sd), p(rs), Z(T), *where[1],
+                                                p(out[1]), Z(H * D), p(out16), Z(H * D), C.byref(left), hs, len(step), tile_min, p(ws), Z(nb), C.byref(fresh), None, C.byref(done), None))
+        sync()
+        assert left.value == (T >= tile_min) and not done.value
+        got = out16.float() if left.value else out[1]
+        assert same(got, out[0].to(torch.bfloat16).float() if left.value else out[0])
+        assert all(same(a, b) for a, b in zip(slots[0].mem, slots[1].mem))
