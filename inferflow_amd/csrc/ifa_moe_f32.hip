@@ -278,9 +278,10 @@ __global__ void __launch_bounds__(256) k_moe_up_rows(const float *__restrict__ h
 // waves are in flight as with eight), their weighted partial sums reduced once (six rows of four experts of 704 columns 21.6 -> 12.4 us).
 // SHARED: the first of the rows' workgroups (one more than rows) are the shared expert's output product of all rows (k_lin_rows' sums, times sigmoid of a row's gate) into rows of their own, which
 // the norm behind adds: six rows of four experts of 704 and a shared one of 1408 to 1024 columns 13.0 + 9.8 -> 17.9 us.  (Added by the wave that has the row's sum, which reads the shared weights
-// once a row: 19.9; the shared expert's workgroups behind the others: 19.7.)
-constexpr int SH_ROWS = 8;
-__device__ __forceinline__ void shared_down(const IfaMoeShared &S, int rows, int W, int wave, int nwaves)
+// once a row: 19.9; the shared expert's workgroups behind the others: 19.7.)  A form for each number of rows (SHARED; 0: without): with eight rows in every step a model of six such layers
+// took 446 / 470 / 549 / 565 / 607 / 649 us a step of 1 / 2 / 3 / 4 / 5 / 6 rows, now 432 / 457 / 530 / 555 / 597 / 645 (two launches: 460 / 496 / 555 / 599 / 653 / 680).
+template <int SH_ROWS>
+__device__ __forceinline__ void shared_down(const IfaMoeShared &S, int W, int wave, int nwaves)
 {
     constexpr int SP = 4;          // (pieces of 512 columns asked for ahead)
     const int lane = threadIdx.x & 63;
@@ -300,7 +301,7 @@ __device__ __forceinline__ void shared_down(const IfaMoeShared &S, int rows, int
                 float4 a[SH_ROWS][2];
 #pragma unroll
                 for (int t = 0; t < SH_ROWS; t++) {
-                    const float *r = S.act + (size_t)min(t, rows - 1) * S.lda + min(k, S.ff - 8);
+                    const float *r = S.act + (size_t)t * S.lda + min(k, S.ff - 8);
                     a[t][0] = *reinterpret_cast<const float4 *>(r); a[t][1] = *reinterpret_cast<const float4 *>(r + 4);
                 }
                 if (k >= S.ff) continue;
@@ -316,18 +317,18 @@ __device__ __forceinline__ void shared_down(const IfaMoeShared &S, int rows, int
         for (int t = 0; t < SH_ROWS; t++) acc[t] = wave_sum(acc[t]);
 #pragma unroll
         for (int t = 0; t < SH_ROWS; t++)
-            if (lane == t && t < rows) S.out[(size_t)t * S.ldo + c] = acc[t] * sigmoid_f(S.gate[(size_t)t * S.ldg]);
+            if (lane == t) S.out[(size_t)t * S.ldo + c] = acc[t] * sigmoid_f(S.gate[(size_t)t * S.ldg]);
     }
 }
-template <int NK, bool SHARED>
+template <int NK, int SHARED>
 __global__ void __launch_bounds__(256) k_moe_down_rows(const float *__restrict__ h, size_t ldh, int W, int F, int experts, int top, const bf16_t *__restrict__ down,
                                                        const int *__restrict__ idx, const float *__restrict__ wgt, const float *__restrict__ act,
-                                                       int accumulate, float *__restrict__ y, size_t ldy, int vec, std::conditional_t<SHARED, IfaMoeShared, int> S)
+                                                       int accumulate, float *__restrict__ y, size_t ldy, int vec, std::conditional_t<(SHARED > 0), IfaMoeShared, int> S)
 {
     const int lane = threadIdx.x & 63, wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), nwaves = gridDim.x * (blockDim.x >> 6);
     int t = blockIdx.y;
-    if constexpr (SHARED) {
-        if (t == 0) { shared_down(S, (int)gridDim.y - 1, W, wave, nwaves); return; }
+    if constexpr (SHARED > 0) {
+        if (t == 0) { shared_down<SHARED>(S, W, wave, nwaves); return; }
         t--;
     }
     for (int c = wave; c < W; c += nwaves) {
@@ -701,8 +702,12 @@ static int moe_experts(const char *who, int gated, int glu_kind, float limit, co
         const dim3 grid(std::min(1024u, ifa_cdiv((size_t)width, 4)), (unsigned)rows + (shared ? 1u : 0u));
 #define IFA_DOWN(NK, SH, S) hipLaunchKernelGGL((k_moe_down_rows<NK, SH>), grid, dim3(256), 0, s, h, ldh, width, ff, experts, top, (const bf16_t *)down_bf16, idx_dev, (const float *)wgt_f32, \
                                                actb, accumulate ? 1 : 0, (float *)y_f32, ldy, vec_d, S)
-        if (top <= 4) { if (shared) IFA_DOWN(4, true, *shared); else IFA_DOWN(4, false, 0); }
-        else { if (shared) IFA_DOWN(8, true, *shared); else IFA_DOWN(8, false, 0); }
+#define IFA_DOWN_SH(NK) switch (shared ? (int)rows : 0) { \
+            case 0: IFA_DOWN(NK, 0, 0); break; case 1: IFA_DOWN(NK, 1, *shared); break; case 2: IFA_DOWN(NK, 2, *shared); break; case 3: IFA_DOWN(NK, 3, *shared); break; \
+            case 4: IFA_DOWN(NK, 4, *shared); break; case 5: IFA_DOWN(NK, 5, *shared); break; case 6: IFA_DOWN(NK, 6, *shared); break; case 7: IFA_DOWN(NK, 7, *shared); break; \
+            default: IFA_DOWN(NK, 8, *shared); }
+        if (top <= 4) IFA_DOWN_SH(4) else IFA_DOWN_SH(8)
+#undef IFA_DOWN_SH
 #undef IFA_DOWN
         IFA_LAUNCH_CHECK();
         return IFA_OK;

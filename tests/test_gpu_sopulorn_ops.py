@@ -293,7 +293,8 @@ def test_embedding_rows_in_pieces_of_four_columns_and_one_by_one(W):
         assert int(slots.mem[0].view(torch.int32)[4]) == 7 and int(slots.mem[1].view(torch.int32)[4]) == 12
 
 
-@pytest.mark.parametrize("T,W,F,SF,E,top", [(1, 64, 24, 8, 6, 2), (6, 128, 64, 1408, 16, 4), (8, 40, 10, 520, 3, 3), (5, 14, 6, 2048, 70, 8), (7, 64, 16, 2056, 16, 9), (2, 16, 8, 4104, 1, 1)])
+@pytest.mark.parametrize("T,W,F,SF,E,top", [(1, 64, 24, 8, 6, 2), (6, 128, 64, 1408, 16, 4), (8, 40, 10, 520, 3, 3), (5, 14, 6, 2048, 70, 8), (7, 64, 16, 2056, 16, 9), (2, 16, 8, 4104, 1, 1), (3, 24, 16, 1032, 5, 3), (4, 36, 8, 72, 12, 6),
+                                                (1, 20, 8, 520, 9, 7)])
 def test_shared_expert_in_the_experts_last_launch_leaves_the_bits_of_its_own(T, W, F, SF, E, top):
     """the output product beside the sum over the experts, in one launch and in two: pieces of 512 columns whole and ragged, more of them than are asked for ahead, rows of activations, gates and
     outputs with strides; the experts' rows onto what is there and in its place; and the norm behind both, which adds them up"""
