@@ -787,7 +787,8 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
         const IfaMoeShared shared = {(const bf16_t *)L.T(IFA_LT_X_SH_DOWN).data, n->m3, SFP, (int)SFP, n->proj + L.c2_sg, N2, n->m1, W};
         // (its activations are there; its rows go beside the experts', added up by the norm behind them, which takes such rows)
         const bool with_shared = !choose && SFP > 0 && left == GLU_32 && n->mix_max >= W && W % 4 == 0 && W <= 8192
-                                 && (((uintptr_t)L.T(IFA_LT_NORM2B).data | (uintptr_t)next_norm) & 7) == 0 && ifa_moe_shared_fits(shared);
+                                 && (((uintptr_t)L.T(IFA_LT_NORM2B).data | (uintptr_t)next_norm) & 7) == 0 && ifa_moe_shared_fits(shared)
+                                 && ifa_moe_shared_pays(T, W, SFP);
         if (choose && (rc = ifa_moe_route_top_f32(n->proj + L.c2_router, N2, T, sp.x_experts, sp.x_top, nullptr, n->moe_idx, n->moe_wgt, s))) return rc;
         rc = !choose ? ifa_moe_experts_gated_top_rows_shared(n->proj + L.c2_router, N2, n->h, W, T, (int)W, sp.x_ff, sp.x_experts, sp.x_top, L.T(IFA_LT_X_UP).data, L.T(IFA_LT_X_DOWN).data,
                                                       n->moe_idx, n->moe_wgt, n->moe_ws, n->moe_ws_bytes, n->m2, W, 0, with_shared ? &shared : nullptr, s)

@@ -804,6 +804,11 @@ int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const voi
                                                  nullptr, stream);
 }
 
+// A wave of the shared expert's workgroups reads all rows' activations for one output: with many weights and three rows and more the launch of its own, which has two outputs a wave there, is the
+// faster one.  One launch / two, 2 to 8 rows, two of eight experts: 6144 x 4096 0.96 to 1.00, 4096 x 8192 and 8192 x 4096 0.95 to 1.04 (from four rows on 0.97 to 1.04), 8192 x 8192 0.99 for two
+// rows and 1.06 to 1.13 for more; 16.8 M weights and less 0.70 to 0.97.
+bool ifa_moe_shared_pays(size_t rows, size_t width, size_t ff) { return rows <= 2 || width * ff <= (size_t)24 << 20; }
+
 bool ifa_moe_shared_fits(const IfaMoeShared &S)
 {
     return S.ff >= 8 && S.ff % 8 == 0 && S.lda >= (size_t)S.ff && S.lda % 4 == 0 && (((uintptr_t)S.down | (uintptr_t)S.act) & 15) == 0;

@@ -81,3 +81,11 @@ def test_errors_are_codes_not_exceptions():
     assert b"null" in L.ifa_last_error()
     assert L.ifa_gemv(dt.F32, 1, 1, 32, dt.F16, 1, None, 1, None) == -1
     assert L.ifa_device_count() >= 0
+
+
+def test_shared_expert_goes_beside_the_experts_where_one_launch_is_no_slower():
+    import ctypes as C
+    pays = ia.lib().ifa_moe_shared_pays
+    pays.restype, pays.argtypes = C.c_bool, [C.c_size_t] * 3
+    assert all(pays(t, 1024, 1408) and pays(t, 6144, 4096) for t in range(1, 9))
+    assert pays(2, 8192, 8192) and not any(pays(t, 8192, 8192) or pays(t, 4096, 8192) for t in range(3, 9))
