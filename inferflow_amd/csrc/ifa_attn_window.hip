@@ -628,6 +628,12 @@ __device__ __forceinline__ FewSeq few_of(const TileArgs &A, int id, At at)
 // beside the tiles, the chunks' outputs beside the shares.  Alone, each of them left most of the chip idle: 601 rows of width 1024 (8 heads, 2 of keys) 4.6 + 6.3 + 15.2, 29.4 + 4.9 and
 // 9.2 + 12 us, together 16.0, 29.2 and 13.3; 2048 rows of width 2048 (16 heads, 4) 6.6 + 9.0 + 32, 140 + 10.6
 // and 13.4 + 27.4, together 42.7, 140.6 and 38.3
+// At most SIDE_SEQS sequences: a chunk's workgroup finds its sequence by going through them, and has more others beside it to hide that in launches of its own; and the states beside the tiles up
+// to SIDE_PASS workgroups, each of which takes a tile's place on its compute unit (100 KB of LDS), in a launch of their own beyond.  A model's prompts, us, with the launches of its own / shared /
+// shared but for the states, n sequences of up to l tokens: width 1024, 128 such workgroups a sequence: 16 x 300 1884 / 1808 / 1813, 24 x 200 2263 / 2218 / 2202, 32 x 130 2185 / 2176 / 2129,
+// 32 x 400 4418 / 4461 / 4385, 64 x 130 3632 / 3898 / 3641, 64 x 200 4707 / 4991 / 4752, 128 x 150 7578 / 8711 / 7958; width 2048, 256 a sequence: 1 x 2048 4372 / 4265 / 4328, 16 x 200
+// 3144 / 3170 / 3127, 32 x 200 6075 / 6245 / 6059
+constexpr int SIDE_SEQS = 32, SIDE_PASS = 2048;
 struct SideArgs { ifachunk::ChunkArgs c; int chunks, zc, first, pass, per; };          // zc: pieces of 64 value columns; workgroups of the first and third launch, of the second (per: a head's)
 
 // The item (of n) that a number running over all items' counts falls into, or -1; id becomes the number inside it.  A wave looks at 64 items at a time (walked by one thread,
@@ -1513,13 +1519,15 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
             }
             SideArgs S;
             memset(&S, 0, sizeof(S));
+            if (n_seqs > SIDE_SEQS) side = nullptr;          // (*side_done stays false)
             if (side) {
                 size_t chunks = 0;
                 const int rc = ifa_chunk_args(&S.c, &chunks, 0, side->q, side->ldq, side->k, side->ldk, side->v, side->ldv, side->heads, side->heads, side->dk, side->dv, side->decay, nullptr,
                                               nullptr, seqs_dev, seqs_host, n_seqs, slot_base_dev, side->state_off, side->ws, side->ws_bytes, side->out, side->ldo);
                 if (rc) return rc;
                 S.chunks = (int)chunks; S.zc = (side->dv + 63) / 64; S.first = S.chunks * side->heads * S.zc; S.per = (side->dk * side->dv + 64 * WT_WAVES - 1) / (64 * WT_WAVES);
-                S.pass = S.per * side->heads * n_seqs;
+                const size_t pass = (size_t)S.per * side->heads * n_seqs;
+                S.pass = pass <= SIDE_PASS ? (int)pass : 0;
             }
             const bool turn = F.rot_dims > 0 || F.q_rows > 0 || F.norm_w;
             IFA_REQUIRE(!side || !turn, "%s: the linear attention goes beside keys that are not turned", who);
@@ -1531,6 +1539,7 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
                        if (side) hipLaunchKernelGGL((k_attn_parts<K, V, false, true>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, S); \
                        else if (turn) hipLaunchKernelGGL((k_attn_parts<K, V, true, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, 0); \
                        else hipLaunchKernelGGL((k_attn_parts<K, V, false, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, 0); \
+                       if (side && !S.pass) ifa_linear_pass(S.c, stream); \
                        if (vec) hipLaunchKernelGGL((k_attn_tile<K, V, true>), dim3(tile_wgs), dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A, hx, (int)t.groups, S); \
                        else hipLaunchKernelGGL((k_attn_tile<K, V, false>), dim3(tile_wgs), dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A, hx, (int)t.groups, S); }
 #define IFA_WTV(K) { if (NTV == 1) IFA_WT(K, 1) else if (NTV == 2) IFA_WT(K, 2) else if (NTV == 3) IFA_WT(K, 3) else IFA_WT(K, 4) }

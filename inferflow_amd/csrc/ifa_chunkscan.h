@@ -235,3 +235,5 @@ __device__ __forceinline__ void chunk_out(const ChunkArgs &A, int id, int h, int
 int ifa_chunk_args(ifachunk::ChunkArgs *out, size_t *n_chunks, int kind, const void *q_f32, size_t ldq, const void *k_f32, size_t ldk, const void *v_f32, size_t ldv, int heads, int qk_heads,
                    int dk, int dv, const void *decay_head_f32, const void *decay_row_f32, const void *beta_row_f32, const void *seqs_dev, const void *seqs_host, int n_seqs,
                    void *const *slot_base_dev, size_t state_off, void *ws, size_t ws_bytes, void *out_f32, size_t ldo);
+// the second launch of kind 0 by itself
+void ifa_linear_pass(const ifachunk::ChunkArgs &A, ifa_stream stream);

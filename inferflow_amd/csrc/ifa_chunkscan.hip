@@ -255,7 +255,7 @@ int ifa_state_chunked_f32(int kind, const void *q_f32, size_t ldq, const void *k
     const dim3 per_chunk((unsigned)chunks, (unsigned)heads, ifa_cdiv((size_t)dv, 64));
     if (kind == 0) {
         hipLaunchKernelGGL(k_linear_chunk, per_chunk, dim3(256), 0, s, A);
-        hipLaunchKernelGGL(k_linear_pass, dim3(ifa_cdiv((size_t)dk * dv, 256), (unsigned)heads, (unsigned)n_seqs), dim3(256), 0, s, A);
+        ifa_linear_pass(A, stream);
         const bool vec = ldv % 4 == 0 && ((uintptr_t)v_f32 & 15) == 0;
         if (dk == 64) { if (vec) hipLaunchKernelGGL((k_chunk_out<0, 64, true>), per_chunk, dim3(256), 0, s, A); else hipLaunchKernelGGL((k_chunk_out<0, 64, false>), per_chunk, dim3(256), 0, s, A); }
         else { if (vec) hipLaunchKernelGGL((k_chunk_out<0, 128, true>), per_chunk, dim3(256), 0, s, A); else hipLaunchKernelGGL((k_chunk_out<0, 128, false>), per_chunk, dim3(256), 0, s, A); }
@@ -270,6 +270,11 @@ int ifa_state_chunked_f32(int kind, const void *q_f32, size_t ldq, const void *k
 }
 
 } // extern "C"
+
+void ifa_linear_pass(const ChunkArgs &A, ifa_stream stream)
+{
+    hipLaunchKernelGGL(k_linear_pass, dim3(ifa_cdiv((size_t)A.dk * A.dv, 256), (unsigned)A.heads, (unsigned)A.n_seqs), dim3(256), 0, ifa_s(stream), A);
+}
 
 int ifa_chunk_args(ChunkArgs *args, size_t *n_chunks, int kind, const void *q_f32, size_t ldq, const void *k_f32, size_t ldk, const void *v_f32, size_t ldv, int heads, int qk_heads,
                    int dk, int dv, const void *decay_head_f32, const void *decay_row_f32, const void *beta_row_f32, const void *seqs_dev, const void *seqs_host, int n_seqs,

@@ -178,3 +178,53 @@ def test_rows_of_windowed_attention_stored_on_the_way(H, G, D, norm, window, kee
         got = out16.float() if left.value else out[1]
         assert same(got, out[0].to(torch.bfloat16).float() if left.value else out[0])
         assert all(same(a, b) for a, b in zip(slots[0].mem, slots[1].mem))
+
+
+# as many sequences as go beside the attention, one more, and so many heads and columns that the states are handed on in a launch of their own (more than 2048 workgroups of 512)
+@pytest.mark.parametrize("LH,dk,dv,n,beside", [(2, 64, 64, 32, True), (2, 64, 64, 33, False), (8, 128, 96, 10, True), (8, 128, 96, 11, True), (9, 128, 128, 32, True)])
+def test_linear_attention_of_many_sequences(LH, dk, dv, n, beside):
+    H, G, D, NB, k_off, most = 4, 2, 64, 12, 8, 160
+    rng = np.random.default_rng(LH * n + dv)
+    v_off = k_off + most * G * D
+    s_off = v_off + most * G * D
+    L = capi()
+    rel, sink = devbf(bf16_round(rng.standard_normal((NB, H)))), devbf(bf16_round(rng.standard_normal(H)))
+    bucket = devi(np.minimum(np.arange(most), NB - 1))
+    decay = dev32(rng.uniform(0.9, 1.0, LH))
+    slots = [Slots(n, s_off + LH * dk * dv) for _ in range(2)]
+    lens = [int(k) for k in rng.integers(1, 80, n)]
+    for behind in (0, 1):          # (a prompt each, then a portion behind it)
+        seqs = [(k, behind * k, q) for q, k in enumerate(lens)]
+        sd, rs, T, hs = tables(seqs)
+        ck = H * D
+        lq = ck + G * D
+        lk, lv = lq + LH * dk, lq + 2 * LH * dk
+        N = lv + LH * dv
+        proj = dev32(rng.standard_normal((T, N)))
+        nb = L.ifa_attention_tile_workspace_bytes(hs, n, H, G, D, D, 50, 3)
+        ws = torch.full((nb // 4 + 4,), 7.0, dtype=torch.float32, device="cuda")
+        sb = L.ifa_state_chunked_workspace_bytes(0, Z(sum((k + 63) // 64 for k, _, _ in seqs)), LH, dk, dv)
+        sws = torch.full((sb // 4 + 4,), 7.0, dtype=torch.float32, device="cuda")
+        out = [torch.zeros((T, H * D), dtype=torch.float32, device="cuda") for _ in range(2)]
+        lin = [torch.zeros((T, LH * dv), dtype=torch.float32, device="cuda") for _ in range(2)]
+        out16 = torch.zeros((T, H * D), dtype=torch.bfloat16, device="cuda")
+        where = [(p(s.table), Z(k_off), Z(v_off)) for s in slots]
+
+        def alone(i):
+            ia.check(L.ifa_state_chunked_f32(0, at(proj, lq), Z(N), at(proj, lk), Z(N), at(proj, lv), Z(N), LH, LH, dk, dv, p(decay), None, None, p(sd), hs, n, p(slots[i].table), Z(s_off),
+                                             p(sws), Z(sb), p(lin[i]), Z(LH * dv), None))
+        ia.check(L.ifa_kv_store_f32(at(proj, ck), Z(N), at(proj, ck), Z(N), G, D, 1, F32(1e-5), p(sd), p(rs), Z(T), *where[0], None))
+        ia.check(L.ifa_attention_window_f32(p(proj), Z(N), H, G, D, 1, F32(1e-5), F32(8.0), F32(20.0), 50, 3, p(rel), p(bucket), NB, p(sink), p(sd), p(rs), Z(T), *where[0], p(out[0]),
+                                            Z(H * D), hs, n, 16, p(ws), Z(nb), None))
+        alone(0); sync()
+        fresh = Fresh(at(proj, ck), N, at(proj, ck), N, 1, None, 1e-5, 0, None, 0, None)
+        side = Side(at(proj, lq), at(proj, lk), at(proj, lv), N, N, N, LH, dk, dv, decay.data_ptr(), s_off, sws.data_ptr(), sb, lin[1].data_ptr(), LH * dv)
+        left, done = C.c_bool(False), C.c_bool(not beside)
+        ia.check(L.ifa_attention_window_to_bf16(p(proj), Z(N), H, G, D, 1, F32(1e-5), F32(8.0), F32(20.0), 50, 3, p(rel), p(bucket), NB, p(sink), p(sd), p(rs), Z(T), *where[1],
+                                                p(out[1]), Z(H * D), p(out16), Z(H * D), C.byref(left), hs, n, 16, p(ws), Z(nb), C.byref(fresh), C.byref(side), C.byref(done), None))
+        if not done.value:
+            alone(1)
+        sync()
+        assert done.value == beside and left.value
+        assert same(out16.float(), out[0].to(torch.bfloat16).float()) and same(lin[0], lin[1])
+        assert all(same(a, b) for a, b in zip(slots[0].mem, slots[1].mem))
