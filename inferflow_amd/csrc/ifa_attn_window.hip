@@ -610,7 +610,9 @@ __host__ __device__ __forceinline__ TileBlocks tile_blocks(int p0, int nq, int w
 
 // marks, shares: where the blocks' marks and the chunks' partial results begin in the workspace (floats), behind the operands
 // few: a step's sequences, where there are up to FEW, and the chunks of those behind, the tiles and the operand blocks of those in front of each: tables in memory, each behind the other, were a
-// microsecond a trip in front of everything else
+// microsecond a trip in front of everything else.  Four: every further one is 28 bytes of arguments and a choice in front of each place, in three launches a layer.  With eight, steps of five to
+// eight sequences are 0.2 to 1 % of a whole prompt faster (Sopulorn of width 1024, 5 x 400 tokens 1326 -> 1317 us, 8 x 200 1208 -> 1198) and steps of one to four, the most frequent ones, 0.3 to
+// 1.3 % slower (1 x 16 770 -> 780, 1 x 601 1112 -> 1118, 3 x 411 1152 -> 1160); with sixteen everything is 1 to 2 % slower (Gelarax 1 x 601 1052 -> 1067, Sopulorn 16 x 100 1095 -> 1115)
 constexpr int FEW = 4;
 struct FewSeq { SeqDesc sd; int chunk0, tile0, block0; };
 struct TileArgs { int n_seqs, hpw, cb, tiles; size_t marks, shares; int n_few; FewSeq few[FEW]; };

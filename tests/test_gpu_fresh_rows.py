@@ -44,13 +44,15 @@ def same(a, b):
 
 MAX = 700
 ONE, PART, MANY = [[(70, 0, 0)], [(45, 70, 0)]], [[(33, 0, 1), (17, 0, 0), (40, 0, 2)], [(21, 40, 2), (64, 33, 1), (18, 17, 0)]], [[(20 + q, 0, q) for q in range(6)]]
+FOUR, FIVE = [[(9 + 15 * q, 0, q) for q in range(4)], [(33 - q, 9 + 15 * q, q) for q in range(4)]], [[(40 - 3 * q, 0, q) for q in range(5)]]          # (as many as a launch's arguments hold, one more)
 
 
 # heads a workgroup shares (1, 2, 4) and more of them than a wave turns at once, heads of whole and of ragged 32s, values of their own size, nothing / a part / all of a head turned, windows
 # behind kept tokens, up to four sequences and more, portions that begin inside a block, long enough for several chunks; the last: fewer rows than the tiled form takes
 @pytest.mark.parametrize("H,G,D,DV,rot,window,keep,steps,tile_min", [
     (8, 2, 128, 128, 64, 0, 0, ONE, 16), (4, 1, 128, 64, 128, 0, 0, PART, 16), (12, 3, 64, 96, 32, 40, 5, PART, 16), (6, 3, 96, 32, 0, 33, 70, ONE, 16), (5, 5, 40, 48, 10, 0, 0, PART, 16),
-    (20, 5, 32, 128, 32, 0, 0, MANY, 16), (2, 2, 128, 128, 126, 100, 40, [[(650, 0, 0)]], 16), (8, 2, 72, 100, 64, 0, 0, [[(9, 0, 0)], [(6, 9, 0)]], 16), (3, 1, 30, 33, 30, 0, 0, PART, 16)])
+    (20, 5, 32, 128, 32, 0, 0, MANY, 16), (2, 2, 128, 128, 126, 100, 40, [[(650, 0, 0)]], 16), (8, 2, 72, 100, 64, 0, 0, [[(9, 0, 0)], [(6, 9, 0)]], 16), (3, 1, 30, 33, 30, 0, 0, PART, 16),
+    (4, 2, 64, 64, 32, 45, 3, FOUR, 16), (4, 2, 64, 64, 32, 45, 3, FIVE, 16)])
 @pytest.mark.parametrize("own", [True, False])
 def test_rows_of_rotated_attention_stored_on_the_way(H, G, D, DV, rot, window, keep, steps, tile_min, own):
     rng = np.random.default_rng(H * D + rot)
@@ -94,7 +96,8 @@ def test_rows_of_rotated_attention_stored_on_the_way(H, G, D, DV, rot, window, k
 # the linear attention's keys of 64 and 128, value columns that are no multiple of 64, rows of v off 16 bytes, one chunk of keys a tile (no shares to join) and several
 @pytest.mark.parametrize("H,G,D,LH,dk,dv,pad,window,keep,steps,tile_min", [
     (8, 2, 128, 8, 64, 128, 0, 200, 4, [[(601, 0, 0)], [(65, 601, 0)]], 16), (4, 4, 64, 3, 128, 96, 1, 90, 0, PART, 16), (2, 1, 32, 2, 64, 32, 0, 1 << 20, 0, MANY, 16),
-    (4, 2, 96, 2, 64, 64, 0, 50, 0, [[(40, 0, 0)]], 64), (16, 4, 128, 16, 64, 128, 0, 128, 2, [[(130, 0, 3), (64, 0, 1)]], 16)])
+    (4, 2, 96, 2, 64, 64, 0, 50, 0, [[(40, 0, 0)]], 64), (16, 4, 128, 16, 64, 128, 0, 128, 2, [[(130, 0, 3), (64, 0, 1)]], 16),
+    (4, 2, 64, 2, 64, 64, 0, 45, 3, FOUR, 16), (4, 2, 64, 2, 64, 64, 0, 45, 3, FIVE, 16)])
 def test_linear_attention_in_the_windowed_attentions_launches(H, G, D, LH, dk, dv, pad, window, keep, steps, tile_min):
     rng = np.random.default_rng(H * D + dv)
     NB, k_off = 12, 8
