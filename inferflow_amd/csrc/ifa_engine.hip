@@ -669,6 +669,7 @@ int ifa_model_get_buffer(ifa_model *m, const char *name, int layer, void **dptr,
     else if (!strcmp(name, "x2")) { p = m->x2; b = (size_t)c.dim * 2; }
     else if (!strcmp(name, "dqkv")) { p = m->dqkv; b = ((size_t)c.heads + 2 * (size_t)c.kv_heads) * c.head_dim * 2; }
     else if (!strcmp(name, "att")) { p = m->att; b = (size_t)c.heads * c.head_dim * 2; }
+    else if (!strcmp(name, "q")) { p = m->q; b = (size_t)m->scratch_tokens * c.heads * c.head_dim * 2; }          // (the last layer's of a prompt: turned in place, or not by the launch that turns them itself)
     else if (!strcmp(name, "attq")) { p = m->attq; b = m->attq ? xq_image_bytes(c.heads * c.head_dim) : 0; }
     else if (!strcmp(name, "a")) { p = m->a; b = (size_t)c.dim * 2; }
     else if (!strcmp(name, "t1")) { p = m->t1; b = (size_t)c.ffn * 2; }

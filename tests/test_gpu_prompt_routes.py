@@ -288,15 +288,65 @@ def test_batched_steps_of_many_queries_agree_with_the_rows_products_and_replay(k
 @pytest.mark.parametrize("T", [4, 8, 9, 31, 32, 33, 62, 63])
 @pytest.mark.parametrize("order,shape", [(2, {}), (1, dict(kv_heads=8)), (2, dict(dim=1024, heads=8, kv_heads=2, head_dim=128, ffn=1408))], ids=["7b", "pairs_kv8", "w1024_kv2"])
 def test_rotation_and_attention_of_short_prompts_in_one_launch_leave_the_bits_of_two(order, shape, T):
-    """one tile of queries and two, whole and ragged; heads that share keys; both ways of pairing: every row's logits and the last layer's cache rows"""
-    wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=96, layers=2, vocab=600, rope_order=order, **shape)
+    """one tile of queries and two, whole and ragged; heads that share keys; both ways of pairing: every row's logits and the last layer's cache rows.  The one launch leaves the step's query rows
+    as they came, the two turn them in place (but the first one): which of them ran"""
+    wk, _, s = synth.build("llama2_7b", dt.Q4_B32T1A, dt.F16, max_ctx=96, layers=2, vocab=600, quant_threshold=0, rope_order=order, **shape)
     toks = np.random.default_rng(T).integers(3, 600, T).astype(np.int32)
-    out = []
+    out, qs = [], []
     for on in (1, 0):
         wk.set_option("attn_fresh", on)
         tok, lg = _rows(wk, toks, 600)
         out.append((tok, lg) + tuple(np.array(wk.read_buffer(n, 1, nbytes=96 * s["kv_heads"] * s["head_dim"] * 2)) for n in ("kcache", "vcache")))
+        qs.append(np.array(wk.read_buffer("q", nbytes=T * s["heads"] * s["head_dim"] * 2)).reshape(T, -1))
     wk.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+    assert np.array_equal(qs[0][0], qs[1][0]) and (qs[0][1:] != qs[1][1:]).any(axis=1).all()
     assert out[0][2].any() and np.isfinite(out[0][1]).all()
+
+
+@pytest.mark.parametrize("T,H,G,order,extra", [(4, 2, 2, 2, 0), (31, 4, 1, 1, 8), (32, 6, 2, 2, 0), (33, 3, 3, 1, 0), (63, 4, 2, 2, 16)])
+def test_rotation_cache_rows_and_attention_of_one_launch_against_64_bits(T, H, G, order, extra):
+    """Queries, keys and values of order 1.  Turned halfs are off by 2^-11 of their size, so a score by about 2^-11 sqrt 2 of its size (at most 6 here), its own rounding 2^-9 at most; a weight by
+    as much of itself, its rounding 2^-11; so rows of values up to 4.5: 4.5 (2^-8 + 2^-9 + 2^-11) < 0.03.  Keys in the cache: 2^-11 of values up to 6.5.  Values: the same bits."""
+    L, D = g.capi(), 128
+    rng = np.random.default_rng(T)
+    q, k, v = (torch.from_numpy(rng.standard_normal((T, n, D)).astype(np.float16)).cuda() for n in (H, G, G))
+    keep = [t.clone() for t in (q, k, v)]
+    a = np.arange(T)[:, None] * 10000.0 ** (-np.arange(D // 2) / (D // 2))
+    tab = torch.from_numpy(np.stack([np.cos(a), np.sin(a)], -1).astype(np.float32)).cuda()
+    row = G * D + extra
+    kc, vc = (torch.full((T + 2, row), 7.0, dtype=torch.float16, device="cuda") for _ in range(2))
+    out = torch.full((T + 1, H, D), 7.0, dtype=torch.float16, device="cuda")
+    f = L.ifa_attention_fresh
+    f.argtypes = [g.C.c_void_p] * 4 + [g.C.c_int] * 4 + [g.C.c_float, g.C.c_int, g.C.c_float] + [g.C.c_void_p] * 2 + [g.C.c_size_t] + [g.C.c_void_p] * 2
+
+    def call(tokens=T, heads=H, dim=D, turn=order, part=1.0, kcache=kc, stride=row):
+        return f(g.p(q), g.p(k), g.p(v), g.p(tab), tokens, heads, G, dim, 1.0, turn, part, g.p(kcache), g.p(vc), stride, g.p(out), None)
+    # what it leaves to other launches: too few rows and too many, other heads, no turn and a part of one, rows of the cache off 16 bytes (2: IFA_ERR_STATE); nothing is written
+    declined = [call(tokens=3), call(tokens=64), call(dim=64), call(turn=0), call(part=0.5), call(stride=row + 4), call(kcache=kc.reshape(-1)[4:])]
+    g.sync()
+    assert len(set(declined)) == 1 and declined[0] != 0 and all(bool((t == 7.0).all()) for t in (kc, vc, out))
+    assert call() == 0
+    g.sync()
+    assert all(torch.equal(x, y) for x, y in zip((q, k, v), keep))
+
+    def turned(z):
+        z = g.host(z).astype(np.float64)
+        lo, hi = (z[..., :D // 2], z[..., D // 2:]) if order == 2 else (z[..., 0::2], z[..., 1::2])
+        c, s = np.cos(a)[:, None, :], np.sin(a)[:, None, :]
+        x, y = lo * c - hi * s, lo * s + hi * c
+        return np.concatenate([x, y], -1) if order == 2 else np.stack([x, y], -1).reshape(z.shape)
+    qt, kt, vf = turned(q), turned(k), g.host(v).astype(np.float64)
+    kgot, vgot = g.host(kc), g.host(vc)
+    assert np.abs(kgot[:T, :G * D].reshape(T, G, D) - kt).max() < 2.0 ** -11 * 6.5
+    assert np.array_equal(vgot[:T, :G * D].reshape(T, G, D), g.host(v))
+    assert (kgot[T:] == 7.0).all() and (vgot[T:] == 7.0).all() and (kgot[:, G * D:] == 7.0).all() and (vgot[:, G * D:] == 7.0).all()
+    got = g.host(out)
+    assert (got[T] == 7.0).all()
+    for h in range(H):
+        s = qt[:, h] @ kt[:, h // (H // G)].T / np.sqrt(D)
+        assert np.abs(s).max() < 6
+        e = np.where(np.tril(np.ones((T, T), bool)), np.exp(s - s.max(1, keepdims=True)), 0.0)
+        want = e / e.sum(1, keepdims=True) @ vf[:, h // (H // G)]
+        assert np.abs(got[:T, h] - want).max() < 0.03, (h, np.abs(got[:T, h] - want).max())
