@@ -1,5 +1,5 @@
 """The mixture of experts of a prompt as run_sandwich_layer runs it -- choice and counts, places of the pairs beside the shared expert's activations, grouped products, the sum of a row's pairs
-inside the norm behind them -- against the launches of their own (ifa_moe_route_top_f32, ifa_moe_experts_gated_bf16, ifa_glu_to_bf16's form, ifa_norm_add_norm_f32), bit for bit: the same
+inside the norm behind them -- against the launches of their own (ifa_moe_route_top_f32, ifa_moe_experts_gated_f32 over the same rows, ifa_norm_add_norm_f32 and its bfloat16 form), bit for bit: the same
 products and the same sums in the same order."""
 import ctypes as C
 
@@ -21,9 +21,10 @@ class Prompt(C.Structure):          # IfaMoePrompt (csrc/ifa_rows_fused.h)
                 ("sh_gate_up", C.c_void_p), ("sh_ld", C.c_size_t), ("sh_ff", C.c_int), ("sh_gate", C.c_void_p), ("sh_ldg", C.c_size_t), ("sh_act", C.c_void_p), ("sh_ldo", C.c_size_t)]
 
 
-# rows of one block and of several (16 rows, and 32 of them from 4097 rows on), row tiles of 64 and 128, one expert, experts around a wave's and the ballots' widths, the most there may be
+# rows of one block and of several (16 rows, and 32 of them from 4097 rows on), row tiles of 64 and 128, one expert, experts around a wave's and the ballots' widths, the most there may be, rows of one and of two pieces a thread of the norm
 @pytest.mark.parametrize("T,W,F,E,top,SF", [(9, 448, 64, 5, 2, 64), (17, 448, 64, 16, 4, 72), (16, 512, 64, 1, 1, 0), (300, 448, 72, 16, 4, 100), (257, 448, 64, 64, 3, 66), (70, 448, 64, 65, 8, 64),
-                                            (40, 448, 64, 512, 9, 0), (4099, 448, 64, 7, 2, 64), (1100, 512, 64, 3, 3, 128), (4500, 1024, 64, 16, 4, 0)])
+                                            (40, 448, 64, 512, 9, 0), (4099, 448, 64, 7, 2, 64), (1100, 512, 64, 3, 3, 128), (4500, 1024, 64, 16, 4, 0),
+                                            (20, 4096, 64, 5, 2, 64), (20, 4160, 64, 5, 2, 64), (12, 8192, 64, 3, 2, 0)])
 def test_experts_of_a_prompt_against_their_launches_one_by_one(T, W, F, E, top, SF):
     rng = np.random.default_rng(T + E)
     g = torch.Generator(device="cuda"); g.manual_seed(T + E)
@@ -39,7 +40,7 @@ def test_experts_of_a_prompt_against_their_launches_one_by_one(T, W, F, E, top, 
     gu = (torch.randn((E * 2 * F, W), generator=g, device="cuda") * W ** -0.5).to(torch.bfloat16)
     dn = (torch.randn((E * W, F), generator=g, device="cuda") * F ** -0.5).to(torch.bfloat16)
     wa, wb = (devbf(bf16_round(rng.standard_normal(W))) for _ in range(2))
-    x = torch.randn((T, W), generator=g, device="cuda"); x_w = x.clone()
+    x = torch.randn((T, W), generator=g, device="cuda"); x_w, x_16 = x.clone(), x.clone()
     m = torch.randn((T, W), generator=g, device="cuda") if SF else None
     L, Z = capi(), C.c_size_t
     nb = L.ifa_moe_workspace_bytes(T, top, W, 3 * F, E)
@@ -65,6 +66,11 @@ def test_experts_of_a_prompt_against_their_launches_one_by_one(T, W, F, E, top, 
     assert torch.equal(idx, idx_w) and np.array_equal(wgt.cpu().numpy(), wgt_w.cpu().numpy(), equal_nan=True)
     assert np.array_equal(x.cpu().numpy(), x_w.cpu().numpy(), equal_nan=True) and np.array_equal(h.cpu().numpy(), h_w.cpu().numpy(), equal_nan=True)
     assert torch.isfinite(h[7:]).all()
+    # the form that leaves bfloat16 rows, as layers' products read them: those rows rounded
+    h_16 = torch.zeros((T, W), dtype=torch.bfloat16, device="cuda")
+    ia.check(L.ifa_norm_add_norm_moe(p(x_16), Z(W), Z(T), Z(W), p(m) if SF else None, Z(W), pos, rows, top, p(wa), p(wb), C.c_float(1.0), C.c_float(1e-5), None, p(h_16), Z(W), None)); sync()
+    assert np.array_equal(x_16.cpu().numpy(), x_w.cpu().numpy(), equal_nan=True)
+    assert np.array_equal(h_16.float().cpu().numpy(), h.to(torch.bfloat16).float().cpu().numpy(), equal_nan=True)
     if SF:          # against the same sum in 64 bits: rounded once to bfloat16, 2^-9 of the value; 32-bit exponentials below that
         s = proj[:, E + 1:].double().cpu()
         want = s[:, :SF] * torch.sigmoid(s[:, :SF]) * s[:, SF:2 * SF] * torch.sigmoid(proj[:, E:E + 1].double().cpu())

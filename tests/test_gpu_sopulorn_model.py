@@ -391,6 +391,24 @@ def test_experts_over_the_rows_that_the_norm_has_left_in_bfloat16(tmp_path, T):
         assert_close(fx.rel_err(out[9], oracle_logits(cfg, w, toks)), "bfloat16", TOL16, T)
 
 
+@pytest.mark.parametrize("T", [9, 130])
+def test_experts_of_prompts_that_are_sorted_by_one_workgroup(tmp_path, T):
+    """bfloat16 rows for experts whose choice goes through launches of its own: a shared expert too narrow for bfloat16 rows, more than 512 experts; the bits of operands rounded on their way
+    (a16_min 0), and the oracle"""
+    import inferflow_amd as ia
+    cfg = fx.config([fx.attention_layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=fx.moe(experts=5, top=2, ff=200, shared=40)),
+                     fx.attention_layer(heads=2, kv_heads=1, dim=32, vdim=32, mlp=fx.moe(experts=520, top=3, ff=64, shared=72))], width=448, vocab=97)
+    w, toks, out = fx.random_weights(cfg, 37), tokens_for(cfg, T, 38), {}
+    eng = engine_for(tmp_path, cfg, w, "bfloat16", 192, 1)
+    for border in (0, 9):
+        run_whole(eng, tokens_for(cfg, 40, 39))
+        ia.check(ia.lib().ifa_model_set_option(eng.worker(), b"a16_min", border))
+        out[border] = run_whole(eng, toks)[0]
+    eng.close()
+    assert np.array_equal(out[0], out[9])
+    assert_close(fx.rel_err(out[9], oracle_logits(cfg, w, toks)), "bfloat16", TOL16, T)
+
+
 def test_generation_over_bfloat16_rows_of_single_tokens_beside_longer_and_longer_prompts(tmp_path):
     """a16_min 1: the captured step reads the buffers of rounded activations, which a longer prompt allocates anew: the tokens of uncaptured steps"""
     import inferflow_amd as ia
