@@ -627,9 +627,9 @@ __device__ __forceinline__ FewSeq few_of(const TileArgs &A, int id, At at)
 }
 
 // The windowed attention's launches may bring the decayed linear attention's of the same layer with them (IfaLinearSide): chunk sums beside the keys' operands, the states from chunk to chunk
-// beside the tiles, the chunks' outputs beside the shares.  Alone, each of them left most of the chip idle: 601 rows of width 1024 (8 heads, 2 of keys) 4.6 + 6.3 + 15.2, 29.4 + 4.9 and
-// 9.2 + 12 us, together 16.0, 29.2 and 13.3; 2048 rows of width 2048 (16 heads, 4) 6.6 + 9.0 + 32, 140 + 10.6
-// and 13.4 + 27.4, together 42.7, 140.6 and 38.3
+// beside the tiles, the chunks' outputs beside the shares.  Alone, each of them left most of the chip idle: 601 rows of width 1024 (8 heads, 2 of keys) 4.8 + 6.1 + 15.0, 27.6 + 4.9 and
+// 9.0 + 11.2 us, together 15.9, 24.8 and 12.8; 2048 rows of width 2048 (16 heads, 4) 6.2 + 8.4 + 30.2, 114.9 + 9.9 and 11.6 + 23.8, together 38.2, 111.3 and 32.5 (tiles whose queries are asked
+// for at once, see k_attn_tile, in the second figures only)
 // At most SIDE_SEQS sequences: a chunk's workgroup finds its sequence by going through them, and has more others beside it to hide that in launches of its own; and the states beside the tiles up
 // to SIDE_PASS workgroups, each of which takes a tile's place on its compute unit (100 KB of LDS), in a launch of their own beyond.  A model's prompts, us, with the launches of its own / shared /
 // shared but for the states, n sequences of up to l tokens: width 1024, 128 such workgroups a sequence: 16 x 300 1884 / 1808 / 1813, 24 x 200 2263 / 2218 / 2202, 32 x 130 2185 / 2176 / 2129,

@@ -759,7 +759,8 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
         if ((rc = glu_down(m, left, 3, sp.f_limit, n->proj + L.c2_fg, N2, F, nullptr, 0, (const bf16_t *)L.T(IFA_LT_FFN_DOWN).data, W, T, nullptr, nullptr, 0, n->m2))) return rc;
     } else {
         int left = GLU_COLUMNS;
-        // prompts: the choice, the sort and the shared expert's activations in one launch, the sum of a row's pairs and of the shared expert inside the norm behind them
+        // prompts: the choice in a launch with its counts, the pairs' places and the shared expert's activations in the next one, the sum of a row's pairs and of the shared expert inside the norm
+        // behind the products
         const size_t SFP = (size_t)sp.x_shared_ff;
         if (moe16 && sp.x_experts <= 512 && (SFP == 0 || takes_a16(n, SFP, T))) {
             if ((rc = linear_in(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2))) return rc;
@@ -776,8 +777,7 @@ int run_sandwich_layer(ifa_model *m, LLayer &L, size_t T, int nseq, bool h_ready
             const float *pair_rows = nullptr;
             if ((rc = ifa_moe_prompt(M, &pair_pos, &pair_rows, s))) return rc;
             if (SFP && (rc = ifa_linear_bf16_both(L.T(IFA_LT_X_SH_DOWN).data, W, SFP, n->a16, a16_stride(SFP), T, nullptr, nullptr, 1.0f, 0, 0, n->m2, nullptr, W, 0, 0, s))) return rc;
-            return ifa_norm_add_norm_moe(n->x, W, T, W, SFP ? n->m2 : nullptr, W, pair_pos, pair_rows, sp.x_top, L.T(IFA_LT_NORM2B).data, next_norm, w_off, c.eps, in16 ? nullptr : n->h,
-                                         in16 ? n->h16 : nullptr, W, s);
+            return ifa_norm_add_norm_moe(n->x, W, T, W, SFP ? n->m2 : nullptr, W, pair_pos, pair_rows, sp.x_top, L.T(IFA_LT_NORM2B).data, next_norm, w_off, c.eps, nullptr, n->h16, W, s);
         }
         if (T <= 8 && sp.x_shared_ff > 0 && !takes_a16(n, W, T)) rc = linear_glu(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2, 0, 0, L.c2_shg, (size_t)sp.x_shared_ff, 0, 0.0f, &left);
         else rc = linear_in(m, L.w_in2, N2, W, n->h, h16, T, L.b_in2, n->proj, N2);

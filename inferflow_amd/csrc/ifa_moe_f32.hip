@@ -6,10 +6,11 @@
 //   experts  y[t] (+)= sum_k wgt[t][k] * E_{idx[t][k]}(h[t]),  E_e(h) = W_down[e] act(W_up[e] h),  identity: E(h) = h
 //            (gated experts: E_e(h) = W_down[e] (silu(W_gate[e] h) * (W_up[e] h)), gate and up rows of an expert stored back to back)
 // Few rows (decode steps): every (row, choice) pair streams its expert's matrices, a wave per output (k_moe_up_rows / k_moe_down_rows).
-// Many rows: the pairs are sorted by expert (k_moe_sort: counts, offsets and tiles of 64 rows of one expert, all in one workgroup),
-// both products run grouped on the matrix cores (ifa_linear_bf16w_grouped: gather of the rows in the first, activation in its epilogue,
-// the pair's weight in the second's) and k_moe_combine adds a row's pairs in the fixed order of its choices.  No atomics on values: a
-// row's result does not depend on what else is in the step.
+// Many rows: the pairs are sorted by expert (counts, offsets and tiles of rows of one expert), both products run grouped on the matrix
+// cores (gather of the rows in the first, activation in its epilogue, the pair's weight in the second's), and a row's pairs are added in
+// the fixed order of its choices.  ifa_moe_prompt (choice by the largest logits, bfloat16 rows, up to 512 experts): sorted by many
+// workgroups (k_moe_route_count, k_moe_place_glu), added by the norm behind (k_norm_add_norm_reg, ifa_ops_f32.hip).  Otherwise sorted
+// by one (k_moe_sort) and added by k_moe_combine.  No atomics on values: a row's result does not depend on what else is in the step.
 #include <algorithm>
 #include <cstring>
 #include "ifa_host.h"
@@ -277,7 +278,7 @@ __global__ void __launch_bounds__(256) k_moe_up_rows(const float *__restrict__ h
 // experts are walked NK at a time with their loads issued side by side (a step is bound by requests in flight: four experts take 130 registers, so that twice as many
 // waves are in flight as with eight), their weighted partial sums reduced once (six rows of four experts of 704 columns 21.6 -> 12.4 us).
 // SHARED: the first of the rows' workgroups (one more than rows) are the shared expert's output product of all rows (k_lin_rows' sums, times sigmoid of a row's gate) into rows of their own, which
-// the norm behind adds: six rows of four experts of 704 and a shared one of 1408 to 1024 columns 13.0 + 9.8 -> 17.9 us.  (Added by the wave that has the row's sum, which reads the shared weights
+// the norm behind adds: six rows of four experts of 704 and a shared one of 1408 to 1024 columns 13.0 + 9.8 -> 16.5 us.  (With a form for eight rows 17.9; added by the wave that has the row's sum, which reads the shared weights
 // once a row: 19.9; the shared expert's workgroups behind the others: 19.7.)  A form for each number of rows (SHARED; 0: without): with eight rows in every step a model of six such layers
 // took 446 / 470 / 549 / 565 / 607 / 649 us a step of 1 / 2 / 3 / 4 / 5 / 6 rows, now 432 / 457 / 530 / 555 / 597 / 645 (two launches: 460 / 496 / 555 / 599 / 653 / 680).
 template <int SH_ROWS>
@@ -414,7 +415,7 @@ __global__ void __launch_bounds__(1024) k_moe_sort(const int *__restrict__ idx, 
 }
 
 // The same in two launches of many workgroups, for the choice by the largest logits (k_moe_route_top's, a wave a row): k_moe_route_count leaves, for each block of `rb` rows, how many of its
-// pairs chose each expert, k_moe_place adds these counts up and gives the pairs their places, in their order.  One workgroup took 7.8 us for 787 rows of 16 experts, top 4, and 13.6 for 2048:
+// pairs chose each expert, k_moe_place_glu adds these counts up and gives the pairs their places, in their order.  One workgroup took 7.8 us for 787 rows of 16 experts, top 4, and 13.6 for 2048:
 // the pairs come and go through one compute unit, and its threads' counters wait for each other.  At most 512 experts (LDS) and 256 blocks (a placing workgroup reads all their counts).
 constexpr int PLACE_EXPERTS = 512, PLACE_BLOCKS = 256, PLACE_WAVES = 16;
 size_t route_count_smem(int experts, int top) { return ((size_t)experts + PLACE_WAVES * (size_t)(experts + top)) * 4; }
@@ -795,13 +796,6 @@ int ifa_moe_experts_gated_top_rows_shared(const void *logits_f32, size_t ldl, co
     R.logits = (const float *)logits_f32; R.ld = ldl; R.n_all = experts; R.score_kind = 2; R.idx = idx_dev; R.wgt = (float *)wgt_f32;
     return moe_experts("moe_experts_gated_top_rows", 1, 0, 0.0f, h_f32, ldh, rows, width, ff, experts, 0, top, 0, gate_up_bf16, down_bf16, idx_dev, wgt_f32, 1, ws, ws_bytes, y_f32, ldy,
                        accumulate, stream, &R, nullptr, shared);
-}
-
-int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
-                                   const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream)
-{
-    return ifa_moe_experts_gated_top_rows_shared(logits_f32, ldl, h_f32, ldh, rows, width, ff, experts, top, gate_up_bf16, down_bf16, idx_dev, wgt_f32, ws, ws_bytes, y_f32, ldy, accumulate,
-                                                 nullptr, stream);
 }
 
 // A wave of the shared expert's workgroups reads all rows' activations for one output: with many weights and three rows and more the launch of its own, which has two outputs a wave there, is the

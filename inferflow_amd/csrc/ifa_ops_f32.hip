@@ -138,7 +138,7 @@ __global__ void __launch_bounds__(256) k_group_rmsnorm(const float *__restrict__
 // workgroup of a sequence's first row is the only one that reads the token the slot holds, and it leaves the sequence's last token
 // of this step there: no other workgroup touches that cell.
 // VEC: pieces of four columns, the first one of the row's embedding asked for beside the row's place, and the slot's cell by a sequence's first row alone: one by one behind the place and the slot a
-// launch took 8.4 / 17.0 us for 6 / 2048 rows of 1024, now 6.7 / 7.2
+// launch took 8.8 / 7.5 / 12.6 us for 6 / 639 / 2048 rows of 1024, now 7.6 / 4.6 / 9.2
 template <bool VEC>
 __global__ void __launch_bounds__(256) k_embed_pair(const bf16_t *__restrict__ embed, int vocab, int width, const bf16_t *__restrict__ pair, int buckets,
                                                     int mul_prev, int mul_cur, const int *__restrict__ tokens, const SeqDesc *__restrict__ seqs,

@@ -117,8 +117,6 @@ extern "C" int ifa_norm_add_norm_moe(void *x_f32, size_t ldx, size_t rows, size_
 struct IfaMoeShared { const ifa32::bf16_t *down; const float *act; size_t lda; int ff; const float *gate; size_t ldg; float *out; size_t ldo; };
 extern "C" bool ifa_moe_shared_fits(const IfaMoeShared &S);
 extern "C" bool ifa_moe_shared_pays(size_t rows, size_t width, size_t ff);          // ... and in which the one launch is no slower than two
-extern "C" int ifa_moe_experts_gated_top_rows(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
-                                   const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, ifa_stream stream);
 extern "C" int ifa_moe_experts_gated_top_rows_shared(const void *logits_f32, size_t ldl, const void *h_f32, size_t ldh, size_t rows, int width, int ff, int experts, int top, const void *gate_up_bf16,
                                           const void *down_bf16, int *idx_dev, void *wgt_f32, void *ws, size_t ws_bytes, void *y_f32, size_t ldy, int accumulate, const IfaMoeShared *shared,
                                           ifa_stream stream);

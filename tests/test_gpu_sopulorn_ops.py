@@ -256,7 +256,7 @@ def test_choice_by_the_largest_logits_inside_the_experts_first_launch(T, W, F, E
     idx, idx_w = (torch.full((T, top), -1, dtype=torch.int32, device="cuda") for _ in range(2))
     wgt, wgt_w = (torch.zeros((T, top), dtype=torch.float32, device="cuda") for _ in range(2))
     y, y_w = (torch.full((T, W + 1), 0.5, dtype=torch.float32, device="cuda") for _ in range(2))
-    ia.check(L.ifa_moe_experts_gated_top_rows(p(dz), Z(E + 3), p(dh), Z(W), Z(T), W, F, E, top, p(gu), p(dd), p(idx), p(wgt), p(ws), Z(nb), p(y), Z(W + 1), 1, None)); sync()
+    ia.check(L.ifa_moe_experts_gated_top_rows_shared(p(dz), Z(E + 3), p(dh), Z(W), Z(T), W, F, E, top, p(gu), p(dd), p(idx), p(wgt), p(ws), Z(nb), p(y), Z(W + 1), 1, None, None)); sync()
     some = [t for t in range(T) if t != 6]
     ia.check(L.ifa_moe_route_top_f32(p(dz), E + 3, T, E, top, None, p(idx_w), p(wgt_w), None))
     got, i, iw = y.cpu().numpy(), idx.cpu().numpy(), idx_w.cpu().numpy()
@@ -314,7 +314,7 @@ def test_shared_expert_in_the_experts_last_launch_leaves_the_bits_of_its_own(T, 
         y, y_w = (torch.full((T, W + 1), 0.5, dtype=torch.float32, device="cuda") for _ in range(2))
         args = [p(dz), Z(E), p(dh), Z(W), Z(T), W, F, E, top, p(gu), p(dd), p(idx), p(wgt), p(ws), Z(nb)]
         ia.check(L.ifa_moe_experts_gated_top_rows_shared(*args, p(y), Z(W + 1), acc, C.byref(shared), None))
-        ia.check(L.ifa_moe_experts_gated_top_rows(*args, p(y_w), Z(W + 1), acc, None))
+        ia.check(L.ifa_moe_experts_gated_top_rows_shared(*args, p(y_w), Z(W + 1), acc, None, None))
         ia.check(L.ifa_linear_bf16w_gated_rows(p(sd), Z(W), Z(SF), p(act), Z(SF + 4), Z(T), C.c_void_p(gate.data_ptr() + 4), Z(3), 0, p(out_w), Z(W + 2), None)); sync()
         assert torch.equal(y, y_w) and torch.equal(out, out_w) and torch.isfinite(y).all() and torch.isfinite(out).all()
     if W % 4:
