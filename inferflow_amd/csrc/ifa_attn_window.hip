@@ -767,163 +767,256 @@ __device__ __forceinline__ void angle_of(int pos, const double *__restrict__ fre
     cs[i] = (float)cn; cs[half + i] = (float)sn;
 }
 
-// turn_head of a head of at most 128 that a wave holds, two values a lane (lane and lane + 64); w: the norm's weights (1: none), cs: the cosines and sines of the lane's pairs
-struct Turn { int half, from[2]; bool first[2]; float w[2]; };
-__device__ __forceinline__ Turn turn_of(int dim, int rot_dims, const bf16_t *nw_, int lane)
+// turn_head of a head of at most 64 E that a wave holds, E values a lane (lane and lane + 64); w: the norm's weights (1: none), cs: the cosines and sines of the lane's pairs
+template <int E> struct Turn { int half, from[E]; bool first[E]; float w[E]; };
+template <int E>
+__device__ __forceinline__ Turn<E> turn_of(int dim, int rot_dims, const bf16_t *nw_, int lane)
 {
-    Turn u;
+    Turn<E> u;
     u.half = rot_dims / 2;
 #pragma unroll
-    for (int e = 0; e < 2; e++) { const int c = lane + 64 * e; u.w[e] = nw_ ? bf2f(nw_[min(c, dim - 1)]) : 1.0f; u.first[e] = c < u.half; u.from[e] = c < u.half ? c + u.half : c - u.half; }
+    for (int e = 0; e < E; e++) { const int c = lane + 64 * e; u.w[e] = nw_ ? bf2f(nw_[min(c, dim - 1)]) : 1.0f; u.first[e] = c < u.half; u.from[e] = c < u.half ? c + u.half : c - u.half; }
     return u;
 }
 // the factor of a held head's root mean square norm
-__device__ __forceinline__ float norm_held(const float (&v)[2], int dim, float eps, int lane)
+template <int E>
+__device__ __forceinline__ float norm_held(const float (&v)[E], int dim, float eps, int lane)
 {
     float s = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 2; e++) if (lane + 64 * e < dim) s = fmaf(v[e], v[e], s);
+    for (int e = 0; e < E; e++) if (lane + 64 * e < dim) s = fmaf(v[e], v[e], s);
     return 1.0f / sqrtf(wave_sum(s) / (float)dim + eps);
 }
-__device__ __forceinline__ void turn_held(float (&v)[2], const Turn &u, int dim, bool norm, float eps, int rot_dims, const float (&cv)[2], const float (&sv)[2], int lane)
+template <int E>
+__device__ __forceinline__ void turn_held(float (&v)[E], const Turn<E> &u, int dim, bool norm, float eps, int rot_dims, const float (&cv)[E], const float (&sv)[E], int lane)
 {
-    float r = 1.0f, val[2];
-    if (norm) r = norm_held(v, dim, eps, lane);
+    float r = 1.0f, val[E];
+    if (norm) r = norm_held<E>(v, dim, eps, lane);
 #pragma unroll
-    for (int e = 0; e < 2; e++) val[e] = v[e] * r * u.w[e];
+    for (int e = 0; e < E; e++) val[e] = v[e] * r * u.w[e];
 #pragma unroll
-    for (int e = 0; e < 2; e++) {
-        const float a = __shfl(val[0], u.from[e] & 63, 64), b = __shfl(val[1], u.from[e] & 63, 64), oth = u.from[e] < 64 ? a : b;
+    for (int e = 0; e < E; e++) {
+        float oth = __shfl(val[0], u.from[e] & 63, 64);
+        if constexpr (E == 2) { const float b = __shfl(val[1], u.from[e] & 63, 64); oth = u.from[e] < 64 ? oth : b; }
         v[e] = lane + 64 * e >= rot_dims ? val[e] : (u.first[e] ? val[e] * cv[e] - oth * sv[e] : val[e] * cv[e] + oth * sv[e]);
     }
 }
-__device__ __forceinline__ void turn_angles(const float *cs, const Turn &u, int rot_dims, int lane, float (&cv)[2], float (&sv)[2])
+template <int E>
+__device__ __forceinline__ void turn_angles(const float *cs, const Turn<E> &u, int rot_dims, int lane, float (&cv)[E], float (&sv)[E])
 {
 #pragma unroll
-    for (int e = 0; e < 2; e++) {
+    for (int e = 0; e < E; e++) {
         const int c = lane + 64 * e, fi = u.first[e] ? c : c - u.half;
         const bool in = c < rot_dims;
         cv[e] = in ? cs[fi] : 1.0f; sv[e] = in ? cs[u.half + fi] : 0.0f;
     }
 }
 
-// a row's heads in place, eight at a time, all their values asked for beside the row's place: a wave (cs: its own)
-template <class Pos>
-__device__ __forceinline__ void turn_row(float *q, int heads, int dim, const bf16_t *nw_, float eps, int rot_dims, const double *freq, float *cs, int lane, Pos position)
+// a row's heads in place, eight at a time (those of part `part` of `parts`), all their values asked for beside the row's place: a wave (cs: its own)
+constexpr int HB = 8;
+template <int E, class Pos>
+__device__ __forceinline__ void turn_row(float *q, int heads, int part, int parts, int dim, const bf16_t *nw_, float eps, int rot_dims, const double *freq, float *cs, int lane, Pos position)
 {
-    constexpr int HB = 8;
-    const Turn u = turn_of(dim, rot_dims, nw_, lane);
-    float cv[2], sv[2];
-    for (int h0 = 0; h0 < heads; h0 += HB) {
-        float v[HB][2];
+    const Turn<E> u = turn_of<E>(dim, rot_dims, nw_, lane);
+    float cv[E], sv[E];
+    for (int h0 = HB * part; h0 < heads; h0 += HB * parts) {
+        float v[HB][E];
 #pragma unroll
         for (int h = 0; h < HB; h++)
 #pragma unroll
-            for (int e = 0; e < 2; e++) v[h][e] = q[(size_t)min(h0 + h, heads - 1) * dim + min(lane + 64 * e, dim - 1)];
-        if (h0 == 0) {
+            for (int e = 0; e < E; e++) v[h][e] = q[(size_t)min(h0 + h, heads - 1) * dim + min(lane + 64 * e, dim - 1)];
+        if (h0 == HB * part) {
             const int pos = position();
             for (int i = lane; i < u.half; i += 64) angle_of(pos, freq, i, u.half, cs);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");          // (the wave's own)
-            turn_angles(cs, u, rot_dims, lane, cv, sv);
+            turn_angles<E>(cs, u, rot_dims, lane, cv, sv);
         }
 #pragma unroll
         for (int h = 0; h < HB; h++) {
-            turn_held(v[h], u, dim, nw_ != nullptr, eps, rot_dims, cv, sv, lane);
+            turn_held<E>(v[h], u, dim, nw_ != nullptr, eps, rot_dims, cv, sv, lane);
 #pragma unroll
-            for (int e = 0; e < 2; e++) if (h0 + h < heads && lane + 64 * e < dim) q[(size_t)(h0 + h) * dim + lane + 64 * e] = v[h][e];
+            for (int e = 0; e < E; e++) if (h0 + h < heads && lane + 64 * e < dim) q[(size_t)(h0 + h) * dim + lane + 64 * e] = v[h][e];
         }
     }
 }
 
 // What a step brings to the cache (k null: nothing, or it is there already): keys as projected, normed and turned as k_kv_store_f32 and k_qk_rope_store do, and values; q_rows: the step's
-// queries are normed and turned in place, four rows a workgroup behind the blocks'.
-struct FreshKV { const float *k; size_t ldk; const float *v; size_t ldv; int norm; const bf16_t *norm_w; float eps; int rot_dims; const double *freq; int q_rows; const bf16_t *q_norm_w; float *q; };          // (q_rows 0: the queries are not turned)
+// queries are normed and turned in place by waves behind the blocks' workgroups, q_parts of them a row.
+struct FreshKV { const float *k; size_t ldk; const float *v; size_t ldv; int norm; const bf16_t *norm_w; float eps; int rot_dims; const double *freq; int q_rows, q_parts, q_wgs; const bf16_t *q_norm_w; float *q; };          // (q_rows 0: the queries are not turned)
 
-// A workgroup per (head of keys, block of the step, keys or values): the rows of a block into its operands -- once per layer and step, not once per tile that reads the block -- and those that the
-// step brings into the cache on their way: a position is in one of the step's blocks, and only there.  Keys go through LDS, all asked for at once.  Bound by its launch and its trips to
-// memory (reads 4, writes 6 bytes per value; fresh rows: 10).  Rows past the sequence's last: that row again (their scores are masked).
-// (A launch that stored the rows and one that read them back: 601 rows of 2 heads of 128 4.6 + 6.3 us; with 8 heads of queries turned 787 rows 8.4 + 6.6, 2048 11.6 + 7.1; now 11.2 and 13.7, the queries in the same launch.)
-// TURN: something is turned, or normed with a weight.  Without it (keys that are normed at most) the angles' and the turns' code is not there: steps of a few rows walk through the kernel's code once,
-// and 17 KB of it take 8.1 us for 19 rows of 2 heads of 128, 32 KB with both 9.9 (two launches, as above, 3.3 + 5.4 and the gap between them).
-template <int NTK, int NTV, bool TURN, bool SIDE>
-__global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, FreshKV F, int blocks, std::conditional_t<SIDE, SideArgs, int> side)
+// the sequence of the step's block `at`, which becomes the number inside it; false: there is none
+__device__ __forceinline__ bool block_seq(const WinAttnArgs &P, const TileArgs &A, int &at, SeqDesc &sd)
 {
-    constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK, KROW = DK + 4, VI = (4 * DV + 255) / 256;
+    if (A.n_few) { const FewSeq f = few_of(A, at, [](const FewSeq &x) { return x.block0; }); sd = f.sd; at -= f.block0; return true; }
+    const int sq = item_of(A.n_seqs, at, [&](int x) { if (x < 0) return 0; const SeqDesc &b = P.seqs[x]; return seq_blocks(b.pos0, b.n, P.window, P.keep_first).count; });
+    if (sq < 0) return false;
+    sd = P.seqs[sq];
+    return true;
+}
+
+// grid (kv heads, blocks of the step): the cache rows of a block into its operands, where everything is in the cache already -- once per layer and step, not once per tile that reads the block.
+// Bound by its launch and one trip to memory (reads 4, writes 6 bytes per value).  Rows past the sequence's last: that row again (their scores are masked).
+template <int NTK, int NTV>
+__global__ void __launch_bounds__(256) k_attn_parts_kept(WinAttnArgs P, TileArgs A)
+{
+    constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK;
+    const int tid = threadIdx.x, kvh = blockIdx.x, dk = P.dim, dv = P.vdim;
+    int at = blockIdx.y;
+    SeqDesc sd;
+    if (!block_seq(P, A, at, sd)) return;
+    const SeqBlocks sb = seq_blocks(sd.pos0, sd.n, P.window, P.keep_first);
+    const int kb0 = (at < sb.kept ? at : sb.first + at - sb.kept) * WT_K, last = sd.pos0 + sd.n - 1;
+    const size_t kvd = (size_t)P.kv_heads * dk, vvd = (size_t)P.kv_heads * dv;
+    gfloat *kc = (gfloat *)(P.slot_base[sd.slot] + P.k_off + (size_t)kvh * dk), *vc = (gfloat *)(P.slot_base[sd.slot] + P.v_off + (size_t)kvh * dv);
+    bf16x8w *dst = (bf16x8w *)P.ws + ((size_t)blockIdx.y * P.kv_heads + kvh) * kBlockPieces<NTK, NTV>;
+    const bool vec = dk % 4 == 0 && P.k_off % 4 == 0;      // (arena bases are 256-byte aligned)
+    bool odd = false;          // an infinity or NaN among the thread's values
+    for (int e = tid; e < WT_K * (DK / 8); e += 256) {
+        const int key = e / (DK / 8), c8 = e % (DK / 8), c = 8 * c8;
+        gfloat *row = kc + (size_t)min(kb0 + key, last) * kvd;
+        float v[8];
+        if (vec) {
+            const f32x4w lo = *(gf32x4 *)(row + min(c, dk - 4)), hi = *(gf32x4 *)(row + min(c + 4, dk - 4));
+#pragma unroll
+            for (int x = 0; x < 4; x++) { v[x] = c < dk ? lo[x] : 0.0f; v[4 + x] = c + 4 < dk ? hi[x] : 0.0f; }
+        } else {
+#pragma unroll
+            for (int x = 0; x < 8; x++) { const float f = row[min(c + x, dk - 1)]; v[x] = c + x < dk ? f : 0.0f; }
+        }
+        odd |= not_finite(v);
+        const Parts t = parts_of(v);
+#pragma unroll
+        for (int pl = 0; pl < 3; pl++) dst[(pl * KS + (c8 >> 1)) * 64 + 32 * (c8 & 1) + key] = t.p[pl];
+    }
+    dst += 3 * KS * 64;
+    for (int e = tid; e < 4 * DV; e += 256) {
+        const int d = e % DV, sg = e / DV, k0 = 16 * (sg >> 1) + 4 * (sg & 1);
+        float v[8];
+#pragma unroll
+        for (int x = 0; x < 8; x++) { const float f = vc[(size_t)min(kb0 + k0 + 8 * (x >> 2) + (x & 3), last) * vvd + min(d, dv - 1)]; v[x] = d < dv ? f : 0.0f; }
+        odd |= not_finite(v);
+        const Parts t = parts_of(v);
+#pragma unroll
+        for (int pl = 0; pl < 3; pl++) dst[((pl * NTV + (d >> 5)) * 2 + (sg >> 1)) * 64 + 32 * (sg & 1) + (d & 31)] = t.p[pl];
+    }
+    const int any = __syncthreads_or(odd);
+    if (tid < 4) ((uint32_t *)(P.ws + A.marks))[4 * ((size_t)blockIdx.y * P.kv_heads + kvh) + tid] = any ? 1u : 0u;
+}
+
+// Workgroups that a block's keys, or its values, of so many 32s are shared out to: the chain of a step of a few rows (a head's angles in double, its norm, its turn) is as long as the keys a wave has.
+__host__ __device__ constexpr int part_shares(int NT) { return NT > 2 ? 2 : 1; }
+
+// ... with rows that the step brings: a workgroup per (head of keys, block of the step, share of its keys or values) lays a block's rows out as operands and stores those of the step into the cache on
+// their way: a position is in one of the step's blocks, and only there.  Fresh keys go through LDS, all asked for at once.  In front of them, for they take longest, the step's queries, normed and turned
+// in place: a wave per row and up to all of its heads, fewer where there are few rows.  Rows past the sequence's last: that row as it came (their scores are masked).
+// TURN: something is turned, or normed with a weight.  Without it (keys that are normed at most) the angles' and the turns' code is not there: steps of a few rows walk through the kernel's code once.
+// us, the launch that stored the rows + the one that read them back -> this one: 2 heads of keys of 128, 19 rows 3.3 + 5.4 -> 6.6, 100 rows 4.0 + 6.3 -> 6.5; with 8 heads of queries, 64 of 128 columns
+// turned, 639 rows 8.7 + 6.4 -> 9.6, 2048 12.4 + 6.9 -> 12.9.  See fresh_pays for where the two launches stay.
+template <int NTK, int NTV, bool TURN, bool SIDE>
+__global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, FreshKV F, std::conditional_t<SIDE, SideArgs, int> side)
+{
+    constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK, KROW = DK + 4, E = (DK + 63) / 64;
+    constexpr int KH = part_shares(NTK), VH = part_shares(NTV), KN = WT_K / KH, KI = (KN * (DK / 8) + 255) / 256, VN = 4 * DV / VH, VI = (VN + 255) / 256;
     int id = blockIdx.x;
     if constexpr (SIDE) {
         if (id < side.first) { ifachunk::linear_chunk(side.c, id % side.chunks, id / side.chunks % side.c.heads, id / side.chunks / side.c.heads); return; }
         id -= side.first;
     }
-    extern __shared__ __attribute__((aligned(16))) float part_lds[];          // [32][KROW], [32][rot_dims]
-    float *rows = part_lds, *cs = part_lds + WT_K * KROW;
+    extern __shared__ __attribute__((aligned(16))) float part_lds[];          // [KN][KROW], [KN][rot_dims] (queries: [4][rot_dims])
+    float *rows = part_lds, *cs = part_lds + KN * KROW;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = P.dim, dv = P.vdim, half = F.rot_dims / 2;
-    if constexpr (TURN)
-        if (id >= 2 * P.kv_heads * blocks) {          // queries, a row a wave
-            const int t = 4 * (id - 2 * P.kv_heads * blocks) + wave;
-            if (t < F.q_rows) turn_row(F.q + (size_t)t * P.ldq, P.heads, dk, F.q_norm_w, F.eps, F.rot_dims, F.freq, cs + wave * F.rot_dims, lane, [&]() {
+    if constexpr (TURN) {
+        if (id < F.q_wgs) {          // queries
+            const int w = 4 * id + wave, t = w / F.q_parts;
+            if (t < F.q_rows) turn_row<E>(F.q + (size_t)t * P.ldq, P.heads, w % F.q_parts, F.q_parts, dk, F.q_norm_w, F.eps, F.rot_dims, F.freq, cs + wave * F.rot_dims, lane, [&]() {
                     const SeqDesc sd = A.n_few ? few_of(A, t, [](const FewSeq &x) { return x.sd.row0; }).sd : P.seqs[P.row_seq[t]];
                     return sd.pos0 + t - sd.row0;
                 });
             return;
         }
-    const bool keys = (id & 1) == 0;
-    const int kvh = (id >> 1) % P.kv_heads, place = (id >> 1) / P.kv_heads;
+        id -= F.q_wgs;
+    }
+    const int share = id % (KH + VH), kvh = id / (KH + VH) % P.kv_heads, place = id / (KH + VH) / P.kv_heads;
+    const bool keys = share < KH;
     int at = place;
     SeqDesc sd;
-    if (A.n_few) { const FewSeq f = few_of(A, place, [](const FewSeq &x) { return x.block0; }); sd = f.sd; at -= f.block0; }
-    else {
-        const int sq = item_of(A.n_seqs, at, [&](int x) { if (x < 0) return 0; const SeqDesc &b = P.seqs[x]; return seq_blocks(b.pos0, b.n, P.window, P.keep_first).count; });
-        if (sq < 0) return;
-        sd = P.seqs[sq];
-    }
+    if (!block_seq(P, A, at, sd)) return;
     const SeqBlocks sb = seq_blocks(sd.pos0, sd.n, P.window, P.keep_first);
-    const int kb0 = (at < sb.kept ? at : sb.first + at - sb.kept) * WT_K, last = sd.pos0 + sd.n - 1, fresh0 = F.k ? sd.pos0 : 0x7FFFFFFF;          // positions from fresh0 on are the step's
+    const int kb0 = (at < sb.kept ? at : sb.first + at - sb.kept) * WT_K, k0b = keys ? KN * share : 0, last = sd.pos0 + sd.n - 1, fresh0 = F.k ? sd.pos0 : 0x7FFFFFFF;          // positions from fresh0 on are the step's
     typedef __attribute__((address_space(1))) float gfloat_w;
     bf16x8w *dst = (bf16x8w *)P.ws + ((size_t)place * P.kv_heads + kvh) * kBlockPieces<NTK, NTV>;
     bool odd = false;          // an infinity or NaN among the thread's values
-    if (keys) {
+    if (keys && kb0 + WT_K <= fresh0) {          // cached rows alone: pieces of eight columns as they are read
+        gfloat *kc = (gfloat *)(P.slot_base[sd.slot] + P.k_off + (size_t)kvh * dk);
+        const bool vec = dk % 4 == 0 && P.k_off % 4 == 0;          // (arena bases are 256-byte aligned)
+        f32x4w raw[KI][2];
+#pragma unroll
+        for (int u = 0; u < KI; u++) {
+            const int e = min(tid + 256 * u, KN * (DK / 8) - 1), key = k0b + e / (DK / 8), c = 8 * (e % (DK / 8));
+            gfloat *row = kc + (size_t)min(kb0 + key, last) * P.kv_heads * dk;
+            if (vec) { raw[u][0] = *(gf32x4 *)(row + min(c, dk - 4)); raw[u][1] = *(gf32x4 *)(row + min(c + 4, dk - 4)); }
+            else {
+#pragma unroll
+                for (int x = 0; x < 8; x++) raw[u][x >> 2][x & 3] = row[min(c + x, dk - 1)];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < KI; u++) {
+            const int e = tid + 256 * u, key = k0b + e / (DK / 8), c8 = e % (DK / 8);
+            if (e >= KN * (DK / 8)) break;
+            float f[8];
+#pragma unroll
+            for (int x = 0; x < 8; x++) f[x] = 8 * c8 + x < dk ? raw[u][x >> 2][x & 3] : 0.0f;
+            odd |= not_finite(f);
+            const Parts t = parts_of(f);
+#pragma unroll
+            for (int pl = 0; pl < 3; pl++) dst[(pl * KS + (c8 >> 1)) * 64 + 32 * (c8 & 1) + key] = t.p[pl];
+        }
+    } else if (keys) {
         const size_t kvd = (size_t)P.kv_heads * dk;
         gfloat_w *kc = (gfloat_w *)(P.slot_base[sd.slot] + P.k_off + (size_t)kvh * dk);
-        constexpr int KW = WT_K / 4;          // keys a wave, two values of each a lane
-        float v[KW][2];
+        constexpr int KW = KN / 4;          // keys a wave, E values of each a lane
+        float v[KW][E];
 #pragma unroll
         for (int x = 0; x < KW; x++) {
-            const int j = min(kb0 + KW * wave + x, last);
+            const int j = min(kb0 + k0b + KW * wave + x, last);
             gfloat *row = (gfloat *)F.k + (size_t)(sd.row0 + j - sd.pos0) * F.ldk + (size_t)kvh * dk;
             if (kb0 < fresh0 && j < fresh0) row = (gfloat *)kc + (size_t)j * kvd;          // (blocks of the step alone do not wait for the slot's place)
 #pragma unroll
-            for (int e = 0; e < 2; e++) v[x][e] = row[min(lane + 64 * e, dk - 1)];
+            for (int e = 0; e < E; e++) v[x][e] = row[min(lane + 64 * e, dk - 1)];
         }
-        Turn u;
+        Turn<E> u;
         if constexpr (TURN) {
-            u = turn_of(dk, F.rot_dims, F.norm_w, lane);
-            if (kb0 + WT_K > fresh0) {
-                for (int e = lane; e < KW * half; e += 64) { const int key = KW * wave + e / half; angle_of(kb0 + key, F.freq, e % half, half, cs + key * F.rot_dims); }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");          // (the wave's own)
+            u = turn_of<E>(dk, F.rot_dims, F.norm_w, lane);
+            for (int e = lane; e < KW * half; e += 64) {
+                const int key = KW * wave + e / half, j = kb0 + k0b + key;
+                if (j >= fresh0 && j <= last) angle_of(j, F.freq, e % half, half, cs + key * F.rot_dims);
             }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");          // (the wave's own)
         }
 #pragma unroll
         for (int x = 0; x < KW; x++) {
-            const int key = KW * wave + x, j = kb0 + key;
-            if (min(j, last) >= fresh0) {          // (beyond the last: turned by another angle, masked like the row again)
+            const int key = KW * wave + x, j = kb0 + k0b + key;
+            if (j >= fresh0 && j <= last) {          // (beyond the last: that row as it came, masked)
                 if constexpr (TURN) {
-                    float cv[2], sv[2];
-                    turn_angles(cs + key * F.rot_dims, u, F.rot_dims, lane, cv, sv);
-                    turn_held(v[x], u, dk, F.norm != 0, F.eps, F.rot_dims, cv, sv, lane);
+                    float cv[E], sv[E];
+                    turn_angles<E>(cs + key * F.rot_dims, u, F.rot_dims, lane, cv, sv);
+                    turn_held<E>(v[x], u, dk, F.norm != 0, F.eps, F.rot_dims, cv, sv, lane);
                 } else if (F.norm) {
-                    const float r = norm_held(v[x], dk, F.eps, lane);
-                    v[x][0] *= r; v[x][1] *= r;
+                    const float r = norm_held<E>(v[x], dk, F.eps, lane);
+#pragma unroll
+                    for (int e = 0; e < E; e++) v[x][e] *= r;
                 }
             }
 #pragma unroll
-            for (int e = 0; e < 2; e++) {
+            for (int e = 0; e < E; e++) {
                 const int c = lane + 64 * e;
                 if (c < DK) rows[key * KROW + c] = c < dk ? v[x][e] : 0.0f;
                 if (c < dk && j >= fresh0 && j <= last) kc[(size_t)j * kvd + c] = v[x][e];
             }
         }
         __syncthreads();
-        for (int e = tid; e < WT_K * (DK / 8); e += 256) {
+        for (int e = tid; e < KN * (DK / 8); e += 256) {
             const int key = e / (DK / 8), c8 = e % (DK / 8);
             const float *row = rows + key * KROW + 8 * c8;
             float f[8];
@@ -933,7 +1026,7 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, F
             odd |= not_finite(f);
             const Parts t = parts_of(f);
 #pragma unroll
-            for (int pl = 0; pl < 3; pl++) dst[(pl * KS + (c8 >> 1)) * 64 + 32 * (c8 & 1) + key] = t.p[pl];
+            for (int pl = 0; pl < 3; pl++) dst[(pl * KS + (c8 >> 1)) * 64 + 32 * (c8 & 1) + k0b + key] = t.p[pl];
         }
     } else {
         const size_t vvd = (size_t)P.kv_heads * dv;
@@ -941,7 +1034,7 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, F
         float v[VI][8];
 #pragma unroll
         for (int u = 0; u < VI; u++) {
-            const int e = min(tid + 256 * u, 4 * DV - 1), d = e % DV, sg = e / DV, k0 = 16 * (sg >> 1) + 4 * (sg & 1);
+            const int e = (share - KH) * VN + min(tid + 256 * u, VN - 1), d = e % DV, sg = e / DV, k0 = 16 * (sg >> 1) + 4 * (sg & 1);
 #pragma unroll
             for (int x = 0; x < 8; x++) {
                 const int j = min(kb0 + k0 + 8 * (x >> 2) + (x & 3), last);
@@ -953,8 +1046,8 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, F
         dst += 3 * KS * 64;
 #pragma unroll
         for (int u = 0; u < VI; u++) {
-            const int e = tid + 256 * u, d = e % DV, sg = e / DV, k0 = 16 * (sg >> 1) + 4 * (sg & 1);
-            if (e >= 4 * DV) break;
+            const int e = (share - KH) * VN + tid + 256 * u, d = e % DV, sg = e / DV, k0 = 16 * (sg >> 1) + 4 * (sg & 1);
+            if (tid + 256 * u >= VN) break;
 #pragma unroll
             for (int x = 0; x < 8; x++) {
                 const int j = kb0 + k0 + 8 * (x >> 2) + (x & 3);
@@ -968,7 +1061,7 @@ __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, F
         }
     }
     const int any = __syncthreads_or(odd);
-    if (tid == 0) ((uint32_t *)(P.ws + A.marks))[2 * ((size_t)place * P.kv_heads + kvh) + (keys ? 0 : 1)] = any ? 1u : 0u;
+    if (tid == 0) ((uint32_t *)(P.ws + A.marks))[4 * ((size_t)place * P.kv_heads + kvh) + share] = any ? 1u : 0u;
 }
 
 // Key rows of dim <= 32 NTK and value rows of vdim <= 32 NTV floats.  VEC: rows of whole, aligned 16-byte pieces in q and the output.
@@ -1010,13 +1103,18 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
                 __builtin_amdgcn_global_load_lds((wa_glb_t *)(src + (u + wave) * 64 + lane), (wa_lds_t *)(dst + (u + wave) * 64), 16, 0, 0);
     };
     // which of the chunk's blocks (64 at a time) have a mark
-    typedef uint32_t u32x2w __attribute__((ext_vector_type(2)));          // (its keys, its values)
-    auto mark_of = [&](int b) -> u32x2w {
+    typedef uint32_t u32x4w __attribute__((ext_vector_type(4)));          // (its shares, see k_attn_parts)
+    auto mark_of = [&](int b) -> u32x4w {
         const int x = min(b + lane, b1 - 1), block = x < tb.kept ? x : tb.first + x - tb.kept, at = block < sb.kept ? block : sb.kept + block - sb.first;
-        return ((const __attribute__((address_space(1))) u32x2w *)(P.ws + A.marks))[(size_t)(block0 + at) * P.kv_heads + kvh];
+        return ((const __attribute__((address_space(1))) u32x4w *)(P.ws + A.marks))[(size_t)(block0 + at) * P.kv_heads + kvh];
     };
-    auto marked = [&](int b, u32x2w m) -> uint64_t { return __builtin_amdgcn_ballot_w64((m[0] | m[1]) != 0 && b + lane < b1); };
-    u32x2w first;
+    auto marked = [&](int b, u32x4w m) -> uint64_t {
+        uint32_t any = m[0] | m[1];
+        if constexpr (part_shares(NTK) + part_shares(NTV) > 2) any |= m[2];
+        if constexpr (part_shares(NTK) + part_shares(NTV) > 3) any |= m[3];
+        return __builtin_amdgcn_ballot_w64(any != 0 && b + lane < b1);
+    };
+    u32x4w first;
     // All of the lane's query at once (queries past the tile's last: that one again, not stored), in front of the first block's operands, behind whose requests it would wait for them: asked
     // for by fours behind these, and every eight values looked at for ones that would round to infinity, a launch took 28.3 us for 601 rows of 8 heads, now 25.3 (2048 rows of 16 heads 122.8, 118.9).
     float qv[KS][8];
@@ -1326,7 +1424,7 @@ TilePlan tile_plan(const ifa_seq_desc *sh, int n_seqs, int heads, int kv_heads, 
     }
     t.tiles = nbs.size();
     t.mark_at = t.blocks * (size_t)kv_heads * 3 * 64 * 16 * (size_t)(2 * NTK + 2 * NTV);
-    t.op_bytes = t.mark_at + (t.blocks * (size_t)kv_heads * 8 + 15) / 16 * 16;
+    t.op_bytes = t.mark_at + t.blocks * (size_t)kv_heads * 16;
     const size_t hx = (size_t)(heads / t.hpw), share = (size_t)WT_WAVES * 32 * ((size_t)vdim + 2) * 4;
     size_t cb = std::max<size_t>({2, total * hx / WT_SLOTS, (most + WT_MAX_CHUNKS - 1) / WT_MAX_CHUNKS});
     auto chunks = [&]() { return (most + cb - 1) / cb; };
@@ -1340,6 +1438,19 @@ TilePlan tile_plan(const ifa_seq_desc *sh, int n_seqs, int heads, int kv_heads, 
     t.cb = (int)cb; t.chunks = (int)chunks(); t.groups = groups();
     t.bytes = t.op_bytes + (t.chunks > 1 ? t.tiles * hx * (size_t)t.chunks * share : 0);
     return t;
+}
+
+// Whether a step's rows are stored, and its queries turned, by the launch that lays the operands out (one) or by a launch in front of it (two).  One saves a launch and the rows' way back, and shares a
+// row's heads out where rows are few; two has smaller kernels, of which twice as many workgroups are on the chip: where there are more than fit at once (fresh blocks: a workgroup counts whole, a
+// cached one for an eighth) they win, unless the queries are so many that their own launch takes long.  us one / two: 8 heads, 8 of keys, of 128: 16 rows 19.5 / 24.4, 200 33 / 38, 2048 93 / 94,
+// 64 prompts of 20 54.6 / 49.8, 32 of 100 77 / 70; 2 heads of keys, a token each of 16 users behind 300 37.7 / 43.2, of 64 behind 500 81.0 / 79.0; 64 heads, 8 of keys: 16 rows 20.7 / 41.4, 32 of 100
+// 193 / 243; 32 heads, as many of keys, of 64: 30 rows behind 4000 81 / 98.
+constexpr int TURN_WAVES = 1024;          // waves that turn queries, as many as stand on the chip at once: a row's heads are shared out to get there
+bool fresh_pays(const ifa_seq_desc *sh, int n_seqs, size_t rows, size_t blocks, int wgs, bool own, int turned_heads)
+{
+    size_t fresh = 0;
+    if (own) for (int q = 0; q < n_seqs; q++) fresh += (size_t)((sh[q].pos0 + sh[q].n - 1) / WT_K - sh[q].pos0 / WT_K + 1);
+    return fresh * wgs + (blocks - fresh) * wgs / 8 <= 1024 + rows * turned_heads / 24;
 }
 
 // (the rows of a step's sequences follow each other)
@@ -1498,6 +1609,11 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
     P.sink = (const bf16_t *)sink_bf16; P.sink_fixed = sink_fixed; P.sink_score = sink_score;
     P.seqs = (const SeqDesc *)seqs_dev; P.row_seq = row_seq_dev; P.slot_base = (float *const *)slot_base_dev;
     P.k_off = k_off; P.v_off = v_off; P.out = (float *)out_f32; P.ldo = ldo; P.out16 = nullptr; P.ld16 = 0; P.ws = nullptr; P.nsplit = 1;
+    auto store_fresh = [&]() -> int {
+        return fresh->turn_q ? ifa_qk_rope_store_f32((void *)q_f32, ldq, heads, fresh->k, fresh->ldk, fresh->v, fresh->ldv, kv_heads, dim, vdim, fresh->q_norm_w, fresh->norm_w, fresh->eps,
+                                                     fresh->rot_dims, fresh->freq, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, stream)
+                             : ifa_kv_store_f32(fresh->k, fresh->ldk, fresh->v, fresh->ldv, kv_heads, dim, fresh->norm, fresh->eps, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, stream);
+    };
     // prompts: the tiled matrix-core kernels (heads of up to 128 dimensions, zero-padded to whole 32s); single tokens and other sizes: a workgroup per row.
     // With a workspace the bfloat16 form, from the smallest tiled step on (8 heads of 128: 16 rows 15.5 against 17.8 us, 256 rows 33 against 71, 64 rows behind 3000 keys 49 against 719).
     // Not for one row: its grids follow from the HOST's positions, and a step of one row is captured once and replayed while the position on the device goes on.
@@ -1513,15 +1629,22 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
             const bool vec = dim % 4 == 0 && vdim % 4 == 0 && ldq % 4 == 0 && ldo % 4 == 0 && (uintptr_t)q_f32 % 16 == 0 && (uintptr_t)out_f32 % 16 == 0
                              && (!out_bf16 || (ld16 % 4 == 0 && (uintptr_t)out_bf16 % 8 == 0));
             const int hx = heads / t.hpw;
+            if (n_seqs > SIDE_SEQS) side = nullptr;          // (*side_done stays false)
+            if (fresh && !side && !fresh_pays((const ifa_seq_desc *)seqs_host, n_seqs, rows, t.blocks, kv_heads * (part_shares(NTK) + part_shares(NTV)), fresh->k != nullptr,
+                                              fresh->turn_q ? heads : 0)) {
+                if (const int rc = store_fresh()) return rc;
+                fresh = nullptr;
+            }
             FreshKV F;
             memset(&F, 0, sizeof(F));
             if (fresh) {
                 F.k = fresh->k; F.ldk = fresh->ldk; F.v = fresh->v; F.ldv = fresh->ldv; F.norm = fresh->norm; F.norm_w = fresh->norm_w; F.eps = fresh->eps; F.rot_dims = fresh->rot_dims;
                 F.freq = fresh->freq; F.q_rows = fresh->turn_q ? (int)rows : 0; F.q_norm_w = fresh->q_norm_w; F.q = (float *)q_f32;
             }
+            F.q_parts = (int)std::max<size_t>(1, std::min<size_t>(TURN_WAVES / rows, ((size_t)heads + HB - 1) / HB));
+            F.q_wgs = (int)(((size_t)F.q_rows * F.q_parts + 3) / 4);
             SideArgs S;
             memset(&S, 0, sizeof(S));
-            if (n_seqs > SIDE_SEQS) side = nullptr;          // (*side_done stays false)
             if (side) {
                 size_t chunks = 0;
                 const int rc = ifa_chunk_args(&S.c, &chunks, 0, side->q, side->ldq, side->k, side->ldk, side->v, side->ldv, side->heads, side->heads, side->dk, side->dv, side->decay, nullptr,
@@ -1531,16 +1654,17 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
                 const size_t pass = (size_t)S.per * side->heads * n_seqs;
                 S.pass = pass <= SIDE_PASS ? (int)pass : 0;
             }
-            const bool turn = F.rot_dims > 0 || F.q_rows > 0 || F.norm_w;
+            const bool turn = F.rot_dims > 0 || F.q_rows > 0 || F.norm_w, kept = !F.k && !F.q_rows && !side;
             IFA_REQUIRE(!side || !turn, "%s: the linear attention goes beside keys that are not turned", who);
-            const unsigned part_wgs = (unsigned)(S.first + 2 * kv_heads * t.blocks + ((size_t)F.q_rows + 3) / 4), tile_wgs = (unsigned)(hx * t.groups + S.pass);
-#define IFA_WT(K, V) { const size_t smem_p = (size_t)WT_K * (32 * K + 4 + F.rot_dims) * 4; \
+            const unsigned part_wgs = (unsigned)(S.first + (size_t)(part_shares(NTK) + part_shares(NTV)) * kv_heads * t.blocks + F.q_wgs), tile_wgs = (unsigned)(hx * t.groups + S.pass);
+#define IFA_WT(K, V) { const size_t smem_p = ((size_t)(WT_K / part_shares(K)) * (32 * K + 4) + (size_t)std::max(WT_K / part_shares(K), 4) * F.rot_dims) * 4; \
                        const size_t smem_t = (size_t)2 * kBlockPieces<K, V> * 16 + WT_WAVES * 64 * 4; \
                        const void *fn = vec ? (const void *)k_attn_tile<K, V, true> : (const void *)k_attn_tile<K, V, false>; \
                        IFA_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_t)); \
-                       if (side) hipLaunchKernelGGL((k_attn_parts<K, V, false, true>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, S); \
-                       else if (turn) hipLaunchKernelGGL((k_attn_parts<K, V, true, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, 0); \
-                       else hipLaunchKernelGGL((k_attn_parts<K, V, false, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, (int)t.blocks, 0); \
+                       if (kept) hipLaunchKernelGGL((k_attn_parts_kept<K, V>), dim3((unsigned)kv_heads, (unsigned)t.blocks), dim3(256), 0, ifa_s(stream), P, A); \
+                       else if (side) hipLaunchKernelGGL((k_attn_parts<K, V, false, true>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, S); \
+                       else if (turn) hipLaunchKernelGGL((k_attn_parts<K, V, true, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, 0); \
+                       else hipLaunchKernelGGL((k_attn_parts<K, V, false, false>), dim3(part_wgs), dim3(256), smem_p, ifa_s(stream), P, A, F, 0); \
                        if (side && !S.pass) ifa_linear_pass(S.c, stream); \
                        if (vec) hipLaunchKernelGGL((k_attn_tile<K, V, true>), dim3(tile_wgs), dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A, hx, (int)t.groups, S); \
                        else hipLaunchKernelGGL((k_attn_tile<K, V, false>), dim3(tile_wgs), dim3(64 * WT_WAVES), smem_t, ifa_s(stream), P, A, hx, (int)t.groups, S); }
@@ -1562,12 +1686,7 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
             return IFA_OK;
         }
     }
-    if (fresh) {
-        const int rc = fresh->turn_q ? ifa_qk_rope_store_f32((void *)q_f32, ldq, heads, fresh->k, fresh->ldk, fresh->v, fresh->ldv, kv_heads, dim, vdim, fresh->q_norm_w, fresh->norm_w, fresh->eps,
-                                                             fresh->rot_dims, fresh->freq, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, stream)
-                     : ifa_kv_store_f32(fresh->k, fresh->ldk, fresh->v, fresh->ldv, kv_heads, dim, fresh->norm, fresh->eps, seqs_dev, row_seq_dev, rows, slot_base_dev, k_off, v_off, stream);
-        if (rc) return rc;
-    }
+    if (fresh) { if (const int rc = store_fresh()) return rc; }
     // prompts without a workspace (or with one that the operands do not fit, or of more key blocks than a grid has)
     if (rows >= (size_t)tile_min_rows && n_seqs > 0 && dim <= 128 && vdim <= 128) {
         const ifa_seq_desc *sh = (const ifa_seq_desc *)seqs_host;

@@ -45,14 +45,17 @@ def same(a, b):
 MAX = 700
 ONE, PART, MANY = [[(70, 0, 0)], [(45, 70, 0)]], [[(33, 0, 1), (17, 0, 0), (40, 0, 2)], [(21, 40, 2), (64, 33, 1), (18, 17, 0)]], [[(20 + q, 0, q) for q in range(6)]]
 FOUR, FIVE = [[(9 + 15 * q, 0, q) for q in range(4)], [(33 - q, 9 + 15 * q, q) for q in range(4)]], [[(40 - 3 * q, 0, q) for q in range(5)]]          # (as many as a launch's arguments hold, one more)
+TWO = [[(9, 0, q) for q in range(64)], [(1, 9, q) for q in range(64)], [(130, 10, q) for q in range(12)], [(1, 140, q) for q in range(12)] + [(40, 10, 20)]]          # (many short ones, single tokens, ...)
 
 
 # heads a workgroup shares (1, 2, 4) and more of them than a wave turns at once, heads of whole and of ragged 32s, values of their own size, nothing / a part / all of a head turned, windows
-# behind kept tokens, up to four sequences and more, portions that begin inside a block, long enough for several chunks; the last: fewer rows than the tiled form takes
+# behind kept tokens, up to four sequences and more, portions that begin inside a block, long enough for several chunks, fewer rows than the tiled form takes; steps whose rows a launch in front stores;
+# many heads of queries, shared out to the waves of few rows
 @pytest.mark.parametrize("H,G,D,DV,rot,window,keep,steps,tile_min", [
     (8, 2, 128, 128, 64, 0, 0, ONE, 16), (4, 1, 128, 64, 128, 0, 0, PART, 16), (12, 3, 64, 96, 32, 40, 5, PART, 16), (6, 3, 96, 32, 0, 33, 70, ONE, 16), (5, 5, 40, 48, 10, 0, 0, PART, 16),
     (20, 5, 32, 128, 32, 0, 0, MANY, 16), (2, 2, 128, 128, 126, 100, 40, [[(650, 0, 0)]], 16), (8, 2, 72, 100, 64, 0, 0, [[(9, 0, 0)], [(6, 9, 0)]], 16), (3, 1, 30, 33, 30, 0, 0, PART, 16),
-    (4, 2, 64, 64, 32, 45, 3, FOUR, 16), (4, 2, 64, 64, 32, 45, 3, FIVE, 16)])
+    (4, 2, 64, 64, 32, 45, 3, FOUR, 16), (4, 2, 64, 64, 32, 45, 3, FIVE, 16),
+    (8, 8, 128, 128, 128, 0, 0, TWO, 16), (40, 1, 128, 128, 64, 0, 0, PART, 16), (72, 2, 64, 64, 64, 30, 0, ONE, 16), (33, 3, 96, 128, 96, 0, 0, ONE, 16)])
 @pytest.mark.parametrize("own", [True, False])
 def test_rows_of_rotated_attention_stored_on_the_way(H, G, D, DV, rot, window, keep, steps, tile_min, own):
     rng = np.random.default_rng(H * D + rot)
@@ -61,7 +64,7 @@ def test_rows_of_rotated_attention_stored_on_the_way(H, G, D, DV, rot, window, k
     L = capi()
     nw, kw = devbf(bf16_round(1 + 0.1 * rng.standard_normal(D))), devbf(bf16_round(1 + 0.1 * rng.standard_normal(D)))
     freq = torch.from_numpy(10000.0 ** -(np.arange(max(rot // 2, 1)) / max(rot // 2, 1))).cuda()
-    slots = [Slots(6, v_off + MAX * G * DV) for _ in range(2)]
+    slots = [Slots(1 + max(q for step in steps for _, _, q in step), v_off + MAX * G * DV) for _ in range(2)]
     if not own:          # another layer's rows
         for a, b in zip(slots[0].mem, slots[1].mem):
             a.copy_(torch.from_numpy(rng.standard_normal(a.numel()).astype(np.float32))); b.copy_(a)
