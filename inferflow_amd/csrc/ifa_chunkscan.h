@@ -110,7 +110,8 @@ __device__ __forceinline__ void linear_pass(const ChunkArgs &A, int e, int h, in
     const int nc = (sd.n + CL - 1) / CL;
     const double d = (double)A.decay_head[h];
     const float whole = (float)power(d, CL), part = (float)power(d, sd.n - (nc - 1) * CL);
-    float *state = A.slot_base[sd.slot] + A.state_off + (size_t)h * per + e;
+    // (a pointer from a table in memory: unless it is said to be global, its accesses wait for everything under way)
+    __attribute__((address_space(1))) float *state = (__attribute__((address_space(1))) float *)(A.slot_base[sd.slot] + A.state_off + (size_t)h * per + e);
     float S = sd.pos0 > 0 ? *state : 0.0f;
     float *p = A.st + ((size_t)first * A.heads + h) * per + e;
     const size_t step = (size_t)A.heads * per;
