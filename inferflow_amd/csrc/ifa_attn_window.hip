@@ -903,8 +903,11 @@ __global__ void __launch_bounds__(256) k_attn_parts_kept(WinAttnArgs P, TileArgs
     if (tid < 4) ((uint32_t *)(P.ws + A.marks))[4 * ((size_t)blockIdx.y * P.kv_heads + kvh) + tid] = any ? 1u : 0u;
 }
 
-// Workgroups that a block's keys, or its values, of so many 32s are shared out to: the chain of a step of a few rows (a head's angles in double, its norm, its turn) is as long as the keys a wave has.
-__host__ __device__ constexpr int part_shares(int NT) { return NT > 2 ? 2 : 1; }
+// Workgroups that a block's keys and its values of so many 32s are shared out to: the chain of a step of a few rows (a head's angles in double, its norm, its turn) is as long as the keys a wave has.
+// us with the attention, keys of 64 columns in one and in two: 16 heads (4 of keys) turned, 16 rows 18.7 / 15.5, 200 28.4 / 25.4, 2048 87.0 / 86.4; normed alone 18.4 / 16.3, 29.7 / 27.7, 57.4 / 55.4
+// (two launches 17.0, 29.0, 59).
+__host__ __device__ constexpr int key_shares(int NT) { return NT > 1 ? 2 : 1; }
+__host__ __device__ constexpr int value_shares(int NT) { return NT > 2 ? 2 : 1; }
 
 // ... with rows that the step brings: a workgroup per (head of keys, block of the step, share of its keys or values) lays a block's rows out as operands and stores those of the step into the cache on
 // their way: a position is in one of the step's blocks, and only there.  Fresh keys go through LDS, all asked for at once.  In front of them, for they take longest, the step's queries, normed and turned
@@ -916,7 +919,7 @@ template <int NTK, int NTV, bool TURN, bool SIDE>
 __global__ void __launch_bounds__(256) k_attn_parts(WinAttnArgs P, TileArgs A, FreshKV F, std::conditional_t<SIDE, SideArgs, int> side)
 {
     constexpr int DK = 32 * NTK, DV = 32 * NTV, KS = 2 * NTK, KROW = DK + 4, E = (DK + 63) / 64;
-    constexpr int KH = part_shares(NTK), VH = part_shares(NTV), KN = WT_K / KH, KI = (KN * (DK / 8) + 255) / 256, VN = 4 * DV / VH, VI = (VN + 255) / 256;
+    constexpr int KH = key_shares(NTK), VH = value_shares(NTV), KN = WT_K / KH, KI = (KN * (DK / 8) + 255) / 256, VN = 4 * DV / VH, VI = (VN + 255) / 256;
     int id = blockIdx.x;
     if constexpr (SIDE) {
         if (id < side.first) { ifachunk::linear_chunk(side.c, id % side.chunks, id / side.chunks % side.c.heads, id / side.chunks / side.c.heads); return; }
@@ -1110,8 +1113,8 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
     };
     auto marked = [&](int b, u32x4w m) -> uint64_t {
         uint32_t any = m[0] | m[1];
-        if constexpr (part_shares(NTK) + part_shares(NTV) > 2) any |= m[2];
-        if constexpr (part_shares(NTK) + part_shares(NTV) > 3) any |= m[3];
+        if constexpr (key_shares(NTK) + value_shares(NTV) > 2) any |= m[2];
+        if constexpr (key_shares(NTK) + value_shares(NTV) > 3) any |= m[3];
         return __builtin_amdgcn_ballot_w64(any != 0 && b + lane < b1);
     };
     u32x4w first;
@@ -1630,7 +1633,7 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
                              && (!out_bf16 || (ld16 % 4 == 0 && (uintptr_t)out_bf16 % 8 == 0));
             const int hx = heads / t.hpw;
             if (n_seqs > SIDE_SEQS) side = nullptr;          // (*side_done stays false)
-            if (fresh && !side && !fresh_pays((const ifa_seq_desc *)seqs_host, n_seqs, rows, t.blocks, kv_heads * (part_shares(NTK) + part_shares(NTV)), fresh->k != nullptr,
+            if (fresh && !side && !fresh_pays((const ifa_seq_desc *)seqs_host, n_seqs, rows, t.blocks, kv_heads * (key_shares(NTK) + value_shares(NTV)), fresh->k != nullptr,
                                               fresh->turn_q ? heads : 0)) {
                 if (const int rc = store_fresh()) return rc;
                 fresh = nullptr;
@@ -1656,8 +1659,8 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
             }
             const bool turn = F.rot_dims > 0 || F.q_rows > 0 || F.norm_w, kept = !F.k && !F.q_rows && !side;
             IFA_REQUIRE(!side || !turn, "%s: the linear attention goes beside keys that are not turned", who);
-            const unsigned part_wgs = (unsigned)(S.first + (size_t)(part_shares(NTK) + part_shares(NTV)) * kv_heads * t.blocks + F.q_wgs), tile_wgs = (unsigned)(hx * t.groups + S.pass);
-#define IFA_WT(K, V) { const size_t smem_p = ((size_t)(WT_K / part_shares(K)) * (32 * K + 4) + (size_t)std::max(WT_K / part_shares(K), 4) * F.rot_dims) * 4; \
+            const unsigned part_wgs = (unsigned)(S.first + (size_t)(key_shares(NTK) + value_shares(NTV)) * kv_heads * t.blocks + F.q_wgs), tile_wgs = (unsigned)(hx * t.groups + S.pass);
+#define IFA_WT(K, V) { const size_t smem_p = ((size_t)(WT_K / key_shares(K)) * (32 * K + 4) + (size_t)std::max(WT_K / key_shares(K), 4) * F.rot_dims) * 4; \
                        const size_t smem_t = (size_t)2 * kBlockPieces<K, V> * 16 + WT_WAVES * 64 * 4; \
                        const void *fn = vec ? (const void *)k_attn_tile<K, V, true> : (const void *)k_attn_tile<K, V, false>; \
                        IFA_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_t)); \
