@@ -1119,7 +1119,8 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
     };
     u32x4w first;
     // All of the lane's query at once (queries past the tile's last: that one again, not stored), in front of the first block's operands, behind whose requests it would wait for them: asked
-    // for by fours behind these, and every eight values looked at for ones that would round to infinity, a launch took 28.3 us for 601 rows of 8 heads, now 25.3 (2048 rows of 16 heads 122.8, 118.9).
+    // for by fours behind these, and every eight values looked at for ones that would round to infinity, a launch took 28.3 us for 601 rows of 8 heads,
+    // now 25.3 (2048 rows of 16 heads 122.8, 118.9; of 8 heads, whose tiles take ten blocks each, 60.1, 60.3).
     float qv[KS][8];
     {
         gfloat *qr = (gfloat *)P.q + (size_t)(r0 + min(32 * qsub + i, nq - 1)) * P.ldq + (size_t)h * dk;
@@ -1328,14 +1329,14 @@ __global__ void __launch_bounds__(64 * WT_WAVES, 2) k_attn_tile(WinAttnArgs P, T
 // did for all 128 columns, two chunks at a time.  us: Sopulorn 2048 tokens 13.7 -> 11.0, three prompts of 730 in all 10.4 -> 6.9; Gelarax 2048 of width 2048 13.7 -> 12.1, 601 of width 1024
 // 11.3 -> 9.0.  (The shares of all 32 possible chunks asked for at once: 208 registers, twice as long.)
 constexpr int WC_COLS = 32;
-__device__ __forceinline__ void tile_combine(const WinAttnArgs &P, const TileArgs &A, int hx, int bx, int tile_g, int z)
+__device__ __forceinline__ void tile_combine(const WinAttnArgs &P, const TileArgs &A, bool few, int hx, int bx, int tile_g, int z)
 {
     __shared__ float ms[WT_MAX_CHUNKS][32], ls[WT_MAX_CHUNKS][32], rows[32][WC_COLS + 1];
     const int tid = threadIdx.x, wave = z % WT_WAVES, c0 = z / WT_WAVES * WC_COLS, h = bx * A.hpw + wave % A.hpw, qsub = wave / A.hpw, dv = P.vdim;
     const int qw = 32 * (WT_WAVES / A.hpw), ncol = min(WC_COLS, dv - c0);
     int tile = tile_g;
     SeqDesc sd;
-    if (A.n_few) { const FewSeq f = few_of(A, tile_g, [](const FewSeq &x) { return x.tile0; }); sd = f.sd; tile -= f.tile0; }
+    if (few) { const FewSeq f = few_of(A, tile_g, [](const FewSeq &x) { return x.tile0; }); sd = f.sd; tile -= f.tile0; }
     else {
         const int sq = item_of(A.n_seqs, tile, [&](int x) { return x >= 0 ? (P.seqs[x].n + qw - 1) / qw : 0; });
         if (sq < 0) return;
@@ -1393,7 +1394,9 @@ __device__ __forceinline__ void tile_combine(const WinAttnArgs &P, const TileArg
     }
 }
 
-__global__ void __launch_bounds__(256) k_attn_tile_combine(WinAttnArgs P, TileArgs A) { tile_combine(P, A, gridDim.x, blockIdx.x, blockIdx.y, blockIdx.z); }
+// (FEW_SEQS: a kernel for either side, the choice in front of a place costs 0.5 us: 16 sequences behind 300 keys 7.0 -> 6.5 us, 12 of 30 rows 7.6 -> 7.0, one of 2000 10.4 -> 10.1)
+template <bool FEW_SEQS>
+__global__ void __launch_bounds__(256) k_attn_tile_combine(WinAttnArgs P, TileArgs A) { tile_combine(P, A, FEW_SEQS, gridDim.x, blockIdx.x, blockIdx.y, blockIdx.z); }
 
 // ... behind the chunks' outputs of the linear attention beside it
 template <int DK, bool VEC>
@@ -1402,7 +1405,7 @@ __global__ void __launch_bounds__(256, ifachunk::chunk_out_waves(0, DK)) k_attn_
     int id = blockIdx.x;
     if (id < side.first) { ifachunk::chunk_out<0, DK, VEC>(side.c, id % side.chunks, id / side.chunks % side.c.heads, id / side.chunks / side.c.heads); return; }
     id -= side.first;
-    tile_combine(P, A, hx, id % hx, id / hx % A.tiles, id / hx / A.tiles);
+    tile_combine(P, A, A.n_few != 0, hx, id % hx, id / hx % A.tiles, id / hx / A.tiles);
 }
 
 // How a step's tiles are shared out: hpw query heads and qw queries per workgroup, cb key blocks per chunk, up to `chunks` chunks per tile, so that the
@@ -1684,7 +1687,8 @@ static int attention_launch(const char *who, const void *q_f32, size_t ldq, int 
                 if (side->dk == 64) IFA_JO(64) else IFA_JO(128)
 #undef IFA_JO
                 *side_done = true;
-            } else if (joins) hipLaunchKernelGGL(k_attn_tile_combine, dim3((unsigned)hx, (unsigned)t.tiles, joins), dim3(256), 0, ifa_s(stream), P, A);
+            } else if (joins && A.n_few) hipLaunchKernelGGL(k_attn_tile_combine<true>, dim3((unsigned)hx, (unsigned)t.tiles, joins), dim3(256), 0, ifa_s(stream), P, A);
+            else if (joins) hipLaunchKernelGGL(k_attn_tile_combine<false>, dim3((unsigned)hx, (unsigned)t.tiles, joins), dim3(256), 0, ifa_s(stream), P, A);
             IFA_LAUNCH_CHECK();
             return IFA_OK;
         }

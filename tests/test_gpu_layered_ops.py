@@ -445,10 +445,11 @@ def test_infinities_and_nan_in_chunks_reach_no_earlier_token_and_no_other_column
 
 
 # edges of the tiled kernel with a workspace: query tiles of 64 / 128 / 256 (groups of 4, 2, 1 heads), key blocks of 32, windows and kept tokens that begin and end
-# inside blocks and meet in one, one chunk and many (short and long key ranges beside each other), continued sequences, head sizes that are not whole 32s or 4s
+# inside blocks and meet in one, one chunk and many (short and long key ranges beside each other), continued sequences, four (placed by the launch's arguments) and five, head sizes that are not whole 32s or 4s
 TILE_WS = [(4, 1, 128, 128, 1 << 30, 0, [(0, 16)], 1.0), (8, 2, 128, 128, 1 << 30, 0, [(0, 65)], 1.0), (8, 2, 64, 128, 1 << 30, 0, [(0, 700), (0, 3), (610, 90)], 1.0),
            (4, 2, 96, 32, 40, 0, [(0, 257)], 1.0), (3, 3, 32, 96, 33, 31, [(0, 300), (500, 33)], 1.0), (6, 2, 128, 64, 64, 33, [(95, 70), (0, 64)], 1.0),
            (4, 1, 36, 20, 100, 70, [(0, 310)], 1.0), (2, 1, 127, 101, 32, 0, [(0, 129), (31, 32)], 1.0), (8, 2, 128, 128, 1024, 4, [(0, 1300)], 1.0),
+           (8, 2, 64, 96, 1 << 30, 0, [(0, 700), (0, 3), (610, 90), (300, 40)], 1.0), (8, 2, 64, 96, 1 << 30, 0, [(0, 700), (0, 3), (610, 90), (300, 40), (900, 1)], 1.0),
            (5, 1, 5, 3, 17, 300, [(200, 150)], 1.0), (8, 2, 128, 128, 1 << 30, 0, [(0, 200)], 1e4), (8, 2, 128, 128, 1 << 30, 0, [(0, 200)], 1e-7)]
 
 
