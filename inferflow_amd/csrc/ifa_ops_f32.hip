@@ -441,7 +441,7 @@ __global__ void __launch_bounds__(1024) k_argmax_f32(const float *__restrict__ l
 // The same for one row of many columns in two launches: a workgroup per part of the row (one compute unit takes a row of 32000, 128 KB, no faster than 7.9 us), then a wave over the parts.  step:
 // the row is a decode step's: its token goes on to be the next one's, inside the step's graph (a launch of its own behind it before: 235.3 -> 230.6 us a token of a Gelarax model of width 1024).
 constexpr int AM_PART = 1024, AM_PARTS = 64;          // columns a part (more where a row has more of them), most parts
-constexpr size_t AM_ONE = 20480;                      // rows that one workgroup takes as fast
+constexpr size_t AM_ONE = 40960;                      // columns of a row that one workgroup takes as fast
 struct AmBest { float v; int i; };
 __device__ __forceinline__ void am_wave(AmBest &b)
 {
@@ -697,8 +697,9 @@ size_t ifa_argmax_parts_bytes() { return AM_PARTS * sizeof(AmBest); }
 int ifa_argmax_parts_f32(const float *logits, size_t n, size_t row_stride, size_t rows, const int *excluded_dev, int *out_dev, void *ws, const IfaStepAdvance *step, ifa_stream stream)
 {
     IFA_REQUIRE(logits && out_dev && ws && n > 0 && rows > 0 && n < (1u << 30) && (!step || rows == 1), "ifa_argmax_parts_f32: bad arguments");
-    // (more rows: a workgroup each, side by side -- six rows of 32000 9.2 us in one launch, no more than the two.  Short rows with no step behind them: one launch is the shorter way, us from the first
-    // launch's start to the last one's end for rows of 4096 / 16384 / 32000 / 65536 / 128256: one 6.6 / 8.2 / 10.2 / 14.2 / 22.8, two 8.9 / 8.9 / 8.8 / 8.9 / 8.8)
+    // (more rows: a workgroup each, side by side -- six rows of 32000 9.2 us in one launch, no more than the two.  Short rows with no step behind them: one launch is the shorter way.  us at the
+    // end of a prompt's pass, where neither kernel's code is at hand, from the head product's end: rows of 24576 / 32000 / 40960 / 49152 / 65536 / 131072: one 7.0 / 9.2 / 9.2 to 10.4 / 10 to 11.2 / 12 to 13 / 21,
+    // two 8.7 to 10.6 for all of them)
     if (rows > 1 || (!step && n <= AM_ONE)) return ifa_argmax_rows_f32(logits, n, row_stride, rows, excluded_dev, out_dev, stream);
     const size_t part = std::max<size_t>(AM_PART, ((n + AM_PARTS - 1) / AM_PARTS + 3) / 4 * 4), parts = (n + part - 1) / part;
     const IfaStepAdvance st = step ? *step : IfaStepAdvance{};
